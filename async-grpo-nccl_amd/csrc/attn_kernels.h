@@ -30,9 +30,10 @@
 // while the dK/dV kernel holds two accumulator sets (128 registers) plus its K and V operands, runs one wavefront per
 // SIMD and has its step software-pipelined by hand (one MFMA per softmax element); splitting it into a dV and a dK
 // launch (two wavefronts per SIMD each, S computed twice) measured slower, as did a second LDS buffer.  The second
-// forms, the defaults (varlen_attn_fwd2_kernel, varlen_attn_dq2_kernel, varlen_attn_dkv2_kernel, further down),
+// forms (varlen_attn_fwd2_kernel and varlen_attn_dq2_kernel, the defaults, and varlen_attn_dkv2_kernel, further down)
 // move tiles global -> LDS directly and schedule every LDS access by hand; the dK/dV one deals a wavefront's
-// work to a pair so that it, too, runs two wavefronts per SIMD.
+// work to a pair so that it, too, runs two wavefronts per SIMD.  The default dK/dV kernel is a third form,
+// varlen_attn_dkv3_kernel in attn_keyside.h: four independent wavefronts on 64 keys, one per SIMD, no barriers.
 // Launch order: work-groups start in the order of a device-built list, tiles with the most steps first (a third of
 // a launch was tail before), and in the query-side kernels the query heads of one K/V group share an XCD.
 #pragma once
@@ -1741,7 +1742,7 @@ __global__ __launch_bounds__(256, 2) void varlen_attn_dq2_kernel(AttnParams p) {
 }
 
 // seg_start[t], seg_end[t] from cu_seqlens (tokens outside every segment stand alone)
-__global__ void segment_bounds_kernel(const int* cu, int nseq, int T, int* seg_start, int* seg_end) {
+static __global__ void segment_bounds_kernel(const int* cu, int nseq, int T, int* seg_start, int* seg_end) {
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= T) return;
   // largest i with cu[i] <= t
@@ -1776,7 +1777,7 @@ __host__ __device__ inline long long attn_order_offset(int T, int list) {     //
 __host__ __device__ inline long long attn_bounds_elems(int T) { return attn_order_offset(T, 3) + (T + 31) / 32; }
 
 constexpr int kAttnOrderSlices = 8;      // work-groups per list: each ranks 1/8 of the list's tiles
-__global__ void attn_tile_order_kernel(const int* seg_start, const int* seg_end, int T, int causal, int* ws) {
+static __global__ void attn_tile_order_kernel(const int* seg_start, const int* seg_end, int T, int causal, int* ws) {
   __shared__ int wk[kAttnMaxSorted], rk[kAttnMaxSorted / kAttnOrderSlices];
   const int list = blockIdx.x;                       // 0: keys; 1, 2, 3: queries 128 / 64 / 32
   const bool keys = list == 0;

@@ -6,6 +6,10 @@
 
 using namespace fgrpo;
 
+namespace fgrpo {
+int launch_attn_dkv3(int D, const AttnParams& p, hipStream_t st);      // launch_attn_keyside.hip
+}
+
 namespace {
 // Query heads per work-group of the query-side kernels (tile = 128 / heads tokens).  Short segments gain from short
 // tiles (less masked work on the diagonal and at segment boundaries) as long as the heads of a group fill the
@@ -144,6 +148,7 @@ int fgrpo_varlen_attn_bwd(const void* dout, const void* q, const void* k, const 
   }
   rc = launch_query_side<DqLauncher>(D, attn_heads_per_group(Hq / Hkv, T, n_seq), p, T, Hq, Hkv, bounds_ws, st);
   if (rc) return rc;
+  if (g_tune.attn_dkv != 1 && g_tune.attn_dkv != 2) return launch_attn_dkv3(D, p, st);
   const dim3 grid_k(Hkv, (T + kAttnBQ - 1) / kAttnBQ);
   if (g_tune.attn_dkv == 1) {
     if (D == 128) hipLaunchKernelGGL(varlen_attn_dkv_kernel<128>, grid_k, dim3(256), 0, st, p);

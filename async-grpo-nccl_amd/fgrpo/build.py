@@ -23,7 +23,10 @@ _ALT = "" if LIB_PATH == os.path.join(CSRC, "libfgrpo.so") else "_" + os.path.sp
 USAGE_PATH = os.path.join(CSRC, f"resource_usage{_ALT}.json")
 OBJ_DIR = os.path.join(CSRC, "build" + _ALT)
 
-SOURCES = ["fgrpo_api.hip", "launch_lmhead.hip", "launch_gemm.hip", "launch_attn.hip"]
+SOURCES = ["fgrpo_api.hip", "launch_lmhead.hip", "launch_gemm.hip", "launch_attn.hip", "launch_attn_keyside.hip"]
+# this unit keeps its accumulators in named accumulation registers: the results of the matrix instructions the compiler
+# schedules must stay out of those
+SOURCE_FLAGS = {"launch_attn_keyside.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]}
 
 HIPCC_FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC",
@@ -47,6 +50,8 @@ TWO_PER_SIMD = ("TileCfgILi256ELi256ELi64ELi2ELi4ELi2ELi2ELb1EE",      # id 8
                 "varlen_attn_fwd2_kernel", "varlen_attn_dq2_kernel", "varlen_attn_dkv2_kernel")
 # attention kernels whose LDS reads are inline assembly: a spilled register could be one whose data is still on its way
 ASM_READ_ATTN = ("varlen_attn_fwd2_kernel", "varlen_attn_dq2_kernel", "varlen_attn_dkv2_kernel")
+# ... and the one that runs one wavefront per SIMD (accumulators in the accumulation registers): no spills either
+ASM_READ_ONE_PER_SIMD = ("varlen_attn_dkv3_kernel",)
 MUST_EXIST = TILE_KERNELS + ("varlen_attn_fwd_kernel", "varlen_attn_dq_kernel", "varlen_attn_dkv_kernel") + ASM_READ_ATTN
 
 _FIELDS = {
@@ -83,7 +88,7 @@ def check_resource_usage(usage: dict) -> list:
         if tile and ASM_READ_CFG.search(name) and (u.get("scratch", 0) or u.get("vgpr_spill", 0)):
             bad.append(f"{name}: inline-assembly fragment reads with {u.get('vgpr_spill')} spilled VGPRs "
                        f"({u.get('scratch')} B/lane of scratch)")
-        if any(k in name for k in ASM_READ_ATTN) and (u.get("scratch", 0) or u.get("vgpr_spill", 0)):
+        if any(k in name for k in ASM_READ_ATTN + ASM_READ_ONE_PER_SIMD) and (u.get("scratch", 0) or u.get("vgpr_spill", 0)):
             bad.append(f"{name}: inline-assembly fragment reads with {u.get('vgpr_spill')} spilled VGPRs "
                        f"({u.get('scratch')} B/lane of scratch)")
         if any(k in name for k in TWO_PER_SIMD) and (tile or "varlen" in name):
@@ -99,7 +104,7 @@ def check_resource_usage(usage: dict) -> list:
 def _compile(src: str, verbose: bool):
     hipcc = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
     obj = os.path.join(OBJ_DIR, os.path.splitext(src)[0] + ".o")
-    cmd = [hipcc, *HIPCC_FLAGS, *os.environ.get("FGRPO_EXTRA_FLAGS", "").split(), "-c", os.path.join(CSRC, src), "-o", obj]
+    cmd = [hipcc, *HIPCC_FLAGS, *SOURCE_FLAGS.get(src, []), *os.environ.get("FGRPO_EXTRA_FLAGS", "").split(), "-c", os.path.join(CSRC, src), "-o", obj]
     if verbose:
         print(" ".join(cmd), flush=True)
     res = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)

@@ -473,3 +473,21 @@ def test_both_query_side_kernels_give_identical_results(dev):
         check(dev, "register-staged query-side kernels, head dim 64", 1000, [0, 130, 385, 390, 900, 1000], 14, 2, False, seed=22, D=64)
     finally:
         _lib.set_tuning(attn_qside=0, attn_heads=0)
+
+
+@pytest.mark.parametrize("T,cu,Hq,Hkv,causal,D", [
+    (1, [0, 1], 1, 1, True, 128), (31, [0, 31], 3, 1, True, 128), (33, [0, 1, 33], 2, 2, False, 64),
+    (64, [0, 64], 4, 4, True, 64), (65, [0, 63, 65], 5, 1, True, 128), (96, [0, 40, 96], 7, 1, False, 128),
+    (130, [0, 64, 128, 130], 14, 2, True, 64), (197, [0, 97, 129, 197], 6, 2, True, 128), (450, [0, 450], 1, 1, False, 64),
+])
+def test_key_side_kernel_at_the_edges_of_its_tiles(dev, T, cu, Hq, Hkv, causal, D):
+    """Four wavefronts share 64 keys and deal (32 queries, head) items among themselves: fewer items than wavefronts,
+    item counts off a multiple of four, last key and query blocks of every fill, segments that end on and beside a
+    tile edge.  Against the fp32 oracle; twice, bit for bit."""
+    from fgrpo import ops
+    check(dev, "key-side kernel", T, cu, Hq, Hkv, causal, seed=T, D=D)
+    q, k, v, do = (x.to(dev) for x in make(T, Hq, Hkv, T, D=D))
+    cu_t = torch.tensor(cu, dtype=torch.int32, device=dev)
+    out, lse = ops.varlen_attn_fwd(q, k, v, cu_t, None, causal)
+    a, b = (ops.varlen_attn_bwd(do, q, k, v, out, lse, cu_t, None, causal) for _ in range(2))
+    assert all(torch.equal(x, y) for x, y in zip(a, b))
