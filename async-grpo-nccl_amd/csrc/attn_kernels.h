@@ -62,7 +62,7 @@ struct AttnParams {
   float* lse;            // [Hq][T], natural log of the softmax denominator
   // backward
   const bf16_t* dout;    // [T][Hq][HD] contiguous
-  float* delta;          // [Hq][T] rowsum(dO * O): written by the dQ kernel, read by the dK/dV kernel
+  float* delta;          // [Hq][T] -rowsum(dO * O): written by the dQ kernel, read by the dK/dV kernel (negated: it is the addend of dP)
   const bf16_t* out_fwd; // [T][Hq][HD] the forward's output (backward only)
   bf16_t* dq;            // [T][Hq][HD] contiguous
   bf16_t* dk;            // [T][Hkv][HD] contiguous
@@ -405,7 +405,7 @@ __global__ __launch_bounds__(256, 2) void varlen_attn_dq_kernel(AttnParams p) {
       }
     }
     dl += attn_swap32(dl);
-    if (valid && h == 0) p.delta[(long long)hq * p.T + tq] = dl;    // for the dK/dV kernel, launched after this one
+    if (valid && h == 0) p.delta[(long long)hq * p.T + tq] = -dl;   // negated, for the dK/dV kernel, launched after this one
   }
   const float c = p.scale * kLog2e;
 
@@ -522,7 +522,7 @@ __global__ __launch_bounds__(256) void varlen_attn_dkv_kernel(AttnParams p) {
         const int t = qb + threadIdx.x;
         const bool ok = t < q_end;
         n_lse = ok ? p.lse[(long long)hq * p.T + t] * kLog2e : 0.f;
-        n_dl = ok ? p.delta[(long long)hq * p.T + t] : 0.f;
+        n_dl = ok ? -p.delta[(long long)hq * p.T + t] : 0.f;
         n_lo = ok ? p.seg_start[t] : 1;
         n_hi = ok ? (p.causal ? t : p.seg_end[t] - 1) : 0;
       }
@@ -862,7 +862,7 @@ __global__ __launch_bounds__(512) void varlen_attn_dkv2_kernel(AttnParams p) {
       const bool ok = r_t < q_end;
       const uint32_t rw = lds0 + kRw + buf * kRows + threadIdx.x * 4;
       lds_write_u32_asm<0>(rw, __float_as_uint(ok ? r_lse * kLog2e : 0.f));
-      lds_write_u32_asm<kAttnBK * 4>(rw, __float_as_uint(ok ? r_dl : 0.f));
+      lds_write_u32_asm<kAttnBK * 4>(rw, __float_as_uint(ok ? -r_dl : 0.f));
       lds_write_u32_asm<2 * kAttnBK * 4>(rw, (uint32_t)(ok ? r_lo : 1));
       lds_write_u32_asm<3 * kAttnBK * 4>(rw, (uint32_t)(ok ? (p.causal ? r_t : r_end - 1) : 0));
     }
@@ -1533,7 +1533,7 @@ __global__ __launch_bounds__(256, 2) void varlen_attn_dq2_kernel(AttnParams p) {
       }
     }
     dl += attn_swap32(dl);
-    if (valid && h == 0) p.delta[(long long)hq * p.T + tq] = dl;    // for the dK/dV kernel, launched after this one
+    if (valid && h == 0) p.delta[(long long)hq * p.T + tq] = -dl;   // negated, for the dK/dV kernel, launched after this one
   }
   const float c = p.scale * kLog2e;
 #pragma unroll

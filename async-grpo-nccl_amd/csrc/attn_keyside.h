@@ -1,7 +1,7 @@
 // dK / dV of the packed attention with one wavefront per SIMD and no barrier in its loop (head dimension HD = 128 or
 // 64).  A work-group owns 64 keys of one K/V head; its four wavefronts deal the work on those keys among themselves -
 // item n = (32 queries, query head) goes to wavefront n % 4 - and each walks its items alone: it brings the item's
-// Q / dO rows into two LDS buffers of its own (global -> LDS, an item ahead), waits for nothing but its own loads,
+// Q / dO rows into two LDS buffers of its own (global -> LDS, two items ahead), waits for nothing but its own loads,
 // and keeps both accumulators for all 64 keys (256 accumulation registers at HD = 128).  The four accumulator sets are
 // added in a fixed order at the end, through LDS: bit-reproducible, no atomics.
 //
@@ -15,30 +15,34 @@
 // rate, of the ~70 that direct-to-LDS loads sustain.
 //
 // Measured, dQ + dK/dV, paired kernel -> this one on one box: 4 segments of 8192 tokens, 28 / 4 heads of 128:
-// 7.20 -> 6.17 ms; 32768 tokens in segments of 128..1024, 12 / 2 heads of 128: 442 -> 409 us; 12345 such tokens, 14 / 2
-// heads of 64: 245 -> 143 us; 6535 tokens, 12 / 2 heads of 128: 160 -> 101 us.  It was faster at every size tried, so
-// no rule picks between the two.  Counters at the long shape: matrix pipe 0.58 busy, a fifth of the time waiting
-// for tiles (with every load aimed at one tile: 5.38 ms).
+// 7.20 -> 6.00 ms; 32768 tokens in segments of 128..1024, 12 / 2 heads of 128: 442 -> 393 us; 12345 such tokens, 14 / 2
+// heads of 64: 245 -> 109 us; 8773 tokens in segments of up to 8192, 14 / 2 heads of 64: 1222 -> 735 us.  It was faster
+// at every size tried, so no rule picks between the two.  Counters at the long shape: matrix pipe 0.61 busy at 1.81
+// GHz, the power limit; at the short ones the clock is 2.4 GHz and the pipe 0.38 busy: opening and closing a
+// work-group and the masked items weigh there.
 //
 // Orientation and register permutation as in attn_kernels.h (S = Q K^T: a lane owns a key).  One item, with the
 // vector work of one stage behind the matrix instructions of the next (a 32x32x16 instruction hides about 20 cycles
 // of it):
-//   S(both key blocks)            | loads of the next item issued between the instructions
-//   dP                            | P = exp2(S c - lse) of rows 0..7 of each lane's 16, packed to bf16
-//   dV += P^T dO   (rows 0..7)    | P of rows 8..15
-//   dV             (rows 8..15)   | dS = P (dP - delta) of rows 0..7
-//   dK += dS^T Q   (rows 0..7)    | dS of rows 8..15
-//   dK             (rows 8..15)   | first Q fragments of the next item on their way
+//   S of key block 0             |
+//   S of key block 1             | P = exp2(S c - lse) of key block 0
+//   dP of both                   | P of key block 1
+//   dV += P^T dO   (rows 0..7 of each lane's 16)  | dS = P (dP - delta) of rows 0..7
+//   dK += dS^T Q   (rows 0..7)   | dS of rows 8..15
+//   dK             (rows 8..15)  | Q loads of the item after next, into the rows just read
+//   dV             (rows 8..15)  | its dO loads; first Q fragments of the next item on their way
 // -delta enters as the addend of dP's first instruction.  K lives in registers (64 keys x HD), V in LDS, shared by
 // the four wavefronts (both in registers would exceed the file beside the accumulators).
 #pragma once
 #include "attn_kernels.h"
 
+#define FGRPO_LDS_AT(a) ((__attribute__((address_space(3))) void*)(uint32_t)(a))      // LDS pointer from a byte address
+
 namespace fgrpo {
 
 constexpr int kDkv3Keys = 64, kDkv3Rows = 32;
 template <int HD>
-constexpr int kDkv3Buf = 2 * kDkv3Rows * HD * 2 + 512;                 // Q | dO | lse, delta | seg_start, seg_end of 32 queries
+constexpr int kDkv3Buf = 2 * kDkv3Rows * HD * 2 + 512;                 // Q | dO | lse | -delta of 32 queries
 template <int HD>
 constexpr int kDkv3SumStride = HD * 4 + 32;                            // fp32 row of the closing sum: the two lane halves (rows 4 apart) hit different banks
 template <int HD>
@@ -87,11 +91,10 @@ __device__ __forceinline__ void dkv3_acc_clear() {
   if constexpr (HD == 128) asm volatile("v_accvgpr_write_b32 a[%0], 0" : : "n"(REG) : FGRPO_DKV3_CLOBBER_256);
   else asm volatile("v_accvgpr_write_b32 a[%0], 0" : : "n"(REG) : FGRPO_DKV3_CLOBBER_128);
 }
-template <int REG>
-__device__ __forceinline__ float dkv3_acc_read() {
-  float x;
-  asm volatile("v_accvgpr_read_b32 %0, a[%1]" : "=v"(x) : "n"(REG));
-  return x;
+template <int REG, int OFF>
+__device__ __forceinline__ void dkv3_acc_to_lds(uint32_t addr) {       // LDS instructions take their data from these registers directly
+  static_assert(OFF >= 0 && OFF < 65536, "DS offset field");
+  asm volatile("ds_write_b32 %0, a[%1] offset:%2" : : "v"(addr), "n"(REG), "n"(OFF) : "memory");
 }
 
 template <int HD>
@@ -147,6 +150,17 @@ __global__ __launch_bounds__(256, 1) void varlen_attn_dkv3_kernel(AttnParams p) 
 #pragma unroll
     for (int st = 0; st < KS; ++st) kf[kb][st] = __builtin_bit_cast(u32x4_t, f[st]);
   }
+  // the queries that see the lane's key: key_n of them, from the key itself (causal) or its segment's start on; kept
+  // relative to the lane's first row of a query block
+  int key_lo[2];
+  uint32_t key_n[2];
+#pragma unroll
+  for (int kb = 0; kb < 2; ++kb) {
+    const int key = min(k0 + 32 * kb + (lane & 31), p.T - 1), lo = p.causal ? key : p.seg_start[key];
+    key_lo[kb] = lo - 4 * h;
+    key_n[kb] = k0 + 32 * kb + (lane & 31) < p.T ? (uint32_t)max(min(p.seg_end[key], q_end) - lo, 0) : 0u;
+    asm volatile("" : "+v"(key_lo[kb]), "+v"(key_n[kb]));
+  }
   const float c = p.scale * kLog2e;
 
   // accumulator blocks: dV[kb][nb] = kb DB + nb, dK behind them
@@ -154,7 +168,10 @@ __global__ __launch_bounds__(256, 1) void varlen_attn_dkv3_kernel(AttnParams p) 
   static_for<4 * DB * 16>([&](auto rc) { dkv3_acc_clear<HD, decltype(rc)::value>(); });
 
   // ---- loads of an item.  Instruction i of a tile fills its KiB i: RPI rows; lane l lands at 16 l of it, i.e. row
-  // i RPI + l / (HD/8), chunk slot l % (HD/8), and fetches the chunk the swizzle puts there (four or two patterns)
+  // i RPI + l / (HD/8), chunk slot l % (HD/8), and fetches the chunk the swizzle puts there (four or two patterns).
+  // Two items are in flight: a buffer's Q rows (with the per-query scalars) are free when the item's last Q^T
+  // fragments have been read, three quarters through it, its dO rows an eighth later, and the item after next takes
+  // them at once.
   constexpr int RPI = 1024 / RB, NLD = kDkv3Rows / RPI, NPAT = HD == 128 ? 4 : 2;
   const long long do_st = (long long)p.Hq * HD;
   uint32_t foq[NPAT], fod[NPAT];
@@ -165,64 +182,74 @@ __global__ __launch_bounds__(256, 1) void varlen_attn_dkv3_kernel(AttnParams p) 
     fod[i] = (uint32_t)((row * do_st + ch * 8) * 2);
   }
   const int sq = (int)(RPI * p.q_st * 2), sd = (int)(RPI * do_st * 2);
-  // lanes 0..31 bring lse and seg_start of the 32 queries, lanes 32..63 delta and seg_end
-  const float* sc0 = h ? p.delta : p.lse;
-  const int* sc1 = h ? p.seg_end : p.seg_start;
-  const uint32_t T = (uint32_t)p.T;
-  // the walk goes from the last queries to the first, heads inside: work-groups on the same segment start at the same
-  // rows and pass over them together, so that one L2 serves them all
-  int g_n = wave % G, qb_n = q_begin + (nqb - 1 - wave / G) * kDkv3Rows;      // the item the next loads bring
+  // The walk goes from the last queries to the first, heads inside: work-groups on the same segment start at the same
+  // rows and pass over them together, so that one L2 serves them all.  A step of it is a few additions.
+  int g_f = wave % G, qb_f = q_begin + (nqb - 1 - wave / G) * kDkv3Rows;      // the item the loads are at
+  const char* f_qp = (const char*)(p.q + (long long)(hkv * G + g_f) * p.q_sh + (long long)qb_f * p.q_st);
+  const char* f_dp = (const char*)(p.dout + (long long)(hkv * G + g_f) * HD + (long long)qb_f * do_st);
+  long long f_qb = ((long long)q_end - qb_f - 1) * p.q_st * 2 + RB;           // bytes to the end of the head's last row
+  long long f_db = ((long long)q_end - qb_f - 1) * do_st * 2 + RB;
+  // per-query scalars: rows past the end of the queries read what lies there or zero: finite, and hidden
+  const uint32_t los = (lane & 31) * 4;
+  const __amdgpu_buffer_rsrc_t rsl = make_rsrc(p.lse + (long long)hkv * G * p.T, (uint32_t)G * (uint32_t)p.T * 4);
+  const __amdgpu_buffer_rsrc_t rsx = make_rsrc(p.delta + (long long)hkv * G * p.T, (uint32_t)G * (uint32_t)p.T * 4);
   __amdgpu_buffer_rsrc_t rsq, rsd;
-  const float* l_p0 = nullptr;
-  const int* l_p1 = nullptr;
-  auto fetch_setup = [&](bool more) {      // without a next item the loads go out all the same, to an empty range (zeros) and the last scalars
-    const int hq = hkv * G + g_n;
-    const long long rows = (long long)q_end - qb_n;            // >= 1
-    long long bq = more ? (rows - 1) * p.q_st * 2 + RB : 0, bd = more ? (rows - 1) * do_st * 2 + RB : 0;
+  const long long h_q = p.q_sh * 2, r_q = (long long)kDkv3Rows * p.q_st * 2, r_d = (long long)kDkv3Rows * do_st * 2;
+  auto fetch_setup = [&](bool more) {      // without an item the loads go out all the same: to an empty range (zeros), the last item's scalars
+    long long bq = more ? f_qb : 0, bd = more ? f_db : 0;
     if (bq > 0xffffffffLL) bq = 0xffffffffLL;
     if (bd > 0xffffffffLL) bd = 0xffffffffLL;
-    rsq = make_rsrc(p.q + (long long)hq * p.q_sh + (long long)qb_n * p.q_st, (uint32_t)bq);
-    rsd = make_rsrc(p.dout + (long long)hq * HD + (long long)qb_n * do_st, (uint32_t)bd);
-    const uint32_t row = (uint32_t)min(qb_n + (lane & 31), q_end - 1);
-    l_p0 = sc0 + ((unsigned long long)hq * T + row);
-    l_p1 = sc1 + row;
+    rsq = make_rsrc(f_qp, (uint32_t)bq);
+    rsd = make_rsrc(f_dp, (uint32_t)bd);
   };
-  auto fetch_piece = [&](auto ic, char* buf) {                 // 2 NLD + 2 instructions
+  auto fetch_advance = [&]() {             // four items on
+    g_f += 4;
+    f_qp += 4 * h_q, f_dp += 4 * HD * 2;
+    while (g_f >= G) {
+      g_f -= G, qb_f -= kDkv3Rows;
+      f_qp -= G * h_q + r_q, f_dp -= (long long)G * HD * 2 + r_d;
+      f_qb += r_q, f_db += r_d;
+    }
+  };
+  auto fetch_q = [&](auto ic, uint32_t buf, int step) {                   // NLD + 2 instructions: Q rows, scalars
     constexpr int i = decltype(ic)::value;
-    if constexpr (i < NLD) __builtin_amdgcn_raw_ptr_buffer_load_lds(rsq, FGRPO_LDS_PTR(buf + i * 1024), 16, (int)foq[i % NPAT], i * sq, 0, 0);
-    else if constexpr (i < 2 * NLD)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rsd, FGRPO_LDS_PTR(buf + i * 1024), 16, (int)fod[i % NPAT], (i - NLD) * sd, 0, 0);
-    else if constexpr (i == 2 * NLD) __builtin_amdgcn_global_load_lds(FGRPO_GLOBAL_PTR(l_p0), FGRPO_LDS_PTR(buf + kSc), 4, 0, 0);
-    else __builtin_amdgcn_global_load_lds(FGRPO_GLOBAL_PTR(l_p1), FGRPO_LDS_PTR(buf + kSc + 256), 4, 0, 0);
+    if constexpr (i < NLD) __builtin_amdgcn_raw_ptr_buffer_load_lds(rsq, FGRPO_LDS_AT(buf + i * 1024), 16, (int)foq[i % NPAT], i * step, 0, 0);
+    else if constexpr (i == NLD) __builtin_amdgcn_raw_ptr_buffer_load_lds(rsl, FGRPO_LDS_AT(buf + kSc), 4, (int)los, (g_f * p.T + qb_f) * 4, 0, 0);
+    else __builtin_amdgcn_raw_ptr_buffer_load_lds(rsx, FGRPO_LDS_AT(buf + kSc + 256), 4, (int)los, (g_f * p.T + qb_f) * 4, 0, 0);
   };
-  auto advance = [&]() {
-    g_n += 4;
-    while (g_n >= G) g_n -= G, qb_n -= kDkv3Rows;
+  auto fetch_d = [&](auto ic, uint32_t buf, int step) {                   // NLD instructions: dO rows
+    constexpr int i = decltype(ic)::value;
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsd, FGRPO_LDS_AT(buf + kT + i * 1024), 16, (int)fod[i % NPAT], i * step, 0, 0);
   };
-  char* buf_w = smem + wave * 2 * kBuf;
   auto fence = []() { __builtin_amdgcn_sched_barrier(0); };
 #pragma unroll
   for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
     for (int st = 0; st < KS; ++st) asm volatile("" : "+v"(kf[kb][st]));      // complete before the loop
 
-  int qb = qb_n;                                               // the item being computed
+  int g_c = g_f, qb = qb_f;                                    // the item being computed
+  constexpr int kItemLoads = 2 * NLD + 2;
   if (wave < NI) {
-    fetch_setup(true);
-    static_for<2 * NLD + 2>([&](auto ic) { fetch_piece(ic, buf_w); });
-    if (wave + 4 < NI) advance();
+    static_for<2>([&](auto bc) {
+      constexpr int b = decltype(bc)::value;
+      const bool more = wave + 4 * b < NI;
+      if (b == 1 && more) fetch_advance();
+      fetch_setup(more);
+      static_for<NLD + 2>([&](auto ic) { fetch_q(ic, base_w + b * kBuf, sq); });
+      static_for<NLD>([&](auto ic) { fetch_d(ic, base_w + b * kBuf, sd); });
+    });
+    FGRPO_WAIT_VMCNT(kItemLoads);                              // the V rows (requested first) and the first item
+  } else {
+    FGRPO_WAIT_VMCNT(0);
   }
-  FGRPO_WAIT_VMCNT(0);
-  wg_barrier();                                                // the V tile is there too
+  wg_barrier();                                                // the whole V tile is there
 
-  u32x4_t qa[QG];                                              // first half of the Q fragments, carried across items
-  auto req_rows = [&](auto offc, auto stc, u32x4_t& f) { f = lds_read_u128_asm<decltype(offc)::value>(rowc[decltype(stc)::value]); };
+  u32x4_t qf[KS];                                              // Q rows of the item; the first half is requested by the item before
+  auto req_q = [&](auto offc, auto stc) { qf[decltype(stc)::value] = lds_read_u128_asm<decltype(offc)::value>(rowc[decltype(stc)::value]); };
   auto item = [&](auto curc, int n) {
     constexpr int cur = decltype(curc)::value, qt = cur * kBuf, dot = qt + kT, sct = cur * kBuf, nxt = (cur ^ 1) * kBuf;
-    const bool more = n + 4 < NI;
     const bool masked = qb < q_full || qb + kDkv3Rows > q_end;
-    char* nbuf = buf_w + nxt;
-    u32x4_t qh[QG], fo[2][2], fv[2][2][2], nd[4], l4[2][2];
+    u32x4_t fo[2][2], fv[2][2][2], nd[4], l4[4];
     AttnTr ta[DB], tb[DB];
     f32x16_t s[2], dp[2];
     u32x4_t pp[2][2], ds[2][2];                                // P, dS as operands: [key block][rows 8 s2 ..]
@@ -242,14 +269,12 @@ __global__ __launch_bounds__(256, 1) void varlen_attn_dkv3_kernel(AttnParams p) 
         t[db] = attn_rd_tr_asm<decltype(offc)::value>(tr[db][0], tr[db][1]);
       });
     };
-    auto e_el = [&](auto ec) {                                 // element e of a half: key block e % 2, row 8 half + e / 2
-      return [&](auto halfc) {
-        constexpr int e = decltype(ec)::value, half = decltype(halfc)::value, kb = e % 2, r = 8 * half + e / 2;
-        s[kb][r] = fast_exp2(__builtin_fmaf(s[kb][r], c, -__uint_as_float(l4[half][(e / 2) / 4][(e / 2) % 4])));
-        asm volatile("" : "+v"(s[kb][r]));
-      };
+    auto e_el = [&](auto kbc, auto rc) {                       // P in place of S
+      constexpr int kb = decltype(kbc)::value, r = decltype(rc)::value;
+      s[kb][r] = fast_exp2(__builtin_fmaf(s[kb][r], c, -__uint_as_float(l4[r / 4][r % 4])));
+      asm volatile("" : "+v"(s[kb][r]));
     };
-    auto f_el = [&](auto ec, auto halfc) {
+    auto f_el = [&](auto ec, auto halfc) {                     // dS in place of dP: element e of a half is key block e % 2, row 8 half + e / 2
       constexpr int e = decltype(ec)::value, half = decltype(halfc)::value, kb = e % 2, r = 8 * half + e / 2;
       dp[kb][r] = s[kb][r] * dp[kb][r];
       asm volatile("" : "+v"(dp[kb][r]));
@@ -259,110 +284,105 @@ __global__ __launch_bounds__(256, 1) void varlen_attn_dkv3_kernel(AttnParams p) 
                          pack_bf16x2(x[8 * half + 4], x[8 * half + 5]), pack_bf16x2(x[8 * half + 6], x[8 * half + 7])};
       return v;
     };
+    // hidden pairs of a key block become -inf; a branch of its own around the selects
+    auto hide = [&](auto kbc) {
+      constexpr int kb = decltype(kbc)::value;
+      int qv = qb;
+      asm volatile("" : "+s"(qv));                             // formed here: hoisted, it would be computed for every item
+      const uint32_t q0 = (uint32_t)(qv - key_lo[kb]);
+#pragma unroll
+      for (int r = 0; r < 16; ++r) s[kb][r] = q0 + (uint32_t)(8 * (r >> 2) + (r & 3)) < key_n[kb] ? s[kb][r] : -INFINITY;
+    };
+    // vector work w = 0 .. N - 1 dealt evenly to instructions m = M0 .. M1 - 1 of a run
+    auto deal = [&](auto nc, auto mc, auto m0c, auto m1c, auto&& side) {
+      constexpr int N = decltype(nc)::value, m = decltype(mc)::value - decltype(m0c)::value, M = decltype(m1c)::value - decltype(m0c)::value;
+      if constexpr (m >= 0 && m < M)
+        static_for<N>([&](auto wc) {
+          constexpr int w = decltype(wc)::value;
+          if constexpr (w >= N * m / M && w < N * (m + 1) / M) side(wc);
+        });
+    };
+#define FGRPO_IC(x) std::integral_constant<int, (x)>{}
     using H0 = std::integral_constant<int, 0>;
     using H1 = std::integral_constant<int, 1>;
-    using AV = std::integral_constant<int, kAccV>;
-    using AK = std::integral_constant<int, kAccK>;
 
-    // ---- S, first half of the k steps; the next item's loads go out between the instructions
-    fetch_setup(more);
-    static_for<QG>([&](auto ic) { req_rows(std::integral_constant<int, qt>{}, std::integral_constant<int, QG + decltype(ic)::value>{}, qh[decltype(ic)::value]); });
-    wait_lgkm<QG>();
+    // ---- S of key block 0
+    static_for<QG>([&](auto ic) { req_q(FGRPO_IC(qt), FGRPO_IC(QG + decltype(ic)::value)); });
+    static_for<4>([&](auto gc) { l4[decltype(gc)::value] = lds_read_u128_asm<sct + 32 * decltype(gc)::value>(scl); });
+    wait_lgkm<QG + 4>();
     fence();
-    constexpr int NF = 2 * NLD + 2, PF = (NF + 2 * KS - 1) / (2 * KS);      // loads behind each S instruction
-    auto s_mma = [&](u32x4_t& f, auto stc) {
-      constexpr int st = decltype(stc)::value;
-      attn_settle(f);
-      static_for<2>([&](auto kbc) {
-        constexpr int kb = decltype(kbc)::value;
-        if constexpr (st == 0) s[kb] = attn_mfma(f, kf[kb][st], f32x16_t{0.f});
-        else s[kb] = attn_mfma(f, kf[kb][st], s[kb]);
-        fence();
-        static_for<PF>([&](auto jc) {
-          constexpr int i = (2 * st + kb) * PF + decltype(jc)::value;
-          if constexpr (i < NF) fetch_piece(std::integral_constant<int, i>{}, nbuf);
-        });
-        fence();
-      });
+    auto s_mma = [&](auto kbc, auto stc) {
+      constexpr int kb = decltype(kbc)::value, st = decltype(stc)::value;
+      if constexpr (kb == 0) attn_settle(qf[st]);
+      if constexpr (st == 0) s[kb] = attn_mfma(qf[st], kf[kb][st], f32x16_t{0.f});
+      else s[kb] = attn_mfma(qf[st], kf[kb][st], s[kb]);
+      fence();
     };
-    static_for<QG>([&](auto ic) { s_mma(qa[decltype(ic)::value], ic); });
-    // ---- second half; -delta and the first dP group are on their way
-    static_for<4>([&](auto gc) { nd[decltype(gc)::value] = lds_read_u128_asm<sct + 128 + 32 * decltype(gc)::value>(scl); });
-    req_dp(H0{});
-    wait_lgkm<4 + 6>();
+    static_for<QG>([&](auto ic) { s_mma(H0{}, ic); });
+    wait_lgkm<0>();
     fence();
-    static_for<QG>([&](auto ic) { s_mma(qh[decltype(ic)::value], std::integral_constant<int, QG + decltype(ic)::value>{}); });
-    if (masked) {      // hidden pairs become -inf; a branch of its own around the selects
-      const int key0 = k0 + (lane & 31);
-      static_for<4>([&](auto gc) {
+    static_for<QG>([&](auto ic) {
+      constexpr int i = decltype(ic)::value;
+      s_mma(H0{}, FGRPO_IC(QG + i));
+      deal(FGRPO_IC(4), ic, FGRPO_IC(0), FGRPO_IC(QG), [&](auto gc) {
         constexpr int gr = decltype(gc)::value;
-        u32x4_t lo4 = lds_read_u128_asm<sct + 256 + 32 * gr>(scl), en4 = lds_read_u128_asm<sct + 384 + 32 * gr>(scl);
-        wait_lgkm<0>();
-        fence();
-        attn_settle(lo4);
-        attn_settle(en4);
+        attn_settle(l4[gr]);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int q = qb + 8 * gr + 4 * h + e;
-          const int hi = q < q_end ? (p.causal ? q : (int)en4[e] - 1) : -1;
-#pragma unroll
-          for (int kb = 0; kb < 2; ++kb) {
-            const int key = key0 + 32 * kb;
-            s[kb][4 * gr + e] = ((int)(key >= (int)lo4[e]) & (int)(key <= hi)) ? s[kb][4 * gr + e] : -INFINITY;
-          }
-        }
+        for (int e = 0; e < 4; ++e) l4[gr][e] = __float_as_uint(__uint_as_float(l4[gr][e]) * kLog2e);
+        attn_settle(l4[gr]);
       });
       fence();
-    }
-    // ---- dP: groups of two k steps, P of rows 0..7 behind all but the first
-    f32x16_t ndelta;
+    });
+    if (masked) hide(H0{});
+    // ---- S of key block 1 | P of key block 0
+    static_for<4>([&](auto gc) { nd[decltype(gc)::value] = lds_read_u128_asm<sct + 256 + 32 * decltype(gc)::value>(scl); });
+    static_for<KS>([&](auto ic) {
+      constexpr int i = decltype(ic)::value;
+      s_mma(H1{}, ic);
+      deal(FGRPO_IC(16), ic, FGRPO_IC(1), FGRPO_IC(KS), [&](auto rc) { e_el(H0{}, rc); });
+      fence();
+      if constexpr (i == KS / 2 - 1) {
+        FGRPO_WAIT_VMCNT(kItemLoads);                          // this item's dO rows: later loads are the next item's
+        req_dp(H0{});
+        fence();
+      }
+    });
+    if (masked) hide(H1{});
+    // ---- dP, starting from -delta | P of key block 1
     static_for<NG>([&](auto gc) {
       constexpr int g = decltype(gc)::value;
-      if constexpr (g + 1 < NG) req_dp(std::integral_constant<int, g + 1>{});
-      if constexpr (g == 0) static_for<2>([&](auto ic) { l4[0][decltype(ic)::value] = lds_read_u128_asm<sct + 32 * decltype(ic)::value>(scl); });
-      if constexpr (g + 1 == NG) {
-        static_for<2>([&](auto ic) { l4[1][decltype(ic)::value] = lds_read_u128_asm<sct + 64 + 32 * decltype(ic)::value>(scl); });
-        req_tr(std::integral_constant<int, dot>{}, ta);
-      }
-      wait_lgkm<(g + 1 < NG ? 6 : 0) + (g == 0 ? 2 : 0) + (g + 1 == NG ? 2 + 2 * DB : 0)>();
+      if constexpr (g + 1 < NG) req_dp(FGRPO_IC(g + 1));
+      else req_tr(FGRPO_IC(dot), ta);
+      wait_lgkm<(g + 1 < NG ? 6 : 2 * DB)>();
       fence();
-      if constexpr (g == 0) {
-#pragma unroll
-        for (int gr = 0; gr < 4; ++gr) {
-          attn_settle(nd[gr]);
-#pragma unroll
-          for (int e = 0; e < 4; ++e) ndelta[4 * gr + e] = -__uint_as_float(nd[gr][e]);
-        }
-      }
-      if constexpr (g == 1) {
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-          attn_settle(l4[0][i]);
-#pragma unroll
-          for (int e = 0; e < 4; ++e) l4[0][i][e] = __float_as_uint(__uint_as_float(l4[0][i][e]) * kLog2e);
-        }
-      }
       static_for<2>([&](auto ic) {
         constexpr int i = decltype(ic)::value, st = 2 * g + i;
         attn_settle(fo[g % 2][i]);
         static_for<2>([&](auto kbc) {
-          constexpr int kb = decltype(kbc)::value, m = 4 * (g - 1) + 2 * i + kb, M = 4 * (NG - 1);
+          constexpr int kb = decltype(kbc)::value, m = 4 * g + 2 * i + kb;
           attn_settle(fv[g % 2][i][kb]);
-          dp[kb] = attn_mfma(fo[g % 2][i], fv[g % 2][i][kb], st == 0 ? ndelta : dp[kb]);
+          if constexpr (st == 0) {
+            f32x16_t ndelta;
+#pragma unroll
+            for (int gr = 0; gr < 4; ++gr) {
+              if constexpr (kb == 0) attn_settle(nd[gr]);
+#pragma unroll
+              for (int e = 0; e < 4; ++e) ndelta[4 * gr + e] = __uint_as_float(nd[gr][e]);
+            }
+            dp[kb] = attn_mfma(fo[0][0], fv[0][0][kb], ndelta);
+          } else {
+            dp[kb] = attn_mfma(fo[g % 2][i], fv[g % 2][i][kb], dp[kb]);
+          }
           fence();
-          if constexpr (g >= 1)
-            static_for<16>([&](auto ec) {
-              constexpr int e = decltype(ec)::value;
-              if constexpr (e >= 16 * m / M && e < 16 * (m + 1) / M) e_el(ec)(H0{});
-            });
+          deal(FGRPO_IC(16), FGRPO_IC(m), FGRPO_IC(1), FGRPO_IC(2 * KS), [&](auto rc) { e_el(H1{}, rc); });
           fence();
         });
       });
     });
 #pragma unroll
     for (int kb = 0; kb < 2; ++kb) pp[kb][0] = pack(s[kb], 0);
-    // ---- dV and dK in quarters of 2 DB instructions
-    constexpr int NQ = 2 * DB, EPI = 16 / NQ;                  // vector elements behind each instruction
+    // ---- dV and dK in quarters of NQ instructions
+    constexpr int NQ = 2 * DB;
     auto quarter = [&](AttnTr (&t)[DB], u32x4_t (&op)[2][2], auto s2c, auto accc, auto&& side) {
       constexpr int s2 = decltype(s2c)::value, acc = decltype(accc)::value;
       static_for<DB>([&](auto dc) {
@@ -372,66 +392,82 @@ __global__ __launch_bounds__(256, 1) void varlen_attn_dkv3_kernel(AttnParams p) 
           constexpr int kb = decltype(kbc)::value;
           dkv3_mfma<HD, acc + kb * DB + db, db == 0>(op[kb][s2], b);
           fence();
-          static_for<EPI>([&](auto jc) { side(std::integral_constant<int, (2 * db + kb) * EPI + decltype(jc)::value>{}); });
+          side(FGRPO_IC(2 * db + kb));
           fence();
         });
       });
     };
-    req_tr(std::integral_constant<int, dot + 16 * RB>{}, tb);
+    // dV, rows 0..7 | P of the other rows packed, dS of rows 0..7
+    req_tr(FGRPO_IC(qt), tb);
     wait_lgkm<2 * DB>();
     fence();
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      attn_settle(l4[1][i]);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) l4[1][i][e] = __float_as_uint(__uint_as_float(l4[1][i][e]) * kLog2e);
-    }
-    quarter(ta, pp, H0{}, AV{}, [&](auto ec) { e_el(ec)(H1{}); });
-#pragma unroll
-    for (int kb = 0; kb < 2; ++kb) pp[kb][1] = pack(s[kb], 1);
-    req_tr(std::integral_constant<int, qt>{}, ta);
-    wait_lgkm<2 * DB>();
-    fence();
-    quarter(tb, pp, H1{}, AV{}, [&](auto ec) { f_el(ec, H0{}); });
+    quarter(ta, pp, H0{}, FGRPO_IC(kAccV), [&](auto mc) {
+      deal(FGRPO_IC(2), mc, FGRPO_IC(0), FGRPO_IC(2), [&](auto kbc) { pp[decltype(kbc)::value][1] = pack(s[decltype(kbc)::value], 1); });
+      deal(FGRPO_IC(16), mc, FGRPO_IC(1), FGRPO_IC(NQ), [&](auto ec) { f_el(ec, H0{}); });
+    });
 #pragma unroll
     for (int kb = 0; kb < 2; ++kb) ds[kb][0] = pack(dp[kb], 0);
-    req_tr(std::integral_constant<int, qt + 16 * RB>{}, tb);
+    // dK, rows 0..7 | dS of the other rows
+    req_tr(FGRPO_IC(qt + 16 * RB), ta);
     wait_lgkm<2 * DB>();
     fence();
-    quarter(ta, ds, H0{}, AK{}, [&](auto ec) { f_el(ec, H1{}); });
+    quarter(tb, ds, H0{}, FGRPO_IC(kAccK), [&](auto mc) {
+      deal(FGRPO_IC(16), mc, FGRPO_IC(0), FGRPO_IC(NQ), [&](auto ec) { f_el(ec, H1{}); });
+    });
 #pragma unroll
     for (int kb = 0; kb < 2; ++kb) ds[kb][1] = pack(dp[kb], 1);
-    FGRPO_WAIT_VMCNT(0);                                       // the next item is in its buffer
-    static_for<QG>([&](auto ic) { req_rows(std::integral_constant<int, nxt>{}, ic, qa[decltype(ic)::value]); });
-    wait_lgkm<QG>();
+    // dK, rows 8..15 | the Q rows and scalars of the item after next
+    const bool more2 = n + 8 < NI;
+    // destinations and row offsets are formed here: held across the loop they would fill the scalar registers
+    uint32_t bufs = base_w;
+    int sqv = sq, sdv = sd;
+    asm volatile("" : "+s"(bufs), "+s"(sqv), "+s"(sdv));
+    if (more2) fetch_advance();
+    fetch_setup(more2);
+    req_tr(FGRPO_IC(dot + 16 * RB), tb);
+    wait_lgkm<2 * DB>();                                       // everything of this item's Q rows and scalars has been read
     fence();
-    qb = qb_n;
-    if (n + 8 < NI) advance();                                 // else the walk stays on the last item there is
-    quarter(tb, ds, H1{}, AK{}, [](auto) {});
+    quarter(ta, ds, H1{}, FGRPO_IC(kAccK), [&](auto mc) {
+      deal(FGRPO_IC(NLD + 2), mc, FGRPO_IC(0), FGRPO_IC(NQ), [&](auto ic) { fetch_q(ic, bufs + qt, sqv); });
+    });
+    // dV, rows 8..15 | its dO rows; the first Q rows of the next item on their way
+    FGRPO_WAIT_VMCNT(kItemLoads);                              // the next item's Q rows: later loads are its dO rows and the Q rows just requested
+    static_for<QG>([&](auto ic) { req_q(FGRPO_IC(nxt), ic); });
+    wait_lgkm<QG>();                                           // everything of this item's dO rows has been read
+    fence();
+    g_c += 4;
+    while (g_c >= G) g_c -= G, qb -= kDkv3Rows;
+    quarter(tb, pp, H1{}, FGRPO_IC(kAccV), [&](auto mc) {
+      deal(FGRPO_IC(NLD), mc, FGRPO_IC(0), FGRPO_IC(NQ), [&](auto ic) { fetch_d(ic, bufs + qt, sdv); });
+    });
   };
   if (wave < NI) {
-    static_for<QG>([&](auto ic) { req_rows(std::integral_constant<int, 0>{}, ic, qa[decltype(ic)::value]); });
+    static_for<QG>([&](auto ic) { req_q(FGRPO_IC(0), ic); });
     for (int n = wave; n < NI; n += 8) {
-      item(std::integral_constant<int, 0>{}, n);
-      if (n + 4 < NI) item(std::integral_constant<int, 1>{}, n + 4);
+      item(FGRPO_IC(0), n);
+      if (n + 4 < NI) item(FGRPO_IC(1), n + 4);
     }
     wait_lgkm<0>();
 #pragma unroll
-    for (int i = 0; i < QG; ++i) attn_settle(qa[i]);
+    for (int i = 0; i < QG; ++i) attn_settle(qf[i]);
+    FGRPO_WAIT_VMCNT(0);                                       // the loads that brought nothing: the buffers are about to be reused
   }
+#undef FGRPO_IC
   asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");           // the last matrix instructions have written their accumulators
 
   // ---- the four sets of accumulators, added in wavefront order; 16-byte stores of eight columns
+  // (lane and thread index formed anew: held across the loop they would cost registers it does not have)
   constexpr int SS = kDkv3SumStride<HD>;
+  const int lane_e = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)), tid_e = wave * 64 + lane_e;
   auto sum_store = [&](auto accc, float mul, bf16_t* out) {
     constexpr int acc = decltype(accc)::value;
     wg_barrier();                                              // the tiles / the previous sums are no longer read
-    const uint32_t w0 = lds0 + wave * (kDkv3Keys * SS) + (4 * h) * SS + (lane & 31) * 4;
+    const uint32_t w0 = lds0 + wave * (kDkv3Keys * SS) + (4 * (lane_e >> 5)) * SS + (lane_e & 31) * 4;
     static_for<2>([&](auto kbc) {
       static_for<DB>([&](auto nbc) {
         static_for<16>([&](auto rc) {
           constexpr int kb = decltype(kbc)::value, nb = decltype(nbc)::value, r = decltype(rc)::value;
-          lds_write_u32_asm<(32 * kb + 8 * (r / 4) + r % 4) * SS + nb * 128>(w0, __float_as_uint(dkv3_acc_read<16 * (acc + kb * DB + nb) + r>()));
+          dkv3_acc_to_lds<16 * (acc + kb * DB + nb) + r, (32 * kb + 8 * (r / 4) + r % 4) * SS + nb * 128>(w0);
         });
       });
     });
@@ -439,23 +475,25 @@ __global__ __launch_bounds__(256, 1) void varlen_attn_dkv3_kernel(AttnParams p) 
     wg_barrier();
 #pragma unroll
     for (int i = 0; i < kDkv3Keys * HD / 8 / 256; ++i) {
-      const int piece = threadIdx.x + 256 * i, row = piece / (HD / 8), col = piece % (HD / 8);
+      const int piece = tid_e + 256 * i, row = piece / (HD / 8), col = piece % (HD / 8);
       const uint32_t a = lds0 + row * SS + col * 32;
-      float x[8];
+      u32x4_t part[4][2];
       static_for<4>([&](auto wc) {
         constexpr int w = decltype(wc)::value;
         const uint32_t aw = a + w * (kDkv3Keys * SS);
-        u32x4_t lo = lds_read_u128_asm<0>(aw), hi = lds_read_u128_asm<16>(aw);
-        wait_lgkm<0>();
-        fence();
-        attn_settle(lo);
-        attn_settle(hi);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          x[j] = (w == 0 ? 0.f : x[j]) + __uint_as_float(lo[j]);
-          x[4 + j] = (w == 0 ? 0.f : x[4 + j]) + __uint_as_float(hi[j]);
-        }
+        part[w][0] = lds_read_u128_asm<0>(aw);
+        part[w][1] = lds_read_u128_asm<16>(aw);
       });
+      wait_lgkm<0>();
+      fence();
+      float x[8];
+#pragma unroll
+      for (int w = 0; w < 4; ++w)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          if (j % 4 == 0) attn_settle(part[w][j / 4]);
+          x[j] = (w == 0 ? 0.f : x[j]) + __uint_as_float(part[w][j / 4][j % 4]);
+        }
 #pragma unroll
       for (int j = 0; j < 8; ++j) x[j] *= mul;
       const int kk = k0 + row;

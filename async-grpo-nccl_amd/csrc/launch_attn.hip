@@ -148,7 +148,9 @@ int fgrpo_varlen_attn_bwd(const void* dout, const void* q, const void* k, const 
   }
   rc = launch_query_side<DqLauncher>(D, attn_heads_per_group(Hq / Hkv, T, n_seq), p, T, Hq, Hkv, bounds_ws, st);
   if (rc) return rc;
-  if (g_tune.attn_dkv != 1 && g_tune.attn_dkv != 2) return launch_attn_dkv3(D, p, st);
+  // the scalar offsets of the third form are 32-bit: (queries x heads of a group) x 4 bytes and the two bounds arrays
+  const bool dkv3_fits = (long long)T * (Hq / Hkv) * 4 < (1LL << 31) && (long long)T * 8 < (1LL << 31);
+  if (g_tune.attn_dkv != 1 && g_tune.attn_dkv != 2 && dkv3_fits) return launch_attn_dkv3(D, p, st);
   const dim3 grid_k(Hkv, (T + kAttnBQ - 1) / kAttnBQ);
   if (g_tune.attn_dkv == 1) {
     if (D == 128) hipLaunchKernelGGL(varlen_attn_dkv_kernel<128>, grid_k, dim3(256), 0, st, p);
