@@ -1,5 +1,6 @@
 // dK / dV of the packed attention with one wavefront per SIMD and no barrier in its loop (head dimension HD = 128 or
-// 64).  A work-group owns 64 keys of one K/V head; its four wavefronts deal the work on those keys among themselves -
+// 64).  A work-group owns 64 keys of one K/V head (32 at HD = 64, where two
+// work-groups then share a CU); its four wavefronts deal the work on those keys among themselves -
 // item n = (32 queries, query head) goes to wavefront n % 4 - and each walks its items alone: it brings the item's
 // Q / dO rows into two LDS buffers of its own (global -> LDS, two items ahead), waits for nothing but its own loads,
 // and keeps both accumulators for all 64 keys (256 accumulation registers at HD = 128).  The four accumulator sets are
@@ -16,7 +17,7 @@
 //
 // Measured, dQ + dK/dV, paired kernel -> this one on one box: 4 segments of 8192 tokens, 28 / 4 heads of 128:
 // 7.20 -> 6.00 ms; 32768 tokens in segments of 128..1024, 12 / 2 heads of 128: 442 -> 393 us; 12345 such tokens, 14 / 2
-// heads of 64: 245 -> 109 us; 8773 tokens in segments of up to 8192, 14 / 2 heads of 64: 1222 -> 735 us.  It was faster
+// heads of 64: 245 -> 99 us; one segment of 8192 tokens, 14 / 2 heads of 64: 1222 -> 617 us.  It was faster
 // at every size tried, so no rule picks between the two.  Counters at the long shape: matrix pipe 0.61 busy at 1.81
 // GHz, the power limit; at the short ones the clock is 2.4 GHz and the pipe 0.38 busy: opening and closing a
 // work-group and the masked items weigh there.
@@ -40,15 +41,15 @@
 
 namespace fgrpo {
 
-constexpr int kDkv3Keys = 64, kDkv3Rows = 32;
+constexpr int kDkv3Rows = 32;                                          // queries of an item
 template <int HD>
 constexpr int kDkv3Buf = 2 * kDkv3Rows * HD * 2 + 512;                 // Q | dO | lse | -delta of 32 queries
 template <int HD>
 constexpr int kDkv3SumStride = HD * 4 + 32;                            // fp32 row of the closing sum: the two lane halves (rows 4 apart) hit different banks
-template <int HD>
-constexpr int kDkv3LoopLds = 4 * 2 * kDkv3Buf<HD> + kDkv3Keys * HD * 2;
-template <int HD>
-constexpr int kDkv3Lds = kDkv3LoopLds<HD> > 4 * kDkv3Keys * kDkv3SumStride<HD> ? kDkv3LoopLds<HD> : 4 * kDkv3Keys * kDkv3SumStride<HD>;
+template <int HD, int KB>
+constexpr int kDkv3LoopLds = 4 * 2 * kDkv3Buf<HD> + 32 * KB * HD * 2;
+template <int HD, int KB>
+constexpr int kDkv3Lds = kDkv3LoopLds<HD, KB> > 4 * 32 * KB * kDkv3SumStride<HD> ? kDkv3LoopLds<HD, KB> : 4 * 32 * KB * kDkv3SumStride<HD>;
 
 // The accumulators live in fixed accumulation registers, a[16 n : 16 n + 15] for block n, named in the instructions:
 // at HD = 128 they are all 256 of them, and a register allocator that may move or copy a block has nowhere to put it
@@ -56,11 +57,13 @@ constexpr int kDkv3Lds = kDkv3LoopLds<HD> > 4 * kDkv3Keys * kDkv3SumStride<HD> ?
 // compiler keeps nothing of its own there; the build checks that the kernel spills nothing.
 // The compiler's hazard table does not see these instructions: the first one behind vector arithmetic that formed an
 // operand carries two wait states, instructions on one block are at least four matrix instructions apart.
-#define FGRPO_DKV3_CLOBBER_128 \
+#define FGRPO_DKV3_CLOBBER_64 \
   "a0", "a1", "a2", "a3", "a4", "a5", "a6", "a7", "a8", "a9", "a10", "a11", "a12", "a13", "a14", "a15", \
   "a16", "a17", "a18", "a19", "a20", "a21", "a22", "a23", "a24", "a25", "a26", "a27", "a28", "a29", "a30", "a31", \
   "a32", "a33", "a34", "a35", "a36", "a37", "a38", "a39", "a40", "a41", "a42", "a43", "a44", "a45", "a46", "a47", \
-  "a48", "a49", "a50", "a51", "a52", "a53", "a54", "a55", "a56", "a57", "a58", "a59", "a60", "a61", "a62", "a63", \
+  "a48", "a49", "a50", "a51", "a52", "a53", "a54", "a55", "a56", "a57", "a58", "a59", "a60", "a61", "a62", "a63"
+#define FGRPO_DKV3_CLOBBER_128 \
+  FGRPO_DKV3_CLOBBER_64, \
   "a64", "a65", "a66", "a67", "a68", "a69", "a70", "a71", "a72", "a73", "a74", "a75", "a76", "a77", "a78", "a79", \
   "a80", "a81", "a82", "a83", "a84", "a85", "a86", "a87", "a88", "a89", "a90", "a91", "a92", "a93", "a94", "a95", \
   "a96", "a97", "a98", "a99", "a100", "a101", "a102", "a103", "a104", "a105", "a106", "a107", "a108", "a109", "a110", "a111", \
@@ -75,21 +78,24 @@ constexpr int kDkv3Lds = kDkv3LoopLds<HD> > 4 * kDkv3Keys * kDkv3SumStride<HD> ?
   "a208", "a209", "a210", "a211", "a212", "a213", "a214", "a215", "a216", "a217", "a218", "a219", "a220", "a221", "a222", "a223", \
   "a224", "a225", "a226", "a227", "a228", "a229", "a230", "a231", "a232", "a233", "a234", "a235", "a236", "a237", "a238", "a239", \
   "a240", "a241", "a242", "a243", "a244", "a245", "a246", "a247", "a248", "a249", "a250", "a251", "a252", "a253", "a254", "a255"
-template <int HD, int BLK, bool FIRST>
+// NACC accumulation registers in use; FIRST: behind vector arithmetic
+template <int NACC, int BLK, bool FIRST>
 __device__ __forceinline__ void dkv3_mfma(u32x4_t a, u32x4_t b) {
   constexpr int r0 = 16 * BLK, r1 = r0 + 15;
-  if constexpr (HD == 128) {
-    if constexpr (FIRST) asm volatile("s_nop 1\n\tv_mfma_f32_32x32x16_bf16 a[%2:%3], %0, %1, a[%2:%3]" : : "v"(a), "v"(b), "n"(r0), "n"(r1) : FGRPO_DKV3_CLOBBER_256);
-    else asm volatile("v_mfma_f32_32x32x16_bf16 a[%2:%3], %0, %1, a[%2:%3]" : : "v"(a), "v"(b), "n"(r0), "n"(r1) : FGRPO_DKV3_CLOBBER_256);
-  } else {
-    if constexpr (FIRST) asm volatile("s_nop 1\n\tv_mfma_f32_32x32x16_bf16 a[%2:%3], %0, %1, a[%2:%3]" : : "v"(a), "v"(b), "n"(r0), "n"(r1) : FGRPO_DKV3_CLOBBER_128);
-    else asm volatile("v_mfma_f32_32x32x16_bf16 a[%2:%3], %0, %1, a[%2:%3]" : : "v"(a), "v"(b), "n"(r0), "n"(r1) : FGRPO_DKV3_CLOBBER_128);
-  }
+  static_assert(r1 < NACC && (NACC == 64 || NACC == 128 || NACC == 256), "accumulator block");
+#define FGRPO_DKV3_MFMA(clobber)                                                                                            \
+  if constexpr (FIRST) asm volatile("s_nop 1\n\tv_mfma_f32_32x32x16_bf16 a[%2:%3], %0, %1, a[%2:%3]" : : "v"(a), "v"(b), "n"(r0), "n"(r1) : clobber); \
+  else asm volatile("v_mfma_f32_32x32x16_bf16 a[%2:%3], %0, %1, a[%2:%3]" : : "v"(a), "v"(b), "n"(r0), "n"(r1) : clobber)
+  if constexpr (NACC == 256) { FGRPO_DKV3_MFMA(FGRPO_DKV3_CLOBBER_256); }
+  else if constexpr (NACC == 128) { FGRPO_DKV3_MFMA(FGRPO_DKV3_CLOBBER_128); }
+  else { FGRPO_DKV3_MFMA(FGRPO_DKV3_CLOBBER_64); }
+#undef FGRPO_DKV3_MFMA
 }
-template <int HD, int REG>
+template <int NACC, int REG>
 __device__ __forceinline__ void dkv3_acc_clear() {
-  if constexpr (HD == 128) asm volatile("v_accvgpr_write_b32 a[%0], 0" : : "n"(REG) : FGRPO_DKV3_CLOBBER_256);
-  else asm volatile("v_accvgpr_write_b32 a[%0], 0" : : "n"(REG) : FGRPO_DKV3_CLOBBER_128);
+  if constexpr (NACC == 256) asm volatile("v_accvgpr_write_b32 a[%0], 0" : : "n"(REG) : FGRPO_DKV3_CLOBBER_256);
+  else if constexpr (NACC == 128) asm volatile("v_accvgpr_write_b32 a[%0], 0" : : "n"(REG) : FGRPO_DKV3_CLOBBER_128);
+  else asm volatile("v_accvgpr_write_b32 a[%0], 0" : : "n"(REG) : FGRPO_DKV3_CLOBBER_64);
 }
 template <int REG, int OFF>
 __device__ __forceinline__ void dkv3_acc_to_lds(uint32_t addr) {       // LDS instructions take their data from these registers directly
@@ -97,8 +103,10 @@ __device__ __forceinline__ void dkv3_acc_to_lds(uint32_t addr) {       // LDS in
   asm volatile("ds_write_b32 %0, a[%1] offset:%2" : : "v"(addr), "n"(REG), "n"(OFF) : "memory");
 }
 
-template <int HD>
-__global__ __launch_bounds__(256, 1) void varlen_attn_dkv3_kernel(AttnParams p) {
+// KB key blocks of 32 (2: one wavefront per SIMD; 1, head dimension 64: two)
+template <int HD, int KB>
+__global__ __launch_bounds__(256, KB == 2 ? 1 : 2) void varlen_attn_dkv3_kernel(AttnParams p) {
+  constexpr int kKeys = 32 * KB;
   constexpr int KS = HD / 16, DB = HD / 32, RB = HD * 2, kT = kDkv3Rows * RB, kBuf = kDkv3Buf<HD>;
   constexpr int QG = KS / 2, NG = KS / 2;              // row fragments of a half of S; groups of two k steps of dP
   constexpr int kSc = 2 * kT;                          // per-query scalars inside a buffer
@@ -108,15 +116,16 @@ __global__ __launch_bounds__(256, 1) void varlen_attn_dkv3_kernel(AttnParams p) 
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int G = p.Hq / p.Hkv;
   const int hkv = blockIdx.x % p.Hkv, rank = blockIdx.x / p.Hkv;
-  const int ntile = (p.T + kDkv3Keys - 1) / kDkv3Keys, n128 = (p.T + 127) / 128;
-  const int tile = min(max(p.order_k[rank >> 1], 0), n128 - 1) * 2 + (rank & 1);      // clamped: the list may come from the caller
+  constexpr int kPer128 = 128 / kKeys;
+  const int ntile = (p.T + kKeys - 1) / kKeys, n128 = (p.T + 127) / 128;
+  const int tile = min(max(p.order_k[rank / kPer128], 0), n128 - 1) * kPer128 + rank % kPer128;      // clamped: the list may come from the caller
   if (tile >= ntile) return;
-  const int k0 = tile * kDkv3Keys, klast = min(k0 + kDkv3Keys, p.T) - 1;
+  const int k0 = tile * kKeys, klast = min(k0 + kKeys, p.T) - 1;
   const int q_begin = max(__builtin_amdgcn_readfirstlane(p.causal ? k0 : p.seg_start[k0]), 0);      // inside [0, T]
   const int q_end = min(__builtin_amdgcn_readfirstlane(p.seg_end[klast]), p.T);
   // one segment holds every key of the tile: queries from `q_full` on that are complete blocks see all of it
   const bool one_segment = __builtin_amdgcn_readfirstlane(p.seg_start[k0]) == __builtin_amdgcn_readfirstlane(p.seg_start[klast]);
-  const int q_full = !one_segment ? 0x7fffffff : p.causal ? k0 + kDkv3Keys - 1 : q_begin;
+  const int q_full = !one_segment ? 0x7fffffff : p.causal ? k0 + kKeys - 1 : q_begin;
   const int nqb = q_end > q_begin ? (q_end - q_begin + kDkv3Rows - 1) / kDkv3Rows : 0;
   const int NI = nqb * G;
 
@@ -135,37 +144,10 @@ __global__ __launch_bounds__(256, 1) void varlen_attn_dkv3_kernel(AttnParams p) 
   }
   const uint32_t scl = base_w + kSc + h * 16;                  // + array * 128 + row group * 32
 
-  // V tile -> LDS by the whole work-group; rows past the end of the keys read as zero
-  {
-    const uint32_t fvo = attn_dma_lane_offset<HD>(wave, lane, p.v_st);
-    attn_dma_tile<HD>(p.v + (long long)hkv * p.v_sh, p.v_st, k0, klast + 1, fvo, smem + 4 * 2 * kBuf + wave * 1024);
-  }
-  // K rows of the two key blocks as operands
-  u32x4_t kf[2][KS];
-#pragma unroll
-  for (int kb = 0; kb < 2; ++kb) {
-    bf16x8_t f[KS];
-    const int key = k0 + 32 * kb + (lane & 31);
-    attn_row_operand(f, p.k + (long long)min(key, p.T - 1) * p.k_st + (long long)hkv * p.k_sh, key < p.T, h);
-#pragma unroll
-    for (int st = 0; st < KS; ++st) kf[kb][st] = __builtin_bit_cast(u32x4_t, f[st]);
-  }
-  // the queries that see the lane's key: key_n of them, from the key itself (causal) or its segment's start on; kept
-  // relative to the lane's first row of a query block
-  int key_lo[2];
-  uint32_t key_n[2];
-#pragma unroll
-  for (int kb = 0; kb < 2; ++kb) {
-    const int key = min(k0 + 32 * kb + (lane & 31), p.T - 1), lo = p.causal ? key : p.seg_start[key];
-    key_lo[kb] = lo - 4 * h;
-    key_n[kb] = k0 + 32 * kb + (lane & 31) < p.T ? (uint32_t)max(min(p.seg_end[key], q_end) - lo, 0) : 0u;
-    asm volatile("" : "+v"(key_lo[kb]), "+v"(key_n[kb]));
-  }
   const float c = p.scale * kLog2e;
 
   // accumulator blocks: dV[kb][nb] = kb DB + nb, dK behind them
-  constexpr int kAccV = 0, kAccK = 2 * DB;
-  static_for<4 * DB * 16>([&](auto rc) { dkv3_acc_clear<HD, decltype(rc)::value>(); });
+  constexpr int kAccV = 0, kAccK = KB * DB, NACC = 2 * KB * DB * 16;
 
   // ---- loads of an item.  Instruction i of a tile fills its KiB i: RPI rows; lane l lands at 16 l of it, i.e. row
   // i RPI + l / (HD/8), chunk slot l % (HD/8), and fetches the chunk the swizzle puts there (four or two patterns).
@@ -222,26 +204,56 @@ __global__ __launch_bounds__(256, 1) void varlen_attn_dkv3_kernel(AttnParams p) 
     __builtin_amdgcn_raw_ptr_buffer_load_lds(rsd, FGRPO_LDS_AT(buf + kT + i * 1024), 16, (int)fod[i % NPAT], i * step, 0, 0);
   };
   auto fence = []() { __builtin_amdgcn_sched_barrier(0); };
-#pragma unroll
-  for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-    for (int st = 0; st < KS; ++st) asm volatile("" : "+v"(kf[kb][st]));      // complete before the loop
 
+  // What a work-group needs before it can start, one round trip behind the other only where an address depends on it:
+  // V tile and first item, then the K rows and the key ranges, then the second item (not waited for here)
+  {
+    const int row = wave * RPI + lane / (HD / 8), ch = (lane % (HD / 8)) ^ attn_swz<HD>(row);      // 4 RPI rows a step: the same swizzle
+    const uint32_t fvo = (uint32_t)((row * p.v_st + ch * 8) * 2);
+    const __amdgpu_buffer_rsrc_t rsv = make_rsrc(p.v + (long long)hkv * p.v_sh + (long long)k0 * p.v_st, (uint32_t)min((klast - k0) * p.v_st * 2 + RB, 0xffffffffLL));
+#pragma unroll
+    for (int i = 0; i < kKeys / RPI / 4; ++i)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rsv, FGRPO_LDS_AT(lds0 + 4 * 2 * kBuf + wave * 1024 + i * 4096), 16, (int)fvo, (int)(i * 4 * RPI * p.v_st * 2), 0, 0);
+  }
   int g_c = g_f, qb = qb_f;                                    // the item being computed
   constexpr int kItemLoads = 2 * NLD + 2;
-  if (wave < NI) {
-    static_for<2>([&](auto bc) {
-      constexpr int b = decltype(bc)::value;
-      const bool more = wave + 4 * b < NI;
-      if (b == 1 && more) fetch_advance();
-      fetch_setup(more);
-      static_for<NLD + 2>([&](auto ic) { fetch_q(ic, base_w + b * kBuf, sq); });
-      static_for<NLD>([&](auto ic) { fetch_d(ic, base_w + b * kBuf, sd); });
-    });
-    FGRPO_WAIT_VMCNT(kItemLoads);                              // the V rows (requested first) and the first item
-  } else {
-    FGRPO_WAIT_VMCNT(0);
+  auto fetch_item = [&](auto bc) {
+    constexpr int b = decltype(bc)::value;
+    const bool more = wave + 4 * b < NI;
+    if (b == 1 && more) fetch_advance();
+    fetch_setup(more);
+    static_for<NLD + 2>([&](auto ic) { fetch_q(ic, base_w + b * kBuf, sq); });
+    static_for<NLD>([&](auto ic) { fetch_d(ic, base_w + b * kBuf, sd); });
+  };
+  if (wave < NI) fetch_item(std::integral_constant<int, 0>{});
+  // K rows of the key blocks as operands
+  u32x4_t kf[KB][KS];
+  // the queries that see the lane's key: key_n of them, from the key itself (causal) or its segment's start on; kept
+  // relative to the lane's first row of a query block
+  int key_lo[KB];
+  uint32_t key_n[KB];
+#pragma unroll
+  for (int kb = 0; kb < KB; ++kb) {
+    bf16x8_t f[KS];
+    const int key = k0 + 32 * kb + (lane & 31), kc = min(key, p.T - 1);
+    attn_row_operand(f, p.k + (long long)kc * p.k_st + (long long)hkv * p.k_sh, key < p.T, h);
+#pragma unroll
+    for (int st = 0; st < KS; ++st) kf[kb][st] = __builtin_bit_cast(u32x4_t, f[st]);
+    const int lo = p.causal ? kc : p.seg_start[kc];
+    key_lo[kb] = lo - 4 * h;
+    key_n[kb] = key < p.T ? (uint32_t)max(min(p.seg_end[kc], q_end) - lo, 0) : 0u;
   }
+  fence();
+  if (wave < NI) fetch_item(std::integral_constant<int, 1>{});
+  static_for<NACC>([&](auto rc) { dkv3_acc_clear<NACC, decltype(rc)::value>(); });      // under the loads
+#pragma unroll
+  for (int kb = 0; kb < KB; ++kb) {
+#pragma unroll
+    for (int st = 0; st < KS; ++st) asm volatile("" : "+v"(kf[kb][st]));                // complete before the loop
+    asm volatile("" : "+v"(key_lo[kb]), "+v"(key_n[kb]));
+  }
+  if (wave < NI) FGRPO_WAIT_VMCNT(kItemLoads);                 // everything but the second item
+  else FGRPO_WAIT_VMCNT(0);
   wg_barrier();                                                // the whole V tile is there
 
   u32x4_t qf[KS];                                              // Q rows of the item; the first half is requested by the item before
@@ -249,10 +261,10 @@ __global__ __launch_bounds__(256, 1) void varlen_attn_dkv3_kernel(AttnParams p) 
   auto item = [&](auto curc, int n) {
     constexpr int cur = decltype(curc)::value, qt = cur * kBuf, dot = qt + kT, sct = cur * kBuf, nxt = (cur ^ 1) * kBuf;
     const bool masked = qb < q_full || qb + kDkv3Rows > q_end;
-    u32x4_t fo[2][2], fv[2][2][2], nd[4], l4[4];
+    u32x4_t fo[2][2], fv[2][2][KB], nd[4], l4[4];
     AttnTr ta[DB], tb[DB];
-    f32x16_t s[2], dp[2];
-    u32x4_t pp[2][2], ds[2][2];                                // P, dS as operands: [key block][rows 8 s2 ..]
+    f32x16_t s[KB], dp[KB];
+    u32x4_t pp[KB][2], ds[KB][2];                               // P, dS as operands: [key block][rows 8 s2 ..]
     auto req_dp = [&](auto gc) {                               // dP group: k steps 2 g, 2 g + 1: dO rows, V rows of both key blocks
       constexpr int g = decltype(gc)::value;
       static_for<2>([&](auto ic) {
@@ -260,7 +272,7 @@ __global__ __launch_bounds__(256, 1) void varlen_attn_dkv3_kernel(AttnParams p) 
         fo[g % 2][i] = lds_read_u128_asm<dot>(rowc[st]);
         const uint32_t va = rowc[st] + v_delta;
         fv[g % 2][i][0] = lds_read_u128_asm<0>(va);
-        fv[g % 2][i][1] = lds_read_u128_asm<32 * RB>(va);
+        if constexpr (KB == 2) fv[g % 2][i][KB - 1] = lds_read_u128_asm<32 * RB>(va);
       });
     };
     auto req_tr = [&](auto offc, AttnTr (&t)[DB]) {
@@ -274,8 +286,8 @@ __global__ __launch_bounds__(256, 1) void varlen_attn_dkv3_kernel(AttnParams p) 
       s[kb][r] = fast_exp2(__builtin_fmaf(s[kb][r], c, -__uint_as_float(l4[r / 4][r % 4])));
       asm volatile("" : "+v"(s[kb][r]));
     };
-    auto f_el = [&](auto ec, auto halfc) {                     // dS in place of dP: element e of a half is key block e % 2, row 8 half + e / 2
-      constexpr int e = decltype(ec)::value, half = decltype(halfc)::value, kb = e % 2, r = 8 * half + e / 2;
+    auto f_el = [&](auto ec, auto halfc) {                     // dS in place of dP: element e of a half is key block e % KB, row 8 half + e / KB
+      constexpr int e = decltype(ec)::value, half = decltype(halfc)::value, kb = e % KB, r = 8 * half + e / KB;
       dp[kb][r] = s[kb][r] * dp[kb][r];
       asm volatile("" : "+v"(dp[kb][r]));
     };
@@ -334,32 +346,38 @@ __global__ __launch_bounds__(256, 1) void varlen_attn_dkv3_kernel(AttnParams p) 
       fence();
     });
     if (masked) hide(H0{});
-    // ---- S of key block 1 | P of key block 0
-    static_for<4>([&](auto gc) { nd[decltype(gc)::value] = lds_read_u128_asm<sct + 256 + 32 * decltype(gc)::value>(scl); });
-    static_for<KS>([&](auto ic) {
-      constexpr int i = decltype(ic)::value;
-      s_mma(H1{}, ic);
-      deal(FGRPO_IC(16), ic, FGRPO_IC(1), FGRPO_IC(KS), [&](auto rc) { e_el(H0{}, rc); });
+    constexpr int GD = 2 + 2 * KB;                             // LDS reads of a dP group
+    auto open_dp = [&]() {                                     // -delta and the first group on their way
+      static_for<4>([&](auto gc) { nd[decltype(gc)::value] = lds_read_u128_asm<sct + 256 + 32 * decltype(gc)::value>(scl); });
+      FGRPO_WAIT_VMCNT(kItemLoads);                            // this item's dO rows: later loads are the next item's
+      req_dp(H0{});
       fence();
-      if constexpr (i == KS / 2 - 1) {
-        FGRPO_WAIT_VMCNT(kItemLoads);                          // this item's dO rows: later loads are the next item's
-        req_dp(H0{});
+    };
+    // ---- S of key block 1 | P of key block 0
+    if constexpr (KB == 2) {
+      static_for<KS>([&](auto ic) {
+        constexpr int i = decltype(ic)::value;
+        s_mma(FGRPO_IC(KB - 1), ic);
+        deal(FGRPO_IC(16), ic, FGRPO_IC(1), FGRPO_IC(KS), [&](auto rc) { e_el(H0{}, rc); });
         fence();
-      }
-    });
-    if (masked) hide(H1{});
-    // ---- dP, starting from -delta | P of key block 1
+        if constexpr (i == KS / 2 - 1) open_dp();
+      });
+      if (masked) hide(FGRPO_IC(KB - 1));
+    } else {
+      open_dp();
+    }
+    // ---- dP, starting from -delta | P of the last key block
     static_for<NG>([&](auto gc) {
       constexpr int g = decltype(gc)::value;
       if constexpr (g + 1 < NG) req_dp(FGRPO_IC(g + 1));
       else req_tr(FGRPO_IC(dot), ta);
-      wait_lgkm<(g + 1 < NG ? 6 : 2 * DB)>();
+      wait_lgkm<(g + 1 < NG ? GD : 2 * DB)>();
       fence();
       static_for<2>([&](auto ic) {
         constexpr int i = decltype(ic)::value, st = 2 * g + i;
         attn_settle(fo[g % 2][i]);
-        static_for<2>([&](auto kbc) {
-          constexpr int kb = decltype(kbc)::value, m = 4 * g + 2 * i + kb;
+        static_for<KB>([&](auto kbc) {
+          constexpr int kb = decltype(kbc)::value, m = KB * (2 * g + i) + kb;
           attn_settle(fv[g % 2][i][kb]);
           if constexpr (st == 0) {
             f32x16_t ndelta;
@@ -374,25 +392,25 @@ __global__ __launch_bounds__(256, 1) void varlen_attn_dkv3_kernel(AttnParams p) 
             dp[kb] = attn_mfma(fo[g % 2][i], fv[g % 2][i][kb], dp[kb]);
           }
           fence();
-          deal(FGRPO_IC(16), FGRPO_IC(m), FGRPO_IC(1), FGRPO_IC(2 * KS), [&](auto rc) { e_el(H1{}, rc); });
+          deal(FGRPO_IC(16), FGRPO_IC(m), FGRPO_IC(1), FGRPO_IC(KB * KS), [&](auto rc) { e_el(FGRPO_IC(KB - 1), rc); });
           fence();
         });
       });
     });
 #pragma unroll
-    for (int kb = 0; kb < 2; ++kb) pp[kb][0] = pack(s[kb], 0);
+    for (int kb = 0; kb < KB; ++kb) pp[kb][0] = pack(s[kb], 0);
     // ---- dV and dK in quarters of NQ instructions
-    constexpr int NQ = 2 * DB;
-    auto quarter = [&](AttnTr (&t)[DB], u32x4_t (&op)[2][2], auto s2c, auto accc, auto&& side) {
+    constexpr int NQ = KB * DB, EH = 8 * KB;                   // EH: elements of half the rows
+    auto quarter = [&](AttnTr (&t)[DB], u32x4_t (&op)[KB][2], auto s2c, auto accc, auto&& side) {
       constexpr int s2 = decltype(s2c)::value, acc = decltype(accc)::value;
       static_for<DB>([&](auto dc) {
         constexpr int db = decltype(dc)::value;
         const u32x4_t b = attn_settle_tr(t[db]);
-        static_for<2>([&](auto kbc) {
+        static_for<KB>([&](auto kbc) {
           constexpr int kb = decltype(kbc)::value;
-          dkv3_mfma<HD, acc + kb * DB + db, db == 0>(op[kb][s2], b);
+          dkv3_mfma<NACC, acc + kb * DB + db, db == 0>(op[kb][s2], b);
           fence();
-          side(FGRPO_IC(2 * db + kb));
+          side(FGRPO_IC(KB * db + kb));
           fence();
         });
       });
@@ -402,20 +420,20 @@ __global__ __launch_bounds__(256, 1) void varlen_attn_dkv3_kernel(AttnParams p) 
     wait_lgkm<2 * DB>();
     fence();
     quarter(ta, pp, H0{}, FGRPO_IC(kAccV), [&](auto mc) {
-      deal(FGRPO_IC(2), mc, FGRPO_IC(0), FGRPO_IC(2), [&](auto kbc) { pp[decltype(kbc)::value][1] = pack(s[decltype(kbc)::value], 1); });
-      deal(FGRPO_IC(16), mc, FGRPO_IC(1), FGRPO_IC(NQ), [&](auto ec) { f_el(ec, H0{}); });
+      deal(FGRPO_IC(KB), mc, FGRPO_IC(0), FGRPO_IC(KB), [&](auto kbc) { pp[decltype(kbc)::value][1] = pack(s[decltype(kbc)::value], 1); });
+      deal(FGRPO_IC(EH), mc, FGRPO_IC(1), FGRPO_IC(NQ), [&](auto ec) { f_el(ec, H0{}); });
     });
 #pragma unroll
-    for (int kb = 0; kb < 2; ++kb) ds[kb][0] = pack(dp[kb], 0);
+    for (int kb = 0; kb < KB; ++kb) ds[kb][0] = pack(dp[kb], 0);
     // dK, rows 0..7 | dS of the other rows
     req_tr(FGRPO_IC(qt + 16 * RB), ta);
     wait_lgkm<2 * DB>();
     fence();
     quarter(tb, ds, H0{}, FGRPO_IC(kAccK), [&](auto mc) {
-      deal(FGRPO_IC(16), mc, FGRPO_IC(0), FGRPO_IC(NQ), [&](auto ec) { f_el(ec, H1{}); });
+      deal(FGRPO_IC(EH), mc, FGRPO_IC(0), FGRPO_IC(NQ), [&](auto ec) { f_el(ec, H1{}); });
     });
 #pragma unroll
-    for (int kb = 0; kb < 2; ++kb) ds[kb][1] = pack(dp[kb], 1);
+    for (int kb = 0; kb < KB; ++kb) ds[kb][1] = pack(dp[kb], 1);
     // dK, rows 8..15 | the Q rows and scalars of the item after next
     const bool more2 = n + 8 < NI;
     // destinations and row offsets are formed here: held across the loop they would fill the scalar registers
@@ -462,8 +480,8 @@ __global__ __launch_bounds__(256, 1) void varlen_attn_dkv3_kernel(AttnParams p) 
   auto sum_store = [&](auto accc, float mul, bf16_t* out) {
     constexpr int acc = decltype(accc)::value;
     wg_barrier();                                              // the tiles / the previous sums are no longer read
-    const uint32_t w0 = lds0 + wave * (kDkv3Keys * SS) + (4 * (lane_e >> 5)) * SS + (lane_e & 31) * 4;
-    static_for<2>([&](auto kbc) {
+    const uint32_t w0 = lds0 + wave * (kKeys * SS) + (4 * (lane_e >> 5)) * SS + (lane_e & 31) * 4;
+    static_for<KB>([&](auto kbc) {
       static_for<DB>([&](auto nbc) {
         static_for<16>([&](auto rc) {
           constexpr int kb = decltype(kbc)::value, nb = decltype(nbc)::value, r = decltype(rc)::value;
@@ -474,13 +492,13 @@ __global__ __launch_bounds__(256, 1) void varlen_attn_dkv3_kernel(AttnParams p) 
     wait_lgkm<0>();
     wg_barrier();
 #pragma unroll
-    for (int i = 0; i < kDkv3Keys * HD / 8 / 256; ++i) {
+    for (int i = 0; i < kKeys * HD / 8 / 256; ++i) {
       const int piece = tid_e + 256 * i, row = piece / (HD / 8), col = piece % (HD / 8);
       const uint32_t a = lds0 + row * SS + col * 32;
       u32x4_t part[4][2];
       static_for<4>([&](auto wc) {
         constexpr int w = decltype(wc)::value;
-        const uint32_t aw = a + w * (kDkv3Keys * SS);
+        const uint32_t aw = a + w * (kKeys * SS);
         part[w][0] = lds_read_u128_asm<0>(aw);
         part[w][1] = lds_read_u128_asm<16>(aw);
       });

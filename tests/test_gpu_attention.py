@@ -481,7 +481,7 @@ def test_both_query_side_kernels_give_identical_results(dev):
     (130, [0, 64, 128, 130], 14, 2, True, 64), (197, [0, 97, 129, 197], 6, 2, True, 128), (450, [0, 450], 1, 1, False, 64),
 ])
 def test_key_side_kernel_at_the_edges_of_its_tiles(dev, T, cu, Hq, Hkv, causal, D):
-    """Four wavefronts share 64 keys and deal (32 queries, head) items among themselves: fewer items than wavefronts,
+    """Four wavefronts share 64 keys (32 at head dimension 64) and deal (32 queries, head) items among themselves: fewer items than wavefronts,
     item counts off a multiple of four, last key and query blocks of every fill, segments that end on and beside a
     tile edge.  Against the fp32 oracle; twice, bit for bit."""
     from fgrpo import ops
