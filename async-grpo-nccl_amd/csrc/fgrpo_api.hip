@@ -617,7 +617,7 @@ int logprob_fwd_impl(const void* hidden, const void* weight, const void* bias, c
     if (rc2) return rc2;
     CombineParams c{part, pl.xt + t0, (const long long*)labels + t0, count, V, nsplit, lp_out + t0,
                     ent_out ? ent_out + t0 : nullptr, lse_out ? lse_out + t0 : nullptr};
-    hipLaunchKernelGGL(lmhead_fwd_combine_kernel, dim3((count + 255) / 256), dim3(256), 0, st, c);
+    launch_fwd_combine(c, st);
     HIP_TRY(hipGetLastError());
     return 0;
   };

@@ -1,0 +1,67 @@
+"""GPU tests of what small and prompt-heavy batches take: the merge of finely split vocabularies, evaluation without
+a gradient, and the log-probability worker's skipping of masked positions."""
+import pytest
+import torch
+
+from test_gpu_dropin import TinyLM, make_samples
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("T,V,H", [(1, 131, 64), (15, 4099, 64), (17, 40000, 128), (300, 40000, 64), (513, 70001, 64)])
+def test_vocabulary_splits_are_merged_at_every_count(dev, T, V, H):
+    """From one split to many more than a token has threads; against the soft-max in fp32 on the same bf16 operands.
+    Tolerance: fp32 sums over V terms in another order, a few ulp of values below 16."""
+    from fgrpo import ops
+    g = torch.Generator().manual_seed(T)
+    h = torch.randn(T, H, generator=g).bfloat16().to(dev)
+    w = (torch.randn(V, H, generator=g) * 0.1).bfloat16().to(dev)
+    y = torch.randint(0, V, (T,), generator=g).to(dev)
+    lp, ent, lse = ops.lmhead_logprob_fwd(h, w, None, y)
+    x = h.float() @ w.float().t()
+    want = torch.logsumexp(x, 1)
+    p = torch.softmax(x, 1)
+    assert (lse - want).abs().max() <= 2e-5
+    assert (lp - (x.gather(1, y[:, None])[:, 0] - want)).abs().max() <= 4e-5
+    assert (ent - (want - (p * x).sum(1))).abs().max() <= 4e-5
+
+
+def test_evaluation_of_a_trainable_head_prepares_no_backward(dev):
+    """Under no_grad the results are those of the differentiable call and carry no graph."""
+    from fgrpo import ops
+    g = torch.Generator().manual_seed(0)
+    h = torch.randn(700, 1024, generator=g).bfloat16().to(dev).requires_grad_(True)
+    w = (torch.randn(9000, 1024, generator=g) * 0.02).bfloat16().to(dev).requires_grad_(True)
+    y = torch.randint(0, 9000, (700,), generator=g).to(dev)
+    old, adv = torch.randn(700, generator=g).to(dev) - 9, torch.randn(700, generator=g).to(dev)
+    lp, ent = ops.lmhead_logprob(h, w, None, y)
+    step = ops.fused_grpo_loss(h, w, None, y, old, adv)
+    with torch.no_grad():
+        lp0, ent0 = ops.lmhead_logprob(h, w, None, y)
+        step0 = ops.fused_grpo_loss(h, w, None, y, old, adv)
+    assert lp.requires_grad and step[0].requires_grad and not lp0.requires_grad and not step0[0].requires_grad
+    assert torch.equal(lp.detach(), lp0) and torch.equal(ent, ent0)
+    for a, b in zip(step, step0):
+        assert torch.allclose(a.detach(), b, rtol=1e-5, atol=1e-6)      # the chunked step may split the vocabulary otherwise
+
+
+def test_logprob_worker_skips_prompts_and_returns_the_same(dev):
+    """A prompt-heavy batch above the size from which masked rows are left out: the same values where a label is
+    scored, zeros elsewhere."""
+    from fgrpo import ops
+    from grpo_loss import make_grpo_forward
+    from workers import LogProbHarness
+    torch.manual_seed(0)
+    model = TinyLM(tied=False).to(dev).bfloat16()
+    make_grpo_forward(model, mode="eval")
+    harness = LogProbHarness(model, dev)
+    samples = make_samples(n=130)
+    assert sum(len(s["sample_ids"]) for s in samples) >= ops.COMPACT_MIN_TOKENS
+    got = harness.compute_log_probs_from_samples(samples, packed=True).buffer.clone()
+    keep, ops.COMPACT_MIN_TOKENS = ops.COMPACT_MIN_TOKENS, 1 << 30
+    try:
+        want = harness.compute_log_probs_from_samples(samples, packed=True).buffer
+    finally:
+        ops.COMPACT_MIN_TOKENS = keep
+    assert torch.equal(got == 0, want == 0)
+    assert (got - want).abs().max() <= 2e-5
