@@ -616,7 +616,15 @@ def _want_keep(T: int, H: int, V: int, dtype, needs_grad: bool, keep_logits=None
     return ok and mode == "auto" and logits_keep_bytes(T, V) <= KEEP_WHOLE_MAX_BYTES
 
 
-def _logprob_fwd_rows(hidden, weight, bias, labels_shifted, temperature, idx, needs_grad=False, keep_logits=None):
+def _wants_grad(*tensors) -> bool:
+    """Whether a backward can reach any of these.  Asked outside the autograd functions: inside one, the gradient mode
+    is always off and ``needs_input_grad`` repeats ``requires_grad`` even under ``torch.no_grad()`` - an evaluation of
+    a trainable head would then prepare a backward that never comes (the kept forward writes [T, V] in bf16)."""
+    return torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in tensors)
+
+
+def _logprob_fwd_rows(hidden, weight, bias, labels_shifted, temperature, idx, needs_grad=False, keep_logits=None,
+                      want_lse=True):
     """Forward on the rows ``idx`` (or on all rows when idx is None); outputs scattered back into [T] vectors.
     Returns (lp, ent, lse, hidden used, labels used, kept logits | None)."""
     if idx is not None:
@@ -625,7 +633,7 @@ def _logprob_fwd_rows(hidden, weight, bias, labels_shifted, temperature, idx, ne
     else:
         y = labels_shifted
     keep = _want_keep(hidden.shape[0], hidden.shape[1], weight.shape[0], weight.dtype, needs_grad, keep_logits)
-    res = lmhead_logprob_fwd(hidden, weight, bias, y, temperature, keep=keep)
+    res = lmhead_logprob_fwd(hidden, weight, bias, y, temperature, want_lse=want_lse, keep=keep)
     lp, ent, lse = res[:3]
     kept = res[3] if keep else None
     if idx is not None:
@@ -768,10 +776,13 @@ class _LMHeadLogprob(torch.autograd.Function):
         ctx.temperature = temperature
         ctx.panel_hint = panel_hint
         ctx.mark_non_differentiable(ent)
+        ctx.set_materialize_grads(False)
         return lp, ent
 
     @staticmethod
     def backward(ctx, g_lp, _g_ent):
+        if g_lp is None:
+            return (None,) * 8
         h_used, weight, bias, y_used, lse, idx = ctx.saved_tensors
         bias = bias if ctx.has_bias else None
         need = (ctx.needs_input_grad[0], ctx.needs_input_grad[1], ctx.has_bias and ctx.needs_input_grad[2])
@@ -843,10 +854,13 @@ class _FusedGRPOLoss(torch.autograd.Function):
         ctx.save_for_backward(h_used, weight, bias if bias is not None else hidden.new_empty(0), y_used, lse, g,
                               idx if idx is not None else hidden.new_empty(0))
         ctx.mark_non_differentiable(ent, lr, c1, l1, l2, lp)
+        ctx.set_materialize_grads(False)      # else autograd fills a zero tensor for each of the six others
         return loss, ent, lr, c1, l1, l2, lp
 
     @staticmethod
     def backward(ctx, g_loss, *_unused):
+        if g_loss is None:
+            return (None,) * 19
         grads, ctx.grads = ctx.grads, None
         if grads is not None:
             # the chunked step left the gradients of the loss itself: multiply by the upstream scalar (on the device;
@@ -877,10 +891,13 @@ class _GRPOLossFromLogprobs(torch.autograd.Function):
         ctx.save_for_backward(g)
         ctx.lp_dtype = lp.dtype
         ctx.mark_non_differentiable(lr, c1, l1, l2)
+        ctx.set_materialize_grads(False)
         return loss, lr, c1, l1, l2
 
     @staticmethod
     def backward(ctx, g_loss, *_unused):
+        if g_loss is None:
+            return (None,) * 12
         (g,) = ctx.saved_tensors
         return ((g * g_loss).to(ctx.lp_dtype),) + (None,) * 11
 
@@ -896,7 +913,13 @@ def grpo_loss_from_logprobs(lp, labels_shifted, old_lp, adv, ref_lp=None, cu_seq
 
 def lmhead_logprob(hidden, weight, bias, labels_shifted, temperature=1.0, panel_hint=0,
                    compact=False, keep_logits=None) -> Tuple[torch.Tensor, torch.Tensor]:
-    return _LMHeadLogprob.apply(hidden, weight, bias, labels_shifted, float(temperature), int(panel_hint), compact if torch.is_tensor(compact) else bool(compact),
+    compact = compact if torch.is_tensor(compact) else bool(compact)
+    if not _wants_grad(hidden, weight, bias):
+        _grad_mode(keep_logits)                  # refuses an unknown mode, as the differentiable path does
+        idx = _valid_rows(labels_shifted, compact)
+        return _logprob_fwd_rows(hidden, weight, bias, labels_shifted, float(temperature), idx, False, "recompute",
+                                 want_lse=False)[:2]
+    return _LMHeadLogprob.apply(hidden, weight, bias, labels_shifted, float(temperature), int(panel_hint), compact,
                                 keep_logits)
 
 
@@ -907,6 +930,16 @@ def fused_grpo_loss(hidden, weight, bias, labels_shifted, old_lp, adv, ref_lp=No
     """(loss, entropy, log_ratio, clip1, unclipped, clipped, lp); only loss carries a gradient.
     ``keep_logits``: how the gradients are formed, see ``KEEP_LOGITS`` (None = that module default);
     ``chunk_tokens``: token chunk of the chunked step (0 = ``chunk_tokens_for``)."""
+    if not _wants_grad(hidden, weight, bias):
+        # a loss nobody will differentiate (evaluation): projection and objective only
+        _grad_mode(keep_logits)
+        idx = _valid_rows(labels_shifted, compact if torch.is_tensor(compact) else bool(compact))
+        lp, ent = _logprob_fwd_rows(hidden, weight, bias, labels_shifted, float(temperature), idx, False, "recompute",
+                                    want_lse=False)[:2]
+        loss, _g, lr, c1, l1, l2, _scal = grpo_loss_fwd(lp, old_lp, ref_lp, adv, labels_shifted, cu_seqlens, float(clip_low),
+                                                        float(clip_high), float(clip_ratio_c), float(kl_beta), loss_agg_mode,
+                                                        float(denom_override))
+        return loss, ent, lr, c1, l1, l2, lp
     return _FusedGRPOLoss.apply(hidden, weight, bias, labels_shifted, old_lp, adv, ref_lp, cu_seqlens,
                                 float(temperature), float(clip_low), float(clip_high), float(clip_ratio_c),
                                 float(kl_beta), loss_agg_mode, float(denom_override), int(panel_hint),
@@ -1022,6 +1055,8 @@ class _VarlenAttention(torch.autograd.Function):
 def varlen_attention(q, k, v, cu_seqlens, softmax_scale=None, causal=True, bounds=None) -> torch.Tensor:
     """Differentiable packed self-attention on the HIP kernels (bf16 in, bf16 out).  ``bounds``: segment scratch of an
     earlier call with the same ``cu_seqlens`` and ``causal`` (see ``attention_bounds``)."""
+    if not _wants_grad(q, k, v):
+        return varlen_attn_fwd(q, k, v, cu_seqlens, softmax_scale, causal, bounds=bounds)[0]
     return _VarlenAttention.apply(q, k, v, cu_seqlens, softmax_scale, causal, bounds)
 
 

@@ -14,6 +14,7 @@ from typing import List
 import numpy as np
 import torch
 
+from fgrpo import ops
 from grpo_loss import compute_dual_clip_grpo_loss, make_grpo_forward
 from sample_processing_utils import PackedLogProbs, _fill, post_process_batch
 
@@ -98,8 +99,18 @@ class LogProbHarness:
         for k in lens:
             view[1, off:off + k] = np.arange(k)
             off += k
+        # Positions without a valid next-token label (prompts) have logprob and entropy 0 by definition: when they are a
+        # sizeable part of the batch the LM head is given the list of the others, known here on the host, and skips
+        # them (the same threshold as the trainer's loss, see grpo_loss.compute_dual_clip_grpo_loss).
+        extra = {}
+        if total >= ops.COMPACT_MIN_TOKENS:
+            scored = np.flatnonzero(view[2, 1:] != -100)
+            if 0 < scored.size < ops.COMPACT_MAX_VALID_FRACTION * total:
+                rows = torch.empty(scored.size, dtype=torch.long).pin_memory()
+                rows.numpy()[:] = scored
+                extra["compact_masked_tokens"] = rows.to(self.device, non_blocking=True)
         dev = host.to(self.device, non_blocking=True)
-        out = self.actor_module_fsdp(input_ids=dev[0:1], attention_mask=None, position_ids=dev[1:2], labels=dev[2:3])
+        out = self.actor_module_fsdp(input_ids=dev[0:1], attention_mask=None, position_ids=dev[1:2], labels=dev[2:3], **extra)
         # one device->host copy for the whole batch into one pinned buffer
         ent = getattr(out, "entropy", None)
         rows = 2 if ent is not None else 1
