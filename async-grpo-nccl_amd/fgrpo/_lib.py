@@ -7,7 +7,7 @@ from __future__ import annotations
 import ctypes as C
 import os
 
-from .build import LIB_PATH
+from .build import BINDING_PATH, LIB_PATH
 
 ERR = {-1: "bad argument", -2: "unsupported", -3: "workspace", -4: "HIP error", -5: "alignment"}
 
@@ -91,6 +91,27 @@ def load() -> C.CDLL:
         fn.argtypes = args
     _lib = lib
     return lib
+
+
+_native = None
+
+
+def native():
+    """The autograd nodes over the library (``csrc/torch_binding.cpp``), handed the entry points of the copy ``load``
+    returned; raise if they are not built."""
+    global _native
+    if _native is not None:
+        return _native
+    lib = load()
+    if not os.path.exists(BINDING_PATH):
+        raise RuntimeError(f"fgrpo: {BINDING_PATH} is missing - build it with `python -m fgrpo.build`")
+    import importlib.util
+    spec = importlib.util.spec_from_file_location("_fgrpo_torch", BINDING_PATH)
+    mod = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(mod)
+    mod.init({name: C.cast(getattr(lib, name), C.c_void_p).value for name in SIGNATURES})
+    _native = mod
+    return mod
 
 
 def check(rc: int, what: str) -> None:

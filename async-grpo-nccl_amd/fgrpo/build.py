@@ -115,10 +115,37 @@ def _is_noise(line: str) -> bool:
     return "packed-fp32-ops" in line or "kernel-resource-usage" in line or line.startswith("In file included from")
 
 
+BINDING_SOURCE = "torch_binding.cpp"
+BINDING_PATH = os.path.join(CSRC, "_fgrpo_torch.so")
+
+
+def build_binding(verbose: bool = True) -> str:
+    """The autograd nodes over the library (host code only), as an extension module next to it."""
+    import sysconfig
+    import torch
+    from torch.utils import cpp_extension as ext
+    abi = int(torch._C._GLIBCXX_USE_CXX11_ABI)
+    tmp = BINDING_PATH + ".linking"
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           "-DTORCH_EXTENSION_NAME=_fgrpo_torch", "-DTORCH_API_INCLUDE_EXTENSION_H", f"-D_GLIBCXX_USE_CXX11_ABI={abi}",
+           *[f"-I{p}" for p in ext.include_paths("cuda")], f"-I{sysconfig.get_paths()['include']}",
+           os.path.join(CSRC, BINDING_SOURCE), "-o", tmp, *[f"-L{p}" for p in ext.library_paths("cuda")],
+           "-ltorch", "-ltorch_cpu", "-ltorch_hip", "-lc10", "-lc10_hip", "-ltorch_python"]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    res = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"{BINDING_SOURCE} failed to build:\n" + res.stdout)
+    os.replace(tmp, BINDING_PATH)
+    return BINDING_PATH
+
+
 def build(verbose: bool = True, only=None) -> str:
     """Compile every translation unit (or those named in ``only``, reusing the other objects) and link."""
     os.makedirs(OBJ_DIR, exist_ok=True)
     todo = [s for s in SOURCES if only is None or s in only]
+    side = concurrent.futures.ThreadPoolExecutor(max_workers=1)
+    binding = side.submit(build_binding, verbose) if only is None or BINDING_SOURCE in only else None
     by_source = {}
     if only is not None and os.path.exists(USAGE_PATH):
         by_source = json.load(open(USAGE_PATH)).get("sources", {})
@@ -167,6 +194,8 @@ def build(verbose: bool = True, only=None) -> str:
             os.remove(tmp)
         raise RuntimeError("link failed:\n" + res.stdout)
     os.replace(tmp, LIB_PATH)
+    if binding is not None:
+        binding.result()
     return LIB_PATH
 
 

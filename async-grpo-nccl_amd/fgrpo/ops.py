@@ -578,6 +578,9 @@ CHUNK_TOKENS = 8192
 CHUNK_MAX_BYTES = 8 << 30
 
 
+_NATIVE_MODES = {"auto": 0, "recompute": 1, "whole": 2, "chunked": 3}     # as csrc/torch_binding.cpp numbers them
+
+
 def _grad_mode(keep_logits):
     mode = KEEP_LOGITS if keep_logits is None else keep_logits
     if mode is True or mode == "whole":
@@ -793,7 +796,8 @@ class _LMHeadLogprob(torch.autograd.Function):
 
 
 class _FusedGRPOLoss(torch.autograd.Function):
-    """Projection -> logprob -> dual-clip objective in one autograd node.  The
+    """Projection -> logprob -> dual-clip objective in one autograd node, for batches some of whose rows are left out
+    of the projection (the others take the node of csrc/torch_binding.cpp).  The
     backward receives the scalar upstream gradient as a device pointer."""
 
     @staticmethod
@@ -930,20 +934,32 @@ def fused_grpo_loss(hidden, weight, bias, labels_shifted, old_lp, adv, ref_lp=No
     """(loss, entropy, log_ratio, clip1, unclipped, clipped, lp); only loss carries a gradient.
     ``keep_logits``: how the gradients are formed, see ``KEEP_LOGITS`` (None = that module default);
     ``chunk_tokens``: token chunk of the chunked step (0 = ``chunk_tokens_for``)."""
-    if not _wants_grad(hidden, weight, bias):
-        # a loss nobody will differentiate (evaluation): projection and objective only
-        _grad_mode(keep_logits)
-        idx = _valid_rows(labels_shifted, compact if torch.is_tensor(compact) else bool(compact))
+    if loss_agg_mode not in ("token_mean", "sample_mean"):
+        raise ValueError(f"Invalid loss_agg_mode: {loss_agg_mode}")
+    mode = _grad_mode(keep_logits)
+    compact = compact if torch.is_tensor(compact) else bool(compact)
+    wants_grad = _wants_grad(hidden, weight, bias)
+    idx = _valid_rows(labels_shifted, compact)
+    if idx is None and _fwd_event_sink is None and hidden.shape[0] > 0:
+        V = weight.shape[0]
+        chunk = int(chunk_tokens) if chunk_tokens and chunk_tokens > 0 else chunk_bound_for(V)
+        return _lib.native().fused_step(hidden, weight, bias, labels_shifted, old_lp, adv, ref_lp, cu_seqlens,
+                                        float(temperature), float(clip_low), float(clip_high), float(clip_ratio_c),
+                                        float(kl_beta), loss_agg_mode == "sample_mean", float(denom_override),
+                                        int(panel_hint), _NATIVE_MODES[mode], chunk, KEEP_WHOLE_MAX_BYTES)
+    # rows left out of the projection (gathered and scattered with torch), a timed forward, an empty batch
+    if not wants_grad:
         lp, ent = _logprob_fwd_rows(hidden, weight, bias, labels_shifted, float(temperature), idx, False, "recompute",
                                     want_lse=False)[:2]
         loss, _g, lr, c1, l1, l2, _scal = grpo_loss_fwd(lp, old_lp, ref_lp, adv, labels_shifted, cu_seqlens, float(clip_low),
                                                         float(clip_high), float(clip_ratio_c), float(kl_beta), loss_agg_mode,
                                                         float(denom_override))
         return loss, ent, lr, c1, l1, l2, lp
+    compact = idx if idx is not None else False
     return _FusedGRPOLoss.apply(hidden, weight, bias, labels_shifted, old_lp, adv, ref_lp, cu_seqlens,
                                 float(temperature), float(clip_low), float(clip_high), float(clip_ratio_c),
                                 float(kl_beta), loss_agg_mode, float(denom_override), int(panel_hint),
-                                compact if torch.is_tensor(compact) else bool(compact), keep_logits, int(chunk_tokens))
+                                compact, keep_logits, int(chunk_tokens))
 
 
 # --------------------------------------------------------------------------- packed variable-length attention
@@ -1037,27 +1053,10 @@ def varlen_attn_bwd(dout: torch.Tensor, q: torch.Tensor, k: torch.Tensor, v: tor
     return dq, dk, dv
 
 
-class _VarlenAttention(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, q, k, v, cu_seqlens, softmax_scale, causal, bounds=None):
-        out, lse, bounds = varlen_attn_fwd(q, k, v, cu_seqlens, softmax_scale, causal, return_bounds=True, bounds=bounds)
-        ctx.save_for_backward(q, k, v, out, lse, cu_seqlens, bounds)
-        ctx.softmax_scale, ctx.causal = softmax_scale, causal
-        return out
-
-    @staticmethod
-    def backward(ctx, dout):
-        q, k, v, out, lse, cu, bounds = ctx.saved_tensors
-        dq, dk, dv = varlen_attn_bwd(dout.to(torch.bfloat16), q, k, v, out, lse, cu, ctx.softmax_scale, ctx.causal, bounds)
-        return dq, dk, dv, None, None, None, None
-
-
 def varlen_attention(q, k, v, cu_seqlens, softmax_scale=None, causal=True, bounds=None) -> torch.Tensor:
     """Differentiable packed self-attention on the HIP kernels (bf16 in, bf16 out).  ``bounds``: segment scratch of an
     earlier call with the same ``cu_seqlens`` and ``causal`` (see ``attention_bounds``)."""
-    if not _wants_grad(q, k, v):
-        return varlen_attn_fwd(q, k, v, cu_seqlens, softmax_scale, causal, bounds=bounds)[0]
-    return _VarlenAttention.apply(q, k, v, cu_seqlens, softmax_scale, causal, bounds)
+    return _lib.native().varlen_attention(q, k, v, cu_seqlens, softmax_scale, bool(causal), bounds)
 
 
 def attention_bounds(cu_seqlens: torch.Tensor, T: int, causal: bool = True) -> torch.Tensor:
