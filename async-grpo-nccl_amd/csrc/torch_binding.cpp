@@ -412,7 +412,10 @@ Tensor varlen_attention(const Tensor& q, const Tensor& k, const Tensor& v, const
                     a.bounds.is_contiguous(),
                 "fgrpo: bounds does not come from an attention call of this shape");
   }
-  const bool wanted = at::GradMode::is_enabled() && (q.requires_grad() || k.requires_grad() || v.requires_grad());
+  // a forward-mode tangent goes to the node as well, which refuses it (also where gradients are off)
+  auto dual = [](const Tensor& t) { return t._fw_grad(0).defined(); };
+  const bool wanted = (at::GradMode::is_enabled() && (q.requires_grad() || k.requires_grad() || v.requires_grad())) ||
+                      dual(q) || dual(k) || dual(v);
   return wanted ? VarlenAttention::apply(q, k, v, a) : VarlenAttention::forward(nullptr, q, k, v, a);
 }
 

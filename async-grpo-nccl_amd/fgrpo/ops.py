@@ -9,6 +9,7 @@ from __future__ import annotations
 from typing import Optional, Tuple
 
 import torch
+from torch.autograd import forward_ad
 
 from . import _lib
 
@@ -622,8 +623,13 @@ def _want_keep(T: int, H: int, V: int, dtype, needs_grad: bool, keep_logits=None
 def _wants_grad(*tensors) -> bool:
     """Whether a backward can reach any of these.  Asked outside the autograd functions: inside one, the gradient mode
     is always off and ``needs_input_grad`` repeats ``requires_grad`` even under ``torch.no_grad()`` - an evaluation of
-    a trainable head would then prepare a backward that never comes (the kept forward writes [T, V] in bf16)."""
-    return torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in tensors)
+    a trainable head would then prepare a backward that never comes (the kept forward writes [T, V] in bf16).
+    Forward-mode tangents count too, under ``no_grad`` as well: the autograd functions refuse them, a call past those
+    would drop them in silence."""
+    tensors = [t for t in tensors if t is not None]
+    if forward_ad._current_level >= 0 and any(forward_ad.unpack_dual(t).tangent is not None for t in tensors):
+        return True
+    return torch.is_grad_enabled() and any(t.requires_grad for t in tensors)
 
 
 def _logprob_fwd_rows(hidden, weight, bias, labels_shifted, temperature, idx, needs_grad=False, keep_logits=None,

@@ -65,3 +65,21 @@ def test_logprob_worker_skips_prompts_and_returns_the_same(dev):
         ops.COMPACT_MIN_TOKENS = keep
     assert torch.equal(got == 0, want == 0)
     assert (got - want).abs().max() <= 2e-5
+
+
+def test_forward_mode_tangents_are_refused(dev):
+    """No node implements forward-mode derivatives; a call that needs no backward must not drop a tangent in silence."""
+    import torch.autograd.forward_ad as fwAD
+    from fgrpo import ops
+    cu = torch.tensor([0, 40], dtype=torch.int32, device=dev)
+    q, k, v = (torch.randn(40, n, 64, device=dev).bfloat16() for n in (4, 2, 2))
+    h, w = torch.randn(70, 64, device=dev).bfloat16(), torch.randn(300, 64, device=dev).bfloat16()
+    y = torch.randint(0, 300, (70,), device=dev)
+    idx = torch.arange(0, 70, 2, device=dev)
+    with fwAD.dual_level(), torch.no_grad():
+        dq, dh = fwAD.make_dual(q, torch.ones_like(q)), fwAD.make_dual(h, torch.ones_like(h))
+        for call in (lambda: ops.varlen_attention(dq, k, v, cu), lambda: ops.lmhead_logprob(dh, w, None, y),
+                     lambda: ops.fused_grpo_loss(dh, w, None, y, None, torch.ones(70, device=dev), compact=idx),
+                     lambda: ops.fused_grpo_loss(dh, w, None, y, None, torch.ones(70, device=dev))):
+            with pytest.raises(RuntimeError, match="(?i)jvp"):
+                call()
