@@ -83,3 +83,30 @@ def test_forward_mode_tangents_are_refused(dev):
                      lambda: ops.fused_grpo_loss(dh, w, None, y, None, torch.ones(70, device=dev))):
             with pytest.raises(RuntimeError, match="(?i)jvp"):
                 call()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("N,V,ld", [(1, 5, 8), (3, 2048, 2048), (5, 8191, 8192), (2, 8200, 8208), (4, 10247, 10247), (3, 16392, 16400)])
+def test_row_kernels_at_the_edges_of_their_strides(dev, dtype, N, V, ld):
+    """Log-probabilities, entropy and gradient on rows that end inside a chunk, a stride of one or four chunks, or are
+    not 16-byte aligned; one row ignored.  Against fp64; fp32 sums over V terms, bf16 results rounded to 2^-8."""
+    from fgrpo import ops
+    g = torch.Generator().manual_seed(V)
+    store = (torch.randn(N, ld, generator=g) * 3).to(dtype)
+    x = store.to(dev)[:, :V]
+    y = torch.randint(0, V, (N,), generator=g)
+    y[0] = V - 1
+    if N > 1:
+        y[1] = -100
+    lp, ent, lse = ops.logits_logprob_entropy(x, y.to(dev), -100)
+    gt = torch.randn(N, generator=g)
+    dx = ops.logits_logprob_bwd(x, y.to(dev), -100, gt.to(dev), lse).cpu().double()
+    xd = store[:, :V].double()
+    ls = torch.log_softmax(xd, 1)
+    live = (y >= 0).double()
+    want_lp = ls.gather(1, y.clamp(min=0)[:, None])[:, 0] * live
+    want_dx = (torch.nn.functional.one_hot(y.clamp(min=0), V) - ls.exp()) * (gt.double() * live)[:, None]
+    assert (lp.cpu().double() - want_lp).abs().max() <= 1e-5
+    assert (ent.cpu().double() + (ls.exp() * ls).sum(1)).abs().max() <= 2e-5
+    tol = (2 ** -8 if dtype == torch.bfloat16 else 2e-6) * want_dx.abs() + 1e-6 * gt.double().abs()[:, None]
+    assert ((dx - want_dx).abs() <= tol).all()
