@@ -126,6 +126,20 @@ template <class C>
 __device__ __forceinline__ int acc16_col(int wn, int j, int e, int lane) {
   return wn * C::WTN + j * 32 + 16 * ((e >> 2) & 1) + (lane & 15);
 }
+// Sub-tile (wm, wn) of a wavefront.  Wavefronts w and w + 4 share a SIMD.  CROSSED (the contraction-major gradient
+// products): the two lie in different row halves AND different column halves, so that a tile with one half outside
+// the matrix (rows or columns) leaves every SIMD one wavefront that computes and one that only loads (wave_is_live).
+template <class C, bool CROSSED>
+__device__ __forceinline__ void wave_coords(int wave, int& wm, int& wn) {
+  if constexpr (CROSSED) {
+    static_assert(C::WM == 2 && C::WN == 4, "wavefront grid");
+    wm = (wave ^ (wave >> 2)) & 1;
+    wn = wave >> 1;
+  } else {
+    wm = wave / C::WN;
+    wn = wave % C::WN;
+  }
+}
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32x4_t;
 // acc<registers 4Q .. 4Q+3> += a (16 rows x 32 k) * b (16 columns x 32 k)
 template <int Q>
@@ -474,7 +488,7 @@ __device__ __forceinline__ void early_barrier_pipeline(int nk_total, char* smem,
 //   load_a(stage_ptr, I, KK): fragment a(I, KK % 2) of slice KK / 2;  load_b(stage_ptr, JC, K2): fragment b(JC/2, JC%2).
 template <class C, int LPT, int RA, int RB, class IssueOne, class LoadA, class LoadB>
 __device__ __forceinline__ void early_barrier_pipeline16(int nk_total, char* smem, f32x16_t (&acc)[C::TM][C::TN],
-                                                         IssueOne&& issue_one, LoadA&& load_a, LoadB&& load_b) {
+                                                         bool live, IssueOne&& issue_one, LoadA&& load_a, LoadB&& load_b) {
   constexpr int KK = 4;
   constexpr int TM = C::TM, NB = 2 * C::TN;           // a fragments per sub-step, b fragments per K slice
   static_assert(kMi16<C> && C::BK == 64, "16x16x32 schedule: 8-wavefront 256x256x64 tile");
@@ -497,6 +511,16 @@ __device__ __forceinline__ void early_barrier_pipeline16(int nk_total, char* sme
   };
   FGRPO_WAIT_VMCNT(0);
   wg_barrier();                                       // step 0 is in buffer 0
+  if (!live) {
+    // a sub-tile outside the matrix: this wavefront's share of the loads and every barrier, nothing else
+    for (int kt = 1; kt < nk_total; ++kt) {
+      static_for<LPT>([&](auto q) { issue_one(kt & 1, decltype(q)::value); });
+      FGRPO_WAIT_VMCNT(0);
+      wg_barrier();                                   // the one inside step kt - 1: step kt is in LDS, the other buffer is free
+    }
+    wg_barrier();
+    return;
+  }
   int steps_issued = nk_total > 0 ? 1 : 0;
   bool active = steps_issued < nk_total;              // a step is being loaded
   int tgt = 1;                                        // ... into this buffer
@@ -584,6 +608,14 @@ __device__ __forceinline__ void early_barrier_pipeline16(int nk_total, char* sme
   for (; kt + 2 < nk_total; ++kt) step(kt, std::true_type{});
   for (; kt < nk_total; ++kt) step(kt, std::false_type{});
   wg_barrier();                                       // LDS may be reused by the caller
+}
+
+// Whether a wavefront's sub-tile holds anything of the matrix.  Those that do not skip the matrix instructions and LDS
+// reads of the main loop (their accumulators stay zero).  In the contraction-major gradient products only: the LM-head
+// kernels keep their statistics in registers across the loop and would spill.
+template <class C>
+__device__ __forceinline__ bool wave_is_live(const GemmOperands& g, int row0, int col0, int wm, int wn) {
+  return row0 + wm * C::WTM < g.M && col0 + wn * C::WTN < g.N;
 }
 
 // MODE 0: the whole contraction.  MODE 2: only issue the loads of K step 0 into buffer 0 and return (the caller
@@ -712,7 +744,7 @@ __device__ __forceinline__ void gemm_mainloop_dma(const GemmOperands& g, int row
 #pragma unroll
     for (int k2 = 0; k2 < 2; ++k2) fc16[k2] = ((4 * k2 + (lane >> 4)) ^ sw16) * 16;
     early_barrier_pipeline16<C, LPT, 1, 1>(
-        nk_total, smem, acc, issue_one,
+        nk_total, smem, acc, true, issue_one,
         [&](const char* st, auto i, auto kk) {
           constexpr int kkv = decltype(kk)::value;
           return lds_read_b128_asm<(decltype(i)::value * 32 + 16 * (kkv & 1)) * C::ROWB>(lds_addr(st) + fa16 + fc16[kkv >> 1]);
@@ -997,7 +1029,8 @@ __device__ __forceinline__ void gemm_mainloop_km(const GemmOperands& g, int row0
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);   // wavefront-uniform
-  const int wm = wave / C::WN, wn = wave % C::WN;
+  int wm, wn;
+  wave_coords<C, MI16>(wave, wm, wn);
 
   // ---- loader ------------------------------------------------------------------------------
   uint32_t aoff[C::PA], boff[C::PB];            // per-lane byte offset of each load inside the step's slice
@@ -1186,7 +1219,7 @@ __device__ __forceinline__ void gemm_mainloop_km(const GemmOperands& g, int row0
 #pragma unroll
     for (int jc = 0; jc < 2 * C::TN; ++jc) fkb16[jc] = REG + k16_row + km16_off(wn * C::WTN + (jc >> 1) * 32 + 16 * (jc & 1));
     early_barrier_pipeline16<C, LPT, AKM ? 2 : 1, BKM ? 2 : 1>(
-        nk_total, smem, acc, issue_one,
+        nk_total, smem, acc, wave_is_live<C>(g, row0, col0, wm, wn), issue_one,
         [&](const char* st, auto ic, auto kc) -> bf16x8_t {
           constexpr int i = decltype(ic)::value, kk = decltype(kc)::value, k2 = kk >> 1, rh = kk & 1;
           if constexpr (AKM)

@@ -761,7 +761,8 @@ template <class C, bool AKM = false, bool BKM = false, bool SPLITK = false>
 __global__ __launch_bounds__(C::NT, C::OCC) void gemm_store_kernel(const StoreParams p0) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm = wave / C::WN, wn = wave % C::WN;
+  int wm, wn;
+  wave_coords<C, kMi16<C> && (AKM || BKM)>(wave, wm, wn);
 
   if constexpr (SPLITK) {
     static_assert(!AKM && BKM && kMi16<C>, "split contraction: dHidden's layouts on the 16x16x32 tile");

@@ -110,3 +110,19 @@ def test_row_kernels_at_the_edges_of_their_strides(dev, dtype, N, V, ld):
     assert (ent.cpu().double() + (ls.exp() * ls).sum(1)).abs().max() <= 2e-5
     tol = (2 ** -8 if dtype == torch.bfloat16 else 2e-6) * want_dx.abs() + 1e-6 * gt.double().abs()[:, None]
     assert ((dx - want_dx).abs() <= tol).all()
+
+
+@pytest.mark.parametrize("a_km", [True, False])
+@pytest.mark.parametrize("M,N", [(1, 1), (128, 256), (129, 128), (256, 129), (100, 40), (384, 640), (300, 200)])
+def test_gradient_products_on_tiles_with_a_half_outside(dev, M, N, a_km):
+    """Rows or columns that fill at most half of the last 256-wide tile: the wavefronts of the other half only load.
+    Against fp64 on the same bf16 operands: fp32 sums of K = 448 products of order one."""
+    from fgrpo import ops
+    K = 448
+    g = torch.Generator().manual_seed(M * 1000 + N)
+    Mp, Np = (M + 255) // 256 * 256, (N + 255) // 256 * 256
+    A = torch.randn(K, Mp, generator=g).bfloat16() if a_km else torch.randn(M, K, generator=g).bfloat16()
+    B = torch.randn(N, K, generator=g).bfloat16() if a_km else torch.randn(K, Np, generator=g).bfloat16()
+    out = ops.gemm_kmajor(A.to(dev), B.to(dev), a_km, not a_km, M, N, K).cpu().double()
+    Ad, Bd = (A[:, :M].double().t(), B.double()) if a_km else (A.double(), B[:, :N].double().t())
+    assert (out - Ad @ Bd.t()).abs().max() <= 2e-4
