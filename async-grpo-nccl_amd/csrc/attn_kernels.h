@@ -67,7 +67,28 @@ struct AttnParams {
   bf16_t* dq;            // [T][Hq][HD] contiguous
   bf16_t* dk;            // [T][Hkv][HD] contiguous
   bf16_t* dv;
+  // launches whose tiles are dealt to several work-groups (SPLIT kernels, see attn_parts); q: query side, k: key side
+  int parts_q, per_q, blocks_q;      // most parts of a tile, steps a part is meant to walk, work-groups of one part
+  int parts_k, per_k, blocks_k;      // the same; steps: items of a wavefront
+  float* part_q;         // [parts_q][T][Hq][HD] O of the part, relative to its own maximum, or its dQ / scale
+  float2* part_ml;       // [parts_q][Hq][T] forward: maximum and sum of the part
+  float* part_k;         // [parts_k][2][T][Hkv][HD] dK / scale and dV of the part
 };
+
+// A tile that walks `steps` steps, all its work-group's own chain, may be dealt to several work-groups: each walks its
+// share and leaves fp32 sums, which a last launch adds up in a fixed order (no atomics: bit-reproducible).  How many,
+// every kernel of the call derives from the segment bounds.
+__device__ __forceinline__ int attn_parts(int steps, int parts, int per) {
+  const int n = (steps + per - 1) / per;
+  return n < 1 ? 1 : n > parts ? parts : n;
+}
+// keys a query tile of RB tokens from q0 on walks: [k_begin, k_end)
+__device__ __forceinline__ void attn_query_tile_keys(const AttnParams& p, int q0, int RB, int& k_begin, int& k_end) {
+  const int last = q0 + RB - 1 < p.T ? q0 + RB - 1 : p.T - 1;
+  k_begin = max(p.seg_start[q0], 0);
+  k_end = min(p.causal ? last + 1 : p.seg_end[last], p.T);
+}
+__device__ __forceinline__ int attn_steps(int k_begin, int k_end) { return k_end > k_begin ? (k_end - k_begin + kAttnBK - 1) / kAttnBK : 0; }
 
 typedef short i16x4_t __attribute__((ext_vector_type(4)));
 
@@ -201,6 +222,16 @@ __device__ __forceinline__ void attn_store_rowmajor(const f32x16_t (&acc)[DB], f
       pk.y = pack_bf16x2(acc[db][4 * g + 2] * mul, acc[db][4 * g + 3] * mul);
       *(uint2*)(row_ptr + 32 * db + 8 * g + 4 * h) = pk;
     }
+}
+
+// ... and the same accumulator as it is, in fp32
+template <int DB>
+__device__ __forceinline__ void attn_store_partial(const f32x16_t (&acc)[DB], float* row_ptr, int h) {
+#pragma unroll
+  for (int db = 0; db < DB; ++db)
+#pragma unroll
+    for (int g = 0; g < 4; ++g)
+      *(float4*)(row_ptr + 32 * db + 8 * g + 4 * h) = make_float4(acc[db][4 * g], acc[db][4 * g + 1], acc[db][4 * g + 2], acc[db][4 * g + 3]);
 }
 
 // ---------------------------------------------------------------------------------------------------------
@@ -1265,7 +1296,7 @@ struct AttnTileCursor {
   }
 };
 
-template <int HD, int HB>
+template <int HD, int HB, bool SPLIT = false>
 __global__ __launch_bounds__(256, 2) void varlen_attn_fwd2_kernel(AttnParams p) {
   constexpr int KS = HD / 16, DB = HD / 32, kAttnTile = kAttnBK * HD * 2, kHD = HD, G4 = KS / 2;
   __shared__ __attribute__((aligned(16))) char smem[4 * kAttnTile];      // [buffer][K | V]
@@ -1280,7 +1311,8 @@ __global__ __launch_bounds__(256, 2) void varlen_attn_fwd2_kernel(AttnParams p) 
   // work-group -> (tile, K/V head, query heads): as in varlen_attn_fwd_kernel
   constexpr int WPH = 4 / HB, RB = 32 * WPH;
   const int G = p.Hq / p.Hkv, NB = (G + HB - 1) / HB;
-  const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
+  const int part = SPLIT ? (int)blockIdx.x / p.blocks_q : 0, bid = (int)blockIdx.x - part * (SPLIT ? p.blocks_q : 0);
+  const int xcd = bid & 7, slot = bid >> 3;
   const int unit = (slot / NB) * 8 + xcd;
   const int ntile = (p.T + RB - 1) / RB;
   if (unit >= ntile * p.Hkv) return;
@@ -1294,8 +1326,16 @@ __global__ __launch_bounds__(256, 2) void varlen_attn_fwd2_kernel(AttnParams p) 
   const int lo = valid ? p.seg_start[tq] : 1;
   const int hi = valid ? (p.causal ? tq : p.seg_end[tq] - 1) : 0;
   const int last = (q0 + RB - 1 < p.T ? q0 + RB - 1 : p.T - 1);
-  const int k_begin = max(__builtin_amdgcn_readfirstlane(p.seg_start[q0]), 0);
-  const int k_end = min(__builtin_amdgcn_readfirstlane(p.causal ? last + 1 : p.seg_end[last]), p.T);
+  int k_begin = max(__builtin_amdgcn_readfirstlane(p.seg_start[q0]), 0);
+  int k_end = min(__builtin_amdgcn_readfirstlane(p.causal ? last + 1 : p.seg_end[last]), p.T);
+  int np = 1;
+  if constexpr (SPLIT) {                   // this part's share of the steps
+    const int steps = attn_steps(k_begin, k_end);
+    np = attn_parts(steps, p.parts_q, p.per_q);
+    if (part >= np) return;
+    k_end = min(k_end, k_begin + kAttnBK * (steps * (part + 1) / np));
+    k_begin += kAttnBK * (steps * part / np);
+  }
   const int wfirst = q0 + 32 * (wave % WPH), wlast = (wfirst + 31 < p.T ? wfirst + 31 : p.T - 1);
   const bool wave_on = head_ok && wfirst < p.T;
   const int w_lo = wave_on ? p.seg_start[wfirst] : 1;
@@ -1464,6 +1504,15 @@ __global__ __launch_bounds__(256, 2) void varlen_attn_fwd2_kernel(AttnParams p) 
   float l_lo, l_hi;
   attn_halves(l_run, l_lo, l_hi);
   const float l = l_lo + l_hi;
+  if constexpr (SPLIT) {
+    if (np > 1) {
+      if (valid) {
+        attn_store_partial(acc_o, p.part_q + (((long long)part * p.T + tq) * p.Hq + hq) * kHD, h);
+        if (h == 0) p.part_ml[((long long)part * p.Hq + hq) * p.T + tq] = make_float2(m_run, l);
+      }
+      return;
+    }
+  }
   if (valid) {
     const float inv = l > 0.f ? 1.f / l : 0.f;
     attn_store_rowmajor(acc_o, inv, p.out + ((long long)tq * p.Hq + hq) * kHD, h);
@@ -1475,7 +1524,7 @@ __global__ __launch_bounds__(256, 2) void varlen_attn_fwd2_kernel(AttnParams p) 
 // with the vector arithmetic of one 32-key half placed behind the matrix instructions of the other (see the step);
 // row fragments arrive in groups of four k steps, two groups in flight, the K^T fragments of the dQ products a
 // phase ahead.
-template <int HD, int HB>
+template <int HD, int HB, bool SPLIT = false>
 __global__ __launch_bounds__(256, 2) void varlen_attn_dq2_kernel(AttnParams p) {
   constexpr int KS = HD / 16, DB = HD / 32, kAttnTile = kAttnBK * HD * 2, kHD = HD;
   __shared__ __attribute__((aligned(16))) char smem[4 * kAttnTile];      // [buffer][K | V]
@@ -1490,7 +1539,8 @@ __global__ __launch_bounds__(256, 2) void varlen_attn_dq2_kernel(AttnParams p) {
   // work-group -> (tile, K/V head, query heads): as in varlen_attn_dq_kernel
   constexpr int WPH = 4 / HB, RB = 32 * WPH;
   const int G = p.Hq / p.Hkv, NB = (G + HB - 1) / HB;
-  const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
+  const int part = SPLIT ? (int)blockIdx.x / p.blocks_q : 0, bid = (int)blockIdx.x - part * (SPLIT ? p.blocks_q : 0);
+  const int xcd = bid & 7, slot = bid >> 3;
   const int unit = (slot / NB) * 8 + xcd;
   const int ntile = (p.T + RB - 1) / RB;
   if (unit >= ntile * p.Hkv) return;
@@ -1504,8 +1554,16 @@ __global__ __launch_bounds__(256, 2) void varlen_attn_dq2_kernel(AttnParams p) {
   const int lo = valid ? p.seg_start[tq] : 1;
   const int hi = valid ? (p.causal ? tq : p.seg_end[tq] - 1) : 0;
   const int last = (q0 + RB - 1 < p.T ? q0 + RB - 1 : p.T - 1);
-  const int k_begin = max(__builtin_amdgcn_readfirstlane(p.seg_start[q0]), 0);
-  const int k_end = min(__builtin_amdgcn_readfirstlane(p.causal ? last + 1 : p.seg_end[last]), p.T);
+  int k_begin = max(__builtin_amdgcn_readfirstlane(p.seg_start[q0]), 0);
+  int k_end = min(__builtin_amdgcn_readfirstlane(p.causal ? last + 1 : p.seg_end[last]), p.T);
+  int np = 1;
+  if constexpr (SPLIT) {                   // this part's share of the steps
+    const int steps = attn_steps(k_begin, k_end);
+    np = attn_parts(steps, p.parts_q, p.per_q);
+    if (part >= np) return;
+    k_end = min(k_end, k_begin + kAttnBK * (steps * (part + 1) / np));
+    k_begin += kAttnBK * (steps * part / np);
+  }
   const int wfirst = q0 + 32 * (wave % WPH), wlast = (wfirst + 31 < p.T ? wfirst + 31 : p.T - 1);
   const bool wave_on = head_ok && wfirst < p.T;
   const int w_lo = wave_on ? p.seg_start[wfirst] : 1;
@@ -1533,7 +1591,7 @@ __global__ __launch_bounds__(256, 2) void varlen_attn_dq2_kernel(AttnParams p) {
       }
     }
     dl += attn_swap32(dl);
-    if (valid && h == 0) p.delta[(long long)hq * p.T + tq] = -dl;   // negated, for the dK/dV kernel, launched after this one
+    if (valid && h == 0 && part == 0) p.delta[(long long)hq * p.T + tq] = -dl;   // negated, for the dK/dV kernel, launched after this one
   }
   const float c = p.scale * kLog2e;
 #pragma unroll
@@ -1738,7 +1796,60 @@ __global__ __launch_bounds__(256, 2) void varlen_attn_dq2_kernel(AttnParams p) {
     step(std::integral_constant<int, 0>{}, kb);
     if (kb + kAttnBK < k_end) step(std::integral_constant<int, 1>{}, kb + kAttnBK);
   }
+  if constexpr (SPLIT) {
+    if (np > 1) {
+      if (valid) attn_store_partial(acc, p.part_q + (((long long)part * p.T + tq) * p.Hq + hq) * kHD, h);
+      return;
+    }
+  }
   if (valid) attn_store_rowmajor(acc, p.scale, p.dq + ((long long)tq * p.Hq + hq) * kHD, h);   // dS was kept / scale
+}
+
+// Sums of the parts of a query tile, in part order: eight columns of one (token, head) a thread.  Rows of tiles that were
+// not dealt out are already in place.  FWD: every part is relative to its own maximum.
+template <int HD, bool FWD>
+__device__ __forceinline__ void attn_merge_query_row(const AttnParams& p, int RB, long long idx) {
+  const int col = (int)(idx % (HD / 8)) * 8;
+  const long long row = idx / (HD / 8);                    // token * Hq + head
+  const int hq = (int)(row % p.Hq);
+  const int t = (int)(row / p.Hq);
+  if (t >= p.T) return;
+  int k_begin, k_end;
+  attn_query_tile_keys(p, t / RB * RB, RB, k_begin, k_end);
+  const int np = attn_parts(attn_steps(k_begin, k_end), p.parts_q, p.per_q);
+  if (np <= 1) return;
+  float x[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) x[e] = 0.f;
+  float mul = p.scale, m = -INFINITY, l = 0.f;
+  if constexpr (FWD) {
+    for (int j = 0; j < np; ++j) m = fmaxf(m, p.part_ml[((long long)j * p.Hq + hq) * p.T + t].x);
+  }
+  const float m_use = m == -INFINITY ? 0.f : m;
+  for (int j = 0; j < np; ++j) {
+    const float* src = p.part_q + ((long long)j * p.T * p.Hq + row) * HD + col;
+    const float4 a = *(const float4*)src, b = *(const float4*)(src + 4);
+    float w = 1.f;
+    if constexpr (FWD) {
+      const float2 ml = p.part_ml[((long long)j * p.Hq + hq) * p.T + t];
+      w = fast_exp2((ml.x - m_use) * (p.scale * kLog2e));
+      l = __builtin_fmaf(ml.y, w, l);
+    }
+    const float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+#pragma unroll
+    for (int e = 0; e < 8; ++e) x[e] = FWD ? __builtin_fmaf(v[e], w, x[e]) : x[e] + v[e];
+  }
+  if constexpr (FWD) {
+    mul = l > 0.f ? 1.f / l : 0.f;
+    if (col == 0) p.lse[(long long)hq * p.T + t] = l > 0.f ? m * p.scale + __logf(l) : -INFINITY;
+  }
+#pragma unroll
+  for (int e = 0; e < 8; ++e) x[e] *= mul;
+  *(bf16x8_t*)((FWD ? p.out : p.dq) + row * HD + col) = attn_pack8(x);
+}
+template <int HD>
+static __global__ __launch_bounds__(256) void attn_merge_fwd_kernel(AttnParams p, int RB) {
+  attn_merge_query_row<HD, true>(p, RB, (long long)blockIdx.x * 256 + threadIdx.x);
 }
 
 // seg_start[t], seg_end[t] from cu_seqlens (tokens outside every segment stand alone)

@@ -103,8 +103,14 @@ __device__ __forceinline__ void dkv3_acc_to_lds(uint32_t addr) {       // LDS in
   asm volatile("ds_write_b32 %0, a[%1] offset:%2" : : "v"(addr), "n"(REG), "n"(OFF) : "memory");
 }
 
-// KB key blocks of 32 (2: one wavefront per SIMD; 1, head dimension 64: two)
-template <int HD, int KB>
+// Items of a key tile: 32-query blocks from q_begin on x query heads of the group
+__device__ __forceinline__ int attn_key_items(int q_begin, int q_end, int G) {
+  return q_end > q_begin ? (q_end - q_begin + kDkv3Rows - 1) / kDkv3Rows * G : 0;
+}
+
+// KB key blocks of 32 (2: one wavefront per SIMD; 1, head dimension 64: two).  SPLIT: a tile's items are dealt to the
+// wavefronts of several work-groups (attn_parts), item n to wavefront n % (4 np) of them.
+template <int HD, int KB, bool SPLIT>
 __global__ __launch_bounds__(256, KB == 2 ? 1 : 2) void varlen_attn_dkv3_kernel(AttnParams p) {
   constexpr int kKeys = 32 * KB;
   constexpr int KS = HD / 16, DB = HD / 32, RB = HD * 2, kT = kDkv3Rows * RB, kBuf = kDkv3Buf<HD>;
@@ -115,7 +121,8 @@ __global__ __launch_bounds__(256, KB == 2 ? 1 : 2) void varlen_attn_dkv3_kernel(
   const int lane = threadIdx.x & 63, h = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int G = p.Hq / p.Hkv;
-  const int hkv = blockIdx.x % p.Hkv, rank = blockIdx.x / p.Hkv;
+  const int share = SPLIT ? (int)blockIdx.x / p.blocks_k : 0, bid = (int)blockIdx.x - share * (SPLIT ? p.blocks_k : 0);
+  const int hkv = bid % p.Hkv, rank = bid / p.Hkv;
   constexpr int kPer128 = 128 / kKeys;
   const int ntile = (p.T + kKeys - 1) / kKeys, n128 = (p.T + 127) / 128;
   const int tile = min(max(p.order_k[rank / kPer128], 0), n128 - 1) * kPer128 + rank % kPer128;      // clamped: the list may come from the caller
@@ -128,6 +135,10 @@ __global__ __launch_bounds__(256, KB == 2 ? 1 : 2) void varlen_attn_dkv3_kernel(
   const int q_full = !one_segment ? 0x7fffffff : p.causal ? k0 + kKeys - 1 : q_begin;
   const int nqb = q_end > q_begin ? (q_end - q_begin + kDkv3Rows - 1) / kDkv3Rows : 0;
   const int NI = nqb * G;
+  const int np = SPLIT ? attn_parts((NI + 3) / 4, p.parts_k, p.per_k) : 1;
+  if (SPLIT && share >= np) return;
+  const int first = wave + 4 * share, stride = 4 * np;          // this wavefront's items
+  const int stride_g = SPLIT ? stride % G : 4, stride_b = SPLIT ? stride / G : 0;      // ... in heads and query blocks
 
   // per-lane LDS addresses, this wavefront's buffer base included (see AttnLane)
   const uint32_t base_w = lds0 + wave * 2 * kBuf;
@@ -166,7 +177,7 @@ __global__ __launch_bounds__(256, KB == 2 ? 1 : 2) void varlen_attn_dkv3_kernel(
   const int sq = (int)(RPI * p.q_st * 2), sd = (int)(RPI * do_st * 2);
   // The walk goes from the last queries to the first, heads inside: work-groups on the same segment start at the same
   // rows and pass over them together, so that one L2 serves them all.  A step of it is a few additions.
-  int g_f = wave % G, qb_f = q_begin + (nqb - 1 - wave / G) * kDkv3Rows;      // the item the loads are at
+  int g_f = first % G, qb_f = q_begin + (nqb - 1 - first / G) * kDkv3Rows;      // the item the loads are at
   const char* f_qp = (const char*)(p.q + (long long)(hkv * G + g_f) * p.q_sh + (long long)qb_f * p.q_st);
   const char* f_dp = (const char*)(p.dout + (long long)(hkv * G + g_f) * HD + (long long)qb_f * do_st);
   long long f_qb = ((long long)q_end - qb_f - 1) * p.q_st * 2 + RB;           // bytes to the end of the head's last row
@@ -184,7 +195,15 @@ __global__ __launch_bounds__(256, KB == 2 ? 1 : 2) void varlen_attn_dkv3_kernel(
     rsq = make_rsrc(f_qp, (uint32_t)bq);
     rsd = make_rsrc(f_dp, (uint32_t)bd);
   };
-  auto fetch_advance = [&]() {             // four items on
+  auto fetch_advance = [&]() {             // `stride` items on
+    if constexpr (SPLIT) {
+      int dg = stride_g, db = stride_b;
+      if (g_f + dg >= G) dg -= G, ++db;
+      g_f += dg, qb_f -= db * kDkv3Rows;
+      f_qp += dg * h_q - db * r_q, f_dp += (long long)dg * HD * 2 - db * r_d;
+      f_qb += db * r_q, f_db += db * r_d;
+      return;
+    }
     g_f += 4;
     f_qp += 4 * h_q, f_dp += 4 * HD * 2;
     while (g_f >= G) {
@@ -219,13 +238,13 @@ __global__ __launch_bounds__(256, KB == 2 ? 1 : 2) void varlen_attn_dkv3_kernel(
   constexpr int kItemLoads = 2 * NLD + 2;
   auto fetch_item = [&](auto bc) {
     constexpr int b = decltype(bc)::value;
-    const bool more = wave + 4 * b < NI;
+    const bool more = first + stride * b < NI;
     if (b == 1 && more) fetch_advance();
     fetch_setup(more);
     static_for<NLD + 2>([&](auto ic) { fetch_q(ic, base_w + b * kBuf, sq); });
     static_for<NLD>([&](auto ic) { fetch_d(ic, base_w + b * kBuf, sd); });
   };
-  if (wave < NI) fetch_item(std::integral_constant<int, 0>{});
+  if (first < NI) fetch_item(std::integral_constant<int, 0>{});
   // K rows of the key blocks as operands
   u32x4_t kf[KB][KS];
   // the queries that see the lane's key: key_n of them, from the key itself (causal) or its segment's start on; kept
@@ -244,7 +263,7 @@ __global__ __launch_bounds__(256, KB == 2 ? 1 : 2) void varlen_attn_dkv3_kernel(
     key_n[kb] = key < p.T ? (uint32_t)max(min(p.seg_end[kc], q_end) - lo, 0) : 0u;
   }
   fence();
-  if (wave < NI) fetch_item(std::integral_constant<int, 1>{});
+  if (first < NI) fetch_item(std::integral_constant<int, 1>{});
   static_for<NACC>([&](auto rc) { dkv3_acc_clear<NACC, decltype(rc)::value>(); });      // under the loads
 #pragma unroll
   for (int kb = 0; kb < KB; ++kb) {
@@ -252,7 +271,7 @@ __global__ __launch_bounds__(256, KB == 2 ? 1 : 2) void varlen_attn_dkv3_kernel(
     for (int st = 0; st < KS; ++st) asm volatile("" : "+v"(kf[kb][st]));                // complete before the loop
     asm volatile("" : "+v"(key_lo[kb]), "+v"(key_n[kb]));
   }
-  if (wave < NI) FGRPO_WAIT_VMCNT(kItemLoads);                 // everything but the second item
+  if (first < NI) FGRPO_WAIT_VMCNT(kItemLoads);                 // everything but the second item
   else FGRPO_WAIT_VMCNT(0);
   wg_barrier();                                                // the whole V tile is there
 
@@ -435,7 +454,7 @@ __global__ __launch_bounds__(256, KB == 2 ? 1 : 2) void varlen_attn_dkv3_kernel(
 #pragma unroll
     for (int kb = 0; kb < KB; ++kb) ds[kb][1] = pack(dp[kb], 1);
     // dK, rows 8..15 | the Q rows and scalars of the item after next
-    const bool more2 = n + 8 < NI;
+    const bool more2 = n + 2 * stride < NI;
     // destinations and row offsets are formed here: held across the loop they would fill the scalar registers
     uint32_t bufs = base_w;
     int sqv = sq, sdv = sd;
@@ -453,17 +472,22 @@ __global__ __launch_bounds__(256, KB == 2 ? 1 : 2) void varlen_attn_dkv3_kernel(
     static_for<QG>([&](auto ic) { req_q(FGRPO_IC(nxt), ic); });
     wait_lgkm<QG>();                                           // everything of this item's dO rows has been read
     fence();
-    g_c += 4;
-    while (g_c >= G) g_c -= G, qb -= kDkv3Rows;
+    if constexpr (SPLIT) {
+      g_c += stride_g, qb -= stride_b * kDkv3Rows;
+      if (g_c >= G) g_c -= G, qb -= kDkv3Rows;
+    } else {
+      g_c += 4;
+      while (g_c >= G) g_c -= G, qb -= kDkv3Rows;
+    }
     quarter(tb, pp, H1{}, FGRPO_IC(kAccV), [&](auto mc) {
       deal(FGRPO_IC(NLD), mc, FGRPO_IC(0), FGRPO_IC(NQ), [&](auto ic) { fetch_d(ic, bufs + qt, sdv); });
     });
   };
-  if (wave < NI) {
+  if (first < NI) {
     static_for<QG>([&](auto ic) { req_q(FGRPO_IC(0), ic); });
-    for (int n = wave; n < NI; n += 8) {
+    for (int n = first; n < NI; n += 2 * stride) {
       item(FGRPO_IC(0), n);
-      if (n + 4 < NI) item(FGRPO_IC(1), n + 4);
+      if (n + stride < NI) item(FGRPO_IC(1), n + stride);
     }
     wait_lgkm<0>();
 #pragma unroll
@@ -477,7 +501,7 @@ __global__ __launch_bounds__(256, KB == 2 ? 1 : 2) void varlen_attn_dkv3_kernel(
   // (lane and thread index formed anew: held across the loop they would cost registers it does not have)
   constexpr int SS = kDkv3SumStride<HD>;
   const int lane_e = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)), tid_e = wave * 64 + lane_e;
-  auto sum_store = [&](auto accc, float mul, bf16_t* out) {
+  auto sum_store = [&](auto accc, float mul, bf16_t* out, int which) {
     constexpr int acc = decltype(accc)::value;
     wg_barrier();                                              // the tiles / the previous sums are no longer read
     const uint32_t w0 = lds0 + wave * (kKeys * SS) + (4 * (lane_e >> 5)) * SS + (lane_e & 31) * 4;
@@ -512,15 +536,57 @@ __global__ __launch_bounds__(256, KB == 2 ? 1 : 2) void varlen_attn_dkv3_kernel(
           if (j % 4 == 0) attn_settle(part[w][j / 4]);
           x[j] = (w == 0 ? 0.f : x[j]) + __uint_as_float(part[w][j / 4][j % 4]);
         }
+      const int kk = k0 + row;
+      const bool partial = SPLIT && np > 1;
+      if (SPLIT && partial && kk < p.T) {
+        float4* dst = (float4*)(p.part_k + ((((long long)share * 2 + which) * p.T + kk) * p.Hkv + hkv) * HD + col * 8);
+        dst[0] = make_float4(x[0], x[1], x[2], x[3]);
+        dst[1] = make_float4(x[4], x[5], x[6], x[7]);
+      }
 #pragma unroll
       for (int j = 0; j < 8; ++j) x[j] *= mul;
-      const int kk = k0 + row;
-      if (kk < p.T) *(bf16x8_t*)(out + ((long long)kk * p.Hkv + hkv) * HD + col * 8) = attn_pack8(x);
+      if (kk < p.T && !partial) *(bf16x8_t*)(out + ((long long)kk * p.Hkv + hkv) * HD + col * 8) = attn_pack8(x);
     }
     wait_lgkm<0>();
   };
-  sum_store(std::integral_constant<int, kAccK>{}, p.scale, p.dk);
-  sum_store(std::integral_constant<int, kAccV>{}, 1.f, p.dv);
+  sum_store(std::integral_constant<int, kAccK>{}, p.scale, p.dk, 0);
+  sum_store(std::integral_constant<int, kAccV>{}, 1.f, p.dv, 1);
+}
+
+// Sums of the parts, in part order, of dK and dV (key tiles of kKeys) and of dQ (query tiles of RB tokens): eight columns
+// of one row a thread.  Rows of tiles that were not dealt out are already in place.
+template <int HD, int kKeys>
+static __global__ __launch_bounds__(256) void attn_merge_bwd_kernel(AttnParams p, int RB, long long nq, long long nk) {
+  long long idx = (long long)blockIdx.x * 256 + threadIdx.x;
+  if (idx < nq) {
+    attn_merge_query_row<HD, false>(p, RB, idx);
+    return;
+  }
+  idx -= nq;
+  if (idx >= 2 * nk) return;
+  const int which = idx >= nk;
+  if (which) idx -= nk;
+  const int col = (int)(idx % (HD / 8)) * 8;
+  const long long row = idx / (HD / 8);                        // key * Hkv + head
+  const int kk = (int)(row / p.Hkv);
+  const int k0 = kk / kKeys * kKeys, klast = min(k0 + kKeys, p.T) - 1;
+  const int items = attn_key_items(max(p.causal ? k0 : p.seg_start[k0], 0), min(p.seg_end[klast], p.T), p.Hq / p.Hkv);
+  const int np = attn_parts((items + 3) / 4, p.parts_k, p.per_k);
+  if (np <= 1) return;
+  float x[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) x[e] = 0.f;
+  for (int j = 0; j < np; ++j) {
+    const float* src = p.part_k + (((long long)j * 2 + which) * p.T * p.Hkv + row) * HD + col;
+    const float4 a = *(const float4*)src, b = *(const float4*)(src + 4);
+    const float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+#pragma unroll
+    for (int e = 0; e < 8; ++e) x[e] += v[e];
+  }
+  const float mul = which ? 1.f : p.scale;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) x[e] *= mul;
+  *(bf16x8_t*)((which ? p.dv : p.dk) + row * HD + col) = attn_pack8(x);
 }
 
 }  // namespace fgrpo

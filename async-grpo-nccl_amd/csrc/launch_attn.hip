@@ -7,7 +7,11 @@
 using namespace fgrpo;
 
 namespace fgrpo {
+constexpr int kAttnMaxParts = 8;
+constexpr size_t kAttnSplitMaxBytes = 256u << 20;
 int launch_attn_dkv3(int D, const AttnParams& p, hipStream_t st);      // launch_attn_keyside.hip
+int attn_keyside_keys(int D);
+int launch_attn_merge_bwd(int D, const AttnParams& p, int rb, hipStream_t st);
 }
 
 namespace {
@@ -27,7 +31,8 @@ int launch_query_side(int D, int hb, AttnParams& p, int T, int Hq, int Hkv, int3
   const int rb = 128 / hb, G = Hq / Hkv;
   p.order_q = bounds_ws + attn_order_offset(T, hb == 1 ? 1 : hb == 2 ? 2 : 3);
   const long long units = (long long)((T + rb - 1) / rb) * Hkv;            // (tile, K/V head)
-  const dim3 grid((unsigned)(((units + 7) / 8 * 8) * ((G + hb - 1) / hb)));
+  p.blocks_q = (int)(((units + 7) / 8 * 8) * ((G + hb - 1) / hb));
+  const dim3 grid((unsigned)p.blocks_q * (p.parts_q > 1 ? p.parts_q : 1));
   if (D == 128) {
     if (hb == 1) Launcher<128, 1>::run(grid, st, p);
     else if (hb == 2) Launcher<128, 2>::run(grid, st, p);
@@ -44,6 +49,7 @@ template <int HD, int HB>
 struct FwdLauncher {
   static void run(dim3 grid, hipStream_t st, const AttnParams& p) {
     if (g_tune.attn_qside == 1) hipLaunchKernelGGL((varlen_attn_fwd_kernel<HD, HB>), grid, dim3(256), 0, st, p);
+    else if (p.parts_q > 1) hipLaunchKernelGGL((varlen_attn_fwd2_kernel<HD, HB, true>), grid, dim3(256), 0, st, p);
     else hipLaunchKernelGGL((varlen_attn_fwd2_kernel<HD, HB>), grid, dim3(256), 0, st, p);
   }
 };
@@ -51,9 +57,67 @@ template <int HD, int HB>
 struct DqLauncher {
   static void run(dim3 grid, hipStream_t st, const AttnParams& p) {
     if (g_tune.attn_qside == 1 || g_tune.attn_qside == 3) hipLaunchKernelGGL((varlen_attn_dq_kernel<HD, HB>), grid, dim3(256), 0, st, p);
+    else if (p.parts_q > 1) hipLaunchKernelGGL((varlen_attn_dq2_kernel<HD, HB, true>), grid, dim3(256), 0, st, p);
     else hipLaunchKernelGGL((varlen_attn_dq2_kernel<HD, HB>), grid, dim3(256), 0, st, p);
   }
 };
+// How the tiles of a launch are dealt to several work-groups (attn_parts).  A launch of few tiles ends when its longest
+// chain of steps does, however idle the device is; sharing a chain costs fp32 sums through memory and one more launch.
+// Both sides are estimated, in us, from what was measured: `step` for a step of a work-group alone on its CU, half as
+// much again where two share one; 4 us for the additional launch, 3 TB/s for the sums, written and read.  The tiles of a
+// causal launch walk 0 .. chain steps, evenly; segments of one call are taken to be as long as their mean (twice that
+// at most: the number of parts allowed for).  Decided by shapes alone.  Kernel times, whole | dealt out: forward, one
+// segment of 777 tokens, 12 / 2 heads of 128: 25.6 | 16.1 us, of 6000 tokens 183 | 160; 3 segments of 1024 tokens 29.2 |
+// 42, which the estimate refuses.
+struct SplitPlan {
+  int parts = 1, per = 1;
+};
+SplitPlan plan_split(long long wgs, int per_cu, double chain, bool causal, double step, size_t bytes_a_part) {
+  SplitPlan best;
+  const double cus = num_cus(), slots = cus * per_cu, fill = causal ? 0.5 : 1.0;
+  auto shared = [&](double n) {            // step time with n work-groups in flight
+    const double over = per_cu > 1 ? n / cus - 1.0 : 0.0;
+    return step * (1.0 + 0.5 * (over < 0.0 ? 0.0 : over > 1.0 ? 1.0 : over));
+  };
+  const double load = (double)wgs * chain * fill / slots * shared(2.0 * slots);
+  const double whole = chain * shared((double)wgs) > load ? chain * shared((double)wgs) : load;
+  double least = 0.85 * whole;
+  for (int n = 2; n <= kAttnMaxParts; ++n) {
+    const int per = (int)(chain / n) + 1;
+    if ((size_t)n * bytes_a_part > kAttnSplitMaxBytes || per < 2) break;
+    const double x = chain / per;          // parts of the longest tile
+    const double mean = causal ? x / 2 + 0.5 : x, sums = causal ? mean - 1.0 / x : mean;
+    const double walk = per * shared(wgs * mean);
+    const double cost = (walk > load ? walk : load) + 4.0 + sums * (double)bytes_a_part * 2.0 / 3.0e6;
+    if (cost >= least) continue;
+    least = cost;
+    const int parts = (int)(2.0 * x) + 1, fit = (int)(kAttnSplitMaxBytes / bytes_a_part);
+    best.parts = parts < kAttnMaxParts ? parts : kAttnMaxParts;
+    if (best.parts > fit) best.parts = fit;
+    best.per = per;
+  }
+  return best;
+}
+SplitPlan plan_query_split(int T, int n_seq, int Hq, int Hkv, int D, int causal, bool forward) {
+  if (g_tune.attn_qside == 1 || (!forward && g_tune.attn_qside == 3)) return SplitPlan();
+  const int hb = attn_heads_per_group(Hq / Hkv, T, n_seq), rb = 128 / hb, G = Hq / Hkv;
+  const long long wgs = (long long)((T + rb - 1) / rb) * Hkv * ((G + hb - 1) / hb);
+  return plan_split(wgs, 2, (double)T / n_seq / kAttnBK, causal, D == 128 ? 1.6 : forward ? 1.15 : 1.3,
+                    (size_t)T * Hq * (D * 4 + (forward ? 8 : 0)));
+}
+SplitPlan plan_key_split(int T, int n_seq, int Hq, int Hkv, int D, int causal) {
+  if (g_tune.attn_dkv == 1 || g_tune.attn_dkv == 2) return SplitPlan();
+  const int keys = attn_keyside_keys(D);
+  const long long wgs = (long long)((T + keys - 1) / keys) * Hkv;
+  const double chain = (double)T / n_seq / 32 * (Hq / Hkv) / 4;                // items of one of the four wavefronts
+  return plan_split(wgs, D == 128 ? 1 : 2, chain, causal, D == 128 ? 1.3 : 0.65, (size_t)T * Hkv * D * 8);
+}
+size_t align256(size_t n) { return (n + 255) / 256 * 256; }
+size_t query_split_bytes(const SplitPlan& s, int T, int Hq, int D, bool forward) {
+  if (s.parts <= 1) return 0;
+  return align256((size_t)s.parts * T * Hq * D * 4) + (forward ? align256((size_t)s.parts * T * Hq * 8) : 0);
+}
+size_t key_split_bytes(const SplitPlan& s, int T, int Hkv, int D) { return s.parts <= 1 ? 0 : align256((size_t)s.parts * T * Hkv * D * 8); }
 }  // namespace
 
 extern "C" {
@@ -103,10 +167,24 @@ int fgrpo_varlen_attn_bounds(const int32_t* cu, int n_seq, int T, int causal, in
   return 0;
 }
 
+size_t fgrpo_varlen_attn_workspace(int T, int n_seq, int Hq, int Hkv, int D, int causal, int backward) {
+  if (T <= 0 || n_seq <= 0 || Hq <= 0 || Hkv <= 0 || Hq % Hkv != 0 || (D != 128 && D != 64)) return 0;
+  const size_t q = query_split_bytes(plan_query_split(T, n_seq, Hq, Hkv, D, causal, !backward), T, Hq, D, !backward);
+  return backward ? q + key_split_bytes(plan_key_split(T, n_seq, Hq, Hkv, D, causal), T, Hkv, D) : q;
+}
+
 int fgrpo_varlen_attn_fwd(const void* q, const void* k, const void* v, long long q_st, long long q_sh, long long k_st,
                           long long k_sh, long long v_st, long long v_sh, const int32_t* cu, int n_seq, int T, int Hq,
                           int Hkv, int D, float scale, int causal, void* out, float* lse, int32_t* bounds_ws,
                           int bounds_valid, void* stream) {
+  return fgrpo_varlen_attn_fwd_ws(q, k, v, q_st, q_sh, k_st, k_sh, v_st, v_sh, cu, n_seq, T, Hq, Hkv, D, scale, causal, out,
+                                  lse, bounds_ws, bounds_valid, nullptr, 0, stream);
+}
+
+int fgrpo_varlen_attn_fwd_ws(const void* q, const void* k, const void* v, long long q_st, long long q_sh, long long k_st,
+                          long long k_sh, long long v_st, long long v_sh, const int32_t* cu, int n_seq, int T, int Hq,
+                          int Hkv, int D, float scale, int causal, void* out, float* lse, int32_t* bounds_ws,
+                          int bounds_valid, void* ws, size_t ws_bytes, void* stream) {
   hipStream_t st = (hipStream_t)stream;
   int rc = check_attn("varlen_attn_fwd", q, k, v, q_st, q_sh, k_st, k_sh, v_st, v_sh, cu, n_seq, T, Hq, Hkv, D, scale, bounds_ws);
   if (rc) return rc;
@@ -120,13 +198,37 @@ int fgrpo_varlen_attn_fwd(const void* q, const void* k, const void* v, long long
     rc = fgrpo_varlen_attn_bounds(cu, n_seq, T, causal, bounds_ws, stream);
     if (rc) return rc;
   }
-  return launch_query_side<FwdLauncher>(D, attn_heads_per_group(Hq / Hkv, T, n_seq), p, T, Hq, Hkv, bounds_ws, st);
+  const int hb = attn_heads_per_group(Hq / Hkv, T, n_seq);
+  SplitPlan sp = plan_query_split(T, n_seq, Hq, Hkv, D, causal, true);
+  const size_t need = query_split_bytes(sp, T, Hq, D, true);
+  if (!ws || need == 0) sp = SplitPlan();
+  else if (ws_bytes < need) return fail(FGRPO_ERR_WORKSPACE, "varlen_attn_fwd: workspace %zu < %zu", ws_bytes, need);
+  else if (!aligned16(ws)) return fail(FGRPO_ERR_ALIGN, "varlen_attn_fwd: workspace must be 16-byte aligned");
+  p.parts_q = sp.parts, p.per_q = sp.per;
+  p.part_q = (float*)ws;
+  p.part_ml = (float2*)((char*)ws + align256((size_t)sp.parts * T * Hq * D * 4));
+  rc = launch_query_side<FwdLauncher>(D, hb, p, T, Hq, Hkv, bounds_ws, st);
+  if (rc || sp.parts <= 1) return rc;
+  const unsigned blocks = (unsigned)(((long long)T * Hq * (D / 8) + 255) / 256);
+  if (D == 128) hipLaunchKernelGGL(attn_merge_fwd_kernel<128>, dim3(blocks), dim3(256), 0, st, p, 128 / hb);
+  else hipLaunchKernelGGL(attn_merge_fwd_kernel<64>, dim3(blocks), dim3(256), 0, st, p, 128 / hb);
+  HIP_TRY(hipGetLastError());
+  return 0;
 }
 
 int fgrpo_varlen_attn_bwd(const void* dout, const void* q, const void* k, const void* v, const void* out, const float* lse,
                           long long q_st, long long q_sh, long long k_st, long long k_sh, long long v_st, long long v_sh,
                           const int32_t* cu, int n_seq, int T, int Hq, int Hkv, int D, float scale, int causal, void* dq,
                           void* dk, void* dv, float* delta_ws, int32_t* bounds_ws, int bounds_valid, void* stream) {
+  return fgrpo_varlen_attn_bwd_ws(dout, q, k, v, out, lse, q_st, q_sh, k_st, k_sh, v_st, v_sh, cu, n_seq, T, Hq, Hkv, D, scale, causal, dq, dk, dv, delta_ws,
+                                  bounds_ws, bounds_valid, nullptr, 0, stream);
+}
+
+int fgrpo_varlen_attn_bwd_ws(const void* dout, const void* q, const void* k, const void* v, const void* out, const float* lse,
+                          long long q_st, long long q_sh, long long k_st, long long k_sh, long long v_st, long long v_sh,
+                          const int32_t* cu, int n_seq, int T, int Hq, int Hkv, int D, float scale, int causal, void* dq,
+                          void* dk, void* dv, float* delta_ws, int32_t* bounds_ws, int bounds_valid, void* ws,
+                             size_t ws_bytes, void* stream) {
   hipStream_t st = (hipStream_t)stream;
   int rc = check_attn("varlen_attn_bwd", q, k, v, q_st, q_sh, k_st, k_sh, v_st, v_sh, cu, n_seq, T, Hq, Hkv, D, scale, bounds_ws);
   if (rc) return rc;
@@ -146,11 +248,25 @@ int fgrpo_varlen_attn_bwd(const void* dout, const void* q, const void* k, const 
     rc = fgrpo_varlen_attn_bounds(cu, n_seq, T, causal, bounds_ws, stream);
     if (rc) return rc;
   }
-  rc = launch_query_side<DqLauncher>(D, attn_heads_per_group(Hq / Hkv, T, n_seq), p, T, Hq, Hkv, bounds_ws, st);
-  if (rc) return rc;
+  const int hb = attn_heads_per_group(Hq / Hkv, T, n_seq);
+  SplitPlan sq = plan_query_split(T, n_seq, Hq, Hkv, D, causal, false), sk = plan_key_split(T, n_seq, Hq, Hkv, D, causal);
+  const size_t need_q = query_split_bytes(sq, T, Hq, D, false), need = need_q + key_split_bytes(sk, T, Hkv, D);
+  if (!ws || need == 0) sq = sk = SplitPlan();
+  else if (ws_bytes < need) return fail(FGRPO_ERR_WORKSPACE, "varlen_attn_bwd: workspace %zu < %zu", ws_bytes, need);
+  else if (!aligned16(ws)) return fail(FGRPO_ERR_ALIGN, "varlen_attn_bwd: workspace must be 16-byte aligned");
   // the scalar offsets of the third form are 32-bit: (queries x heads of a group) x 4 bytes and the two bounds arrays
-  const bool dkv3_fits = (long long)T * (Hq / Hkv) * 4 < (1LL << 31) && (long long)T * 8 < (1LL << 31);
-  if (g_tune.attn_dkv != 1 && g_tune.attn_dkv != 2 && dkv3_fits) return launch_attn_dkv3(D, p, st);
+  const bool dkv3 = g_tune.attn_dkv != 1 && g_tune.attn_dkv != 2 && (long long)T * (Hq / Hkv) * 4 < (1LL << 31) && (long long)T * 8 < (1LL << 31);
+  if (!dkv3) sq = sk = SplitPlan();
+  p.parts_q = sq.parts, p.per_q = sq.per, p.parts_k = sk.parts, p.per_k = sk.per;
+  p.part_q = (float*)ws;
+  p.part_k = (float*)((char*)ws + need_q);
+  rc = launch_query_side<DqLauncher>(D, hb, p, T, Hq, Hkv, bounds_ws, st);
+  if (rc) return rc;
+  if (dkv3) {
+    rc = launch_attn_dkv3(D, p, st);
+    if (rc || (sq.parts <= 1 && sk.parts <= 1)) return rc;
+    return launch_attn_merge_bwd(D, p, 128 / hb, st);
+  }
   const dim3 grid_k(Hkv, (T + kAttnBQ - 1) / kAttnBQ);
   if (g_tune.attn_dkv == 1) {
     if (D == 128) hipLaunchKernelGGL(varlen_attn_dkv_kernel<128>, grid_k, dim3(256), 0, st, p);

@@ -8,9 +8,17 @@ namespace fgrpo {
 template <int HD, int KB>
 static int launch(const AttnParams& p, hipStream_t st) {
   const long long ranks = (long long)((p.T + 127) / 128) * (4 / KB);          // every 128-key tile of the launch order, in pieces of 32 KB keys
-  const int rc = raise_lds<varlen_attn_dkv3_kernel<HD, KB>>(kDkv3Lds<HD, KB>);
-  if (rc) return rc;
-  hipLaunchKernelGGL((varlen_attn_dkv3_kernel<HD, KB>), dim3((unsigned)(ranks * p.Hkv)), dim3(256), (kDkv3Lds<HD, KB>), st, p);
+  AttnParams a = p;
+  a.blocks_k = (int)(ranks * p.Hkv);
+  if (p.parts_k > 1) {
+    const int rc = raise_lds<varlen_attn_dkv3_kernel<HD, KB, true>>(kDkv3Lds<HD, KB>);
+    if (rc) return rc;
+    hipLaunchKernelGGL((varlen_attn_dkv3_kernel<HD, KB, true>), dim3((unsigned)a.blocks_k * p.parts_k), dim3(256), (kDkv3Lds<HD, KB>), st, a);
+  } else {
+    const int rc = raise_lds<varlen_attn_dkv3_kernel<HD, KB, false>>(kDkv3Lds<HD, KB>);
+    if (rc) return rc;
+    hipLaunchKernelGGL((varlen_attn_dkv3_kernel<HD, KB, false>), dim3((unsigned)a.blocks_k), dim3(256), (kDkv3Lds<HD, KB>), st, a);
+  }
   HIP_TRY(hipGetLastError());
   return 0;
 }
@@ -21,6 +29,17 @@ static int launch(const AttnParams& p, hipStream_t st) {
 // 57 -> 48; two blocks were slower at every size.
 int launch_attn_dkv3(int D, const AttnParams& p, hipStream_t st) {
   return D == 128 ? launch<128, 2>(p, st) : launch<64, 1>(p, st);
+}
+
+int attn_keyside_keys(int D) { return D == 128 ? 64 : 32; }
+
+int launch_attn_merge_bwd(int D, const AttnParams& p, int rb, hipStream_t st) {
+  const long long nq = p.parts_q > 1 ? (long long)p.T * p.Hq * (D / 8) : 0, nk = p.parts_k > 1 ? (long long)p.T * p.Hkv * (D / 8) : 0;
+  const dim3 grid((unsigned)((nq + 2 * nk + 255) / 256));
+  if (D == 128) hipLaunchKernelGGL((attn_merge_bwd_kernel<128, 64>), grid, dim3(256), 0, st, p, rb, nq, nk);
+  else hipLaunchKernelGGL((attn_merge_bwd_kernel<64, 32>), grid, dim3(256), 0, st, p, rb, nq, nk);
+  HIP_TRY(hipGetLastError());
+  return 0;
 }
 
 }  // namespace fgrpo

@@ -40,8 +40,9 @@ struct Api {
   FGRPO_ENTRY(fgrpo_grpo_step_chunked_workspace);
   FGRPO_ENTRY(fgrpo_grpo_step_chunked);
   FGRPO_ENTRY(fgrpo_scale_inplace);
-  FGRPO_ENTRY(fgrpo_varlen_attn_fwd);
-  FGRPO_ENTRY(fgrpo_varlen_attn_bwd);
+  FGRPO_ENTRY(fgrpo_varlen_attn_workspace);
+  FGRPO_ENTRY(fgrpo_varlen_attn_fwd_ws);
+  FGRPO_ENTRY(fgrpo_varlen_attn_bwd_ws);
 } api;
 
 void init(const std::unordered_map<std::string, uint64_t>& at) {
@@ -68,8 +69,9 @@ void init(const std::unordered_map<std::string, uint64_t>& at) {
   FGRPO_SET(fgrpo_grpo_step_chunked_workspace);
   FGRPO_SET(fgrpo_grpo_step_chunked);
   FGRPO_SET(fgrpo_scale_inplace);
-  FGRPO_SET(fgrpo_varlen_attn_fwd);
-  FGRPO_SET(fgrpo_varlen_attn_bwd);
+  FGRPO_SET(fgrpo_varlen_attn_workspace);
+  FGRPO_SET(fgrpo_varlen_attn_fwd_ws);
+  FGRPO_SET(fgrpo_varlen_attn_bwd_ws);
 }
 
 void check(int rc, const char* what) { TORCH_CHECK(rc == 0, "fgrpo ", what, " failed (", rc, "): ", api.fgrpo_last_error()); }
@@ -344,6 +346,12 @@ Tensor attn_operand(const Tensor& t, const char* name) {
 }
 int64_t bounds_numel(int64_t T) { return 2 * T + 2 * ((T + 127) / 128) + (T + 63) / 64 + (T + 31) / 32; }
 
+// scratch of a call on a batch with few tiles; none elsewhere
+Tensor attn_workspace(const Tensor& q, const Tensor& cu, int Hkv, bool causal, bool backward) {
+  const size_t n = api.fgrpo_varlen_attn_workspace((int)q.size(0), (int)cu.numel() - 1, (int)q.size(1), Hkv, (int)q.size(2), causal, backward);
+  return n > 0 ? workspace(n, q) : Tensor();
+}
+
 struct AttnArgs {
   Tensor cu, bounds;
   bool bounds_valid, causal;
@@ -358,11 +366,12 @@ struct VarlenAttention : torch::autograd::Function<VarlenAttention> {
     Tensor out = at::empty({T, Hq, D}, o), lse = at::empty({Hq, T}, o.dtype(at::kFloat));
     if (!a.bounds_valid) a.bounds = at::empty({bounds_numel(T)}, o.dtype(at::kInt));
     OnDevice d(q);
+    const Tensor ws = attn_workspace(q, a.cu, Hkv, a.causal, false);
     if (T > 0)
-      check(api.fgrpo_varlen_attn_fwd(ptr(q), ptr(k), ptr(v), q.stride(0), q.stride(1), k.stride(0), k.stride(1), v.stride(0),
+      check(api.fgrpo_varlen_attn_fwd_ws(ptr(q), ptr(k), ptr(v), q.stride(0), q.stride(1), k.stride(0), k.stride(1), v.stride(0),
                                       v.stride(1), a.cu.data_ptr<int32_t>(), (int)a.cu.numel() - 1, T, Hq, Hkv, D,
                                       (float)a.scale, a.causal, out.data_ptr(), fptr(lse), a.bounds.data_ptr<int32_t>(),
-                                      a.bounds_valid, d.stream()),
+                                      a.bounds_valid, ws.defined() ? ws.data_ptr() : nullptr, ws.defined() ? (size_t)ws.numel() : 0, d.stream()),
             "varlen_attn_fwd");
     if (ctx) {
       ctx->save_for_backward({q_, k_, v_, out, lse, a.cu, a.bounds});
@@ -383,12 +392,14 @@ struct VarlenAttention : torch::autograd::Function<VarlenAttention> {
     Tensor dq = at::empty({T, Hq, D}, o), dk = at::empty({T, Hkv, D}, o), dv = at::empty({T, Hkv, D}, o);
     Tensor delta = at::empty({Hq, T}, o.dtype(at::kFloat));
     OnDevice d(q);
+    const Tensor ws = attn_workspace(q, cu, Hkv, ctx->saved_data["causal"].toBool(), true);
     if (T > 0)
-      check(api.fgrpo_varlen_attn_bwd(ptr(dout), ptr(q), ptr(k), ptr(v), ptr(out), fptr(lse), q.stride(0), q.stride(1),
+      check(api.fgrpo_varlen_attn_bwd_ws(ptr(dout), ptr(q), ptr(k), ptr(v), ptr(out), fptr(lse), q.stride(0), q.stride(1),
                                       k.stride(0), k.stride(1), v.stride(0), v.stride(1), cu.data_ptr<int32_t>(),
                                       (int)cu.numel() - 1, T, Hq, Hkv, D, (float)ctx->saved_data["scale"].toDouble(),
                                       ctx->saved_data["causal"].toBool(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(),
-                                      fptr(delta), bounds.data_ptr<int32_t>(), 1, d.stream()),
+                                      fptr(delta), bounds.data_ptr<int32_t>(), 1, ws.defined() ? ws.data_ptr() : nullptr,
+                                      ws.defined() ? (size_t)ws.numel() : 0, d.stream()),
             "varlen_attn_bwd");
     return {dq, dk, dv, Tensor()};
   }

@@ -338,6 +338,15 @@ int fgrpo_varlen_attn_fwd(const void* q, const void* k, const void* v, long long
                           long long k_stride_t, long long k_stride_h, long long v_stride_t, long long v_stride_h,
                           const int32_t* cu_seqlens, int n_seq, int T, int Hq, int Hkv, int D, float softmax_scale,
                           int causal, void* out, float* lse, int32_t* bounds_ws, int bounds_valid, void* stream);
+/* The same with a workspace (16-byte aligned, fgrpo_varlen_attn_workspace bytes; 0 bytes: nothing to gain at this shape,
+ * ws may be null): a batch with too few tiles for the device has the keys of a tile dealt to several work-groups, whose
+ * fp32 partial results meet there.  Another order of the same sums; without a workspace nothing is dealt out. */
+size_t fgrpo_varlen_attn_workspace(int T, int n_seq, int Hq, int Hkv, int D, int causal, int backward);
+int fgrpo_varlen_attn_fwd_ws(const void* q, const void* k, const void* v, long long q_stride_t, long long q_stride_h,
+                             long long k_stride_t, long long k_stride_h, long long v_stride_t, long long v_stride_h,
+                             const int32_t* cu_seqlens, int n_seq, int T, int Hq, int Hkv, int D, float softmax_scale,
+                             int causal, void* out, float* lse, int32_t* bounds_ws, int bounds_valid, void* ws,
+                             size_t ws_bytes, void* stream);
 
 /* Backward of the above (autograd of flash_attn_varlen_func in the reference).  dout, out
  * [T, Hq, D] bf16 contiguous; dq [T, Hq, D], dk / dv [T, Hkv, D] bf16 contiguous;
@@ -348,6 +357,12 @@ int fgrpo_varlen_attn_bwd(const void* dout, const void* q, const void* k, const 
                           long long k_stride_h, long long v_stride_t, long long v_stride_h, const int32_t* cu_seqlens,
                           int n_seq, int T, int Hq, int Hkv, int D, float softmax_scale, int causal, void* dq, void* dk,
                           void* dv, float* delta_ws, int32_t* bounds_ws, int bounds_valid, void* stream);
+int fgrpo_varlen_attn_bwd_ws(const void* dout, const void* q, const void* k, const void* v, const void* out,
+                             const float* lse, long long q_stride_t, long long q_stride_h, long long k_stride_t,
+                             long long k_stride_h, long long v_stride_t, long long v_stride_h, const int32_t* cu_seqlens,
+                             int n_seq, int T, int Hq, int Hkv, int D, float softmax_scale, int causal, void* dq, void* dk,
+                             void* dv, float* delta_ws, int32_t* bounds_ws, int bounds_valid, void* ws, size_t ws_bytes,
+                             void* stream);
 
 #ifdef __cplusplus
 }
