@@ -134,12 +134,30 @@ int check_operands(const GemmOperands& g, int bk) {
   return 0;
 }
 
-int launch_convert(const void* src, int src_is_f32, long long ld_src, int R, int Cn, int Rpad, int Cpad, bf16_t* hi,
-                   bf16_t* lo, long long ld_dst, int transpose, hipStream_t st) {
-  ConvertParams p{src, src_is_f32, ld_src, R, Cn, Rpad, Cpad, hi, lo, ld_dst, transpose};
-  dim3 grid((unsigned)((Cpad + 63) / 64), (unsigned)((Rpad + 63) / 64));
-  if (transpose ? (Rpad > ld_dst) : (Cpad > ld_dst)) return fail(FGRPO_ERR_BAD_ARG, "convert: padded extent exceeds ld");
-  hipLaunchKernelGGL(convert_pad_kernel, grid, dim3(256), 0, st, p);
+ConvertJob convert_job(const void* src, long long ld_src, int R, int Cn) {
+  ConvertJob j;
+  memset(&j, 0, sizeof(j));
+  j.src = src, j.ld_src = ld_src, j.R = R, j.Cn = Cn;
+  return j;
+}
+
+int launch_convert(int src_is_f32, ConvertJob a, ConvertJob b, hipStream_t st) {
+  ConvertParams p{{a, b}, src_is_f32};
+  for (ConvertJob& j : p.job) {
+    if (!j.src || (!j.hi && !j.t_hi)) {
+      j.tiles_c = 1, j.tiles = 0;
+      continue;
+    }
+    if ((j.hi && j.Cpad > j.ld) || (j.t_hi && j.Rpad > j.ld_t)) return fail(FGRPO_ERR_BAD_ARG, "convert: padded extent exceeds ld");
+    const int cols = j.hi && j.Cpad > j.Cn ? j.Cpad : j.Cn, rows = j.t_hi && j.Rpad > j.R ? j.Rpad : j.R;
+    j.tiles_c = (cols + 63) / 64;
+    const long long tiles = (long long)j.tiles_c * ((rows + 63) / 64);
+    if (tiles >= (1LL << 30)) return fail(FGRPO_ERR_UNSUPPORTED, "convert: matrix too large");
+    j.tiles = (int)tiles;
+  }
+  const unsigned blocks = (unsigned)(p.job[0].tiles + p.job[1].tiles);
+  if (blocks == 0) return 0;
+  hipLaunchKernelGGL(convert_pad_kernel, dim3(blocks), dim3(256), 0, st, p);
   HIP_TRY(hipGetLastError());
   return 0;
 }
@@ -275,19 +293,22 @@ void plan_fwd(const Tuning& tn, FwdPlan& pl, void* ws, int T, int H, int V, int 
 
 // Fill the operands of the logits contraction: A = weight side, B = hidden side.
 int stage_logit_operands(GemmOperands& g, const void* hidden, const void* weight, int T, int H, int V, int dtype,
-                         bool copy_ops, int Hp, bf16_t* w_hi, bf16_t* w_lo, bf16_t* h_hi, bf16_t* h_lo, hipStream_t st) {
+                         bool copy_ops, int Hp, bf16_t* w_hi, bf16_t* w_lo, bf16_t* h_hi, bf16_t* h_lo, hipStream_t st,
+                         const ConvertJob* wT = nullptr, const ConvertJob* hT = nullptr) {
+  // wT, hT: transposed copies wanted of the two (backward), made by the same launch
+  ConvertJob jw = wT ? *wT : convert_job(weight, H, V, H), jh = hT ? *hT : convert_job(hidden, H, T, H);
   g.M = V;
   g.N = T;
   if (!copy_ops) {
     g.nseg = 1;
     g.seg[0] = GemmSeg{(const bf16_t*)weight, (const bf16_t*)hidden, H};
     g.lda = g.ldb = H;
-    return 0;
+    return launch_convert(dtype == FGRPO_F32, jw, jh, st);
   }
   const int f32 = (dtype == FGRPO_F32);
-  int rc = launch_convert(weight, f32, H, V, H, V, Hp, w_hi, f32 ? w_lo : nullptr, Hp, 0, st);
-  if (rc) return rc;
-  rc = launch_convert(hidden, f32, H, T, H, T, Hp, h_hi, f32 ? h_lo : nullptr, Hp, 0, st);
+  jw.hi = w_hi, jw.lo = f32 ? w_lo : nullptr, jh.hi = h_hi, jh.lo = f32 ? h_lo : nullptr;
+  jw.ld = jh.ld = Hp, jw.Cpad = jh.Cpad = Hp;
+  int rc = launch_convert(f32, jw, jh, st);
   if (rc) return rc;
   g.lda = g.ldb = Hp;
   if (f32) {
@@ -357,8 +378,58 @@ int run_store_gemm_kmajor(const Tuning& tn, StoreParams p, bool akm, bool bkm, h
   return launch_store_kmajor(akm, bkm, p, st);
 }
 
-int run_store_gemm(const Tuning& tn, StoreParams p, int variant, hipStream_t st) {
+// A small product (128 x 128 tiles, few of them) is one serial walk over its contraction, 0.65 us a K step: 33 us for each
+// gradient of 643 tokens x 1000 entries x 64.  Contracted in pieces it ends sooner for 4 us of one more launch and the
+// fp32 pieces through memory.  Pieces: whole 64-wide K steps, the same range of every segment; 0 = one piece.  fp32
+// operands (three segments) only: a bf16 token's gradient row does not depend on how many tokens there are.
+int small_split(int M, int N, int K, int nseg, size_t max_elems, int* kchunk) {
+  if (nseg != 3) return 0;
+  const int steps = K / 64;
+  const long long tiles = (long long)((M + 127) / 128) * ((N + 127) / 128), ld = round_up(N, 4);
+  int best = 0;
+  double least = 0.85 * steps * nseg * 0.65;
+  for (int ks = 2; ks <= 16 && ks <= steps; ++ks) {
+    if (tiles * ks > 2LL * num_cus() || (size_t)ks * M * ld > max_elems) break;
+    const int per = (steps + ks - 1) / ks, used = (steps + per - 1) / per;
+    const double cost = per * nseg * 0.65 + 4.0 + (double)used * M * ld * 8.0 / 3.0e6;
+    if (cost < least) least = cost, best = used, *kchunk = per * 64;
+  }
+  return best;
+}
+size_t small_split_elems(const Tuning& tn, int M, int N, int K, int nseg) {
+  int kchunk = 0;
+  if (pick_variant(tn, tn.gemm_variant, M, N) != 4) return 0;
+  return (size_t)small_split(M, N, K, nseg, (size_t)1 << 40, &kchunk) * M * round_up(N, 4);
+}
+
+// part: room for part_elems floats of pieces (null: none)
+int run_store_gemm(const Tuning& tn, StoreParams p, int variant, hipStream_t st, float* part = nullptr, size_t part_elems = 0) {
   variant = pick_variant(tn, variant, p.g.M, p.g.N);
+  if (variant == 4 && part && p.g.a_blk == 0 && !p.row_scale && !p.alpha_dev) {
+    int kchunk = 0;
+    const int ks = small_split(p.g.M, p.g.N, p.g.seg[0].K, p.g.nseg, part_elems, &kchunk);
+    for (int s = 1; s < p.g.nseg; ++s)
+      if (p.g.seg[s].K != p.g.seg[0].K) return fail(FGRPO_ERR_BAD_ARG, "gemm: segments of different length");
+    if (ks > 1) {
+      int rc = check_operands(p.g, kCfg[4].bk);
+      if (rc) return rc;
+      StoreParams q = p;
+      q.ksplit = ks, q.kchunk = kchunk;
+      q.ldc = round_up(p.g.N, 4);
+      q.part_slice = (long long)p.g.M * q.ldc;
+      q.c_in = nullptr, q.c_out_bf16 = nullptr, q.c_out_f32 = part;
+      q.tiles_m = (p.g.M + kCfg[4].bm - 1) / kCfg[4].bm;
+      q.tiles_n = (p.g.N + kCfg[4].bn - 1) / kCfg[4].bn;
+      q.wide_stores = 1;
+      q.nblocks = q.tiles_m * q.tiles_n * ks;
+      rc = launch_store_small_split(q, st);
+      if (rc) return rc;
+      hipLaunchKernelGGL(small_split_sum_kernel, dim3((unsigned)(((long long)p.g.M * p.g.N + 255) / 256)), dim3(256), 0, st, part, ks,
+                         q.part_slice, q.ldc, p.g.M, p.g.N, p.ldc, p.c_in, p.c_out_f32, p.c_out_bf16);
+      HIP_TRY(hipGetLastError());
+      return 0;
+    }
+  }
   if (p.g.a_blk != 0 && variant != 6 && variant != 7 && variant != 8) variant = 8;  // loops that know the layout
   const CfgInfo& c = kCfg[variant];
   int rc = check_operands(p.g, c.bk);
@@ -386,6 +457,8 @@ struct BwdPlan {
   bf16_t *tv_hi, *tv_lo, *vt_hi, *vt_lo;      // dS panels
   float* bias32;
   float* dh_acc;                              // [T x H] fp32 when more than one panel
+  float* part;                                // pieces of a split contraction (small problems), part_elems of them
+  size_t part_elems;
   size_t bytes;
 };
 
@@ -482,6 +555,11 @@ void plan_bwd(const Tuning& tn, BwdPlan& pl, void* ws, int T, int H, int V, int 
   }
   pl.bias32 = has_bias ? cv.take<float>((size_t)V) : nullptr;
   pl.dh_acc = (want_dh && pl.npanels > 1 && !pl.f32) ? cv.take<float>((size_t)T * H) : nullptr;
+  const int rows = V < pl.panel ? V : pl.panel, nseg = pl.f32 ? 3 : 1;
+  const size_t e_dh = want_dh && !pl.kmajor_dh ? small_split_elems(tn, T, H, (int)round_up(rows, pl.bm), nseg) : 0;
+  const size_t e_dw = want_dw && !pl.kmajor ? small_split_elems(tn, rows, H, pl.tiles_t * pl.bn, nseg) : 0;
+  pl.part_elems = e_dh > e_dw ? e_dh : e_dw;
+  pl.part = pl.part_elems ? cv.take<float>(pl.part_elems) : nullptr;
   pl.bytes = cv.total();
 }
 
@@ -732,23 +810,18 @@ int fgrpo_lmhead_bwd(const void* hidden, const void* weight, const void* bias, c
 
   DsParams d;
   memset(&d, 0, sizeof(d));
+  // with the contraction-major copies for the two gradient GEMMs
+  ConvertJob wT = convert_job(weight, H, V, H), hT = convert_job(hidden, H, T, H);
+  if (want_dh && !pl.kmajor_dh) wT.t_hi = pl.wT_hi, wT.t_lo = pl.wT_lo, wT.ld_t = wT.Rpad = pl.Vpad;
+  if (want_dw && !pl.kmajor) hT.t_hi = pl.hT_hi, hT.t_lo = pl.hT_lo, hT.ld_t = hT.Rpad = pl.Tpad;
   int rc = stage_logit_operands(d.g, hidden, weight, T, H, V, dtype, pl.copy_ops, pl.Hp, pl.w_hi, pl.w_lo, pl.h_hi,
-                                pl.h_lo, st);
+                                pl.h_lo, st, &wT, &hT);
   if (rc) return rc;
   rc = check_operands(d.g, kCfg[pl.variant].bk);
   if (rc) return rc;
   if (bias) {
     hipLaunchKernelGGL(to_f32_kernel, dim3((V + 255) / 256), dim3(256), 0, st, bias, f32, pl.bias32, V);
     HIP_TRY(hipGetLastError());
-  }
-  // contraction-major copies for the two gradient GEMMs
-  if (want_dh && !pl.kmajor_dh) {
-    rc = launch_convert(weight, f32, H, V, H, pl.Vpad, H, pl.wT_hi, pl.wT_lo, pl.Vpad, 1, st);
-    if (rc) return rc;
-  }
-  if (want_dw && !pl.kmajor) {
-    rc = launch_convert(hidden, f32, H, T, H, pl.Tpad, H, pl.hT_hi, pl.hT_lo, pl.Tpad, 1, st);
-    if (rc) return rc;
   }
   d.bias = bias ? pl.bias32 : nullptr;
   d.labels = (const long long*)labels;
@@ -826,7 +899,7 @@ int fgrpo_lmhead_bwd(const void* hidden, const void* weight, const void* bias, c
       }
       {
         PhaseScope ph(kPhaseDh, st);
-        rc = pl.kmajor_dh ? run_store_gemm_kmajor(tn, s, false, true, st) : run_store_gemm(tn, s, tn.gemm_variant, st);
+        rc = pl.kmajor_dh ? run_store_gemm_kmajor(tn, s, false, true, st) : run_store_gemm(tn, s, tn.gemm_variant, st, pl.part, pl.part_elems);
       }
       if (rc) return rc;
     }
@@ -861,7 +934,7 @@ int fgrpo_lmhead_bwd(const void* hidden, const void* weight, const void* bias, c
         s.c_out_bf16 = (bf16_t*)dW_out + (size_t)v0 * H;
       {
         PhaseScope ph(kPhaseDw, st);
-        rc = pl.kmajor ? run_store_gemm_kmajor(tn, s, true, true, st) : run_store_gemm(tn, s, tn.gemm_variant, st);
+        rc = pl.kmajor ? run_store_gemm_kmajor(tn, s, true, true, st) : run_store_gemm(tn, s, tn.gemm_variant, st, pl.part, pl.part_elems);
       }
       if (rc) return rc;
     }

@@ -165,10 +165,10 @@ __device__ __forceinline__ void zero_acc(f32x16_t (&acc)[C::TM][C::TN]) {
 // acc += A[row0 : row0+BM, :] * B[col0 : col0+BN, :]^T over all segments.
 // Must be called by every thread of the work-group (it contains barriers).  On
 // return all LDS reads have completed and a barrier has been passed, so the
-// caller may reuse `smem`.
+// caller may reuse `smem`.  klen > 0: only the range [k0, k0 + klen) of every segment.
 template <class C>
 __device__ __forceinline__ void gemm_mainloop(const GemmOperands& g, int row0, int col0, char* smem,
-                                              f32x16_t (&acc)[C::TM][C::TN]) {
+                                              f32x16_t (&acc)[C::TM][C::TN], int k0 = 0, int klen = 0) {
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = tid >> 6;
@@ -196,9 +196,9 @@ __device__ __forceinline__ void gemm_mainloop(const GemmOperands& g, int row0, i
   const int fr_b = C::BM * C::ROWB + (wn * C::WTN + (lane & 31)) * C::ROWB + (lane >> 5) * 16;
 
   for (int s = 0; s < g.nseg; ++s) {
-    const char* Ab = (const char*)(g.seg[s].A + (long long)row0 * g.lda);
-    const char* Bb = (const char*)(g.seg[s].B + (long long)col0 * g.ldb);
-    const int nk = g.seg[s].K / C::BK;
+    const char* Ab = (const char*)(g.seg[s].A + (long long)row0 * g.lda + k0);
+    const char* Bb = (const char*)(g.seg[s].B + (long long)col0 * g.ldb + k0);
+    const int nk = (klen > 0 ? klen : g.seg[s].K) / C::BK;
 
     u32x4_t ra[C::PA], rb[C::PB];
 #pragma unroll

@@ -755,8 +755,9 @@ __device__ __forceinline__ void store_tile_lds(const StoreParams& p, f32x16_t (&
   }
 }
 
-// SPLITK (a K-contiguous, column-blocked A and a contraction-major B only): the tiles of a device round that would
-// otherwise run nearly empty are contracted in ksplit pieces by ksplit work-groups each.
+// SPLITK: the tiles of a device round that would otherwise run nearly empty are contracted in ksplit pieces by ksplit
+// work-groups each (a K-contiguous, column-blocked A and a contraction-major B: dHidden's last round; both operands
+// K-contiguous: the products of a small problem, piece ks taking the same K range of every segment).
 template <class C, bool AKM = false, bool BKM = false, bool SPLITK = false>
 __global__ __launch_bounds__(C::NT, C::OCC) void gemm_store_kernel(const StoreParams p0) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
@@ -764,7 +765,20 @@ __global__ __launch_bounds__(C::NT, C::OCC) void gemm_store_kernel(const StorePa
   int wm, wn;
   wave_coords<C, kMi16<C> && (AKM || BKM)>(wave, wm, wn);
 
-  if constexpr (SPLITK) {
+  if constexpr (SPLITK && !BKM) {
+    StoreParams p = p0;
+    const int tiles = p.tiles_m * p.tiles_n;
+    const int ks = (int)blockIdx.x / tiles, t = (int)blockIdx.x - ks * tiles;
+    const int row0 = t % p.tiles_m * C::BM, col0 = t / p.tiles_m * C::BN;
+    const int k0 = ks * p.kchunk;
+    const int klen = (p.g.seg[0].K - k0) < p.kchunk ? (p.g.seg[0].K - k0) : p.kchunk;      // > 0: the launcher sees to it
+    f32x16_t acc[C::TM][C::TN];
+    zero_acc<C>(acc);
+    gemm_mainloop<C>(p0.g, row0, col0, smem, acc, k0, klen);
+    p.c_out_f32 += (long long)ks * p.part_slice;
+    store_tile_lds<C, false, false>(p, acc, p.alpha, row0, col0, wm, wn, lane, wave, smem);
+    return;
+  } else if constexpr (SPLITK) {
     static_assert(!AKM && BKM && kMi16<C>, "split contraction: dHidden's layouts on the 16x16x32 tile");
     StoreParams p = p0;
     const int lid = xcd_contiguous_id(blockIdx.x, gridDim.x);

@@ -64,55 +64,72 @@ inline void launch_fwd_combine(const CombineParams& c, hipStream_t st) {
 }
 
 // ---------------------------------------------------------------------------
-// Operand preparation: copy / transpose a [R x Cn] matrix (fp32 or bf16) into a
-// zero-padded bf16 buffer, optionally also emitting the bf16 low half of an fp32
-// source (x ~= hi + lo).  Destination is [Rpad x ld] (or [Cpad x ld] transposed).
+// Operand preparation: a [R x Cn] matrix (fp32 or bf16) into zero-padded bf16 copies, as it lies and / or transposed,
+// optionally also the bf16 low half of an fp32 source (x ~= hi + lo).  One launch takes both operands of the LM head and
+// reads each once: the matrices are small, and a launch of its own for each of the six copies of a backward cost 7 us
+// (most of it sixteen loads one behind the other; all sixteen are requested first now).
 // ---------------------------------------------------------------------------
-struct ConvertParams {
-  const void* src;
-  int src_is_f32;
+struct ConvertJob {
+  const void* src;        // null: no such job
   long long ld_src;
-  int R, Cn;          // logical source shape
-  int Rpad, Cpad;     // padded extents written
-  bf16_t* hi;
-  bf16_t* lo;         // or null
-  long long ld_dst;
-  int transpose;
+  int R, Cn;              // source shape
+  int Cpad;               // columns of the straight copy written (zeros from Cn on)
+  int Rpad;               // columns of the transposed copy written (zeros from R on)
+  bf16_t *hi, *lo;        // straight copy [R][ld], or null; lo null: no low half
+  long long ld;
+  bf16_t *t_hi, *t_lo;    // transposed copy [Cn][ld_t], or null
+  long long ld_t;
+  int tiles_c, tiles;     // 64 x 64 tiles along the columns / in all
+};
+struct ConvertParams {
+  ConvertJob job[2];
+  int src_is_f32;
 };
 
 __global__ __launch_bounds__(256) void convert_pad_kernel(const ConvertParams p) {
-  __shared__ float th[64][65];
-  __shared__ float tl[64][65];
-  const int r0 = blockIdx.y * 64, c0 = blockIdx.x * 64;
+  __shared__ float tile[64][65];
+  const bool second = (int)blockIdx.x >= p.job[0].tiles;
+  const ConvertJob& j = second ? p.job[1] : p.job[0];
+  const int w = (int)blockIdx.x - (second ? p.job[0].tiles : 0);
+  const int r0 = w / j.tiles_c * 64, c0 = w % j.tiles_c * 64;
   const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;  // 64 x 4
-  for (int rr = ty; rr < 64; rr += 4) {
-    const int r = r0 + rr, c = c0 + tx;
-    float v = 0.f;
-    if (r < p.R && c < p.Cn) {
-      const long long o = (long long)r * p.ld_src + c;
-      v = p.src_is_f32 ? ((const float*)p.src)[o] : bf16_to_f32(((const bf16_t*)p.src)[o]);
+  float v[16];
+  {
+    const int c = c0 + tx;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const int r = r0 + ty + 4 * i;
+      const long long o = (long long)r * j.ld_src + c;
+      const bool ok = r < j.R && c < j.Cn;
+      v[i] = !ok ? 0.f : p.src_is_f32 ? ((const float*)j.src)[o] : bf16_to_f32(((const bf16_t*)j.src)[o]);
     }
-    const float h = bf16_to_f32(f32_to_bf16_rn(v));
-    th[rr][tx] = h;
-    tl[rr][tx] = v - h;
   }
-  __syncthreads();
-  if (!p.transpose) {
-    for (int rr = ty; rr < 64; rr += 4) {
-      const int r = r0 + rr, c = c0 + tx;
-      if (r < p.Rpad && c < p.Cpad) {
-        const long long o = (long long)r * p.ld_dst + c;
-        p.hi[o] = f32_to_bf16_rn(th[rr][tx]);
-        if (p.lo) p.lo[o] = f32_to_bf16_rn(tl[rr][tx]);
+  auto low = [](float x) { return f32_to_bf16_rn(x - bf16_to_f32(f32_to_bf16_rn(x))); };
+  if (j.hi) {
+    const int c = c0 + tx;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const int r = r0 + ty + 4 * i;
+      if (r < j.R && c < j.Cpad) {
+        const long long o = (long long)r * j.ld + c;
+        j.hi[o] = f32_to_bf16_rn(v[i]);
+        if (j.lo) j.lo[o] = low(v[i]);
       }
     }
-  } else {
-    for (int cc = ty; cc < 64; cc += 4) {
-      const int c = c0 + cc, r = r0 + tx;
-      if (c < p.Cpad && r < p.Rpad) {
-        const long long o = (long long)c * p.ld_dst + r;
-        p.hi[o] = f32_to_bf16_rn(th[tx][cc]);
-        if (p.lo) p.lo[o] = f32_to_bf16_rn(tl[tx][cc]);
+  }
+  if (j.t_hi) {
+#pragma unroll
+    for (int i = 0; i < 16; ++i) tile[ty + 4 * i][tx] = v[i];
+    __syncthreads();
+    const int r = r0 + tx;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const int c = c0 + ty + 4 * i;
+      if (c < j.Cn && r < j.Rpad) {
+        const long long o = (long long)c * j.ld_t + r;
+        const float x = tile[tx][ty + 4 * i];
+        j.t_hi[o] = f32_to_bf16_rn(x);
+        if (j.t_lo) j.t_lo[o] = low(x);
       }
     }
   }
@@ -340,6 +357,27 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* part, i
   o.x = pack_bf16x2(s.x * a, s.y * a);
   o.y = pack_bf16x2(s.z * a, s.w * a);
   *(uint2*)(out + (long long)m * ld + n) = o;
+}
+
+// The same for the small products, whose slices have a row pitch of their own: out = c_in + sum of the slices, fp32 or bf16.
+__global__ __launch_bounds__(256) void small_split_sum_kernel(const float* part, int ksplit, long long slice, long long ld_part,
+                                                              int M, int N, long long ldc, const float* c_in,
+                                                              float* out_f32, bf16_t* out_bf16) {
+  const long long q = (long long)blockIdx.x * 256 + threadIdx.x;
+  if (q >= (long long)M * N) return;
+  const int m = (int)(q / N), n = (int)(q - (long long)m * N);
+  const float* src = part + (long long)m * ld_part + n;
+  const long long o = (long long)m * ldc + n;
+  float s = c_in ? c_in[o] : 0.f;
+  for (int k0 = 0; k0 < ksplit; k0 += 8) {                // eight loads in flight
+    float v[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) v[k] = k0 + k < ksplit ? src[(long long)(k0 + k) * slice] : 0.f;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) s += v[k];
+  }
+  if (out_f32) out_f32[o] = s;
+  else out_bf16[o] = f32_to_bf16_rn(s);
 }
 
 // dbias from the kept numerators: out[v] = sum_t a_t * E'[t][v].  One block owns 64 columns; its four row groups

@@ -126,3 +126,21 @@ def test_gradient_products_on_tiles_with_a_half_outside(dev, M, N, a_km):
     out = ops.gemm_kmajor(A.to(dev), B.to(dev), a_km, not a_km, M, N, K).cpu().double()
     Ad, Bd = (A[:, :M].double().t(), B.double()) if a_km else (A.double(), B[:, :N].double().t())
     assert (out - Ad @ Bd.t()).abs().max() <= 2e-4
+
+
+@pytest.mark.parametrize("T,H,V", [(100, 64, 500), (1, 64, 4099), (129, 96, 8000), (643, 64, 1000), (2000, 256, 777), (700, 72, 3001)])
+def test_fp32_gradients_of_small_heads(dev, T, H, V):
+    """Both gradients with the contraction in pieces, over segments of 64 and ragged ends.  Against fp64; products of
+    operands split into two bf16 halves: 2^-16 of the norm each way, tripled for the sums of dLogits' own error."""
+    from fgrpo import ops
+    g = torch.Generator().manual_seed(T + V)
+    h, w = torch.randn(T, H, generator=g), torch.randn(V, H, generator=g) * 0.1
+    y = torch.randint(0, V, (T,), generator=g)
+    gt = torch.randn(T, generator=g)
+    hd, wd = h.double().requires_grad_(True), w.double().requires_grad_(True)
+    lp = torch.log_softmax(hd @ wd.t(), 1).gather(1, y[:, None])[:, 0]
+    want = torch.autograd.grad(lp, (hd, wd), gt.double())
+    hg, wg = h.to(dev).requires_grad_(True), w.to(dev).requires_grad_(True)
+    got = torch.autograd.grad(ops.lmhead_logprob(hg, wg, None, y.to(dev))[0], (hg, wg), gt.to(dev))
+    for a, b in zip(got, want):
+        assert (a.cpu().double() - b).norm() <= 6 * 2 ** -16 * b.norm()
