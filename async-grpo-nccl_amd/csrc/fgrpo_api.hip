@@ -603,19 +603,24 @@ KeepAux keep_aux_of(void* keep, int T, int V) {
 // The pre-pass of the kept forward: the reference's sample of the vocabulary - the plain forward kernel over the
 // first rows of W; only the maxima of its per-split partials are used - then one dot product per token.
 // `p`: the forward's parameters for these tokens (operands staged, bias, labels, temperature); part: scratch for
-// min(2, nsplit) x T partials.
+// min(kPrepassSplits, nsplit) x T partials.  A small batch takes the 128 x 128 tile: its few 256 x 256 tiles would each be
+// one serial walk over H on a device otherwise idle (777 tokens, H = 1536: 46 us; so 26), while more than two of
+// the small ones per CU gain nothing (32768 tokens: 53 us on the large).
+constexpr int kPrepassSplits = 4;
 int keep_prepass(const FwdParams& p, const void* hidden, const void* weight, const int64_t* labels, int T, int H, int V,
                  int nsplit, float4* part, const KeepAux& aux, int nflags, hipStream_t st) {
   FwdParams sp = p;
   const int vs = V < kKeepSampleRows ? V : kKeepSampleRows;
   sp.g.M = vs;
   sp.g.N = T;
-  sp.tiles_v = (vs + kCfg[8].bm - 1) / kCfg[8].bm;
-  sp.tiles_t = (T + kCfg[8].bn - 1) / kCfg[8].bn;
+  const long long small_tiles = (long long)((vs + kCfg[4].bm - 1) / kCfg[4].bm) * ((T + kCfg[4].bn - 1) / kCfg[4].bn);
+  const int variant = small_tiles <= 2LL * num_cus() ? 4 : 8;
+  sp.tiles_v = (vs + kCfg[variant].bm - 1) / kCfg[variant].bm;
+  sp.tiles_t = (T + kCfg[variant].bn - 1) / kCfg[variant].bn;
   sp.nsplit = sp.tiles_v < nsplit ? sp.tiles_v : nsplit;
   sp.part = part;
   sp.keep = nullptr;
-  int rc = launch_fwd_variant(8, sp, st);
+  int rc = launch_fwd_variant(variant, sp, st);
   if (rc) return rc;
   KeepRefParams r{(const bf16_t*)hidden, (const bf16_t*)weight, p.bias, (const long long*)labels, T, H, V, p.inv_temp,
                   part, sp.nsplit, aux.ref2, aux.xy, aux.flag, nflags};
@@ -1532,7 +1537,7 @@ void plan_chunked(const Tuning& tn, ChunkedPlan& pl, void* ws, int T, int H, int
   pl.ref2 = cv.take<float>((size_t)T);
   pl.xy = cv.take<float>((size_t)T);
   pl.flags = cv.take<int>((size_t)pl.nchunks);
-  pl.pre_part = cv.take<float4>(2 * (size_t)T);
+  pl.pre_part = cv.take<float4>(kPrepassSplits * (size_t)T);
   pl.pre_xt = cv.take<float>((size_t)T);
   pl.pre_bias32 = has_bias ? cv.take<float>((size_t)V) : nullptr;
   pl.bytes = cv.total();
@@ -1615,7 +1620,7 @@ int fgrpo_grpo_step_chunked(const void* hidden, const void* weight, const void* 
     bp.inv_temp = inv_temp;
     bp.group_t = tn.fwd_group_t > 0 ? tn.fwd_group_t : 1;
     bp.xt = pl.pre_xt;
-    rc = keep_prepass(bp, hidden, weight, labels, T, H, V, 2, pl.pre_part, KeepAux{pl.ref2, pl.xy, pl.flags, true},
+    rc = keep_prepass(bp, hidden, weight, labels, T, H, V, kPrepassSplits, pl.pre_part, KeepAux{pl.ref2, pl.xy, pl.flags, true},
                       pl.nchunks, st);
     if (rc) return rc;
   }
