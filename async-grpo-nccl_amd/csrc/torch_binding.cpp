@@ -131,7 +131,7 @@ enum GradMode { kNone = 0, kRecompute = 1, kWhole = 2, kChunked = 3 };
 
 struct StepArgs {
   Tensor labels, old_lp, adv, ref_lp, cu;      // shifted labels; per-token inputs; segment boundaries (sample mean)
-  double temperature, clip_low, clip_high, clip_c, kl_beta, denom;
+  double inv_temp, clip_low, clip_high, clip_c, kl_beta, denom;
   bool by_sample;
   int64_t panel_hint;
   int mode, chunk_tokens;
@@ -144,7 +144,7 @@ struct Grads {
 
 // Gradients of the projection by the recomputing pair or on the kept numerators, given g = d loss / d lp.
 Grads lmhead_backward(const Tensor& h, const Tensor& w, const Tensor& b, const Tensor& y, const Tensor& lse, const Tensor& g,
-                      const Tensor& gout, double temperature, int64_t hint, const Tensor& kept, bool nh, bool nw, bool nb) {
+                      const Tensor& gout, double inv_temp, int64_t hint, const Tensor& kept, bool nh, bool nw, bool nb) {
   const int T = (int)h.size(0), H = (int)h.size(1), V = (int)w.size(0), code = dtype_code(w);
   Grads r;
   if (nh) r.dh = at::empty_like(h, at::MemoryFormat::Contiguous);
@@ -157,14 +157,14 @@ Grads lmhead_backward(const Tensor& h, const Tensor& w, const Tensor& b, const T
   if (kept.defined()) {
     Tensor ws = workspace(api.fgrpo_lmhead_bwd_kept_workspace(T, H, V, code), h);
     check(api.fgrpo_lmhead_bwd_kept(ptr(h), ptr(w), ptr(b), y.data_ptr<int64_t>(), fptr(lse), fptr(g), fptr(scale),
-                                    (float)(1.0 / temperature), T, H, V, code, kept.data_ptr(), (size_t)kept.numel(),
+                                    (float)inv_temp, T, H, V, code, kept.data_ptr(), (size_t)kept.numel(),
                                     const_cast<void*>(ptr(r.dh)), const_cast<void*>(ptr(r.dw)), const_cast<void*>(ptr(r.db)),
                                     ws.data_ptr(), (size_t)ws.numel(), d.stream()),
           "lmhead_bwd_kept");
   } else {
     Tensor ws = workspace(api.fgrpo_lmhead_bwd_workspace(T, H, V, code, hint), h);
     check(api.fgrpo_lmhead_bwd(ptr(h), ptr(w), ptr(b), y.data_ptr<int64_t>(), fptr(lse), fptr(g), fptr(scale),
-                               (float)(1.0 / temperature), T, H, V, code, const_cast<void*>(ptr(r.dh)),
+                               (float)inv_temp, T, H, V, code, const_cast<void*>(ptr(r.dh)),
                                const_cast<void*>(ptr(r.dw)), const_cast<void*>(ptr(r.db)), hint, ws.data_ptr(),
                                (size_t)ws.numel(), d.stream()),
           "lmhead_bwd");
@@ -186,7 +186,7 @@ StepOut step_forward(const Tensor& h, const Tensor& w, const Tensor& b, const St
   for (Tensor* t : {&o.lp, &o.ent, &o.lse, &o.g, &o.lr, &o.c1, &o.l1, &o.l2}) *t = at::empty({T}, f32);
   Tensor scal = at::empty({4}, f32);
   o.loss = at::empty({}, f32);
-  const float it = (float)(1.0 / a.temperature);
+  const float it = (float)a.inv_temp;
   const int nseq = a.cu.defined() ? (int)a.cu.numel() - 1 : 0;
   const int agg = a.by_sample ? FGRPO_AGG_SAMPLE_MEAN : FGRPO_AGG_TOKEN_MEAN;
   const int64_t* y = a.labels.data_ptr<int64_t>();
@@ -250,7 +250,7 @@ struct FusedStep : torch::autograd::Function<FusedStep> {
     ctx->saved_data["db"] = o.grads.db;
     ctx->saved_data["kept"] = o.kept;
     ctx->saved_data["fresh"] = a.mode == kChunked;
-    ctx->saved_data["temperature"] = a.temperature;
+    ctx->saved_data["inv_temp"] = a.inv_temp;
     ctx->saved_data["hint"] = a.panel_hint;
     ctx->saved_data["nh"] = a.need_h;
     ctx->saved_data["nw"] = a.need_w;
@@ -280,7 +280,7 @@ struct FusedStep : torch::autograd::Function<FusedStep> {
     sd["kept"] = Tensor();                       // released by the first backward
     const Tensor h = in_place(saved[0]), w = in_place(saved[1]);
     const Tensor b = saved[2].defined() ? saved[2].detach().to(w.scalar_type()).contiguous() : Tensor();
-    Grads r = lmhead_backward(h, w, b, saved[3], saved[4], saved[5], gout, sd["temperature"].toDouble(), sd["hint"].toInt(),
+    Grads r = lmhead_backward(h, w, b, saved[3], saved[4], saved[5], gout, sd["inv_temp"].toDouble(), sd["hint"].toInt(),
                               kept, sd["nh"].toBool(), sd["nw"].toBool(), sd["nb"].toBool());
     return {r.dh, r.dw, r.db, Tensor()};
   }
@@ -289,7 +289,7 @@ struct FusedStep : torch::autograd::Function<FusedStep> {
 // mode: 0 "auto", 1 "recompute", 2 "whole", 3 "chunked" (what the gradients come from, where one is wanted)
 variable_list fused_step(const Tensor& hidden, const Tensor& weight, const std::optional<Tensor>& bias_, const Tensor& labels,
                          const std::optional<Tensor>& old_lp, const Tensor& adv, const std::optional<Tensor>& ref_lp,
-                         const std::optional<Tensor>& cu, double temperature, double clip_low, double clip_high, double clip_c,
+                         const std::optional<Tensor>& cu, double inv_temp, double clip_low, double clip_high, double clip_c,
                          double kl_beta, bool by_sample, double denom, int64_t panel_hint, int mode, int64_t chunk_tokens,
                          int64_t keep_whole_max_bytes) {
   const Tensor bias = opt(bias_);
@@ -310,7 +310,7 @@ variable_list fused_step(const Tensor& hidden, const Tensor& weight, const std::
   a.ref_lp = per_token(opt(ref_lp), T, "ref_logprobs");
   if (cu.has_value()) a.cu = cu->to(hidden.device(), at::kInt).contiguous();
   require_one_gpu(hidden, a.old_lp, a.ref_lp, a.cu);
-  a.temperature = temperature, a.clip_low = clip_low, a.clip_high = clip_high, a.clip_c = clip_c, a.kl_beta = kl_beta;
+  a.inv_temp = inv_temp, a.clip_low = clip_low, a.clip_high = clip_high, a.clip_c = clip_c, a.kl_beta = kl_beta;
   a.denom = denom, a.by_sample = by_sample, a.panel_hint = panel_hint, a.chunk_tokens = (int)chunk_tokens;
   const bool on = at::GradMode::is_enabled();
   a.need_h = on && hidden.requires_grad();

@@ -32,6 +32,14 @@ def test_product_path_refuses_cpu_tensors():
         G.logprobs_from_logits(torch.randn(4, 9), torch.zeros(4, dtype=torch.long))
 
 
+def test_fused_step_refuses_a_zero_temperature():
+    """Its reciprocal would be infinite; the refusal comes before any tensor is looked at."""
+    from fgrpo import ops
+    h, w, y = torch.randn(4, 64), torch.randn(10, 64), torch.zeros(4, dtype=torch.long)
+    with pytest.raises(ZeroDivisionError):
+        ops.fused_grpo_loss(h, w, None, y, torch.zeros(4), torch.zeros(4), temperature=0.0)
+
+
 def test_foreign_per_token_fn_needs_the_gpu_too():
     """A caller-supplied per_token_fn takes the materialised-logits route; that route has no CPU version either."""
     import grpo_loss as G
