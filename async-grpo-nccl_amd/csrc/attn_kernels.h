@@ -75,6 +75,8 @@ struct AttnParams {
   float* part_k;         // [parts_k][2][T][Hkv][HD] dK / scale and dV of the part
 };
 
+constexpr int kAttnMaxParts = 8;      // parts of a tile at most
+constexpr int kAttnMergeWide = 4;     // parts whose sums are fetched together
 // A tile that walks `steps` steps, all its work-group's own chain, may be dealt to several work-groups: each walks its
 // share and leaves fp32 sums, which a last launch adds up in a fixed order (no atomics: bit-reproducible).  How many,
 // every kernel of the call derives from the segment bounds.
@@ -1805,8 +1807,14 @@ __global__ __launch_bounds__(256, 2) void varlen_attn_dq2_kernel(AttnParams p) {
   if (valid) attn_store_rowmajor(acc, p.scale, p.dq + ((long long)tq * p.Hq + hq) * kHD, h);   // dS was kept / scale
 }
 
+__device__ __forceinline__ void attn_load8(const float* src, float (&v)[8]) {
+  const float4 a = *(const float4*)src, b = *(const float4*)(src + 4);
+  v[0] = a.x, v[1] = a.y, v[2] = a.z, v[3] = a.w, v[4] = b.x, v[5] = b.y, v[6] = b.z, v[7] = b.w;
+}
 // Sums of the parts of a query tile, in part order: eight columns of one (token, head) a thread.  Rows of tiles that were
 // not dealt out are already in place.  FWD: every part is relative to its own maximum.
+// Bound by latency: a thread's time is its chain of round trips, so the loads of kAttnMergeWide parts go out together (the
+// first part again for those a tile does not have).  777 tokens with 12 heads of 128: 5.2 -> 4.3 us.
 template <int HD, bool FWD>
 __device__ __forceinline__ void attn_merge_query_row(const AttnParams& p, int RB, long long idx) {
   const int col = (int)(idx % (HD / 8)) * 8;
@@ -1822,22 +1830,33 @@ __device__ __forceinline__ void attn_merge_query_row(const AttnParams& p, int RB
 #pragma unroll
   for (int e = 0; e < 8; ++e) x[e] = 0.f;
   float mul = p.scale, m = -INFINITY, l = 0.f;
+  float2 ml[kAttnMaxParts];
   if constexpr (FWD) {
-    for (int j = 0; j < np; ++j) m = fmaxf(m, p.part_ml[((long long)j * p.Hq + hq) * p.T + t].x);
+#pragma unroll
+    for (int j = 0; j < kAttnMaxParts; ++j) ml[j] = p.part_ml[((long long)(j < np ? j : 0) * p.Hq + hq) * p.T + t];
+#pragma unroll
+    for (int j = 0; j < kAttnMaxParts; ++j) m = j < np ? fmaxf(m, ml[j].x) : m;
   }
   const float m_use = m == -INFINITY ? 0.f : m;
-  for (int j = 0; j < np; ++j) {
-    const float* src = p.part_q + ((long long)j * p.T * p.Hq + row) * HD + col;
-    const float4 a = *(const float4*)src, b = *(const float4*)(src + 4);
-    float w = 1.f;
-    if constexpr (FWD) {
-      const float2 ml = p.part_ml[((long long)j * p.Hq + hq) * p.T + t];
-      w = fast_exp2((ml.x - m_use) * (p.scale * kLog2e));
-      l = __builtin_fmaf(ml.y, w, l);
-    }
-    const float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+  const float* src = p.part_q + row * HD + col;
+  const long long slice = (long long)p.T * p.Hq * HD;
 #pragma unroll
-    for (int e = 0; e < 8; ++e) x[e] = FWD ? __builtin_fmaf(v[e], w, x[e]) : x[e] + v[e];
+  for (int j0 = 0; j0 < kAttnMaxParts; j0 += kAttnMergeWide) {
+    if (j0 >= np) break;
+    float v[kAttnMergeWide][8];
+#pragma unroll
+    for (int u = 0; u < kAttnMergeWide; ++u) attn_load8(src + (j0 + u < np ? j0 + u : 0) * slice, v[u]);
+#pragma unroll
+    for (int u = 0; u < kAttnMergeWide; ++u) {
+      if (j0 + u >= np) continue;
+      float w = 1.f;
+      if constexpr (FWD) {
+        w = fast_exp2((ml[j0 + u].x - m_use) * (p.scale * kLog2e));
+        l = __builtin_fmaf(ml[j0 + u].y, w, l);
+      }
+#pragma unroll
+      for (int e = 0; e < 8; ++e) x[e] = FWD ? __builtin_fmaf(v[u][e], w, x[e]) : x[e] + v[u][e];
+    }
   }
   if constexpr (FWD) {
     mul = l > 0.f ? 1.f / l : 0.f;

@@ -576,12 +576,18 @@ static __global__ __launch_bounds__(256) void attn_merge_bwd_kernel(AttnParams p
   float x[8];
 #pragma unroll
   for (int e = 0; e < 8; ++e) x[e] = 0.f;
-  for (int j = 0; j < np; ++j) {
-    const float* src = p.part_k + (((long long)j * 2 + which) * p.T * p.Hkv + row) * HD + col;
-    const float4 a = *(const float4*)src, b = *(const float4*)(src + 4);
-    const float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+  const float* src = p.part_k + ((long long)which * p.T * p.Hkv + row) * HD + col;
+  const long long slice = 2LL * p.T * p.Hkv * HD;
 #pragma unroll
-    for (int e = 0; e < 8; ++e) x[e] += v[e];
+  for (int j0 = 0; j0 < kAttnMaxParts; j0 += kAttnMergeWide) {
+    if (j0 >= np) break;
+    float v[kAttnMergeWide][8];
+#pragma unroll
+    for (int u = 0; u < kAttnMergeWide; ++u) attn_load8(src + (j0 + u < np ? j0 + u : 0) * slice, v[u]);
+#pragma unroll
+    for (int u = 0; u < kAttnMergeWide; ++u)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) x[e] = j0 + u < np ? x[e] + v[u][e] : x[e];
   }
   const float mul = which ? 1.f : p.scale;
 #pragma unroll

@@ -7,7 +7,6 @@
 using namespace fgrpo;
 
 namespace fgrpo {
-constexpr int kAttnMaxParts = 8;
 constexpr size_t kAttnSplitMaxBytes = 256u << 20;
 int launch_attn_dkv3(int D, const AttnParams& p, hipStream_t st);      // launch_attn_keyside.hip
 int attn_keyside_keys(int D);
