@@ -182,11 +182,11 @@ __global__ __launch_bounds__(256, KB == 2 ? 1 : 2) void varlen_attn_dkv3_kernel(
   const char* f_dp = (const char*)(p.dout + (long long)(hkv * G + g_f) * HD + (long long)qb_f * do_st);
   long long f_qb = ((long long)q_end - qb_f - 1) * p.q_st * 2 + RB;           // bytes to the end of the head's last row
   long long f_db = ((long long)q_end - qb_f - 1) * do_st * 2 + RB;
-  // per-query scalars: rows past the end of the queries read what lies there or zero: finite, and hidden
+  // per-query scalars: the descriptors end with the queries of the head the item reads (the scalar offset counts in the
+  // range check), so that rows past them, another segment's, read as zero like their Q and dO: those may be NaN
   const uint32_t los = (lane & 31) * 4;
-  const __amdgpu_buffer_rsrc_t rsl = make_rsrc(p.lse + (long long)hkv * G * p.T, (uint32_t)G * (uint32_t)p.T * 4);
-  const __amdgpu_buffer_rsrc_t rsx = make_rsrc(p.delta + (long long)hkv * G * p.T, (uint32_t)G * (uint32_t)p.T * 4);
-  __amdgpu_buffer_rsrc_t rsq, rsd;
+  const float *lse_g = p.lse + (long long)hkv * G * p.T, *delta_g = p.delta + (long long)hkv * G * p.T;
+  __amdgpu_buffer_rsrc_t rsq, rsd, rsl, rsx;
   const long long h_q = p.q_sh * 2, r_q = (long long)kDkv3Rows * p.q_st * 2, r_d = (long long)kDkv3Rows * do_st * 2;
   auto fetch_setup = [&](bool more) {      // without an item the loads go out all the same: to an empty range (zeros), the last item's scalars
     long long bq = more ? f_qb : 0, bd = more ? f_db : 0;
@@ -194,6 +194,9 @@ __global__ __launch_bounds__(256, KB == 2 ? 1 : 2) void varlen_attn_dkv3_kernel(
     if (bd > 0xffffffffLL) bd = 0xffffffffLL;
     rsq = make_rsrc(f_qp, (uint32_t)bq);
     rsd = make_rsrc(f_dp, (uint32_t)bd);
+    const uint32_t bs = (uint32_t)(g_f * p.T + q_end) * 4;
+    rsl = make_rsrc(lse_g, bs);
+    rsx = make_rsrc(delta_g, bs);
   };
   auto fetch_advance = [&]() {             // `stride` items on
     if constexpr (SPLIT) {
@@ -315,14 +318,15 @@ __global__ __launch_bounds__(256, KB == 2 ? 1 : 2) void varlen_attn_dkv3_kernel(
                          pack_bf16x2(x[8 * half + 4], x[8 * half + 5]), pack_bf16x2(x[8 * half + 6], x[8 * half + 7])};
       return v;
     };
-    // hidden pairs of a key block become -inf; a branch of its own around the selects
+    // P of a hidden pair is zero, whatever its query's lse is (a NaN row of another segment in the same block must not
+    // reach this key); a branch of its own around the selects
     auto hide = [&](auto kbc) {
       constexpr int kb = decltype(kbc)::value;
       int qv = qb;
       asm volatile("" : "+s"(qv));                             // formed here: hoisted, it would be computed for every item
       const uint32_t q0 = (uint32_t)(qv - key_lo[kb]);
 #pragma unroll
-      for (int r = 0; r < 16; ++r) s[kb][r] = q0 + (uint32_t)(8 * (r >> 2) + (r & 3)) < key_n[kb] ? s[kb][r] : -INFINITY;
+      for (int r = 0; r < 16; ++r) s[kb][r] = q0 + (uint32_t)(8 * (r >> 2) + (r & 3)) < key_n[kb] ? s[kb][r] : 0.f;
     };
     // vector work w = 0 .. N - 1 dealt evenly to instructions m = M0 .. M1 - 1 of a run
     auto deal = [&](auto nc, auto mc, auto m0c, auto m1c, auto&& side) {
@@ -364,7 +368,6 @@ __global__ __launch_bounds__(256, KB == 2 ? 1 : 2) void varlen_attn_dkv3_kernel(
       });
       fence();
     });
-    if (masked) hide(H0{});
     constexpr int GD = 2 + 2 * KB;                             // LDS reads of a dP group
     auto open_dp = [&]() {                                     // -delta and the first group on their way
       static_for<4>([&](auto gc) { nd[decltype(gc)::value] = lds_read_u128_asm<sct + 256 + 32 * decltype(gc)::value>(scl); });
@@ -381,7 +384,7 @@ __global__ __launch_bounds__(256, KB == 2 ? 1 : 2) void varlen_attn_dkv3_kernel(
         fence();
         if constexpr (i == KS / 2 - 1) open_dp();
       });
-      if (masked) hide(FGRPO_IC(KB - 1));
+      if (masked) hide(H0{});
     } else {
       open_dp();
     }
@@ -416,6 +419,7 @@ __global__ __launch_bounds__(256, KB == 2 ? 1 : 2) void varlen_attn_dkv3_kernel(
         });
       });
     });
+    if (masked) hide(FGRPO_IC(KB - 1));
 #pragma unroll
     for (int kb = 0; kb < KB; ++kb) pp[kb][0] = pack(s[kb], 0);
     // ---- dV and dK in quarters of NQ instructions

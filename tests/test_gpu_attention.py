@@ -491,3 +491,32 @@ def test_key_side_kernel_at_the_edges_of_its_tiles(dev, T, cu, Hq, Hkv, causal, 
     out, lse = ops.varlen_attn_fwd(q, k, v, cu_t, None, causal)
     a, b = (ops.varlen_attn_bwd(do, q, k, v, out, lse, cu_t, None, causal) for _ in range(2))
     assert all(torch.equal(x, y) for x, y in zip(a, b))
+
+
+@pytest.mark.parametrize("bad", [float("nan"), float("inf")])
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("T,cu,Hq,Hkv,D", [
+    (300, [0, 200, 300], 4, 2, 128), (300, [0, 215, 300], 3, 1, 64), (170, [0, 161, 162, 170], 2, 2, 128),
+    (290, [0, 270], 4, 4, 64), (400, [0, 385], 2, 1, 128), (1500, [0, 1290, 1500], 4, 1, 128), (1500, [0, 1415], 14, 2, 64)])
+def test_a_non_finite_query_stays_in_its_own_sample(dev, T, cu, Hq, Hkv, D, causal, bad):
+    """Query rows behind the first sample - the next one's, or padding behind the last - turn non-finite: the last
+    query block of the first sample reaches up to 31 rows past its end.  Its results are those of the clean batch, bit
+    for bit: dQ and dV of every row, dK of the keys whose tiles lie inside it (in the tile it shares, a zero of dS
+    meets the NaN row itself)."""
+    from fgrpo import ops
+    q, k, v, do = (x.to(dev) for x in make(T, Hq, Hkv, T + D, D=D))
+    cu_t = torch.tensor(cu, dtype=torch.int32, device=dev)
+    end = cu[1]
+
+    def run(queries):
+        a = [x.clone().requires_grad_(True) for x in (queries, k, v)]
+        out = ops.varlen_attention(*a, cu_t, None, causal)
+        return (out.detach(),) + torch.autograd.grad(out, a, do)
+    want = run(q)
+    hurt = q.clone()
+    hurt[end:end + 32] = bad
+    got = run(hurt)
+    assert not torch.isfinite(got[0][end]).all()
+    rows = dict(out=end, dq=end, dk=end // 128 * 128, dv=end)
+    for (name, n), x, y in zip(rows.items(), got, want):
+        assert torch.isfinite(y[:n]).all() and torch.equal(x[:n], y[:n]), name
