@@ -37,6 +37,10 @@
 #pragma once
 #include "attn_kernels.h"
 
+#ifndef FGRPO_MFMA_VGPR_FORM
+#error "compile this unit with -mllvm -amdgpu-mfma-vgpr-form=1 -DFGRPO_MFMA_VGPR_FORM=1: else the compiler overwrites the accumulators below"
+#endif
+
 #define FGRPO_LDS_AT(a) ((__attribute__((address_space(3))) void*)(uint32_t)(a))      // LDS pointer from a byte address
 
 namespace fgrpo {
@@ -54,7 +58,8 @@ constexpr int kDkv3Lds = kDkv3LoopLds<HD, KB> > 4 * 32 * KB * kDkv3SumStride<HD>
 // The accumulators live in fixed accumulation registers, a[16 n : 16 n + 15] for block n, named in the instructions:
 // at HD = 128 they are all 256 of them, and a register allocator that may move or copy a block has nowhere to put it
 // (left to it, the loop spilled 260 registers).  Every instruction lists the whole range as clobbered, so that the
-// compiler keeps nothing of its own there; the build checks that the kernel spills nothing.
+// compiler keeps nothing of its own there across one of them; that it puts nothing there in between (a clobber does not
+// reserve a register) takes -amdgpu-mfma-vgpr-form, and the build reads in the compiler's assembly that it did not.
 // The compiler's hazard table does not see these instructions: the first one behind vector arithmetic that formed an
 // operand carries two wait states, instructions on one block are at least four matrix instructions apart.
 #define FGRPO_DKV3_CLOBBER_64 \

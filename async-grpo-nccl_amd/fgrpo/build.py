@@ -24,9 +24,13 @@ USAGE_PATH = os.path.join(CSRC, f"resource_usage{_ALT}.json")
 OBJ_DIR = os.path.join(CSRC, "build" + _ALT)
 
 SOURCES = ["fgrpo_api.hip", "launch_lmhead.hip", "launch_gemm.hip", "launch_attn.hip", "launch_attn_keyside.hip"]
-# this unit keeps its accumulators in named accumulation registers: the results of the matrix instructions the compiler
-# schedules must stay out of those
-SOURCE_FLAGS = {"launch_attn_keyside.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]}
+# This unit keeps its accumulators in named accumulation registers across whole loops.  A clobber list does not reserve
+# them: between two of its statements the compiler may use them, and without this flag it puts the results of the matrix
+# instructions it schedules itself into a[0:15], over the first accumulator, spilling nothing.  The define lets the
+# source refuse a compilation without the flag; whether the compiler kept out is read off its assembly
+# (check_named_accumulators).
+SOURCE_FLAGS = {"launch_attn_keyside.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1", "-DFGRPO_MFMA_VGPR_FORM=1"]}
+NAMED_ACCUMULATORS = {"launch_attn_keyside.hip": "varlen_attn_dkv3_kernel"}
 
 HIPCC_FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC",
@@ -50,9 +54,11 @@ TWO_PER_SIMD = ("TileCfgILi256ELi256ELi64ELi2ELi4ELi2ELi2ELb1EE",      # id 8
                 "varlen_attn_fwd2_kernel", "varlen_attn_dq2_kernel", "varlen_attn_dkv2_kernel")
 # attention kernels whose LDS reads are inline assembly: a spilled register could be one whose data is still on its way
 ASM_READ_ATTN = ("varlen_attn_fwd2_kernel", "varlen_attn_dq2_kernel", "varlen_attn_dkv2_kernel")
-# ... and the one that runs one wavefront per SIMD (accumulators in the accumulation registers): no spills either
-ASM_READ_ONE_PER_SIMD = ("varlen_attn_dkv3_kernel",)
-MUST_EXIST = TILE_KERNELS + ("varlen_attn_fwd_kernel", "varlen_attn_dq_kernel", "varlen_attn_dkv_kernel") + ASM_READ_ATTN
+# ... and the one with named accumulation registers (head dimension x key blocks of them): no spills either, and exactly
+# those; with one key block it runs two wavefronts per SIMD
+ASM_READ_NAMED_ACC = ("varlen_attn_dkv3_kernel",)
+NAMED_ACC_SHAPE = re.compile(r"varlen_attn_dkv3_kernelILi(\d+)ELi(\d+)E")
+MUST_EXIST = TILE_KERNELS + ("varlen_attn_fwd_kernel", "varlen_attn_dq_kernel", "varlen_attn_dkv_kernel") + ASM_READ_ATTN + ASM_READ_NAMED_ACC
 
 _FIELDS = {
     "TotalSGPRs": "sgprs", "VGPRs": "vgprs", "AGPRs": "agprs", "ScratchSize [bytes/lane]": "scratch",
@@ -88,27 +94,62 @@ def check_resource_usage(usage: dict) -> list:
         if tile and ASM_READ_CFG.search(name) and (u.get("scratch", 0) or u.get("vgpr_spill", 0)):
             bad.append(f"{name}: inline-assembly fragment reads with {u.get('vgpr_spill')} spilled VGPRs "
                        f"({u.get('scratch')} B/lane of scratch)")
-        if any(k in name for k in ASM_READ_ATTN + ASM_READ_ONE_PER_SIMD) and (u.get("scratch", 0) or u.get("vgpr_spill", 0)):
+        if any(k in name for k in ASM_READ_ATTN + ASM_READ_NAMED_ACC) and (u.get("scratch", 0) or u.get("vgpr_spill", 0)):
             bad.append(f"{name}: inline-assembly fragment reads with {u.get('vgpr_spill')} spilled VGPRs "
                        f"({u.get('scratch')} B/lane of scratch)")
         if any(k in name for k in TWO_PER_SIMD) and (tile or "varlen" in name):
             if u.get("vgprs", 0) > 256 or u.get("agprs", 0) or u.get("scratch", 0):
                 bad.append(f"{name}: {u.get('vgprs')} VGPRs, {u.get('agprs')} AGPRs, {u.get('scratch')} B/lane of "
                            "scratch do not fit two wavefronts per SIMD")
+        shape = NAMED_ACC_SHAPE.search(name)
+        if shape:
+            acc, one_block = int(shape.group(1)) * int(shape.group(2)), shape.group(2) == "1"
+            if u.get("agprs", 0) != acc or (one_block and u.get("vgprs", 0) + acc > 256):
+                bad.append(f"{name}: {u.get('vgprs')} VGPRs and {u.get('agprs')} AGPRs; its accumulators are {acc} AGPRs"
+                           + (" and two wavefronts share a SIMD" if one_block else ""))
     for key, n in seen.items():
         if n == 0:
             bad.append(f"no kernel named *{key}* in the compiler's report (guard out of date?)")
     return bad
 
 
+def check_named_accumulators(asm: str, family: str) -> list:
+    """Problems (strings) with the compiler's assembly of kernels that keep values in named accumulation registers:
+    outside inline assembly no instruction of theirs may name one."""
+    bad, cur, inline, seen, uses = [], None, False, 0, 0
+    for line in asm.splitlines():
+        label = re.match(r"^(_Z\w+):", line)
+        if label:
+            cur = label.group(1) if family in label.group(1) else None
+            inline = False
+            seen += cur is not None
+        elif line.startswith(".Lfunc_end"):
+            cur = None
+        elif "#ASMSTART" in line or "#ASMEND" in line:
+            inline = "#ASMSTART" in line
+        elif cur and re.search(r"\ba(\d+\b|\[\d)", line.split(";")[0]) and not line.lstrip().startswith("."):
+            uses += inline
+            if not inline:
+                bad.append(f"{cur}: the compiler uses accumulation registers that are named: {line.strip()}")
+    if not seen or not uses:
+        bad.append(f"no kernel named *{family}* with named accumulation registers in the assembly (guard out of date?)")
+    return bad
+
+
 def _compile(src: str, verbose: bool):
     hipcc = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
     obj = os.path.join(OBJ_DIR, os.path.splitext(src)[0] + ".o")
-    cmd = [hipcc, *HIPCC_FLAGS, *SOURCE_FLAGS.get(src, []), *os.environ.get("FGRPO_EXTRA_FLAGS", "").split(), "-c", os.path.join(CSRC, src), "-o", obj]
+    flags = [*HIPCC_FLAGS, *SOURCE_FLAGS.get(src, []), *os.environ.get("FGRPO_EXTRA_FLAGS", "").split()]
+    cmd = [hipcc, *flags, "-c", os.path.join(CSRC, src), "-o", obj]
     if verbose:
         print(" ".join(cmd), flush=True)
+    family, listing = NAMED_ACCUMULATORS.get(src), None
+    if family:                                   # the same compilation once more, as assembly, beside it
+        listing = subprocess.Popen([hipcc, *flags, "--cuda-device-only", "-S", os.path.join(CSRC, src), "-o", "-"],
+                                   stdout=subprocess.PIPE, stderr=subprocess.DEVNULL, text=True)
     res = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
-    return src, obj, res.returncode, res.stdout
+    problems = check_named_accumulators(listing.communicate()[0], family) if family else []
+    return src, obj, res.returncode, res.stdout, problems
 
 
 def _is_noise(line: str) -> bool:
@@ -146,12 +187,13 @@ def build(verbose: bool = True, only=None) -> str:
     todo = [s for s in SOURCES if only is None or s in only]
     side = concurrent.futures.ThreadPoolExecutor(max_workers=1)
     binding = side.submit(build_binding, verbose) if only is None or BINDING_SOURCE in only else None
-    by_source = {}
+    by_source, assembly = {}, {}
     if only is not None and os.path.exists(USAGE_PATH):
-        by_source = json.load(open(USAGE_PATH)).get("sources", {})
+        last = json.load(open(USAGE_PATH))
+        by_source, assembly = last.get("sources", {}), last.get("assembly_problems", {})
     with concurrent.futures.ThreadPoolExecutor(max_workers=len(SOURCES)) as pool:
         results = list(pool.map(lambda s: _compile(s, verbose), todo))
-    for src, obj, rc, out in results:
+    for src, obj, rc, out, bad in results:
         # remarks carry source excerpts on the following lines ("  2 | ..." and "    | ^"): drop those too
         keep, skip = [], 0
         for line in out.splitlines():
@@ -168,7 +210,7 @@ def build(verbose: bool = True, only=None) -> str:
             raise RuntimeError(f"hipcc failed on {src}:\n" + shown)
         if verbose and shown.strip():
             print(shown)
-        by_source[src] = parse_resource_usage(out)
+        by_source[src], assembly[src] = parse_resource_usage(out), bad
     objs = [os.path.join(OBJ_DIR, os.path.splitext(s)[0] + ".o") for s in SOURCES]
     missing = [o for o in objs if not os.path.exists(o)]
     if missing:
@@ -176,9 +218,9 @@ def build(verbose: bool = True, only=None) -> str:
     # The guard decides before anything is linked: a build it refuses leaves no library behind (a stale one from an
     # earlier build is removed too), so nothing can load the kernels it exists to block.
     usage = {k: v for src in SOURCES for k, v in by_source.get(src, {}).items()}
-    problems = check_resource_usage(usage)
-    json.dump({"sources": by_source, "kernels": usage, "problems": problems}, open(USAGE_PATH, "w"), indent=1,
-              sort_keys=True)
+    problems = check_resource_usage(usage) + [p for src in SOURCES for p in assembly.get(src, [])]
+    json.dump({"sources": by_source, "kernels": usage, "assembly_problems": assembly, "problems": problems},
+              open(USAGE_PATH, "w"), indent=1, sort_keys=True)
     if problems:
         if os.path.exists(LIB_PATH):
             os.remove(LIB_PATH)

@@ -13,6 +13,8 @@ B = importlib.import_module("fgrpo.build")     # the package re-exports the func
 
 ASM_KERNEL = "_ZN5fgrpo17lmhead_fwd_kernelINS_7TileCfgILi256ELi256ELi64ELi2ELi4ELi2ELi2ELb1EEEEEvNS_9FwdParamsE"
 REG_KERNEL = "_ZN5fgrpo17gemm_store_kernelINS_7TileCfgILi256ELi256ELi64ELi2ELi2ELi1ELi2ELb0EEELb0ELb0EEEvNS_11StoreParamsE"
+KEY_SIDE_128 = "_ZN5fgrpo23varlen_attn_dkv3_kernelILi128ELi2ELb0EEEvNS_10AttnParamsE"
+KEY_SIDE_64 = "_ZN5fgrpo23varlen_attn_dkv3_kernelILi64ELi1ELb1EEEvNS_10AttnParamsE"
 
 
 def remarks(name, vgprs=200, agprs=0, scratch=0, vspill=0, sspill=0):
@@ -40,6 +42,7 @@ def full_report(**over):
                   "varlen_attn_dq_kernelILi128ELi1EE", "varlen_attn_dkv_kernelILi128EE", "varlen_attn_fwd2_kernelILi128ELi1EE",
                   "varlen_attn_dq2_kernelILi128ELi1EE", "varlen_attn_dkv2_kernelILi128EE"):
         text += "\n" + remarks("_ZN5fgrpo" + other)
+    text += "\n" + remarks(KEY_SIDE_128, vgprs=238, agprs=256) + "\n" + remarks(KEY_SIDE_64, vgprs=118, agprs=64)
     return B.parse_resource_usage(text)
 
 
@@ -96,3 +99,48 @@ def test_guard_covers_the_hand_scheduled_attention_kernels():
     assert problems and any("varlen_attn_dkv2_kernel" in x for x in problems)
     gone = {k: v for k, v in base.items() if "varlen_attn_dq2_kernel" not in k}
     assert any("varlen_attn_dq2_kernel" in x for x in B.check_resource_usage(gone))
+
+
+@pytest.mark.parametrize("name,over", [(KEY_SIDE_128, dict(vgpr_spill=1)), (KEY_SIDE_128, dict(scratch=4)), (KEY_SIDE_128, dict(agprs=240)),
+                                       (KEY_SIDE_64, dict(agprs=80)), (KEY_SIDE_64, dict(vgprs=200)), (KEY_SIDE_64, dict(vgpr_spill=1))])
+def test_guard_covers_the_kernel_with_named_accumulators(name, over):
+    """No spills, exactly the accumulation registers it names, two wavefronts per SIMD at one key block; and it exists."""
+    base = full_report()
+    assert B.check_resource_usage(base) == []
+    hurt = dict(base)
+    hurt[name] = dict(base[name], **over)
+    assert any(name in x for x in B.check_resource_usage(hurt))
+    gone = {k: v for k, v in base.items() if "dkv3" not in k}
+    assert any("varlen_attn_dkv3_kernel" in x for x in B.check_resource_usage(gone))
+
+
+ASM_OK = """
+_ZN5fgrpo23varlen_attn_dkv3_kernelILi64ELi1ELb0EEEvNS_10AttnParamsE: ; @_ZN5fgrpo
+\tv_mfma_f32_32x32x16_bf16 v[2:17], v[18:21], v[22:25], 0 ; a[0:15] would be wrong
+\t;;#ASMSTART
+\ts_nop 1
+\tv_mfma_f32_32x32x16_bf16 a[0:15], v[2:5], v[6:9], a[0:15]
+\t;;#ASMEND
+\ts_endpgm
+.Lfunc_end0:
+_ZN5fgrpo21attn_merge_bwd_kernelILi64ELi32EEEvNS_10AttnParamsEixx:
+\tv_accvgpr_read_b32 v0, a3
+"""
+
+
+@pytest.mark.parametrize("line", ["v_mfma_f32_32x32x16_bf16 a[0:15], v[2:5], v[6:9], 0", "v_accvgpr_read_b32 v0, a0",
+                                  "v_accvgpr_write_b32 a[3], v1", "ds_write_b32 v0, a12 offset:16"])
+def test_assembly_guard_rejects_the_compilers_own_use_of_named_accumulators(line):
+    """What a compilation without the flag puts there: results of its own matrix instructions, in no report as a spill."""
+    assert B.check_named_accumulators(ASM_OK, "varlen_attn_dkv3_kernel") == []
+    hurt = ASM_OK.replace("\ts_endpgm", "\t" + line + "\n\ts_endpgm")
+    assert B.check_named_accumulators(hurt, "varlen_attn_dkv3_kernel")
+    assert B.check_named_accumulators(ASM_OK, "another_kernel")
+
+
+def test_key_side_unit_refuses_a_compilation_without_its_flag():
+    import subprocess
+    unit = os.path.join(B.CSRC, "launch_attn_keyside.hip")
+    res = subprocess.run([os.environ.get("HIPCC", "/opt/rocm/bin/hipcc"), "--offload-arch=gfx950", "-std=c++17", "-E",
+                          "--cuda-device-only", unit, "-o", os.devnull], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+    assert res.returncode != 0 and "amdgpu-mfma-vgpr-form" in res.stdout
