@@ -236,10 +236,13 @@ StepOut step_forward(const Tensor& h, const Tensor& w, const Tensor& b, const St
   return o;
 }
 
-// (loss, entropy, log_ratio, clip1, unclipped, clipped, lp); only the loss carries a gradient.
+// (loss, entropy, log_ratio, clip1, unclipped, clipped, lp); only the loss carries a gradient.  The three per-token inputs
+// get none, and are read in the form StepArgs holds them in; they are inputs of the node so that autograd sees them: a
+// forward-mode tangent on one is refused, not dropped, and one that requires a gradient makes the loss require one.
 struct FusedStep : torch::autograd::Function<FusedStep> {
   static variable_list forward(AutogradContext* ctx, const Tensor& hidden, const Tensor& weight,
-                               const std::optional<Tensor>& bias_, const StepArgs& a) {
+                               const std::optional<Tensor>& bias_, const std::optional<Tensor>& /*old_lp*/,
+                               const Tensor& /*adv*/, const std::optional<Tensor>& /*ref_lp*/, const StepArgs& a) {
     const Tensor bias = opt(bias_);
     const Tensor h = in_place(hidden), w = in_place(weight);
     const Tensor b = bias.defined() ? bias.detach().to(w.scalar_type()).contiguous() : Tensor();
@@ -262,7 +265,7 @@ struct FusedStep : torch::autograd::Function<FusedStep> {
   }
   static variable_list backward(AutogradContext* ctx, variable_list gs) {
     const Tensor gout = gs[0];
-    if (!gout.defined()) return {Tensor(), Tensor(), Tensor(), Tensor()};
+    if (!gout.defined()) return variable_list(7);
     auto& sd = ctx->saved_data;
     if (sd["fresh"].toBool()) {
       sd["fresh"] = false;
@@ -273,7 +276,7 @@ struct FusedStep : torch::autograd::Function<FusedStep> {
       for (const Tensor& t : {r.dh, r.dw, r.db})
         if (t.defined() && t.numel() > 0)
           check(api.fgrpo_scale_inplace(t.data_ptr(), t.numel(), dtype_code(t), fptr(scale), d.stream()), "scale_inplace");
-      return {r.dh, r.dw, r.db, Tensor()};
+      return {r.dh, r.dw, r.db, Tensor(), Tensor(), Tensor(), Tensor()};
     }
     const auto saved = ctx->get_saved_variables();
     const Tensor kept = sd["kept"].toTensor();
@@ -282,7 +285,7 @@ struct FusedStep : torch::autograd::Function<FusedStep> {
     const Tensor b = saved[2].defined() ? saved[2].detach().to(w.scalar_type()).contiguous() : Tensor();
     Grads r = lmhead_backward(h, w, b, saved[3], saved[4], saved[5], gout, sd["inv_temp"].toDouble(), sd["hint"].toInt(),
                               kept, sd["nh"].toBool(), sd["nw"].toBool(), sd["nb"].toBool());
-    return {r.dh, r.dw, r.db, Tensor()};
+    return {r.dh, r.dw, r.db, Tensor(), Tensor(), Tensor(), Tensor()};
   }
 };
 
@@ -333,7 +336,7 @@ variable_list fused_step(const Tensor& hidden, const Tensor& weight, const std::
       if (mode == 2 || (keep_ok && (int64_t)api.fgrpo_logits_keep_bytes((int)T, (int)V) <= keep_whole_max_bytes)) a.mode = kWhole;
     }
   }
-  return FusedStep::apply(hidden, weight, bias_, a);
+  return FusedStep::apply(hidden, weight, bias_, old_lp, adv, ref_lp, a);
 }
 
 // ---------------------------------------------------------------------------------------------- packed attention

@@ -944,7 +944,7 @@ def fused_grpo_loss(hidden, weight, bias, labels_shifted, old_lp, adv, ref_lp=No
         raise ValueError(f"Invalid loss_agg_mode: {loss_agg_mode}")
     mode = _grad_mode(keep_logits)
     compact = compact if torch.is_tensor(compact) else bool(compact)
-    wants_grad = _wants_grad(hidden, weight, bias)
+    wants_grad = _wants_grad(hidden, weight, bias, old_lp, adv, ref_lp)
     idx = _valid_rows(labels_shifted, compact)
     if idx is None and _fwd_event_sink is None and hidden.shape[0] > 0:
         V = weight.shape[0]

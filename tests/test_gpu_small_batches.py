@@ -144,3 +144,33 @@ def test_fp32_gradients_of_small_heads(dev, T, H, V):
     got = torch.autograd.grad(ops.lmhead_logprob(hg, wg, None, y.to(dev))[0], (hg, wg), gt.to(dev))
     for a, b in zip(got, want):
         assert (a.cpu().double() - b).norm() <= 6 * 2 ** -16 * b.norm()
+
+
+@pytest.mark.parametrize("compact", [False, True])
+@pytest.mark.parametrize("which", ["old_lp", "adv", "ref_lp"])
+def test_per_token_inputs_are_inputs_of_the_node(dev, which, compact):
+    """They take no gradient, but autograd sees them: a forward-mode tangent is refused with and without gradients, and
+    one that requires a gradient gives a loss that does (and a backward that leaves it none)."""
+    import torch.autograd.forward_ad as fwAD
+    from fgrpo import ops
+    h, w = torch.randn(70, 64, device=dev).bfloat16(), torch.randn(300, 64, device=dev).bfloat16()
+    y = torch.randint(0, 300, (70,), device=dev)
+    tok = dict(old_lp=torch.randn(70, device=dev) - 6, adv=torch.randn(70, device=dev), ref_lp=torch.randn(70, device=dev) - 6)
+    extra = dict(kl_beta=0.01, compact=torch.arange(0, 70, 2, device=dev) if compact else False)
+
+    def call(hidden, **over):
+        t = dict(tok, **over)
+        return ops.fused_grpo_loss(hidden, w, None, y, t["old_lp"], t["adv"], t["ref_lp"], **extra)
+    plain = call(h)
+    leaf = tok[which].clone().requires_grad_(True)
+    out = call(h, **{which: leaf})
+    assert not plain[0].requires_grad and out[0].requires_grad and torch.equal(out[0].detach(), plain[0])
+    out[0].backward()
+    assert leaf.grad is None
+    for hidden in (h, h.clone().requires_grad_(True)):
+        with fwAD.dual_level():
+            dual = fwAD.make_dual(tok[which], torch.ones_like(tok[which]))
+            with pytest.raises(RuntimeError, match="(?i)jvp"):
+                call(hidden, **{which: dual})
+            with torch.no_grad(), pytest.raises(RuntimeError, match="(?i)jvp"):
+                call(hidden, **{which: dual})
