@@ -438,6 +438,7 @@ Tensor varlen_attention(const Tensor& q, const Tensor& k, const Tensor& v, const
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.doc() = "autograd nodes over libfgrpo";
   m.def("init", &init);
-  m.def("fused_step", &fused_step);
-  m.def("varlen_attention", &varlen_attention);
+  // without the interpreter lock: a call may wait, for memory or for room in a full launch queue, and other threads run
+  m.def("fused_step", &fused_step, py::call_guard<py::gil_scoped_release>());
+  m.def("varlen_attention", &varlen_attention, py::call_guard<py::gil_scoped_release>());
 }

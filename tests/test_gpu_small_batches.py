@@ -174,3 +174,54 @@ def test_per_token_inputs_are_inputs_of_the_node(dev, which, compact):
                 call(hidden, **{which: dual})
             with torch.no_grad(), pytest.raises(RuntimeError, match="(?i)jvp"):
                 call(hidden, **{which: dual})
+
+
+@pytest.mark.parametrize("entry", ["varlen_attention", "fused_step"])
+def test_native_calls_release_the_interpreter_lock(dev, entry):
+    """With a switch interval nobody waits out, another thread runs only while a call of this one has let go of the
+    lock: it must get on again and again in a row of native calls."""
+    import sys
+    import threading
+    import time
+    from fgrpo import _lib
+    native = _lib.native()
+    cu = torch.tensor([0, 600], dtype=torch.int32, device=dev)
+    q, k, v = (torch.randn(600, n, 128, device=dev).bfloat16() for n in (4, 2, 2))
+    h, w = torch.randn(600, 256, device=dev).bfloat16(), torch.randn(3000, 256, device=dev).bfloat16()
+    y, tok = torch.randint(0, 3000, (600,), device=dev), torch.randn(600, device=dev)
+    if entry == "varlen_attention":
+        def call():
+            return native.varlen_attention(q, k, v, cu, None, True, None)
+    else:
+        def call():
+            return native.fused_step(h, w, None, y, tok, tok, None, None, 1.0, 0.2, 0.2, 3.0, 0.0, False, 0.0, 0, 0, 256, 0)
+    with torch.no_grad():
+        call()
+        torch.cuda.synchronize()
+        ran, stop = [0], threading.Event()
+
+        def other():
+            while not stop.is_set():
+                ran[0] += 1
+                time.sleep(2e-4)              # gives the lock up by itself
+
+        interval = sys.getswitchinterval()
+        thread = threading.Thread(target=other)
+        thread.start()
+        sys.setswitchinterval(1000.0)
+        try:
+            time.sleep(0.05)                  # from here on its waits for the lock are of the long kind
+            before, got_on, calls, kept = ran[0], 0, 0, []       # kept: a tensor's end may release the lock too
+            while calls < 4000 and got_on < 20:
+                kept.append(call())
+                got_on += ran[0] > before
+                before = ran[0]
+                calls += 1
+        finally:
+            sys.setswitchinterval(interval)
+            stop.set()
+            thread.join()
+            torch.cuda.synchronize()
+    # most calls are too short for the other thread to wake in
+    print(f"[lock] {entry}: the other thread got on during {got_on} of {calls} calls", flush=True)
+    assert got_on == 20
