@@ -385,6 +385,7 @@ def make_grpo_forward(model, temperature: float = 1.0, mode: str = 'training', u
         else:
             raise ValueError(f"Invalid mode: {mode}")
 
+    _forward.takes_compact_masked_tokens = True
     model.__original_forward = model.forward
     model.forward = _forward
     return model

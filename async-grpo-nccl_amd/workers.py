@@ -8,6 +8,7 @@ are not reproduced; the model is any module patched by
 load time: attention wrapper, then the forward patch)."""
 from __future__ import annotations
 
+import inspect
 from types import SimpleNamespace
 from typing import List
 
@@ -74,6 +75,19 @@ class TrainerHarness:
         return metrics
 
 
+def _takes_row_list(model) -> bool:
+    """Whether ``compact_masked_tokens`` reaches a forward that ``make_grpo_forward`` made, through wrappers that hand
+    any keyword on; another forward may refuse it."""
+    while model is not None:
+        forward = getattr(model, "forward", None)
+        if getattr(forward, "takes_compact_masked_tokens", False):
+            return True
+        if not callable(forward) or all(p.kind is not p.VAR_KEYWORD for p in inspect.signature(forward).parameters.values()):
+            return False
+        model = getattr(model, "module", None) or getattr(model, "_orig_mod", None)
+    return False
+
+
 class LogProbHarness:
     """No-grad per-sample logprobs and entropies of packed samples."""
 
@@ -103,7 +117,7 @@ class LogProbHarness:
         # sizeable part of the batch the LM head is given the list of the others, known here on the host, and skips
         # them (the same threshold as the trainer's loss, see grpo_loss.compute_dual_clip_grpo_loss).
         extra = {}
-        if total >= ops.COMPACT_MIN_TOKENS:
+        if total >= ops.COMPACT_MIN_TOKENS and _takes_row_list(self.actor_module_fsdp):
             scored = np.flatnonzero(view[2, 1:] != -100)
             if 0 < scored.size < ops.COMPACT_MAX_VALID_FRACTION * total:
                 rows = torch.empty(scored.size, dtype=torch.long).pin_memory()

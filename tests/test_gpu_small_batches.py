@@ -225,3 +225,41 @@ def test_native_calls_release_the_interpreter_lock(dev, entry):
     # most calls are too short for the other thread to wake in
     print(f"[lock] {entry}: the other thread got on during {got_on} of {calls} calls", flush=True)
     assert got_on == 20
+
+
+@pytest.mark.parametrize("wrapped", [False, True])
+def test_logprob_worker_runs_any_model_of_the_four_inputs(dev, wrapped):
+    """The list of scored rows goes to forwards that take it, through a wrapper too; a model with a forward of its own
+    gets the four inputs and nothing else, however prompt-heavy the batch."""
+    from types import SimpleNamespace
+    from fgrpo import ops
+    from grpo_loss import make_grpo_forward
+    from workers import LogProbHarness
+
+    class Wrapper(torch.nn.Module):
+        def __init__(self, inner):
+            super().__init__()
+            self.module = inner
+
+        def forward(self, *args, **kwargs):
+            got.update(kwargs)
+            return self.module(*args, **kwargs)
+
+    class Narrow(Wrapper):
+        def forward(self, input_ids, attention_mask, position_ids, labels):
+            return self.module(input_ids=input_ids, attention_mask=attention_mask, position_ids=position_ids, labels=labels)
+
+    class Own(torch.nn.Module):
+        def forward(self, input_ids, attention_mask, position_ids, labels):
+            return SimpleNamespace(loss=input_ids.float().view(-1), entropy=position_ids.float().view(-1))
+    got = {}
+    samples = make_samples(n=130)
+    assert sum(len(s["sample_ids"]) for s in samples) >= ops.COMPACT_MIN_TOKENS
+    own = Wrapper(Own()) if wrapped else Own()
+    res = LogProbHarness(own, dev).compute_log_probs_from_samples(samples)
+    assert [r["logprobs"] for r in res] == [[float(t) for t in s["sample_ids"]] for s in samples]
+    torch.manual_seed(0)
+    model = make_grpo_forward(TinyLM(tied=False).to(dev).bfloat16(), mode="eval")
+    LogProbHarness(Wrapper(model), dev).compute_log_probs_from_samples(samples)
+    assert "compact_masked_tokens" in got
+    LogProbHarness(Narrow(model), dev).compute_log_probs_from_samples(samples)
