@@ -17,8 +17,8 @@ namespace {
 // Query heads per work-group of the query-side kernels (tile = 128 / heads tokens).  Short segments gain from short
 // tiles (less masked work on the diagonal and at segment boundaries) as long as the heads of a group fill the
 // work-group; long ones do not care, and a lone head per K/V head has nothing to share.
-int attn_heads_per_group(int G, int T, int n_seq) {
-  if (g_tune.attn_heads == 1 || g_tune.attn_heads == 2 || g_tune.attn_heads == 4) return g_tune.attn_heads;
+int attn_heads_per_group(const Tuning& tn, int G, int T, int n_seq) {
+  if (tn.attn_heads == 1 || tn.attn_heads == 2 || tn.attn_heads == 4) return tn.attn_heads;
   if (G <= 1 || (long long)T >= 8192LL * n_seq) return 1;      // measured: -10..-22 % up to 2048-token segments, +1 % at 8192
   if (G % 4 == 0) return 4;
   if (G % 2 == 0) return 2;
@@ -26,36 +26,36 @@ int attn_heads_per_group(int G, int T, int n_seq) {
 }
 
 template <template <int, int> class Launcher>
-int launch_query_side(int D, int hb, AttnParams& p, int T, int Hq, int Hkv, int32_t* bounds_ws, hipStream_t st) {
+int launch_query_side(const Tuning& tn, int D, int hb, AttnParams& p, int T, int Hq, int Hkv, int32_t* bounds_ws, hipStream_t st) {
   const int rb = 128 / hb, G = Hq / Hkv;
   p.order_q = bounds_ws + attn_order_offset(T, hb == 1 ? 1 : hb == 2 ? 2 : 3);
   const long long units = (long long)((T + rb - 1) / rb) * Hkv;            // (tile, K/V head)
   p.blocks_q = (int)(((units + 7) / 8 * 8) * ((G + hb - 1) / hb));
   const dim3 grid((unsigned)p.blocks_q * (p.parts_q > 1 ? p.parts_q : 1));
   if (D == 128) {
-    if (hb == 1) Launcher<128, 1>::run(grid, st, p);
-    else if (hb == 2) Launcher<128, 2>::run(grid, st, p);
-    else Launcher<128, 4>::run(grid, st, p);
+    if (hb == 1) Launcher<128, 1>::run(tn, grid, st, p);
+    else if (hb == 2) Launcher<128, 2>::run(tn, grid, st, p);
+    else Launcher<128, 4>::run(tn, grid, st, p);
   } else {
-    if (hb == 1) Launcher<64, 1>::run(grid, st, p);
-    else if (hb == 2) Launcher<64, 2>::run(grid, st, p);
-    else Launcher<64, 4>::run(grid, st, p);
+    if (hb == 1) Launcher<64, 1>::run(tn, grid, st, p);
+    else if (hb == 2) Launcher<64, 2>::run(tn, grid, st, p);
+    else Launcher<64, 4>::run(tn, grid, st, p);
   }
   HIP_TRY(hipGetLastError());
   return 0;
 }
 template <int HD, int HB>
 struct FwdLauncher {
-  static void run(dim3 grid, hipStream_t st, const AttnParams& p) {
-    if (g_tune.attn_qside == 1) hipLaunchKernelGGL((varlen_attn_fwd_kernel<HD, HB>), grid, dim3(256), 0, st, p);
+  static void run(const Tuning& tn, dim3 grid, hipStream_t st, const AttnParams& p) {
+    if (tn.attn_qside == 1) hipLaunchKernelGGL((varlen_attn_fwd_kernel<HD, HB>), grid, dim3(256), 0, st, p);
     else if (p.parts_q > 1) hipLaunchKernelGGL((varlen_attn_fwd2_kernel<HD, HB, true>), grid, dim3(256), 0, st, p);
     else hipLaunchKernelGGL((varlen_attn_fwd2_kernel<HD, HB>), grid, dim3(256), 0, st, p);
   }
 };
 template <int HD, int HB>
 struct DqLauncher {
-  static void run(dim3 grid, hipStream_t st, const AttnParams& p) {
-    if (g_tune.attn_qside == 1 || g_tune.attn_qside == 3) hipLaunchKernelGGL((varlen_attn_dq_kernel<HD, HB>), grid, dim3(256), 0, st, p);
+  static void run(const Tuning& tn, dim3 grid, hipStream_t st, const AttnParams& p) {
+    if (tn.attn_qside == 1 || tn.attn_qside == 3) hipLaunchKernelGGL((varlen_attn_dq_kernel<HD, HB>), grid, dim3(256), 0, st, p);
     else if (p.parts_q > 1) hipLaunchKernelGGL((varlen_attn_dq2_kernel<HD, HB, true>), grid, dim3(256), 0, st, p);
     else hipLaunchKernelGGL((varlen_attn_dq2_kernel<HD, HB>), grid, dim3(256), 0, st, p);
   }
@@ -97,15 +97,15 @@ SplitPlan plan_split(long long wgs, int per_cu, double chain, bool causal, doubl
   }
   return best;
 }
-SplitPlan plan_query_split(int T, int n_seq, int Hq, int Hkv, int D, int causal, bool forward) {
-  if (g_tune.attn_qside == 1 || (!forward && g_tune.attn_qside == 3)) return SplitPlan();
-  const int hb = attn_heads_per_group(Hq / Hkv, T, n_seq), rb = 128 / hb, G = Hq / Hkv;
+SplitPlan plan_query_split(const Tuning& tn, int T, int n_seq, int Hq, int Hkv, int D, int causal, bool forward) {
+  if (tn.attn_qside == 1 || (!forward && tn.attn_qside == 3)) return SplitPlan();
+  const int hb = attn_heads_per_group(tn, Hq / Hkv, T, n_seq), rb = 128 / hb, G = Hq / Hkv;
   const long long wgs = (long long)((T + rb - 1) / rb) * Hkv * ((G + hb - 1) / hb);
   return plan_split(wgs, 2, (double)T / n_seq / kAttnBK, causal, D == 128 ? 1.6 : forward ? 1.15 : 1.3,
                     (size_t)T * Hq * (D * 4 + (forward ? 8 : 0)));
 }
-SplitPlan plan_key_split(int T, int n_seq, int Hq, int Hkv, int D, int causal) {
-  if (g_tune.attn_dkv == 1 || g_tune.attn_dkv == 2) return SplitPlan();
+SplitPlan plan_key_split(const Tuning& tn, int T, int n_seq, int Hq, int Hkv, int D, int causal) {
+  if (tn.attn_dkv == 1 || tn.attn_dkv == 2) return SplitPlan();
   const int keys = attn_keyside_keys(D);
   const long long wgs = (long long)((T + keys - 1) / keys) * Hkv;
   const double chain = (double)T / n_seq / 32 * (Hq / Hkv) / 4;                // items of one of the four wavefronts
@@ -168,8 +168,9 @@ int fgrpo_varlen_attn_bounds(const int32_t* cu, int n_seq, int T, int causal, in
 
 size_t fgrpo_varlen_attn_workspace(int T, int n_seq, int Hq, int Hkv, int D, int causal, int backward) {
   if (T <= 0 || n_seq <= 0 || Hq <= 0 || Hkv <= 0 || Hq % Hkv != 0 || (D != 128 && D != 64)) return 0;
-  const size_t q = query_split_bytes(plan_query_split(T, n_seq, Hq, Hkv, D, causal, !backward), T, Hq, D, !backward);
-  return backward ? q + key_split_bytes(plan_key_split(T, n_seq, Hq, Hkv, D, causal), T, Hkv, D) : q;
+  const Tuning tn = g_tune;
+  const size_t q = query_split_bytes(plan_query_split(tn, T, n_seq, Hq, Hkv, D, causal, !backward), T, Hq, D, !backward);
+  return backward ? q + key_split_bytes(plan_key_split(tn, T, n_seq, Hq, Hkv, D, causal), T, Hkv, D) : q;
 }
 
 int fgrpo_varlen_attn_fwd(const void* q, const void* k, const void* v, long long q_st, long long q_sh, long long k_st,
@@ -197,8 +198,9 @@ int fgrpo_varlen_attn_fwd_ws(const void* q, const void* k, const void* v, long l
     rc = fgrpo_varlen_attn_bounds(cu, n_seq, T, causal, bounds_ws, stream);
     if (rc) return rc;
   }
-  const int hb = attn_heads_per_group(Hq / Hkv, T, n_seq);
-  SplitPlan sp = plan_query_split(T, n_seq, Hq, Hkv, D, causal, true);
+  const Tuning tn = g_tune;   // one reading of the tuning state per call: the kernel launched is the one the split was planned for
+  const int hb = attn_heads_per_group(tn, Hq / Hkv, T, n_seq);
+  SplitPlan sp = plan_query_split(tn, T, n_seq, Hq, Hkv, D, causal, true);
   const size_t need = query_split_bytes(sp, T, Hq, D, true);
   if (!ws || need == 0) sp = SplitPlan();
   else if (ws_bytes < need) return fail(FGRPO_ERR_WORKSPACE, "varlen_attn_fwd: workspace %zu < %zu", ws_bytes, need);
@@ -206,7 +208,7 @@ int fgrpo_varlen_attn_fwd_ws(const void* q, const void* k, const void* v, long l
   p.parts_q = sp.parts, p.per_q = sp.per;
   p.part_q = (float*)ws;
   p.part_ml = (float2*)((char*)ws + align256((size_t)sp.parts * T * Hq * D * 4));
-  rc = launch_query_side<FwdLauncher>(D, hb, p, T, Hq, Hkv, bounds_ws, st);
+  rc = launch_query_side<FwdLauncher>(tn, D, hb, p, T, Hq, Hkv, bounds_ws, st);
   if (rc || sp.parts <= 1) return rc;
   const unsigned blocks = (unsigned)(((long long)T * Hq * (D / 8) + 255) / 256);
   if (D == 128) hipLaunchKernelGGL(attn_merge_fwd_kernel<128>, dim3(blocks), dim3(256), 0, st, p, 128 / hb);
@@ -247,19 +249,20 @@ int fgrpo_varlen_attn_bwd_ws(const void* dout, const void* q, const void* k, con
     rc = fgrpo_varlen_attn_bounds(cu, n_seq, T, causal, bounds_ws, stream);
     if (rc) return rc;
   }
-  const int hb = attn_heads_per_group(Hq / Hkv, T, n_seq);
-  SplitPlan sq = plan_query_split(T, n_seq, Hq, Hkv, D, causal, false), sk = plan_key_split(T, n_seq, Hq, Hkv, D, causal);
+  const Tuning tn = g_tune;   // one reading of the tuning state per call: the kernel launched is the one the split was planned for
+  const int hb = attn_heads_per_group(tn, Hq / Hkv, T, n_seq);
+  SplitPlan sq = plan_query_split(tn, T, n_seq, Hq, Hkv, D, causal, false), sk = plan_key_split(tn, T, n_seq, Hq, Hkv, D, causal);
   const size_t need_q = query_split_bytes(sq, T, Hq, D, false), need = need_q + key_split_bytes(sk, T, Hkv, D);
   if (!ws || need == 0) sq = sk = SplitPlan();
   else if (ws_bytes < need) return fail(FGRPO_ERR_WORKSPACE, "varlen_attn_bwd: workspace %zu < %zu", ws_bytes, need);
   else if (!aligned16(ws)) return fail(FGRPO_ERR_ALIGN, "varlen_attn_bwd: workspace must be 16-byte aligned");
   // the scalar offsets of the third form are 32-bit: (queries x heads of a group) x 4 bytes and the two bounds arrays
-  const bool dkv3 = g_tune.attn_dkv != 1 && g_tune.attn_dkv != 2 && (long long)T * (Hq / Hkv) * 4 < (1LL << 31) && (long long)T * 8 < (1LL << 31);
+  const bool dkv3 = tn.attn_dkv != 1 && tn.attn_dkv != 2 && (long long)T * (Hq / Hkv) * 4 < (1LL << 31) && (long long)T * 8 < (1LL << 31);
   if (!dkv3) sq = sk = SplitPlan();
   p.parts_q = sq.parts, p.per_q = sq.per, p.parts_k = sk.parts, p.per_k = sk.per;
   p.part_q = (float*)ws;
   p.part_k = (float*)((char*)ws + need_q);
-  rc = launch_query_side<DqLauncher>(D, hb, p, T, Hq, Hkv, bounds_ws, st);
+  rc = launch_query_side<DqLauncher>(tn, D, hb, p, T, Hq, Hkv, bounds_ws, st);
   if (rc) return rc;
   if (dkv3) {
     rc = launch_attn_dkv3(D, p, st);
@@ -267,7 +270,7 @@ int fgrpo_varlen_attn_bwd_ws(const void* dout, const void* q, const void* k, con
     return launch_attn_merge_bwd(D, p, 128 / hb, st);
   }
   const dim3 grid_k(Hkv, (T + kAttnBQ - 1) / kAttnBQ);
-  if (g_tune.attn_dkv == 1) {
+  if (tn.attn_dkv == 1) {
     if (D == 128) hipLaunchKernelGGL(varlen_attn_dkv_kernel<128>, grid_k, dim3(256), 0, st, p);
     else hipLaunchKernelGGL(varlen_attn_dkv_kernel<64>, grid_k, dim3(256), 0, st, p);
   } else if (D == 128) {

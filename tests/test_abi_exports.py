@@ -89,3 +89,12 @@ def test_backward_panel_plan_respects_the_bound(lib_path):
             assert lib.fgrpo_lmhead_bwd_workspace(T, H, V, 0, hint) >= 2 * cols * T
     assert lib.fgrpo_lmhead_bwd_panel_cols(32768, 1536, 151936, 0, 0) == 21760      # 7 panels: 510 dW tiles each
     assert lib.fgrpo_lmhead_bwd_panel_cols(0, 1536, 151936, 0, 0) < 0
+
+
+def test_attention_calls_read_the_tuning_state_once():
+    """A call that plans a division and then launches must do both by one reading of the settings: another thread may
+    change them in between, and the merge of parts that no kernel wrote would overwrite a finished result."""
+    text = open(os.path.join(ROOT, "async-grpo-nccl_amd", "csrc", "launch_attn.hip")).read()
+    readings = [line.strip() for line in text.splitlines() if "g_tune" in line]
+    assert readings and all(line.startswith("const Tuning tn = g_tune;") for line in readings)
+    assert all(function.count("g_tune") <= 1 for function in text.split("\n}\n"))
