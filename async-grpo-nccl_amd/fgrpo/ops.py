@@ -949,10 +949,10 @@ def fused_grpo_loss(hidden, weight, bias, labels_shifted, old_lp, adv, ref_lp=No
     if idx is None and _fwd_event_sink is None and hidden.shape[0] > 0:
         V = weight.shape[0]
         chunk = int(chunk_tokens) if chunk_tokens and chunk_tokens > 0 else chunk_bound_for(V)
-        return _lib.native().fused_step(hidden, weight, bias, labels_shifted, old_lp, adv, ref_lp, cu_seqlens,
-                                        1.0 / float(temperature), float(clip_low), float(clip_high), float(clip_ratio_c),
-                                        float(kl_beta), loss_agg_mode == "sample_mean", float(denom_override),
-                                        int(panel_hint), _NATIVE_MODES[mode], chunk, KEEP_WHOLE_MAX_BYTES)
+        return tuple(_lib.native().fused_step(hidden, weight, bias, labels_shifted, old_lp, adv, ref_lp, cu_seqlens,
+                                              1.0 / float(temperature), float(clip_low), float(clip_high), float(clip_ratio_c),
+                                              float(kl_beta), loss_agg_mode == "sample_mean", float(denom_override),
+                                              int(panel_hint), _NATIVE_MODES[mode], chunk, KEEP_WHOLE_MAX_BYTES))
     # rows left out of the projection (gathered and scattered with torch), a timed forward, an empty batch
     if not wants_grad:
         lp, ent = _logprob_fwd_rows(hidden, weight, bias, labels_shifted, float(temperature), idx, False, "recompute",

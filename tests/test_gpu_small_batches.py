@@ -263,3 +263,14 @@ def test_logprob_worker_runs_any_model_of_the_four_inputs(dev, wrapped):
     LogProbHarness(Wrapper(model), dev).compute_log_probs_from_samples(samples)
     assert "compact_masked_tokens" in got
     LogProbHarness(Narrow(model), dev).compute_log_probs_from_samples(samples)
+
+
+@pytest.mark.parametrize("trainable", [False, True])
+@pytest.mark.parametrize("compact", [False, True])
+def test_fused_step_returns_a_tuple_on_every_path(dev, compact, trainable):
+    """As every autograd node written in Python does: callers test for it, add to it, use it as a key."""
+    from fgrpo import ops
+    h, w = (torch.randn(n, 64, device=dev).bfloat16().requires_grad_(trainable) for n in (70, 300))
+    out = ops.fused_grpo_loss(h, w, None, torch.randint(0, 300, (70,), device=dev), torch.randn(70, device=dev),
+                              torch.randn(70, device=dev), compact=torch.arange(0, 70, 2, device=dev) if compact else False)
+    assert type(out) is tuple and len(out) == 7
