@@ -803,7 +803,7 @@ class _LMHeadLogprob(torch.autograd.Function):
 
 class _FusedGRPOLoss(torch.autograd.Function):
     """Projection -> logprob -> dual-clip objective in one autograd node, for batches some of whose rows are left out
-    of the projection (the others take the node of csrc/torch_binding.cpp).  The
+    of the projection and for calls under ``torch.jit.trace`` (the others take the node of csrc/torch_binding.cpp).  The
     backward receives the scalar upstream gradient as a device pointer."""
 
     @staticmethod
@@ -924,7 +924,7 @@ def grpo_loss_from_logprobs(lp, labels_shifted, old_lp, adv, ref_lp=None, cu_seq
 def lmhead_logprob(hidden, weight, bias, labels_shifted, temperature=1.0, panel_hint=0,
                    compact=False, keep_logits=None) -> Tuple[torch.Tensor, torch.Tensor]:
     compact = compact if torch.is_tensor(compact) else bool(compact)
-    if not _wants_grad(hidden, weight, bias):
+    if not torch.jit.is_tracing() and not _wants_grad(hidden, weight, bias):
         _grad_mode(keep_logits)                  # refuses an unknown mode, as the differentiable path does
         idx = _valid_rows(labels_shifted, compact)
         return _logprob_fwd_rows(hidden, weight, bias, labels_shifted, float(temperature), idx, False, "recompute",
@@ -944,6 +944,11 @@ def fused_grpo_loss(hidden, weight, bias, labels_shifted, old_lp, adv, ref_lp=No
         raise ValueError(f"Invalid loss_agg_mode: {loss_agg_mode}")
     mode = _grad_mode(keep_logits)
     compact = compact if torch.is_tensor(compact) else bool(compact)
+    if torch.jit.is_tracing():       # a trace records a node written in Python as itself, of any other call only the empty outputs
+        return _FusedGRPOLoss.apply(hidden, weight, bias, labels_shifted, old_lp, adv, ref_lp, cu_seqlens,
+                                    float(temperature), float(clip_low), float(clip_high), float(clip_ratio_c),
+                                    float(kl_beta), loss_agg_mode, float(denom_override), int(panel_hint),
+                                    compact, keep_logits, int(chunk_tokens))
     wants_grad = _wants_grad(hidden, weight, bias, old_lp, adv, ref_lp)
     idx = _valid_rows(labels_shifted, compact)
     if idx is None and _fwd_event_sink is None and hidden.shape[0] > 0:
@@ -1059,9 +1064,28 @@ def varlen_attn_bwd(dout: torch.Tensor, q: torch.Tensor, k: torch.Tensor, v: tor
     return dq, dk, dv
 
 
+class _VarlenAttention(torch.autograd.Function):
+    """The attention node for calls under ``torch.jit.trace`` (the others take that of csrc/torch_binding.cpp)."""
+
+    @staticmethod
+    def forward(ctx, q, k, v, cu_seqlens, softmax_scale, causal, bounds):
+        out, lse, bounds = varlen_attn_fwd(q, k, v, cu_seqlens, softmax_scale, causal, return_bounds=True, bounds=bounds)
+        ctx.save_for_backward(q, k, v, out, lse, cu_seqlens, bounds)
+        ctx.softmax_scale, ctx.causal = softmax_scale, causal
+        return out
+
+    @staticmethod
+    def backward(ctx, dout):
+        q, k, v, out, lse, cu, bounds = ctx.saved_tensors
+        dq, dk, dv = varlen_attn_bwd(dout.to(torch.bfloat16), q, k, v, out, lse, cu, ctx.softmax_scale, ctx.causal, bounds)
+        return dq, dk, dv, None, None, None, None
+
+
 def varlen_attention(q, k, v, cu_seqlens, softmax_scale=None, causal=True, bounds=None) -> torch.Tensor:
     """Differentiable packed self-attention on the HIP kernels (bf16 in, bf16 out).  ``bounds``: segment scratch of an
     earlier call with the same ``cu_seqlens`` and ``causal`` (see ``attention_bounds``)."""
+    if torch.jit.is_tracing():
+        return _VarlenAttention.apply(q, k, v, cu_seqlens, softmax_scale, bool(causal), bounds)
     return _lib.native().varlen_attention(q, k, v, cu_seqlens, softmax_scale, bool(causal), bounds)
 
 

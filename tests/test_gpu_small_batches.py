@@ -274,3 +274,33 @@ def test_fused_step_returns_a_tuple_on_every_path(dev, compact, trainable):
     out = ops.fused_grpo_loss(h, w, None, torch.randint(0, 300, (70,), device=dev), torch.randn(70, device=dev),
                               torch.randn(70, device=dev), compact=torch.arange(0, 70, 2, device=dev) if compact else False)
     assert type(out) is tuple and len(out) == 7
+
+
+@pytest.mark.parametrize("trainable", [False, True])
+@pytest.mark.parametrize("call", ["fused", "fused_rows", "logprob", "attention"])
+def test_traced_calls_run_the_kernels(dev, call, trainable):
+    """A trace replays the call on new inputs, with its gradients: results of the eager call, bit for bit (the batch is
+    too small for divided tiles)."""
+    from fgrpo import ops
+    g = torch.Generator().manual_seed(5)
+    rand = lambda *shape: torch.randn(*shape, generator=g).to(dev)
+    y = torch.randint(0, 300, (70,), generator=g).to(dev)
+    tok, cu, rows = (rand(70) - 6, rand(70)), torch.tensor([0, 30, 70], dtype=torch.int32, device=dev), torch.arange(0, 70, 2, device=dev)
+    f = dict(fused=lambda a, b: ops.fused_grpo_loss(a, b, None, y, *tok),
+             fused_rows=lambda a, b: ops.fused_grpo_loss(a, b, None, y, *tok, compact=rows),
+             logprob=lambda a, b: ops.lmhead_logprob(a, b, None, y),
+             attention=lambda a, b: ops.varlen_attention(a, b, b, cu))[call]
+    shapes = ((70, 4, 64), (70, 2, 64)) if call == "attention" else ((70, 64), (300, 64))
+
+    def leaves():
+        return [rand(*s).bfloat16().requires_grad_(trainable) for s in shapes]
+    traced = torch.jit.trace(f, tuple(leaves()), check_trace=False)
+    args = leaves()
+    whole = lambda out: out if isinstance(out, tuple) else (out,)
+    want, got = whole(f(*args)), whole(traced(*args))
+    assert len(want) == len(got) and all(torch.equal(a, b) for a, b in zip(got, want))
+    assert got[0].requires_grad == trainable
+    if trainable:
+        up = rand(want[0].numel()).to(want[0].dtype).view_as(want[0])
+        for a, b in zip(torch.autograd.grad(got[0], args, up), torch.autograd.grad(want[0], args, up)):
+            assert torch.equal(a, b)
