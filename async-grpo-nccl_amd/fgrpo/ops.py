@@ -34,7 +34,12 @@ def _require_cuda(*tensors) -> torch.device:
 
 
 def _ptr(t: Optional[torch.Tensor]):
-    return None if t is None else t.data_ptr()
+    """Address for a kernel (None: null).  Every optional operand passes here too: a host address would fault the GPU."""
+    if t is None:
+        return None
+    if not t.is_cuda:
+        raise RuntimeError("fgrpo: tensors must live on the GPU (the HIP path has no CPU fallback)")
+    return t.data_ptr()
 
 
 def _stream() -> int:

@@ -304,3 +304,21 @@ def test_traced_calls_run_the_kernels(dev, call, trainable):
         up = rand(want[0].numel()).to(want[0].dtype).view_as(want[0])
         for a, b in zip(torch.autograd.grad(got[0], args, up), torch.autograd.grad(want[0], args, up)):
             assert torch.equal(a, b)
+
+
+def test_host_operands_are_refused(dev):
+    """Operands beside the ones that decide the device: an address in host memory, or labels for fewer rows than there
+    are, must end in an error before anything is launched."""
+    from fgrpo import ops
+    y, lp, old, adv = torch.randint(0, 300, (70,), device=dev), *(torch.randn(70, device=dev) for _ in range(3))
+    h, w = torch.randn(70, 64, device=dev).bfloat16(), torch.randn(300, 64, device=dev).bfloat16()
+    rows, logits = torch.arange(0, 70, 2, device=dev), torch.randn(70, 300, device=dev)
+    for call in (lambda: ops.grpo_loss_from_logprobs(lp, y, old.cpu(), adv),
+                 lambda: ops.grpo_loss_from_logprobs(lp, y, old, adv, ref_lp=old.cpu(), kl_beta=0.1),
+                 lambda: ops.fused_grpo_loss(h, w, None, y, old.cpu(), adv),
+                 lambda: ops.fused_grpo_loss(h, w, None, y, old.cpu(), adv, compact=rows),
+                 lambda: ops.logits_logprob_entropy(logits, y.cpu(), None),
+                 lambda: ops.logits_logprob_bwd(logits, y, None, lp.cpu(), lp),
+                 lambda: ops.grpo_metrics(rows, lp, old.cpu(), None, adv, lp, lp, 0.2, 0.2)):
+        with pytest.raises(RuntimeError, match="must live on the GPU"):
+            call()

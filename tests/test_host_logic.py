@@ -160,3 +160,10 @@ def test_packed_logprobs_container():
         spu.PackedLogProbs(buf.double(), [0, 6])
     with pytest.raises(ValueError):
         p.attach([{}])
+
+
+def test_host_addresses_are_not_handed_to_kernels():
+    from fgrpo import ops
+    assert ops._ptr(None) is None
+    with pytest.raises(RuntimeError, match="must live on the GPU"):
+        ops._ptr(torch.zeros(4))
