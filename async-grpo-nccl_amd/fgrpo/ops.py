@@ -461,6 +461,14 @@ def cu_seqlens_from_position_ids(position_ids: torch.Tensor, max_segments: Optio
     return out[:n]
 
 
+def _row_labels(labels: Optional[torch.Tensor], rows: int) -> Optional[torch.Tensor]:
+    if labels is None:
+        return None
+    if labels.numel() < rows:
+        raise RuntimeError(f"fgrpo: {labels.numel()} labels for {rows} rows of logits")
+    return labels.reshape(-1).to(torch.int64).contiguous()
+
+
 def logits_logprob_entropy(logits: torch.Tensor, labels: Optional[torch.Tensor], ignore_index: Optional[int],
                            want_lp=True, want_ent=True, want_lse=True):
     """Row soft-max statistics of materialised logits [N,V] (bf16/fp32, row stride allowed)."""
@@ -474,7 +482,7 @@ def logits_logprob_entropy(logits: torch.Tensor, labels: Optional[torch.Tensor],
     lp, ent, lse = (mk() if want_lp else None), (mk() if want_ent else None), (mk() if want_lse else None)
     if N == 0:
         return lp, ent, lse
-    lab = None if labels is None else labels.reshape(-1).to(torch.int64).contiguous()
+    lab = _row_labels(labels, N)
     with torch.cuda.device(dev):
         rc = lib.fgrpo_logits_logprob_entropy(_ptr(logits), code, logits.stride(0), N, V, _ptr(lab),
                                               int(ignore_index if ignore_index is not None else 0),
@@ -490,7 +498,7 @@ def logits_logprob_bwd(logits, labels, ignore_index, g, lse) -> torch.Tensor:
     out = torch.empty((N, V), dtype=logits.dtype, device=dev)
     if N == 0:
         return out
-    lab = labels.reshape(-1).to(torch.int64).contiguous()
+    lab = _row_labels(labels, N)
     with torch.cuda.device(dev):
         rc = lib.fgrpo_logits_logprob_bwd(_ptr(logits), _code(logits.dtype), logits.stride(0), N, V, _ptr(lab),
                                           int(ignore_index if ignore_index is not None else 0),

@@ -322,3 +322,12 @@ def test_host_operands_are_refused(dev):
                  lambda: ops.grpo_metrics(rows, lp, old.cpu(), None, adv, lp, lp, 0.2, 0.2)):
         with pytest.raises(RuntimeError, match="must live on the GPU"):
             call()
+
+
+def test_labels_for_fewer_rows_than_there_are_are_refused(dev):
+    from fgrpo import ops
+    y, lp, logits = torch.randint(0, 300, (70,), device=dev), torch.randn(70, device=dev), torch.randn(70, 300, device=dev)
+    with pytest.raises(RuntimeError, match="69 labels for 70 rows"):
+        ops.logits_logprob_entropy(logits, y[:69], None)
+    with pytest.raises(RuntimeError, match="69 labels for 70 rows"):
+        ops.logits_logprob_bwd(logits, y[:69], None, lp, lp)
