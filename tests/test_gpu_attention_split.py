@@ -7,10 +7,30 @@ from oracle import attn_oracle as AO
 
 pytestmark = pytest.mark.gpu
 
-SHAPES = [  # tokens, segment bounds, query heads, K/V heads, head dimension
-    (777, [0, 777], 12, 2, 128), (513, [0, 513], 4, 1, 128), (1500, [0, 1500], 14, 2, 64), (1025, [0, 1025], 8, 8, 64),
-    (2047, [0, 1024, 1030, 2047], 28, 4, 128), (1990, [0, 3, 900, 1990], 3, 1, 64), (4200, [0, 4200], 2, 1, 128),
-    (1300, [0, 1216, 1300], 16, 4, 128), (6000, [0, 6000], 12, 2, 128), (640, [0, 640], 1, 1, 128)]
+# tokens, segment bounds, query heads, K/V heads, head dimension, and which launches have tiles dealt out (f: forward,
+# q: dQ, k: dK/dV) with the causal mask and without
+SHAPES = [
+    (777, [0, 777], 12, 2, 128, "fqk", "k"), (513, [0, 513], 4, 1, 128, "fqk", "fqk"), (1500, [0, 1500], 14, 2, 64, "fqk", "k"),
+    (1025, [0, 1025], 8, 8, 64, "fq", "fq"), (2047, [0, 1024, 1030, 2047], 28, 4, 128, "k", "k"),
+    (1990, [0, 3, 900, 1990], 3, 1, 64, "fqk", "q"), (4200, [0, 4200], 2, 1, 128, "fqk", "fqk"),
+    (1300, [0, 1216, 1300], 16, 4, 128, "k", ""), (6000, [0, 6000], 12, 2, 128, "fqk", "k"), (640, [0, 640], 1, 1, 128, "fq", "fq")]
+CASES = [(*shape[:5], causal, sides) for shape in SHAPES for causal, sides in ((True, shape[5]), (False, shape[6])) if sides]
+
+
+def divided(T, n_seq, Hq, Hkv, D, causal):
+    """Which launches of a call deal tiles out: those that ask for scratch, the backward's two with the other switched to
+    a kernel that cannot."""
+    from fgrpo import _lib
+    need = lambda backward: _lib.load().fgrpo_varlen_attn_workspace(T, n_seq, Hq, Hkv, D, causal, backward) > 0
+    found = "f" if need(0) else ""
+    try:
+        _lib.set_tuning(attn_dkv=1)
+        found += "q" if need(1) else ""
+        _lib.set_tuning(attn_dkv=0, attn_qside=3)
+        found += "k" if need(1) else ""
+    finally:
+        _lib.set_tuning(attn_dkv=0, attn_qside=0)
+    return found
 
 
 def operands(T, Hq, Hkv, D, dev):
@@ -18,14 +38,11 @@ def operands(T, Hq, Hkv, D, dev):
     return [torch.randn(T, n, D, generator=g).bfloat16().to(dev) for n in (Hq, Hkv, Hkv, Hq)]
 
 
-@pytest.mark.parametrize("causal", [True, False])
-@pytest.mark.parametrize("T,cu,Hq,Hkv,D", SHAPES)
-def test_divided_tiles_agree_with_whole_ones(dev, T, cu, Hq, Hkv, D, causal):
+@pytest.mark.parametrize("T,cu,Hq,Hkv,D,causal,sides", CASES)
+def test_divided_tiles_agree_with_whole_ones(dev, T, cu, Hq, Hkv, D, causal, sides):
     """Two roundings to bf16 (probabilities, result) of 2^-9 at most on either side: 2^-7 of the norm between them."""
-    from fgrpo import _lib, ops
-    lib = _lib.load()
-    if causal:       # without the mask some of the shapes fill the device as they are
-        assert lib.fgrpo_varlen_attn_workspace(T, len(cu) - 1, Hq, Hkv, D, causal, 1) > 0, "this shape is meant to be divided"
+    from fgrpo import ops
+    assert divided(T, len(cu) - 1, Hq, Hkv, D, causal) == sides
     q, k, v, do = operands(T, Hq, Hkv, D, dev)
     cu_t = torch.tensor(cu, dtype=torch.int32, device=dev)
     out0, lse = ops.varlen_attn_fwd(q, k, v, cu_t, None, causal)
@@ -42,16 +59,20 @@ def test_divided_tiles_agree_with_whole_ones(dev, T, cu, Hq, Hkv, D, causal):
         assert (x.float() - y.float()).norm() <= 2 ** -7 * y.float().norm(), name
 
 
-def test_divided_forward_against_the_oracle(dev):
+@pytest.mark.parametrize("T,cu,Hq,Hkv,D,causal,sides", [c for c in CASES if c[0] < 2000])
+def test_divided_tiles_against_the_oracle(dev, T, cu, Hq, Hkv, D, causal, sides):
+    """Every launch that is divided (all three at both head dimensions).  Probabilities and results are rounded to bf16,
+    2^-9 each: 2^-8 of the norm for the output and dV; dS, from a delta of the rounded output, is rounded once more
+    on the way to dQ and dK: 2^-7."""
     from fgrpo import ops
-    T, cu, Hq, Hkv, D = SHAPES[4]
     q, k, v, do = operands(T, Hq, Hkv, D, dev)
-    cu_t = torch.tensor(cu, dtype=torch.int32, device=dev)
-    with torch.no_grad():
-        out = ops.varlen_attention(q, k, v, cu_t)
-    want = AO.varlen_attention(q.float().cpu(), k.float().cpu(), v.float().cpu(), torch.tensor(cu), causal=True)
-    want = want[0] if isinstance(want, tuple) else want
-    assert (out.float().cpu() - want).norm() <= 2 ** -8 * want.norm()
+    a, o = [[x.clone().to(d, t).requires_grad_(True) for x in (q, k, v)] for d, t in ((dev, torch.bfloat16), ("cpu", torch.float32))]
+    got = ops.varlen_attention(*a, torch.tensor(cu, dtype=torch.int32, device=dev), None, causal)
+    want = AO.varlen_attention(*o, torch.tensor(cu), causal=causal)
+    got, want = (got, *torch.autograd.grad(got, a, do)), (want, *torch.autograd.grad(want, o, do.float().cpu()))
+    for name, x, y, tol in zip(("out", "dq", "dk", "dv"), got, want, (2 ** -8, 2 ** -7, 2 ** -7, 2 ** -8)):
+        err = ((x.detach().float().cpu() - y.detach()).norm() / y.detach().norm()).item()
+        assert err <= tol, name
 
 
 def test_workspace_is_checked(dev):
