@@ -77,13 +77,18 @@ class TrainerHarness:
 
 def _takes_row_list(model) -> bool:
     """Whether ``compact_masked_tokens`` reaches a forward that ``make_grpo_forward`` made, through wrappers that hand
-    any keyword on; another forward may refuse it."""
+    any keyword on; another forward may refuse it.  A function that wraps such a forward (``functools.wraps``) carries
+    its mark and its signature: what counts is what the function itself takes."""
     while model is not None:
         forward = getattr(model, "forward", None)
+        try:
+            params = inspect.signature(forward, follow_wrapped=False).parameters.values()
+        except (TypeError, ValueError):          # a compiled forward (torch.jit) has none
+            return False
+        if not any(p.kind is p.VAR_KEYWORD or p.name == "compact_masked_tokens" for p in params):
+            return False
         if getattr(forward, "takes_compact_masked_tokens", False):
             return True
-        if not callable(forward) or all(p.kind is not p.VAR_KEYWORD for p in inspect.signature(forward).parameters.values()):
-            return False
         model = getattr(model, "module", None) or getattr(model, "_orig_mod", None)
     return False
 

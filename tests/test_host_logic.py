@@ -167,3 +167,33 @@ def test_host_addresses_are_not_handed_to_kernels():
     assert ops._ptr(None) is None
     with pytest.raises(RuntimeError, match="must live on the GPU"):
         ops._ptr(torch.zeros(4))
+
+
+def test_the_list_of_scored_rows_goes_to_forwards_that_take_it():
+    import functools
+    from types import SimpleNamespace
+    from workers import _takes_row_list
+
+    def made(input_ids=None, labels=None, **unused):
+        return None
+    made.takes_compact_masked_tokens = True
+
+    @functools.wraps(made)
+    def wide(*args, **kwargs):
+        return made(*args, **kwargs)
+
+    @functools.wraps(made)
+    def narrow(input_ids, labels):
+        return made(input_ids=input_ids, labels=labels)
+
+    class Own(torch.nn.Module):
+        def forward(self, input_ids, labels):
+            return input_ids + labels
+
+    traced = torch.jit.trace(Own(), (torch.zeros(1), torch.zeros(1)))
+    inner = SimpleNamespace(forward=made)
+    assert _takes_row_list(inner) and _takes_row_list(SimpleNamespace(forward=wide))
+    assert _takes_row_list(SimpleNamespace(forward=lambda **kw: None, module=inner))
+    for model in (Own(), traced, SimpleNamespace(forward=narrow), SimpleNamespace(forward=narrow, module=inner),
+                  SimpleNamespace(forward=lambda **kw: None), SimpleNamespace(forward=lambda **kw: None, module=traced), lambda **kw: None):
+        assert not _takes_row_list(model)
