@@ -75,17 +75,27 @@ class TrainerHarness:
         return metrics
 
 
+def _takes_keyword(forward, name: str) -> bool:
+    """Whether the function itself, not one that it says it wraps, takes the keyword.  Asked for every batch: a plain
+    function or method is read off its code object (1 us, a signature 33)."""
+    code = getattr(getattr(forward, "__func__", forward), "__code__", None)
+    if code is not None:
+        own = code.co_varnames[code.co_posonlyargcount:code.co_argcount + code.co_kwonlyargcount]
+        return bool(code.co_flags & inspect.CO_VARKEYWORDS) or name in own
+    try:
+        params = inspect.signature(forward, follow_wrapped=False).parameters.values()
+    except (TypeError, ValueError):              # a compiled forward (torch.jit) has none
+        return False
+    return any(p.kind is p.VAR_KEYWORD or (p.name == name and p.kind is not p.POSITIONAL_ONLY) for p in params)
+
+
 def _takes_row_list(model) -> bool:
     """Whether ``compact_masked_tokens`` reaches a forward that ``make_grpo_forward`` made, through wrappers that hand
     any keyword on; another forward may refuse it.  A function that wraps such a forward (``functools.wraps``) carries
     its mark and its signature: what counts is what the function itself takes."""
     while model is not None:
         forward = getattr(model, "forward", None)
-        try:
-            params = inspect.signature(forward, follow_wrapped=False).parameters.values()
-        except (TypeError, ValueError):          # a compiled forward (torch.jit) has none
-            return False
-        if not any(p.kind is p.VAR_KEYWORD or p.name == "compact_masked_tokens" for p in params):
+        if not _takes_keyword(forward, "compact_masked_tokens"):
             return False
         if getattr(forward, "takes_compact_masked_tokens", False):
             return True

@@ -197,3 +197,37 @@ def test_the_list_of_scored_rows_goes_to_forwards_that_take_it():
     for model in (Own(), traced, SimpleNamespace(forward=narrow), SimpleNamespace(forward=narrow, module=inner),
                   SimpleNamespace(forward=lambda **kw: None), SimpleNamespace(forward=lambda **kw: None, module=traced), lambda **kw: None):
         assert not _takes_row_list(model)
+
+
+def test_what_a_forward_takes_is_read_as_its_signature_says():
+    import functools
+    import inspect
+    from workers import _takes_keyword
+
+    class Call:
+        def __call__(self, a, *, rows=None):
+            return a
+
+        def method(self, rows):
+            return rows
+
+        @classmethod
+        def made(cls, **kw):
+            return kw
+
+        @staticmethod
+        def free(a, *args):
+            return a
+
+    def local_only(a):
+        rows = a
+        return rows
+
+    def two(a, rows):
+        return a, rows
+    for f in (Call(), Call().method, Call.made, Call.free, local_only, two, lambda a, rows=1: a, lambda rows, /: rows,
+              functools.partial(two, 1), functools.partial(local_only), Call().__call__):
+        params = inspect.signature(f, follow_wrapped=False).parameters.values()
+        want = any(p.kind is p.VAR_KEYWORD or (p.name == "rows" and p.kind is not p.POSITIONAL_ONLY) for p in params)
+        assert _takes_keyword(f, "rows") == want
+    assert not _takes_keyword(None, "rows") and not _takes_keyword(torch.jit.script(torch.nn.Linear(2, 2)).forward, "rows")
