@@ -331,3 +331,28 @@ def test_labels_for_fewer_rows_than_there_are_are_refused(dev):
         ops.logits_logprob_entropy(logits, y[:69], None)
     with pytest.raises(RuntimeError, match="69 labels for 70 rows"):
         ops.logits_logprob_bwd(logits, y[:69], None, lp, lp)
+
+
+@pytest.mark.parametrize("wrong,message", [
+    (lambda o: dict(labels=o["labels"][:69]), "one entry per token"),
+    (lambda o: dict(old_lp=o["old_lp"][:69]), "old_logprobs has 69 elements"),
+    (lambda o: dict(adv=o["adv"][:69]), "advantages has 69 elements"),
+    (lambda o: dict(ref_lp=o["adv"][:69]), "ref_logprobs has 69 elements"),
+    (lambda o: dict(bias=o["weight"][:299, 0]), "bias must have V elements"),
+    (lambda o: dict(weight=o["weight"][:, :63]), "mismatch"),
+    (lambda o: dict(weight=o["weight"].float()), "share a dtype"),
+    (lambda o: dict(hidden=o["hidden"].half(), weight=o["weight"].half()), "bf16 and fp32 only"),
+    (lambda o: dict(adv=o["adv"].cpu()), "must live on the GPU"),
+    (lambda o: dict(labels=o["labels"].cpu()), "must live on the GPU"),
+    (lambda o: dict(loss_agg_mode="sample_mean"), "needs cu_seqlens"),
+    (lambda o: dict(keep_logits="chunked"), "is not supported")])
+def test_native_step_refuses_operands_that_do_not_fit(dev, wrong, message):
+    """The node in C++ takes its operands' addresses itself: each of its checks must end the call before a launch."""
+    from fgrpo import ops
+    at = dict(hidden=torch.randn(70, 64, device=dev).bfloat16(), weight=torch.randn(300, 64, device=dev).bfloat16(), bias=None,
+              labels=torch.randint(0, 300, (70,), device=dev), old_lp=torch.randn(70, device=dev), adv=torch.randn(70, device=dev))
+    at.update(wrong(at))
+    operands = [at.pop(name) for name in ("hidden", "weight", "bias", "labels", "old_lp", "adv")]
+    operands[0].requires_grad_(True)
+    with pytest.raises(RuntimeError, match=message):
+        ops.fused_grpo_loss(*operands, **at)
