@@ -61,7 +61,8 @@ constexpr int kDkv3Lds = kDkv3LoopLds<HD, KB> > 4 * 32 * KB * kDkv3SumStride<HD>
 // compiler keeps nothing of its own there across one of them; that it puts nothing there in between (a clobber does not
 // reserve a register) takes -amdgpu-mfma-vgpr-form, and the build reads in the compiler's assembly that it did not.
 // The compiler's hazard table does not see these instructions: the first one behind vector arithmetic that formed an
-// operand carries two wait states, instructions on one block are at least four matrix instructions apart.
+// operand carries two wait states, and two instructions on one block, KB * DB matrix instructions apart (eight at HD = 128,
+// two at HD = 64), accumulate into the identical register range, an order the hardware keeps by itself.
 #define FGRPO_DKV3_CLOBBER_64 \
   "a0", "a1", "a2", "a3", "a4", "a5", "a6", "a7", "a8", "a9", "a10", "a11", "a12", "a13", "a14", "a15", \
   "a16", "a17", "a18", "a19", "a20", "a21", "a22", "a23", "a24", "a25", "a26", "a27", "a28", "a29", "a30", "a31", \
@@ -429,6 +430,7 @@ __global__ __launch_bounds__(256, KB == 2 ? 1 : 2) void varlen_attn_dkv3_kernel(
     for (int kb = 0; kb < KB; ++kb) pp[kb][0] = pack(s[kb], 0);
     // ---- dV and dK in quarters of NQ instructions
     constexpr int NQ = KB * DB, EH = 8 * KB;                   // EH: elements of half the rows
+    static_assert(NQ >= 2, "two instructions on one accumulator block never follow each other directly");
     auto quarter = [&](AttnTr (&t)[DB], u32x4_t (&op)[KB][2], auto s2c, auto accc, auto&& side) {
       constexpr int s2 = decltype(s2c)::value, acc = decltype(accc)::value;
       static_for<DB>([&](auto dc) {

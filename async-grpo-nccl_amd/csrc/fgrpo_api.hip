@@ -381,7 +381,8 @@ int run_store_gemm_kmajor(const Tuning& tn, StoreParams p, bool akm, bool bkm, h
 // A small product (128 x 128 tiles, few of them) is one serial walk over its contraction, 0.65 us a K step: 33 us for each
 // gradient of 643 tokens x 1000 entries x 64.  Contracted in pieces it ends sooner for 4 us of one more launch and the
 // fp32 pieces through memory.  Pieces: whole 64-wide K steps, the same range of every segment; 0 = one piece.  fp32
-// operands (three segments) only: a bf16 token's gradient row does not depend on how many tokens there are.
+// operands (three segments) only: a bf16 product's walk is a third as long and stays whole, so that the order of its sums
+// depends on its tile alone.
 int small_split(int M, int N, int K, int nseg, size_t max_elems, int* kchunk) {
   if (nseg != 3) return 0;
   const int steps = K / 64;

@@ -65,9 +65,10 @@ struct DqLauncher {
 // Both sides are estimated, in us, from what was measured: `step` for a step of a work-group alone on its CU, half as
 // much again where two share one; 4 us for the additional launch, 3 TB/s for the sums, written and read.  The tiles of a
 // causal launch walk 0 .. chain steps, evenly; segments of one call are taken to be as long as their mean (twice that
-// at most: the number of parts allowed for).  Decided by shapes alone.  Kernel times, whole | dealt out: forward, one
-// segment of 777 tokens, 12 / 2 heads of 128: 25.6 | 16.1 us, of 6000 tokens 183 | 160; 3 segments of 1024 tokens 29.2 |
-// 42, which the estimate refuses.
+// at most: the number of parts allowed for); one long segment among many short ones is judged by that mean and may stay
+// whole.  Decided by shapes alone.  Whole | dealt out, merge launch included, 12 / 2 heads of 128: one segment of 777
+// tokens, forward 25.2 | 19.2 us, backward 86.7 | 44.2; of 6000 tokens 182 | 161 and 584 | 465; 3 segments of 1024 tokens,
+// backward (dK/dV alone is dealt out) 106 | 85, forward 29.2 | 42, which the estimate refuses.
 struct SplitPlan {
   int parts = 1, per = 1;
 };
