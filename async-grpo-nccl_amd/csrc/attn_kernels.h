@@ -1224,7 +1224,13 @@ __global__ __launch_bounds__(512) void varlen_attn_dkv2_kernel(AttnParams p) {
 //  * every LDS fragment read is inline assembly, requested in groups a group ahead of the matrix instructions that
 //    use it, with counted waits (left to the compiler, each matrix instruction waits for a fragment requested one
 //    instruction earlier: an LDS round trip per 32-cycle instruction); the dO^T / V^T fragments of the second
-//    product are on their way while the softmax arithmetic runs.
+//    product are on their way while the softmax arithmetic runs;
+//  * everything a work-group needs before its first step is one round trip behind its tile number, no load waits for
+//    another, and rows are moved as they lie in memory (AttnRows).  Row loads, first tiles and delta of dQ took 7.5 us of
+//    a work-group's 26.5 at segments of 128..1024 tokens with 12 / 2 heads of 128, of the forward's 20.5 2.5; now 5.5 of
+//    23.3 (Q, dO and O come from HBM, 96 KiB a work-group: bandwidth) and 1.9 of 19.1.  Forward + backward of that
+//    batch, dK/dV's opening included: 540 -> 498 us; 12345 tokens with 14 / 2 heads of 64: 140 -> 132; one sample of
+//    777 tokens, forward: 25.9 -> 24.9; 4 x 8192 tokens with 28 / 4 heads: 8.00 -> 7.91 ms.
 // Every value an asm read delivers passes through attn_settle() right after its wait (see varlen_attn_dkv2_kernel).
 // ---------------------------------------------------------------------------------------------------------
 struct AttnTr {
@@ -1245,6 +1251,82 @@ __device__ __forceinline__ u32x4_t attn_settle_tr(AttnTr& f) {
 __device__ __forceinline__ void attn_settle(u32x4_t& v) { asm volatile("" : "+v"(v)); }
 __device__ __forceinline__ f32x16_t attn_mfma(u32x4_t a, u32x4_t b, f32x16_t acc) {
   return FGRPO_MFMA(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), acc);
+}
+
+// The 32 rows of a wavefront (`rows` of them exist: fewer at the end of the axis, or none), read and written as they lie in
+// memory: instruction i moves 1 KiB, rows i * RPI .., 16 bytes a lane.  Read with each lane on its own row, which is how
+// the matrix instructions want them, an instruction touches 32 rows and takes the address unit about 115 cycles instead
+// of 15; so rows change hands in LDS, in a swizzled patch of the wavefront's own (32 rows, see attn_swz).  The descriptor
+// ends with the last row: rows past it read as zero and are not written.
+template <int HD>
+struct AttnRows {
+  static constexpr int RPI = 1024 / (HD * 2);
+  uint32_t step;                     // bytes from an instruction's rows to the next one's
+  uint32_t off;                      // the lane's place in its KiB of memory ...
+  __amdgpu_buffer_rsrc_t rs;
+  __device__ __forceinline__ AttnRows(const bf16_t* first_row, long long st, int rows, int lane) {
+    long long bytes = rows > 0 ? (rows - 1) * st * 2 + HD * 2 : 0;
+    if (bytes > 0xffffffffLL) bytes = 0xffffffffLL;
+    rs = make_rsrc(first_row, (uint32_t)bytes);
+    off = (uint32_t)(lane / (HD / 8) * st * 2) + lane % (HD / 8) * 16;
+    step = (uint32_t)(RPI * st * 2);
+  }
+  static __device__ __forceinline__ uint32_t place(uint32_t patch, int i, int lane) {      // ... and of its KiB of the patch
+    const int row = i * RPI + lane / (HD / 8);
+    return patch + row * (HD * 2) + ((lane % (HD / 8) ^ attn_swz<HD>(row)) << 4);
+  }
+  __device__ __forceinline__ void load(u32x4_t (&r)[HD / 16]) const {
+#pragma unroll
+    for (int i = 0; i < HD / 16; ++i) r[i] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rs, (int)off, (int)(i * step), 0));
+  }
+  __device__ __forceinline__ void store(const u32x4_t (&r)[HD / 16]) const {
+#pragma unroll
+    for (int i = 0; i < HD / 16; ++i) __builtin_amdgcn_raw_buffer_store_b128(r[i], rs, (int)off, (int)(i * step), 0);
+  }
+};
+// loaded rows -> operand: the lane's own row (lane % 32), chunks 2 s + lane / 32.  rowc: AttnLane::rowc, the patch's base included
+template <int HD>
+__device__ __forceinline__ void attn_rows_operand(bf16x8_t (&f)[HD / 16], const u32x4_t (&r)[HD / 16], uint32_t patch, const uint32_t (&rowc)[HD / 16], int lane) {
+#pragma unroll
+  for (int i = 0; i < HD / 16; ++i) lds_write_u128_asm<0>(AttnRows<HD>::place(patch, i, lane), r[i]);
+  u32x4_t v[HD / 16];
+#pragma unroll
+  for (int st = 0; st < HD / 16; ++st) v[st] = lds_read_u128_asm<0>(rowc[st]);      // a wavefront's LDS instructions run in order
+  wait_lgkm<0>();
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int st = 0; st < HD / 16; ++st) {
+    attn_settle(v[st]);
+    f[st] = __builtin_bit_cast(bf16x8_t, v[st]);
+  }
+}
+// transposed accumulator (HD/32 blocks of 32 d x 32 tokens, the lane's token = its column) -> bf16 rows in memory.  The lanes
+// n and n + 32 of a token hold alternate groups of four columns: they swap one group of every two, and each writes
+// eight columns, 16 bytes, at once.
+template <int HD>
+__device__ __forceinline__ void attn_store_rows(const f32x16_t (&acc)[HD / 32], float mul, const AttnRows<HD>& dst, uint32_t patch,
+                                                const uint32_t (&rowc)[HD / 16], int lane) {
+#pragma unroll
+  for (int db = 0; db < HD / 32; ++db)
+#pragma unroll
+    for (int g = 0; g < 4; g += 2) {
+      uint32_t x[2], y[2];                   // groups g and g + 1
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        x[i] = pack_bf16x2(acc[db][4 * g + 2 * i] * mul, acc[db][4 * g + 2 * i + 1] * mul);
+        y[i] = pack_bf16x2(acc[db][4 * g + 4 + 2 * i] * mul, acc[db][4 * g + 5 + 2 * i] * mul);
+        asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1" : "+v"(x[i]), "+v"(y[i]));
+      }
+      lds_write_u128_asm<0>(rowc[2 * db + g / 2], u32x4_t{x[0], x[1], y[0], y[1]});      // columns 32 db + 8 (g + h) ..: chunk 4 db + g + h
+    }
+  u32x4_t v[HD / 16];
+#pragma unroll
+  for (int i = 0; i < HD / 16; ++i) v[i] = lds_read_u128_asm<0>(AttnRows<HD>::place(patch, i, lane));
+  wait_lgkm<0>();
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int i = 0; i < HD / 16; ++i) attn_settle(v[i]);
+  dst.store(v);
 }
 
 // Direct-to-LDS fetch of 64-row tiles by a 256-thread work-group: instruction i of wavefront w fills the KiB
@@ -1323,13 +1405,18 @@ __global__ __launch_bounds__(256, 2) void varlen_attn_fwd2_kernel(AttnParams p) 
   const bool head_ok = head_g < G;
   const int hq = hkv * G + (head_ok ? head_g : G - 1);
   const int q0 = min(max(p.order_q[unit / p.Hkv], 0), ntile - 1) * RB;
-  const int tq = q0 + 32 * (wave % WPH) + (lane & 31);
-  const bool valid = head_ok && tq < p.T;
-  const int lo = valid ? p.seg_start[tq] : 1;
-  const int hi = valid ? (p.causal ? tq : p.seg_end[tq] - 1) : 0;
-  const int last = (q0 + RB - 1 < p.T ? q0 + RB - 1 : p.T - 1);
-  int k_begin = max(__builtin_amdgcn_readfirstlane(p.seg_start[q0]), 0);
-  int k_end = min(__builtin_amdgcn_readfirstlane(p.causal ? last + 1 : p.seg_end[last]), p.T);
+  const int last = min(q0 + RB, p.T) - 1;
+  // this wavefront's queries wfirst .. wlast, what they see, and the walk of the work-group: indices are clamped instead
+  // of branched around, so that all of it is one round trip behind the tile number
+  const int wfirst = q0 + 32 * (wave % WPH), wl = min(wfirst + 31, p.T - 1), wf = min(wfirst, wl);
+  const int wrows = head_ok ? max(wl - wfirst + 1, 0) : 0;      // 32, fewer at the end of the axis, or none (a tile may end before its last wavefront's queries)
+  const int tq = wfirst + (lane & 31);
+  const bool valid = (lane & 31) < wrows, wave_full = wrows == 32;
+  const int s_first = p.seg_start[q0], s_wf = p.seg_start[wf], s_wl = p.seg_start[wl], s_tq = p.seg_start[min(tq, p.T - 1)];
+  int e_last = last + 1, e_wl = wl + 1, e_wf = wf + 1, e_tq = tq + 1;      // one past the last key seen
+  if (!p.causal) e_last = p.seg_end[last], e_wl = p.seg_end[wl], e_wf = p.seg_end[wf], e_tq = p.seg_end[min(tq, p.T - 1)];
+  int k_begin = max(__builtin_amdgcn_readfirstlane(s_first), 0);           // wavefront-uniform loop bounds, inside [0, T]
+  int k_end = min(__builtin_amdgcn_readfirstlane(e_last), p.T);
   int np = 1;
   if constexpr (SPLIT) {                   // this part's share of the steps
     const int steps = attn_steps(k_begin, k_end);
@@ -1338,26 +1425,10 @@ __global__ __launch_bounds__(256, 2) void varlen_attn_fwd2_kernel(AttnParams p) 
     k_end = min(k_end, k_begin + kAttnBK * (steps * (part + 1) / np));
     k_begin += kAttnBK * (steps * part / np);
   }
-  const int wfirst = q0 + 32 * (wave % WPH), wlast = (wfirst + 31 < p.T ? wfirst + 31 : p.T - 1);
-  const bool wave_on = head_ok && wfirst < p.T;
-  const int w_lo = wave_on ? p.seg_start[wfirst] : 1;
-  const int w_hi = wave_on ? (p.causal ? wlast : p.seg_end[wlast] - 1) : 0;
-  const bool wave_full = wave_on && wfirst + 31 < p.T;
-  const int w_lo_max = wave_full ? p.seg_start[wlast] : 0x7fffffff;
-  const int w_hi_min = wave_full ? (p.causal ? wfirst : p.seg_end[wfirst] - 1) : -1;
-
-  bf16x8_t qf[KS];
-  attn_row_operand(qf, p.q + (long long)(valid ? tq : 0) * p.q_st + (long long)hq * p.q_sh, valid, h);
-#pragma unroll
-  for (int st = 0; st < KS; ++st) asm volatile("" : "+v"(qf[st]));     // complete before the loop: nothing in it waits for them behind a tile load
-
-  f32x16_t acc_o[DB];
-#pragma unroll
-  for (int db = 0; db < DB; ++db)
-#pragma unroll
-    for (int r = 0; r < 16; ++r) acc_o[db][r] = 0.f;
-  float m_run = -INFINITY, l_run = 0.f;
-  const float c = p.scale * kLog2e;
+  const bool wave_on = wrows > 0;
+  const int w_lo = wave_on ? s_wf : 1, w_hi = wave_on ? e_wl - 1 : 0;
+  // keys in [w_lo_max, w_hi_min] are visible to every query of the wavefront (only when all 32 rows exist)
+  const int w_lo_max = wave_full ? s_wl : 0x7fffffff, w_hi_min = wave_full ? e_wf - 1 : -1;
 
   const bf16_t* kbase = p.k + (long long)hkv * p.k_sh;
   const bf16_t* vbase = p.v + (long long)hkv * p.v_sh;
@@ -1372,7 +1443,27 @@ __global__ __launch_bounds__(256, 2) void varlen_attn_fwd2_kernel(AttnParams p) 
     ck.next();
     cv.next();
   };
+  // the first tiles and the query rows travel together
   if (k_begin < k_end) fetch(0);
+  u32x4_t rq[KS];
+  AttnRows<HD>(p.q + (long long)wf * p.q_st + (long long)hq * p.q_sh, p.q_st, wrows, lane).load(rq);
+  __builtin_amdgcn_sched_barrier(0);
+
+  const int lo = valid ? s_tq : 1, hi = valid ? e_tq - 1 : 0;
+  f32x16_t acc_o[DB];
+#pragma unroll
+  for (int db = 0; db < DB; ++db)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc_o[db][r] = 0.f;
+  float m_run = -INFINITY, l_run = 0.f;
+  const float c = p.scale * kLog2e;
+  // the rows pass through this wavefront's part of the second buffer, which the first step fills again
+  const uint32_t patch = lds0 + 2 * kAttnTile + wave * (32 * HD * 2);
+  uint32_t rowp[KS];
+#pragma unroll
+  for (int st = 0; st < KS; ++st) rowp[st] = (uint32_t)L.rowc[st] + (patch - lds0);
+  bf16x8_t qf[KS];
+  attn_rows_operand<HD>(qf, rq, patch, rowp, lane);
   FGRPO_WAIT_VMCNT(0);
   wg_barrier();
   // a step on LDS buffer `cur`, a compile-time constant: buffer, tile and block are the instruction's offset field
@@ -1515,11 +1606,18 @@ __global__ __launch_bounds__(256, 2) void varlen_attn_fwd2_kernel(AttnParams p) 
       return;
     }
   }
-  if (valid) {
-    const float inv = l > 0.f ? 1.f / l : 0.f;
-    attn_store_rowmajor(acc_o, inv, p.out + ((long long)tq * p.Hq + hq) * kHD, h);
-    if (h == 0) p.lse[(long long)hq * p.T + tq] = l > 0.f ? m_run * p.scale + __logf(l) : -INFINITY;
+  // the tiles have been read: rows leave through this wavefront's part of the first buffer (lane formed anew: held across
+  // the loop, what hangs on it would cost registers)
+  const int lane_e = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
+  const uint32_t patch_out = lds0 + wave * (32 * HD * 2);
+  uint32_t rowo[KS];
+  {
+    const AttnLane<HD> E = attn_lane<HD>(lane_e);
+#pragma unroll
+    for (int st = 0; st < KS; ++st) rowo[st] = patch_out + (uint32_t)E.rowc[st];
   }
+  attn_store_rows<HD>(acc_o, l > 0.f ? 1.f / l : 0.f, AttnRows<HD>(p.out + ((long long)wf * p.Hq + hq) * kHD, (long long)p.Hq * kHD, wrows, lane_e), patch_out, rowo, lane_e);
+  if (lane_e < wrows) p.lse[(long long)hq * p.T + wf + lane_e] = l > 0.f ? m_run * p.scale + __logf(l) : -INFINITY;
 }
 
 // dQ in the same form (see varlen_attn_fwd2_kernel).  A 64-key step runs as six phases of eight matrix instructions
@@ -1551,13 +1649,18 @@ __global__ __launch_bounds__(256, 2) void varlen_attn_dq2_kernel(AttnParams p) {
   const bool head_ok = head_g < G;
   const int hq = hkv * G + (head_ok ? head_g : G - 1);
   const int q0 = min(max(p.order_q[unit / p.Hkv], 0), ntile - 1) * RB;
-  const int tq = q0 + 32 * (wave % WPH) + (lane & 31);
-  const bool valid = head_ok && tq < p.T;
-  const int lo = valid ? p.seg_start[tq] : 1;
-  const int hi = valid ? (p.causal ? tq : p.seg_end[tq] - 1) : 0;
-  const int last = (q0 + RB - 1 < p.T ? q0 + RB - 1 : p.T - 1);
-  int k_begin = max(__builtin_amdgcn_readfirstlane(p.seg_start[q0]), 0);
-  int k_end = min(__builtin_amdgcn_readfirstlane(p.causal ? last + 1 : p.seg_end[last]), p.T);
+  const int last = min(q0 + RB, p.T) - 1;
+  // this wavefront's queries wfirst .. wlast, what they see, and the walk of the work-group: indices are clamped instead
+  // of branched around, so that all of it is one round trip behind the tile number
+  const int wfirst = q0 + 32 * (wave % WPH), wl = min(wfirst + 31, p.T - 1), wf = min(wfirst, wl);
+  const int wrows = head_ok ? max(wl - wfirst + 1, 0) : 0;      // 32, fewer at the end of the axis, or none (a tile may end before its last wavefront's queries)
+  const int tq = wfirst + (lane & 31);
+  const bool valid = (lane & 31) < wrows, wave_full = wrows == 32;
+  const int s_first = p.seg_start[q0], s_wf = p.seg_start[wf], s_wl = p.seg_start[wl], s_tq = p.seg_start[min(tq, p.T - 1)];
+  int e_last = last + 1, e_wl = wl + 1, e_wf = wf + 1, e_tq = tq + 1;      // one past the last key seen
+  if (!p.causal) e_last = p.seg_end[last], e_wl = p.seg_end[wl], e_wf = p.seg_end[wf], e_tq = p.seg_end[min(tq, p.T - 1)];
+  int k_begin = max(__builtin_amdgcn_readfirstlane(s_first), 0);           // wavefront-uniform loop bounds, inside [0, T]
+  int k_end = min(__builtin_amdgcn_readfirstlane(e_last), p.T);
   int np = 1;
   if constexpr (SPLIT) {                   // this part's share of the steps
     const int steps = attn_steps(k_begin, k_end);
@@ -1566,48 +1669,10 @@ __global__ __launch_bounds__(256, 2) void varlen_attn_dq2_kernel(AttnParams p) {
     k_end = min(k_end, k_begin + kAttnBK * (steps * (part + 1) / np));
     k_begin += kAttnBK * (steps * part / np);
   }
-  const int wfirst = q0 + 32 * (wave % WPH), wlast = (wfirst + 31 < p.T ? wfirst + 31 : p.T - 1);
-  const bool wave_on = head_ok && wfirst < p.T;
-  const int w_lo = wave_on ? p.seg_start[wfirst] : 1;
-  const int w_hi = wave_on ? (p.causal ? wlast : p.seg_end[wlast] - 1) : 0;
-  const bool wave_full = wave_on && wfirst + 31 < p.T;
-  const int w_lo_max = wave_full ? p.seg_start[wlast] : 0x7fffffff;
-  const int w_hi_min = wave_full ? (p.causal ? wfirst : p.seg_end[wfirst] - 1) : -1;
-
-  bf16x8_t qf[KS], dof[KS];
-  attn_row_operand(qf, p.q + (long long)(valid ? tq : 0) * p.q_st + (long long)hq * p.q_sh, valid, h);
-  attn_row_operand(dof, p.dout + ((long long)(valid ? tq : 0) * p.Hq + hq) * kHD, valid, h);
-  const float lse2 = valid ? p.lse[(long long)hq * p.T + tq] * kLog2e : 0.f;
-  // delta = rowsum(dO * O) of the lane's query: each lane half holds alternate 8-element pieces of the row
-  float dl = 0.f;
-  {
-    bf16x8_t of[KS];
-    attn_row_operand(of, p.out_fwd + ((long long)(valid ? tq : 0) * p.Hq + hq) * kHD, valid, h);
-#pragma unroll
-    for (int st = 0; st < KS; ++st) {
-      const u32x4_t x = __builtin_bit_cast(u32x4_t, dof[st]), y = __builtin_bit_cast(u32x4_t, of[st]);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        dl += __uint_as_float(x[i] << 16) * __uint_as_float(y[i] << 16);
-        dl += __uint_as_float(x[i] & 0xffff0000u) * __uint_as_float(y[i] & 0xffff0000u);
-      }
-    }
-    dl += attn_swap32(dl);
-    if (valid && h == 0 && part == 0) p.delta[(long long)hq * p.T + tq] = -dl;   // negated, for the dK/dV kernel, launched after this one
-  }
-  const float c = p.scale * kLog2e;
-#pragma unroll
-  for (int st = 0; st < KS; ++st) asm volatile("" : "+v"(qf[st]), "+v"(dof[st]));     // complete before the loop
-  // finite also for a query that sees no key at all (lse = -inf; every pair of such a query is hidden and gets its
-  // zero from the score, see hide() below): -inf * c + inf would be a NaN
-  float lse2_v = lse2 == -INFINITY ? 0.f : lse2;
-  asm volatile("" : "+v"(lse2_v));
-
-  f32x16_t acc[DB];
-#pragma unroll
-  for (int db = 0; db < DB; ++db)
-#pragma unroll
-    for (int r = 0; r < 16; ++r) acc[db][r] = 0.f;
+  const bool wave_on = wrows > 0;
+  const int w_lo = wave_on ? s_wf : 1, w_hi = wave_on ? e_wl - 1 : 0;
+  // keys in [w_lo_max, w_hi_min] are visible to every query of the wavefront (only when all 32 rows exist)
+  const int w_lo_max = wave_full ? s_wl : 0x7fffffff, w_hi_min = wave_full ? e_wf - 1 : -1;
 
   const bf16_t* kbase = p.k + (long long)hkv * p.k_sh;
   const bf16_t* vbase = p.v + (long long)hkv * p.v_sh;
@@ -1622,7 +1687,49 @@ __global__ __launch_bounds__(256, 2) void varlen_attn_dq2_kernel(AttnParams p) {
     ck.next();
     cv.next();
   };
+  // the first tiles, the rows of Q, dO and O and the log-sum-exps travel together
   if (k_begin < k_end) fetch(0);
+  u32x4_t rq[KS], rdo[KS], ro[KS];
+  const long long o_st = (long long)p.Hq * kHD, o_off = (long long)wf * o_st + (long long)hq * kHD;
+  AttnRows<HD>(p.q + (long long)wf * p.q_st + (long long)hq * p.q_sh, p.q_st, wrows, lane).load(rq);
+  AttnRows<HD>(p.dout + o_off, o_st, wrows, lane).load(rdo);
+  AttnRows<HD>(p.out_fwd + o_off, o_st, wrows, lane).load(ro);
+  const float lse2 = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(make_rsrc(p.lse + (long long)hq * p.T + wf, (uint32_t)wrows * 4), (lane & 31) * 4, 0, 0)) * kLog2e;
+  __builtin_amdgcn_sched_barrier(0);
+
+  const int lo = valid ? s_tq : 1, hi = valid ? e_tq - 1 : 0;
+  const float c = p.scale * kLog2e;
+  f32x16_t acc[DB];
+#pragma unroll
+  for (int db = 0; db < DB; ++db)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[db][r] = 0.f;
+  // the rows pass through this wavefront's part of the second buffer, which the first step fills again
+  const uint32_t patch = lds0 + 2 * kAttnTile + wave * (32 * HD * 2);
+  uint32_t rowp[KS];
+#pragma unroll
+  for (int st = 0; st < KS; ++st) rowp[st] = (uint32_t)L.rowc[st] + (patch - lds0);
+  bf16x8_t qf[KS], dof[KS], of[KS];
+  attn_rows_operand<HD>(qf, rq, patch, rowp, lane);
+  attn_rows_operand<HD>(dof, rdo, patch, rowp, lane);
+  attn_rows_operand<HD>(of, ro, patch, rowp, lane);
+  // delta = rowsum(dO * O) of the lane's query: each lane half holds alternate 8-element pieces of the row
+  float dl = 0.f;
+#pragma unroll
+  for (int st = 0; st < KS; ++st) {
+    const u32x4_t x = __builtin_bit_cast(u32x4_t, dof[st]), y = __builtin_bit_cast(u32x4_t, of[st]);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      dl += __uint_as_float(x[i] << 16) * __uint_as_float(y[i] << 16);
+      dl += __uint_as_float(x[i] & 0xffff0000u) * __uint_as_float(y[i] & 0xffff0000u);
+    }
+  }
+  dl += attn_swap32(dl);
+  if (valid && h == 0 && part == 0) p.delta[(long long)hq * p.T + tq] = -dl;   // negated, for the dK/dV kernel, launched after this one
+  // finite also for a query that sees no key at all (lse = -inf; every pair of such a query is hidden and gets its
+  // zero from the score, see hide() below): -inf * c + inf would be a NaN
+  float lse2_v = lse2 == -INFINITY ? 0.f : lse2;
+  asm volatile("" : "+v"(lse2_v));
   FGRPO_WAIT_VMCNT(0);
   wg_barrier();
   // a step on LDS buffer `cur`, a compile-time constant: buffer, tile and block are the instruction's offset field
@@ -1804,7 +1911,17 @@ __global__ __launch_bounds__(256, 2) void varlen_attn_dq2_kernel(AttnParams p) {
       return;
     }
   }
-  if (valid) attn_store_rowmajor(acc, p.scale, p.dq + ((long long)tq * p.Hq + hq) * kHD, h);   // dS was kept / scale
+  // the tiles have been read: rows leave through this wavefront's part of the first buffer (lane formed anew: held across
+  // the loop, what hangs on it would cost registers)
+  const int lane_e = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
+  const uint32_t patch_out = lds0 + wave * (32 * HD * 2);
+  uint32_t rowo[KS];
+  {
+    const AttnLane<HD> E = attn_lane<HD>(lane_e);
+#pragma unroll
+    for (int st = 0; st < KS; ++st) rowo[st] = patch_out + (uint32_t)E.rowc[st];
+  }
+  attn_store_rows<HD>(acc, p.scale, AttnRows<HD>(p.dq + ((long long)wf * p.Hq + hq) * kHD, (long long)p.Hq * kHD, wrows, lane_e), patch_out, rowo, lane_e);   // dS was kept / scale
 }
 
 __device__ __forceinline__ void attn_load8(const float* src, float (&v)[8]) {

@@ -233,16 +233,24 @@ __global__ __launch_bounds__(256, KB == 2 ? 1 : 2) void varlen_attn_dkv3_kernel(
   };
   auto fence = []() { __builtin_amdgcn_sched_barrier(0); };
 
-  // What a work-group needs before it can start, one round trip behind the other only where an address depends on it:
-  // V tile and first item, then the K rows and the key ranges, then the second item (not waited for here)
+  // What a work-group needs before it can start, all of it under way at once: the V tile, the K tile (both shared; K stays in
+  // wavefront 0's second buffer until every wavefront has read its operands) and the first items.  Read with each lane on
+  // its own row, K was 16 instructions a wavefront of which each touches 32 rows: 5.8 us from the segment bounds to the first
+  // item, of 46 a work-group took at segments of 128..1024 tokens; now 3.7.
+  constexpr uint32_t kStage = kBuf;
   {
     const int row = wave * RPI + lane / (HD / 8), ch = (lane % (HD / 8)) ^ attn_swz<HD>(row);      // 4 RPI rows a step: the same swizzle
-    const uint32_t fvo = (uint32_t)((row * p.v_st + ch * 8) * 2);
-    const __amdgpu_buffer_rsrc_t rsv = make_rsrc(p.v + (long long)hkv * p.v_sh + (long long)k0 * p.v_st, (uint32_t)min((klast - k0) * p.v_st * 2 + RB, 0xffffffffLL));
+    auto shared_tile = [&](const bf16_t* first, long long st, uint32_t lds) {
+      const uint32_t off = (uint32_t)((row * st + ch * 8) * 2);
+      const __amdgpu_buffer_rsrc_t rs = make_rsrc(first, (uint32_t)min((klast - k0) * st * 2 + RB, 0xffffffffLL));
 #pragma unroll
-    for (int i = 0; i < kKeys / RPI / 4; ++i)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rsv, FGRPO_LDS_AT(lds0 + 4 * 2 * kBuf + wave * 1024 + i * 4096), 16, (int)fvo, (int)(i * 4 * RPI * p.v_st * 2), 0, 0);
+      for (int i = 0; i < kKeys / RPI / 4; ++i)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, FGRPO_LDS_AT(lds + wave * 1024 + i * 4096), 16, (int)off, (int)(i * 4 * RPI * st * 2), 0, 0);
+    };
+    shared_tile(p.k + (long long)hkv * p.k_sh + (long long)k0 * p.k_st, p.k_st, lds0 + kStage);
+    shared_tile(p.v + (long long)hkv * p.v_sh + (long long)k0 * p.v_st, p.v_st, lds0 + 4 * 2 * kBuf);
   }
+  static_assert(kKeys * RB <= kBuf && kKeys % (4 * RPI) == 0, "the K tile fits a buffer, in whole instructions of every wavefront");
   int g_c = g_f, qb = qb_f;                                    // the item being computed
   constexpr int kItemLoads = 2 * NLD + 2;
   auto fetch_item = [&](auto bc) {
@@ -254,35 +262,38 @@ __global__ __launch_bounds__(256, KB == 2 ? 1 : 2) void varlen_attn_dkv3_kernel(
     static_for<NLD>([&](auto ic) { fetch_d(ic, base_w + b * kBuf, sd); });
   };
   if (first < NI) fetch_item(std::integral_constant<int, 0>{});
-  // K rows of the key blocks as operands
-  u32x4_t kf[KB][KS];
+  static_for<NACC>([&](auto rc) { dkv3_acc_clear<NACC, decltype(rc)::value>(); });      // under the loads
   // the queries that see the lane's key: key_n of them, from the key itself (causal) or its segment's start on; kept
   // relative to the lane's first row of a query block
   int key_lo[KB];
   uint32_t key_n[KB];
 #pragma unroll
   for (int kb = 0; kb < KB; ++kb) {
-    bf16x8_t f[KS];
     const int key = k0 + 32 * kb + (lane & 31), kc = min(key, p.T - 1);
-    attn_row_operand(f, p.k + (long long)kc * p.k_st + (long long)hkv * p.k_sh, key < p.T, h);
-#pragma unroll
-    for (int st = 0; st < KS; ++st) kf[kb][st] = __builtin_bit_cast(u32x4_t, f[st]);
     const int lo = p.causal ? kc : p.seg_start[kc];
     key_lo[kb] = lo - 4 * h;
     key_n[kb] = key < p.T ? (uint32_t)max(min(p.seg_end[kc], q_end) - lo, 0) : 0u;
-  }
-  fence();
-  if (first < NI) fetch_item(std::integral_constant<int, 1>{});
-  static_for<NACC>([&](auto rc) { dkv3_acc_clear<NACC, decltype(rc)::value>(); });      // under the loads
-#pragma unroll
-  for (int kb = 0; kb < KB; ++kb) {
-#pragma unroll
-    for (int st = 0; st < KS; ++st) asm volatile("" : "+v"(kf[kb][st]));                // complete before the loop
     asm volatile("" : "+v"(key_lo[kb]), "+v"(key_n[kb]));
   }
-  if (first < NI) FGRPO_WAIT_VMCNT(kItemLoads);                 // everything but the second item
-  else FGRPO_WAIT_VMCNT(0);
-  wg_barrier();                                                // the whole V tile is there
+  FGRPO_WAIT_VMCNT(0);
+  wg_barrier();                                                // the whole K and V tiles are there
+  u32x4_t kf[KB][KS];                                          // K rows of the key blocks as operands
+  {
+    const uint32_t ka = lds0 + kStage - base_w;
+#pragma unroll
+    for (int st = 0; st < KS; ++st) {
+      kf[0][st] = lds_read_u128_asm<0>(rowc[st] + ka);
+      if constexpr (KB == 2) kf[KB - 1][st] = lds_read_u128_asm<32 * RB>(rowc[st] + ka);
+    }
+  }
+  wait_lgkm<0>();
+  fence();
+#pragma unroll
+  for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+    for (int st = 0; st < KS; ++st) attn_settle(kf[kb][st]);
+  wg_barrier();                                                // K has been read: the second item may have the buffer
+  if (first < NI) fetch_item(std::integral_constant<int, 1>{});
 
   u32x4_t qf[KS];                                              // Q rows of the item; the first half is requested by the item before
   auto req_q = [&](auto offc, auto stc) { qf[decltype(stc)::value] = lds_read_u128_asm<decltype(offc)::value>(rowc[decltype(stc)::value]); };

@@ -14,6 +14,9 @@ int launch_attn_merge_bwd(int D, const AttnParams& p, int rb, hipStream_t st);
 }
 
 namespace {
+// The hand-scheduled query-side kernels address a wavefront's 32 query rows with 32-bit byte offsets.
+bool wave_rows_in_reach(long long q_st, int Hq, int D) { return 31 * q_st * 2 + D * 2 < (1LL << 32) && 62LL * Hq * D + D * 2 < (1LL << 32); }
+
 // Query heads per work-group of the query-side kernels (tile = 128 / heads tokens).  Short segments gain from short
 // tiles (less masked work on the diagonal and at segment boundaries) as long as the heads of a group fill the
 // work-group; long ones do not care, and a lone head per K/V head has nothing to share.
@@ -199,7 +202,8 @@ int fgrpo_varlen_attn_fwd_ws(const void* q, const void* k, const void* v, long l
     rc = fgrpo_varlen_attn_bounds(cu, n_seq, T, causal, bounds_ws, stream);
     if (rc) return rc;
   }
-  const Tuning tn = g_tune;   // one reading of the tuning state per call: the kernel launched is the one the split was planned for
+  Tuning tn = g_tune;         // one reading of the tuning state per call: the kernel launched is the one the split was planned for
+  if (!wave_rows_in_reach(q_st, Hq, D)) tn.attn_qside = 1;
   const int hb = attn_heads_per_group(tn, Hq / Hkv, T, n_seq);
   SplitPlan sp = plan_query_split(tn, T, n_seq, Hq, Hkv, D, causal, true);
   const size_t need = query_split_bytes(sp, T, Hq, D, true);
@@ -250,7 +254,8 @@ int fgrpo_varlen_attn_bwd_ws(const void* dout, const void* q, const void* k, con
     rc = fgrpo_varlen_attn_bounds(cu, n_seq, T, causal, bounds_ws, stream);
     if (rc) return rc;
   }
-  const Tuning tn = g_tune;   // one reading of the tuning state per call: the kernel launched is the one the split was planned for
+  Tuning tn = g_tune;         // one reading of the tuning state per call: the kernel launched is the one the split was planned for
+  if (!wave_rows_in_reach(q_st, Hq, D)) tn.attn_qside = 1;
   const int hb = attn_heads_per_group(tn, Hq / Hkv, T, n_seq);
   SplitPlan sq = plan_query_split(tn, T, n_seq, Hq, Hkv, D, causal, false), sk = plan_key_split(tn, T, n_seq, Hq, Hkv, D, causal);
   const size_t need_q = query_split_bytes(sq, T, Hq, D, false), need = need_q + key_split_bytes(sk, T, Hkv, D);

@@ -58,6 +58,20 @@ def check(dev, name, T, cu, Hq, Hkv, causal, seed=0, softmax_scale=None, backwar
         assert rel <= GRAD_REL, f"{name}: {nm} max error {rel} of the largest entry"
 
 
+@pytest.mark.parametrize("stride,Hq,D", [(69273656, 2, 64), (69273664, 2, 64), (69273656, 3, 128), (69273664, 3, 128)])
+def test_forward_of_query_rows_far_apart(dev, stride, Hq, D):
+    """Either side of the last token stride whose 32 rows 32-bit offsets reach, where the kernel changes (69273656):
+    both compute the same products in the same order, so the results are those of packed rows bit for bit."""
+    from fgrpo import ops
+    T = 3
+    q, k, v, _ = (x.to(dev) for x in make(T, Hq, 1, seed=5, D=D))
+    far = torch.empty((T - 1) * stride + Hq * D, dtype=torch.bfloat16, device=dev).as_strided((T, Hq, D), (stride, D, 1))
+    far.copy_(q)
+    cu = torch.tensor([0, T], dtype=torch.int32, device=dev)
+    for name, a, b in zip(("out", "lse"), ops.varlen_attn_fwd(q, k, v, cu), ops.varlen_attn_fwd(far, k, v, cu)):
+        assert torch.equal(a, b), name
+
+
 @pytest.mark.parametrize("causal", [True, False])
 def test_small_segments_share_a_tile(dev, causal):
     check(dev, "short segments", 200, [0, 5, 6, 70, 71, 72, 200], 4, 2, causal, seed=1)
