@@ -114,6 +114,33 @@ __device__ __forceinline__ int attn_key_items(int q_begin, int q_end, int G) {
   return q_end > q_begin ? (q_end - q_begin + kDkv3Rows - 1) / kDkv3Rows * G : 0;
 }
 
+// Which 128-key tile, K/V head and piece (of kPer128 a tile is dealt in) work-group `bid` takes.  Work-groups go to the 8
+// XCDs round-robin (work-group b runs on XCD b % 8, each with its own L2).  All pieces of a tile and head run on one XCD, one
+// behind the other: they read the same Q and dO rows; and where the K/V heads divide eight, an XCD stays with one head.
+// The units (tile, head) that no longer go round the eight are dealt to all of them piece by piece.
+// With the pieces of a tile on several XCDs each row came through several L2s; dQ + dK/dV, before -> after: 32768 tokens
+// in segments of 128..512, 14 / 2 heads of 64 181 -> 148 us; 36000 in 128..2048, 16 / 4 heads of 128 654 -> 639; 9000 in
+// 128..1024, 28 / 4 heads 216.5 -> 213.7; 4 x 8192, 28 / 4 heads 5.70 -> 5.50 ms; 32 / 8 heads of 64 unchanged (the
+// same order as before).  Runs of neighbouring tiles on one XCD (256 .. 4096 tokens) were no better, and worse where they
+// disturbed the order by work; so were XCDs taken in alternating direction, which mixes the heads.
+struct KeyPick {
+  int rank, head, piece;       // rank: place in the launch order; negative: no work
+};
+__host__ __device__ inline KeyPick attn_key_pick(int bid, int ntile, int pieces, int Hkv) {
+  const int xcd = bid & 7, slot = bid >> 3, units = ntile * Hkv, rounds = units / 8;
+  int u = slot / pieces * 8 + xcd, piece = slot % pieces;
+  if (slot >= rounds * pieces) {
+    const int i = (slot - rounds * pieces) * 8 + xcd;
+    u = rounds * 8 + i / pieces, piece = i % pieces;
+    if (u >= units) return KeyPick{-1, 0, 0};
+  }
+  return KeyPick{u / Hkv, u % Hkv, piece};
+}
+inline long long attn_key_blocks(long long ntile, int pieces, int Hkv) {      // work-groups of a launch (or of one share): whole rows of eight
+  const long long units = ntile * Hkv, rounds = units / 8;
+  return 8 * (rounds * pieces + ((units - 8 * rounds) * pieces + 7) / 8);
+}
+
 // KB key blocks of 32 (2: one wavefront per SIMD; 1, head dimension 64: two).  SPLIT: a tile's items are dealt to the
 // wavefronts of several work-groups (attn_parts), item n to wavefront n % (4 np) of them.
 template <int HD, int KB, bool SPLIT>
@@ -128,10 +155,12 @@ __global__ __launch_bounds__(256, KB == 2 ? 1 : 2) void varlen_attn_dkv3_kernel(
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int G = p.Hq / p.Hkv;
   const int share = SPLIT ? (int)blockIdx.x / p.blocks_k : 0, bid = (int)blockIdx.x - share * (SPLIT ? p.blocks_k : 0);
-  const int hkv = bid % p.Hkv, rank = bid / p.Hkv;
   constexpr int kPer128 = 128 / kKeys;
   const int ntile = (p.T + kKeys - 1) / kKeys, n128 = (p.T + 127) / 128;
-  const int tile = min(max(p.order_k[rank / kPer128], 0), n128 - 1) * kPer128 + rank % kPer128;      // clamped: the list may come from the caller
+  const KeyPick pick = attn_key_pick(bid, n128, kPer128, p.Hkv);
+  if (pick.rank < 0) return;
+  const int hkv = pick.head;
+  const int tile = min(max(p.order_k[pick.rank], 0), n128 - 1) * kPer128 + pick.piece;      // clamped: the list may come from the caller
   if (tile >= ntile) return;
   const int k0 = tile * kKeys, klast = min(k0 + kKeys, p.T) - 1;
   const int q_begin = max(__builtin_amdgcn_readfirstlane(p.causal ? k0 : p.seg_start[k0]), 0);      // inside [0, T]

@@ -7,9 +7,8 @@ namespace fgrpo {
 
 template <int HD, int KB>
 static int launch(const AttnParams& p, hipStream_t st) {
-  const long long ranks = (long long)((p.T + 127) / 128) * (4 / KB);          // every 128-key tile of the launch order, in pieces of 32 KB keys
   AttnParams a = p;
-  a.blocks_k = (int)(ranks * p.Hkv);
+  a.blocks_k = (int)attn_key_blocks((p.T + 127) / 128, 4 / KB, p.Hkv);      // every 128-key tile, in pieces of 32 KB keys
   if (p.parts_k > 1) {
     const int rc = raise_lds<varlen_attn_dkv3_kernel<HD, KB, true>>(kDkv3Lds<HD, KB>);
     if (rc) return rc;

@@ -58,6 +58,14 @@ def check(dev, name, T, cu, Hq, Hkv, causal, seed=0, softmax_scale=None, backwar
         assert rel <= GRAD_REL, f"{name}: {nm} max error {rel} of the largest entry"
 
 
+@pytest.mark.parametrize("T,cu,Hq,Hkv,D", [
+    (100, [0, 100], 9, 9, 64), (260, [0, 130, 260], 5, 5, 128), (1000, [0, 400, 1000], 9, 3, 64),
+    (1025, [0, 1, 700, 1025], 7, 7, 128), (1100, [0, 1100], 6, 3, 128), (900, [0, 129, 900], 16, 16, 64)])
+def test_key_tiles_reach_every_head_once(dev, T, cu, Hq, Hkv, D):
+    """Numbers of (key tile, K/V head) units that do not go round the eight XCDs: fewer than eight, one too many, one short."""
+    check(dev, "key tiles", T, cu, Hq, Hkv, True, seed=T, D=D)
+
+
 @pytest.mark.parametrize("stride,Hq,D", [(69273656, 2, 64), (69273664, 2, 64), (69273656, 3, 128), (69273664, 3, 128)])
 def test_forward_of_query_rows_far_apart(dev, stride, Hq, D):
     """Either side of the last token stride whose 32 rows 32-bit offsets reach, where the kernel changes (69273656):
