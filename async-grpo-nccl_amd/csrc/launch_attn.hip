@@ -14,8 +14,10 @@ int launch_attn_merge_bwd(int D, const AttnParams& p, int rb, hipStream_t st);
 }
 
 namespace {
-// The hand-scheduled query-side kernels address a wavefront's 32 query rows with 32-bit byte offsets.
+// The hand-scheduled query-side kernels address a wavefront's 32 query rows with 32-bit byte offsets; rows farther apart
+// take the register-staged ones.
 bool wave_rows_in_reach(long long q_st, int Hq, int D) { return 31 * q_st * 2 + D * 2 < (1LL << 32) && 62LL * Hq * D + D * 2 < (1LL << 32); }
+int query_side_form(const Tuning& tn, long long q_st, int Hq, int D) { return wave_rows_in_reach(q_st, Hq, D) ? tn.attn_qside : 1; }
 
 // Query heads per work-group of the query-side kernels (tile = 128 / heads tokens).  Short segments gain from short
 // tiles (less masked work on the diagonal and at segment boundaries) as long as the heads of a group fill the
@@ -29,36 +31,36 @@ int attn_heads_per_group(const Tuning& tn, int G, int T, int n_seq) {
 }
 
 template <template <int, int> class Launcher>
-int launch_query_side(const Tuning& tn, int D, int hb, AttnParams& p, int T, int Hq, int Hkv, int32_t* bounds_ws, hipStream_t st) {
+int launch_query_side(int form, int D, int hb, AttnParams& p, int T, int Hq, int Hkv, int32_t* bounds_ws, hipStream_t st) {
   const int rb = 128 / hb, G = Hq / Hkv;
   p.order_q = bounds_ws + attn_order_offset(T, hb == 1 ? 1 : hb == 2 ? 2 : 3);
   const long long units = (long long)((T + rb - 1) / rb) * Hkv;            // (tile, K/V head)
   p.blocks_q = (int)(((units + 7) / 8 * 8) * ((G + hb - 1) / hb));
   const dim3 grid((unsigned)p.blocks_q * (p.parts_q > 1 ? p.parts_q : 1));
   if (D == 128) {
-    if (hb == 1) Launcher<128, 1>::run(tn, grid, st, p);
-    else if (hb == 2) Launcher<128, 2>::run(tn, grid, st, p);
-    else Launcher<128, 4>::run(tn, grid, st, p);
+    if (hb == 1) Launcher<128, 1>::run(form, grid, st, p);
+    else if (hb == 2) Launcher<128, 2>::run(form, grid, st, p);
+    else Launcher<128, 4>::run(form, grid, st, p);
   } else {
-    if (hb == 1) Launcher<64, 1>::run(tn, grid, st, p);
-    else if (hb == 2) Launcher<64, 2>::run(tn, grid, st, p);
-    else Launcher<64, 4>::run(tn, grid, st, p);
+    if (hb == 1) Launcher<64, 1>::run(form, grid, st, p);
+    else if (hb == 2) Launcher<64, 2>::run(form, grid, st, p);
+    else Launcher<64, 4>::run(form, grid, st, p);
   }
   HIP_TRY(hipGetLastError());
   return 0;
 }
 template <int HD, int HB>
 struct FwdLauncher {
-  static void run(const Tuning& tn, dim3 grid, hipStream_t st, const AttnParams& p) {
-    if (tn.attn_qside == 1) hipLaunchKernelGGL((varlen_attn_fwd_kernel<HD, HB>), grid, dim3(256), 0, st, p);
+  static void run(int form, dim3 grid, hipStream_t st, const AttnParams& p) {
+    if (form == 1) hipLaunchKernelGGL((varlen_attn_fwd_kernel<HD, HB>), grid, dim3(256), 0, st, p);
     else if (p.parts_q > 1) hipLaunchKernelGGL((varlen_attn_fwd2_kernel<HD, HB, true>), grid, dim3(256), 0, st, p);
     else hipLaunchKernelGGL((varlen_attn_fwd2_kernel<HD, HB>), grid, dim3(256), 0, st, p);
   }
 };
 template <int HD, int HB>
 struct DqLauncher {
-  static void run(const Tuning& tn, dim3 grid, hipStream_t st, const AttnParams& p) {
-    if (tn.attn_qside == 1 || tn.attn_qside == 3) hipLaunchKernelGGL((varlen_attn_dq_kernel<HD, HB>), grid, dim3(256), 0, st, p);
+  static void run(int form, dim3 grid, hipStream_t st, const AttnParams& p) {
+    if (form == 1 || form == 3) hipLaunchKernelGGL((varlen_attn_dq_kernel<HD, HB>), grid, dim3(256), 0, st, p);
     else if (p.parts_q > 1) hipLaunchKernelGGL((varlen_attn_dq2_kernel<HD, HB, true>), grid, dim3(256), 0, st, p);
     else hipLaunchKernelGGL((varlen_attn_dq2_kernel<HD, HB>), grid, dim3(256), 0, st, p);
   }
@@ -101,8 +103,8 @@ SplitPlan plan_split(long long wgs, int per_cu, double chain, bool causal, doubl
   }
   return best;
 }
-SplitPlan plan_query_split(const Tuning& tn, int T, int n_seq, int Hq, int Hkv, int D, int causal, bool forward) {
-  if (tn.attn_qside == 1 || (!forward && tn.attn_qside == 3)) return SplitPlan();
+SplitPlan plan_query_split(const Tuning& tn, int form, int T, int n_seq, int Hq, int Hkv, int D, int causal, bool forward) {
+  if (form == 1 || (!forward && form == 3)) return SplitPlan();
   const int hb = attn_heads_per_group(tn, Hq / Hkv, T, n_seq), rb = 128 / hb, G = Hq / Hkv;
   const long long wgs = (long long)((T + rb - 1) / rb) * Hkv * ((G + hb - 1) / hb);
   return plan_split(wgs, 2, (double)T / n_seq / kAttnBK, causal, D == 128 ? 1.6 : forward ? 1.15 : 1.3,
@@ -173,7 +175,7 @@ int fgrpo_varlen_attn_bounds(const int32_t* cu, int n_seq, int T, int causal, in
 size_t fgrpo_varlen_attn_workspace(int T, int n_seq, int Hq, int Hkv, int D, int causal, int backward) {
   if (T <= 0 || n_seq <= 0 || Hq <= 0 || Hkv <= 0 || Hq % Hkv != 0 || (D != 128 && D != 64)) return 0;
   const Tuning tn = g_tune;
-  const size_t q = query_split_bytes(plan_query_split(tn, T, n_seq, Hq, Hkv, D, causal, !backward), T, Hq, D, !backward);
+  const size_t q = query_split_bytes(plan_query_split(tn, tn.attn_qside, T, n_seq, Hq, Hkv, D, causal, !backward), T, Hq, D, !backward);
   return backward ? q + key_split_bytes(plan_key_split(tn, T, n_seq, Hq, Hkv, D, causal), T, Hkv, D) : q;
 }
 
@@ -202,10 +204,9 @@ int fgrpo_varlen_attn_fwd_ws(const void* q, const void* k, const void* v, long l
     rc = fgrpo_varlen_attn_bounds(cu, n_seq, T, causal, bounds_ws, stream);
     if (rc) return rc;
   }
-  Tuning tn = g_tune;         // one reading of the tuning state per call: the kernel launched is the one the split was planned for
-  if (!wave_rows_in_reach(q_st, Hq, D)) tn.attn_qside = 1;
-  const int hb = attn_heads_per_group(tn, Hq / Hkv, T, n_seq);
-  SplitPlan sp = plan_query_split(tn, T, n_seq, Hq, Hkv, D, causal, true);
+  const Tuning tn = g_tune;   // one reading of the tuning state per call: the kernel launched is the one the split was planned for
+  const int form = query_side_form(tn, q_st, Hq, D), hb = attn_heads_per_group(tn, Hq / Hkv, T, n_seq);
+  SplitPlan sp = plan_query_split(tn, form, T, n_seq, Hq, Hkv, D, causal, true);
   const size_t need = query_split_bytes(sp, T, Hq, D, true);
   if (!ws || need == 0) sp = SplitPlan();
   else if (ws_bytes < need) return fail(FGRPO_ERR_WORKSPACE, "varlen_attn_fwd: workspace %zu < %zu", ws_bytes, need);
@@ -213,7 +214,7 @@ int fgrpo_varlen_attn_fwd_ws(const void* q, const void* k, const void* v, long l
   p.parts_q = sp.parts, p.per_q = sp.per;
   p.part_q = (float*)ws;
   p.part_ml = (float2*)((char*)ws + align256((size_t)sp.parts * T * Hq * D * 4));
-  rc = launch_query_side<FwdLauncher>(tn, D, hb, p, T, Hq, Hkv, bounds_ws, st);
+  rc = launch_query_side<FwdLauncher>(form, D, hb, p, T, Hq, Hkv, bounds_ws, st);
   if (rc || sp.parts <= 1) return rc;
   const unsigned blocks = (unsigned)(((long long)T * Hq * (D / 8) + 255) / 256);
   if (D == 128) hipLaunchKernelGGL(attn_merge_fwd_kernel<128>, dim3(blocks), dim3(256), 0, st, p, 128 / hb);
@@ -254,10 +255,9 @@ int fgrpo_varlen_attn_bwd_ws(const void* dout, const void* q, const void* k, con
     rc = fgrpo_varlen_attn_bounds(cu, n_seq, T, causal, bounds_ws, stream);
     if (rc) return rc;
   }
-  Tuning tn = g_tune;         // one reading of the tuning state per call: the kernel launched is the one the split was planned for
-  if (!wave_rows_in_reach(q_st, Hq, D)) tn.attn_qside = 1;
-  const int hb = attn_heads_per_group(tn, Hq / Hkv, T, n_seq);
-  SplitPlan sq = plan_query_split(tn, T, n_seq, Hq, Hkv, D, causal, false), sk = plan_key_split(tn, T, n_seq, Hq, Hkv, D, causal);
+  const Tuning tn = g_tune;   // one reading of the tuning state per call: the kernel launched is the one the split was planned for
+  const int form = query_side_form(tn, q_st, Hq, D), hb = attn_heads_per_group(tn, Hq / Hkv, T, n_seq);
+  SplitPlan sq = plan_query_split(tn, form, T, n_seq, Hq, Hkv, D, causal, false), sk = plan_key_split(tn, T, n_seq, Hq, Hkv, D, causal);
   const size_t need_q = query_split_bytes(sq, T, Hq, D, false), need = need_q + key_split_bytes(sk, T, Hkv, D);
   if (!ws || need == 0) sq = sk = SplitPlan();
   else if (ws_bytes < need) return fail(FGRPO_ERR_WORKSPACE, "varlen_attn_bwd: workspace %zu < %zu", ws_bytes, need);
@@ -268,7 +268,7 @@ int fgrpo_varlen_attn_bwd_ws(const void* dout, const void* q, const void* k, con
   p.parts_q = sq.parts, p.per_q = sq.per, p.parts_k = sk.parts, p.per_k = sk.per;
   p.part_q = (float*)ws;
   p.part_k = (float*)((char*)ws + need_q);
-  rc = launch_query_side<DqLauncher>(tn, D, hb, p, T, Hq, Hkv, bounds_ws, st);
+  rc = launch_query_side<DqLauncher>(form, D, hb, p, T, Hq, Hkv, bounds_ws, st);
   if (rc) return rc;
   if (dkv3) {
     rc = launch_attn_dkv3(D, p, st);
