@@ -120,7 +120,7 @@ class LogProbHarness:
         self.actor_module_fsdp.eval()
         lens = [len(s["sample_ids"]) for s in samples]
         total = sum(lens)
-        host = torch.empty((3, total), dtype=torch.long).pin_memory() if total else torch.empty((3, 0), dtype=torch.long)
+        host = torch.empty((3, total), dtype=torch.long, pin_memory=total > 0)
         view = host.numpy()
         _fill(view[0], samples, "sample_ids", lens)
         _fill(view[2], samples, "labels", lens, default=-100)
@@ -135,7 +135,7 @@ class LogProbHarness:
         if total >= ops.COMPACT_MIN_TOKENS and _takes_row_list(self.actor_module_fsdp):
             scored = np.flatnonzero(view[2, 1:] != -100)
             if 0 < scored.size < ops.COMPACT_MAX_VALID_FRACTION * total:
-                rows = torch.empty(scored.size, dtype=torch.long).pin_memory()
+                rows = torch.empty(scored.size, dtype=torch.long, pin_memory=True)
                 rows.numpy()[:] = scored
                 extra["compact_masked_tokens"] = rows.to(self.device, non_blocking=True)
         dev = host.to(self.device, non_blocking=True)
@@ -143,7 +143,7 @@ class LogProbHarness:
         # one device->host copy for the whole batch into one pinned buffer
         ent = getattr(out, "entropy", None)
         rows = 2 if ent is not None else 1
-        buf = torch.empty((rows, total), dtype=torch.float32).pin_memory() if total else torch.empty((rows, 0), dtype=torch.float32)
+        buf = torch.empty((rows, total), dtype=torch.float32, pin_memory=total > 0)
         stacked = out.loss.detach().float().reshape(1, -1) if ent is None else \
             torch.stack((out.loss.detach().float().reshape(-1), ent.detach().float().reshape(-1)))
         buf.copy_(stacked, non_blocking=True)

@@ -231,3 +231,41 @@ def test_what_a_forward_takes_is_read_as_its_signature_says():
         want = any(p.kind is p.VAR_KEYWORD or (p.name == "rows" and p.kind is not p.POSITIONAL_ONLY) for p in params)
         assert _takes_keyword(f, "rows") == want
     assert not _takes_keyword(None, "rows") and not _takes_keyword(torch.jit.script(torch.nn.Linear(2, 2)).forward, "rows")
+
+
+class _Int(int):
+    pass
+
+
+@pytest.mark.parametrize("dtype", [np.int64, np.float32])
+@pytest.mark.parametrize("items", [
+    [], [7], list(range(-3, 900)), (1, 2, 3), [2 ** 63 - 1, -2 ** 63], [2 ** 63], [True, 2], [_Int(5), 6], [np.int64(9), 1],
+    [1.0, 2.5, -0.0], [0.1] * 700, [float("nan"), float("inf"), -float("inf")], [3.5e38], [1e-45, 1e-50], [np.float32(0.5), 1.0],
+    [1, 2.0], [None], ["4"], [1, None]])
+def test_packed_lists_are_what_numpy_makes_of_them(dtype, items):
+    """Every form of entry, those that are read natively and those that are not: the same values, or the same error."""
+    from sample_processing_utils import _fill
+
+    def outcome(write):
+        dst = np.full(len(items) + 2, 77, dtype=dtype)
+        try:
+            write(dst[1:-1])
+        except (TypeError, ValueError, OverflowError) as e:
+            return type(e)
+        assert dst[0] == 77 and dst[-1] == 77
+        return dst.tobytes()
+
+    def by_numpy(piece):
+        piece[:] = np.fromiter(items, dtype=dtype, count=len(items))
+    with np.errstate(all="ignore"):
+        assert outcome(lambda piece: _fill(piece, [{"x": items}], "x", [len(items)])) == outcome(by_numpy)
+
+
+def test_packed_lists_of_several_samples_follow_each_other():
+    from sample_processing_utils import _fill
+    dst = np.zeros(9, dtype=np.int64)
+    _fill(dst, [{"x": [1, 2]}, {}, {"x": (np.int32(3),)}, {"x": torch.tensor([4, 5])}, {"x": []}, {"x": (6, 7)}], "x",
+          [2, 2, 1, 2, 0, 2], default=-100)
+    assert dst.tolist() == [1, 2, -100, -100, 3, 4, 5, 6, 7]
+    with pytest.raises(ValueError):
+        _fill(dst, [{"x": [1, 2]}], "x", [3])
