@@ -403,15 +403,32 @@ size_t small_split_elems(const Tuning& tn, int M, int N, int K, int nseg) {
   return (size_t)small_split(M, N, K, nseg, (size_t)1 << 40, &kchunk) * M * round_up(N, 4);
 }
 
-// part: room for part_elems floats of pieces (null: none)
-int run_store_gemm(const Tuning& tn, StoreParams p, int variant, hipStream_t st, float* part = nullptr, size_t part_elems = 0) {
+// The products of one panel that are contracted in pieces, collected for one launch and one sum.
+struct SmallSplits {
+  SmallSplitPair pair;
+  SmallSumPair sums;
+  int n = 0, blocks = 0, sum_blocks = 0;
+};
+int launch_small_splits(const SmallSplits& q, hipStream_t st) {
+  const int rc = launch_small_split(q.pair, q.blocks, st);
+  if (rc) return rc;
+  hipLaunchKernelGGL(small_split_sum_kernel, dim3((unsigned)q.sum_blocks), dim3(256), 0, st, q.sums);
+  HIP_TRY(hipGetLastError());
+  return 0;
+}
+
+// part: room for part_elems floats of pieces (null: none).  A product that is contracted in pieces is added to `splits`,
+// whose launch is the caller's.
+int run_store_gemm(const Tuning& tn, StoreParams p, int variant, hipStream_t st, SmallSplits* splits = nullptr,
+                   float* part = nullptr, size_t part_elems = 0) {
   variant = pick_variant(tn, variant, p.g.M, p.g.N);
-  if (variant == 4 && part && p.g.a_blk == 0 && !p.row_scale && !p.alpha_dev) {
+  if (variant == 4 && splits && part && p.g.a_blk == 0 && !p.row_scale && !p.alpha_dev) {
     int kchunk = 0;
     const int ks = small_split(p.g.M, p.g.N, p.g.seg[0].K, p.g.nseg, part_elems, &kchunk);
     for (int s = 1; s < p.g.nseg; ++s)
       if (p.g.seg[s].K != p.g.seg[0].K) return fail(FGRPO_ERR_BAD_ARG, "gemm: segments of different length");
-    if (ks > 1) {
+    const long long sum_blocks = ((long long)p.g.M * p.g.N + 255) / 256;
+    if (ks > 1 && splits->n < 2 && splits->sum_blocks + sum_blocks < (1LL << 31)) {
       int rc = check_operands(p.g, kCfg[4].bk);
       if (rc) return rc;
       StoreParams q = p;
@@ -423,11 +440,18 @@ int run_store_gemm(const Tuning& tn, StoreParams p, int variant, hipStream_t st,
       q.tiles_n = (p.g.N + kCfg[4].bn - 1) / kCfg[4].bn;
       q.wide_stores = 1;
       q.nblocks = q.tiles_m * q.tiles_n * ks;
-      rc = launch_store_small_split(q, st);
-      if (rc) return rc;
-      hipLaunchKernelGGL(small_split_sum_kernel, dim3((unsigned)(((long long)p.g.M * p.g.N + 255) / 256)), dim3(256), 0, st, part, ks,
-                         q.part_slice, q.ldc, p.g.M, p.g.N, p.ldc, p.c_in, p.c_out_f32, p.c_out_bf16);
-      HIP_TRY(hipGetLastError());
+      const SmallSumJob sum{part, ks, q.part_slice, q.ldc, p.g.M, p.g.N, p.ldc, p.c_in, p.c_out_f32, p.c_out_bf16};
+      if (splits->n == 0) {
+        splits->pair.p[0] = splits->pair.p[1] = q;
+        splits->sums.job[0] = splits->sums.job[1] = sum;
+        splits->pair.first = q.nblocks;
+        splits->sums.first = (int)sum_blocks;
+      }
+      splits->pair.p[splits->n] = q;
+      splits->sums.job[splits->n] = sum;
+      ++splits->n;
+      splits->blocks += q.nblocks;
+      splits->sum_blocks += (int)sum_blocks;
       return 0;
     }
   }
@@ -458,8 +482,8 @@ struct BwdPlan {
   bf16_t *tv_hi, *tv_lo, *vt_hi, *vt_lo;      // dS panels
   float* bias32;
   float* dh_acc;                              // [T x H] fp32 when more than one panel
-  float* part;                                // pieces of a split contraction (small problems), part_elems of them
-  size_t part_elems;
+  float *part_dh, *part_dw;                   // pieces of the split contractions (small problems)
+  size_t part_dh_elems, part_dw_elems;
   size_t bytes;
 };
 
@@ -557,10 +581,10 @@ void plan_bwd(const Tuning& tn, BwdPlan& pl, void* ws, int T, int H, int V, int 
   pl.bias32 = has_bias ? cv.take<float>((size_t)V) : nullptr;
   pl.dh_acc = (want_dh && pl.npanels > 1 && !pl.f32) ? cv.take<float>((size_t)T * H) : nullptr;
   const int rows = V < pl.panel ? V : pl.panel, nseg = pl.f32 ? 3 : 1;
-  const size_t e_dh = want_dh && !pl.kmajor_dh ? small_split_elems(tn, T, H, (int)round_up(rows, pl.bm), nseg) : 0;
-  const size_t e_dw = want_dw && !pl.kmajor ? small_split_elems(tn, rows, H, pl.tiles_t * pl.bn, nseg) : 0;
-  pl.part_elems = e_dh > e_dw ? e_dh : e_dw;
-  pl.part = pl.part_elems ? cv.take<float>(pl.part_elems) : nullptr;
+  pl.part_dh_elems = want_dh && !pl.kmajor_dh ? small_split_elems(tn, T, H, (int)round_up(rows, pl.bm), nseg) : 0;
+  pl.part_dw_elems = want_dw && !pl.kmajor ? small_split_elems(tn, rows, H, pl.tiles_t * pl.bn, nseg) : 0;
+  pl.part_dh = pl.part_dh_elems ? cv.take<float>(pl.part_dh_elems) : nullptr;
+  pl.part_dw = pl.part_dw_elems ? cv.take<float>(pl.part_dw_elems) : nullptr;
   pl.bytes = cv.total();
 }
 
@@ -860,6 +884,7 @@ int fgrpo_lmhead_bwd(const void* hidden, const void* weight, const void* bias, c
                 : tn.fwd_group_t > 0 ? tn.fwd_group_t : 1;
     const int kv = d.tiles_v * pl.bm;        // written panel width
     const int kt = pl.tiles_t * pl.bn;       // written token extent
+    SmallSplits splits;
     {
       PhaseScope ph(kPhaseDlogits, st);
       rc = launch_ds_variant(pl.variant, f32 != 0, d, st);
@@ -905,7 +930,7 @@ int fgrpo_lmhead_bwd(const void* hidden, const void* weight, const void* bias, c
       }
       {
         PhaseScope ph(kPhaseDh, st);
-        rc = pl.kmajor_dh ? run_store_gemm_kmajor(tn, s, false, true, st) : run_store_gemm(tn, s, tn.gemm_variant, st, pl.part, pl.part_elems);
+        rc = pl.kmajor_dh ? run_store_gemm_kmajor(tn, s, false, true, st) : run_store_gemm(tn, s, tn.gemm_variant, st, &splits, pl.part_dh, pl.part_dh_elems);
       }
       if (rc) return rc;
     }
@@ -940,8 +965,13 @@ int fgrpo_lmhead_bwd(const void* hidden, const void* weight, const void* bias, c
         s.c_out_bf16 = (bf16_t*)dW_out + (size_t)v0 * H;
       {
         PhaseScope ph(kPhaseDw, st);
-        rc = pl.kmajor ? run_store_gemm_kmajor(tn, s, true, true, st) : run_store_gemm(tn, s, tn.gemm_variant, st, pl.part, pl.part_elems);
+        rc = pl.kmajor ? run_store_gemm_kmajor(tn, s, true, true, st) : run_store_gemm(tn, s, tn.gemm_variant, st, &splits, pl.part_dw, pl.part_dw_elems);
       }
+      if (rc) return rc;
+    }
+    if (splits.n > 0) {
+      PhaseScope ph(want_dw ? kPhaseDw : kPhaseDh, st);
+      rc = launch_small_splits(splits, st);
       if (rc) return rc;
     }
     if (dbias_out) {
@@ -1374,11 +1404,7 @@ int fgrpo_loss_fwd(const float* lp, const float* old_lp, const float* ref_lp, co
   p.loss = loss_out;
   p.scal = scal_out;
   if (agg_mode == FGRPO_AGG_SAMPLE_MEAN) {
-    // tokens outside every segment keep weight 0
-    hipLaunchKernelGGL(fill_f32_kernel, dim3((T + 255) / 256), dim3(256), 0, st, tokw, 0.f, T);
-    HIP_TRY(hipGetLastError());
-    hipLaunchKernelGGL(segment_valid_weight_kernel, dim3((nseq + 3) / 4), dim3(256), 0, st, p.labels, cu, nseq, T, segc,
-                       tokw);
+    launch_segment_weights(p.labels, cu, nseq, T, segc, tokw, st);
     HIP_TRY(hipGetLastError());
     p.tokw = tokw;
     p.seg_cnt = segc;
@@ -1401,11 +1427,7 @@ int fgrpo_loss_prepare(const int64_t* labels, const int32_t* cu, int nseq, int T
   if (by_sample && (!cu || nseq <= 0 || !tokw_out || !seg_cnt_out))
     return fail(FGRPO_ERR_BAD_ARG, "loss_prepare: sample_mean needs cu_seqlens, tokw_out and seg_cnt_out");
   if (by_sample) {
-    // tokens outside every segment keep weight 0
-    hipLaunchKernelGGL(fill_f32_kernel, dim3((T + 255) / 256), dim3(256), 0, st, tokw_out, 0.f, T);
-    HIP_TRY(hipGetLastError());
-    hipLaunchKernelGGL(segment_valid_weight_kernel, dim3((nseq + 3) / 4), dim3(256), 0, st, (const long long*)labels, cu,
-                       nseq, T, seg_cnt_out, tokw_out);
+    launch_segment_weights((const long long*)labels, cu, nseq, T, seg_cnt_out, tokw_out, st);
     HIP_TRY(hipGetLastError());
   }
   hipLaunchKernelGGL(grpo_loss_prepare_kernel, dim3(1), dim3(1024), 0, st, (const long long*)labels, T,

@@ -134,7 +134,7 @@ int launch_store_variant(int variant, const StoreParams& p, hipStream_t st);
 // 256x256x64 tile with one or both operands contraction-major
 int launch_store_kmajor(bool akm, bool bkm, const StoreParams& p, hipStream_t st);
 int launch_store_splitk(const StoreParams& p, hipStream_t st);
-// 128x128x64 tile, both operands K-contiguous, contraction in p.ksplit pieces of p.kchunk
-int launch_store_small_split(const StoreParams& p, hipStream_t st);
+// 128x128x64 tile, operands K-contiguous, one or two products with their contractions in pieces
+int launch_small_split(const SmallSplitPair& p, int nblocks, hipStream_t st);
 
 }  // namespace fgrpo

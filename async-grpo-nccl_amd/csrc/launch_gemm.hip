@@ -21,9 +21,8 @@ int launch_store_splitk(const StoreParams& p, hipStream_t st) {
   return launch_tile_kernel<gemm_store_kernel<Cfg8, false, true, true>, Cfg8>(p, p.nblocks, st);
 }
 
-int launch_store_small_split(const StoreParams& p, hipStream_t st) {
-  static_assert(kStoreViaLds<Cfg4>, "the pieces leave through the LDS patch");
-  return launch_tile_kernel<gemm_store_kernel<Cfg4, false, false, true>, Cfg4>(p, p.nblocks, st);
+int launch_small_split(const SmallSplitPair& p, int nblocks, hipStream_t st) {
+  return launch_tile_kernel<gemm_small_split_kernel<Cfg4>, Cfg4>(p, nblocks, st);
 }
 
 int launch_store_kmajor(bool akm, bool bkm, const StoreParams& p, hipStream_t st) {

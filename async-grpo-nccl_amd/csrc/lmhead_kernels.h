@@ -756,8 +756,7 @@ __device__ __forceinline__ void store_tile_lds(const StoreParams& p, f32x16_t (&
 }
 
 // SPLITK: the tiles of a device round that would otherwise run nearly empty are contracted in ksplit pieces by ksplit
-// work-groups each (a K-contiguous, column-blocked A and a contraction-major B: dHidden's last round; both operands
-// K-contiguous: the products of a small problem, piece ks taking the same K range of every segment).
+// work-groups each (a K-contiguous, column-blocked A and a contraction-major B: dHidden's last round).
 template <class C, bool AKM = false, bool BKM = false, bool SPLITK = false>
 __global__ __launch_bounds__(C::NT, C::OCC) void gemm_store_kernel(const StoreParams p0) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
@@ -765,20 +764,7 @@ __global__ __launch_bounds__(C::NT, C::OCC) void gemm_store_kernel(const StorePa
   int wm, wn;
   wave_coords<C, kMi16<C> && (AKM || BKM)>(wave, wm, wn);
 
-  if constexpr (SPLITK && !BKM) {
-    StoreParams p = p0;
-    const int tiles = p.tiles_m * p.tiles_n;
-    const int ks = (int)blockIdx.x / tiles, t = (int)blockIdx.x - ks * tiles;
-    const int row0 = t % p.tiles_m * C::BM, col0 = t / p.tiles_m * C::BN;
-    const int k0 = ks * p.kchunk;
-    const int klen = (p.g.seg[0].K - k0) < p.kchunk ? (p.g.seg[0].K - k0) : p.kchunk;      // > 0: the launcher sees to it
-    f32x16_t acc[C::TM][C::TN];
-    zero_acc<C>(acc);
-    gemm_mainloop<C>(p0.g, row0, col0, smem, acc, k0, klen);
-    p.c_out_f32 += (long long)ks * p.part_slice;
-    store_tile_lds<C, false, false>(p, acc, p.alpha, row0, col0, wm, wn, lane, wave, smem);
-    return;
-  } else if constexpr (SPLITK) {
+  if constexpr (SPLITK) {
     static_assert(!AKM && BKM && kMi16<C>, "split contraction: dHidden's layouts on the 16x16x32 tile");
     StoreParams p = p0;
     const int lid = xcd_contiguous_id(blockIdx.x, gridDim.x);
@@ -874,6 +860,38 @@ __global__ __launch_bounds__(C::NT, C::OCC) void gemm_store_kernel(const StorePa
     case 2: store_tile<C, false, true, MI16>(p, acc, alpha, row0, col0, wm, wn, lane); break;
     default: store_tile<C, true, true, MI16>(p, acc, alpha, row0, col0, wm, wn, lane); break;
   }
+}
+
+// The two gradient products of a small problem, contracted in pieces and in one launch: work-groups below `first` belong
+// to p[0], the others to p[1].  Piece ks of a product takes the same K range of every segment (all operands K-contiguous)
+// and leaves its fp32 tile in slice ks.  Neither product fills the device: side by side they take the time of the
+// longer one, and their sums one launch (fp32, 643 tokens x 1000 entries x 64: 9 + 9 us and 4 + 4 for the sums one behind
+// the other; the whole step with the launch of tail_kernels.h's segment weights 148.5 -> 138.4 us, one box, sides in turn).
+struct SmallSplitPair {
+  StoreParams p[2];
+  int first;
+};
+template <class C>
+__global__ __launch_bounds__(C::NT, C::OCC) void gemm_small_split_kernel(const SmallSplitPair pair) {
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  static_assert(kStoreViaLds<C>, "the pieces leave through the LDS patch");
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  int wm, wn;
+  wave_coords<C, false>(wave, wm, wn);
+  const bool second = (int)blockIdx.x >= pair.first;           // work-group uniform
+  const StoreParams& src = pair.p[second ? 1 : 0];
+  StoreParams p = src;
+  const int id = (int)blockIdx.x - (second ? pair.first : 0);
+  const int tiles = p.tiles_m * p.tiles_n;
+  const int ks = id / tiles, t = id - ks * tiles;
+  const int row0 = t % p.tiles_m * C::BM, col0 = t / p.tiles_m * C::BN;
+  const int k0 = ks * p.kchunk;
+  const int klen = (p.g.seg[0].K - k0) < p.kchunk ? (p.g.seg[0].K - k0) : p.kchunk;      // > 0: the launcher sees to it
+  f32x16_t acc[C::TM][C::TN];
+  zero_acc<C>(acc);
+  gemm_mainloop<C>(src.g, row0, col0, smem, acc, k0, klen);
+  p.c_out_f32 += (long long)ks * p.part_slice;
+  store_tile_lds<C, false, false>(p, acc, p.alpha, row0, col0, wm, wn, lane, wave, smem);
 }
 
 }  // namespace fgrpo

@@ -360,24 +360,38 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* part, i
 }
 
 // The same for the small products, whose slices have a row pitch of their own: out = c_in + sum of the slices, fp32 or bf16.
-__global__ __launch_bounds__(256) void small_split_sum_kernel(const float* part, int ksplit, long long slice, long long ld_part,
-                                                              int M, int N, long long ldc, const float* c_in,
-                                                              float* out_f32, bf16_t* out_bf16) {
-  const long long q = (long long)blockIdx.x * 256 + threadIdx.x;
-  if (q >= (long long)M * N) return;
-  const int m = (int)(q / N), n = (int)(q - (long long)m * N);
-  const float* src = part + (long long)m * ld_part + n;
-  const long long o = (long long)m * ldc + n;
-  float s = c_in ? c_in[o] : 0.f;
-  for (int k0 = 0; k0 < ksplit; k0 += 8) {                // eight loads in flight
+struct SmallSumJob {
+  const float* part;         // ksplit slices of [M][ld_part], `slice` elements apart
+  int ksplit;
+  long long slice, ld_part;
+  int M, N;
+  long long ldc;
+  const float* c_in;
+  float* out_f32;
+  bf16_t* out_bf16;
+};
+struct SmallSumPair {
+  SmallSumJob job[2];
+  int first;                 // work-groups of job[0]
+};
+__global__ __launch_bounds__(256) void small_split_sum_kernel(const SmallSumPair pair) {
+  const bool second = (int)blockIdx.x >= pair.first;
+  const SmallSumJob& p = pair.job[second ? 1 : 0];
+  const long long q = (long long)((int)blockIdx.x - (second ? pair.first : 0)) * 256 + threadIdx.x;
+  if (q >= (long long)p.M * p.N) return;
+  const int m = (int)(q / p.N), n = (int)(q - (long long)m * p.N);
+  const float* src = p.part + (long long)m * p.ld_part + n;
+  const long long o = (long long)m * p.ldc + n;
+  float s = p.c_in ? p.c_in[o] : 0.f;
+  for (int k0 = 0; k0 < p.ksplit; k0 += 8) {              // eight loads in flight
     float v[8];
 #pragma unroll
-    for (int k = 0; k < 8; ++k) v[k] = k0 + k < ksplit ? src[(long long)(k0 + k) * slice] : 0.f;
+    for (int k = 0; k < 8; ++k) v[k] = k0 + k < p.ksplit ? src[(long long)(k0 + k) * p.slice] : 0.f;
 #pragma unroll
     for (int k = 0; k < 8; ++k) s += v[k];
   }
-  if (out_f32) out_f32[o] = s;
-  else out_bf16[o] = f32_to_bf16_rn(s);
+  if (p.out_f32) p.out_f32[o] = s;
+  else p.out_bf16[o] = f32_to_bf16_rn(s);
 }
 
 // dbias from the kept numerators: out[v] = sum_t a_t * E'[t][v].  One block owns 64 columns; its four row groups

@@ -34,10 +34,6 @@ __device__ __forceinline__ void clamp_range(int& b, int& e, int n) {
   e = e < b ? b : (e > n ? n : e);
 }
 
-__global__ void fill_f32_kernel(float* dst, float v, int n) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) dst[i] = v;
-}
 __global__ void fill_i64_kernel(long long* dst, long long v, int n) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) dst[i] = v;
@@ -47,10 +43,36 @@ __global__ void fill_i64_kernel(long long* dst, long long v, int n) {
 // Segment (sample) statistics over cu_seqlens: one wavefront per segment.
 // ---------------------------------------------------------------------------
 // cnt[s] = number of valid (label != -100) tokens of segment s; tokw[t] = 1/cnt
-// of the token's segment (0 when the segment has no valid token).
-__global__ void segment_valid_weight_kernel(const long long* labels, const int* cu, int nseq, int T, int* cnt, float* tokw) {
-  const int s = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
+// of the token's segment (0 when the segment has no valid token, and for tokens outside every segment).
+// Work-groups past the segments' write the zeros: a token no range covers lies below every boundary, at or above all
+// of them, or - in a vector that runs backwards - between its last boundary and its first.  One launch instead of a
+// fill in front of the segments: a step of 643 tokens is bound by its launches (figures at gemm_small_split_kernel).
+constexpr int kSegmentsPerGroup = 4, kZeroTokensPerGroup = 4096;
+__global__ __launch_bounds__(64 * kSegmentsPerGroup) void segment_valid_weight_kernel(const long long* labels, const int* cu,
+                                                                                      int nseq, int T, int* cnt, float* tokw) {
+  const int seg_groups = (nseq + kSegmentsPerGroup - 1) / kSegmentsPerGroup;
+  const int s = blockIdx.x * kSegmentsPerGroup + (threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
+  if ((int)blockIdx.x >= seg_groups) {
+    int lo = T, hi = 0;
+    for (int i = lane; i <= nseq; i += 64) {
+      const int b = cu[i] < 0 ? 0 : (cu[i] > T ? T : cu[i]);
+      lo = b < lo ? b : lo;
+      hi = b > hi ? b : hi;
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+      const int l2 = __shfl_xor(lo, o), h2 = __shfl_xor(hi, o);
+      lo = l2 < lo ? l2 : lo;
+      hi = h2 > hi ? h2 : hi;
+    }
+    const int first = cu[0], last = cu[nseq];
+    const int t0 = ((int)blockIdx.x - seg_groups) * kZeroTokensPerGroup;
+    const int t1 = T - t0 < kZeroTokensPerGroup ? T : t0 + kZeroTokensPerGroup;
+    for (int t = t0 + (int)threadIdx.x; t < t1; t += 64 * kSegmentsPerGroup)
+      if (t < lo || t >= hi || (t >= last && t < first)) tokw[t] = 0.f;
+    return;
+  }
   if (s >= nseq) return;
   int b = cu[s], e = cu[s + 1];
   clamp_range(b, e, T);
@@ -63,6 +85,11 @@ __global__ void segment_valid_weight_kernel(const long long* labels, const int* 
 }
 
 // out[t] = values[s] for every token of segment s
+inline void launch_segment_weights(const long long* labels, const int* cu, int nseq, int T, int* cnt, float* tokw, hipStream_t st) {
+  const int groups = (nseq + kSegmentsPerGroup - 1) / kSegmentsPerGroup + (T + kZeroTokensPerGroup - 1) / kZeroTokensPerGroup;
+  hipLaunchKernelGGL(segment_valid_weight_kernel, dim3(groups), dim3(64 * kSegmentsPerGroup), 0, st, labels, cu, nseq, T, cnt, tokw);
+}
+
 __global__ void segment_broadcast_kernel(const void* values, int values_f64, const int* cu, int nseq, int T, float* out) {
   const int s = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;

@@ -146,6 +146,48 @@ def test_fp32_gradients_of_small_heads(dev, T, H, V):
         assert (a.cpu().double() - b).norm() <= 6 * 2 ** -16 * b.norm()
 
 
+@pytest.mark.parametrize("panel_elems", [0, 643 * 256])
+@pytest.mark.parametrize("T,H,V", [(643, 64, 1000), (129, 96, 8000), (2000, 256, 777)])
+def test_fp32_gradients_do_not_depend_on_which_are_wanted(dev, T, H, V, panel_elems):
+    """The two products share launches where both are contracted in pieces; their sums are the same alone, bit for bit,
+    and with the vocabulary in several panels."""
+    from fgrpo import ops
+    gen = torch.Generator().manual_seed(T + V)
+    h, w = torch.randn(T, H, generator=gen).to(dev), (torch.randn(V, H, generator=gen) * 0.05).to(dev)
+    y = torch.randint(0, V, (T,), generator=gen).to(dev)
+    g = torch.randn(T, generator=gen).to(dev)
+    lse = torch.logsumexp(h.double() @ w.double().t(), 1).float()
+    dh, dw, _ = ops.lmhead_bwd(h, w, None, y, lse, g, None, 1.0, True, True, False, panel_elems)
+    only_h, none, _ = ops.lmhead_bwd(h, w, None, y, lse, g, None, 1.0, True, False, False, panel_elems)
+    assert none is None and torch.equal(only_h, dh)
+    none, only_w, _ = ops.lmhead_bwd(h, w, None, y, lse, g, None, 1.0, False, True, False, panel_elems)
+    assert none is None and torch.equal(only_w, dw)
+
+
+@pytest.mark.parametrize("T,bounds", [(643, [0, 40, 41, 41, 643]), (9000, [5, 100, 8000]), (4097, [0, 4097]), (4096, [4095, 4096]),
+                                      (300, [0, 100, 300, 0]), (300, [200, 50]), (300, [-7, 20, 400]), (1, [0, 0])])
+def test_segment_weights_cover_every_token(dev, T, bounds):
+    """1 / (scored tokens of the sample), zero outside every sample: boundaries that start late, end early, repeat, leave
+    the batch or run backwards."""
+    from fgrpo import ops
+    gen = torch.Generator().manual_seed(T)
+    y = torch.randint(0, 9, (T,), generator=gen)
+    y[torch.rand(T, generator=gen) < 0.3] = -100
+    want = torch.zeros(T)
+    filled = 0
+    for b, e in zip(bounds[:-1], bounds[1:]):
+        b = min(max(b, 0), T)
+        e = min(max(e, b), T)
+        n = int((y[b:e] != -100).sum())
+        want[b:e] = 1.0 / n if n else 0.0
+        filled += n > 0
+    junk = torch.full((64, T), float("nan"), device=dev)      # what the next allocations may be cut from
+    del junk
+    tokw, pre = ops.loss_prepare(y.to(dev), torch.tensor(bounds, dtype=torch.int32), "sample_mean")
+    assert torch.equal(tokw.cpu(), want)
+    assert pre.tolist()[:3] == [max(filled, 1), int((y != -100).sum()), filled]
+
+
 @pytest.mark.parametrize("compact", [False, True])
 @pytest.mark.parametrize("which", ["old_lp", "adv", "ref_lp"])
 def test_per_token_inputs_are_inputs_of_the_node(dev, which, compact):
