@@ -654,10 +654,27 @@ int keep_prepass(const FwdParams& p, const void* hidden, const void* weight, con
   return 0;
 }
 
+// The objective's arrays from token t0 on (a whole number of kLossGroup tokens)
+LossParams loss_from(LossParams q, int t0) {
+  q.old_lp = q.old_lp ? q.old_lp + t0 : nullptr;
+  q.ref_lp = q.ref_lp ? q.ref_lp + t0 : nullptr;
+  q.adv += t0;
+  q.labels += t0;
+  q.tokw = q.tokw ? q.tokw + t0 : nullptr;
+  q.g += t0;
+  q.log_ratio = q.log_ratio ? q.log_ratio + t0 : nullptr;
+  q.clip1 = q.clip1 ? q.clip1 + t0 : nullptr;
+  q.unclipped = q.unclipped ? q.unclipped + t0 : nullptr;
+  q.clipped = q.clipped ? q.clipped + t0 : nullptr;
+  q.partial += 2 * (size_t)(t0 / kLossGroup);
+  return q;
+}
+
+// loss: the objective of these tokens, formed by the merge of the vocabulary splits (its normaliser is known: loss->pre)
 int logprob_fwd_impl(const void* hidden, const void* weight, const void* bias, const int64_t* labels, float inv_temp,
                       int T, int H, int V, int dtype, float* lp_out, float* ent_out, float* lse_out, void* ws,
                       size_t ws_bytes, void* stream, void* keep = nullptr, const Tuning* snapshot = nullptr,
-                      const KeepAux* aux_in = nullptr) {
+                      const KeepAux* aux_in = nullptr, const LossParams* loss = nullptr) {
   hipStream_t st = (hipStream_t)stream;
   if (!hidden || !weight || !labels || !lp_out) return fail(FGRPO_ERR_BAD_ARG, "logprob_fwd: null argument");
   if (T <= 0 || H <= 0 || V <= 0) return fail(FGRPO_ERR_BAD_ARG, "logprob_fwd: T=%d H=%d V=%d", T, H, V);
@@ -724,8 +741,13 @@ int logprob_fwd_impl(const void* hidden, const void* weight, const void* bias, c
     const int rc2 = keep ? launch_fwd_keep(q, st) : launch_fwd_variant(pl.variant, q, st);
     if (rc2) return rc2;
     CombineParams c{part, pl.xt + t0, (const long long*)labels + t0, count, V, nsplit, lp_out + t0,
-                    ent_out ? ent_out + t0 : nullptr, lse_out ? lse_out + t0 : nullptr};
-    launch_fwd_combine(c, st);
+                    ent_out ? ent_out + t0 : nullptr, lse_out ? lse_out + t0 : nullptr, LossParams()};
+    if (loss) {
+      c.loss = loss_from(*loss, t0);
+      launch_fwd_combine<true>(c, st);
+    } else {
+      launch_fwd_combine<false>(c, st);
+    }
     HIP_TRY(hipGetLastError());
     return 0;
   };
@@ -1140,8 +1162,9 @@ int kept_bwd_impl(const Tuning& tn, const void* hidden, const void* weight, cons
   {
     PhaseScope ph(kPhaseDlogits, st);
     KeepPrepParams k{ek, blk, aux.ref2, aux.xy, (const long long*)labels, lse, g, gout_dev, inv_temp,
-                     (const bf16_t*)hidden, T, H, V, pl.row_scale, flag};
-    hipLaunchKernelGGL(keep_backward_prep_kernel, dim3((T + 3) / 4), dim3(256), 0, st, k);
+                     (const bf16_t*)hidden, T, H, V, pl.row_scale, flag, want_dw ? pl.hidden_scaled : nullptr, kept_hs_ld(T), Tpad,
+                     skip_dead ? pl.k_runs : nullptr, skip_dead ? pl.m_tile_live : nullptr, (T + 63) / 64, Tpad / 64};
+    launch_keep_backward_prep(k, st);
     HIP_TRY(hipGetLastError());
     {
       // Out-of-range batches (the forward raised the buffer's flag): the decision is taken on the device.  This launch
@@ -1173,13 +1196,6 @@ int kept_bwd_impl(const Tuning& tn, const void* hidden, const void* weight, cons
       d.gate = flag;
       rc = launch_ds_variant(8, false, d, st);
       if (rc) return rc;
-    }
-    if (want_dw)
-      hipLaunchKernelGGL(keep_scaled_transpose_kernel, dim3(Tpad / 64, H / 64), dim3(256), 0, st, (const bf16_t*)hidden,
-                         (const float*)pl.row_scale, T, H, Tpad, kept_hs_ld(T), pl.hidden_scaled);
-    if (skip_dead) {
-      KeepLiveParams lv{pl.row_scale, T, (T + 63) / 64, Tpad / 64, pl.k_runs, pl.m_tile_live};
-      hipLaunchKernelGGL(keep_live_runs_kernel, dim3(1), dim3(1024), 0, st, lv);
     }
   }
   HIP_TRY(hipGetLastError());
@@ -1556,7 +1572,7 @@ void plan_chunked(const Tuning& tn, ChunkedPlan& pl, void* ws, int T, int H, int
   pl.bwd_ws = cv.take<char>(pl.bwd_bytes);
   pl.dw_acc = (want_dw && pl.nchunks > 1) ? cv.take<float>((size_t)V * H) : nullptr;
   pl.db_acc = (want_db && pl.nchunks > 1) ? cv.take<float>((size_t)V) : nullptr;
-  pl.partial = cv.take<double>(2 * (size_t)((T + kLossThreads - 1) / kLossThreads));
+  pl.partial = cv.take<double>(2 * (size_t)((T + kLossGroup - 1) / kLossGroup));
   pl.ref2 = cv.take<float>((size_t)T);
   pl.xy = cv.take<float>((size_t)T);
   pl.flags = cv.take<int>((size_t)pl.nchunks);
@@ -1625,6 +1641,18 @@ int fgrpo_grpo_step_chunked(const void* hidden, const void* weight, const void* 
   lp.pre = pre;
   lp.loss = loss_out;
   lp.scal = scal_out;
+  lp.T = T;
+  lp.old_lp = old_lp;
+  lp.ref_lp = ref_lp;
+  lp.adv = adv;
+  lp.labels = (const long long*)labels;
+  lp.tokw = tokw;
+  lp.g = g_out;
+  lp.log_ratio = log_ratio;
+  lp.clip1 = clip1;
+  lp.unclipped = unclipped;
+  lp.clipped = clipped;
+  lp.partial = pl.partial;
 
   {
     // references of the kept numerators for the tokens of every chunk, in one pass before the first chunk
@@ -1654,34 +1682,16 @@ int fgrpo_grpo_step_chunked(const void* hidden, const void* weight, const void* 
     const int t0 = first[ci], cnt = pl.sizes[ci];
     const char* h_c = (const char*)hidden + (size_t)t0 * H * esz;
     const KeepAux aux{pl.ref2 + t0, pl.xy + t0, pl.flags + ci, true};
+    // the objective on this chunk's tokens: the normaliser is known (pre), so g is final as it is written
+    const LossParams q = loss_from(lp, t0);
     int rc;
     {
       PhaseScope ph(kPhaseFwd, st);
       rc = logprob_fwd_impl(h_c, weight, bias, labels + t0, inv_temp, cnt, H, V, dtype, lp_out + t0,
                             ent_out ? ent_out + t0 : nullptr, lse_out + t0, pl.fwd_ws, pl.fwd_bytes, stream, pl.keep, &tn,
-                            &aux);
+                            &aux, &q);
     }
     if (rc) return rc;
-    {
-      // the objective on this chunk's tokens: the normaliser is known (pre), so g is final as it is written
-      PhaseScope ph(kPhaseOther, st);
-      LossParams q = lp;
-      q.lp = lp_out + t0;
-      q.old_lp = old_lp ? old_lp + t0 : nullptr;
-      q.ref_lp = ref_lp ? ref_lp + t0 : nullptr;
-      q.adv = adv + t0;
-      q.labels = (const long long*)labels + t0;
-      q.tokw = tokw ? tokw + t0 : nullptr;
-      q.T = cnt;
-      q.g = g_out + t0;
-      q.log_ratio = log_ratio ? log_ratio + t0 : nullptr;
-      q.clip1 = clip1 ? clip1 + t0 : nullptr;
-      q.unclipped = unclipped ? unclipped + t0 : nullptr;
-      q.clipped = clipped ? clipped + t0 : nullptr;
-      q.partial = pl.partial + 2 * (size_t)(t0 / kLossThreads);     // chunks start on whole blocks of the token kernel
-      hipLaunchKernelGGL(grpo_loss_tokens_kernel, dim3((cnt + kLossThreads - 1) / kLossThreads), dim3(kLossThreads), 0, st, q);
-      HIP_TRY(hipGetLastError());
-    }
     if (dH_out || dW_out || dbias_out) {
       const bool first = ci == 0, last = ci == pl.nchunks - 1;
       KeptBwdSums sums;
@@ -1701,25 +1711,40 @@ int fgrpo_grpo_step_chunked(const void* hidden, const void* weight, const void* 
   }
   {
     PhaseScope ph(kPhaseOther, st);
-    const int nblocks = (T + kLossThreads - 1) / kLossThreads;
-    lp.T = T;
-    lp.partial = pl.partial;
-    hipLaunchKernelGGL(grpo_loss_finalize_kernel, dim3(1), dim3(kLossThreads), 0, st, lp, nblocks);
+    hipLaunchKernelGGL(grpo_loss_finalize_kernel, dim3(1), dim3(kLossThreads), 0, st, lp, (T + kLossGroup - 1) / kLossGroup);
     HIP_TRY(hipGetLastError());
   }
   return 0;
 }
 
 int fgrpo_scale_inplace(void* x, long long n, int dtype, const float* scale_dev, void* stream) {
-  if (!x || !scale_dev || n < 0) return fail(FGRPO_ERR_BAD_ARG, "scale_inplace: bad argument");
+  if (!x) return fail(FGRPO_ERR_BAD_ARG, "scale_inplace: bad argument");
+  return fgrpo_scale_gradients(x, n, nullptr, 0, nullptr, 0, dtype, scale_dev, stream);
+}
+
+int fgrpo_scale_gradients(void* dh, long long n_dh, void* dw, long long n_dw, void* db, long long n_db, int dtype,
+                          const float* scale_dev, void* stream) {
+  ScaleParams p;
+  memset(&p, 0, sizeof(p));
+  void* const x[3] = {dh, dw, db};
+  const long long n[3] = {n_dh, n_dw, n_db};
+  if (!scale_dev) return fail(FGRPO_ERR_BAD_ARG, "scale_inplace: bad argument");
   if (dtype != FGRPO_BF16 && dtype != FGRPO_F32) return fail(FGRPO_ERR_BAD_ARG, "scale_inplace: dtype=%d", dtype);
-  if (!aligned16(x)) return fail(FGRPO_ERR_ALIGN, "scale_inplace: the array must be 16-byte aligned");
-  if (n == 0) return 0;
-  const long long nv = n / (dtype == FGRPO_F32 ? 4 : 8);
-  long long nb = (nv + 255) / 256;
-  nb = nb < 1 ? 1 : (nb > 4096 ? 4096 : nb);
-  hipLaunchKernelGGL(scale_inplace_kernel, dim3((unsigned)nb), dim3(256), 0, (hipStream_t)stream, x, n,
-                     dtype == FGRPO_F32, scale_dev);
+  int arrays = 0, blocks = 0;
+  for (int i = 0; i < 3; ++i) {
+    if (n[i] < 0 || (n[i] > 0 && !x[i])) return fail(FGRPO_ERR_BAD_ARG, "scale_inplace: bad argument");
+    if (x[i] && !aligned16(x[i])) return fail(FGRPO_ERR_ALIGN, "scale_inplace: the array must be 16-byte aligned");
+    if (!x[i] || n[i] == 0) continue;
+    const long long nb = (n[i] / (dtype == FGRPO_F32 ? 4 : 8) + 255) / 256;
+    p.x[arrays] = x[i], p.n[arrays] = n[i], p.first[arrays] = blocks;
+    blocks += (int)(nb < 1 ? 1 : (nb > 4096 ? 4096 : nb));
+    ++arrays;
+  }
+  if (arrays == 0) return 0;
+  for (int i = arrays; i < 4; ++i) p.first[i] = blocks;
+  p.is_f32 = dtype == FGRPO_F32;
+  p.scale = scale_dev;
+  hipLaunchKernelGGL(scale_inplace_kernel, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream, p);
   HIP_TRY(hipGetLastError());
   return 0;
 }

@@ -3,6 +3,7 @@
 // Included by exactly one translation unit (the kernels here are ordinary external functions).
 #pragma once
 #include "lmhead_kernels.h"
+#include "tail_kernels.h"
 
 namespace fgrpo {
 
@@ -16,9 +17,13 @@ struct CombineParams {
   float* lp;    // [T]
   float* ent;   // [T] or null
   float* lse;   // [T] or null
+  // LOSS kernels only: the objective of these tokens (its arrays start at the same token, its normaliser is known), formed
+  // where the log-probability is.  loss.partial takes {sum, scored tokens} of every kLossGroup tokens.
+  LossParams loss;
 };
+constexpr int kLossGroup = 16;
 
-template <int SUB>
+template <int SUB, bool LOSS>
 __global__ __launch_bounds__(256) void lmhead_fwd_combine_kernel(const CombineParams p) {
   constexpr int TOK = 256 / SUB;
   __shared__ float sm[SUB > 1 ? 3 * 256 : 1];
@@ -40,27 +45,45 @@ __global__ __launch_bounds__(256) void lmhead_fwd_combine_kernel(const CombinePa
     const int last = p.nsplit < SUB ? p.nsplit : SUB;
     for (int u = 1; u < last; ++u) lse_merge(m, s, sx, sm[u * TOK + tok], sm[256 + u * TOK + tok], sm[512 + u * TOK + tok]);
   }
-  if (n >= p.T) return;
-  const float lse = m + logf(s);
-  if (p.lse) p.lse[n] = lse;
-  const long long lab = p.labels[n];
-  const bool valid = (lab != -100);
-  float lp = 0.f, ent = 0.f;
-  if (valid) {
-    // a label outside [0, V) has no target logit: report NaN rather than a silent number
-    lp = (lab >= 0 && lab < p.V) ? (p.xt[n] - lse) : __uint_as_float(0x7fc00000u);
-    ent = lse - sx / s;
+  float term = 0.f;
+  bool scored = false;
+  if (n < p.T) {
+    const float lse = m + logf(s);
+    if (p.lse) p.lse[n] = lse;
+    const long long lab = p.labels[n];
+    float lp = 0.f, ent = 0.f;
+    if (lab != -100) {
+      // a label outside [0, V) has no target logit: report NaN rather than a silent number
+      lp = (lab >= 0 && lab < p.V) ? (p.xt[n] - lse) : __uint_as_float(0x7fc00000u);
+      ent = lse - sx / s;
+    }
+    p.lp[n] = lp;
+    if (p.ent) p.ent[n] = ent;
+    if constexpr (LOSS) term = grpo_token(p.loss, n, lp, scored);
   }
-  p.lp[n] = lp;
-  if (p.ent) p.ent[n] = ent;
+  if constexpr (LOSS) {                        // whole groups of sixteen lanes hold sixteen neighbouring tokens
+    double sum = (double)term, cnt = scored ? 1.0 : 0.0;
+#pragma unroll
+    for (int o = kLossGroup / 2; o > 0; o >>= 1) {
+      sum += __shfl_xor(sum, o);
+      cnt += __shfl_xor(cnt, o);
+    }
+    if (n < p.T && n % kLossGroup == 0) {
+      p.loss.partial[2 * (n / kLossGroup)] = sum;
+      p.loss.partial[2 * (n / kLossGroup) + 1] = cnt;
+    }
+  }
 }
 
 // Few splits mean many tokens: one thread each.  Small token counts are split up to 128 ways so that the forward
 // fills the device, and one thread then walks that many loads in sequence (777 tokens, 60 splits: 20.6 us; with 16
 // threads a token 5; 4 splits of 8192 tokens take 5 us either way).
+// The objective rides along where its normaliser is known beforehand: a launch less per token chunk (4.8 us each between
+// kernels that wait for one another).
+template <bool LOSS>
 inline void launch_fwd_combine(const CombineParams& c, hipStream_t st) {
-  if (c.nsplit >= 8) hipLaunchKernelGGL(lmhead_fwd_combine_kernel<16>, dim3((c.T + 15) / 16), dim3(256), 0, st, c);
-  else hipLaunchKernelGGL(lmhead_fwd_combine_kernel<1>, dim3((c.T + 255) / 256), dim3(256), 0, st, c);
+  if (c.nsplit >= 8) hipLaunchKernelGGL((lmhead_fwd_combine_kernel<16, LOSS>), dim3((c.T + 15) / 16), dim3(256), 0, st, c);
+  else hipLaunchKernelGGL((lmhead_fwd_combine_kernel<1, LOSS>), dim3((c.T + 255) / 256), dim3(256), 0, st, c);
 }
 
 // ---------------------------------------------------------------------------
@@ -277,62 +300,197 @@ struct KeepPrepParams {
   // factor as 1 for tokens with a gradient, 0 for the others - the gradient products that follow are the same
   // launches either way.
   const int* gate;
+  // B operand of the dW product, contraction-contiguous (null: not wanted): out[h][t] = a_t * hidden[t][h] for t < T, zero
+  // up to Tpad (the contraction runs over whole 64-token steps; the kept buffer's rows past T read as zero, and zero
+  // times a stale value must not be a NaN); rows are ld_scaled elements apart.  H % 64 == 0, Tpad % 64 == 0,
+  // ld_scaled >= Tpad, ld_scaled % 8 == 0.
+  bf16_t* hidden_scaled;
+  long long ld_scaled;
+  int Tpad;
+  // Which parts of the token axis carry a gradient at all (row factor a_t != 0; null: not wanted): zero-advantage samples
+  // and ignored labels form long stretches of dead rows, which the gradient GEMMs skip - the dHidden product by 256-row
+  // tile (m_tile_live), the dW product, whose contraction runs over the tokens, by K step of 64 rows (k_runs: the list
+  // of live runs gemm_mainloop_km walks).  If the rows alternate more often than the list can hold, it is written as
+  // one run over everything (the products are then merely not shortened).
+  int* k_runs;               // [2 + 2 * kRunCap]
+  int* m_tile_live;          // [ceil(T / 256)]
+  int n_chunks;              // ceil(T / 64), at most kLiveMaxChunks
+  int k_steps;               // K steps of the dW product (round_up(T, 256) / 64)
 };
+constexpr int kLiveMaxChunks = 32768;      // 2 M tokens: beyond that nothing is skipped (the lists say "all live")
 
-__global__ __launch_bounds__(256) void keep_backward_prep_kernel(const KeepPrepParams p) {
-  const int t = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-  if (t >= p.T) return;
+// a_t of a token
+__device__ __forceinline__ float keep_row_factor(const KeepPrepParams& p, int t, bool recompute) {
   const long long lab = p.labels[t];
-  const bool recompute = p.gate != nullptr && *p.gate != 0;
-  float a = 0.f;
-  if (lab >= 0 && lab < p.V) {
-    const float c = p.gtok[t] * (p.gout ? *p.gout : 1.f) * p.inv_temp;
-    const float d2 = p.ref2[t] - p.lse[t] * kLog2e;        // log2 s_t
-    a = recompute ? (c != 0.f ? 1.f : 0.f) : -c * fast_exp2(d2);
-    if (lane == 0 && !recompute) {
-      // p_y - 1 from the fp32 quantities: log p_y = x_y/temperature - lse
-      const float pm1 = expm1f(p.xy[t] - p.lse[t]);
-      p.e[(lab >> 8) * p.blk + (long long)t * 256 + (lab & 255)] = f32_to_bf16_rn(pm1 * fast_exp2(-d2));
-    }
-  }
-  if (lane == 0) p.row_scale[t] = a;
+  if (lab < 0 || lab >= p.V) return 0.f;
+  const float c = p.gtok[t] * (p.gout ? *p.gout : 1.f) * p.inv_temp;
+  if (recompute) return c != 0.f ? 1.f : 0.f;
+  return -c * fast_exp2(p.ref2[t] - p.lse[t] * kLog2e);        // c * (-s_t)
 }
 
-// B operand of the dW product, contraction-contiguous: out[h][t] = a_t * hidden[t][h] for t < T, zero up to Tpad
-// (the contraction runs over whole 64-token steps; the kept buffer's rows past T read as zero, and zero times a
-// stale value must not be a NaN); rows of `out` are ld elements apart.  64 x 64 tiles through LDS; H % 64 == 0,
-// Tpad % 64 == 0, ld >= Tpad, ld % 8 == 0.
-__global__ __launch_bounds__(256) void keep_scaled_transpose_kernel(const bf16_t* hidden, const float* row_scale, int T,
-                                                                    int H, int Tpad, long long ld, bf16_t* out) {
-  __shared__ uint16_t tile[64][66];
-  const int t0 = blockIdx.x * 64, h0 = blockIdx.y * 64;
-  const int r = threadIdx.x >> 3, cidx = threadIdx.x & 7;
+// The live lists: thread i owns a contiguous piece of the 64-row chunks.  `sm`: kLiveLds bytes.
+constexpr int kLiveLds = kLiveMaxChunks + 2 * 1025 * 4 + 2 * 16 * 4;
+__device__ __forceinline__ void keep_live_runs(const KeepPrepParams& p, bool recompute, char* sm) {
+  unsigned char* live = (unsigned char*)sm;
+  int* starts_before = (int*)(sm + kLiveMaxChunks);
+  int* live_before = starts_before + 1025;
+  int *wave_s = live_before + 1025, *wave_l = wave_s + 16;
+  const int tid = threadIdx.x;
+  // chunk flags: one wavefront per chunk, 64 rows each
+  // (four chunks per wavefront and round, so that four loads are in flight at a time)
+  for (int c4 = (tid >> 6) * 4; c4 < p.n_chunks; c4 += 64) {
+    float v[4];
 #pragma unroll
-  for (int half = 0; half < 2; ++half) {
-    const int tl = r + 32 * half, t = t0 + tl;
-    u32x4_t v = {0u, 0u, 0u, 0u};
-    float a = 0.f;
-    if (t < T) {
-      v = *(const u32x4_t*)(hidden + (long long)t * H + h0 + 8 * cidx);
-      a = row_scale[t];
+    for (int k = 0; k < 4; ++k) {
+      const int t = (c4 + k) * 64 + (tid & 63);
+      v[k] = (c4 + k < p.n_chunks && t < p.T) ? keep_row_factor(p, t, recompute) : 0.f;
     }
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const uint32_t pk = pack_bf16x2(a * __uint_as_float(v[e] << 16), a * __uint_as_float(v[e] & 0xffff0000u));
-      tile[tl][8 * cidx + 2 * e] = (uint16_t)(pk & 0xffffu);
-      tile[tl][8 * cidx + 2 * e + 1] = (uint16_t)(pk >> 16);
+    for (int k = 0; k < 4; ++k) {
+      const bool any = __builtin_amdgcn_ballot_w64(v[k] != 0.f) != 0;
+      if ((tid & 63) == 0 && c4 + k < p.n_chunks) live[c4 + k] = any ? 1 : 0;
     }
   }
   __syncthreads();
+  for (int m = tid; m * 4 < p.n_chunks; m += 1024) {
+    int any = 0;
+    for (int c = m * 4; c < m * 4 + 4 && c < p.n_chunks; ++c) any |= live[c];
+    p.m_tile_live[m] = any;
+  }
+  const int per = (p.n_chunks + 1023) / 1024;
+  const int c0 = tid * per, c1 = (c0 + per < p.n_chunks ? c0 + per : p.n_chunks);
+  int ns = 0, nl = 0;
+  for (int c = c0; c < c1; ++c) {
+    nl += live[c];
+    ns += live[c] && (c == 0 || !live[c - 1]);
+  }
+  // inclusive prefix of (ns, nl) over the 1024 threads: shuffles inside the wavefront, the 16 wavefront totals in LDS
+  {
+    int is = ns, il = nl;
+    const int lane = tid & 63, wv = tid >> 6;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const int us = __shfl_up(is, d, 64), ul = __shfl_up(il, d, 64);
+      if (lane >= d) {
+        is += us;
+        il += ul;
+      }
+    }
+    if (lane == 63) {
+      wave_s[wv] = is;
+      wave_l[wv] = il;
+    }
+    __syncthreads();
+    int bs = 0, bl = 0;
+    for (int w = 0; w < wv; ++w) {
+      bs += wave_s[w];
+      bl += wave_l[w];
+    }
+    starts_before[tid + 1] = bs + is;
+    live_before[tid + 1] = bl + il;
+    if (tid == 0) starts_before[0] = live_before[0] = 0;
+  }
+  __syncthreads();
+  const int n_runs = starts_before[1024], n_live = live_before[1024];
+  if (n_runs > kRunCap) {                  // too fragmented for the list: one run over every K step
+    if (tid == 0) {
+      p.k_runs[0] = 1;
+      p.k_runs[1] = p.k_steps;
+      p.k_runs[2] = 0;
+      p.k_runs[2 + kRunCap] = p.k_steps;
+    }
+    return;
+  }
+  if (tid == 0) {
+    p.k_runs[0] = n_runs;
+    p.k_runs[1] = n_live;
+  }
+  int k = starts_before[tid];              // runs that start before this thread's piece
+  for (int c = c0; c < c1; ++c) {
+    if (!live[c]) continue;
+    if (c == 0 || !live[c - 1]) p.k_runs[2 + k++] = c;                       // run k starts here
+    if (c + 1 >= p.n_chunks || !live[c + 1]) p.k_runs[2 + kRunCap + k - 1] = c + 1;   // and the current run ends here
+  }
+}
+
+// One launch for the row factors, the patched targets, the scaled copy of hidden and the live lists: each is a few
+// microseconds of work behind the same per-token scalars, and a launch that waits for the one before costs 4.7.  Work-group
+// 0 forms the lists (when wanted); in the others every 256 threads take a 64 x 64 tile of hidden, neighbours along H, and
+// form their tokens' factors themselves; the first tile of a token writes them.  With the objective in the splits' merge and
+// one launch that scales all gradients, 777 tokens, H = 1536, V = 151936: 1270 -> 1261 us a step, one box, sides in turn.
+__global__ __launch_bounds__(1024) void keep_backward_prep_kernel(const KeepPrepParams p) {
+  constexpr int kTile = 64 * 66;
+  constexpr int kTileLds = 4 * (kTile * 2 + 64 * 4);
+  __shared__ __attribute__((aligned(16))) char sm[kTileLds > kLiveLds ? kTileLds : kLiveLds];
+  const bool recompute = p.gate != nullptr && *p.gate != 0;
+  const int lists = p.k_runs != nullptr ? 1 : 0;
+  if ((int)blockIdx.x < lists) {
+    keep_live_runs(p, recompute, sm);
+    return;
+  }
+  const int tiles_h = p.hidden_scaled != nullptr ? p.H / 64 : 1;
+  const int grp = threadIdx.x >> 8, tid = threadIdx.x & 255;
+  const long long id = (long long)((int)blockIdx.x - lists) * 4 + grp;
+  const int t0 = (int)(id / tiles_h) * 64, h_tile = (int)(id % tiles_h), h0 = h_tile * 64;
+  const bool live = t0 < p.Tpad;                         // the last work-group may have threads to spare
+  uint16_t* tile = (uint16_t*)sm + grp * kTile;
+  float* factor = (float*)(sm + 4 * kTile * 2) + grp * 64;
+  const int r = tid >> 3, cidx = tid & 7;
+  u32x4_t v[2] = {{0u, 0u, 0u, 0u}, {0u, 0u, 0u, 0u}};
+  if (p.hidden_scaled != nullptr && live) {
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+      const int t = t0 + r + 32 * half;
+      if (t < p.T) v[half] = *(const u32x4_t*)(p.hidden + (long long)t * p.H + h0 + 8 * cidx);
+    }
+  }
+  if (tid < 64) {
+    const int t = t0 + tid;
+    float a = 0.f;
+    if (t < p.T) {
+      a = keep_row_factor(p, t, recompute);
+      if (h_tile == 0) {
+        p.row_scale[t] = a;
+        const long long lab = p.labels[t];
+        if (lab >= 0 && lab < p.V && !recompute) {
+          // p_y - 1 from the fp32 quantities: log p_y = x_y/temperature - lse
+          const float d2 = p.ref2[t] - p.lse[t] * kLog2e;        // log2 s_t
+          p.e[(lab >> 8) * p.blk + (long long)t * 256 + (lab & 255)] =
+              f32_to_bf16_rn(expm1f(p.xy[t] - p.lse[t]) * fast_exp2(-d2));
+        }
+      }
+    }
+    factor[tid] = a;
+  }
+  if (p.hidden_scaled == nullptr) return;                // the same for every thread of the launch
+  __syncthreads();
+#pragma unroll
+  for (int half = 0; half < 2; ++half) {
+    const int tl = r + 32 * half;
+    const float a = factor[tl];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const uint32_t pk = pack_bf16x2(a * __uint_as_float(v[half][e] << 16), a * __uint_as_float(v[half][e] & 0xffff0000u));
+      tile[tl * 66 + 8 * cidx + 2 * e] = (uint16_t)(pk & 0xffffu);
+      tile[tl * 66 + 8 * cidx + 2 * e + 1] = (uint16_t)(pk >> 16);
+    }
+  }
+  __syncthreads();
+  if (!live) return;
 #pragma unroll
   for (int half = 0; half < 2; ++half) {
     const int hl = r + 32 * half;
     u32x4_t o;
 #pragma unroll
     for (int e = 0; e < 4; ++e)
-      o[e] = (uint32_t)tile[8 * cidx + 2 * e][hl] | ((uint32_t)tile[8 * cidx + 2 * e + 1][hl] << 16);
-    *(u32x4_t*)(out + (long long)(h0 + hl) * ld + t0 + 8 * cidx) = o;
+      o[e] = (uint32_t)tile[(8 * cidx + 2 * e) * 66 + hl] | ((uint32_t)tile[(8 * cidx + 2 * e + 1) * 66 + hl] << 16);
+    *(u32x4_t*)(p.hidden_scaled + (long long)(h0 + hl) * p.ld_scaled + t0 + 8 * cidx) = o;
   }
+}
+
+inline void launch_keep_backward_prep(const KeepPrepParams& p, hipStream_t st) {
+  const long long tiles = (long long)(p.Tpad / 64) * (p.hidden_scaled != nullptr ? p.H / 64 : 1);
+  hipLaunchKernelGGL(keep_backward_prep_kernel, dim3((unsigned)((tiles + 3) / 4) + (p.k_runs != nullptr ? 1 : 0)), dim3(1024), 0, st, p);
 }
 
 // Sum of the ksplit fp32 slices a split contraction wrote (fixed order: bit-reproducible), times the row factor,
@@ -419,13 +577,25 @@ __global__ void keep_col_sum_kernel(const bf16_t* e, long long blk, const float*
 }
 
 // x[i] *= *scale for a bf16 or fp32 array, 16 bytes per thread and step (n: elements; the base is 16-byte aligned).
-// A scale of exactly 1 leaves the array untouched: every work-group returns after reading the scalar.
-__global__ __launch_bounds__(256) void scale_inplace_kernel(void* x, long long n, int is_f32, const float* scale) {
-  const float s = *scale;
+// A scale of exactly 1 leaves the array untouched: every work-group returns after reading the scalar.  Up to three arrays
+// of one type a launch (the gradients of a step): work-groups [first[i], first[i + 1]) share array i.
+struct ScaleParams {
+  void* x[3];
+  long long n[3];
+  int first[4];
+  int is_f32;
+  const float* scale;
+};
+__global__ __launch_bounds__(256) void scale_inplace_kernel(const ScaleParams p) {
+  const float s = *p.scale;
   if (s == 1.f) return;
+  const int which = (int)blockIdx.x >= p.first[2] ? 2 : (int)blockIdx.x >= p.first[1] ? 1 : 0;
+  void* x = p.x[which];
+  const long long n = p.n[which];
+  const int is_f32 = p.is_f32, block = (int)blockIdx.x - p.first[which], blocks = p.first[which + 1] - p.first[which];
   const long long per = is_f32 ? 4 : 8;
   const long long nv = n / per;
-  for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < nv; i += (long long)gridDim.x * 256) {
+  for (long long i = (long long)block * 256 + threadIdx.x; i < nv; i += (long long)blocks * 256) {
     if (is_f32) {
       float4 v = ((float4*)x)[i];
       v.x *= s, v.y *= s, v.z *= s, v.w *= s;
@@ -438,7 +608,7 @@ __global__ __launch_bounds__(256) void scale_inplace_kernel(void* x, long long n
       ((u32x4_t*)x)[i] = v;
     }
   }
-  if (blockIdx.x == 0 && threadIdx.x == 0)
+  if (block == 0 && threadIdx.x == 0)
     for (long long i = nv * per; i < n; ++i) {
       if (is_f32)
         ((float*)x)[i] *= s;
@@ -447,102 +617,5 @@ __global__ __launch_bounds__(256) void scale_inplace_kernel(void* x, long long n
     }
 }
 
-// Which parts of the token axis carry a gradient at all (row factor a_t != 0): zero-advantage samples and ignored
-// labels form long stretches of dead rows, which the gradient GEMMs skip - the dHidden product by 256-row tile
-// (m_tile_live), the dW product, whose contraction runs over the tokens, by K step of 64 rows (k_runs: the list of
-// live runs gemm_mainloop_km walks).  One work-group; thread i owns a contiguous piece of the 64-row chunks.
-// If the rows alternate more often than the list can hold, k_runs[0] is written as one run over everything
-// (the products are then merely not shortened).
-struct KeepLiveParams {
-  const float* row_scale;    // [T]
-  int T;
-  int n_chunks;              // ceil(T / 64), at most kLiveMaxChunks
-  int k_steps;               // K steps of the dW product (round_up(T, 256) / 64)
-  int* k_runs;               // [2 + 2 * kRunCap]
-  int* m_tile_live;          // [ceil(T / 256)]
-};
-constexpr int kLiveMaxChunks = 32768;      // 2 M tokens: beyond that nothing is skipped (the lists say "all live")
-
-__global__ __launch_bounds__(1024) void keep_live_runs_kernel(const KeepLiveParams p) {
-  __shared__ unsigned char live[kLiveMaxChunks];
-  __shared__ int starts_before[1024 + 1], live_before[1024 + 1];
-  const int tid = threadIdx.x;
-  // chunk flags: one wavefront per chunk, 64 rows each
-  // (four chunks per wavefront and round, so that four loads are in flight at a time)
-  for (int c4 = (tid >> 6) * 4; c4 < p.n_chunks; c4 += 64) {
-    float v[4];
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const int t = (c4 + k) * 64 + (tid & 63);
-      v[k] = (c4 + k < p.n_chunks && t < p.T) ? p.row_scale[t] : 0.f;
-    }
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const bool any = __builtin_amdgcn_ballot_w64(v[k] != 0.f) != 0;
-      if ((tid & 63) == 0 && c4 + k < p.n_chunks) live[c4 + k] = any ? 1 : 0;
-    }
-  }
-  __syncthreads();
-  for (int m = tid; m * 4 < p.n_chunks; m += 1024) {
-    int any = 0;
-    for (int c = m * 4; c < m * 4 + 4 && c < p.n_chunks; ++c) any |= live[c];
-    p.m_tile_live[m] = any;
-  }
-  const int per = (p.n_chunks + 1023) / 1024;
-  const int c0 = tid * per, c1 = (c0 + per < p.n_chunks ? c0 + per : p.n_chunks);
-  int ns = 0, nl = 0;
-  for (int c = c0; c < c1; ++c) {
-    nl += live[c];
-    ns += live[c] && (c == 0 || !live[c - 1]);
-  }
-  // inclusive prefix of (ns, nl) over the 1024 threads: shuffles inside the wavefront, the 16 wavefront totals in LDS
-  {
-    int is = ns, il = nl;
-    const int lane = tid & 63, wv = tid >> 6;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-      const int us = __shfl_up(is, d, 64), ul = __shfl_up(il, d, 64);
-      if (lane >= d) {
-        is += us;
-        il += ul;
-      }
-    }
-    __shared__ int wave_s[16], wave_l[16];
-    if (lane == 63) {
-      wave_s[wv] = is;
-      wave_l[wv] = il;
-    }
-    __syncthreads();
-    int bs = 0, bl = 0;
-    for (int w = 0; w < wv; ++w) {
-      bs += wave_s[w];
-      bl += wave_l[w];
-    }
-    starts_before[tid + 1] = bs + is;
-    live_before[tid + 1] = bl + il;
-    if (tid == 0) starts_before[0] = live_before[0] = 0;
-  }
-  __syncthreads();
-  const int n_runs = starts_before[1024], n_live = live_before[1024];
-  if (n_runs > kRunCap) {                  // too fragmented for the list: one run over every K step
-    if (tid == 0) {
-      p.k_runs[0] = 1;
-      p.k_runs[1] = p.k_steps;
-      p.k_runs[2] = 0;
-      p.k_runs[2 + kRunCap] = p.k_steps;
-    }
-    return;
-  }
-  if (tid == 0) {
-    p.k_runs[0] = n_runs;
-    p.k_runs[1] = n_live;
-  }
-  int k = starts_before[tid];              // runs that start before this thread's piece
-  for (int c = c0; c < c1; ++c) {
-    if (!live[c]) continue;
-    if (c == 0 || !live[c - 1]) p.k_runs[2 + k++] = c;                       // run k starts here
-    if (c + 1 >= p.n_chunks || !live[c + 1]) p.k_runs[2 + kRunCap + k - 1] = c + 1;   // and the current run ends here
-  }
-}
 
 }  // namespace fgrpo

@@ -271,44 +271,47 @@ struct LossParams {
 
 constexpr int kLossThreads = 256;
 
+// The objective of one token with log-probability lp: writes the token's outputs, returns its weighted term (0 where the
+// label is ignored) and whether it counts.
+__device__ __forceinline__ float grpo_token(const LossParams& p, int t, float lp, bool& valid) {
+  valid = p.labels[t] != -100;
+  const float old = p.old_lp ? p.old_lp[t] : lp;
+  const float a = p.adv[t];
+  const float lr = lp - old;
+  const float r = expf(lr);
+  const float lo = 1.0f - p.clip_low, hi = 1.0f + p.clip_high;
+  const float l1 = -a * r;
+  const float rc = fminf(fmaxf(r, lo), hi);
+  const float l2 = -a * rc;
+  const float c1 = fmaxf(l1, l2);
+  const float c2 = fminf(c1, -a * p.clip_c);
+  float tok = (a < 0.f) ? c2 : c1;
+  const bool live = (a > 0.f && r <= hi) || (a < 0.f && r >= lo && r <= p.clip_c);
+  float dtok = live ? -a * r : 0.f;
+  if (p.ref_lp && p.kl_beta != 0.f) {
+    const float d = p.ref_lp[t] - lp;
+    const float ed = expf(d);
+    tok += p.kl_beta * (ed - d - 1.0f);
+    dtok += p.kl_beta * (1.0f - ed);
+  }
+  const float w = valid ? (p.tokw ? p.tokw[t] : 1.0f) : 0.f;
+  float gv = w * dtok;
+  if (p.pre) gv *= (float)p.pre[3];
+  p.g[t] = gv;
+  if (p.log_ratio) p.log_ratio[t] = lr;
+  if (p.clip1) p.clip1[t] = c1;
+  if (p.unclipped) p.unclipped[t] = l1;
+  if (p.clipped) p.clipped[t] = l2;
+  return valid ? w * tok : 0.f;
+}
+
 __global__ __launch_bounds__(kLossThreads) void grpo_loss_tokens_kernel(const LossParams p) {
   __shared__ double sh[2][kLossThreads / 64];
   const int t = blockIdx.x * kLossThreads + threadIdx.x;
   float contrib = 0.f;
-  int cnt = 0;
-  if (t < p.T) {
-    const bool valid = p.labels[t] != -100;
-    const float lp = p.lp[t];
-    const float old = p.old_lp ? p.old_lp[t] : lp;
-    const float a = p.adv[t];
-    const float lr = lp - old;
-    const float r = expf(lr);
-    const float lo = 1.0f - p.clip_low, hi = 1.0f + p.clip_high;
-    const float l1 = -a * r;
-    const float rc = fminf(fmaxf(r, lo), hi);
-    const float l2 = -a * rc;
-    const float c1 = fmaxf(l1, l2);
-    const float c2 = fminf(c1, -a * p.clip_c);
-    float tok = (a < 0.f) ? c2 : c1;
-    const bool live = (a > 0.f && r <= hi) || (a < 0.f && r >= lo && r <= p.clip_c);
-    float dtok = live ? -a * r : 0.f;
-    if (p.ref_lp && p.kl_beta != 0.f) {
-      const float d = p.ref_lp[t] - lp;
-      const float ed = expf(d);
-      tok += p.kl_beta * (ed - d - 1.0f);
-      dtok += p.kl_beta * (1.0f - ed);
-    }
-    const float w = valid ? (p.tokw ? p.tokw[t] : 1.0f) : 0.f;
-    float gv = w * dtok;
-    if (p.pre) gv *= (float)p.pre[3];
-    p.g[t] = gv;
-    if (p.log_ratio) p.log_ratio[t] = lr;
-    if (p.clip1) p.clip1[t] = c1;
-    if (p.unclipped) p.unclipped[t] = l1;
-    if (p.clipped) p.clipped[t] = l2;
-    contrib = valid ? w * tok : 0.f;
-    cnt = valid;
-  }
+  bool valid = false;
+  if (t < p.T) contrib = grpo_token(p, t, p.lp[t], valid);
+  const int cnt = valid;
   double s = wave_sum_d((double)contrib);
   int c = wave_sum_i(cnt);
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;

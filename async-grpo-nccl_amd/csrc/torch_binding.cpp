@@ -40,7 +40,7 @@ struct Api {
   FGRPO_ENTRY(fgrpo_grpo_step_chunked_supported);
   FGRPO_ENTRY(fgrpo_grpo_step_chunked_workspace);
   FGRPO_ENTRY(fgrpo_grpo_step_chunked);
-  FGRPO_ENTRY(fgrpo_scale_inplace);
+  FGRPO_ENTRY(fgrpo_scale_gradients);
   FGRPO_ENTRY(fgrpo_varlen_attn_workspace);
   FGRPO_ENTRY(fgrpo_varlen_attn_fwd_ws);
   FGRPO_ENTRY(fgrpo_varlen_attn_bwd_ws);
@@ -69,7 +69,7 @@ void init(const std::unordered_map<std::string, uint64_t>& at) {
   FGRPO_SET(fgrpo_grpo_step_chunked_supported);
   FGRPO_SET(fgrpo_grpo_step_chunked_workspace);
   FGRPO_SET(fgrpo_grpo_step_chunked);
-  FGRPO_SET(fgrpo_scale_inplace);
+  FGRPO_SET(fgrpo_scale_gradients);
   FGRPO_SET(fgrpo_varlen_attn_workspace);
   FGRPO_SET(fgrpo_varlen_attn_fwd_ws);
   FGRPO_SET(fgrpo_varlen_attn_bwd_ws);
@@ -274,9 +274,11 @@ struct FusedStep : torch::autograd::Function<FusedStep> {
       sd["dh"] = Tensor(), sd["dw"] = Tensor(), sd["db"] = Tensor();
       const Tensor scale = gout.detach().reshape({-1}).to(at::kFloat).contiguous();
       OnDevice d(scale);
-      for (const Tensor& t : {r.dh, r.dw, r.db})
-        if (t.defined() && t.numel() > 0)
-          check(api.fgrpo_scale_inplace(t.data_ptr(), t.numel(), dtype_code(t), fptr(scale), d.stream()), "scale_inplace");
+      auto count = [](const Tensor& t) { return t.defined() ? (long long)t.numel() : 0LL; };
+      auto data = [](const Tensor& t) { return t.defined() ? t.data_ptr() : nullptr; };
+      check(api.fgrpo_scale_gradients(data(r.dh), count(r.dh), data(r.dw), count(r.dw), data(r.db), count(r.db), FGRPO_BF16,
+                                      fptr(scale), d.stream()),
+            "scale_gradients");
       return {r.dh, r.dw, r.db, Tensor(), Tensor(), Tensor(), Tensor()};
     }
     const auto saved = ctx->get_saved_variables();

@@ -51,6 +51,7 @@ SIGNATURES = {
     "fgrpo_grpo_step_chunked": (_i, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _f, _i, _i, _i, _i, _f, _f, _f, _f, _i,
                                      _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _sz, _vp]),
     "fgrpo_scale_inplace": (_i, [_vp, _ll, _i, _vp, _vp]),
+    "fgrpo_scale_gradients": (_i, [_vp, _ll, _vp, _ll, _vp, _ll, _i, _vp, _vp]),
     "fgrpo_metrics": (_i, [_vp, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp, _f, _f, _vp, _vp, _vp]),
     "fgrpo_group_advantages": (_i, [_vp, _i, _vp, _i, _i, _d, _vp, _vp, _vp]),
     "fgrpo_segment_broadcast": (_i, [_vp, _i, _vp, _i, _i, _vp, _vp]),

@@ -227,6 +227,9 @@ int fgrpo_grpo_step_chunked(const void* hidden, const void* weight, const void* 
                             void* dH_out, void* dW_out, void* dbias_out,
                             void* workspace, size_t workspace_bytes, void* stream);
 int fgrpo_scale_inplace(void* x, long long n, int dtype, const float* scale_dev, void* stream);
+/* The same for the gradients of one step in one launch: any of the three may be NULL or empty. */
+int fgrpo_scale_gradients(void* dh, long long n_dh, void* dw, long long n_dw, void* db, long long n_db,
+                          int dtype, const float* scale_dev, void* stream);
 
 /* ---- diagnostics on the output-token positions ---------------------------------
  * Replaces the ~20 .item() reductions of compute_dual_clip_grpo_loss

@@ -240,3 +240,55 @@ def test_chunked_step_is_capturable_in_a_hip_graph(dev):
         torch.cuda.synchronize()
         for a, b in zip(captured, eager):
             assert torch.equal(a, b), f"replay {k}"
+
+
+@pytest.mark.parametrize("T", [1, 15, 17, 63, 65, 257, 513])
+def test_step_at_the_edges_of_its_token_groups(dev, T):
+    """The objective is formed sixteen tokens at a time by the merge of the vocabulary splits, the scaled operand of dW by
+    tiles of 64: against the recomputing pair on the same operands, with a bias, ignored labels and an upstream factor.
+    Tolerances: logprobs of the same products in another order; gradients to bf16 roundings of numerators, rows and results."""
+    from fgrpo import ops
+    H, V = 256, 33001
+    gen = torch.Generator().manual_seed(T)
+    w = (torch.randn(V, H, generator=gen) * 0.05).bfloat16().to(dev)
+    h = torch.randn(T, H, generator=gen).bfloat16().to(dev)
+    b = (torch.randn(V, generator=gen) * 0.3).bfloat16().to(dev)
+    y = torch.randint(0, V, (T,), generator=gen)
+    y[torch.rand(T, generator=gen) < 0.2] = -100
+    y[0] = 5
+    y = y.to(dev)
+    adv = torch.randn(T, generator=gen).to(dev)
+    old = ops.lmhead_logprob_fwd(h, w, b, y)[0] + torch.randn(T, generator=gen).to(dev) * 0.05
+    cu = torch.tensor([0, (T + 1) // 2, T], dtype=torch.int32, device=dev)
+    outs = []
+    for keep in ("chunked", False):
+        args = [x.clone().requires_grad_(True) for x in (h, w, b)]
+        out = ops.fused_grpo_loss(args[0], args[1], args[2], y, old, adv, old - 0.1, cu, 1.0, 0.2, 0.28, 3.0, 0.04, "sample_mean",
+                                  0.0, 0, False, keep, 256)
+        (out[0] * 2.5).backward()
+        outs.append((out, [x.grad for x in args]))
+    (a, ga), (c, gc) = outs
+    assert abs(a[0].item() - c[0].item()) <= 1e-5 * max(1.0, abs(c[0].item()))
+    for p, q in zip(a[1:], c[1:]):
+        assert (p - q).abs().max() <= 2e-5 * max(1.0, float(q.abs().max()))
+    for p, q in zip(ga, gc):
+        assert (p.double() - q.double()).norm() <= 1e-2 * q.double().norm()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("sizes", [(5, 70001, 3), (0, 9, 0), (2048, 0, 17), (0, 0, 0), (1, 1, 4097 * 256 * 8 + 5)])
+def test_gradients_are_scaled_in_one_launch(dev, dtype, sizes):
+    from fgrpo import _lib
+    xs = [torch.randn(n, device=dev).to(dtype) if n else None for n in sizes]
+    for s in (1.0, -2.5):
+        want = [None if x is None else x.clone() if s == 1.0 else (x.float() * s).to(dtype) for x in xs]
+        flat = []
+        for x in xs:
+            flat += [0 if x is None else x.data_ptr(), 0 if x is None else x.numel()]
+        scale = torch.tensor([s], device=dev)
+        rc = _lib.load().fgrpo_scale_gradients(*flat, _lib.F32 if dtype == torch.float32 else _lib.BF16, scale.data_ptr(),
+                                               torch.cuda.current_stream().cuda_stream)
+        assert rc == 0
+        torch.cuda.synchronize()
+        for x, y in zip(xs, want):
+            assert x is None or torch.equal(x, y)
