@@ -1258,6 +1258,9 @@ __device__ __forceinline__ f32x16_t attn_mfma(u32x4_t a, u32x4_t b, f32x16_t acc
 // the matrix instructions want them, an instruction touches 32 rows and takes the address unit about 115 cycles instead
 // of 15; so rows change hands in LDS, in a swizzled patch of the wavefront's own (32 rows, see attn_swz).  The descriptor
 // ends with the last row: rows past it read as zero and are not written.
+// Stores are non-temporal (the last argument's bit 1), here and in dK/dV: nothing of the launch reads them, and K and V keep
+// their place in the L2s.  Forward + backward, one box, sides in turn: 32768 tokens of 128..1024, 12 / 2 heads of 128 507 ->
+// 494 us; 12345, 14 / 2 heads of 64 131 -> 129; 4 x 8192, 28 / 4 heads 7.84 -> 7.80 ms.  Row loads marked so gain nothing.
 template <int HD>
 struct AttnRows {
   static constexpr int RPI = 1024 / (HD * 2);
@@ -1281,7 +1284,7 @@ struct AttnRows {
   }
   __device__ __forceinline__ void store(const u32x4_t (&r)[HD / 16]) const {
 #pragma unroll
-    for (int i = 0; i < HD / 16; ++i) __builtin_amdgcn_raw_buffer_store_b128(r[i], rs, (int)off, (int)(i * step), 0);
+    for (int i = 0; i < HD / 16; ++i) __builtin_amdgcn_raw_buffer_store_b128(r[i], rs, (int)off, (int)(i * step), 2);
   }
 };
 // loaded rows -> operand: the lane's own row (lane % 32), chunks 2 s + lane / 32.  rowc: AttnLane::rowc, the patch's base included

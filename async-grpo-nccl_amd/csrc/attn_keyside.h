@@ -596,7 +596,7 @@ __global__ __launch_bounds__(256, KB == 2 ? 1 : 2) void varlen_attn_dkv3_kernel(
       }
 #pragma unroll
       for (int j = 0; j < 8; ++j) x[j] *= mul;
-      if (kk < p.T && !partial) *(bf16x8_t*)(out + ((long long)kk * p.Hkv + hkv) * HD + col * 8) = attn_pack8(x);
+      if (kk < p.T && !partial) __builtin_nontemporal_store(__builtin_bit_cast(u32x4_t, attn_pack8(x)), (u32x4_t*)(out + ((long long)kk * p.Hkv + hkv) * HD + col * 8));
     }
     wait_lgkm<0>();
   };
