@@ -503,12 +503,18 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* part, i
   const int m = (int)(q / nq), n = (int)(q - (long long)m * nq) * 4;
   const float* src = part + (long long)m * ld + n;
   float4 s = *(const float4*)src;
-  for (int k = 1; k < ksplit; ++k) {
-    const float4 v = *(const float4*)(src + (long long)k * slice);
-    s.x += v.x;
-    s.y += v.y;
-    s.z += v.z;
-    s.w += v.w;
+  for (int k0 = 1; k0 < ksplit; k0 += 8) {                // eight loads in flight
+    float4 v[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) v[k] = *(const float4*)(src + (long long)(k0 + k < ksplit ? k0 + k : 0) * slice);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      if (k0 + k >= ksplit) break;
+      s.x += v[k].x;
+      s.y += v[k].y;
+      s.z += v[k].z;
+      s.w += v[k].w;
+    }
   }
   const float a = row_scale ? row_scale[m] : 1.f;
   uint2 o;

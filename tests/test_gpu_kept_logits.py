@@ -228,6 +228,35 @@ def test_few_tokens_take_the_kept_path_too(dev, tokens):
     assert (dH.cpu()[~valid] == 0).all()
 
 
+@pytest.mark.parametrize("tokens,H,V", [(1, 256, 70001), (200, 256, 70001), (255, 128, 140000), (333, 320, 70001), (520, 512, 40007),
+                                        (1290, 512, 33001)])
+def test_few_token_tiles_fill_the_device(dev, tokens, H, V):
+    """Forward with more than 64 vocabulary splits, six token tiles to a raster group, dHidden's contraction in more than
+    sixteen pieces (their number no multiple of the eight slices summed at a time).  Against fp64 on the same operands:
+    logprobs to fp32 sums over V terms; gradients to bf16 roundings of the numerators, the rows and the results."""
+    from fgrpo import ops
+    assert ops.chunked_supported(tokens, H, V, torch.bfloat16, 8192)
+    gen = torch.Generator().manual_seed(tokens)
+    w = (torch.randn(V, H, generator=gen) * 0.05).bfloat16().to(dev).requires_grad_(True)
+    h = torch.randn(tokens, H, generator=gen).bfloat16().to(dev).requires_grad_(True)
+    y = torch.randint(0, V, (tokens,), generator=gen).to(dev)
+    adv = torch.randn(tokens, generator=gen).to(dev)
+    out = ops.fused_grpo_loss(h, w, None, y, None, adv, keep_logits="chunked", chunk_tokens=8192)
+    dh, dw = torch.autograd.grad(out[0], (h, w))
+    hd, wd = h.detach().double(), w.detach().double()
+    x = hd @ wd.t()
+    lse = torch.logsumexp(x, 1)
+    p = torch.exp(x - lse[:, None])
+    assert (out[6] - (x.gather(1, y[:, None])[:, 0] - lse)).abs().max() <= 4e-5
+    assert (out[1] - (lse - (p * x).sum(1))).abs().max() <= 4e-5
+    del x
+    g = -adv.double() / tokens                                # ratio 1: d loss / d lp = -advantage / tokens
+    p *= -g[:, None]
+    p.scatter_add_(1, y[:, None], g[:, None])
+    for got, want in ((dh, p @ wd), (dw, p.t() @ hd)):
+        assert (got.double() - want).norm() <= 8e-3 * want.norm()
+
+
 @pytest.mark.parametrize("tokens,H", [(64 * 256 + 700, 2048), (9000, 1024), (33 * 256 + 1, 1536)])
 def test_split_contraction_of_the_last_row_tiles(dev, tokens, H):
     """dHidden's row tiles beyond whole device rounds (or all of them, when there are few) have their contraction
