@@ -1271,6 +1271,8 @@ int kept_bwd_impl(const Tuning& tn, const void* hidden, const void* weight, cons
           t.part_slice = (long long)tr * H;
           t.tiles_m = (tr + 255) / 256;
           t.tiles_n = (H + 255) / 256;
+          const int chunks = (t.tiles_n + 7) / 8;
+          t.rr_cols = (t.tiles_n + chunks - 1) / chunks;
           t.nblocks = t.tiles_m * t.tiles_n * sp.ksplit;
           t.wide_stores = can_store_wide(tn, t);
           rc = launch_store_splitk(t, st);

@@ -775,9 +775,13 @@ __global__ __launch_bounds__(C::NT, C::OCC) void gemm_store_kernel(const StorePa
     const int lid = xcd_contiguous_id(blockIdx.x, gridDim.x);
     const int tiles = p.tiles_m * p.tiles_n;
     // pieces of one K range side by side, and of them the column tiles of a row tile: they stream the same slice of
-    // A, the big operand (rows fastest instead: 6.7 against 5.6 ms at T = 16384, H = 1536, V = 151936)
+    // A, the big operand (rows fastest instead: 6.7 against 5.6 ms at T = 16384, H = 1536, V = 151936).  More than eight
+    // column tiles go in chunks of at most eight, every row tile of a chunk before the next: the 32 work-groups of an
+    // XCD then fetch about 12 slices a K step, with all of H = 8192 in a row 33
     const int ks = lid / tiles, w = lid - ks * tiles;
-    const int tm = w / p.tiles_n, tn = w - tm * p.tiles_n;
+    const int chunk = w / (p.tiles_m * p.rr_cols), first_n = chunk * p.rr_cols, w2 = w - first_n * p.tiles_m;
+    const int wide = p.tiles_n - first_n < p.rr_cols ? p.tiles_n - first_n : p.rr_cols;
+    const int tm = w2 / wide, tn = first_n + w2 - tm * wide;
     const int row0 = tm * C::BM, col0 = tn * C::BN;
     const int k0 = ks * p.kchunk;
     const int klen = (p.g.seg[0].K - k0) < p.kchunk ? (p.g.seg[0].K - k0) : p.kchunk;

@@ -84,12 +84,12 @@ __global__ __launch_bounds__(64 * kSegmentsPerGroup) void segment_valid_weight_k
   for (int t = b + lane; t < e; t += 64) tokw[t] = w;
 }
 
-// out[t] = values[s] for every token of segment s
 inline void launch_segment_weights(const long long* labels, const int* cu, int nseq, int T, int* cnt, float* tokw, hipStream_t st) {
   const int groups = (nseq + kSegmentsPerGroup - 1) / kSegmentsPerGroup + (T + kZeroTokensPerGroup - 1) / kZeroTokensPerGroup;
   hipLaunchKernelGGL(segment_valid_weight_kernel, dim3(groups), dim3(64 * kSegmentsPerGroup), 0, st, labels, cu, nseq, T, cnt, tokw);
 }
 
+// out[t] = values[s] for every token of segment s
 __global__ void segment_broadcast_kernel(const void* values, int values_f64, const int* cu, int nseq, int T, float* out) {
   const int s = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;

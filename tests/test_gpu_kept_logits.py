@@ -229,7 +229,7 @@ def test_few_tokens_take_the_kept_path_too(dev, tokens):
 
 
 @pytest.mark.parametrize("tokens,H,V", [(1, 256, 70001), (200, 256, 70001), (255, 128, 140000), (333, 320, 70001), (520, 512, 40007),
-                                        (1290, 512, 33001)])
+                                        (1290, 512, 33001), (300, 2304, 33001), (600, 4160, 33001)])
 def test_few_token_tiles_fill_the_device(dev, tokens, H, V):
     """Forward with more than 64 vocabulary splits, six token tiles to a raster group, dHidden's contraction in more than
     sixteen pieces (their number no multiple of the eight slices summed at a time).  Against fp64 on the same operands:
