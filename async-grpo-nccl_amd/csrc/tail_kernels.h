@@ -42,10 +42,17 @@ __global__ void fill_i64_kernel(long long* dst, long long v, int n) {
 // ---------------------------------------------------------------------------
 // Segment (sample) statistics over cu_seqlens: one wavefront per segment.
 // ---------------------------------------------------------------------------
+__device__ __forceinline__ bool in_a_segment(const int* cu, int nseq, int t) {
+  for (int s = 0; s < nseq; ++s)
+    if (cu[s] <= t && t < cu[s + 1]) return true;
+  return false;
+}
+
 // cnt[s] = number of valid (label != -100) tokens of segment s; tokw[t] = 1/cnt
 // of the token's segment (0 when the segment has no valid token, and for tokens outside every segment).
 // Work-groups past the segments' write the zeros: a token no range covers lies below every boundary, at or above all
-// of them, or - in a vector that runs backwards - between its last boundary and its first.  One launch instead of a
+// of them, or - in a vector that runs backwards - between its last boundary and its first, where the ranges are walked (a
+// stretch that rises again there has its weight from its own wavefront).  One launch instead of a
 // fill in front of the segments: a step of 643 tokens is bound by its launches (figures at gemm_small_split_kernel).
 constexpr int kSegmentsPerGroup = 4, kZeroTokensPerGroup = 4096;
 __global__ __launch_bounds__(64 * kSegmentsPerGroup) void segment_valid_weight_kernel(const long long* labels, const int* cu,
@@ -70,7 +77,7 @@ __global__ __launch_bounds__(64 * kSegmentsPerGroup) void segment_valid_weight_k
     const int t0 = ((int)blockIdx.x - seg_groups) * kZeroTokensPerGroup;
     const int t1 = T - t0 < kZeroTokensPerGroup ? T : t0 + kZeroTokensPerGroup;
     for (int t = t0 + (int)threadIdx.x; t < t1; t += 64 * kSegmentsPerGroup)
-      if (t < lo || t >= hi || (t >= last && t < first)) tokw[t] = 0.f;
+      if (t < lo || t >= hi || (t >= last && t < first && !in_a_segment(cu, nseq, t))) tokw[t] = 0.f;
     return;
   }
   if (s >= nseq) return;

@@ -165,7 +165,8 @@ def test_fp32_gradients_do_not_depend_on_which_are_wanted(dev, T, H, V, panel_el
 
 
 @pytest.mark.parametrize("T,bounds", [(643, [0, 40, 41, 41, 643]), (9000, [5, 100, 8000]), (4097, [0, 4097]), (4096, [4095, 4096]),
-                                      (300, [0, 100, 300, 0]), (300, [200, 50]), (300, [-7, 20, 400]), (1, [0, 0])])
+                                      (300, [0, 100, 300, 0]), (300, [200, 50]), (300, [-7, 20, 400]), (1, [0, 0]),
+                                      (300, [250, 20, 90, 0]), (5000, [4900, 100, 4400, 3, 90, 0])])
 def test_segment_weights_cover_every_token(dev, T, bounds):
     """1 / (scored tokens of the sample), zero outside every sample: boundaries that start late, end early, repeat, leave
     the batch or run backwards."""
