@@ -153,33 +153,33 @@ __device__ __forceinline__ bf16x8_t attn_pack8(const float* x) {
   return __builtin_bit_cast(bf16x8_t, v);
 }
 
-// 64 rows x 256 bytes of one head: global -> registers.  Buffer loads over a descriptor that starts at row `row0`
-// (wavefront-uniform) and ends with row `row_end - 1`: rows from row_end on read as zero, and a load costs one
-// instruction - the lane's byte offset inside the slab is a constant computed once per kernel.
+// 64 rows x 2 HD bytes of one head: global -> registers, rows from row_end on as zeros.  By 64-bit address: the kernels
+// that use this also take the calls whose rows lie farther apart than a descriptor's 32-bit offsets (attn_route.h).  A
+// thread's chunks are whole rows apart, so its place in the slab is one offset, computed once per kernel; rows that do not
+// exist are loaded from a chunk of zeros, without a branch.
+static __device__ u32x4_t attn_no_row;
 template <int HD>
 struct AttnFetch {
-  uint32_t off[HD / 32];      // 64 rows x HD/8 chunks over 256 threads
+  int row;                    // the thread's first row, then every 2048 / HD-th
+  long long off;              // elements
 };
 template <int HD>
 __device__ __forceinline__ AttnFetch<HD> attn_fetch_init(long long st) {
-  AttnFetch<HD> f;
-#pragma unroll
-  for (int i = 0; i < HD / 32; ++i) {
-    const int c = threadIdx.x + 256 * i;
-    f.off[i] = (uint32_t)(((long long)(c / (HD / 8)) * st + (c % (HD / 8)) * 8) * 2);
-  }
-  return f;
+  const int row = threadIdx.x / (HD / 8);
+  return AttnFetch<HD>{row, row * st + threadIdx.x % (HD / 8) * 8};
 }
 template <int HD>
 __device__ __forceinline__ void attn_fetch_rows(u32x4_t (&r)[HD / 32], const AttnFetch<HD>& f, const bf16_t* base, long long st,
                                                 int row0, int row_end) {
-  const long long rows = (long long)row_end - row0;
-  long long bytes = rows > 0 ? (rows - 1) * st * 2 + HD * 2 : 0;
-  if (bytes > 0xffffffffLL) bytes = 0xffffffffLL;
-  const __amdgpu_buffer_rsrc_t rs = make_rsrc(base + (long long)row0 * st, (uint32_t)bytes);
+  constexpr int RPS = 2048 / HD;
+  long long off = f.off;
+  asm volatile("" : "+v"(off));      // addresses are formed anew: the walks would carry each load's as a pointer of its own, and dQ then spills 25 registers
+  const bf16_t* src = base + (long long)row0 * st + off;
 #pragma unroll
-  for (int i = 0; i < HD / 32; ++i)
-    r[i] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rs, (int)f.off[i], 0, 0));
+  for (int i = 0; i < HD / 32; ++i) {
+    const u32x4_t* chunk = (const u32x4_t*)(src + (long long)(i * RPS) * st);
+    r[i] = *(row0 + i * RPS + f.row < row_end ? chunk : &attn_no_row);
+  }
 }
 // ... and registers -> swizzled LDS tile
 template <int HD>

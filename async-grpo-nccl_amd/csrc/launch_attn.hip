@@ -3,6 +3,7 @@
 
 #include "host_common.h"
 #include "attn_kernels.h"
+#include "attn_route.h"
 
 using namespace fgrpo;
 
@@ -14,11 +15,6 @@ int launch_attn_merge_bwd(int D, const AttnParams& p, int rb, hipStream_t st);
 }
 
 namespace {
-// The hand-scheduled query-side kernels address a wavefront's 32 query rows with 32-bit byte offsets; rows farther apart
-// take the register-staged ones.
-bool wave_rows_in_reach(long long q_st, int Hq, int D) { return 31 * q_st * 2 + D * 2 < (1LL << 32) && 62LL * Hq * D + D * 2 < (1LL << 32); }
-int query_side_form(const Tuning& tn, long long q_st, int Hq, int D) { return wave_rows_in_reach(q_st, Hq, D) ? tn.attn_qside : 1; }
-
 // Query heads per work-group of the query-side kernels (tile = 128 / heads tokens).  Short segments gain from short
 // tiles (less masked work on the diagonal and at segment boundaries) as long as the heads of a group fill the
 // work-group; long ones do not care, and a lone head per K/V head has nothing to share.
@@ -110,8 +106,8 @@ SplitPlan plan_query_split(const Tuning& tn, int form, int T, int n_seq, int Hq,
   return plan_split(wgs, 2, (double)T / n_seq / kAttnBK, causal, D == 128 ? 1.6 : forward ? 1.15 : 1.3,
                     (size_t)T * Hq * (D * 4 + (forward ? 8 : 0)));
 }
-SplitPlan plan_key_split(const Tuning& tn, int T, int n_seq, int Hq, int Hkv, int D, int causal) {
-  if (tn.attn_dkv == 1 || tn.attn_dkv == 2) return SplitPlan();
+SplitPlan plan_key_split(int form, int T, int n_seq, int Hq, int Hkv, int D, int causal) {
+  if (form == 1 || form == 2) return SplitPlan();
   const int keys = attn_keyside_keys(D);
   const long long wgs = (long long)((T + keys - 1) / keys) * Hkv;
   const double chain = (double)T / n_seq / 32 * (Hq / Hkv) / 4;                // items of one of the four wavefronts
@@ -176,7 +172,7 @@ size_t fgrpo_varlen_attn_workspace(int T, int n_seq, int Hq, int Hkv, int D, int
   if (T <= 0 || n_seq <= 0 || Hq <= 0 || Hkv <= 0 || Hq % Hkv != 0 || (D != 128 && D != 64)) return 0;
   const Tuning tn = g_tune;
   const size_t q = query_split_bytes(plan_query_split(tn, tn.attn_qside, T, n_seq, Hq, Hkv, D, causal, !backward), T, Hq, D, !backward);
-  return backward ? q + key_split_bytes(plan_key_split(tn, T, n_seq, Hq, Hkv, D, causal), T, Hkv, D) : q;
+  return backward ? q + key_split_bytes(plan_key_split(tn.attn_dkv, T, n_seq, Hq, Hkv, D, causal), T, Hkv, D) : q;
 }
 
 int fgrpo_varlen_attn_fwd(const void* q, const void* k, const void* v, long long q_st, long long q_sh, long long k_st,
@@ -205,7 +201,7 @@ int fgrpo_varlen_attn_fwd_ws(const void* q, const void* k, const void* v, long l
     if (rc) return rc;
   }
   const Tuning tn = g_tune;   // one reading of the tuning state per call: the kernel launched is the one the split was planned for
-  const int form = query_side_form(tn, q_st, Hq, D), hb = attn_heads_per_group(tn, Hq / Hkv, T, n_seq);
+  const int form = attn_query_form(tn.attn_qside, q_st, k_st, v_st, Hq, D), hb = attn_heads_per_group(tn, Hq / Hkv, T, n_seq);
   SplitPlan sp = plan_query_split(tn, form, T, n_seq, Hq, Hkv, D, causal, true);
   const size_t need = query_split_bytes(sp, T, Hq, D, true);
   if (!ws || need == 0) sp = SplitPlan();
@@ -256,27 +252,26 @@ int fgrpo_varlen_attn_bwd_ws(const void* dout, const void* q, const void* k, con
     if (rc) return rc;
   }
   const Tuning tn = g_tune;   // one reading of the tuning state per call: the kernel launched is the one the split was planned for
-  const int form = query_side_form(tn, q_st, Hq, D), hb = attn_heads_per_group(tn, Hq / Hkv, T, n_seq);
-  SplitPlan sq = plan_query_split(tn, form, T, n_seq, Hq, Hkv, D, causal, false), sk = plan_key_split(tn, T, n_seq, Hq, Hkv, D, causal);
+  const int form = attn_query_form(tn.attn_qside, q_st, k_st, v_st, Hq, D), hb = attn_heads_per_group(tn, Hq / Hkv, T, n_seq);
+  const int key_form = attn_key_form(tn.attn_dkv, q_st, k_st, v_st, T, Hq, Hkv, D, attn_keyside_keys(D));
+  SplitPlan sq = plan_query_split(tn, form, T, n_seq, Hq, Hkv, D, causal, false), sk = plan_key_split(key_form, T, n_seq, Hq, Hkv, D, causal);
   const size_t need_q = query_split_bytes(sq, T, Hq, D, false), need = need_q + key_split_bytes(sk, T, Hkv, D);
   if (!ws || need == 0) sq = sk = SplitPlan();
   else if (ws_bytes < need) return fail(FGRPO_ERR_WORKSPACE, "varlen_attn_bwd: workspace %zu < %zu", ws_bytes, need);
   else if (!aligned16(ws)) return fail(FGRPO_ERR_ALIGN, "varlen_attn_bwd: workspace must be 16-byte aligned");
-  // the scalar offsets of the third form are 32-bit: (queries x heads of a group) x 4 bytes and the two bounds arrays
-  const bool dkv3 = tn.attn_dkv != 1 && tn.attn_dkv != 2 && (long long)T * (Hq / Hkv) * 4 < (1LL << 31) && (long long)T * 8 < (1LL << 31);
-  if (!dkv3) sq = sk = SplitPlan();
+  if (key_form != 3) sq = sk = SplitPlan();
   p.parts_q = sq.parts, p.per_q = sq.per, p.parts_k = sk.parts, p.per_k = sk.per;
   p.part_q = (float*)ws;
   p.part_k = (float*)((char*)ws + need_q);
   rc = launch_query_side<DqLauncher>(form, D, hb, p, T, Hq, Hkv, bounds_ws, st);
   if (rc) return rc;
-  if (dkv3) {
+  if (key_form == 3) {
     rc = launch_attn_dkv3(D, p, st);
     if (rc || (sq.parts <= 1 && sk.parts <= 1)) return rc;
     return launch_attn_merge_bwd(D, p, 128 / hb, st);
   }
   const dim3 grid_k(Hkv, (T + kAttnBQ - 1) / kAttnBQ);
-  if (tn.attn_dkv == 1) {
+  if (key_form == 1) {
     if (D == 128) hipLaunchKernelGGL(varlen_attn_dkv_kernel<128>, grid_k, dim3(256), 0, st, p);
     else hipLaunchKernelGGL(varlen_attn_dkv_kernel<64>, grid_k, dim3(256), 0, st, p);
   } else if (D == 128) {

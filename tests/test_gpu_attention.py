@@ -80,6 +80,39 @@ def test_forward_of_query_rows_far_apart(dev, stride, Hq, D):
         assert torch.equal(a, b), name
 
 
+@pytest.mark.parametrize("which", ["q", "k", "v", "qk", "qkv"])
+@pytest.mark.parametrize("rows,past", [(64, 0), (64, 8), (32, 0), (32, 8)])
+@pytest.mark.parametrize("D", [64, 128])
+def test_rows_far_apart_forward_and_backward(dev, which, rows, past, D):
+    """Token strides at which 32 or 64 rows are the last that 32-bit offsets reach, and the next: the results of packed rows,
+    which other tests hold against the oracle.  The kernels may differ, so two roundings to bf16 (probabilities, result)
+    of 2^-9 at most on either side: 2^-7 of the norm between them.  What lies between the rows is NaN."""
+    from fgrpo import ops
+    T, Hq, Hkv = 70, 4, 2
+    stride = (2 ** 32 - 1 - 2 * D) // (2 * (rows - 1)) // 8 * 8 + past
+    q, k, v, do = (x.to(dev) for x in make(T, Hq, Hkv, seed=rows + past, D=D))
+    cu = torch.tensor([0, 33, T], dtype=torch.int32, device=dev)
+
+    def far(x):
+        buf = torch.full(((T - 1) * stride + x[0].numel(),), float("nan"), dtype=torch.bfloat16, device=dev)
+        view = buf.as_strided(x.shape, (stride, D, 1))
+        view.copy_(x)
+        return view
+    print(f"[rows far apart] {which} stride={stride} D={D}", flush=True)
+
+    def results(*operands):
+        a = [x.requires_grad_(True) for x in operands]
+        out = ops.varlen_attention(*a, cu, None, True)
+        return (out.detach(),) + torch.autograd.grad(out, a, do)
+    want = results(q, k, v)
+    got = results(*(far(x.detach()) if name in which else x for name, x in zip("qkv", (q, k, v))))
+    torch.cuda.synchronize()
+    for name, a, b in zip(("out", "dq", "dk", "dv"), got, want):
+        assert (a.float() - b.float()).norm() <= 2 ** -7 * b.float().norm(), name
+    del got
+    torch.cuda.empty_cache()
+
+
 @pytest.mark.parametrize("causal", [True, False])
 def test_small_segments_share_a_tile(dev, causal):
     check(dev, "short segments", 200, [0, 5, 6, 70, 71, 72, 200], 4, 2, causal, seed=1)

@@ -269,3 +269,67 @@ def test_packed_lists_of_several_samples_follow_each_other():
     assert dst.tolist() == [1, 2, -100, -100, 3, 4, 5, 6, 7]
     with pytest.raises(ValueError):
         _fill(dst, [{"x": [1, 2]}], "x", [3])
+
+
+@pytest.fixture(scope="module")
+def attn_route(tmp_path_factory):
+    """csrc/attn_route.h, which is plain C++, behind three C functions."""
+    import ctypes as C
+    import os
+    import subprocess
+    where = tmp_path_factory.mktemp("attn_route")
+    src, lib = str(where / "route.cpp"), str(where / "route.so")
+    with open(src, "w") as f:
+        f.write('#include "attn_route.h"\nextern "C" {\nusing ll = long long;\n'
+                "int reach(ll st, int rows, int D) { return fgrpo::attn_rows_in_reach(st, rows, D); }\n"
+                "int query(int w, ll q, ll k, ll v, int Hq, int D) { return fgrpo::attn_query_form(w, q, k, v, Hq, D); }\n"
+                "int key(int w, ll q, ll k, ll v, int T, int Hq, int Hkv, int D, int keys) {"
+                " return fgrpo::attn_key_form(w, q, k, v, T, Hq, Hkv, D, keys); }\n}\n")
+    csrc = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "async-grpo-nccl_amd", "csrc")
+    subprocess.run([os.environ.get("CXX", "g++"), "-std=c++17", "-O1", "-fPIC", "-shared", f"-I{csrc}", src, "-o", lib], check=True)
+    lib = C.CDLL(lib)
+    lib.reach.argtypes = [C.c_longlong, C.c_int, C.c_int]
+    lib.query.argtypes = [C.c_int] + [C.c_longlong] * 3 + [C.c_int] * 2
+    lib.key.argtypes = [C.c_int] + [C.c_longlong] * 3 + [C.c_int] * 5
+    return lib
+
+
+def _last_stride(rows, D):
+    """Largest multiple of eight elements at which the last byte of `rows` rows is within 32-bit offsets of the first row."""
+    st = (2 ** 32) // (2 * (rows - 1)) // 8 * 8
+    while (rows - 1) * st * 2 + 2 * D > 2 ** 32 - 1:
+        st -= 8
+    return st
+
+
+@pytest.mark.parametrize("rows", [32, 64])
+@pytest.mark.parametrize("D", [64, 128])
+def test_attention_rows_are_in_reach_up_to_the_last_byte(attn_route, rows, D):
+    last = _last_stride(rows, D)
+    for st in (8, 3584, last - 8, last):
+        assert attn_route.reach(st, rows, D) and (rows - 1) * st * 2 + 2 * D < 2 ** 32
+    for st in (last + 8, 2 * last, 2 ** 40, 2 ** 62):
+        assert not attn_route.reach(st, rows, D) and (rows - 1) * st * 2 + 2 * D >= 2 ** 32
+
+
+@pytest.mark.parametrize("D,keys", [(64, 32), (128, 64)])
+def test_attention_rows_out_of_reach_take_the_64_bit_kernels(attn_route, D, keys):
+    """Each stride by itself on both sides of each kernel's reach: 32 rows of Q, 64 of K and V for the query side; 32 of Q and
+    `keys` of K and V, or 64 of Q, for dK/dV."""
+    row, at32, at64 = 2 * D, _last_stride(32, D), _last_stride(64, D)
+    for wanted in (0, 1, 2, 3):
+        form = lambda q=row, k=row, v=row, Hq=4: attn_route.query(wanted, q, k, v, Hq, D)
+        for near in (dict(), dict(q=at64 + 8), dict(q=at32), dict(k=at64), dict(v=at64), dict(Hq=at32 // D)):
+            assert form(**near) == wanted, near
+        for far in (dict(q=at32 + 8), dict(k=at64 + 8), dict(v=at64 + 8), dict(k=2 ** 50), dict(Hq=at32 // D + 1)):
+            assert form(**far) == 1, far
+    at = _last_stride(keys, D)
+    form = lambda w=0, q=row, k=row, v=row, T=1000, Hq=4, Hkv=2: attn_route.key(w, q, k, v, T, Hq, Hkv, D, keys)
+    for near in (dict(), dict(q=at32), dict(k=at), dict(v=at), dict(w=3)):
+        assert form(**near) == 3, near
+    for mid in (dict(k=at + 8), dict(v=at + 8), dict(k=2 ** 50, q=at64), dict(w=2), dict(w=2, k=2 ** 40, q=at64),
+                dict(T=2 ** 28), dict(T=2 ** 28 - 1, Hq=8, Hkv=1)):
+        assert form(**mid) == 2, mid
+    for far in (dict(q=at32 + 8), dict(k=at + 8, q=at64 + 8), dict(w=2, q=at64 + 8), dict(w=1), dict(w=2, T=2 ** 28, q=at32 + 8),
+                dict(Hq=at32 // D + 1, Hkv=1)):
+        assert form(**far) == 1, far
