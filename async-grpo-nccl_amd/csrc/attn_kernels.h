@@ -1343,18 +1343,6 @@ __device__ __forceinline__ uint32_t attn_dma_lane_offset(int wave, int lane, lon
   const int row = wave * RPI + lane / (HD / 8), ch = (lane % (HD / 8)) ^ attn_swz<HD>(row);
   return (uint32_t)(((long long)row * st + ch * 8) * 2);
 }
-template <int HD>
-__device__ __forceinline__ void attn_dma_tile(const bf16_t* base, long long st, int row0, int row_end, uint32_t lane_off,
-                                              char* tile_w /* tile + wave * 1024 */) {
-  constexpr int RPI = 1024 / (HD * 2), NLD = kAttnBK / RPI / 4;
-  const long long rows = (long long)row_end - row0;
-  long long bytes = rows > 0 ? (rows - 1) * st * 2 + HD * 2 : 0;
-  if (bytes > 0xffffffffLL) bytes = 0xffffffffLL;
-  const __amdgpu_buffer_rsrc_t rs = make_rsrc(base + (long long)row0 * st, (uint32_t)bytes);
-#pragma unroll
-  for (int i = 0; i < NLD; ++i)
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, FGRPO_LDS_PTR(tile_w + i * 4096), 16, (int)lane_off, (int)(i * 4 * RPI * st * 2), 0, 0);
-}
 
 // The descriptor of the next 64-row tile, kept up to date by additions: the walk goes down the rows 64 at a time,
 // and forming `base + row0 * st` and the byte count from scratch costs four 64-bit multiplications a tile - scalar
@@ -1371,7 +1359,7 @@ struct AttnTileCursor {
     step = (long long)kAttnBK * st * 2;
   }
   __device__ __forceinline__ void next() { ptr += step, bytes -= step; }
-  // loads of the tile at the cursor, by a 256-thread work-group (see attn_dma_tile)
+  // loads of the tile at the cursor, by a 256-thread work-group (see attn_dma_lane_offset)
   __device__ __forceinline__ void load(long long st, uint32_t lane_off, char* tile_w) const {
     constexpr int RPI = 1024 / (HD * 2), NLD = kAttnBK / RPI / 4;
     long long b = bytes > 0 ? bytes : 0;
