@@ -271,6 +271,21 @@ def test_packed_lists_of_several_samples_follow_each_other():
         _fill(dst, [{"x": [1, 2]}], "x", [3])
 
 
+@pytest.mark.parametrize("missing", ["BINDING_PATH", "LIB_PATH"])
+def test_packing_needs_no_extension_module(monkeypatch, tmp_path, missing):
+    """Where the library or the extension module is not built, packing works as before there was one."""
+    from fgrpo import _lib
+    from sample_processing_utils import _fill
+    monkeypatch.setattr(_lib, missing, str(tmp_path / "not_built.so"))
+    monkeypatch.setattr(_lib, "_lib", None)
+    monkeypatch.setattr(_lib, "_native", None)
+    with pytest.raises(RuntimeError, match="fgrpo.build"):
+        _lib.native()
+    dst = np.zeros(8, dtype=np.int64)
+    _fill(dst, [{"x": np.array([1, 2])}, {"x": torch.tensor([3])}, {"x": [4, 5]}, {"x": (6,)}, {}], "x", [2, 1, 2, 1, 2], default=-100)
+    assert dst.tolist() == [1, 2, 3, 4, 5, 6, -100, -100]
+
+
 @pytest.fixture(scope="module")
 def attn_route(tmp_path_factory):
     """csrc/attn_route.h, which is plain C++, behind three C functions."""
