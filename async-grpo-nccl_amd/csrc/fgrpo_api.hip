@@ -1734,23 +1734,19 @@ int fgrpo_grpo_step_chunked(const void* hidden, const void* weight, const void* 
   return 0;
 }
 
-int fgrpo_scale_inplace(void* x, long long n, int dtype, const float* scale_dev, void* stream) {
-  if (!x) return fail(FGRPO_ERR_BAD_ARG, "scale_inplace: bad argument");
-  return fgrpo_scale_gradients(x, n, nullptr, 0, nullptr, 0, dtype, scale_dev, stream);
-}
-
-int fgrpo_scale_gradients(void* dh, long long n_dh, void* dw, long long n_dw, void* db, long long n_db, int dtype,
-                          const float* scale_dev, void* stream) {
+namespace {
+int scale_arrays(const char* who, void* dh, long long n_dh, void* dw, long long n_dw, void* db, long long n_db, int dtype,
+                 const float* scale_dev, void* stream) {
   ScaleParams p;
   memset(&p, 0, sizeof(p));
   void* const x[3] = {dh, dw, db};
   const long long n[3] = {n_dh, n_dw, n_db};
-  if (!scale_dev) return fail(FGRPO_ERR_BAD_ARG, "scale_inplace: bad argument");
-  if (dtype != FGRPO_BF16 && dtype != FGRPO_F32) return fail(FGRPO_ERR_BAD_ARG, "scale_inplace: dtype=%d", dtype);
+  if (!scale_dev) return fail(FGRPO_ERR_BAD_ARG, "%s: bad argument", who);
+  if (dtype != FGRPO_BF16 && dtype != FGRPO_F32) return fail(FGRPO_ERR_BAD_ARG, "%s: dtype=%d", who, dtype);
   int arrays = 0, blocks = 0;
   for (int i = 0; i < 3; ++i) {
-    if (n[i] < 0 || (n[i] > 0 && !x[i])) return fail(FGRPO_ERR_BAD_ARG, "scale_inplace: bad argument");
-    if (x[i] && !aligned16(x[i])) return fail(FGRPO_ERR_ALIGN, "scale_inplace: the array must be 16-byte aligned");
+    if (n[i] < 0 || (n[i] > 0 && !x[i])) return fail(FGRPO_ERR_BAD_ARG, "%s: bad argument", who);
+    if (x[i] && !aligned16(x[i])) return fail(FGRPO_ERR_ALIGN, "%s: the array must be 16-byte aligned", who);
     if (!x[i] || n[i] == 0) continue;
     const long long nb = (n[i] / (dtype == FGRPO_F32 ? 4 : 8) + 255) / 256;
     p.x[arrays] = x[i], p.n[arrays] = n[i], p.first[arrays] = blocks;
@@ -1764,6 +1760,17 @@ int fgrpo_scale_gradients(void* dh, long long n_dh, void* dw, long long n_dw, vo
   hipLaunchKernelGGL(scale_inplace_kernel, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream, p);
   HIP_TRY(hipGetLastError());
   return 0;
+}
+}  // namespace
+
+int fgrpo_scale_inplace(void* x, long long n, int dtype, const float* scale_dev, void* stream) {
+  if (!x) return fail(FGRPO_ERR_BAD_ARG, "scale_inplace: bad argument");
+  return scale_arrays("scale_inplace", x, n, nullptr, 0, nullptr, 0, dtype, scale_dev, stream);
+}
+
+int fgrpo_scale_gradients(void* dh, long long n_dh, void* dw, long long n_dw, void* db, long long n_db, int dtype,
+                          const float* scale_dev, void* stream) {
+  return scale_arrays("scale_gradients", dh, n_dh, dw, n_dw, db, n_db, dtype, scale_dev, stream);
 }
 
 int fgrpo_metrics(const int64_t* idx, int n, int T, const float* log_ratio, const float* entropy,

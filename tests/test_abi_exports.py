@@ -65,6 +65,18 @@ def test_argument_errors_are_reported_without_a_gpu(lib_path):
     assert lib.fgrpo_get_tuning(b"panel_cols") >= 0
 
 
+def test_scaling_errors_name_the_entry_point(lib_path):
+    from fgrpo import _lib
+    lib = _lib.load()
+    at, odd = 4096, 4098                       # refused before they are looked at
+    for args, rc in (((at, 8, at, 8, at, 8, 0, None, None), -1), ((at, 8, at, 8, at, 8, 7, at, None), -1), ((None, 8, at, 8, at, 8, 0, at, None), -1),
+                     ((at, 8, at, -1, at, 8, 0, at, None), -1), ((at, 8, at, 8, odd, 8, 0, at, None), None)):
+        got = lib.fgrpo_scale_gradients(*args)
+        assert got < 0 and rc in (None, got) and lib.fgrpo_last_error().startswith(b"scale_gradients: "), args
+    for args in ((None, 8, 0, at, None), (at, -1, 0, at, None), (at, 8, 7, at, None), (odd, 8, 0, at, None), (at, 8, 0, None, None)):
+        assert lib.fgrpo_scale_inplace(*args) < 0 and lib.fgrpo_last_error().startswith(b"scale_inplace: "), args
+
+
 def test_backward_panel_plan_respects_the_bound(lib_path):
     """The dLogits panel of the backward: a multiple of 256 columns, never above the caller's bound (rounded up to
     one 256-column block), at most three panels more than the bound alone would need, and by default at most a
