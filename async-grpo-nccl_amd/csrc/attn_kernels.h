@@ -1229,8 +1229,8 @@ __global__ __launch_bounds__(512) void varlen_attn_dkv2_kernel(AttnParams p) {
 //    another, and rows are moved as they lie in memory (AttnRows).  Row loads, first tiles and delta of dQ took 7.5 us of
 //    a work-group's 26.5 at segments of 128..1024 tokens with 12 / 2 heads of 128, of the forward's 20.5 2.5; now 5.5 of
 //    23.3 (Q, dO and O come from HBM, 96 KiB a work-group: bandwidth) and 1.9 of 19.1.  Forward + backward of that
-//    batch, dK/dV's opening included: 540 -> 498 us; 12345 tokens with 14 / 2 heads of 64: 140 -> 132; one sample of
-//    777 tokens, forward: 25.9 -> 24.9; 4 x 8192 tokens with 28 / 4 heads: 8.00 -> 7.91 ms.
+//    batch, dK/dV's opening included: 540 -> 498..505 us; 12345 tokens with 14 / 2 heads of 64: 140 -> 133; one sample of
+//    777 tokens, forward: 26.0 -> 24.9; 4 x 8192 tokens with 28 / 4 heads: 8.00 -> 7.91..8.00 ms.
 // Every value an asm read delivers passes through attn_settle() right after its wait (see varlen_attn_dkv2_kernel).
 // ---------------------------------------------------------------------------------------------------------
 struct AttnTr {

@@ -214,9 +214,15 @@ int choose_nsplit(int tiles_t, int tiles_v, int slots, int forced, int prefer = 
   if (forced > 0) return forced < tiles_v ? forced : tiles_v;
   int best = 1;
   long long best_cost = -1;
-  // One to three token tiles take as many splits as one round of the device holds: at 64 they left up to three quarters of
-  // it idle (kept forward, H = 1536, V = 151936: 200 tokens 440 -> 161 us, 500 451 -> 247, 700 461 -> 340).  More token
-  // tiles keep the cap: beyond one round a split only adds openings.
+  // Token tiles that 64 splits do not make a round of the device of (under slots / 64: three tiles of 256, seven of the
+  // 128-wide configuration, whose work-groups share a CU) take as many splits as one round holds; at 64 they left up to three
+  // quarters of it idle (kept forward, H = 1536, V = 151936: 200 tokens 440 -> 161 us, 500 451 -> 247, 700 461 -> 340).  More
+  // token tiles keep the cap: beyond one round a split only adds openings.  The same for both kernels and both tiles: 128-wide
+  // tiles, H = 4096, V = 32000, plain forward of 100 tokens 180 -> 66 us, of 200 183 -> 85, and at H <= 512, V <= 12000 no
+  // difference (22 us, the launches); recomputing backward, whose dLogits kernel it splits: H = 1536, V = 151936, 200 tokens
+  // 3201 -> 2895, 700 3521 -> 3268; H = 8192, V = 128256, 500 6519 -> 6036; 128-wide, H = 4096, V = 32000, 200 tokens 1036 ->
+  // 872, fp32 1520 -> 1066; H = 64, V = 9000, 300 131 -> 128.  dLogits' raster group does not matter there (eight or six deep
+  // within 0.5 %).
   if (max_split * tiles_t < slots) max_split = slots / tiles_t;
   const int cap = tiles_v < max_split ? tiles_v : max_split;
   auto cost_of = [&](int s) { return split_cost(tiles_t, tiles_v, slots, s); };
@@ -1091,7 +1097,8 @@ DhSplitPlan plan_tail_split(int T, int H, int kv, double* rounds_out = nullptr) 
     const int tail = (tiles_m - main_tiles) * tiles_n;
     if (tail <= 0) continue;
     // more than sixteen pieces where one round holds them (under sixteen tiles): dHidden of 200 tokens at H = 1536, V = 151936,
-    // six tiles, 240 -> 142 us with 42 pieces, their sum included
+    // six tiles, 231 us in 16 pieces and 6 for their sum -> 118 in 38 and 21.  Each
+    // division has to beat the best so far by 5 %, so the next finer one, 40 pieces, is not taken.
     for (int ks = 2; (ks <= 16 && tail * ks <= kDhPartRounds * slots) || tail * ks <= slots; ++ks) {
       const int per = (blocks + ks - 1) / ks;
       if (per < 8) break;                                      // pieces under 32 K steps are not worth their tile store

@@ -875,7 +875,8 @@ __global__ __launch_bounds__(C::NT, C::OCC) void gemm_store_kernel(const StorePa
 // to p[0], the others to p[1].  Piece ks of a product takes the same K range of every segment (all operands K-contiguous)
 // and leaves its fp32 tile in slice ks.  Neither product fills the device: side by side they take the time of the
 // longer one, and their sums one launch (fp32, 643 tokens x 1000 entries x 64: 9 + 9 us and 4 + 4 for the sums one behind
-// the other; the whole step with the launch of tail_kernels.h's segment weights 148.5 -> 138.4 us, one box, sides in turn).
+// the other, 10 and 4 now).  The whole step is bound by its host path: four interleavings on two boxes, with tail_kernels.h's
+// segment weights in one launch as well, gave 131..148 us before and 131..139 after, where runs of one side differ by 10 % or more.
 struct SmallSplitPair {
   StoreParams p[2];
   int first;

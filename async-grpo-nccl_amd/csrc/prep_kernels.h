@@ -75,9 +75,9 @@ __global__ __launch_bounds__(256) void lmhead_fwd_combine_kernel(const CombinePa
   }
 }
 
-// Few splits mean many tokens: one thread each.  Small token counts are split up to 128 ways so that the forward
-// fills the device, and one thread then walks that many loads in sequence (777 tokens, 60 splits: 20.6 us; with 16
-// threads a token 5; 4 splits of 8192 tokens take 5 us either way).
+// Few splits mean many tokens: one thread each.  Small token counts are split as often as fills the device (slots / token
+// tiles: 256 ways for one tile of 256 tokens), and one thread would walk that many loads in sequence (777 tokens, 60 splits:
+// 20.6 us); sixteen threads a token walk up to sixteen each (5 us; 4 splits of 8192 tokens take 5 us either way).
 // The objective rides along where its normaliser is known beforehand: a launch less per token chunk (4.8 us each between
 // kernels that wait for one another).
 template <bool LOSS>

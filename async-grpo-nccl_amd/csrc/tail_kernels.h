@@ -53,7 +53,7 @@ __device__ __forceinline__ bool in_a_segment(const int* cu, int nseq, int t) {
 // Work-groups past the segments' write the zeros: a token no range covers lies below every boundary, at or above all
 // of them, or - in a vector that runs backwards - between its last boundary and its first, where the ranges are walked (a
 // stretch that rises again there has its weight from its own wavefront).  One launch instead of a
-// fill in front of the segments: a step of 643 tokens is bound by its launches (figures at gemm_small_split_kernel).
+// fill in front of the segments (a small step's figures are at gemm_small_split_kernel).
 constexpr int kSegmentsPerGroup = 4, kZeroTokensPerGroup = 4096;
 __global__ __launch_bounds__(64 * kSegmentsPerGroup) void segment_valid_weight_kernel(const long long* labels, const int* cu,
                                                                                       int nseq, int T, int* cnt, float* tokw) {

@@ -192,8 +192,9 @@ int fgrpo_loss_fwd(const float* lp, const float* old_lp, const float* ref_lp, co
  * token's sample) and seg_cnt_out [nseq] for FGRPO_AGG_SAMPLE_MEAN (both may be NULL for TOKEN_MEAN), pre_out [4]
  * doubles = {normaliser, valid tokens, non-empty samples, 1 / normaliser rounded to fp32} - and
  * g_t = d loss / d lp_t is final as soon as lp_t is.  The gradients are those of the loss itself (upstream gradient
- * 1); a caller whose autograd later delivers another upstream scalar multiplies them with fgrpo_scale_inplace
- * (x[i] *= *scale_dev for n elements of `dtype`; a scale of exactly 1 returns without touching the array).
+ * 1); a caller whose autograd later delivers another upstream scalar multiplies them with fgrpo_scale_gradients, all
+ * in one launch, or one array at a time with fgrpo_scale_inplace (x[i] *= *scale_dev for n elements of `dtype`; a scale
+ * of exactly 1 returns without touching the arrays).
  * Executed matrix work: 6 T H V (the reference's own three products), against 8 T H V for the recomputing pair;
  * transient: fgrpo_logits_keep_bytes(chunk, V) + the fp32 dW sum (V x H x 4 bytes, only with more than one chunk).
  * chunk_tokens <= 0: 8192.  No chunk exceeds the bound (rounded down to whole 256-token tiles); under it the tokens
