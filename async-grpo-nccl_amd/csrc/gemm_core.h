@@ -89,7 +89,9 @@ struct TileCfg {
   static constexpr int ROWB = DMA ? BK * 2 : BK * 2 + 16;  // LDS row bytes (register path pads, DMA path swizzles)
   static constexpr int STAGE = (BM + BN) * ROWB;
   static constexpr int NSTAGE = NST_;
-  static constexpr int LDS_BYTES = STAGE * NSTAGE;
+  static constexpr bool MI16 = DMA && NST_ == 2 && NW == 8 && BK == 64 && TM == 4 && TN == 2;   // see kMi16
+  // the 16x16x32 schedule keeps a third buffer for operand A (early_barrier_pipeline16)
+  static constexpr int LDS_BYTES = STAGE * NSTAGE + (MI16 ? BM * ROWB : 0);
   static_assert(BM % (WM * 32) == 0 && BN % (WN * 32) == 0, "tile/wave shape");
   static_assert(BK % 16 == 0 && NT % CPR == 0 && BM % RPP == 0 && BN % RPP == 0, "loader shape");
   static_assert(!DMA || (CPR == 4 || CPR == 8), "DMA path supports BK = 32 or 64");
@@ -117,7 +119,7 @@ __device__ __forceinline__ int acc_col(int wn, int j, int lane) {
 //                                   col = wn*WTN + j*32 + 16*ch + (lane%16)
 // relative to the tile origin.
 template <class C>
-constexpr bool kMi16 = C::DMA && C::NSTAGE == 2 && C::NW == 8 && C::BK == 64 && C::TM == 4 && C::TN == 2;
+constexpr bool kMi16 = C::MI16;
 template <class C>
 __device__ __forceinline__ int acc16_row(int wm, int i, int e, int lane) {
   return wm * C::WTM + i * 32 + 16 * (e >> 3) + 4 * (lane >> 4) + (e & 3);
@@ -485,14 +487,35 @@ __device__ __forceinline__ void early_barrier_pipeline(int nk_total, char* smem,
 // b(j, ch) (16 columns x 32 k) of the slice.  The b fragments of a slice are fetched once, before its first
 // sub-step, and serve both; so the fragment requests alternate between 4 (a only, before an odd sub-step) and
 // 8 (a0, the four b, a1 .. a3, before an even one).
-//   load_a(stage_ptr, I, KK): fragment a(I, KK % 2) of slice KK / 2;  load_b(stage_ptr, JC, K2): fragment b(JC/2, JC%2).
-template <class C, int LPT, int RA, int RB, class IssueOne, class LoadA, class LoadB>
+// Operand A (the streamed one in every use: W in the LM-head kernels, the [T x V] buffer in the gradient products) has
+// three LDS buffers and operand B two.  AHEAD: A is requested almost two K steps before it is needed,
+//   B of step kt + 1 behind the barrier of step kt - 1 (its buffer was freed there), A of step kt + 2 in the next sub-step,
+// and the barrier of step kt waits for all but that youngest A.  With one step of lead for both, as it was, a request that
+// missed the L2 was waited for in every step.  But such waits also keep the work-groups of an XCD together: the first to
+// ask for a slice waits, those behind it find it in the L2.  With the longer lead nothing held them (forward of 40000
+// tokens, H = 5120: past the L2s 36.7 -> 71.8 GB, 6 % fewer cycles at a lower clock, 35.6 -> 36.9 ms); so every
+// kStrictEvery-th step waits for the youngest A as well (33.9 ms; every second step 34.0, every eighth 34.9).  !AHEAD: the
+// one step of lead, for long contractions in many device rounds (dHidden, launch_store_splitk), where the drift adds up
+// from round to round.  Before -> after, one box each: forward that keeps the numerators, T = 8192, H = 1536: 3.28 -> 3.09 ms, H =
+// 3584, T = 16384: 13.14 -> 12.78; dW of 8192 tokens, H = 1536: 3.04 -> 2.98; dHidden of 777 tokens 0.409 -> 0.388.
+//   issue_a(lds, idx) / issue_b(lds, idx): load idx of the next K step of that operand into the buffer at `lds`; the
+//   last one of A (the first one of B, but for step 0's) advances the operand's cursor;
+//   load_a(lds, I, KK): fragment a(I, KK % 2) of slice KK / 2;  load_b(lds, JC, K2): fragment b(JC/2, JC%2).
+// On entry B of step 0 and A of steps 0 and 1 have been issued, in this order (as far as they exist).  DRAIN: wait for
+// all of it (the caller has issued something else since), not just for step 0.
+constexpr int kStrictEvery = 4;                      // a power of two
+template <class C>
+constexpr int kOpBytes = C::BM * C::ROWB;            // one buffer of one operand (32 KiB)
+__device__ __forceinline__ constexpr int mi16_a_buf(int step) { return step % 3; }          // in kOpBytes
+__device__ __forceinline__ constexpr int mi16_b_buf(int step) { return 4 - (step & 1); }    // buffers 2 and 3 are free between tiles
+template <class C, int RA, int RB, bool DRAIN, bool AHEAD, class IssueA, class IssueB, class LoadA, class LoadB>
 __device__ __forceinline__ void early_barrier_pipeline16(int nk_total, char* smem, f32x16_t (&acc)[C::TM][C::TN],
-                                                         bool live, IssueOne&& issue_one, LoadA&& load_a, LoadB&& load_b) {
+                                                         bool live, IssueA&& issue_a, IssueB&& issue_b, LoadA&& load_a,
+                                                         LoadB&& load_b) {
   constexpr int KK = 4;
   constexpr int TM = C::TM, NB = 2 * C::TN;           // a fragments per sub-step, b fragments per K slice
-  static_assert(kMi16<C> && C::BK == 64, "16x16x32 schedule: 8-wavefront 256x256x64 tile");
-  constexpr int NSLOT = kLoadPhases * TM;
+  constexpr int PA = C::PA, PB = C::PB, OP = kOpBytes<C>;
+  static_assert(kMi16<C> && C::BK == 64 && PA == TM && PB == TM, "16x16x32 schedule: 8-wavefront 256x256x64 tile, one load per row group");
   // request list of a sub-step by its parity P (0: a0, b0 .. b(NB-1), a1 ..; 1: a0 .. a(TM-1)), all compile time
   struct Ord {
     static constexpr int nr(int P) { return P == 0 ? TM + NB : TM; }
@@ -509,66 +532,73 @@ __device__ __forceinline__ void early_barrier_pipeline16(int nk_total, char* sme
       return instrs(P, nr(P)) - instrs(P, need(P, i) + 1) + (issuing ? instrs(1 - P, cum(1 - P, i)) : 0);
     }
   };
-  FGRPO_WAIT_VMCNT(0);
-  wg_barrier();                                       // step 0 is in buffer 0
-  if (!live) {
+  if (DRAIN || nk_total < 2) FGRPO_WAIT_VMCNT(0);
+  else FGRPO_WAIT_VMCNT(PA);
+  wg_barrier();                                       // step 0 is in LDS
+  if (AHEAD && nk_total > 1) static_for<PB>([&](auto q) { issue_b(smem + mi16_b_buf(1) * OP, decltype(q)::value); });
+  char *a0 = smem, *a1 = smem + OP, *a2 = smem + 2 * OP;                                    // A of steps kt, kt + 1, kt + 2
+  char *b0 = smem + mi16_b_buf(0) * OP, *b1 = smem + mi16_b_buf(1) * OP;                    // B of steps kt, kt + 1
+  auto rotate = [&]() {
+    char* t = a0;
+    a0 = a1, a1 = a2, a2 = t;
+    t = b0;
+    b0 = b1, b1 = t;
+  };
+  if (!live || nk_total <= 0) {
     // a sub-tile outside the matrix: this wavefront's share of the loads and every barrier, nothing else
-    for (int kt = 1; kt < nk_total; ++kt) {
-      static_for<LPT>([&](auto q) { issue_one(kt & 1, decltype(q)::value); });
+    for (int kt = 0; kt + 1 < nk_total; ++kt) {
+      const bool more = kt + 2 < nk_total;
+      if constexpr (AHEAD) {
+        if (more) static_for<PA>([&](auto q) { issue_a(a2, decltype(q)::value); });
+      } else {
+        static_for<PB>([&](auto q) { issue_b(b1, decltype(q)::value); });
+      }
       FGRPO_WAIT_VMCNT(0);
-      wg_barrier();                                   // the one inside step kt - 1: step kt is in LDS, the other buffer is free
+      wg_barrier();                                   // the one inside step kt: step kt + 1 is in LDS, the buffers of step kt are free
+      if (more) {
+        if constexpr (AHEAD) static_for<PB>([&](auto q) { issue_b(b0, decltype(q)::value); });
+        else static_for<PA>([&](auto q) { issue_a(a2, decltype(q)::value); });
+      }
+      rotate();
     }
     wg_barrier();
     return;
   }
-  int steps_issued = nk_total > 0 ? 1 : 0;
-  bool active = steps_issued < nk_total;              // a step is being loaded
-  int tgt = 1;                                        // ... into this buffer
-  if (active) {
-    ++steps_issued;
-    static_for<LPT>([&](auto q) {
-      if constexpr (decltype(q)::value * NSLOT / LPT < TM) issue_one(1, decltype(q)::value);  // phase 0's share
-    });
-  }
   bf16x8_t af[2][TM], bfr[2][NB];
-  // entry e of the request list of sub-step KN, read from the buffer at `base`
-  auto request = [&](const char* base, auto ec, auto knc) {
+  // entry e of the request list of sub-step KN, read from the buffers at `ba` and `bb`
+  auto request = [&](const char* ba, const char* bb, auto ec, auto knc) {
     constexpr int e = decltype(ec)::value, kn = decltype(knc)::value;
     if constexpr ((kn & 1) == 1) {
-      af[1][e] = load_a(base, ec, knc);
+      af[1][e] = load_a(ba, ec, knc);
     } else if constexpr (e == 0) {
-      af[0][0] = load_a(base, std::integral_constant<int, 0>{}, knc);
+      af[0][0] = load_a(ba, std::integral_constant<int, 0>{}, knc);
     } else if constexpr (e <= NB) {
-      bfr[(kn >> 1) & 1][e - 1] = load_b(base, std::integral_constant<int, e - 1>{}, std::integral_constant<int, (kn >> 1)>{});
+      bfr[(kn >> 1) & 1][e - 1] = load_b(bb, std::integral_constant<int, e - 1>{}, std::integral_constant<int, (kn >> 1)>{});
     } else {
-      af[0][e - NB] = load_a(base, std::integral_constant<int, e - NB>{}, knc);
+      af[0][e - NB] = load_a(ba, std::integral_constant<int, e - NB>{}, knc);
     }
   };
-  static_for<Ord::nr(0)>([&](auto e) { request(smem, e, std::integral_constant<int, 0>{}); });
-  int cur = 0;
+  static_for<Ord::nr(0)>([&](auto e) { request(a0, b0, e, std::integral_constant<int, 0>{}); });
+  // One K step.  STEADY: at least two more steps follow; the body then carries no conditionals at all.
   auto step = [&](int kt, auto steady_c) {
     constexpr bool STEADY = decltype(steady_c)::value;
-    const char* st = smem + cur * C::STAGE;
-    const char* sn = smem + (cur ^ 1) * C::STAGE;
+    constexpr bool more = STEADY;                     // step kt + 2 is loaded during this one
     const bool next = STEADY || kt + 1 < nk_total;
     static_for<KK>([&](auto kkc) {
       constexpr int kk = decltype(kkc)::value;
       constexpr bool last = (kk == KK - 1);
       constexpr int kn = last ? 0 : kk + 1;
       constexpr int P = kk & 1, k2 = kk >> 1;
-      const char* src = last ? sn : st;
+      const char *src_a = last ? a1 : a0, *src_b = last ? b1 : b0;
       const bool issuing = STEADY || !last || next;
       if constexpr (last) {
         if (next) {
-          FGRPO_WAIT_VMCNT_LGKM0(0);                  // my loads of step kt+1 landed; my reads of `cur` returned
-          wg_barrier();
-          active = STEADY || steps_issued < nk_total; // loads of step kt+2 go into the buffer just freed
-          tgt = cur;
-          if (active) ++steps_issued;
+          // my loads of step kt + 1 landed (of step kt + 2 the A loads may be in flight); my reads of step kt returned
+          if (!AHEAD || !more || (kt & (kStrictEvery - 1)) == 0) FGRPO_WAIT_VMCNT_LGKM0(0);
+          else FGRPO_WAIT_VMCNT_LGKM0(PA);
+          wg_barrier();                               // the buffers of step kt are free
         }
       }
-      constexpr int phase = last ? 0 : kk + 1;
-      const bool loads_here = STEADY || (active && phase < kLoadPhases && (phase > 0 || next));
       __builtin_amdgcn_sched_barrier(0);
       static_for<TM>([&](auto ic) {
         constexpr int i = decltype(ic)::value;
@@ -579,11 +609,10 @@ __device__ __forceinline__ void early_barrier_pipeline16(int nk_total, char* sme
         }
         __builtin_amdgcn_sched_barrier(0);
         {
+          // the row group's load: one operand's in the first sub-step, the other's behind the barrier
+          constexpr bool load_here = kk == 0 || last;
           constexpr int R = Ord::cum(1 - P, i + 1) - Ord::cum(1 - P, i);
-          constexpr int slot = phase * TM + i;
-          constexpr int q_lo = (phase < kLoadPhases) ? (slot * LPT + NSLOT - 1) / NSLOT : 0;
-          constexpr int q_hi = (phase < kLoadPhases) ? ((slot + 1) * LPT + NSLOT - 1) / NSLOT : 0;   // loads q_lo .. q_hi-1
-          constexpr int X = R + (q_hi - q_lo);
+          constexpr int X = R + (load_here ? 1 : 0);
           static_for<NB>([&](auto jcc) {
             constexpr int jc = decltype(jcc)::value;       // b fragment (j, ch) = (jc / 2, jc % 2)
             mfma16_slice<2 * P + (jc & 1)>(af[P][i], bfr[k2 & 1][jc], acc[i][jc >> 1]);
@@ -591,9 +620,12 @@ __device__ __forceinline__ void early_barrier_pipeline16(int nk_total, char* sme
               constexpr int x = decltype(xc)::value;
               if constexpr (x * NB / (X > 0 ? X : 1) == jc) {
                 if constexpr (x < R) {
-                  if (issuing) request(src, std::integral_constant<int, Ord::cum(1 - P, i) + x>{}, std::integral_constant<int, kn>{});
-                } else {
-                  if (loads_here) issue_one(tgt, q_lo + (x - R));
+                  if (issuing) request(src_a, src_b, std::integral_constant<int, Ord::cum(1 - P, i) + x>{}, std::integral_constant<int, kn>{});
+                } else if constexpr (!AHEAD && !last) {
+                  if (next) issue_b(b1, i);
+                } else if constexpr (more) {
+                  if constexpr (AHEAD && last) issue_b(b0, i);
+                  else issue_a(a2, i);
                 }
               }
             });
@@ -602,7 +634,7 @@ __device__ __forceinline__ void early_barrier_pipeline16(int nk_total, char* sme
         }
       });
     });
-    cur ^= 1;
+    rotate();
   };
   int kt = 0;
   for (; kt + 2 < nk_total; ++kt) step(kt, std::true_type{});
@@ -625,11 +657,125 @@ __device__ __forceinline__ bool wave_is_live(const GemmOperands& g, int row0, in
 template <class C>
 constexpr bool kSplitPrologue = C::DMA && C::NSTAGE == 2 && (C::BK / 16) % 2 == 0;
 
+// gemm_mainloop_dma on the 16x16x32 schedule.  MODE 2 requests what early_barrier_pipeline16 expects on entry and
+// leaves LDS buffers 2 and 3 (64 KiB from C::STAGE on) to the caller until the MODE 1 call.
+template <class C, int MODE>
+__device__ __forceinline__ void gemm_mainloop_dma16(const GemmOperands& g, int row0, int col0, char* smem,
+                                                    f32x16_t (&acc)[C::TM][C::TN]) {
+  static_assert(kMi16<C>, "16x16x32 MFMAs: 8-wavefront 256x256x64 two-buffer tile only");
+  int tid = threadIdx.x;
+  asm volatile("" : "+v"(tid));                 // the per-lane offsets are formed anew per call (see gemm_mainloop_dma)
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave / C::WN, wn = wave % C::WN;
+  const int lrow = lane / C::CPR, lpc = lane % C::CPR;
+  uint32_t aoff[C::PA], boff[C::PB];
+  const int amax = g.M - 1 - row0, bmax = g.N - 1 - col0;
+#pragma unroll
+  for (int i = 0; i < C::PA; ++i) {
+    const int rt = (i * C::NW + wave) * C::RPI + lrow;
+    const int r = rt < amax ? rt : amax;
+    aoff[i] = (uint32_t)((long long)r * g.lda * 2 + ((lpc ^ lds_swizzle<C, true>(rt)) * 16));
+  }
+#pragma unroll
+  for (int i = 0; i < C::PB; ++i) {
+    const int rt = (i * C::NW + wave) * C::RPI + lrow;
+    const int r = rt < bmax ? rt : bmax;
+    boff[i] = (uint32_t)((long long)r * g.ldb * 2 + ((lpc ^ lds_swizzle<C, true>(rt)) * 16));
+  }
+  const int dst_w = wave * C::RPI * C::ROWB;
+
+  int nk_total = 0;
+  for (int s = 0; s < g.nseg; ++s) nk_total += g.seg[s].K / C::BK;
+
+  // One cursor over (segment, k) per operand: A runs a K step ahead of B.
+  int sa = 0, la = g.seg[0].K / C::BK, sb = 0, lb = la;
+  const char* Abase = (const char*)(g.seg[0].A + (long long)row0 * g.lda);
+  __amdgpu_buffer_rsrc_t rsa = make_rsrc(Abase, 0xffffffffu);
+  __amdgpu_buffer_rsrc_t rsb = make_rsrc(g.seg[0].B + (long long)col0 * g.ldb, 0xffffffffu);
+  uint32_t ka = 0, kb = 0;
+  constexpr int kStepsPerBlk = 256 / C::BK;
+  const long long a_blk_bytes = g.a_blk * 2;
+  int ablk_left = kStepsPerBlk;
+  auto advance_a = [&]() {
+    ka += C::BK * 2;
+    if (--ablk_left == 0) {
+      ablk_left = kStepsPerBlk;
+      if (a_blk_bytes != 0) {                          // next column block of A: re-base the descriptor
+        Abase += a_blk_bytes;
+        rsa = make_rsrc(Abase, 0xffffffffu);
+        ka = 0;
+      }
+    }
+    if (--la == 0 && sa + 1 < g.nseg) {
+      ++sa;
+      la = g.seg[sa].K / C::BK;
+      Abase = (const char*)(g.seg[sa].A + (long long)row0 * g.lda);
+      rsa = make_rsrc(Abase, 0xffffffffu);
+      ka = 0;
+      ablk_left = kStepsPerBlk;
+    }
+  };
+  auto advance_b = [&]() {
+    kb += C::BK * 2;
+    if (--lb == 0 && sb + 1 < g.nseg) {
+      ++sb;
+      lb = g.seg[sb].K / C::BK;
+      rsb = make_rsrc(g.seg[sb].B + (long long)col0 * g.ldb, 0xffffffffu);
+      kb = 0;
+    }
+  };
+  auto load_lds = [&](const __amdgpu_buffer_rsrc_t& rs, char* lds, int idx, uint32_t off, uint32_t k) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, FGRPO_LDS_PTR(lds + dst_w + idx * C::NW * C::RPI * C::ROWB), 16, (int)off, (int)k, 0, FGRPO_DMA_AUX);
+  };
+  auto issue_a = [&](char* lds, int idx) {
+    load_lds(rsa, lds, idx, aoff[idx], ka);
+    if (idx == C::PA - 1) advance_a();
+  };
+  auto issue_b = [&](char* lds, int idx) {
+    if (idx == 0) advance_b();
+    load_lds(rsb, lds, idx, boff[idx], kb);
+  };
+  if constexpr (MODE == 1) {                    // the MODE 2 call issued these
+    if (nk_total > 0) advance_a();
+    if (nk_total > 1) advance_a();
+  } else {
+    if constexpr (MODE == 0) FGRPO_WAIT_VMCNT(0);      // the caller's own loads must not be mistaken for ours
+    if (nk_total > 0) {
+      static_for<C::PB>([&](auto q) { load_lds(rsb, smem + mi16_b_buf(0) * kOpBytes<C>, decltype(q)::value, boff[decltype(q)::value], 0); });
+      static_for<C::PA>([&](auto q) { issue_a(smem, decltype(q)::value); });
+    }
+    if (nk_total > 1) static_for<C::PA>([&](auto q) { issue_a(smem + kOpBytes<C>, decltype(q)::value); });
+    if constexpr (MODE == 2) return;
+  }
+
+  // fragments: lane l reads row (l % 16) of a 16-row block and the 16-byte chunk 4*k2 + l/16 of its 64-wide K slice (16
+  // consecutive rows at one chunk index: conflict-free under the swizzle)
+  const int sw16 = lds_swizzle<C, true>(lane & 15);
+  const int fa16 = (wm * C::WTM + (lane & 15)) * C::ROWB, fb16 = (wn * C::WTN + (lane & 15)) * C::ROWB;
+  int fc16[2];
+#pragma unroll
+  for (int k2 = 0; k2 < 2; ++k2) fc16[k2] = ((4 * k2 + (lane >> 4)) ^ sw16) * 16;
+  early_barrier_pipeline16<C, 1, 1, MODE == 1, true>(
+      nk_total, smem, acc, true, issue_a, issue_b,
+      [&](const char* st, auto i, auto kk) {
+        constexpr int kkv = decltype(kk)::value;
+        return lds_read_b128_asm<(decltype(i)::value * 32 + 16 * (kkv & 1)) * C::ROWB>(lds_addr(st) + fa16 + fc16[kkv >> 1]);
+      },
+      [&](const char* st, auto jc, auto k2) {
+        constexpr int jcv = decltype(jc)::value;
+        return lds_read_b128_asm<((jcv >> 1) * 32 + 16 * (jcv & 1)) * C::ROWB>(lds_addr(st) + fb16 + fc16[decltype(k2)::value]);
+      });
+}
+
 template <class C, int MODE = 0, bool MI16 = false>
 __device__ __forceinline__ void gemm_mainloop_dma(const GemmOperands& g, int row0, int col0, char* smem,
                                                   f32x16_t (&acc)[C::TM][C::TN]) {
   static_assert(MODE == 0 || kSplitPrologue<C>, "split prologue needs the two-buffer schedule");
-  static_assert(!MI16 || kMi16<C>, "16x16x32 MFMAs: 8-wavefront 256x256x64 two-buffer tile only");
+  if constexpr (MI16) {
+    gemm_mainloop_dma16<C, MODE>(g, row0, col0, smem, acc);
+    return;
+  }
   constexpr int D = C::NSTAGE - 1;              // K steps of loads in flight
   constexpr int LPT = C::PA + C::PB;            // loads per thread per K step
   static_assert(D >= 1 && D <= 4 && LPT * (D - 1) < 64, "pipeline depth");
@@ -650,13 +796,13 @@ __device__ __forceinline__ void gemm_mainloop_dma(const GemmOperands& g, int row
   for (int i = 0; i < C::PA; ++i) {
     const int rt = (i * C::NW + wave) * C::RPI + lrow;            // row inside the tile (decides the swizzle)
     const int r = rt < amax ? rt : amax;                          // row actually read
-    aoff[i] = (uint32_t)((long long)r * g.lda * 2 + ((lpc ^ lds_swizzle<C, MI16>(rt)) * 16));
+    aoff[i] = (uint32_t)((long long)r * g.lda * 2 + ((lpc ^ lds_swizzle<C>(rt)) * 16));
   }
 #pragma unroll
   for (int i = 0; i < C::PB; ++i) {
     const int rt = (i * C::NW + wave) * C::RPI + lrow;
     const int r = rt < bmax ? rt : bmax;
-    boff[i] = (uint32_t)((long long)r * g.ldb * 2 + ((lpc ^ lds_swizzle<C, MI16>(rt)) * 16));
+    boff[i] = (uint32_t)((long long)r * g.ldb * 2 + ((lpc ^ lds_swizzle<C>(rt)) * 16));
   }
   const int dst_a = wave * C::RPI * C::ROWB;                      // + i * NW*RPI*ROWB, wave-uniform
   const int dst_b = C::BM * C::ROWB + dst_a;
@@ -735,26 +881,6 @@ __device__ __forceinline__ void gemm_mainloop_dma(const GemmOperands& g, int row
     if constexpr (MODE == 2) return;
   }
 
-  if constexpr (MI16) {
-    // 16x16x32 fragments: lane l reads row (l % 16) of a 16-row block and the 16-byte chunk 4*k2 + l/16 of its
-    // 64-wide K slice (16 consecutive rows at one chunk index: conflict-free under the same swizzle)
-    const int sw16 = lds_swizzle<C, MI16>(lane & 15);
-    const int fa16 = (wm * C::WTM + (lane & 15)) * C::ROWB, fb16 = C::BM * C::ROWB + (wn * C::WTN + (lane & 15)) * C::ROWB;
-    int fc16[2];
-#pragma unroll
-    for (int k2 = 0; k2 < 2; ++k2) fc16[k2] = ((4 * k2 + (lane >> 4)) ^ sw16) * 16;
-    early_barrier_pipeline16<C, LPT, 1, 1>(
-        nk_total, smem, acc, true, issue_one,
-        [&](const char* st, auto i, auto kk) {
-          constexpr int kkv = decltype(kk)::value;
-          return lds_read_b128_asm<(decltype(i)::value * 32 + 16 * (kkv & 1)) * C::ROWB>(lds_addr(st) + fa16 + fc16[kkv >> 1]);
-        },
-        [&](const char* st, auto jc, auto k2) {
-          constexpr int jcv = decltype(jc)::value;
-          return lds_read_b128_asm<((jcv >> 1) * 32 + 16 * (jcv & 1)) * C::ROWB>(lds_addr(st) + fb16 + fc16[decltype(k2)::value]);
-        });
-    return;
-  }
   if constexpr (C::NSTAGE == 2 && (C::BK / 16) % 2 == 0) {
     early_barrier_pipeline<C, LPT, 1, 1>(
         nk_total, smem, acc, issue_one,
@@ -1008,29 +1134,22 @@ __device__ __forceinline__ void gemm_mainloop_la(const GemmOperands& g, int row0
 // Either operand may instead be K-contiguous (X[m][k]) and is then handled as in
 // gemm_mainloop_dma.  One segment, BM = BN = 256, BK = 64, two LDS buffers.
 // ---------------------------------------------------------------------------
-// Chunk-index XOR of k row `kr` of a K-major LDS tile (512-byte rows).  The transposing reads of a 32x32x16 operand
-// take rows k .. k+3 per 16-lane group with the two groups of a pass 32 bytes apart in the row: 4*(k%4) spreads the
-// four rows.  A 16x16x32 operand's groups of a pass read the same columns of rows k and k + 8: bit 3 of k moves
-// them another 32 bytes apart.
-template <bool MI16>
-__device__ __forceinline__ int km_swizzle(int kr) {
-  return MI16 ? (((kr & 3) << 2) | (((kr >> 3) & 1) << 1)) : ((kr & 3) << 2);
-}
-template <class C, bool AKM, bool BKM, bool MI16 = false>
+// Chunk-index XOR of k row `kr` of a K-major LDS tile (512-byte rows).  The transposing reads of a 16-lane group take
+// rows k .. k+3: 4*(k%4) spreads the four; two groups of a pass read the same columns of rows k and k + 8: bit 3 of k
+// moves them 32 bytes apart.
+__device__ __forceinline__ int km_swizzle(int kr) { return ((kr & 3) << 2) | (((kr >> 3) & 1) << 1); }
+template <class C, bool AKM, bool BKM, bool AHEAD = true>
 __device__ __forceinline__ void gemm_mainloop_km(const GemmOperands& g, int row0, int col0, char* smem,
                                                  f32x16_t (&acc)[C::TM][C::TN]) {
-  static_assert(C::DMA && C::NSTAGE == 2 && C::BM == 256 && C::BN == 256 && C::BK == 64, "K-major loop: 256x256x64, 2 buffers");
-  static_assert(!MI16 || kMi16<C>, "16x16x32 MFMAs: 8-wavefront tile only");
-  constexpr int LPT = C::PA + C::PB;
-  constexpr int KK = C::BK / 16;
+  static_assert(kMi16<C> && C::BM == 256 && C::BN == 256, "K-major loop: the 8-wavefront 256x256x64 tile");
   constexpr int KROWB = 512;                    // bytes of one k row of a K-major tile (256 columns)
-  constexpr int REG = C::BM * C::ROWB;          // bytes of one operand region (32 KiB either way)
-  static_assert(C::ROWB == 128 && REG == C::BK * KROWB, "region size");
+  constexpr int OP = kOpBytes<C>;               // bytes of one operand's buffer (32 KiB either way)
+  static_assert(C::ROWB == 128 && OP == C::BK * KROWB, "buffer size");
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);   // wavefront-uniform
   int wm, wn;
-  wave_coords<C, MI16>(wave, wm, wn);
+  wave_coords<C, true>(wave, wm, wn);
 
   // ---- loader ------------------------------------------------------------------------------
   uint32_t aoff[C::PA], boff[C::PB];            // per-lane byte offset of each load inside the step's slice
@@ -1041,22 +1160,22 @@ __device__ __forceinline__ void gemm_mainloop_km(const GemmOperands& g, int row0
     for (int i = 0; i < C::PA; ++i) {
       if constexpr (AKM) {
         const int kr = (i * C::NW + wave) * 2 + (lane >> 5);
-        aoff[i] = (uint32_t)((long long)kr * g.lda * 2) + (uint32_t)((((lane & 31) ^ km_swizzle<MI16>(kr))) * 16);
+        aoff[i] = (uint32_t)((long long)kr * g.lda * 2) + (uint32_t)((((lane & 31) ^ km_swizzle(kr))) * 16);
       } else {
         const int rt = (i * C::NW + wave) * C::RPI + lrow;
         const int r = rt < amax ? rt : amax;
-        aoff[i] = (uint32_t)((long long)r * g.lda * 2 + ((lpc ^ lds_swizzle<C, MI16>(rt)) * 16));
+        aoff[i] = (uint32_t)((long long)r * g.lda * 2 + ((lpc ^ lds_swizzle<C, true>(rt)) * 16));
       }
     }
 #pragma unroll
     for (int i = 0; i < C::PB; ++i) {
       if constexpr (BKM) {
         const int kr = (i * C::NW + wave) * 2 + (lane >> 5);
-        boff[i] = (uint32_t)((long long)kr * g.ldb * 2) + (uint32_t)((((lane & 31) ^ km_swizzle<MI16>(kr))) * 16);
+        boff[i] = (uint32_t)((long long)kr * g.ldb * 2) + (uint32_t)((((lane & 31) ^ km_swizzle(kr))) * 16);
       } else {
         const int rt = (i * C::NW + wave) * C::RPI + lrow;
         const int r = rt < bmax ? rt : bmax;
-        boff[i] = (uint32_t)((long long)r * g.ldb * 2 + ((lpc ^ lds_swizzle<C, MI16>(rt)) * 16));
+        boff[i] = (uint32_t)((long long)r * g.ldb * 2 + ((lpc ^ lds_swizzle<C, true>(rt)) * 16));
       }
     }
   }
@@ -1087,51 +1206,53 @@ __device__ __forceinline__ void gemm_mainloop_km(const GemmOperands& g, int row0
   uint32_t ka = 0, kb = 0;                      // running K byte offset of a K-contiguous operand
   const int dst_w = wave * 1024;                // both layouts: one load fills 1 KiB, loads i are NW KiB apart
 
-  // run list (A K-major; B either way): the issue cursor walks the listed K steps; the compute side never
+  // run list (A K-major; B either way): the cursors walk the listed K steps; the compute side never
   // knows, it consumes LDS buffers in the order they were filled
   const int* runs = AKM ? g.k_runs : nullptr;
   const int n_runs = runs ? runs[0] : 0;
   const int nk_total = runs ? runs[1] : g.seg[0].K / C::BK;
   int run_idx = 0, run_left = 0, cur_step = 0;
+  auto skip_a = [&](long long steps) {           // A's cursor that many K steps on (A K-major)
+    Ap += steps * C::BK * lda2;
+    a_rem -= steps * C::BK;
+    rsa = make_rsrc(Ap, bytes_of(a_rem, lda2, a_col));
+  };
+  auto skip_b = [&](long long steps) {
+    if constexpr (BKM) {
+      Bp += steps * C::BK * ldb2;
+      b_rem -= steps * C::BK;
+      rsb = make_rsrc(Bp, bytes_of(b_rem, ldb2, b_col));
+    } else {
+      kb += (uint32_t)steps * C::BK * 2;
+    }
+  };
   if (runs != nullptr && n_runs > 0) {
     cur_step = runs[2];
     run_left = runs[2 + kRunCap] - cur_step;
-    Ap += (long long)cur_step * C::BK * lda2;
-    a_rem -= (long long)cur_step * C::BK;
-    rsa = make_rsrc(Ap, bytes_of(a_rem, lda2, a_col));
-    if constexpr (BKM) {
-      Bp += (long long)cur_step * C::BK * ldb2;
-      b_rem -= (long long)cur_step * C::BK;
-      rsb = make_rsrc(Bp, bytes_of(b_rem, ldb2, b_col));
-    } else {
-      kb = (uint32_t)cur_step * C::BK * 2;
-    }
+    skip_a(cur_step);
+    skip_b(cur_step);
   }
   const long long a_blk_bytes = (!AKM) ? g.a_blk * 2 : 0;
   int ablk_left = 256 / C::BK;
-  auto issue_one = [&](int stage, int idx) {
-    char* base = smem + stage * C::STAGE;
-    if (idx < C::PA)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rsa, FGRPO_LDS_PTR(base + dst_w + idx * C::NW * 1024), 16, (int)aoff[idx],
-                                               (int)ka, 0, FGRPO_DMA_AUX);
-    else
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rsb, FGRPO_LDS_PTR(base + REG + dst_w + (idx - C::PA) * C::NW * 1024), 16,
-                                               (int)boff[idx - C::PA], (int)kb, 0, FGRPO_DMA_AUX);
-    if (idx == LPT - 1) {                        // next K step
-      long long jump = 1;                        // K steps from this one to the next one to fetch
+  int jump_a = 1, jump_b = 1;                    // K steps from the step A's cursor came from to where it is, and from the one before it
+  auto load_lds = [&](const __amdgpu_buffer_rsrc_t& rs, char* lds, int idx, uint32_t off, uint32_t k) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, FGRPO_LDS_PTR(lds + dst_w + idx * C::NW * 1024), 16, (int)off, (int)k, 0, FGRPO_DMA_AUX);
+  };
+  auto issue_a = [&](char* lds, int idx) {
+    load_lds(rsa, lds, idx, aoff[idx], ka);
+    if (idx == C::PA - 1) {                      // next K step
       if constexpr (AKM) {
+        int jump = 1;
         if (runs != nullptr && --run_left == 0 && run_idx + 1 < n_runs) {   // this run is done: on to the next
           ++run_idx;
           const int s = runs[2 + run_idx];
           jump = s - cur_step;
           run_left = runs[2 + kRunCap + run_idx] - s;
         }
-        cur_step += (int)jump;
-      }
-      if constexpr (AKM) {
-        Ap += jump * C::BK * lda2;
-        a_rem -= jump * C::BK;
-        rsa = make_rsrc(Ap, bytes_of(a_rem, lda2, a_col));
+        cur_step += jump;
+        jump_b = jump_a;                         // B follows a step behind
+        jump_a = jump;
+        skip_a(jump);
       } else {
         ka += C::BK * 2;
         if (--ablk_left == 0) {
@@ -1143,100 +1264,57 @@ __device__ __forceinline__ void gemm_mainloop_km(const GemmOperands& g, int row0
           }
         }
       }
-      if constexpr (BKM) {
-        Bp += jump * C::BK * ldb2;
-        b_rem -= jump * C::BK;
-        rsb = make_rsrc(Bp, bytes_of(b_rem, ldb2, b_col));
-      } else {
-        kb += (uint32_t)jump * C::BK * 2;
-      }
     }
+  };
+  auto issue_b = [&](char* lds, int idx) {
+    if (idx == 0) skip_b(AKM ? jump_b : 1);
+    load_lds(rsb, lds, idx, boff[idx], kb);
   };
 
   // ---- fragment addressing -------------------------------------------------------------------
-  // K-contiguous operand: row (lane%32), chunk (2*kk + lane/32) ^ swizzle(row)
-  const int swn = lds_swizzle<C>(lane & 31);
-  int frn_c[KK];
+  // K-contiguous operand: row l % 16 of a 16-row block, chunk 4*k2 + l/16.  K-major operand:
+  // lane l = 16*g + j supplies row k = 32*k2 + 8*g + 4*r + j/4 (r = 0, 1: the two transposing reads) and the 8 bytes
+  // at column 4*(j%4) of the 16-column block; every 16-lane group gets its own eight k values of the slice.
+  const int sw16 = lds_swizzle<C, true>(lane & 15);
+  const int fa16 = (wm * C::WTM + (lane & 15)) * C::ROWB, fb16 = (wn * C::WTN + (lane & 15)) * C::ROWB;
+  int fc16[2];
 #pragma unroll
-  for (int kk = 0; kk < KK; ++kk) frn_c[kk] = ((kk * 2 + (lane >> 5)) ^ swn) * 16;
-  const int frn_a = (wm * C::WTM + (lane & 31)) * C::ROWB;
-  const int frn_b = REG + (wn * C::WTN + (lane & 31)) * C::ROWB;
-  // K-major operand: lane l = 16*g + j supplies row k = 16*kk + 8*(g/2) + 4*r + j/4 and the 8 bytes at
-  // column (g%2)*16 + 4*(j%4) of the 32-column block; chunk index XOR 4*(k%4) = 4*(j/4)
-  const int j4 = (lane & 15) >> 2;
-  const int frk_row = (8 * (lane >> 5) + j4) * KROWB;                         // + (16*kk + 4*r) * KROWB
-  const int frk_sw = j4 << 2;
-  const int frk_cl = (((lane >> 4) & 1) * 16 + 4 * (lane & 3)) >> 3;          // chunk of the lane's column inside a block
-  const int frk_half = (lane & 1) * 8;
-  auto km_off = [&](int block_col0) {            // byte offset of this lane's 8 bytes inside a k row
-    return ((((block_col0 >> 3) + frk_cl) ^ frk_sw) << 4) + frk_half;
-  };
-  int fka[C::TM], fkb[C::TN];
+  for (int k2 = 0; k2 < 2; ++k2) fc16[k2] = ((4 * k2 + (lane >> 4)) ^ sw16) * 16;
+  const int j4 = (lane & 15) >> 2, g16 = lane >> 4;
+  const int k16_row = (8 * g16 + j4) * KROWB;                      // + (32*k2 + 4*r) * KROWB
+  const int k16_sw = (j4 << 2) | ((g16 & 1) << 1);                 // km_swizzle of the lane's rows
+  const int k16_cl = (lane & 3) >> 1;                              // chunk of the lane's column inside a 16-column block
+  auto km16_off = [&](int block_col0) { return ((((block_col0 >> 3) + k16_cl) ^ k16_sw) << 4) + (lane & 1) * 8; };
+  int fka16[C::TM][2], fkb16[2 * C::TN];
 #pragma unroll
-  for (int i = 0; i < C::TM; ++i) fka[i] = frk_row + km_off(wm * C::WTM + i * 32);
+  for (int i = 0; i < C::TM; ++i)
 #pragma unroll
-  for (int j = 0; j < C::TN; ++j) fkb[j] = REG + frk_row + km_off(wn * C::WTN + j * 32);
+    for (int rh = 0; rh < 2; ++rh) fka16[i][rh] = k16_row + km16_off(wm * C::WTM + i * 32 + 16 * rh);
+#pragma unroll
+  for (int jc = 0; jc < 2 * C::TN; ++jc) fkb16[jc] = k16_row + km16_off(wn * C::WTN + (jc >> 1) * 32 + 16 * (jc & 1));
 
-  auto load_a = [&](const char* st, auto ic, auto kc) -> bf16x8_t {
-    constexpr int i = decltype(ic)::value, kk = decltype(kc)::value;
-    if constexpr (AKM)
-      return lds_read_tr_pair<(16 * kk) * KROWB, (16 * kk + 4) * KROWB>(lds_addr(st) + fka[i]);
-    else
-      return lds_read_b128_asm<i * 32 * C::ROWB>(lds_addr(st) + frn_a + frn_c[kk]);
-  };
-  auto load_b = [&](const char* st, auto jc, auto kc) -> bf16x8_t {
-    constexpr int j = decltype(jc)::value, kk = decltype(kc)::value;
-    if constexpr (BKM)
-      return lds_read_tr_pair<(16 * kk) * KROWB, (16 * kk + 4) * KROWB>(lds_addr(st) + fkb[j]);
-    else
-      return lds_read_b128_asm<j * 32 * C::ROWB>(lds_addr(st) + frn_b + frn_c[kk]);
-  };
-  // ---- pipeline: two buffers, barrier one sub-step early ----
   FGRPO_WAIT_VMCNT(0);
   if (nk_total > 0) {
-#pragma unroll
-    for (int idx = 0; idx < LPT; ++idx) issue_one(0, idx);
+    static_for<C::PB>([&](auto q) { load_lds(rsb, smem + mi16_b_buf(0) * OP, decltype(q)::value, boff[decltype(q)::value], kb); });
+    static_for<C::PA>([&](auto q) { issue_a(smem, decltype(q)::value); });
   }
-  if constexpr (MI16) {
-    // 16x16x32 fragments.  K-contiguous operand: row l % 16 of a 16-row block, chunk 4*k2 + l/16.  K-major operand:
-    // lane l = 16*g + j supplies row k = 32*k2 + 8*g + 4*r + j/4 (r = 0, 1: the two transposing reads) and the 8 bytes
-    // at column 4*(j%4) of the 16-column block; every 16-lane group gets its own eight k values of the slice.
-    const int sw16 = lds_swizzle<C, MI16>(lane & 15);
-    const int fa16 = (wm * C::WTM + (lane & 15)) * C::ROWB, fb16 = REG + (wn * C::WTN + (lane & 15)) * C::ROWB;
-    int fc16[2];
-#pragma unroll
-    for (int k2 = 0; k2 < 2; ++k2) fc16[k2] = ((4 * k2 + (lane >> 4)) ^ sw16) * 16;
-    const int g16 = lane >> 4;
-    const int k16_row = (8 * g16 + j4) * KROWB;                      // + (32*k2 + 4*r) * KROWB
-    const int k16_sw = (j4 << 2) | ((g16 & 1) << 1);                 // km_swizzle of the lane's rows
-    const int k16_cl = (lane & 3) >> 1;                              // chunk of the lane's column inside a 16-column block
-    auto km16_off = [&](int block_col0) { return ((((block_col0 >> 3) + k16_cl) ^ k16_sw) << 4) + frk_half; };
-    int fka16[C::TM][2], fkb16[2 * C::TN];
-#pragma unroll
-    for (int i = 0; i < C::TM; ++i)
-#pragma unroll
-      for (int rh = 0; rh < 2; ++rh) fka16[i][rh] = k16_row + km16_off(wm * C::WTM + i * 32 + 16 * rh);
-#pragma unroll
-    for (int jc = 0; jc < 2 * C::TN; ++jc) fkb16[jc] = REG + k16_row + km16_off(wn * C::WTN + (jc >> 1) * 32 + 16 * (jc & 1));
-    early_barrier_pipeline16<C, LPT, AKM ? 2 : 1, BKM ? 2 : 1>(
-        nk_total, smem, acc, wave_is_live<C>(g, row0, col0, wm, wn), issue_one,
-        [&](const char* st, auto ic, auto kc) -> bf16x8_t {
-          constexpr int i = decltype(ic)::value, kk = decltype(kc)::value, k2 = kk >> 1, rh = kk & 1;
-          if constexpr (AKM)
-            return lds_read_tr_pair<(32 * k2) * KROWB, (32 * k2 + 4) * KROWB>(lds_addr(st) + fka16[i][rh]);
-          else
-            return lds_read_b128_asm<(i * 32 + 16 * rh) * C::ROWB>(lds_addr(st) + fa16 + fc16[k2]);
-        },
-        [&](const char* st, auto jcc, auto k2c) -> bf16x8_t {
-          constexpr int jc = decltype(jcc)::value, k2 = decltype(k2c)::value;
-          if constexpr (BKM)
-            return lds_read_tr_pair<(32 * k2) * KROWB, (32 * k2 + 4) * KROWB>(lds_addr(st) + fkb16[jc]);
-          else
-            return lds_read_b128_asm<((jc >> 1) * 32 + 16 * (jc & 1)) * C::ROWB>(lds_addr(st) + fb16 + fc16[k2]);
-        });
-    return;
-  }
-  early_barrier_pipeline<C, LPT, AKM ? 2 : 1, BKM ? 2 : 1>(nk_total, smem, acc, issue_one, load_a, load_b);
+  if (nk_total > 1) static_for<C::PA>([&](auto q) { issue_a(smem + OP, decltype(q)::value); });
+  early_barrier_pipeline16<C, AKM ? 2 : 1, BKM ? 2 : 1, false, AHEAD>(
+      nk_total, smem, acc, wave_is_live<C>(g, row0, col0, wm, wn), issue_a, issue_b,
+      [&](const char* st, auto ic, auto kc) -> bf16x8_t {
+        constexpr int i = decltype(ic)::value, kk = decltype(kc)::value, k2 = kk >> 1, rh = kk & 1;
+        if constexpr (AKM)
+          return lds_read_tr_pair<(32 * k2) * KROWB, (32 * k2 + 4) * KROWB>(lds_addr(st) + fka16[i][rh]);
+        else
+          return lds_read_b128_asm<(i * 32 + 16 * rh) * C::ROWB>(lds_addr(st) + fa16 + fc16[k2]);
+      },
+      [&](const char* st, auto jcc, auto k2c) -> bf16x8_t {
+        constexpr int jc = decltype(jcc)::value, k2 = decltype(k2c)::value;
+        if constexpr (BKM)
+          return lds_read_tr_pair<(32 * k2) * KROWB, (32 * k2 + 4) * KROWB>(lds_addr(st) + fkb16[jc]);
+        else
+          return lds_read_b128_asm<((jc >> 1) * 32 + 16 * (jc & 1)) * C::ROWB>(lds_addr(st) + fb16 + fc16[k2]);
+      });
 }
 
 template <class C>

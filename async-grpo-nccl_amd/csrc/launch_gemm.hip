@@ -18,6 +18,11 @@ int launch_store_variant(int variant, const StoreParams& p, hipStream_t st) {
 }
 
 int launch_store_splitk(const StoreParams& p, hipStream_t st) {
+  // Pieces of one column chunk walk the same rows of W; from the fifth device round on, work-groups that replace others have
+  // lost step with each other, and the longer lead lets them stay apart.  Longer | shorter lead, ms: H = 5120, T = 8192, five
+  // rounds 10.3 | 9.6; H = 3584, T = 16384, seven 13.1 | 12.9; T = 8192, seven 6.74 | 6.75; four rounds at most: H = 3584, T = 8975
+  // 6.70 | 7.02, T = 2000 1.76 | 1.85; H = 1536, T = 8192 2.72 | 2.79.
+  if (p.nblocks > 4 * num_cus()) return launch_tile_kernel<gemm_store_kernel<Cfg8, false, true, true, false>, Cfg8>(p, p.nblocks, st);
   return launch_tile_kernel<gemm_store_kernel<Cfg8, false, true, true>, Cfg8>(p, p.nblocks, st);
 }
 

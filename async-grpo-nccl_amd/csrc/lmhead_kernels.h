@@ -762,7 +762,8 @@ __device__ __forceinline__ void store_tile_lds(const StoreParams& p, f32x16_t (&
 
 // SPLITK: the tiles of a device round that would otherwise run nearly empty are contracted in ksplit pieces by ksplit
 // work-groups each (a K-contiguous, column-blocked A and a contraction-major B: dHidden's last round).
-template <class C, bool AKM = false, bool BKM = false, bool SPLITK = false>
+// AHEAD: see early_barrier_pipeline16.
+template <class C, bool AKM = false, bool BKM = false, bool SPLITK = false, bool AHEAD = true>
 __global__ __launch_bounds__(C::NT, C::OCC) void gemm_store_kernel(const StoreParams p0) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -794,7 +795,7 @@ __global__ __launch_bounds__(C::NT, C::OCC) void gemm_store_kernel(const StorePa
       p.g.seg[0].B += (long long)k0 * p.g.ldb;
       p.g.seg[0].K = klen;
       p.g.kb_valid = b_rows;
-      gemm_mainloop_km<C, false, true, true>(p.g, row0, col0, smem, acc);
+      gemm_mainloop_km<C, false, true, AHEAD>(p.g, row0, col0, smem, acc);
     }
     p.c_out_f32 += (long long)ks * p.part_slice;
     if (p.wide_stores)
@@ -843,7 +844,7 @@ __global__ __launch_bounds__(C::NT, C::OCC) void gemm_store_kernel(const StorePa
   const bool dead = p.m_tile_live != nullptr && p.m_tile_live[tm] == 0;     // work-group uniform
   if (!dead) {
     if constexpr (AKM || BKM)
-      gemm_mainloop_km<C, AKM, BKM, MI16>(p.g, row0, col0, smem, acc);
+      gemm_mainloop_km<C, AKM, BKM, AHEAD>(p.g, row0, col0, smem, acc);
     else if constexpr (MI16)
       gemm_mainloop_dma<C, 0, true>(p.g, row0, col0, smem, acc);
     else
