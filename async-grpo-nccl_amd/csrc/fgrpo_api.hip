@@ -111,6 +111,7 @@ int* tuning_slot(const char* key) {
   if (!strcmp(key, "wide_stores")) return &g_tune.wide_stores;
   if (!strcmp(key, "keep_panels")) return &g_tune.keep_panels;
   if (!strcmp(key, "keep_skip_dead")) return &g_tune.keep_skip_dead;
+  if (!strcmp(key, "fwd_tail")) return &g_tune.fwd_tail;
   if (!strcmp(key, "tail_split")) return &g_tune.tail_split;
   return nullptr;
 }
@@ -193,6 +194,9 @@ struct FwdPlan {
   // t_main < T, the rest with a split count of their own (`nsplit_rem`), launched right behind them.
   int t_main, nsplit_rem;
   float4* part_rem;
+  // A narrow last tile (FwdParams::tail_nb) of the last region, or tail_nb = 0.
+  int tail_nb, tail_split;
+  float4* part_tail;
   int Hp;            // padded contraction length
   bool copy_ops;     // operands are staged (fp32 split or padding) instead of used in place
   bf16_t *w_hi, *w_lo, *h_hi, *h_lo;
@@ -257,6 +261,48 @@ int fwd_raster_group(const Tuning& tn, int nsplit) {
   return nsplit == 8 ? 4 : g < 6 ? g : 6;
 }
 
+// A last tile of few tokens: 64 NB columns wide it costs a work-group kTailCost[NB] of what a whole one does (24 K steps of
+// H = 1536: 43 us; one this narrow waits for W, which comes from HBM, and no longer for its matrix instructions).  Its
+// vocabulary is dealt out in shares that take as long as the whole tiles', so that it fills part of the round instead of a
+// quarter of it or a round of its own.  Forward at H = 1536, V = 151936, whole | narrow, us: T = 60 131 | 88, 100 136 | 95, 300
+// 208 | 178, 777 468 | 442, 868 408 | 350, 1034 483 | 437; H = 8192, V = 128256: T = 550 1448 | 1330.  From 129 columns on
+// little is left to gain.
+constexpr double kTailCost[3] = {0.0, 0.5, 0.65};
+int tail_columns(const Tuning& tn, int variant, int T) {        // NB, or 0 where the last tile is taken whole
+  const int r = T % kCfg[8].bn;
+  if (variant != 8 || tn.fwd_tail == 0 || tn.fwd_nsplit > 0 || r == 0 || r > 128) return 0;
+  return r <= 64 ? 1 : 2;
+}
+struct TailPlan {
+  int nsplit = 0, tail_split = 0;
+};
+// Shares of the whole tiles and of the narrow one: the cheapest by device rounds x vocabulary tiles of a whole-tile work-group.
+TailPlan plan_tail(int tiles, int nb, int tiles_v, int slots, int prefer, long long* cost_out) {
+  TailPlan best;
+  long long least = -1;
+  auto consider = [&](int ns) {
+    const int per = tiles > 0 ? (tiles_v + ns - 1) / ns : (int)(kTailCost[nb] * ((tiles_v + ns - 1) / ns) + 1.0);
+    int share = (int)(per / kTailCost[nb]);
+    if (share < 1) share = 1;
+    const int nt = tiles > 0 ? (tiles_v + share - 1) / share : ns;
+    const long long blocks = (long long)tiles * ns + nt, cost = (blocks + slots - 1) / slots * per;
+    if (least < 0 || cost < least) least = cost, best.nsplit = ns, best.tail_split = nt;
+    return cost;
+  };
+  int cap = tiles > 0 && slots / tiles > 64 ? slots / tiles : 64;
+  if (tiles == 0) cap = slots;
+  if (cap > tiles_v) cap = tiles_v;
+  for (int ns = 1; ns <= cap; ++ns) consider(ns);
+  if (tiles > 0 && cap >= prefer) {      // the patch an XCD shares, as in choose_nsplit
+    const long long at_best = least;
+    TailPlan keep = best;
+    least = -1;
+    if (consider(prefer) * 100 > at_best * 106) best = keep, least = at_best;
+  }
+  if (cost_out) *cost_out = least;
+  return best;
+}
+
 void plan_fwd(const Tuning& tn, FwdPlan& pl, void* ws, int T, int H, int V, int dtype, bool has_bias) {
   pl.variant = pick_variant(tn, tn.fwd_variant, V, T);
   const CfgInfo& c = kCfg[pl.variant];
@@ -293,6 +339,16 @@ void plan_fwd(const Tuning& tn, FwdPlan& pl, void* ws, int T, int H, int V, int 
       }
     }
   }
+  pl.tail_nb = tail_columns(tn, pl.variant, T);
+  pl.tail_split = 0;
+  if (pl.tail_nb > 0) {
+    const int r0 = pl.t_main < T ? pl.t_main : 0, tiles = (T - r0) / c.bn;      // of the last region
+    int& ns = pl.t_main < T ? pl.nsplit_rem : pl.nsplit;
+    long long cost = 0;
+    const TailPlan t = plan_tail(tiles, pl.tail_nb, pl.tiles_v, slots, prefer, &cost);
+    if (tiles == 0 || cost < split_cost(tiles + 1, pl.tiles_v, slots, ns)) ns = t.nsplit, pl.tail_split = t.tail_split;
+    else pl.tail_nb = 0;
+  }
   pl.Hp = (int)round_up(H, 64);
   pl.copy_ops = (dtype == FGRPO_F32) || (H % 64 != 0);
   Carver cv(ws);
@@ -308,6 +364,7 @@ void plan_fwd(const Tuning& tn, FwdPlan& pl, void* ws, int T, int H, int V, int 
   pl.bias32 = has_bias ? cv.take<float>((size_t)V) : nullptr;
   pl.part = cv.take<float4>((size_t)pl.nsplit * T);
   pl.part_rem = pl.t_main < T ? cv.take<float4>((size_t)pl.nsplit_rem * (T - pl.t_main)) : nullptr;
+  pl.part_tail = pl.tail_split > 0 ? cv.take<float4>((size_t)pl.tail_split * (T % c.bn)) : nullptr;
   pl.xt = cv.take<float>((size_t)T);
   pl.bytes = cv.total();
 }
@@ -748,7 +805,11 @@ int logprob_fwd_impl(const void* hidden, const void* weight, const void* bias, c
     q.g.N = count;
     for (int sg = 0; sg < q.g.nseg; ++sg) q.g.seg[sg].B += (long long)t0 * q.g.ldb;
     q.labels += t0;
-    q.tiles_t = (count + c_bn - 1) / c_bn;
+    const bool narrow = pl.tail_split > 0 && t0 + count == T;
+    q.tiles_t = narrow ? count / c_bn : (count + c_bn - 1) / c_bn;
+    q.tail_nb = narrow ? pl.tail_nb : 0;
+    q.tail_split = narrow ? pl.tail_split : 0;
+    q.part_tail = pl.part_tail;
     q.nsplit = nsplit;
     q.group_t = fwd_raster_group(tn, nsplit);
     q.part = part;
@@ -759,7 +820,8 @@ int logprob_fwd_impl(const void* hidden, const void* weight, const void* bias, c
     }
     const int rc2 = keep ? launch_fwd_keep(q, st) : launch_fwd_variant(pl.variant, q, st);
     if (rc2) return rc2;
-    CombineParams c{part, pl.xt + t0, (const long long*)labels + t0, count, V, nsplit, lp_out + t0,
+    CombineParams c{part, pl.xt + t0, (const long long*)labels + t0, count, V, nsplit, pl.part_tail,
+                    narrow ? q.tiles_t * c_bn : count, q.tail_split, lp_out + t0,
                     ent_out ? ent_out + t0 : nullptr, lse_out ? lse_out + t0 : nullptr, LossParams()};
     if (loss) {
       c.loss = loss_from(*loss, t0);
@@ -833,7 +895,12 @@ int fgrpo_logprob_fwd_static(const void* hidden, const void* weight, const void*
   if (T <= 0 || H <= 0 || V <= 0) return fail(FGRPO_ERR_BAD_ARG, "logprob_fwd_static: T=%d H=%d V=%d", T, H, V);
   if (dtype != FGRPO_BF16 && dtype != FGRPO_F32) return fail(FGRPO_ERR_BAD_ARG, "logprob_fwd_static: dtype=%d", dtype);
   FwdPlan pl;
-  plan_fwd(g_tune, pl, nullptr, T, H, V, dtype, bias != nullptr);
+  Tuning tn = g_tune;
+  plan_fwd(tn, pl, nullptr, T, H, V, dtype, bias != nullptr);
+  if (pl.bytes > FGRPO_STATIC_SCRATCH_BYTES) {      // a narrow last tile may come with more shares of the others
+    tn.fwd_tail = 0;
+    plan_fwd(tn, pl, nullptr, T, H, V, dtype, bias != nullptr);
+  }
   if (pl.bytes > FGRPO_STATIC_SCRATCH_BYTES)
     return fail(FGRPO_ERR_WORKSPACE,
                 "logprob_fwd_static: this call needs %zu bytes of scratch, the built-in buffer holds %u "
@@ -842,7 +909,7 @@ int fgrpo_logprob_fwd_static(const void* hidden, const void* weight, const void*
   int rc = static_scratch_ptr(&ptr);
   if (rc) return rc;
   return logprob_fwd_impl(hidden, weight, bias, labels, inv_temp, T, H, V, dtype, lp_out, ent_out, lse_out, ptr,
-                          FGRPO_STATIC_SCRATCH_BYTES, stream);
+                          FGRPO_STATIC_SCRATCH_BYTES, stream, nullptr, &tn);
 }
 
 size_t fgrpo_lmhead_bwd_workspace(int T, int H, int V, int dtype, long long hint) {

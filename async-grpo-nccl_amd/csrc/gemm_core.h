@@ -501,6 +501,7 @@ __device__ __forceinline__ void early_barrier_pipeline(int nk_total, char* smem,
 //   issue_a(lds, idx) / issue_b(lds, idx): load idx of the next K step of that operand into the buffer at `lds`; the
 //   last one of A (the first one of B, but for step 0's) advances the operand's cursor;
 //   load_a(lds, I, KK): fragment a(I, KK % 2) of slice KK / 2;  load_b(lds, JC, K2): fragment b(JC/2, JC%2).
+// NB: 16-column blocks of operand B a wavefront multiplies, 4 or, on tiles 64 NB columns wide (kTailCols), fewer.
 // On entry B of step 0 and A of steps 0 and 1 have been issued, in this order (as far as they exist).  DRAIN: wait for
 // all of it (the caller has issued something else since), not just for step 0.
 constexpr int kStrictEvery = 4;                      // a power of two
@@ -508,14 +509,14 @@ template <class C>
 constexpr int kOpBytes = C::BM * C::ROWB;            // one buffer of one operand (32 KiB)
 __device__ __forceinline__ constexpr int mi16_a_buf(int step) { return step % 3; }          // in kOpBytes
 __device__ __forceinline__ constexpr int mi16_b_buf(int step) { return 4 - (step & 1); }    // buffers 2 and 3 are free between tiles
-template <class C, int RA, int RB, bool DRAIN, bool AHEAD, class IssueA, class IssueB, class LoadA, class LoadB>
+template <class C, int NB, int RA, int RB, bool DRAIN, bool AHEAD, class IssueA, class IssueB, class LoadA, class LoadB>
 __device__ __forceinline__ void early_barrier_pipeline16(int nk_total, char* smem, f32x16_t (&acc)[C::TM][C::TN],
                                                          bool live, IssueA&& issue_a, IssueB&& issue_b, LoadA&& load_a,
                                                          LoadB&& load_b) {
   constexpr int KK = 4;
-  constexpr int TM = C::TM, NB = 2 * C::TN;           // a fragments per sub-step, b fragments per K slice
-  constexpr int PA = C::PA, PB = C::PB, OP = kOpBytes<C>;
-  static_assert(kMi16<C> && C::BK == 64 && PA == TM && PB == TM, "16x16x32 schedule: 8-wavefront 256x256x64 tile, one load per row group");
+  constexpr int TM = C::TM;                           // a fragments per sub-step; NB: b fragments per K slice
+  constexpr int PA = C::PA, PB = NB, OP = kOpBytes<C>;
+  static_assert(kMi16<C> && C::BK == 64 && PA == TM && C::PB == 4 && NB >= 1 && NB <= 4, "16x16x32 schedule: 8-wavefront 256x256x64 tile, one load per row group");
   // request list of a sub-step by its parity P (0: a0, b0 .. b(NB-1), a1 ..; 1: a0 .. a(TM-1)), all compile time
   struct Ord {
     static constexpr int nr(int P) { return P == 0 ? TM + NB : TM; }
@@ -594,7 +595,7 @@ __device__ __forceinline__ void early_barrier_pipeline16(int nk_total, char* sme
       if constexpr (last) {
         if (next) {
           // my loads of step kt + 1 landed (of step kt + 2 the A loads may be in flight); my reads of step kt returned
-          if (!AHEAD || !more || (kt & (kStrictEvery - 1)) == 0) FGRPO_WAIT_VMCNT_LGKM0(0);
+          if (!AHEAD || !more || (NB == 4 && (kt & (kStrictEvery - 1)) == 0)) FGRPO_WAIT_VMCNT_LGKM0(0);
           else FGRPO_WAIT_VMCNT_LGKM0(PA);
           wg_barrier();                               // the buffers of step kt are free
         }
@@ -610,7 +611,7 @@ __device__ __forceinline__ void early_barrier_pipeline16(int nk_total, char* sme
         __builtin_amdgcn_sched_barrier(0);
         {
           // the row group's load: one operand's in the first sub-step, the other's behind the barrier
-          constexpr bool load_here = kk == 0 || last;
+          constexpr bool load_here = (AHEAD ? kk == 0 : last) || ((AHEAD ? last : kk == 0) && i < PB);
           constexpr int R = Ord::cum(1 - P, i + 1) - Ord::cum(1 - P, i);
           constexpr int X = R + (load_here ? 1 : 0);
           static_for<NB>([&](auto jcc) {
@@ -659,7 +660,8 @@ constexpr bool kSplitPrologue = C::DMA && C::NSTAGE == 2 && (C::BK / 16) % 2 == 
 
 // gemm_mainloop_dma on the 16x16x32 schedule.  MODE 2 requests what early_barrier_pipeline16 expects on entry and
 // leaves LDS buffers 2 and 3 (64 KiB from C::STAGE on) to the caller until the MODE 1 call.
-template <class C, int MODE>
+// NB < 4: the tile is 64 NB columns wide, 16 NB of them a wavefront's.
+template <class C, int MODE, int NB = 4>
 __device__ __forceinline__ void gemm_mainloop_dma16(const GemmOperands& g, int row0, int col0, char* smem,
                                                     f32x16_t (&acc)[C::TM][C::TN]) {
   static_assert(kMi16<C>, "16x16x32 MFMAs: 8-wavefront 256x256x64 two-buffer tile only");
@@ -669,7 +671,7 @@ __device__ __forceinline__ void gemm_mainloop_dma16(const GemmOperands& g, int r
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave / C::WN, wn = wave % C::WN;
   const int lrow = lane / C::CPR, lpc = lane % C::CPR;
-  uint32_t aoff[C::PA], boff[C::PB];
+  uint32_t aoff[C::PA], boff[NB];
   const int amax = g.M - 1 - row0, bmax = g.N - 1 - col0;
 #pragma unroll
   for (int i = 0; i < C::PA; ++i) {
@@ -678,7 +680,7 @@ __device__ __forceinline__ void gemm_mainloop_dma16(const GemmOperands& g, int r
     aoff[i] = (uint32_t)((long long)r * g.lda * 2 + ((lpc ^ lds_swizzle<C, true>(rt)) * 16));
   }
 #pragma unroll
-  for (int i = 0; i < C::PB; ++i) {
+  for (int i = 0; i < NB; ++i) {
     const int rt = (i * C::NW + wave) * C::RPI + lrow;
     const int r = rt < bmax ? rt : bmax;
     boff[i] = (uint32_t)((long long)r * g.ldb * 2 + ((lpc ^ lds_swizzle<C, true>(rt)) * 16));
@@ -742,7 +744,7 @@ __device__ __forceinline__ void gemm_mainloop_dma16(const GemmOperands& g, int r
   } else {
     if constexpr (MODE == 0) FGRPO_WAIT_VMCNT(0);      // the caller's own loads must not be mistaken for ours
     if (nk_total > 0) {
-      static_for<C::PB>([&](auto q) { load_lds(rsb, smem + mi16_b_buf(0) * kOpBytes<C>, decltype(q)::value, boff[decltype(q)::value], 0); });
+      static_for<NB>([&](auto q) { load_lds(rsb, smem + mi16_b_buf(0) * kOpBytes<C>, decltype(q)::value, boff[decltype(q)::value], 0); });
       static_for<C::PA>([&](auto q) { issue_a(smem, decltype(q)::value); });
     }
     if (nk_total > 1) static_for<C::PA>([&](auto q) { issue_a(smem + kOpBytes<C>, decltype(q)::value); });
@@ -752,11 +754,11 @@ __device__ __forceinline__ void gemm_mainloop_dma16(const GemmOperands& g, int r
   // fragments: lane l reads row (l % 16) of a 16-row block and the 16-byte chunk 4*k2 + l/16 of its 64-wide K slice (16
   // consecutive rows at one chunk index: conflict-free under the swizzle)
   const int sw16 = lds_swizzle<C, true>(lane & 15);
-  const int fa16 = (wm * C::WTM + (lane & 15)) * C::ROWB, fb16 = (wn * C::WTN + (lane & 15)) * C::ROWB;
+  const int fa16 = (wm * C::WTM + (lane & 15)) * C::ROWB, fb16 = (wn * 16 * NB + (lane & 15)) * C::ROWB;
   int fc16[2];
 #pragma unroll
   for (int k2 = 0; k2 < 2; ++k2) fc16[k2] = ((4 * k2 + (lane >> 4)) ^ sw16) * 16;
-  early_barrier_pipeline16<C, 1, 1, MODE == 1, true>(
+  early_barrier_pipeline16<C, NB, 1, 1, MODE == 1, true>(
       nk_total, smem, acc, true, issue_a, issue_b,
       [&](const char* st, auto i, auto kk) {
         constexpr int kkv = decltype(kk)::value;
@@ -764,16 +766,16 @@ __device__ __forceinline__ void gemm_mainloop_dma16(const GemmOperands& g, int r
       },
       [&](const char* st, auto jc, auto k2) {
         constexpr int jcv = decltype(jc)::value;
-        return lds_read_b128_asm<((jcv >> 1) * 32 + 16 * (jcv & 1)) * C::ROWB>(lds_addr(st) + fb16 + fc16[decltype(k2)::value]);
+        return lds_read_b128_asm<16 * jcv * C::ROWB>(lds_addr(st) + fb16 + fc16[decltype(k2)::value]);
       });
 }
 
-template <class C, int MODE = 0, bool MI16 = false>
+template <class C, int MODE = 0, bool MI16 = false, int NB = 4>
 __device__ __forceinline__ void gemm_mainloop_dma(const GemmOperands& g, int row0, int col0, char* smem,
                                                   f32x16_t (&acc)[C::TM][C::TN]) {
   static_assert(MODE == 0 || kSplitPrologue<C>, "split prologue needs the two-buffer schedule");
   if constexpr (MI16) {
-    gemm_mainloop_dma16<C, MODE>(g, row0, col0, smem, acc);
+    gemm_mainloop_dma16<C, MODE, NB>(g, row0, col0, smem, acc);
     return;
   }
   constexpr int D = C::NSTAGE - 1;              // K steps of loads in flight
@@ -1299,7 +1301,7 @@ __device__ __forceinline__ void gemm_mainloop_km(const GemmOperands& g, int row0
     static_for<C::PA>([&](auto q) { issue_a(smem, decltype(q)::value); });
   }
   if (nk_total > 1) static_for<C::PA>([&](auto q) { issue_a(smem + OP, decltype(q)::value); });
-  early_barrier_pipeline16<C, AKM ? 2 : 1, BKM ? 2 : 1, false, AHEAD>(
+  early_barrier_pipeline16<C, 4, AKM ? 2 : 1, BKM ? 2 : 1, false, AHEAD>(
       nk_total, smem, acc, wave_is_live<C>(g, row0, col0, wm, wn), issue_a, issue_b,
       [&](const char* st, auto ic, auto kc) -> bf16x8_t {
         constexpr int i = decltype(ic)::value, kk = decltype(kc)::value, k2 = kk >> 1, rh = kk & 1;

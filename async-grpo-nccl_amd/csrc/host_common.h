@@ -91,6 +91,7 @@ struct Tuning {
   int attn_dkv = 0;        // dK/dV kernel: 1 = one wavefront per 32 keys, 2 = a pair of wavefronts per 32 keys; 0 = four independent wavefronts on 64 keys
   int wide_stores = 1;     // GEMM epilogues write 16-byte pieces through an LDS patch where alignment allows
   int keep_skip_dead = 1;  // kept-path backward skips stretches of tokens that carry no gradient
+  int fwd_tail = 1;        // forward: a last token tile of at most 128 tokens is taken narrow
   int tail_split = 1;        // kept-path dHidden: last partial device round as a split contraction; forward: token regions
   int keep_panels = 0;     // kept-logits backward: vocabulary panels of the gradient GEMMs; 0 = one
 };

@@ -9,7 +9,7 @@ namespace fgrpo {
 namespace {
 template <class C>
 int launch_fwd(const FwdParams& p, hipStream_t st) {
-  return launch_tile_kernel<lmhead_fwd_kernel<C>, C>(p, p.tiles_t * p.nsplit, st);
+  return launch_tile_kernel<lmhead_fwd_kernel<C>, C>(p, p.tiles_t * p.nsplit + p.tail_split, st);
 }
 template <class C>
 int launch_ds(const DsParams& p, hipStream_t st) {
@@ -37,7 +37,7 @@ int launch_fwd_variant(int variant, const FwdParams& p, hipStream_t st) {
 }
 
 int launch_fwd_keep(const FwdParams& p, hipStream_t st) {
-  return launch_tile_kernel<lmhead_fwd_kernel<Cfg8, true>, Cfg8>(p, p.tiles_t * p.nsplit, st);
+  return launch_tile_kernel<lmhead_fwd_kernel<Cfg8, true>, Cfg8>(p, p.tiles_t * p.nsplit + p.tail_split, st);
 }
 
 int launch_ds_variant(int variant, bool split, const DsParams& p, hipStream_t st) {

@@ -49,6 +49,10 @@ struct FwdParams {
   float inv_temp;
   int tiles_v, tiles_t, nsplit, group_t;
   float4* part;              // [nsplit][T] : (m, s, sx, unused)
+  // The last tokens, if they are few: a tile 64 * tail_nb columns wide (tail_nb = 1 or 2) behind the tiles_t whole ones, its
+  // vocabulary dealt to tail_split work-groups behind the others.  tail_split = 0: no such tile.  Id 8 only.
+  int tail_nb, tail_split;
+  float4* part_tail;         // [tail_split][T - tiles_t * 256]
   float* xt;                 // [T] target logit (written only where a valid label exists)
   // KEEP kernels only: the soft-max numerators for the backward that does not recompute the logits,
   //   E[t, v] = exp(x_tv / temperature - ref_t)   (bf16; x = W h + b),
@@ -95,15 +99,15 @@ __device__ __forceinline__ void patch_write_quad16(char* patch, int lane_v, int 
   const int slot = ((i * 32 + 16 * rh) >> 2) + (lane_v >> 4);
   lds_write_b64_asm(lds_addr(patch) + tok * ROWP + ((slot ^ (tok & (NSLOT - 1) & 31)) << 3), v.x, v.y);
 }
-template <class C>
+template <class C, int TOK = 32>
 __device__ __forceinline__ void patch_flush(char* patch, bf16_t* out, int lane_v) {
   constexpr int ROWP = C::WTM * 2;
   constexpr int NSLOT = ROWP / 8;
   constexpr int PPT = ROWP / 16, TPP = 64 / PPT;         // 16-byte pieces per token, tokens per store instruction
-  static_assert(64 % PPT == 0 && 32 % TPP == 0 && (NSLOT & (NSLOT - 1)) == 0, "epilogue patch");
-  u32x4_t pv[32 / TPP];
+  static_assert(64 % PPT == 0 && TOK % TPP == 0 && (NSLOT & (NSLOT - 1)) == 0, "epilogue patch");
+  u32x4_t pv[TOK / TPP];
 #pragma unroll
-  for (int r = 0; r < 32 / TPP; ++r) {
+  for (int r = 0; r < TOK / TPP; ++r) {
     const int tok = r * TPP + lane_v / PPT, piece = lane_v % PPT;
     const int m = tok & (NSLOT - 1);
     pv[r] = __builtin_bit_cast(u32x4_t, lds_read_b128_asm<0>(lds_addr(patch) + tok * ROWP + ((piece ^ (m >> 1)) << 4)));
@@ -111,7 +115,7 @@ __device__ __forceinline__ void patch_flush(char* patch, bf16_t* out, int lane_v
   wait_lgkm<0>();
   __builtin_amdgcn_sched_barrier(0);     // nothing that consumes pv may move above the wait
 #pragma unroll
-  for (int r = 0; r < 32 / TPP; ++r) {
+  for (int r = 0; r < TOK / TPP; ++r) {
     const int tok = r * TPP + lane_v / PPT, piece = lane_v % PPT;
     const int m = tok & (NSLOT - 1);
     u32x4_t v = pv[r];
@@ -122,32 +126,21 @@ __device__ __forceinline__ void patch_flush(char* patch, bf16_t* out, int lane_v
   }
 }
 
-template <class C, bool KEEP = false>
-__global__ __launch_bounds__(C::NT, C::OCC) void lmhead_fwd_kernel(const FwdParams p) {
-  extern __shared__ __attribute__((aligned(16))) char smem[];
+// One work-group's walk: tokens from col0 on (64 NB of them on id 8, else the tile's width), vocabulary tiles vt_begin .. vt_end - 1;
+// part[c] takes token col0 + c's statistics.
+template <class C, bool KEEP, int NB>
+__device__ __forceinline__ void lmhead_fwd_walk(const FwdParams& p, char* smem, int col0, int vt_begin, int vt_end, float4* part) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = wave / C::WN, wn = wave % C::WN;
   const int V = p.g.M, T = p.g.N;
 
-  // block -> (token tile, vocabulary split); neighbours on one XCD share both
-  const int lid = xcd_contiguous_id(blockIdx.x, gridDim.x);
-  const int per_group = p.group_t * p.nsplit;
-  const int grp = lid / per_group;
-  const int first_t = grp * p.group_t;
-  const int gsz = (p.tiles_t - first_t) < p.group_t ? (p.tiles_t - first_t) : p.group_t;
-  const int w = lid - grp * per_group;
-  const int tt = first_t + w % gsz;
-  const int split = w / gsz;
-  const int vt_begin = (int)((long long)split * p.tiles_v / p.nsplit);
-  const int vt_end = (int)((long long)(split + 1) * p.tiles_v / p.nsplit);
-  const int col0 = tt * C::BN;
-
   // 16x16x32 MFMAs (kMi16): a lane holds two token columns (ch = 0, 1) of every 32-column block j, 32 vocabulary
   // values of each per tile; otherwise one column and 64 values.  Slot jc = j * NCL + ch.
   constexpr bool MI16 = kMi16<C>;
-  constexpr int NCL = MI16 ? 2 : 1, NS = C::TN * NCL;
+  constexpr int NCL = MI16 ? 2 : 1, NS = MI16 ? NB : C::TN;
+  constexpr int WCOL = MI16 ? 16 * NB : C::WTN, COLS = WCOL * C::WN;      // a wavefront's columns, the tile's
   auto slot_col = [&](int jc) {      // column of slot jc inside the tile
-    return MI16 ? wn * C::WTN + (jc >> 1) * 32 + 16 * (jc & 1) + (lane & 15) : acc_col<C>(wn, jc, lane);
+    return MI16 ? wn * WCOL + 16 * jc + (lane & 15) : acc_col<C>(wn, jc, lane);
   };
   float m_run[NS], s_run[NS], sx_run[NS];
   float ref2[NS];            // KEEP only
@@ -174,7 +167,7 @@ __global__ __launch_bounds__(C::NT, C::OCC) void lmhead_fwd_kernel(const FwdPara
   if constexpr (kSplitPrologue<C>) {
     if (vt_begin < vt_end) {
       f32x16_t none[C::TM][C::TN];
-      gemm_mainloop_dma<C, 2, MI16>(p.g, vt_begin * C::BM, col0, smem, none);
+      gemm_mainloop_dma<C, 2, MI16, NB>(p.g, vt_begin * C::BM, col0, smem, none);
     }
   }
   for (int vt = vt_begin; vt < vt_end; ++vt) {
@@ -182,8 +175,8 @@ __global__ __launch_bounds__(C::NT, C::OCC) void lmhead_fwd_kernel(const FwdPara
     f32x16_t acc[C::TM][C::TN];
     zero_acc<C>(acc);
     if constexpr (kSplitPrologue<C>) {
-      gemm_mainloop_dma<C, 1, MI16>(p.g, row0, col0, smem, acc);
-      if (vt + 1 < vt_end) gemm_mainloop_dma<C, 2, MI16>(p.g, row0 + C::BM, col0, smem, acc);
+      gemm_mainloop_dma<C, 1, MI16, NB>(p.g, row0, col0, smem, acc);
+      if (vt + 1 < vt_end) gemm_mainloop_dma<C, 2, MI16, NB>(p.g, row0 + C::BM, col0, smem, acc);
     } else {
       run_mainloop<C>(p.g, row0, col0, smem, acc);
     }
@@ -287,9 +280,10 @@ __global__ __launch_bounds__(C::NT, C::OCC) void lmhead_fwd_kernel(const FwdPara
       s_run[jc] = s;
       sx_run[jc] = sx;
       if constexpr (KEEP) {
-        if (jc % NCL == NCL - 1)          // the 32-token slab of block column j is complete
-          patch_flush<C>(patch, p.keep + (long long)vt * p.keep_blk + (long long)(col0 + wn * C::WTN + j * 32) * 256 + wm * C::WTM,
-                         lane_v);
+        // the slab of block column j (32 tokens, or the odd 16 of a narrow tile) is complete
+        bf16_t* out = p.keep + (long long)vt * p.keep_blk + (long long)(col0 + wn * WCOL + j * 32) * 256 + wm * C::WTM;
+        if (jc % NCL == NCL - 1) patch_flush<C>(patch, out, lane_v);
+        else if (jc == NS - 1) patch_flush<C, 16>(patch, out, lane_v);
       }
     }
   }
@@ -312,26 +306,52 @@ __global__ __launch_bounds__(C::NT, C::OCC) void lmhead_fwd_kernel(const FwdPara
     lse_merge(m_run[jc], s_run[jc], sx_run[jc], m2, s2, x2);
   }
   // wavefronts stacked along the vocabulary (same wn, different wm) meet in LDS
-  float* red = (float*)smem;  // [WM][BN][3]
+  float* red = (float*)smem;  // [WM][COLS][3]
   if (lane < (MI16 ? 16 : 32)) {
 #pragma unroll
     for (int jc = 0; jc < NS; ++jc) {
-      float* d = red + ((wm * C::BN) + slot_col(jc)) * 3;
+      float* d = red + (wm * COLS + slot_col(jc)) * 3;
       d[0] = m_run[jc];
       d[1] = s_run[jc];
       d[2] = sx_run[jc];
     }
   }
   __syncthreads();
-  for (int c = tid; c < C::BN; c += C::NT) {
+  for (int c = tid; c < COLS; c += C::NT) {
     float m = red[c * 3], s = red[c * 3 + 1], sx = red[c * 3 + 2];
     for (int q = 1; q < C::WM; ++q) {
-      const float* d = red + (q * C::BN + c) * 3;
+      const float* d = red + (q * COLS + c) * 3;
       lse_merge(m, s, sx, d[0], d[1], d[2]);
     }
-    const int n = col0 + c;
-    if (n < T) p.part[(long long)split * T + n] = make_float4(m, s, sx, 0.f);
+    if (col0 + c < T) part[c] = make_float4(m, s, sx, 0.f);
   }
+}
+
+template <class C, bool KEEP = false>
+__global__ __launch_bounds__(C::NT, C::OCC) void lmhead_fwd_kernel(const FwdParams p) {
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  const int T = p.g.N, whole = p.tiles_t * p.nsplit;
+  if constexpr (kMi16<C>) {
+    if ((int)blockIdx.x >= whole) {        // a share of the narrow last tile
+      const int split = (int)blockIdx.x - whole, t0 = p.tiles_t * C::BN;
+      const int b = (int)((long long)split * p.tiles_v / p.tail_split), e = (int)((long long)(split + 1) * p.tiles_v / p.tail_split);
+      float4* part = p.part_tail + (long long)split * (T - t0);
+      if (p.tail_nb == 1) lmhead_fwd_walk<C, KEEP, 1>(p, smem, t0, b, e, part);
+      else lmhead_fwd_walk<C, KEEP, 2>(p, smem, t0, b, e, part);
+      return;
+    }
+  }
+  // block -> (token tile, vocabulary split); neighbours on one XCD share both
+  const int lid = xcd_contiguous_id(blockIdx.x, whole);
+  const int per_group = p.group_t * p.nsplit;
+  const int grp = lid / per_group;
+  const int first_t = grp * p.group_t;
+  const int gsz = (p.tiles_t - first_t) < p.group_t ? (p.tiles_t - first_t) : p.group_t;
+  const int w = lid - grp * per_group;
+  const int tt = first_t + w % gsz;
+  const int split = w / gsz;
+  const int b = (int)((long long)split * p.tiles_v / p.nsplit), e = (int)((long long)(split + 1) * p.tiles_v / p.nsplit);
+  lmhead_fwd_walk<C, KEEP, 4>(p, smem, tt * C::BN, b, e, p.part + (long long)split * T + tt * C::BN);
 }
 
 // ---------------------------------------------------------------------------

@@ -14,6 +14,9 @@ struct CombineParams {
   const float* xt;
   const long long* labels;
   int T, V, nsplit;
+  // tokens from t_tail on have partials of their own, tail_split of them (FwdParams::part_tail); t_tail = T: none
+  const float4* part_tail;
+  int t_tail, tail_split;
   float* lp;    // [T]
   float* ent;   // [T] or null
   float* lse;   // [T] or null
@@ -30,11 +33,14 @@ __global__ __launch_bounds__(256) void lmhead_fwd_combine_kernel(const CombinePa
   const int tok = threadIdx.x % TOK, sub = threadIdx.x / TOK;
   const int n = blockIdx.x * TOK + tok;
   float m = -kNegBig, s = 0.f, sx = 0.f;
-  if (n < p.T && sub < p.nsplit) {
-    const float4 a = p.part[(long long)sub * p.T + n];
+  const bool tail = n >= p.t_tail;
+  const int nsplit = tail ? p.tail_split : p.nsplit, ld = tail ? p.T - p.t_tail : p.T;
+  const float4* part = tail ? p.part_tail + (n - p.t_tail) : p.part + n;
+  if (n < p.T && sub < nsplit) {
+    const float4 a = part[(long long)sub * ld];
     m = a.x, s = a.y, sx = a.z;
-    for (int k = sub + SUB; k < p.nsplit; k += SUB) {
-      const float4 b = p.part[(long long)k * p.T + n];
+    for (int k = sub + SUB; k < nsplit; k += SUB) {
+      const float4 b = part[(long long)k * ld];
       lse_merge(m, s, sx, b.x, b.y, b.z);
     }
   }
@@ -42,7 +48,7 @@ __global__ __launch_bounds__(256) void lmhead_fwd_combine_kernel(const CombinePa
     sm[threadIdx.x] = m, sm[256 + threadIdx.x] = s, sm[512 + threadIdx.x] = sx;
     __syncthreads();
     if (sub > 0) return;
-    const int last = p.nsplit < SUB ? p.nsplit : SUB;
+    const int last = nsplit < SUB ? nsplit : SUB;
     for (int u = 1; u < last; ++u) lse_merge(m, s, sx, sm[u * TOK + tok], sm[256 + u * TOK + tok], sm[512 + u * TOK + tok]);
   }
   float term = 0.f;
@@ -82,7 +88,7 @@ __global__ __launch_bounds__(256) void lmhead_fwd_combine_kernel(const CombinePa
 // kernels that wait for one another).
 template <bool LOSS>
 inline void launch_fwd_combine(const CombineParams& c, hipStream_t st) {
-  if (c.nsplit >= 8) hipLaunchKernelGGL((lmhead_fwd_combine_kernel<16, LOSS>), dim3((c.T + 15) / 16), dim3(256), 0, st, c);
+  if (c.nsplit >= 8 || c.tail_split >= 8) hipLaunchKernelGGL((lmhead_fwd_combine_kernel<16, LOSS>), dim3((c.T + 15) / 16), dim3(256), 0, st, c);
   else hipLaunchKernelGGL((lmhead_fwd_combine_kernel<1, LOSS>), dim3((c.T + 255) / 256), dim3(256), 0, st, c);
 }
 
