@@ -706,24 +706,27 @@ KeepAux keep_aux_of(void* keep, int T, int V) {
 // The pre-pass of the kept forward: the reference's sample of the vocabulary - the plain forward kernel over the
 // first rows of W; only the maxima of its per-split partials are used - then one dot product per token.
 // `p`: the forward's parameters for these tokens (operands staged, bias, labels, temperature); part: scratch for
-// min(kPrepassSplits, nsplit) x T partials.  A small batch takes the 128 x 128 tile: its few 256 x 256 tiles would each be
-// one serial walk over H on a device otherwise idle (777 tokens, H = 1536: 46 us; so 26), while more than two of
-// the small ones per CU gain nothing (32768 tokens: 53 us on the large).
-constexpr int kPrepassSplits = 4;
+// min(kPrepassSplits, nsplit) x T partials.  A small batch takes smaller tiles: its few large ones would each be one serial
+// walk over H on a device otherwise idle.  777 tokens, H = 1536: 256 x 256 46 us, 128 x 128 27, 64 x 64 with four K steps in
+// flight 16; up to two tiles of a kind per CU (32768 tokens: 53 us on the large).
+constexpr int kPrepassSplits = 8;
 int keep_prepass(const FwdParams& p, const void* hidden, const void* weight, const int64_t* labels, int T, int H, int V,
                  int nsplit, float4* part, const KeepAux& aux, int nflags, hipStream_t st) {
   FwdParams sp = p;
   const int vs = V < kKeepSampleRows ? V : kKeepSampleRows;
   sp.g.M = vs;
   sp.g.N = T;
-  const long long small_tiles = (long long)((vs + kCfg[4].bm - 1) / kCfg[4].bm) * ((T + kCfg[4].bn - 1) / kCfg[4].bn);
-  const int variant = small_tiles <= 2LL * num_cus() ? 4 : 8;
-  sp.tiles_v = (vs + kCfg[variant].bm - 1) / kCfg[variant].bm;
-  sp.tiles_t = (T + kCfg[variant].bn - 1) / kCfg[variant].bn;
-  sp.nsplit = sp.tiles_v < nsplit ? sp.tiles_v : nsplit;
+  auto tile = [&](int bm, int bn) {
+    sp.tiles_v = (vs + bm - 1) / bm;
+    sp.tiles_t = (T + bn - 1) / bn;
+    sp.nsplit = sp.tiles_v < nsplit ? sp.tiles_v : nsplit;
+    return (long long)sp.tiles_v * sp.tiles_t <= 2LL * num_cus();
+  };
   sp.part = part;
   sp.keep = nullptr;
-  int rc = launch_fwd_variant(variant, sp, st);
+  int rc = tile(CfgSample::BM, CfgSample::BN)     ? launch_fwd_sample(sp, st)
+           : tile(kCfg[4].bm, kCfg[4].bn)         ? launch_fwd_variant(4, sp, st)
+           : (tile(kCfg[8].bm, kCfg[8].bn), launch_fwd_variant(8, sp, st));
   if (rc) return rc;
   KeepRefParams r{(const bf16_t*)hidden, (const bf16_t*)weight, p.bias, (const long long*)labels, T, H, V, p.inv_temp,
                   part, sp.nsplit, aux.ref2, aux.xy, aux.flag, nflags};
@@ -1232,7 +1235,8 @@ struct KeptBwdSums {
 int kept_bwd_impl(const Tuning& tn, const void* hidden, const void* weight, const void* bias, const int64_t* labels,
                   const float* lse, const float* g, const float* gout_dev, float inv_temp, int T, int H, int V,
                   void* logits_keep, void* dH_out, void* dW_out, void* dbias_out, const KeptBwdSums& sums, void* ws,
-                  size_t ws_bytes, hipStream_t st, const KeepAux* aux_in = nullptr) {
+                  size_t ws_bytes, hipStream_t st, const KeepAux* aux_in = nullptr, const LossParams* loss = nullptr,
+                  int loss_parts = 0) {
   const bool want_dh = dH_out != nullptr, want_dw = dW_out != nullptr || sums.dw_out_f32 != nullptr;
   const bool want_db = dbias_out != nullptr || sums.db_out_f32 != nullptr;
   KeptBwdPlan pl;
@@ -1252,7 +1256,8 @@ int kept_bwd_impl(const Tuning& tn, const void* hidden, const void* weight, cons
     PhaseScope ph(kPhaseDlogits, st);
     KeepPrepParams k{ek, blk, aux.ref2, aux.xy, (const long long*)labels, lse, g, gout_dev, inv_temp,
                      (const bf16_t*)hidden, T, H, V, pl.row_scale, flag, want_dw ? pl.hidden_scaled : nullptr, kept_hs_ld(T), Tpad,
-                     skip_dead ? pl.k_runs : nullptr, skip_dead ? pl.m_tile_live : nullptr, (T + 63) / 64, Tpad / 64};
+                     skip_dead ? pl.k_runs : nullptr, skip_dead ? pl.m_tile_live : nullptr, (T + 63) / 64, Tpad / 64,
+                     loss_parts, loss ? *loss : LossParams()};
     launch_keep_backward_prep(k, st);
     HIP_TRY(hipGetLastError());
     {
@@ -1744,6 +1749,7 @@ int fgrpo_grpo_step_chunked(const void* hidden, const void* weight, const void* 
   lp.unclipped = unclipped;
   lp.clipped = clipped;
   lp.partial = pl.partial;
+  const int loss_parts = (T + kLossGroup - 1) / kLossGroup;
 
   {
     // references of the kept numerators for the tokens of every chunk, in one pass before the first chunk
@@ -1796,13 +1802,13 @@ int fgrpo_grpo_step_chunked(const void* hidden, const void* weight, const void* 
       }
       rc = kept_bwd_impl(tn, h_c, weight, bias, labels + t0, lse_out + t0, g_out + t0, nullptr, inv_temp, cnt, H, V,
                          pl.keep, dH_out ? (char*)dH_out + (size_t)t0 * H * esz : nullptr, dW_out, dbias_out, sums,
-                         pl.bwd_ws, pl.bwd_bytes, st, &aux);
+                         pl.bwd_ws, pl.bwd_bytes, st, &aux, last ? &lp : nullptr, last ? loss_parts : 0);
       if (rc) return rc;
     }
   }
-  {
+  if (!dH_out && !dW_out && !dbias_out) {      // else with the last chunk's preparation
     PhaseScope ph(kPhaseOther, st);
-    hipLaunchKernelGGL(grpo_loss_finalize_kernel, dim3(1), dim3(kLossThreads), 0, st, lp, (T + kLossGroup - 1) / kLossGroup);
+    hipLaunchKernelGGL(grpo_loss_finalize_kernel, dim3(1), dim3(kLossThreads), 0, st, lp, loss_parts);
     HIP_TRY(hipGetLastError());
   }
   return 0;
@@ -1915,6 +1921,15 @@ int fgrpo_build_labels(const int64_t* ids, const int32_t* tok_off, const int32_t
   HIP_TRY(hipGetLastError());
   hipLaunchKernelGGL(build_labels_kernel, dim3((nsamples + 3) / 4), dim3(256), 0, st, (const long long*)ids, tok_off,
                      in_len, out_len, nsamples, T, (long long*)labels_out);
+  HIP_TRY(hipGetLastError());
+  return 0;
+}
+
+int fgrpo_shift_labels(const int64_t* labels, long long rows, int L, int64_t* out, void* stream) {
+  if (!labels || !out || rows <= 0 || L <= 0 || rows * L >= (1LL << 40)) return fail(FGRPO_ERR_BAD_ARG, "shift_labels: bad argument");
+  const long long n = rows * L;
+  hipLaunchKernelGGL(shift_labels_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, (hipStream_t)stream, (const long long*)labels, n, L,
+                     (long long*)out);
   HIP_TRY(hipGetLastError());
   return 0;
 }

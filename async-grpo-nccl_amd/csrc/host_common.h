@@ -42,6 +42,9 @@ typedef TileCfg<256, 128, 32, 2, 2, 2, 3, true> Cfg7;
 typedef TileCfg<256, 256, 64, 2, 4, 2, 2, true> Cfg8;
 typedef TileCfg<256, 256, 32, 2, 4, 2, 5, true> Cfg9;
 constexpr int kNumCfg = 10;
+// The sample of the kept forward's pre-pass on small batches (keep_prepass): 64x64 tiles, four K steps of loads in flight,
+// two work-groups per CU.  No id: nothing else runs on it.
+typedef TileCfg<64, 64, 64, 2, 2, 2, 5, true> CfgSample;
 
 struct CfgInfo {
   int bm, bn, bk, nt, lds, wgs_per_cu;
@@ -127,6 +130,7 @@ int launch_tile_kernel(const P& p, int nblocks, hipStream_t st) {
 // lmhead_variant_built() accepts; the others are refused with FGRPO_ERR_UNSUPPORTED.
 bool lmhead_variant_built(int variant);
 int launch_fwd_variant(int variant, const FwdParams& p, hipStream_t st);
+int launch_fwd_sample(const FwdParams& p, hipStream_t st);      // on CfgSample
 // the forward that also keeps the bf16 logits (tile id 8 only)
 int launch_fwd_keep(const FwdParams& p, hipStream_t st);
 // split: fp32 inputs, dS written as bf16 hi + lo halves (small tile only)

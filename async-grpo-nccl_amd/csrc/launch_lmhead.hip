@@ -36,6 +36,8 @@ int launch_fwd_variant(int variant, const FwdParams& p, hipStream_t st) {
   DISPATCH_LMHEAD(variant, launch_fwd, p, st);
 }
 
+int launch_fwd_sample(const FwdParams& p, hipStream_t st) { return launch_fwd<CfgSample>(p, st); }
+
 int launch_fwd_keep(const FwdParams& p, hipStream_t st) {
   return launch_tile_kernel<lmhead_fwd_kernel<Cfg8, true>, Cfg8>(p, p.tiles_t * p.nsplit + p.tail_split, st);
 }

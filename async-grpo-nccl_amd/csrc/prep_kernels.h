@@ -322,6 +322,9 @@ struct KeepPrepParams {
   int* m_tile_live;          // [ceil(T / 256)]
   int n_chunks;              // ceil(T / 64), at most kLiveMaxChunks
   int k_steps;               // K steps of the dW product (round_up(T, 256) / 64)
+  // > 0: the last work-group adds that many block sums of the objective up to the loss (one launch less)
+  int loss_parts;
+  LossParams loss;
 };
 constexpr int kLiveMaxChunks = 32768;      // 2 M tokens: beyond that nothing is skipped (the lists say "all live")
 
@@ -434,6 +437,10 @@ __global__ __launch_bounds__(1024) void keep_backward_prep_kernel(const KeepPrep
     keep_live_runs(p, recompute, sm);
     return;
   }
+  if (p.loss_parts > 0 && blockIdx.x == gridDim.x - 1) {
+    grpo_loss_finalize(p.loss, p.loss_parts, *(FinalizeLds*)sm);
+    return;
+  }
   const int tiles_h = p.hidden_scaled != nullptr ? p.H / 64 : 1;
   const int grp = threadIdx.x >> 8, tid = threadIdx.x & 255;
   const long long id = (long long)((int)blockIdx.x - lists) * 4 + grp;
@@ -496,7 +503,7 @@ __global__ __launch_bounds__(1024) void keep_backward_prep_kernel(const KeepPrep
 
 inline void launch_keep_backward_prep(const KeepPrepParams& p, hipStream_t st) {
   const long long tiles = (long long)(p.Tpad / 64) * (p.hidden_scaled != nullptr ? p.H / 64 : 1);
-  hipLaunchKernelGGL(keep_backward_prep_kernel, dim3((unsigned)((tiles + 3) / 4) + (p.k_runs != nullptr ? 1 : 0)), dim3(1024), 0, st, p);
+  hipLaunchKernelGGL(keep_backward_prep_kernel, dim3((unsigned)((tiles + 3) / 4) + (p.k_runs != nullptr ? 1 : 0) + (p.loss_parts > 0 ? 1 : 0)), dim3(1024), 0, st, p);
 }
 
 // Sum of the ksplit fp32 slices a split contraction wrote (fixed order: bit-reproducible), times the row factor,

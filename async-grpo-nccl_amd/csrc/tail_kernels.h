@@ -162,6 +162,12 @@ __global__ void build_labels_kernel(const long long* ids, const int* tok_off, co
   }
 }
 
+// Next-token targets of rows of L labels: the row one to the left, -100 in its last column.
+__global__ __launch_bounds__(256) void shift_labels_kernel(const long long* labels, long long n, int L, long long* out) {
+  const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
+  if (i < n) out[i] = (i + 1) % L != 0 ? labels[i + 1] : -100;
+}
+
 // cu_seqlens from position ids: ordered list of the indices t with pos[t] == 0,
 // followed by T.  A single work-group walks the array in order, eight
 // consecutive tokens per thread and round; the rank of a hit is the prefix of
@@ -343,22 +349,27 @@ __global__ __launch_bounds__(kLossThreads) void grpo_loss_tokens_kernel(const Lo
 // kFinalizeBlocks blocks, so the partials are re-read that many times at most)
 // by the normaliser; block 0 publishes the scalars.
 constexpr int kFinalizeBlocks = 256;
-__global__ __launch_bounds__(kLossThreads) void grpo_loss_finalize_kernel(const LossParams p, int nparts) {
-  __shared__ double part[3][kLossThreads / 64];
-  __shared__ double tot[3];
+// The first kLossThreads threads of a work-group work, all of them pass the barriers.
+struct FinalizeLds {
+  double part[3][kLossThreads / 64], tot[3];
+};
+__device__ __forceinline__ void grpo_loss_finalize(const LossParams& p, int nparts, FinalizeLds& sm) {
+  auto& part = sm.part;
+  auto& tot = sm.tot;
+  const bool on = threadIdx.x < kLossThreads;
   {
     // all four wavefronts add their strided share, then one thread adds the four results: a fixed order
     double a = 0.0, b = 0.0, ne = 0.0;
-    for (int i = threadIdx.x; i < nparts; i += kLossThreads) {
+    for (int i = threadIdx.x; on && i < nparts; i += kLossThreads) {
       a += p.partial[2 * i];
       b += p.partial[2 * i + 1];
     }
     if (p.seg_cnt)
-      for (int i = threadIdx.x; i < p.nseq; i += kLossThreads) ne += (p.seg_cnt[i] > 0) ? 1.0 : 0.0;
+      for (int i = threadIdx.x; on && i < p.nseq; i += kLossThreads) ne += (p.seg_cnt[i] > 0) ? 1.0 : 0.0;
     a = wave_sum_d(a);
     b = wave_sum_d(b);
     ne = wave_sum_d(ne);
-    if ((threadIdx.x & 63) == 0) {
+    if (on && (threadIdx.x & 63) == 0) {
       part[0][threadIdx.x >> 6] = a;
       part[1][threadIdx.x >> 6] = b;
       part[2][threadIdx.x >> 6] = ne;
@@ -381,10 +392,10 @@ __global__ __launch_bounds__(kLossThreads) void grpo_loss_finalize_kernel(const 
     nonempty = p.pre[2];
   }
   const float norm = (float)(1.0 / den);
-  if (!p.pre)
+  if (!p.pre && on)
     for (long long t = (long long)blockIdx.x * kLossThreads + threadIdx.x; t < p.T; t += (long long)gridDim.x * kLossThreads)
       p.g[t] *= norm;
-  if (blockIdx.x == 0 && threadIdx.x == 0) {
+  if ((blockIdx.x == 0 || p.pre) && threadIdx.x == 0) {
     *p.loss = (float)(tot[0] / den);
     if (p.scal) {
       p.scal[0] = norm;
@@ -393,6 +404,10 @@ __global__ __launch_bounds__(kLossThreads) void grpo_loss_finalize_kernel(const 
       p.scal[3] = (float)tot[0];
     }
   }
+}
+__global__ __launch_bounds__(kLossThreads) void grpo_loss_finalize_kernel(const LossParams p, int nparts) {
+  __shared__ FinalizeLds sm;
+  grpo_loss_finalize(p, nparts, sm);
 }
 
 // The normaliser of the objective depends on the labels and the segments only: valid tokens (token mean), segments

@@ -41,6 +41,7 @@ struct Api {
   FGRPO_ENTRY(fgrpo_grpo_step_chunked_workspace);
   FGRPO_ENTRY(fgrpo_grpo_step_chunked);
   FGRPO_ENTRY(fgrpo_scale_gradients);
+  FGRPO_ENTRY(fgrpo_shift_labels);
   FGRPO_ENTRY(fgrpo_varlen_attn_workspace);
   FGRPO_ENTRY(fgrpo_varlen_attn_fwd_ws);
   FGRPO_ENTRY(fgrpo_varlen_attn_bwd_ws);
@@ -70,6 +71,7 @@ void init(const std::unordered_map<std::string, uint64_t>& at) {
   FGRPO_SET(fgrpo_grpo_step_chunked_workspace);
   FGRPO_SET(fgrpo_grpo_step_chunked);
   FGRPO_SET(fgrpo_scale_gradients);
+  FGRPO_SET(fgrpo_shift_labels);
   FGRPO_SET(fgrpo_varlen_attn_workspace);
   FGRPO_SET(fgrpo_varlen_attn_fwd_ws);
   FGRPO_SET(fgrpo_varlen_attn_bwd_ws);
@@ -292,6 +294,18 @@ struct FusedStep : torch::autograd::Function<FusedStep> {
   }
 };
 
+// labels [..., L], int64, contiguous -> next-token targets, -100 in the last column
+Tensor shift_labels(const Tensor& labels) {
+  TORCH_CHECK(labels.is_cuda() && labels.scalar_type() == at::kLong && labels.is_contiguous() && labels.dim() > 0, "fgrpo: labels must be contiguous int64 on the GPU");
+  Tensor out = at::empty_like(labels);
+  if (labels.numel() == 0) return out;
+  OnDevice d(labels);
+  const int64_t L = labels.size(-1);
+  TORCH_CHECK(L < (1LL << 31), "fgrpo: rows of ", L, " labels");
+  check(api.fgrpo_shift_labels(labels.data_ptr<int64_t>(), labels.numel() / L, (int)L, out.data_ptr<int64_t>(), d.stream()), "shift_labels");
+  return out;
+}
+
 // mode: 0 "auto", 1 "recompute", 2 "whole", 3 "chunked" (what the gradients come from, where one is wanted)
 variable_list fused_step(const Tensor& hidden, const Tensor& weight, const std::optional<Tensor>& bias_, const Tensor& labels,
                          const std::optional<Tensor>& old_lp, const Tensor& adv, const std::optional<Tensor>& ref_lp,
@@ -482,6 +496,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("init", &init);
   m.def("fill_list", &fill_list);
   // without the interpreter lock: a call may wait, for memory or for room in a full launch queue, and other threads run
+  m.def("shift_labels", &shift_labels, py::call_guard<py::gil_scoped_release>());
   m.def("fused_step", &fused_step, py::call_guard<py::gil_scoped_release>());
   m.def("varlen_attention", &varlen_attention, py::call_guard<py::gil_scoped_release>());
 }

@@ -266,6 +266,9 @@ int fgrpo_segment_broadcast(const void* values, int values_f64, const int32_t* c
 int fgrpo_segment_reduce(const float* x, const int64_t* labels, const int32_t* cu_seqlens, int nseq,
                          int T, float* sum_out, float* mean_out, int32_t* count_out, void* stream);
 
+/* Next-token targets: out[r][i] = labels[r][i + 1], -100 in the last column of every row ([rows][L] int64, contiguous). */
+int fgrpo_shift_labels(const int64_t* labels, long long rows, int L, int64_t* out, void* stream);
+
 /* ---- batch shaping --------------------------------------------------------------
  * fgrpo_output_indices replaces get_output_logits_indices_numba
  * (sample_processing_utils.py:29-67): sample i, packed at token offset
