@@ -8,6 +8,7 @@ from __future__ import annotations
 
 from typing import Optional, Tuple
 
+import numpy as np
 import torch
 from torch.autograd import forward_ad
 
@@ -389,24 +390,26 @@ def segment_reduce(x: torch.Tensor, cu_seqlens: torch.Tensor, labels_shifted: Op
     return s, m, c
 
 
-def output_indices(input_lens, output_lens, device) -> torch.Tensor:
-    """int64 positions of the logits scoring every generated token (see fgrpo_output_indices)."""
+def output_indices_pack(input_lens, output_lens) -> np.ndarray:
+    """What the kernel behind ``output_indices`` reads, int32: token offsets [n], input lengths [n], output offsets [n + 1]."""
+    il = np.asarray(input_lens, dtype=np.int64).reshape(-1)
+    ol = np.asarray(output_lens, dtype=np.int64).reshape(-1)
+    if il.size and int((il + ol).sum()) >= 2 ** 31:
+        raise RuntimeError("fgrpo: packed batch longer than 2^31 tokens")
+    return np.concatenate([np.cumsum(il + ol) - (il + ol), il, [0], np.cumsum(ol)]).astype(np.int32)
+
+
+def output_indices(input_lens, output_lens, device, pack: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """int64 positions of the logits scoring every generated token (see fgrpo_output_indices).  ``pack``: what
+    ``output_indices_pack`` gives for the same lengths, already on the device."""
     lib = _lib.load()
-    il = torch.as_tensor(input_lens, dtype=torch.int64).reshape(-1)
-    ol = torch.as_tensor(output_lens, dtype=torch.int64).reshape(-1)
-    n = il.numel()
-    tok_off = torch.zeros(n, dtype=torch.int64)
-    out_off = torch.zeros(n + 1, dtype=torch.int64)
-    if n:
-        tok_off[1:] = torch.cumsum(il + ol, 0)[:-1]
-        out_off[1:] = torch.cumsum(ol, 0)
-    total = int(out_off[-1])
+    ol = np.asarray(output_lens, dtype=np.int64)
+    n, total = int(np.size(input_lens)), int(ol.sum())
     out = torch.empty(total, dtype=torch.int64, device=device)
     if n == 0 or total == 0:
         return out
-    if int((il + ol).sum()) >= 2 ** 31:
-        raise RuntimeError("fgrpo: packed batch longer than 2^31 tokens")
-    pack = torch.cat([tok_off.to(torch.int32), il.to(torch.int32), out_off.to(torch.int32)]).to(device)
+    if pack is None:
+        pack = torch.from_numpy(output_indices_pack(input_lens, ol)).to(device)
     with torch.cuda.device(device):
         rc = lib.fgrpo_output_indices(pack.data_ptr(), pack.data_ptr() + 4 * n, pack.data_ptr() + 8 * n, n,
                                       total, _ptr(out), _stream())
