@@ -1515,6 +1515,11 @@ int fgrpo_loss_fwd(const float* lp, const float* old_lp, const float* ref_lp, co
   p.clipped = clipped;
   p.loss = loss_out;
   p.scal = scal_out;
+  if (T <= kSmallLossTokens && (agg_mode != FGRPO_AGG_SAMPLE_MEAN || nseq <= kSmallLossTokens)) {
+    hipLaunchKernelGGL(grpo_loss_small_kernel, dim3(1), dim3(1024), 0, st, p, cu, nseq);
+    HIP_TRY(hipGetLastError());
+    return 0;
+  }
   if (agg_mode == FGRPO_AGG_SAMPLE_MEAN) {
     launch_segment_weights(p.labels, cu, nseq, T, segc, tokw, st);
     HIP_TRY(hipGetLastError());

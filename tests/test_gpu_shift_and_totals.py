@@ -38,3 +38,45 @@ def test_loss_is_the_same_with_and_without_gradients(dev, T, chunk):
     assert abs(float(loss.detach()) - float(want)) <= 1e-6 + 1e-6 * abs(float(want))
     dh, = torch.autograd.grad(loss, h)
     assert torch.isfinite(dh).all()
+
+
+@pytest.mark.parametrize("T,bounds", [(1, [0, 1]), (63, [0, 10, 10, 63]), (1024, [0, 1000, 1024]), (1025, [3, 700, 1020]), (2047, [0, 2047]),
+                                      (2048, list(range(0, 2049, 8))), (2049, [0, 5, 2049]), (2048, [0, 3000]), (700, [600, 50, 650])])
+@pytest.mark.parametrize("mode", ["token_mean", "sample_mean"])
+@pytest.mark.parametrize("denom", [0.0, 7.0])
+def test_objective_of_a_small_batch(dev, T, bounds, mode, denom):
+    """One work-group up to 2048 tokens, three launches beyond: the same formula in fp64 from the same log-probabilities.
+    Weights, ratios and products are fp32: a dozen roundings, 2e-6 of the largest term."""
+    from fgrpo import ops
+    g = torch.Generator(device=dev).manual_seed(T)
+    r = lambda s=1.0: torch.randn(T, generator=g, device=dev) * s
+    lp, adv = r(0.3) - 3, r()
+    old, ref = lp + r(0.2), lp + r(0.2)
+    y = torch.randint(0, 9, (T,), generator=g, device=dev)
+    y[torch.rand(T, generator=g, device=dev) < 0.3] = -100
+    cu = torch.tensor(bounds, dtype=torch.int32, device=dev)
+    loss, gr, lr, c1, l1, l2, scal = ops.grpo_loss_fwd(lp, old, ref, adv, y, cu, 0.2, 0.28, 3.0, 0.01, mode, denom)
+    on = (y != -100).double()
+    w, full = torch.zeros_like(on), 0
+    if mode == "sample_mean":
+        for a, b in zip(bounds, bounds[1:]):
+            a, b = max(a, 0), min(b, T)
+            n = float(on[a:b].sum()) if b > a else 0.0
+            if n > 0:
+                w[a:b], full = 1.0 / n, full + 1
+    else:
+        w, full = w + 1, float(on.sum())
+    den = max(denom if denom > 0 else float(full), 1.0)
+    x = lp.double().requires_grad_(True)
+    ratio, a = torch.exp(x - old.double()), adv.double()
+    u, v = -a * ratio, -a * ratio.clamp(0.8, 1.28)
+    m = torch.maximum(u, v)
+    tok = torch.where(a < 0, torch.minimum(m, -a * 3.0), m)
+    d = ref.double() - x
+    tok = tok + 0.01 * (torch.exp(d) - d - 1)
+    want = (w * on * tok).sum() / den
+    gw, = torch.autograd.grad(want, x)
+    big = float((w * on * tok.detach().abs()).sum()) / den + 1e-12
+    assert abs(float(loss) - float(want.detach())) <= 2e-6 * big + 1e-9
+    assert (gr.double() - gw).abs().max() <= 2e-6 * float(gw.abs().max()) + 1e-12
+    assert float(scal[1]) == float(on.sum())
