@@ -214,10 +214,20 @@ long long split_cost(int tiles_t, int tiles_v, int slots, int s) {
   return rounds * per;
 }
 
+// The same in quarters of a tile, a round itself counted as three of them: a work-group opens and closes, and one that
+// replaces another is no longer in step with those it shares W's and hidden's slices with.  Plain forward, V of about 152k, the
+// share that is least without | with the rounds counted, us: H = 1536, 27 token tiles: 46 splits (5 rounds of 13 tiles) 2498 | 9
+// (one of 66) 2390, 35: 29 | 7 3190 | 3122, 41: 43 | 6 3808 | 3583; H = 3584: 27 5578 | 5330, 35 7170 | 6997, 41 8650 | 8020;
+// H = 5120: 28 8055 | 7710, 41 12440 | 11280; H = 896 and the sizes whose choice stays: within 1 %.  By these a round costs 0.6 ..
+// 1.1 tiles.
+long long rounds_cost(int tiles_t, int tiles_v, int slots, int s) {
+  return 4 * split_cost(tiles_t, tiles_v, slots, s) + 3 * (((long long)tiles_t * s + slots - 1) / slots);
+}
+
 int choose_nsplit(int tiles_t, int tiles_v, int slots, int forced, int prefer = 4, int max_split = 64) {
   if (forced > 0) return forced < tiles_v ? forced : tiles_v;
   int best = 1;
-  long long best_cost = -1;
+  long long best_cost = -1, least = -1;
   // Token tiles that 64 splits do not make a round of the device of (under slots / 64: three tiles of 256, seven of the
   // 128-wide configuration, whose work-groups share a CU) take as many splits as one round holds; at 64 they left up to three
   // quarters of it idle (kept forward, H = 1536, V = 151936: 200 tokens 440 -> 161 us, 500 451 -> 247, 700 461 -> 340).  More
@@ -231,11 +241,9 @@ int choose_nsplit(int tiles_t, int tiles_v, int slots, int forced, int prefer = 
   const int cap = tiles_v < max_split ? tiles_v : max_split;
   auto cost_of = [&](int s) { return split_cost(tiles_t, tiles_v, slots, s); };
   for (int s = 1; s <= cap; ++s) {
-    const long long cost = cost_of(s);
-    if (best_cost < 0 || cost < best_cost) {
-      best_cost = cost;
-      best = s;
-    }
+    const long long cost = cost_of(s), with_rounds = rounds_cost(tiles_t, tiles_v, slots, s);
+    if (best_cost < 0 || cost < best_cost) best_cost = cost;
+    if (least < 0 || with_rounds < least) least = with_rounds, best = s;
   }
   // Four splits x eight token tiles (the default raster group) put 32 work-groups = one XCD on an 8 x 4
   // patch of (token tile, vocabulary range): every W slice fetched into that XCD's L2 serves 8 work-groups and
@@ -276,7 +284,7 @@ int tail_columns(const Tuning& tn, int variant, int T) {        // NB, or 0 wher
 struct TailPlan {
   int nsplit = 0, tail_split = 0;
 };
-// Shares of the whole tiles and of the narrow one: the cheapest by device rounds x vocabulary tiles of a whole-tile work-group.
+// Shares of the whole tiles and of the narrow one, the cheapest by rounds_cost.
 TailPlan plan_tail(int tiles, int nb, int tiles_v, int slots, int prefer, long long* cost_out) {
   TailPlan best;
   long long least = -1;
@@ -285,7 +293,7 @@ TailPlan plan_tail(int tiles, int nb, int tiles_v, int slots, int prefer, long l
     int share = (int)(per / kTailCost[nb]);
     if (share < 1) share = 1;
     const int nt = tiles > 0 ? (tiles_v + share - 1) / share : ns;
-    const long long blocks = (long long)tiles * ns + nt, cost = (blocks + slots - 1) / slots * per;
+    const long long rounds = ((long long)tiles * ns + nt + slots - 1) / slots, cost = rounds * (4 * per + 3);      // as rounds_cost
     if (least < 0 || cost < least) least = cost, best.nsplit = ns, best.tail_split = nt;
     return cost;
   };
@@ -331,8 +339,8 @@ void plan_fwd(const Tuning& tn, FwdPlan& pl, void* ws, int T, int H, int V, int 
     if (main_tiles > 0 && main_tiles < pl.tiles_t) {
       const int rem_tiles = pl.tiles_t - main_tiles;
       const int ns_rem = choose_nsplit(rem_tiles, pl.tiles_v, slots, 0, prefer, 128);
-      const long long two = split_cost(main_tiles, pl.tiles_v, slots, prefer) + split_cost(rem_tiles, pl.tiles_v, slots, ns_rem);
-      if (two * 100 <= split_cost(pl.tiles_t, pl.tiles_v, slots, pl.nsplit) * 110) {
+      const long long two = rounds_cost(main_tiles, pl.tiles_v, slots, prefer) + rounds_cost(rem_tiles, pl.tiles_v, slots, ns_rem);
+      if (two * 100 <= rounds_cost(pl.tiles_t, pl.tiles_v, slots, pl.nsplit) * 110) {
         pl.nsplit = prefer;
         pl.t_main = main_tiles * c.bn;
         pl.nsplit_rem = ns_rem;
@@ -346,7 +354,7 @@ void plan_fwd(const Tuning& tn, FwdPlan& pl, void* ws, int T, int H, int V, int 
     int& ns = pl.t_main < T ? pl.nsplit_rem : pl.nsplit;
     long long cost = 0;
     const TailPlan t = plan_tail(tiles, pl.tail_nb, pl.tiles_v, slots, prefer, &cost);
-    if (tiles == 0 || cost < split_cost(tiles + 1, pl.tiles_v, slots, ns)) ns = t.nsplit, pl.tail_split = t.tail_split;
+    if (tiles == 0 || cost < rounds_cost(tiles + 1, pl.tiles_v, slots, ns)) ns = t.nsplit, pl.tail_split = t.tail_split;
     else pl.tail_nb = 0;
   }
   pl.Hp = (int)round_up(H, 64);
@@ -1568,7 +1576,7 @@ double chunk_cost_estimate(int cnt, int H, int V) {
   const int tiles_t = (cnt + 255) / 256, tiles_v = (V + 255) / 256, tiles_h = (H + 255) / 256;
   const int prefer = (16384LL * H * 2 > (192LL << 20)) ? 8 : 4;
   const int ns = choose_nsplit(tiles_t, tiles_v, slots, 0, prefer);
-  const double fwd = (double)split_cost(tiles_t, tiles_v, slots, ns) * (H / 64.0 + 5.0);
+  const double fwd = (double)rounds_cost(tiles_t, tiles_v, slots, ns) / 4 * (H / 64.0 + 5.0);
   double dh_rounds = 0.0;
   (void)plan_tail_split(cnt, H, (int)round_up(V, 256), &dh_rounds);
   const double dh = dh_rounds * (round_up(V, 256) / 64.0 + 8.0);
