@@ -71,59 +71,47 @@ struct FwdParams {
 
 constexpr float kKeepHeadroom2 = 120.f;   // log2 units: exp2(120) * (values <= 1) stays finite in bf16 / fp32
 
-// One 32-token x WTM-entry slab of bf16 values (the sub-tile column block j of a wavefront in the LM-head
-// orientation: lane = token, 16 vocabulary rows per 32x32 block) written to a column-blocked buffer through the
-// wavefront's private LDS patch: a lane's 8 bytes (4 vocabulary entries of one token) would be a 64-line scatter per
-// store instruction; parked in the patch and read back as 16-byte pieces, PPT lanes per token row, every store
-// instruction fills whole 128-byte lines.  Patch rows are unpadded; the 8-byte slots of row n are XOR-swizzled with
-// n so that the 32 lanes of a write hit 32 different slots.  LDS traffic is inline assembly (the compiler would
+// One 32-token x WTM-entry slab of bf16 values (the sub-tile column block j of a wavefront in the LM-head orientation, 16x16x32
+// accumulators: a lane holds two tokens, 4 consecutive vocabulary entries of each per quad) written to a column-blocked buffer
+// through the wavefront's private LDS patch: a lane's 8 bytes would be a 64-line scatter per store instruction; parked in the patch
+// and read back as 16-byte pieces, 16 lanes per token row, every store instruction fills whole 128-byte lines.  Patch rows are
+// 256 bytes, unpadded; row n's pieces are XORed with n % 16, so that the half-wave of a write covers all banks once and the two
+// quads of a piece stay in order.  These instructions stand between a tile's matrix work, with nothing beside them: a quad costs
+// one address instruction (a lane constant XORed with the quad's, added to the row: the token half sits in the offset field), a
+// piece costs none (four addresses per lane, a uniform base for the stores): 468 vector instructions for 64 elements a lane
+// where XORed 8-byte slots, swapped back on the way out, took 588 (forward that keeps: H = 896, 6872 tokens 1815 -> 1796 us; H =
+// 1536, 1500 tokens 720 -> 700, 16384 6147 -> 6124).  LDS traffic is inline assembly (the compiler would
 // otherwise wait for the direct-to-LDS loads of the next tile that are in flight); LDS operations of one wavefront
-// complete in order, so one wait before the stores is enough.  `out` points at (first token of the slab, first
+// complete in order, so one wait before the stores is enough.  `out` (uniform) points at (first token of the slab, first
 // vocabulary entry of the wavefront's rows) in the block.
-// patch_write_quad: entries i*32 + 8*q + 4*(lane/32) + 0..3 of this lane's token (8 bytes) into the patch;
+// patch_write_quad16: entries i*32 + 16*rh + 4*(lane/16) + 0..3 of token 16*ch + lane%16 into the patch;
 // patch_flush: the whole slab out, after every quad of the slab has been written.
 template <class C>
-__device__ __forceinline__ void patch_write_quad(char* patch, int lane_v, int i, int q, uint2 v) {
-  constexpr int ROWP = C::WTM * 2;                       // patch row: one token's WTM entries
-  constexpr int NSLOT = ROWP / 8;                        // 8-byte slots per row
-  const int slot = ((i * 32 + 8 * q) >> 2) + (lane_v >> 5);
-  lds_write_b64_asm(lds_addr(patch) + (lane_v & 31) * ROWP + ((slot ^ (lane_v & (NSLOT - 1) & 31)) << 3), v.x, v.y);
-}
-// the same for the 16x16x32 accumulator layout: the lane's token is row 16*ch + lane%16 of the slab and the quad holds
-// its entries i*32 + 16*rh + 4*(lane/16) + 0..3
-template <class C>
 __device__ __forceinline__ void patch_write_quad16(char* patch, int lane_v, int ch, int i, int rh, uint2 v) {
-  constexpr int ROWP = C::WTM * 2;
-  constexpr int NSLOT = ROWP / 8;
-  const int tok = 16 * ch + (lane_v & 15);
-  const int slot = ((i * 32 + 16 * rh) >> 2) + (lane_v >> 4);
-  lds_write_b64_asm(lds_addr(patch) + tok * ROWP + ((slot ^ (tok & (NSLOT - 1) & 31)) << 3), v.x, v.y);
+  static_assert(C::WTM == 128, "patch rows of 256 bytes");
+  const uint32_t row = lds_addr(patch) + ((lane_v & 15) << 8);
+  const uint32_t at = (((lane_v >> 4) << 3) ^ ((lane_v & 15) << 4)) ^ (uint32_t)(64 * i + 32 * rh);
+  if (ch == 0) lds_write_b64_asm<0>(row + at, v.x, v.y);
+  else lds_write_b64_asm<16 * 256>(row + at, v.x, v.y);
 }
 template <class C, int TOK = 32>
 __device__ __forceinline__ void patch_flush(char* patch, bf16_t* out, int lane_v) {
-  constexpr int ROWP = C::WTM * 2;
-  constexpr int NSLOT = ROWP / 8;
-  constexpr int PPT = ROWP / 16, TPP = 64 / PPT;         // 16-byte pieces per token, tokens per store instruction
-  static_assert(64 % PPT == 0 && TOK % TPP == 0 && (NSLOT & (NSLOT - 1)) == 0, "epilogue patch");
-  u32x4_t pv[TOK / TPP];
-#pragma unroll
-  for (int r = 0; r < TOK / TPP; ++r) {
-    const int tok = r * TPP + lane_v / PPT, piece = lane_v % PPT;
-    const int m = tok & (NSLOT - 1);
-    pv[r] = __builtin_bit_cast(u32x4_t, lds_read_b128_asm<0>(lds_addr(patch) + tok * ROWP + ((piece ^ (m >> 1)) << 4)));
-  }
+  static_assert(C::WTM == 128 && TOK % 16 == 0 && TOK <= 32, "patch rows of 256 bytes");
+  // read r takes tokens 4 r .. 4 r + 3, a row per 16 lanes
+  const uint32_t row = lds_addr(patch) + ((lane_v >> 4) << 8), at = ((lane_v & 15) ^ (lane_v >> 4)) << 4;
+  u32x4_t pv[TOK / 4];
+  static_for<TOK / 4>([&](auto rc) {
+    constexpr int r = decltype(rc)::value;
+    pv[r] = __builtin_bit_cast(u32x4_t, lds_read_b128_asm<r * 1024>(row + (at ^ ((r & 3) << 6))));
+  });
   wait_lgkm<0>();
   __builtin_amdgcn_sched_barrier(0);     // nothing that consumes pv may move above the wait
+  const uint32_t off = (uint32_t)((lane_v >> 4) * 512 + (lane_v & 15) * 16);
 #pragma unroll
-  for (int r = 0; r < TOK / TPP; ++r) {
-    const int tok = r * TPP + lane_v / PPT, piece = lane_v % PPT;
-    const int m = tok & (NSLOT - 1);
-    u32x4_t v = pv[r];
-    if (m & 1) v = u32x4_t{v[2], v[3], v[0], v[1]};       // odd rows hold the two slots of a piece swapped
+  for (int r = 0; r < TOK / 4; ++r)
     // non-temporal: the buffer is written once and read by a later launch; stored normally its 10 GB push the
     // operand tiles out of the L2s (forward kernel at T=32768, H=1536, V=151936: 14.46 ms, non-temporal 12.65)
-    __builtin_nontemporal_store(v, (u32x4_t*)(out + (long long)tok * 256 + piece * 8));
-  }
+    __builtin_nontemporal_store(pv[r], (u32x4_t*)((char*)(out + r * 4 * 256) + off));
 }
 
 // One work-group's walk: tokens from col0 on (64 NB of them on id 8, else the tile's width), vocabulary tiles vt_begin .. vt_end - 1;
@@ -158,9 +146,10 @@ __device__ __forceinline__ void lmhead_fwd_walk(const FwdParams& p, char* smem, 
 
   // KEEP: the wavefront's patch lives behind LDS buffer 0, which the prefetch of the next tile may already be filling
   constexpr int KEEP_PATCH = C::NW * 32 * C::WTM * 2;
-  static_assert(!KEEP || (kSplitPrologue<C> && C::BM == 256 && C::STAGE + KEEP_PATCH <= C::LDS_BYTES),
+  static_assert(!KEEP || (MI16 && kSplitPrologue<C> && C::BM == 256 && C::STAGE + KEEP_PATCH <= C::LDS_BYTES),
                 "kept logits: 256-row tiles on the two-buffer direct-to-LDS loop");
-  char* patch = smem + C::STAGE + wave * (32 * C::WTM * 2);
+  const int wave_u = __builtin_amdgcn_readfirstlane(wave);
+  char* patch = smem + C::STAGE + wave_u * (32 * C::WTM * 2);
 
   // With the two-buffer direct-to-LDS loop the first K slice of the NEXT vocabulary tile is requested before this
   // tile's statistics are folded in, so its latency hides under that arithmetic.
@@ -267,10 +256,7 @@ __device__ __forceinline__ void lmhead_fwd_walk(const FwdParams& p, char* smem, 
           uint2 pk;
           pk.x = pack_bf16x2(ek[0], ek[1]);
           pk.y = pack_bf16x2(ek[2], ek[3]);
-          if constexpr (MI16)
-            patch_write_quad16<C>(patch, lane_v, jc & 1, qq / QPB, qq % QPB, pk);
-          else
-            patch_write_quad<C>(patch, lane_v, qq / QPB, qq % QPB, pk);
+          patch_write_quad16<C>(patch, lane_v, jc & 1, qq / QPB, qq % QPB, pk);
           // pin the running sums here: left alone the compiler first computes all the exponentials of the column
           // (to feed the patch writes) and folds them into the sums afterwards, which keeps all of them in registers
           asm volatile("" : "+v"(s), "+v"(sx));
@@ -281,7 +267,7 @@ __device__ __forceinline__ void lmhead_fwd_walk(const FwdParams& p, char* smem, 
       sx_run[jc] = sx;
       if constexpr (KEEP) {
         // the slab of block column j (32 tokens, or the odd 16 of a narrow tile) is complete
-        bf16_t* out = p.keep + (long long)vt * p.keep_blk + (long long)(col0 + wn * WCOL + j * 32) * 256 + wm * C::WTM;
+        bf16_t* out = p.keep + (long long)vt * p.keep_blk + (long long)(col0 + wave_u % C::WN * WCOL + j * 32) * 256 + wave_u / C::WN * C::WTM;
         if (jc % NCL == NCL - 1) patch_flush<C>(patch, out, lane_v);
         else if (jc == NS - 1) patch_flush<C, 16>(patch, out, lane_v);
       }
@@ -444,7 +430,8 @@ __global__ __launch_bounds__(C::NT, C::OCC) void lmhead_ds_kernel(const DsParams
   constexpr bool kPatchBehind = C::STAGE + PATCH <= C::LDS_BYTES;
   constexpr bool kPrefetch = kSplitPrologue<C> && kPatchBehind;
   static_assert(PATCH <= C::LDS_BYTES && 64 % PPT == 0 && 32 % TPP == 0 && (NSLOT & (NSLOT - 1)) == 0, "epilogue patch");
-  char* patch = smem + (kPatchBehind ? C::STAGE : 0) + wave * (32 * ROWP);
+  const int wave_u = __builtin_amdgcn_readfirstlane(wave);
+  char* patch = smem + (kPatchBehind ? C::STAGE : 0) + wave_u * (32 * ROWP);
   const bool through_lds = !SPLIT && p.tv_blk != 0;
 
   if constexpr (kPrefetch) {
@@ -529,10 +516,13 @@ __global__ __launch_bounds__(C::NT, C::OCC) void lmhead_ds_kernel(const DsParams
             uint2 pk;
             pk.x = pack_bf16x2(ds[0], ds[1]);
             pk.y = pack_bf16x2(ds[2], ds[3]);
-            if constexpr (decltype(via_lds)::value) {
+            if constexpr (decltype(via_lds)::value && MI16) {
+              patch_write_quad16<C>(patch, lane_v, jc & 1, qq / QPB, qq % QPB, pk);
+              continue;
+            } else if constexpr (decltype(via_lds)::value) {
               // 8-byte slot of the quad's first row in the token's patch row
-              const int tok = MI16 ? 16 * (jc & 1) + (lane_v & 15) : (lane_v & 31);
-              const int slot = (rr0 >> 2) + (MI16 ? (lane_v >> 4) : (lane_v >> 5));
+              const int tok = lane_v & 31;
+              const int slot = (rr0 >> 2) + (lane_v >> 5);
               lds_write_b64_asm(lds_addr(patch) + tok * ROWP + ((slot ^ (tok & (NSLOT - 1) & 31)) << 3), pk.x, pk.y);
               continue;
             }
@@ -571,7 +561,11 @@ __global__ __launch_bounds__(C::NT, C::OCC) void lmhead_ds_kernel(const DsParams
           emit(std::false_type{}, std::false_type{});
       }
       if (through_lds && jc % NCL == NCL - 1) {      // the 32-token slab of block column j is complete
-        bf16_t* out = p.tv_hi + (long long)vt * p.tv_blk + (long long)(col0 + wn * C::WTN + j * 32) * 256 + wm * C::WTM;
+        bf16_t* out = p.tv_hi + (long long)vt * p.tv_blk + (long long)(col0 + wave_u % C::WN * C::WTN + j * 32) * 256 + wave_u / C::WN * C::WTM;
+        if constexpr (MI16) {
+          patch_flush<C>(patch, out, lane_v);
+          continue;
+        }
         // inline-assembly LDS traffic (see lds_write_b64_asm): one wait for all reads, LDS operations of a
         // wavefront complete in order, so the reads see this wavefront's writes
         u32x4_t pv[32 / TPP];
