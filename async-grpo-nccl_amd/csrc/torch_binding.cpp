@@ -6,6 +6,7 @@
 // Shapes, types and devices are checked before any pointer is taken; errors are RuntimeErrors.
 #include <torch/extension.h>
 
+#include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPStream.h>
 
 #include <cmath>
@@ -294,14 +295,18 @@ struct FusedStep : torch::autograd::Function<FusedStep> {
   }
 };
 
-// labels [..., L], int64, contiguous -> next-token targets, -100 in the last column
+// labels [..., L] -> next-token targets, -100 in the last column: one launch on plain contiguous int64 memory; anything else
+// (wrapped by a function transform, seen by a dispatch mode, strided, rows past 32 bits) by torch's own operations
 Tensor shift_labels(const Tensor& labels) {
-  TORCH_CHECK(labels.is_cuda() && labels.scalar_type() == at::kLong && labels.is_contiguous() && labels.dim() > 0, "fgrpo: labels must be contiguous int64 on the GPU");
+  const bool wrapped = labels.key_set().has_any(c10::DispatchKeySet({c10::DispatchKey::FuncTorchBatched,
+      c10::DispatchKey::BatchedNestedTensor, c10::DispatchKey::FuncTorchGradWrapper, c10::DispatchKey::Functionalize, c10::DispatchKey::Python}));
+  if (wrapped || c10::impl::TorchDispatchModeTLS::any_modes_set() || !labels.is_cuda() || labels.scalar_type() != at::kLong ||
+      labels.dim() == 0 || !labels.is_contiguous() || labels.size(-1) >= (1LL << 31))
+    return at::constant_pad_nd(labels, {0, 1}, -100).slice(-1, 1).contiguous();
   Tensor out = at::empty_like(labels);
   if (labels.numel() == 0) return out;
   OnDevice d(labels);
   const int64_t L = labels.size(-1);
-  TORCH_CHECK(L < (1LL << 31), "fgrpo: rows of ", L, " labels");
   check(api.fgrpo_shift_labels(labels.data_ptr<int64_t>(), labels.numel() / L, (int)L, out.data_ptr<int64_t>(), d.stream()), "shift_labels");
   return out;
 }

@@ -17,6 +17,17 @@ def test_label_shift_is_the_padded_slice(dev, shape):
             assert torch.equal(ops.shift_labels(view), torch.nn.functional.pad(view, (0, 1), value=-100)[..., 1:])
 
 
+def test_label_shift_under_a_function_transform_and_a_trace(dev):
+    """Wrapped tensors have the plain type in Python: they, and what a dispatch mode records, take torch's operations."""
+    from fgrpo import ops
+    from torch.fx.experimental.proxy_tensor import make_fx
+    x, y = (torch.randint(-100, 1 << 40, (4, 9), device=dev) for _ in range(2))
+    want = lambda t: torch.nn.functional.pad(t, (0, 1), value=-100)[..., 1:]
+    assert torch.equal(torch.func.vmap(ops.shift_labels)(x), want(x))
+    assert torch.equal(make_fx(ops.shift_labels)(x)(y), want(y))
+    assert torch.equal(torch.compile(ops.shift_labels, backend="eager", fullgraph=True)(y), want(y))
+
+
 @pytest.mark.parametrize("T,chunk", [(1, 256), (300, 256), (4096, 8192), (4097, 1024), (16385, 8192)])
 def test_loss_is_the_same_with_and_without_gradients(dev, T, chunk):
     """The launch that closes a step without gradients adds the same block sums in the same order; the token count also
