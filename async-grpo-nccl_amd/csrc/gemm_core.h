@@ -7,9 +7,9 @@
 // (BM/WM) x (BN/WN) sub-tile made of 32x32 MFMA blocks kept in fp32 accumulators.  Four loops, chosen by the
 // tile configuration (run_mainloop) or by the caller:
 //   gemm_mainloop      global -> registers -> LDS, padded LDS rows, two buffers (small tiles, fp32 split path);
-//   gemm_mainloop_dma  global -> LDS directly (buffer_load ... lds), swizzled LDS rows; with two buffers it runs
-//                      the early-barrier schedule below (the default for large problems), with three a plain
-//                      prefetch loop;
+//   gemm_mainloop_dma  global -> LDS directly (buffer_load ... lds), swizzled LDS rows; with two buffers (of operand A three on
+//                      16x16x32 MFMAs) it runs the early-barrier schedule below (the default for large problems), with
+//                      three a plain prefetch loop;
 //   gemm_mainloop_la   direct-to-LDS with four or more BK=32 buffers and one K step of fragment look-ahead;
 //   gemm_mainloop_km   operands whose contraction index is the ROW index as stored (read through
 //                      ds_read_b64_tr_b16), early-barrier schedule.
