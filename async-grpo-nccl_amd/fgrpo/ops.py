@@ -390,10 +390,14 @@ def segment_reduce(x: torch.Tensor, cu_seqlens: torch.Tensor, labels_shifted: Op
     return s, m, c
 
 
+def _lengths(x) -> np.ndarray:
+    """Lengths in any form torch takes on the host (list, array, tensor) as int64 [n]."""
+    return torch.as_tensor(x, dtype=torch.int64).reshape(-1).numpy()
+
+
 def output_indices_pack(input_lens, output_lens) -> np.ndarray:
     """What the kernel behind ``output_indices`` reads, int32: token offsets [n], input lengths [n], output offsets [n + 1]."""
-    il = np.asarray(input_lens, dtype=np.int64).reshape(-1)
-    ol = np.asarray(output_lens, dtype=np.int64).reshape(-1)
+    il, ol = _lengths(input_lens), _lengths(output_lens)
     if il.size and int((il + ol).sum()) >= 2 ** 31:
         raise RuntimeError("fgrpo: packed batch longer than 2^31 tokens")
     return np.concatenate([np.cumsum(il + ol) - (il + ol), il, [0], np.cumsum(ol)]).astype(np.int32)
@@ -403,13 +407,13 @@ def output_indices(input_lens, output_lens, device, pack: Optional[torch.Tensor]
     """int64 positions of the logits scoring every generated token (see fgrpo_output_indices).  ``pack``: what
     ``output_indices_pack`` gives for the same lengths, already on the device."""
     lib = _lib.load()
-    ol = np.asarray(output_lens, dtype=np.int64)
-    n, total = int(np.size(input_lens)), int(ol.sum())
+    il, ol = _lengths(input_lens), _lengths(output_lens)
+    n, total = int(il.size), int(ol.sum())
     out = torch.empty(total, dtype=torch.int64, device=device)
     if n == 0 or total == 0:
         return out
     if pack is None:
-        pack = torch.from_numpy(output_indices_pack(input_lens, ol)).to(device)
+        pack = torch.from_numpy(output_indices_pack(il, ol)).to(device)
     with torch.cuda.device(device):
         rc = lib.fgrpo_output_indices(pack.data_ptr(), pack.data_ptr() + 4 * n, pack.data_ptr() + 8 * n, n,
                                       total, _ptr(out), _stream())

@@ -348,3 +348,28 @@ def test_attention_rows_out_of_reach_take_the_64_bit_kernels(attn_route, D, keys
     for far in (dict(q=at32 + 8), dict(k=at + 8, q=at64 + 8), dict(w=2, q=at64 + 8), dict(w=1), dict(w=2, T=2 ** 28, q=at32 + 8),
                 dict(Hq=at32 // D + 1, Hkv=1)):
         assert form(**far) == 1, far
+
+
+@pytest.mark.parametrize("form", [list, tuple, np.array, torch.tensor, lambda x: [torch.tensor(v) for v in x],
+                                  lambda x: np.array(x, dtype=np.int32), lambda x: torch.tensor(x, dtype=torch.int32).view(2, 2)])
+def test_output_indices_take_lengths_in_any_host_form(monkeypatch, form):
+    """What the kernel is handed, read back as the kernel reads it: n offsets, n input lengths, n + 1 output offsets."""
+    import contextlib
+    import ctypes
+    import types
+    from fgrpo import ops
+    il, ol = [3, 1, 4, 2], [2, 5, 1, 0]
+
+    def kernel(tok, lin, out, n, total, dst, stream):
+        at = lambda p, k, t: np.ctypeslib.as_array((t * k).from_address(p))
+        tok, lin, out = at(tok, n, ctypes.c_int32), at(lin, n, ctypes.c_int32), at(out, n + 1, ctypes.c_int32)
+        for i in range(n):
+            at(dst, total, ctypes.c_int64)[out[i]:out[i + 1]] = tok[i] + lin[i] - 1 + np.arange(out[i + 1] - out[i])
+        return 0
+
+    monkeypatch.setattr(ops._lib, "load", lambda: types.SimpleNamespace(fgrpo_output_indices=kernel))
+    monkeypatch.setattr(ops, "_stream", lambda: 0)
+    monkeypatch.setattr(ops, "_ptr", lambda t: t.data_ptr())
+    monkeypatch.setattr(torch.cuda, "device", lambda d: contextlib.nullcontext())
+    got = ops.output_indices(form(il), form(ol), torch.device("cpu"))
+    assert got.tolist() == O.output_logits_indices(il, ol).tolist()
