@@ -390,33 +390,45 @@ def segment_reduce(x: torch.Tensor, cu_seqlens: torch.Tensor, labels_shifted: Op
     return s, m, c
 
 
-def _lengths(x) -> np.ndarray:
-    """Lengths in any form torch takes on the host (list, array, tensor) as int64 [n]."""
-    return torch.as_tensor(x, dtype=torch.int64).reshape(-1).numpy()
+def _lengths(input_lens, output_lens):
+    """Both lists of lengths, in any form torch takes on the host (list, array, tensor), as int64 [n]; one output length
+    is shared by all samples."""
+    il, ol = (torch.as_tensor(x, dtype=torch.int64).reshape(-1).numpy() for x in (input_lens, output_lens))
+    if il.size and ol.size not in (1, il.size):
+        raise RuntimeError(f"fgrpo: {ol.size} output lengths for {il.size} input lengths")
+    return il, ol
 
 
 def output_indices_pack(input_lens, output_lens) -> np.ndarray:
     """What the kernel behind ``output_indices`` reads, int32: token offsets [n], input lengths [n], output offsets [n + 1]."""
-    il, ol = _lengths(input_lens), _lengths(output_lens)
-    if il.size and int((il + ol).sum()) >= 2 ** 31:
+    il, ol = _lengths(input_lens, output_lens)
+    n = il.size
+    if n and int((il + ol).sum()) >= 2 ** 31:
         raise RuntimeError("fgrpo: packed batch longer than 2^31 tokens")
-    return np.concatenate([np.cumsum(il + ol) - (il + ol), il, [0], np.cumsum(ol)]).astype(np.int32)
+    pack = np.zeros(3 * n + 1, dtype=np.int32)      # as many as the kernel reads, also where ol is shared
+    if n:
+        pack[1:n] = np.cumsum(il + ol)[:-1]
+        pack[n:2 * n] = il
+        pack[2 * n + 1:] = np.cumsum(ol)
+    return pack
 
 
 def output_indices(input_lens, output_lens, device, pack: Optional[torch.Tensor] = None) -> torch.Tensor:
     """int64 positions of the logits scoring every generated token (see fgrpo_output_indices).  ``pack``: what
     ``output_indices_pack`` gives for the same lengths, already on the device."""
     lib = _lib.load()
-    il, ol = _lengths(input_lens), _lengths(output_lens)
-    n, total = int(il.size), int(ol.sum())
+    il, ol = _lengths(input_lens, output_lens)
+    n = int(il.size)
+    total = int(ol.sum()) if n else 0
     out = torch.empty(total, dtype=torch.int64, device=device)
-    if n == 0 or total == 0:
+    if total == 0:
         return out
     if pack is None:
         pack = torch.from_numpy(output_indices_pack(il, ol)).to(device)
+    elif pack.dtype != torch.int32 or pack.numel() != 3 * n + 1 or not pack.is_contiguous():
+        raise RuntimeError("fgrpo: pack must be what output_indices_pack gives for these lengths")
     with torch.cuda.device(device):
-        rc = lib.fgrpo_output_indices(pack.data_ptr(), pack.data_ptr() + 4 * n, pack.data_ptr() + 8 * n, n,
-                                      total, _ptr(out), _stream())
+        rc = lib.fgrpo_output_indices(_ptr(pack), _ptr(pack) + 4 * n, _ptr(pack) + 8 * n, n, total, _ptr(out), _stream())
     _lib.check(rc, "output_indices")
     return out
 

@@ -373,3 +373,23 @@ def test_output_indices_take_lengths_in_any_host_form(monkeypatch, form):
     monkeypatch.setattr(torch.cuda, "device", lambda d: contextlib.nullcontext())
     got = ops.output_indices(form(il), form(ol), torch.device("cpu"))
     assert got.tolist() == O.output_logits_indices(il, ol).tolist()
+
+
+@pytest.mark.parametrize("il,ol", [([3, 4, 5], [2]), ([3], [2]), ([1] * 9, [3] * 9), ([], []), ([], [4])])
+def test_output_indices_pack_holds_what_the_kernel_reads(il, ol):
+    """3 n + 1 entries for n samples, also where one output length is given for all: the kernel reads n + 1 output offsets."""
+    from fgrpo import ops
+    n = len(il)
+    a, b = torch.tensor(il, dtype=torch.int64), torch.tensor(ol, dtype=torch.int64)
+    tok, out = torch.zeros(n, dtype=torch.int64), torch.zeros(n + 1, dtype=torch.int64)
+    tok[1:], out[1:] = torch.cumsum(a + b, 0)[:-1], torch.cumsum(b, 0)
+    assert ops.output_indices_pack(il, ol).tolist() == torch.cat([tok, a, out]).tolist()
+
+
+@pytest.mark.parametrize("il,ol", [([3, 4, 5], [2, 1]), ([3], [2, 1]), ([3, 4], []), ([3, 4, 5], [0, 0])])
+def test_output_indices_refuse_other_numbers_of_lengths(monkeypatch, il, ol):
+    from fgrpo import ops
+    monkeypatch.setattr(ops._lib, "load", lambda: None)
+    for call in (ops.output_indices_pack, lambda *a: ops.output_indices(*a, torch.device("cpu"))):
+        with pytest.raises(RuntimeError):
+            call(il, ol)
