@@ -121,6 +121,14 @@ def native():
     return mod
 
 
+def native_if_built():
+    """``native()``, or None where it (or the library) is not built: for callers with another way to the same result."""
+    try:
+        return native()
+    except RuntimeError:
+        return None
+
+
 def check(rc: int, what: str) -> None:
     if rc != 0:
         msg = load().fgrpo_last_error().decode("utf-8", "replace")

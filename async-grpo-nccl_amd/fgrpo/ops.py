@@ -78,7 +78,9 @@ def shift_labels(labels: torch.Tensor) -> torch.Tensor:
     """labels [..., L] -> next-token targets, -100 in the last column."""
     if type(labels) is torch.Tensor and labels.is_cuda and labels.dtype == torch.int64 and labels.is_contiguous() \
             and labels.dim() > 0 and not torch.jit.is_tracing() and not torch.compiler.is_compiling():   # a trace has to see the operations
-        return _lib.native().shift_labels(labels)
+        native = _lib.native_if_built()
+        if native is not None:
+            return native.shift_labels(labels)
     return torch.nn.functional.pad(labels, (0, 1), value=IGNORE_INDEX)[..., 1:].contiguous()
 
 

@@ -28,6 +28,22 @@ def test_label_shift_under_a_function_transform_and_a_trace(dev):
     assert torch.equal(torch.compile(ops.shift_labels, backend="eager", fullgraph=True)(y), want(y))
 
 
+def test_log_probabilities_without_the_extension_module(dev, monkeypatch):
+    """The log-probability entry point needs the library alone; without the module the shift is torch's."""
+    import grpo_loss as G
+    from fgrpo import _lib, ops
+    g = torch.Generator(device=dev).manual_seed(5)
+    h, w = torch.randn(1, 70, 64, generator=g, device=dev), torch.randn(999, 64, generator=g, device=dev)
+    y = torch.randint(0, 999, (1, 70), generator=g, device=dev)
+    with torch.no_grad():
+        want = G.fused_log_probs_and_entropy_fn(w, None, h, y)
+        monkeypatch.setattr(_lib, "_native", None)
+        monkeypatch.setattr(_lib, "BINDING_PATH", _lib.BINDING_PATH + ".absent")
+        got = G.fused_log_probs_and_entropy_fn(w, None, h, y)
+    assert torch.equal(ops.shift_labels(y), torch.nn.functional.pad(y, (0, 1), value=-100)[..., 1:])
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
 @pytest.mark.parametrize("T,chunk", [(1, 256), (300, 256), (4096, 8192), (4097, 1024), (16385, 8192)])
 def test_loss_is_the_same_with_and_without_gradients(dev, T, chunk):
     """The launch that closes a step without gradients adds the same block sums in the same order; the token count also
