@@ -1523,7 +1523,7 @@ int fgrpo_loss_fwd(const float* lp, const float* old_lp, const float* ref_lp, co
   p.clipped = clipped;
   p.loss = loss_out;
   p.scal = scal_out;
-  if (T <= kSmallLossTokens && (agg_mode != FGRPO_AGG_SAMPLE_MEAN || nseq <= kSmallLossTokens)) {
+  if (T <= kSmallLossTokens && (agg_mode != FGRPO_AGG_SAMPLE_MEAN || nseq <= kSmallLossSegments)) {
     hipLaunchKernelGGL(grpo_loss_small_kernel, dim3(1), dim3(1024), 0, st, p, cu, nseq);
     HIP_TRY(hipGetLastError());
     return 0;

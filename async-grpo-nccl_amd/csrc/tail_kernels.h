@@ -413,8 +413,10 @@ __global__ __launch_bounds__(kLossThreads) void grpo_loss_finalize_kernel(const 
 // The whole objective of a batch this small in one work-group and launch: segment weights, tokens, loss, normalised g.  Three
 // kernels that wait for one another are three launches at 4.7 us, and the host path of so small a step is launches: fp32
 // step of 643 tokens x 1000 entries x 64, three trees in turn on one box, 126..130 -> 119..123 us a pass, its forward 44.5 -> 38.2.
-// A thread takes two tokens at most; from some thousand tokens on the work is worth more than one work-group.
-constexpr int kSmallLossTokens = 2048;
+// A thread takes two tokens at most; from some thousand tokens on the work is worth more than one work-group.  A wavefront takes a
+// segment at a time, 0.5 us each: up to four a wavefront.  On the device alone, three launches | one, us: 643 tokens in 16 segments
+// 7.4 | 5.0, 64 7.5 | 6.6, 96 7.3 | 7.7, 512 8.4 | 21.1; 2048 tokens in 64 8.1 | 7.8, 96 8.2 | 8.9, 2048 13.6 | 71.7.
+constexpr int kSmallLossTokens = 2048, kSmallLossSegments = 64;
 __global__ __launch_bounds__(1024) void grpo_loss_small_kernel(LossParams p, const int* cu, int nseq) {
   __shared__ float weight[kSmallLossTokens];
   __shared__ double sums[3][16];

@@ -68,11 +68,12 @@ def test_loss_is_the_same_with_and_without_gradients(dev, T, chunk):
 
 
 @pytest.mark.parametrize("T,bounds", [(1, [0, 1]), (63, [0, 10, 10, 63]), (1024, [0, 1000, 1024]), (1025, [3, 700, 1020]), (2047, [0, 2047]),
-                                      (2048, list(range(0, 2049, 8))), (2049, [0, 5, 2049]), (2048, [0, 3000]), (700, [600, 50, 650])])
+                                      (2048, list(range(0, 2049, 8))), (1500, list(range(0, 641, 10))), (1500, list(range(0, 651, 10))),
+                                      (2048, list(range(2049))), (2049, [0, 5, 2049]), (2048, [0, 3000]), (700, [600, 50, 650])])
 @pytest.mark.parametrize("mode", ["token_mean", "sample_mean"])
 @pytest.mark.parametrize("denom", [0.0, 7.0])
 def test_objective_of_a_small_batch(dev, T, bounds, mode, denom):
-    """One work-group up to 2048 tokens, three launches beyond: the same formula in fp64 from the same log-probabilities.
+    """One work-group up to 2048 tokens in 64 segments, three launches beyond: the same formula in fp64 from the same log-probabilities.
     Weights, ratios and products are fp32: a dozen roundings, 2e-6 of the largest term."""
     from fgrpo import ops
     g = torch.Generator(device=dev).manual_seed(T)
@@ -107,3 +108,31 @@ def test_objective_of_a_small_batch(dev, T, bounds, mode, denom):
     assert abs(float(loss) - float(want.detach())) <= 2e-6 * big + 1e-9
     assert (gr.double() - gw).abs().max() <= 2e-6 * float(gw.abs().max()) + 1e-12
     assert float(scal[1]) == float(on.sum())
+
+
+def test_many_segments_are_not_walked_by_one_work_group(dev):
+    """A segment costs a wavefront half a microsecond: 2048 of them took one work-group nine times as long as 64; over the
+    device they take less than twice as long."""
+    from fgrpo import ops
+    T = 2048
+    lp, adv, y = torch.randn(T, device=dev), torch.randn(T, device=dev), torch.zeros(T, dtype=torch.long, device=dev)
+
+    def us(segments):
+        cu = torch.linspace(0, T, segments + 1, device=dev).int()
+        call = lambda: ops.grpo_loss_fwd(lp, lp, None, adv, y, cu, 0.2, 0.28, 3.0, 0.0, "sample_mean", 0.0)
+        call()
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            for _ in range(20):
+                call()
+        best = float("inf")
+        for _ in range(5):
+            a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            a.record()
+            graph.replay()
+            b.record()
+            torch.cuda.synchronize()
+            best = min(best, a.elapsed_time(b))
+        return best
+    assert us(T) < 4 * us(64)
