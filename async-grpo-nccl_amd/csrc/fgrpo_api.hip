@@ -269,13 +269,20 @@ int fwd_raster_group(const Tuning& tn, int nsplit) {
   return nsplit == 8 ? 4 : g < 6 ? g : 6;
 }
 
-// A last tile of few tokens: 64 NB columns wide it costs a work-group kTailCost[NB] of what a whole one does (24 K steps of
-// H = 1536: 43 us; one this narrow waits for W, which comes from HBM, and no longer for its matrix instructions).  Its
-// vocabulary is dealt out in shares that take as long as the whole tiles', so that it fills part of the round instead of a
-// quarter of it or a round of its own.  Forward at H = 1536, V = 151936, whole | narrow, us: T = 60 131 | 88, 100 136 | 95, 300
-// 208 | 178, 777 468 | 442, 868 408 | 350, 1034 483 | 437; H = 8192, V = 128256: T = 550 1448 | 1330.  From 129 columns on
-// little is left to gain.
-constexpr double kTailCost[3] = {0.0, 0.5, 0.65};
+// A last tile of few tokens: 64 NB columns wide it costs a work-group tail_cost of what a whole one does (one this narrow
+// waits for W, which comes from HBM, and no longer for its matrix instructions).  Its vocabulary is dealt out in shares that
+// take as long as the whole tiles', so that it fills part of the round instead of a quarter of it or a round of its own.  Plain
+// forward, whole | narrow, us, one run: H = 1536, V = 151936: T = 64 124 | 97, 100 127 | 104, 300 202 | 186, 777 381 | 359, 868
+// 385 | 363, 1034 466 | 439; H = 8192, V = 128256: T = 560 1196 | 1086.  From 129 columns on little is left to gain.
+// The 64-column tile costs more the more tokens it has, and more of a whole one's time past H = 4096, but for multiples of
+// 4096 (why is not known).  Counted as half there, T = 832 (64 tokens in the last tile) at H = 4608 .. 6144 took 1.05 .. 1.07 of the
+// whole tile's time, T = 1600 1.05 .. 1.11; as 0.55 0.96 .. 1.01 and 0.97 .. 1.06, one box with another; as 0.6 0.94 and 0.97.
+// Elsewhere half loses nowhere (T = 832: H = 896 0.89, 1536 and 3584 1.00, 2048 0.94, 4096 0.97, 8192 0.93 .. 0.98), and 0.6 would
+// give up what two whole tiles and a narrow one gain (T = 576: H = 896 0.84, 2048 0.90, 8192 0.91).
+double tail_cost(int nb, int rows, int H) {
+  if (nb == 2) return 0.65;
+  return rows > 8 && H > 4096 && H % 4096 != 0 ? 0.6 : 0.5;
+}
 int tail_columns(const Tuning& tn, int variant, int T) {        // NB, or 0 where the last tile is taken whole
   const int r = T % kCfg[8].bn;
   if (variant != 8 || tn.fwd_tail == 0 || tn.fwd_nsplit > 0 || r == 0 || r > 128) return 0;
@@ -284,13 +291,13 @@ int tail_columns(const Tuning& tn, int variant, int T) {        // NB, or 0 wher
 struct TailPlan {
   int nsplit = 0, tail_split = 0;
 };
-// Shares of the whole tiles and of the narrow one, the cheapest by rounds_cost.
-TailPlan plan_tail(int tiles, int nb, int tiles_v, int slots, int prefer, long long* cost_out) {
+// Shares of the whole tiles and of the narrow one, which costs `narrow` of a whole one, the cheapest by rounds_cost.
+TailPlan plan_tail(int tiles, double narrow, int tiles_v, int slots, int prefer, long long* cost_out) {
   TailPlan best;
   long long least = -1;
   auto consider = [&](int ns) {
-    const int per = tiles > 0 ? (tiles_v + ns - 1) / ns : (int)(kTailCost[nb] * ((tiles_v + ns - 1) / ns) + 1.0);
-    int share = (int)(per / kTailCost[nb]);
+    const int per = tiles > 0 ? (tiles_v + ns - 1) / ns : (int)(narrow * ((tiles_v + ns - 1) / ns) + 1.0);
+    int share = (int)(per / narrow);
     if (share < 1) share = 1;
     const int nt = tiles > 0 ? (tiles_v + share - 1) / share : ns;
     const long long rounds = ((long long)tiles * ns + nt + slots - 1) / slots, cost = rounds * (4 * per + 3);      // as rounds_cost
@@ -353,7 +360,7 @@ void plan_fwd(const Tuning& tn, FwdPlan& pl, void* ws, int T, int H, int V, int 
     const int r0 = pl.t_main < T ? pl.t_main : 0, tiles = (T - r0) / c.bn;      // of the last region
     int& ns = pl.t_main < T ? pl.nsplit_rem : pl.nsplit;
     long long cost = 0;
-    const TailPlan t = plan_tail(tiles, pl.tail_nb, pl.tiles_v, slots, prefer, &cost);
+    const TailPlan t = plan_tail(tiles, tail_cost(pl.tail_nb, T % c.bn, H), pl.tiles_v, slots, prefer, &cost);
     if (tiles == 0 || cost < rounds_cost(tiles + 1, pl.tiles_v, slots, ns)) ns = t.nsplit, pl.tail_split = t.tail_split;
     else pl.tail_nb = 0;
   }

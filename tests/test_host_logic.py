@@ -393,3 +393,15 @@ def test_output_indices_refuse_other_numbers_of_lengths(monkeypatch, il, ol):
     for call in (ops.output_indices_pack, lambda *a: ops.output_indices(*a, torch.device("cpu"))):
         with pytest.raises(RuntimeError):
             call(il, ol)
+
+
+@pytest.mark.parametrize("H,T,narrow", [(4096, 832, 0.5), (4608, 776, 0.5), (4608, 777, 0.6), (5120, 832, 0.6), (6144, 832, 0.6),
+                                        (8192, 832, 0.5), (1536, 832, 0.5), (5120, 896, 0.65)])
+def test_shares_of_a_narrow_last_token_tile(H, T, narrow):
+    """594 vocabulary tiles in 66 shares of nine for three whole token tiles; the narrow one's shares take as long.  Seen in
+    the workspace, which holds 16 bytes a token and share (with 256 CUs, which is also what a host without a GPU plans for)."""
+    from fgrpo import _lib
+    V, up = 152064, lambda n: (n + 255) // 256 * 256
+    shares = -(-594 // int(9 / narrow))
+    want = up(16 * 66 * T) + up(16 * shares * (T % 256)) + up(4 * T) + up(4 * V)
+    assert _lib.load().fgrpo_logprob_fwd_workspace(T, H, V, _lib.BF16) == want
