@@ -17,12 +17,18 @@ int launch_store_variant(int variant, const StoreParams& p, hipStream_t st) {
   return rc;
 }
 
+// dHidden's lead (AHEAD, see early_barrier_pipeline16): work-groups walk the same rows of W, and the longer lead lets those that have
+// lost step with each other stay apart.  They lose it along long contractions and when they replace others, so those take the
+// shorter one.  Before the longer lead existed | longer | shorter, ms: whole tiles over the vocabulary (numerators of the whole batch
+// kept): H = 5120, T = 16384 18.7 | 20.4 | 18.5, 12288 14.6 | 15.5 | 14.7; H = 3584, T = 32768 26.6 | 27.4 | 26.3; H = 1536 11.2 | 11.4 | 10.9;
+// H = 896 .. 2048 and 8192 the same or up to 3 % better with the shorter; two pieces: H = 5120, T = 4500 5.66 | 6.02 | 5.75, 4800 5.79 | 6.13
+// | 5.91.  Panels of the recomputing backward, a quarter of the vocabulary, keep the longer (H = 3584, T = 10400 10.5 | 11.1, longer |
+// shorter), and so do three pieces or more (H = 3584, T = 4500 3.68 | 3.77; H = 6144, T = 4000 5.84 | 5.93) up to four device rounds of
+// them (H = 3584, T = 8975 6.70 | 7.02; H = 1536, T = 8192 2.72 | 2.79; from the fifth on H = 5120, T = 8192 10.3 | 9.6).
+constexpr int kLongContraction = 60000;
 int launch_store_splitk(const StoreParams& p, hipStream_t st) {
-  // Pieces of one column chunk walk the same rows of W; from the fifth device round on, work-groups that replace others have
-  // lost step with each other, and the longer lead lets them stay apart.  Longer | shorter lead, ms: H = 5120, T = 8192, five
-  // rounds 10.3 | 9.6; H = 3584, T = 16384, seven 13.1 | 12.9; T = 8192, seven 6.74 | 6.75; four rounds at most: H = 3584, T = 8975
-  // 6.70 | 7.02, T = 2000 1.76 | 1.85; H = 1536, T = 8192 2.72 | 2.79.
-  if (p.nblocks > 4 * num_cus()) return launch_tile_kernel<gemm_store_kernel<Cfg8, false, true, true, false>, Cfg8>(p, p.nblocks, st);
+  if (p.nblocks > 4 * num_cus() || p.kchunk >= kLongContraction)
+    return launch_tile_kernel<gemm_store_kernel<Cfg8, false, true, true, false>, Cfg8>(p, p.nblocks, st);
   return launch_tile_kernel<gemm_store_kernel<Cfg8, false, true, true>, Cfg8>(p, p.nblocks, st);
 }
 
@@ -34,6 +40,7 @@ int launch_store_kmajor(bool akm, bool bkm, const StoreParams& p, hipStream_t st
   const int nb = p.nblocks;
   if (akm && bkm) return launch_tile_kernel<gemm_store_kernel<Cfg8, true, true>, Cfg8>(p, nb, st);
   if (akm) return launch_tile_kernel<gemm_store_kernel<Cfg8, true, false>, Cfg8>(p, nb, st);
+  if (bkm && p.g.seg[0].K >= kLongContraction) return launch_tile_kernel<gemm_store_kernel<Cfg8, false, true, false, false>, Cfg8>(p, nb, st);
   if (bkm) return launch_tile_kernel<gemm_store_kernel<Cfg8, false, true>, Cfg8>(p, nb, st);
   return fail(FGRPO_ERR_BAD_ARG, "gemm(k-major): no k-major operand");
 }
