@@ -1254,6 +1254,7 @@ int kept_bwd_impl(const Tuning& tn, const void* hidden, const void* weight, cons
                   int loss_parts = 0) {
   const bool want_dh = dH_out != nullptr, want_dw = dW_out != nullptr || sums.dw_out_f32 != nullptr;
   const bool want_db = dbias_out != nullptr || sums.db_out_f32 != nullptr;
+  if (loss_parts > 0 && (!loss || !loss->pre)) return fail(FGRPO_ERR_BAD_ARG, "lmhead_bwd_kept: the loss needs its normaliser");
   KeptBwdPlan pl;
   plan_kept_bwd(tn, pl, ws, T, H, V, bias != nullptr, want_dh, want_dw);
   if (!ws || !aligned16(ws) || ws_bytes < pl.bytes)

@@ -497,20 +497,20 @@ __device__ __forceinline__ void early_barrier_pipeline(int nk_total, char* smem,
 // ask for a slice waits, those behind it find it in the L2.  With the longer lead nothing held them (forward of 40000
 // tokens, H = 5120: past the L2s 36.7 -> 71.8 GB, 6 % fewer cycles at a lower clock, 35.6 -> 36.9 ms); so every
 // kStrictEvery-th step waits for the youngest A as well (33.9 ms; every second step 34.0, every eighth 34.9).  !AHEAD: the
-// one step of lead, for long contractions in many device rounds (dHidden, launch_store_splitk), where the drift adds up
-// from round to round.  Before -> after, one box each: forward that keeps the numerators, T = 8192, H = 1536: 3.28 -> 3.09 ms, H =
+// one step of lead, for dHidden over the whole vocabulary or in many device rounds (launch_store_splitk, launch_store_kmajor), where
+// the drift adds up.  Before -> after, one box each: forward that keeps the numerators, T = 8192, H = 1536: 3.28 -> 3.09 ms, H =
 // 3584, T = 16384: 13.14 -> 12.78; dW of 8192 tokens, H = 1536: 3.04 -> 2.98; dHidden of 777 tokens 0.409 -> 0.388.
 //   issue_a(lds, idx) / issue_b(lds, idx): load idx of the next K step of that operand into the buffer at `lds`; the
 //   last one of A (the first one of B, but for step 0's) advances the operand's cursor;
 //   load_a(lds, I, KK): fragment a(I, KK % 2) of slice KK / 2;  load_b(lds, JC, K2): fragment b(JC/2, JC%2).
-// NB: 16-column blocks of operand B a wavefront multiplies, 4 or, on tiles 64 NB columns wide (kTailCols), fewer.
+// NB: 16-column blocks of operand B a wavefront multiplies, 4 or, on tiles 64 NB columns wide (the forward's narrow last token tile), fewer.
 // On entry B of step 0 and A of steps 0 and 1 have been issued, in this order (as far as they exist).  DRAIN: wait for
 // all of it (the caller has issued something else since), not just for step 0.
 constexpr int kStrictEvery = 4;                      // a power of two
 template <class C>
 constexpr int kOpBytes = C::BM * C::ROWB;            // one buffer of one operand (32 KiB)
-__device__ __forceinline__ constexpr int mi16_a_buf(int step) { return step % 3; }          // in kOpBytes
-__device__ __forceinline__ constexpr int mi16_b_buf(int step) { return 4 - (step & 1); }    // buffers 2 and 3 are free between tiles
+// of step's B, in kOpBytes; A's is step % 3, so that buffers 2 and 3 are free between tiles
+__device__ __forceinline__ constexpr int mi16_b_buf(int step) { return 4 - (step & 1); }
 template <class C, int NB, int RA, int RB, bool DRAIN, bool AHEAD, class IssueA, class IssueB, class LoadA, class LoadB>
 __device__ __forceinline__ void early_barrier_pipeline16(int nk_total, char* smem, f32x16_t (&acc)[C::TM][C::TN],
                                                          bool live, IssueA&& issue_a, IssueB&& issue_b, LoadA&& load_a,
@@ -653,15 +653,16 @@ __device__ __forceinline__ bool wave_is_live(const GemmOperands& g, int row0, in
   return row0 + wm * C::WTM < g.M && col0 + wn * C::WTN < g.N;
 }
 
-// MODE 0: the whole contraction.  MODE 2: only issue the loads of K step 0 into buffer 0 and return (the caller
-// does something else, e.g. the epilogue of the previous tile, while they fly); MODE 1: the contraction, given that
+// MODE 0: the whole contraction.  MODE 2: only issue the first loads and return (the caller does something else, e.g. the
+// epilogue of the previous tile, while they fly): K step 0 into buffer 0 of two, or on the 16x16x32 schedule B of step 0 and A
+// of steps 0 and 1 into operand buffers 4, 0 and 1 (the caller may use what lies between: 64 KiB from C::STAGE on).  MODE 1: the contraction, given that
 // a MODE 2 call for the same tile has been made since the last MODE 0/1 call returned.  Modes 1 and 2 exist for
 // the two-buffer schedule only (kSplitPrologue).
 template <class C>
 constexpr bool kSplitPrologue = C::DMA && C::NSTAGE == 2 && (C::BK / 16) % 2 == 0;
 
 // gemm_mainloop_dma on the 16x16x32 schedule.  MODE 2 requests what early_barrier_pipeline16 expects on entry and
-// leaves LDS buffers 2 and 3 (64 KiB from C::STAGE on) to the caller until the MODE 1 call.
+// leaves operand buffers 2 and 3 to the caller until the MODE 1 call.
 // NB < 4: the tile is 64 NB columns wide, 16 NB of them a wavefront's.
 template <class C, int MODE, int NB = 4>
 __device__ __forceinline__ void gemm_mainloop_dma16(const GemmOperands& g, int row0, int col0, char* smem,

@@ -144,7 +144,7 @@ __device__ __forceinline__ void lmhead_fwd_walk(const FwdParams& p, char* smem, 
     if constexpr (KEEP) ref2[jc] = (n < T) ? p.keep_ref2[n] : -kNegBig;
   }
 
-  // KEEP: the wavefront's patch lives behind LDS buffer 0, which the prefetch of the next tile may already be filling
+  // KEEP: the wavefronts' patches are operand buffers 2 and 3; the prefetch of the next tile may already be filling 0, 1 and 4
   constexpr int KEEP_PATCH = C::NW * 32 * C::WTM * 2;
   static_assert(!KEEP || (MI16 && kSplitPrologue<C> && C::BM == 256 && C::STAGE + KEEP_PATCH <= C::LDS_BYTES),
                 "kept logits: 256-row tiles on the two-buffer direct-to-LDS loop");
@@ -420,9 +420,9 @@ __global__ __launch_bounds__(C::NT, C::OCC) void lmhead_ds_kernel(const DsParams
   // Column-blocked panel: a lane's 8 bytes (4 vocabulary entries of one token) would be a 64-line scatter per
   // store instruction.  The wavefront instead parks 32 tokens x WTM entries in a private LDS patch and writes
   // them out as 16-byte pieces, PPT lanes per token row: every store instruction fills whole 128-byte lines.
-  // Patch rows are unpadded; the 8-byte slots of row n are XOR-swizzled with n, so that the 32 lanes of a write
-  // (one token each) hit 32 different slots.  The patch lives behind LDS buffer 0, which the prefetch of the next
-  // tile may already be filling.
+  // Patch rows are unpadded.  On 16x16x32 MFMAs patch_write_quad16 and patch_flush swizzle them; else the 8-byte slots of row
+  // n are XORed with n, so that the 32 lanes of a write (one token each) hit 32 different slots.  The patch lies from C::STAGE on
+  // where it fits there, beside what the prefetch of the next tile may already be filling.
   constexpr int ROWP = C::WTM * 2;                       // patch row: one token's WTM entries
   constexpr int NSLOT = ROWP / 8;                        // 8-byte slots per row
   constexpr int PPT = ROWP / 16, TPP = 64 / PPT;         // 16-byte pieces per token, tokens per store instruction

@@ -349,7 +349,8 @@ __global__ __launch_bounds__(kLossThreads) void grpo_loss_tokens_kernel(const Lo
 // kFinalizeBlocks blocks, so the partials are re-read that many times at most)
 // by the normaliser; block 0 publishes the scalars.
 constexpr int kFinalizeBlocks = 256;
-// The first kLossThreads threads of a work-group work, all of them pass the barriers.
+// The first kLossThreads threads of a work-group work, all of them pass the barriers.  Without p.pre the whole grid has to be
+// this function's, for g's slices; a work-group of another launch may call it with p.pre only.
 struct FinalizeLds {
   double part[3][kLossThreads / 64], tot[3];
 };
