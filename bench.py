@@ -28,11 +28,11 @@ PEAK_CLOCK_MHZ = 2400.0
 PROFILED_TRAFFIC = {
     # (workload, path): (bytes per launch of the forward kernel, summary under profiles/); a launch of the chunked
     # path is one token chunk
-    ("cfg1", "chunked"): (8.116e+09, "profiles/lmhead_chunked_step_cfg1_counters_pmc.txt"),
-    ("cfg1", "whole"): (3.256e+10, "profiles/lmhead_whole_batch_kept_cfg1_counters_pmc.txt"),
-    ("cfg2", "chunked"): (3.121e+10, "profiles/lmhead_chunked_step_cfg2_counters_pmc.txt"),
-    ("cfg3", "forward"): (3.387e+11, "profiles/lmhead_fwd_kernel_cfg3_counters_pmc.txt"),
-    ("cfg4", "chunked"): (2.172e+10, "profiles/lmhead_chunked_step_cfg4_counters_pmc.txt"),
+    ("cfg1", "chunked"): (8.115e+09, "profiles/lmhead_chunked_step_cfg1_counters_pmc.txt"),
+    ("cfg1", "whole"): (3.258e+10, "profiles/lmhead_whole_batch_kept_cfg1_counters_pmc.txt"),
+    ("cfg2", "chunked"): (3.122e+10, "profiles/lmhead_chunked_step_cfg2_counters_pmc.txt"),
+    ("cfg3", "forward"): (5.279e+11, "profiles/lmhead_fwd_kernel_cfg3_counters_pmc.txt"),
+    ("cfg4", "chunked"): (1.501e+10, "profiles/lmhead_chunked_step_cfg4_counters_pmc.txt"),
 }
 
 
