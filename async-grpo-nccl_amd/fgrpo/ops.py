@@ -77,7 +77,8 @@ def _ws(nbytes: int, device) -> torch.Tensor:
 def shift_labels(labels: torch.Tensor) -> torch.Tensor:
     """labels [..., L] -> next-token targets, -100 in the last column."""
     if type(labels) is torch.Tensor and labels.is_cuda and labels.dtype == torch.int64 and labels.is_contiguous() \
-            and labels.dim() > 0 and not torch.jit.is_tracing() and not torch.compiler.is_compiling():   # a trace has to see the operations
+            and labels.dim() > 0 and not torch.jit.is_tracing() and not torch.compiler.is_compiling() \
+            and not torch._C._is_torch_function_mode_enabled():   # a trace or a mode (a pre-dispatch trace is one) has to see the operations
         native = _lib.native_if_built()
         if native is not None:
             return native.shift_labels(labels)

@@ -28,6 +28,26 @@ def test_label_shift_under_a_function_transform_and_a_trace(dev):
     assert torch.equal(torch.compile(ops.shift_labels, backend="eager", fullgraph=True)(y), want(y))
 
 
+def test_label_shift_under_a_function_mode(dev):
+    """A trace before dispatch is a function mode and no dispatch mode: it, and any other such mode, sees the operations."""
+    from fgrpo import ops
+    from torch.fx.experimental.proxy_tensor import make_fx
+    from torch.overrides import TorchFunctionMode
+    x, y = (torch.randint(-100, 1 << 40, (4, 9), device=dev) for _ in range(2))
+    want = lambda t: torch.nn.functional.pad(t, (0, 1), value=-100)[..., 1:]
+    assert torch.equal(make_fx(ops.shift_labels, pre_dispatch=True)(x)(y), want(y))
+    seen = []
+
+    class Record(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            seen.append(func)
+            return func(*args, **(kwargs or {}))
+
+    with Record():
+        assert torch.equal(ops.shift_labels(x), want(x))
+    assert torch.nn.functional.pad in seen
+
+
 def test_log_probabilities_without_the_extension_module(dev, monkeypatch):
     """The log-probability entry point needs the library alone; without the module the shift is torch's."""
     import grpo_loss as G
