@@ -38,7 +38,11 @@ int launch_small_split(const SmallSplitPair& p, int nblocks, hipStream_t st) {
 
 int launch_store_kmajor(bool akm, bool bkm, const StoreParams& p, hipStream_t st) {
   const int nb = p.nblocks;
-  if (akm && bkm) return launch_tile_kernel<gemm_store_kernel<Cfg8, true, true>, Cfg8>(p, nb, st);
+  // dW of the recomputing backward: the shorter lead as well.  Before the longer one existed | longer | shorter, ms: H = 1536, T =
+  // 8192 2.91 | 3.02 | 2.97, 24000 8.62 | 8.94 | 8.74, 32768 11.9 | 12.4 | 12.2; H = 3584, T = 32768 28.9 | 30.0 | 29.6; H = 5120, T = 16384
+  // 20.3 | 21.1 | 20.8; H = 1536, T = 4500 1.71 | 1.59 | 1.59.  dW of the kept numerators gains from the longer one (H = 1536, four
+  // chunks of 8192 12.0 | 11.6 | 11.7).
+  if (akm && bkm) return launch_tile_kernel<gemm_store_kernel<Cfg8, true, true, false, false>, Cfg8>(p, nb, st);
   if (akm) return launch_tile_kernel<gemm_store_kernel<Cfg8, true, false>, Cfg8>(p, nb, st);
   if (bkm && p.g.seg[0].K >= kLongContraction) return launch_tile_kernel<gemm_store_kernel<Cfg8, false, true, false, false>, Cfg8>(p, nb, st);
   if (bkm) return launch_tile_kernel<gemm_store_kernel<Cfg8, false, true>, Cfg8>(p, nb, st);
