@@ -276,7 +276,7 @@ int fwd_raster_group(const Tuning& tn, int nsplit) {
 // 385 | 363, 1034 466 | 439; H = 8192, V = 128256: T = 560 1196 | 1086.  From 129 columns on little is left to gain.
 // The 64-column tile costs more the more tokens it has, and more of a whole one's time past H = 4096, but for multiples of
 // 4096 (why is not known).  Counted as half there, T = 832 (64 tokens in the last tile) at H = 4608 .. 6144 took 1.05 .. 1.07 of the
-// whole tile's time, T = 1600 1.05 .. 1.11; as 0.55 0.96 .. 1.01 and 0.97 .. 1.06, one box with another; as 0.6 0.94 and 0.97.
+// whole tile's time, T = 1600 1.05 .. 1.11; as 0.55 0.96 .. 1.01 and 0.97 .. 1.06, from run to run; as 0.6 0.94 .. 0.97 and 0.97 .. 0.98.
 // Elsewhere half loses nowhere (T = 832: H = 896 0.89, 1536 and 3584 1.00, 2048 0.94, 4096 0.97, 8192 0.93 .. 0.98), and 0.6 would
 // give up what two whole tiles and a narrow one gain (T = 576: H = 896 0.84, 2048 0.90, 8192 0.91).
 double tail_cost(int nb, int rows, int H) {
