@@ -336,16 +336,16 @@ __global__ __launch_bounds__(256, 2) void varlen_attn_fwd_kernel(AttnParams p) {
       const float m_use = (m_new == -INFINITY) ? 0.f : m_new;
       const float alpha = fast_exp2((m_run - m_use) * c);
       const float mc = m_use * c;
-      float sum = 0.f;
+      float sum[2] = {0.f, 0.f};
 #pragma unroll
       for (int mb = 0; mb < 2; ++mb)
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
           const float e = fast_exp2(__builtin_fmaf(s[mb][r], c, -mc));
           s[mb][r] = e;
-          sum += e;
+          sum[mb] += e;
         }
-      l_run = l_run * alpha + sum;
+      l_run = l_run * alpha + (sum[0] + sum[1]);
       m_run = m_new;
       if (__any(alpha != 1.f)) {      // once the running maxima have settled no lane rescales any more
 #pragma unroll
@@ -466,8 +466,10 @@ __global__ __launch_bounds__(256, 2) void varlen_attn_dq_kernel(AttnParams p) {
 #pragma unroll
       for (int mb = 0; mb < 2; ++mb) {
         f32x16_t s, dp;
+        float ndelta = -dl;
+        asm volatile("" : "+v"(ndelta));                 // spread out anew: sixteen registers that hold it across the loop do not fit
 #pragma unroll
-        for (int r = 0; r < 16; ++r) s[r] = dp[r] = 0.f;
+        for (int r = 0; r < 16; ++r) s[r] = 0.f, dp[r] = ndelta;      // dP - delta
 #pragma unroll
         for (int st = 0; st < KS; ++st) {
           s = FGRPO_MFMA(attn_frag(kt, L, mb, st), qf[st], s);
@@ -476,14 +478,14 @@ __global__ __launch_bounds__(256, 2) void varlen_attn_dq_kernel(AttnParams p) {
         float ds[16];
         if (kb >= w_lo_max && kb + kAttnBK - 1 <= w_hi_min) {   // every pair of this step is visible
 #pragma unroll
-          for (int r = 0; r < 16; ++r) ds[r] = fast_exp2(__builtin_fmaf(s[r], c, -lse2)) * (dp[r] - dl);
+          for (int r = 0; r < 16; ++r) ds[r] = fast_exp2(__builtin_fmaf(s[r], c, -lse2)) * dp[r];
         } else {
 #pragma unroll
           for (int r = 0; r < 16; ++r) {
             const int key = kb + 32 * mb + 8 * (r >> 2) + 4 * h + (r & 3);
             const int vis = (int)(key >= lo) & (int)(key <= hi);
             const float pr = fast_exp2(vis ? __builtin_fmaf(s[r], c, -lse2) : -INFINITY);
-            ds[r] = pr * (dp[r] - dl);
+            ds[r] = pr * dp[r];
           }
         }
 #pragma unroll
@@ -1231,6 +1233,17 @@ __global__ __launch_bounds__(512) void varlen_attn_dkv2_kernel(AttnParams p) {
 //    23.3 (Q, dO and O come from HBM, 96 KiB a work-group: bandwidth) and 1.9 of 19.1.  Forward + backward of that
 //    batch, dK/dV's opening included: 540 -> 498..505 us; 12345 tokens with 14 / 2 heads of 64: 140 -> 133; one sample of
 //    777 tokens, forward: 26.0 -> 24.9; 4 x 8192 tokens with 28 / 4 heads: 8.00 -> 7.91..8.00 ms.
+//  * on short segments vector instructions bind as much as matrix ones (128..1024 tokens, 12 / 2 heads of 128, forward: 0.46
+//    of a SIMD's cycles against 0.31 of its matrix pipe's; the two hardly overlap), so a step has few of them: hidden
+//    scores are found by one unsigned comparison, a 32-key half at a time and only in halves that hold any; the first step
+//    of a wavefront rescales nothing; -delta enters dQ as the addend of dP; the denominator is summed in two chains.
+//    Forward | forward + backward, us, before -> after on one box: that batch 109 | 445 -> 106 | 440; 6000 tokens of
+//    128..2048, 16 / 4 heads 52.8 | 206 -> 46.5 | 192; 2000 of 128..512, 28 / 4 18.7 | 95 -> 17.0 | 91; 777 tokens 19.0 | 60 ->
+//    18.2 | 58; 12345 with 14 / 2 heads of 64 28.8 | 117 -> 27.4 | 113; 4 x 8192, 28 / 4 1860 | 7507 -> 1845 | 7430.
+//    Tried on top and not kept: the next step's first K fragments requested before the barrier (nothing: what is waited for
+//    is issue, not latency); the products of a second half that a wavefront sees nothing of left out (forward +2 % where it
+//    happens, and where it does not); heads and 32-query sub-tiles dealt so that no wavefront idles at seven heads a group
+//    (between -3 and +8 %); tiles of many and few steps side by side in the launch order (+2 .. +10 %).
 // Every value an asm read delivers passes through attn_settle() right after its wait (see varlen_attn_dkv2_kernel).
 // ---------------------------------------------------------------------------------------------------------
 struct AttnTr {
@@ -1362,9 +1375,8 @@ struct AttnTileCursor {
   // loads of the tile at the cursor, by a 256-thread work-group (see attn_dma_lane_offset)
   __device__ __forceinline__ void load(long long st, uint32_t lane_off, char* tile_w) const {
     constexpr int RPI = 1024 / (HD * 2), NLD = kAttnBK / RPI / 4;
-    long long b = bytes > 0 ? bytes : 0;
-    if (b > 0xffffffffLL) b = 0xffffffffLL;
-    const __amdgpu_buffer_rsrc_t rs = make_rsrc(ptr, (uint32_t)b);
+    const int high = (int)(bytes >> 32);       // clamped in halves: the scalar unit compares 32 bits, a 64-bit comparison is a vector instruction's
+    const __amdgpu_buffer_rsrc_t rs = make_rsrc(ptr, high < 0 ? 0u : high > 0 ? 0xffffffffu : (uint32_t)bytes);
 #pragma unroll
     for (int i = 0; i < NLD; ++i)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, FGRPO_LDS_PTR(tile_w + i * 4096), 16, (int)lane_off, (int)(i * 4 * RPI * st * 2), 0, 0);
@@ -1440,13 +1452,15 @@ __global__ __launch_bounds__(256, 2) void varlen_attn_fwd2_kernel(AttnParams p) 
   AttnRows<HD>(p.q + (long long)wf * p.q_st + (long long)hq * p.q_sh, p.q_st, wrows, lane).load(rq);
   __builtin_amdgcn_sched_barrier(0);
 
-  const int lo = valid ? s_tq : 1, hi = valid ? e_tq - 1 : 0;
+  const int lo = s_tq;
+  const uint32_t n_vis = valid ? (uint32_t)max(e_tq - s_tq, 0) : 0u;      // keys lo .. lo + n_vis - 1 are seen
   f32x16_t acc_o[DB];
 #pragma unroll
   for (int db = 0; db < DB; ++db)
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc_o[db][r] = 0.f;
   float m_run = -INFINITY, l_run = 0.f;
+  bool started = false;                    // the accumulators hold something
   const float c = p.scale * kLog2e;
   // the rows pass through this wavefront's part of the second buffer, which the first step fills again
   const uint32_t patch = lds0 + 2 * kAttnTile + wave * (32 * HD * 2);
@@ -1519,22 +1533,18 @@ __global__ __launch_bounds__(256, 2) void varlen_attn_fwd2_kernel(AttnParams p) 
       __builtin_amdgcn_sched_barrier(0);
 
       float mx = -INFINITY;
-      if (kb >= w_lo_max && kb + kAttnBK - 1 <= w_hi_min) {   // every pair of this step is visible
 #pragma unroll
-        for (int mb = 0; mb < 2; ++mb)
+      for (int mb = 0; mb < 2; ++mb) {
+        if (!(kb + 32 * mb >= w_lo_max && kb + 32 * mb + 31 <= w_hi_min)) {      // some pair of this half is hidden
+          const uint32_t k0 = (uint32_t)(kb + 32 * mb + 4 * h - lo);
 #pragma unroll
-          for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[mb][r]);
-      } else {
-#pragma unroll
-        for (int mb = 0; mb < 2; ++mb)
-#pragma unroll
-          for (int r = 0; r < 16; ++r) {
-            const int key = kb + 32 * mb + 8 * (r >> 2) + 4 * h + (r & 3);
-            const float x = (key >= lo && key <= hi) ? s[mb][r] : -INFINITY;
-            s[mb][r] = x;
-            mx = fmaxf(mx, x);
-          }
+          for (int r = 0; r < 16; ++r) s[mb][r] = k0 + (uint32_t)(8 * (r >> 2) + (r & 3)) < n_vis ? s[mb][r] : -INFINITY;
+        }
       }
+#pragma unroll
+      for (int mb = 0; mb < 2; ++mb)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[mb][r]);
       {
         float mlo, mhi;
         attn_halves(mx, mlo, mhi);
@@ -1544,18 +1554,18 @@ __global__ __launch_bounds__(256, 2) void varlen_attn_fwd2_kernel(AttnParams p) 
       const float m_use = (m_new == -INFINITY) ? 0.f : m_new;
       const float alpha = fast_exp2((m_run - m_use) * c);
       const float mc = m_use * c;
-      float sum = 0.f;
+      float sum[2] = {0.f, 0.f};             // two chains of additions
 #pragma unroll
       for (int mb = 0; mb < 2; ++mb)
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
           const float e = fast_exp2(__builtin_fmaf(s[mb][r], c, -mc));
           s[mb][r] = e;
-          sum += e;
+          sum[mb] += e;
         }
-      l_run = l_run * alpha + sum;
+      l_run = l_run * alpha + (sum[0] + sum[1]);
       m_run = m_new;
-      if (__any(alpha != 1.f)) {      // once the running maxima have settled no lane rescales any more
+      if (started && __any(alpha != 1.f)) {      // zeros need no rescaling; once the running maxima have settled no lane rescales any more
 #pragma unroll
         for (int db = 0; db < DB; ++db)
 #pragma unroll
@@ -1576,6 +1586,7 @@ __global__ __launch_bounds__(256, 2) void varlen_attn_fwd2_kernel(AttnParams p) 
         for (int db = 0; db < DB; ++db) acc_o[db] = attn_mfma(attn_settle_tr(vq[q % 2][db]), pf, acc_o[db]);
         __builtin_amdgcn_sched_barrier(0);
       });
+      started = true;
     }
     FGRPO_WAIT_VMCNT(0);            // this wavefront's part of the next tile is in LDS
     wait_lgkm<0>();
@@ -1688,7 +1699,8 @@ __global__ __launch_bounds__(256, 2) void varlen_attn_dq2_kernel(AttnParams p) {
   const float lse2 = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(make_rsrc(p.lse + (long long)hq * p.T + wf, (uint32_t)wrows * 4), (lane & 31) * 4, 0, 0)) * kLog2e;
   __builtin_amdgcn_sched_barrier(0);
 
-  const int lo = valid ? s_tq : 1, hi = valid ? e_tq - 1 : 0;
+  const int lo = s_tq;
+  const uint32_t n_vis = valid ? (uint32_t)max(e_tq - s_tq, 0) : 0u;      // keys lo .. lo + n_vis - 1 are seen
   const float c = p.scale * kLog2e;
   f32x16_t acc[DB];
 #pragma unroll
@@ -1721,6 +1733,10 @@ __global__ __launch_bounds__(256, 2) void varlen_attn_dq2_kernel(AttnParams p) {
   // zero from the score, see hide() below): -inf * c + inf would be a NaN
   float lse2_v = lse2 == -INFINITY ? 0.f : lse2;
   asm volatile("" : "+v"(lse2_v));
+  f32x16_t ndelta;                         // the addend of dP (kept: it is one operand register block of every step)
+#pragma unroll
+  for (int r = 0; r < 16; ++r) ndelta[r] = -dl;
+  asm volatile("" : "+v"(ndelta));
   FGRPO_WAIT_VMCNT(0);
   wg_barrier();
   // a step on LDS buffer `cur`, a compile-time constant: buffer, tile and block are the instruction's offset field
@@ -1728,7 +1744,7 @@ __global__ __launch_bounds__(256, 2) void varlen_attn_dq2_kernel(AttnParams p) {
     constexpr int cur = decltype(curc)::value, kt = cur * 2 * kAttnTile, vt = kt + kAttnTile;
     if (kb + kAttnBK < k_end) fetch(cur ^ 1);     // the next step's tiles; that buffer was last read a step ago, before the barrier
     if (wave_on && kb <= w_hi && kb + kAttnBK > w_lo) {
-      const bool all_vis = kb >= w_lo_max && kb + kAttnBK - 1 <= w_hi_min;       // every pair of this step is visible
+      auto all_vis = [&](int mb) { return kb + 32 * mb >= w_lo_max && kb + 32 * mb + 31 <= w_hi_min; };      // every pair of this half
       // The two 32-key halves of the step as a software pipeline in which the vector arithmetic of a half runs in
       // the shadow of matrix instructions (a 32x32x16 instruction keeps the matrix pipe busy for 32 cycles and the
       // issue port for about 8: four or five vector instructions fit behind each one for free, whereas a wavefront
@@ -1746,7 +1762,7 @@ __global__ __launch_bounds__(256, 2) void varlen_attn_dq2_kernel(AttnParams p) {
 #pragma unroll
         for (int mb = 0; mb < 2; ++mb)
 #pragma unroll
-          for (int r = 0; r < 16; ++r) sc[mb][r] = dp[mb][r] = 0.f;
+          for (int r = 0; r < 16; ++r) sc[mb][r] = 0.f;
         auto fence = []() { __builtin_amdgcn_sched_barrier(0); };
         // group n = 0 .. 7 of the row fragments: product n / 2 (S(0), dP(0), S(1), dP(1)), k steps GR (n % 2) ..
         auto req_g = [&](auto nc) {
@@ -1774,15 +1790,13 @@ __global__ __launch_bounds__(256, 2) void varlen_attn_dq2_kernel(AttnParams p) {
         // sixteen selects: one around a whole phase costs copies of the accumulators it merges.
         auto hide = [&](auto mbc) {
           constexpr int mb = decltype(mbc)::value;
+          const uint32_t k0 = (uint32_t)(kb + 32 * mb + 4 * h - lo);
 #pragma unroll
-          for (int r = 0; r < 16; ++r) {
-            const int key = kb + 32 * mb + 8 * (r >> 2) + 4 * h + (r & 3);
-            sc[mb][r] = ((int)(key >= lo) & (int)(key <= hi)) ? sc[mb][r] : -INFINITY;
-          }
+          for (int r = 0; r < 16; ++r) sc[mb][r] = k0 + (uint32_t)(8 * (r >> 2) + (r & 3)) < n_vis ? sc[mb][r] : -INFINITY;
         };
         auto f_el = [&](auto mbc, auto rc) {             // dS in place of P
           constexpr int mb = decltype(mbc)::value, r = decltype(rc)::value;
-          sc[mb][r] = sc[mb][r] * (dp[mb][r] - dl);
+          sc[mb][r] = sc[mb][r] * dp[mb][r];
           asm volatile("" : "+v"(sc[mb][r]));
         };
         u32x4_t dsf[2][2];
@@ -1800,7 +1814,7 @@ __global__ __launch_bounds__(256, 2) void varlen_attn_dq2_kernel(AttnParams p) {
             constexpr int i = decltype(ic)::value, st = GR * (n % 2) + i;
             attn_settle(fr[n % 2][i]);
             if constexpr (prod % 2 == 0) sc[mb] = attn_mfma(fr[n % 2][i], __builtin_bit_cast(u32x4_t, qf[st]), sc[mb]);
-            else dp[mb] = attn_mfma(fr[n % 2][i], __builtin_bit_cast(u32x4_t, dof[st]), dp[mb]);
+            else dp[mb] = attn_mfma(fr[n % 2][i], __builtin_bit_cast(u32x4_t, dof[st]), st == 0 ? ndelta : dp[mb]);
             fence();       // the matrix instruction first: the vector work then runs while the pipe is busy
             side(ic);
             fence();
@@ -1832,7 +1846,7 @@ __global__ __launch_bounds__(256, 2) void varlen_attn_dq2_kernel(AttnParams p) {
         mma_g(std::integral_constant<int, 1>{}, none);
         // ---- dP(0) + E(0)
         req_g(std::integral_constant<int, 3>{});
-        if (!all_vis) hide(I0{});
+        if (!all_vis(0)) hide(I0{});
         wait_lgkm<GR>();
         fence();
         mma_g(std::integral_constant<int, 2>{}, side_e(I0{}, I0{}));
@@ -1853,7 +1867,7 @@ __global__ __launch_bounds__(256, 2) void varlen_attn_dq2_kernel(AttnParams p) {
         pack(I0{}, I1{});
         // ---- dP(1) + E(1)
         req_g(std::integral_constant<int, 7>{});
-        if (!all_vis) hide(I1{});
+        if (!all_vis(1)) hide(I1{});
         wait_lgkm<GR>();
         fence();
         mma_g(std::integral_constant<int, 6>{}, side_e(I1{}, I0{}));
