@@ -70,7 +70,7 @@ struct AttnParams {
   // launches whose tiles are dealt to several work-groups (SPLIT kernels, see attn_parts); q: query side, k: key side
   int parts_q, per_q, blocks_q;      // most parts of a tile, steps a part is meant to walk, work-groups of one part
   int parts_k, per_k, blocks_k;      // the same; steps: items of a wavefront
-  float* part_q;         // [parts_q][T][Hq][HD] O of the part, relative to its own maximum, or its dQ / scale
+  float* part_q;         // [parts_q][ceil(T / 32)][Hq][32 x HD as attn_store_partial leaves them] O of the part, relative to its own maximum, or its dQ / scale
   float2* part_ml;       // [parts_q][Hq][T] forward: maximum and sum of the part
   float* part_k;         // [parts_k][2][T][Hkv][HD] dK / scale and dV of the part
 };
@@ -226,14 +226,19 @@ __device__ __forceinline__ void attn_store_rowmajor(const f32x16_t (&acc)[DB], f
     }
 }
 
-// ... and the same accumulator as it is, in fp32
+// ... and the same accumulator as it lies in the registers, in fp32: a part's sums of 32 tokens of one head, 1 KiB an instruction.
+// Columns 32 db + 8 g + 4 h .. + 3 of token n of the 32 are the 16 bytes at 64 (4 db + g) + 32 h + n.
+template <int HD>
+__device__ __forceinline__ float* attn_partial(const AttnParams& p, int part, int t, int hq) {
+  return p.part_q + (((long long)part * ((p.T + 31) / 32) + t / 32) * p.Hq + hq) * (32 * HD);
+}
 template <int DB>
-__device__ __forceinline__ void attn_store_partial(const f32x16_t (&acc)[DB], float* row_ptr, int h) {
+__device__ __forceinline__ void attn_store_partial(const f32x16_t (&acc)[DB], float* tile, int lane) {
 #pragma unroll
   for (int db = 0; db < DB; ++db)
 #pragma unroll
     for (int g = 0; g < 4; ++g)
-      *(float4*)(row_ptr + 32 * db + 8 * g + 4 * h) = make_float4(acc[db][4 * g], acc[db][4 * g + 1], acc[db][4 * g + 2], acc[db][4 * g + 3]);
+      *(float4*)(tile + (64 * (4 * db + g) + lane) * 4) = make_float4(acc[db][4 * g], acc[db][4 * g + 1], acc[db][4 * g + 2], acc[db][4 * g + 3]);
 }
 
 // ---------------------------------------------------------------------------------------------------------
@@ -1601,8 +1606,8 @@ __global__ __launch_bounds__(256, 2) void varlen_attn_fwd2_kernel(AttnParams p) 
   const float l = l_lo + l_hi;
   if constexpr (SPLIT) {
     if (np > 1) {
+      if (wrows > 0) attn_store_partial(acc_o, attn_partial<HD>(p, part, wfirst, hq), lane);
       if (valid) {
-        attn_store_partial(acc_o, p.part_q + (((long long)part * p.T + tq) * p.Hq + hq) * kHD, h);
         if (h == 0) p.part_ml[((long long)part * p.Hq + hq) * p.T + tq] = make_float2(m_run, l);
       }
       return;
@@ -1912,7 +1917,7 @@ __global__ __launch_bounds__(256, 2) void varlen_attn_dq2_kernel(AttnParams p) {
   }
   if constexpr (SPLIT) {
     if (np > 1) {
-      if (valid) attn_store_partial(acc, p.part_q + (((long long)part * p.T + tq) * p.Hq + hq) * kHD, h);
+      if (wrows > 0) attn_store_partial(acc, attn_partial<HD>(p, part, wfirst, hq), lane);
       return;
     }
   }
@@ -1929,45 +1934,53 @@ __global__ __launch_bounds__(256, 2) void varlen_attn_dq2_kernel(AttnParams p) {
   attn_store_rows<HD>(acc, p.scale, AttnRows<HD>(p.dq + ((long long)wf * p.Hq + hq) * kHD, (long long)p.Hq * kHD, wrows, lane_e), patch_out, rowo, lane_e);   // dS was kept / scale
 }
 
-__device__ __forceinline__ void attn_load8(const float* src, float (&v)[8]) {
-  const float4 a = *(const float4*)src, b = *(const float4*)(src + 4);
-  v[0] = a.x, v[1] = a.y, v[2] = a.z, v[3] = a.w, v[4] = b.x, v[5] = b.y, v[6] = b.z, v[7] = b.w;
-}
-// Sums of the parts of a query tile, in part order: eight columns of one (token, head) a thread.  Rows of tiles that were
-// not dealt out are already in place.  FWD: every part is relative to its own maximum.
+// Sums of the parts of 32 tokens of one head, in part order, by a work-group of 256 threads: thread (n, i) takes eight columns,
+// 32 db + 8 g .., of token n for 4 db + g = i and i + 8, and the results pass through LDS to leave by rows.  Tiles that were not
+// dealt out are already in place.  FWD: every part is relative to its own maximum.
 // Bound by latency: a thread's time is its chain of round trips, so the loads of kAttnMergeWide parts go out together (the
-// first part again for those a tile does not have).  777 tokens with 12 heads of 128: 5.2 -> 4.3 us.
+// first part again for those a tile does not have).  Partial sums used to lie by rows: a store of a part touched 32 rows, 32 bytes
+// of each, and took the address unit as long as eight.  Forward, merge included, | backward, us, before -> after: one segment of 777
+// tokens with 12 / 2 heads of 128 18.1 | 39.9 -> 16.7 | 38.9, of 2000 37.4 | 93.6 -> 34.1 | 91.5, of 3000 60.8 | 156.7 -> 56.8 | 153.5;
+// 900 with 14 / 2 heads of 64 16.5 | 30.4 -> 15.1 | 29.8.  (Read by threads along a row, with these sums 1 KiB apart, the merge
+// alone took 6 us more.)  Parts half as long or less, which cheaper merges might pay for, are slower still (777 tokens 18.7).
 template <int HD, bool FWD>
-__device__ __forceinline__ void attn_merge_query_row(const AttnParams& p, int RB, long long idx) {
-  const int col = (int)(idx % (HD / 8)) * 8;
-  const long long row = idx / (HD / 8);                    // token * Hq + head
-  const int hq = (int)(row % p.Hq);
-  const int t = (int)(row / p.Hq);
-  if (t >= p.T) return;
+__device__ __forceinline__ void attn_merge_query_tile(const AttnParams& p, int RB, int idx) {
+  constexpr int NC = HD / 64;                              // pieces of eight columns a thread
+  __shared__ __attribute__((aligned(16))) char smem[32 * HD * 2];
+  const int t0 = idx / p.Hq * 32, hq = idx % p.Hq, n = threadIdx.x % 32, i0 = threadIdx.x / 32;
   int k_begin, k_end;
-  attn_query_tile_keys(p, t / RB * RB, RB, k_begin, k_end);
+  attn_query_tile_keys(p, t0 / RB * RB, RB, k_begin, k_end);
   const int np = attn_parts(attn_steps(k_begin, k_end), p.parts_q, p.per_q);
   if (np <= 1) return;
-  float x[8];
+  const int t = min(t0 + n, p.T - 1);
+  float x[NC][8];
 #pragma unroll
-  for (int e = 0; e < 8; ++e) x[e] = 0.f;
+  for (int c = 0; c < NC; ++c)
+#pragma unroll
+    for (int e = 0; e < 8; ++e) x[c][e] = 0.f;
   float mul = p.scale, m = -INFINITY, l = 0.f;
   float2 ml[kAttnMaxParts];
   if constexpr (FWD) {
 #pragma unroll
     for (int j = 0; j < kAttnMaxParts; ++j) ml[j] = p.part_ml[((long long)(j < np ? j : 0) * p.Hq + hq) * p.T + t];
-#pragma unroll
-    for (int j = 0; j < kAttnMaxParts; ++j) m = j < np ? fmaxf(m, ml[j].x) : m;
   }
-  const float m_use = m == -INFINITY ? 0.f : m;
-  const float* src = p.part_q + row * HD + col;
-  const long long slice = (long long)p.T * p.Hq * HD;
+  const float* src = attn_partial<HD>(p, 0, t0, hq) + (64 * i0 + n) * 4;
+  const long long slice = (long long)((p.T + 31) / 32) * p.Hq * (32 * HD);
 #pragma unroll
   for (int j0 = 0; j0 < kAttnMaxParts; j0 += kAttnMergeWide) {
     if (j0 >= np) break;
-    float v[kAttnMergeWide][8];
+    float4 v[kAttnMergeWide][NC][2];
 #pragma unroll
-    for (int u = 0; u < kAttnMergeWide; ++u) attn_load8(src + (j0 + u < np ? j0 + u : 0) * slice, v[u]);
+    for (int u = 0; u < kAttnMergeWide; ++u)
+#pragma unroll
+      for (int c = 0; c < NC; ++c)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) v[u][c][h] = *(const float4*)(src + (j0 + u < np ? j0 + u : 0) * slice + c * (8 * 256) + h * 128);
+    if (FWD && j0 == 0) {
+#pragma unroll
+      for (int j = 0; j < kAttnMaxParts; ++j) m = j < np ? fmaxf(m, ml[j].x) : m;
+    }
+    const float m_use = m == -INFINITY ? 0.f : m;
 #pragma unroll
     for (int u = 0; u < kAttnMergeWide; ++u) {
       if (j0 + u >= np) continue;
@@ -1977,20 +1990,36 @@ __device__ __forceinline__ void attn_merge_query_row(const AttnParams& p, int RB
         l = __builtin_fmaf(ml[j0 + u].y, w, l);
       }
 #pragma unroll
-      for (int e = 0; e < 8; ++e) x[e] = FWD ? __builtin_fmaf(v[u][e], w, x[e]) : x[e] + v[u][e];
+      for (int c = 0; c < NC; ++c)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const float4 q = v[u][c][e / 4];
+          const float y = e % 4 == 0 ? q.x : e % 4 == 1 ? q.y : e % 4 == 2 ? q.z : q.w;
+          x[c][e] = FWD ? __builtin_fmaf(y, w, x[c][e]) : x[c][e] + y;
+        }
     }
   }
   if constexpr (FWD) {
     mul = l > 0.f ? 1.f / l : 0.f;
-    if (col == 0) p.lse[(long long)hq * p.T + t] = l > 0.f ? m * p.scale + __logf(l) : -INFINITY;
+    if (i0 == 0 && t0 + n < p.T) p.lse[(long long)hq * p.T + t] = l > 0.f ? m * p.scale + __logf(l) : -INFINITY;
   }
 #pragma unroll
-  for (int e = 0; e < 8; ++e) x[e] *= mul;
-  *(bf16x8_t*)((FWD ? p.out : p.dq) + row * HD + col) = attn_pack8(x);
+  for (int c = 0; c < NC; ++c) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) x[c][e] *= mul;
+    *(bf16x8_t*)(smem + n * (HD * 2) + (((i0 + 8 * c) ^ attn_swz<HD>(n)) << 4)) = attn_pack8(x[c]);
+  }
+  __syncthreads();
+#pragma unroll
+  for (int c = 0; c < NC; ++c) {
+    const int row = (threadIdx.x + 256 * c) / (HD / 8), ch = threadIdx.x % (HD / 8);
+    if (t0 + row < p.T)
+      *(u32x4_t*)((FWD ? p.out : p.dq) + ((long long)(t0 + row) * p.Hq + hq) * HD + ch * 8) = *(const u32x4_t*)(smem + row * (HD * 2) + ((ch ^ attn_swz<HD>(row)) << 4));
+  }
 }
 template <int HD>
 static __global__ __launch_bounds__(256) void attn_merge_fwd_kernel(AttnParams p, int RB) {
-  attn_merge_query_row<HD, true>(p, RB, (long long)blockIdx.x * 256 + threadIdx.x);
+  attn_merge_query_tile<HD, true>(p, RB, blockIdx.x);
 }
 
 // seg_start[t], seg_end[t] from cu_seqlens (tokens outside every segment stand alone)

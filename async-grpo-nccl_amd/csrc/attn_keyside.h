@@ -604,16 +604,19 @@ __global__ __launch_bounds__(256, KB == 2 ? 1 : 2) void varlen_attn_dkv3_kernel(
   sum_store(std::integral_constant<int, kAccV>{}, 1.f, p.dv, 1);
 }
 
-// Sums of the parts, in part order, of dK and dV (key tiles of kKeys) and of dQ (query tiles of RB tokens): eight columns
-// of one row a thread.  Rows of tiles that were not dealt out are already in place.
+__device__ __forceinline__ void attn_load8(const float* src, float (&v)[8]) {
+  const float4 a = *(const float4*)src, b = *(const float4*)(src + 4);
+  v[0] = a.x, v[1] = a.y, v[2] = a.z, v[3] = a.w, v[4] = b.x, v[5] = b.y, v[6] = b.z, v[7] = b.w;
+}
+// Sums of the parts, in part order, of dQ (the first nq work-groups, see attn_merge_query_tile) and of dK and dV (key tiles of
+// kKeys): eight columns of one row a thread.  Rows of tiles that were not dealt out are already in place.
 template <int HD, int kKeys>
-static __global__ __launch_bounds__(256) void attn_merge_bwd_kernel(AttnParams p, int RB, long long nq, long long nk) {
-  long long idx = (long long)blockIdx.x * 256 + threadIdx.x;
-  if (idx < nq) {
-    attn_merge_query_row<HD, false>(p, RB, idx);
+static __global__ __launch_bounds__(256) void attn_merge_bwd_kernel(AttnParams p, int RB, int nq, long long nk) {
+  if ((int)blockIdx.x < nq) {
+    attn_merge_query_tile<HD, false>(p, RB, blockIdx.x);
     return;
   }
-  idx -= nq;
+  long long idx = (long long)((int)blockIdx.x - nq) * 256 + threadIdx.x;
   if (idx >= 2 * nk) return;
   const int which = idx >= nk;
   if (which) idx -= nk;

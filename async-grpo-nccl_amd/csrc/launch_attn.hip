@@ -68,7 +68,7 @@ struct DqLauncher {
 // causal launch walk 0 .. chain steps, evenly; segments of one call are taken to be as long as their mean (twice that
 // at most: the number of parts allowed for); one long segment among many short ones is judged by that mean and may stay
 // whole.  Decided by shapes alone.  Whole | dealt out, merge launch included, 12 / 2 heads of 128: one segment of 777
-// tokens, forward 25.2 | 19.2 us, backward 86.7 | 44.2; of 6000 tokens 182 | 161 and 584 | 465; 3 segments of 1024 tokens,
+// tokens, forward 25.2 | 19.2 us (16.7 now, see attn_merge_query_tile), backward 86.7 | 44.2 (38.9); of 6000 tokens 182 | 161 and 584 | 465; 3 segments of 1024 tokens,
 // backward (dK/dV alone is dealt out) 106 | 85, forward 29.2 | 42, which the estimate refuses.
 struct SplitPlan {
   int parts = 1, per = 1;
@@ -114,9 +114,10 @@ SplitPlan plan_key_split(int form, int T, int n_seq, int Hq, int Hkv, int D, int
   return plan_split(wgs, D == 128 ? 1 : 2, chain, causal, D == 128 ? 1.3 : 0.65, (size_t)T * Hkv * D * 8);
 }
 size_t align256(size_t n) { return (n + 255) / 256 * 256; }
+size_t query_sums_bytes(const SplitPlan& s, int T, int Hq, int D) { return align256((size_t)s.parts * ((T + 31) / 32 * 32) * Hq * D * 4); }
 size_t query_split_bytes(const SplitPlan& s, int T, int Hq, int D, bool forward) {
   if (s.parts <= 1) return 0;
-  return align256((size_t)s.parts * T * Hq * D * 4) + (forward ? align256((size_t)s.parts * T * Hq * 8) : 0);
+  return query_sums_bytes(s, T, Hq, D) + (forward ? align256((size_t)s.parts * T * Hq * 8) : 0);
 }
 size_t key_split_bytes(const SplitPlan& s, int T, int Hkv, int D) { return s.parts <= 1 ? 0 : align256((size_t)s.parts * T * Hkv * D * 8); }
 }  // namespace
@@ -209,10 +210,10 @@ int fgrpo_varlen_attn_fwd_ws(const void* q, const void* k, const void* v, long l
   else if (!aligned16(ws)) return fail(FGRPO_ERR_ALIGN, "varlen_attn_fwd: workspace must be 16-byte aligned");
   p.parts_q = sp.parts, p.per_q = sp.per;
   p.part_q = (float*)ws;
-  p.part_ml = (float2*)((char*)ws + align256((size_t)sp.parts * T * Hq * D * 4));
+  p.part_ml = (float2*)((char*)ws + query_sums_bytes(sp, T, Hq, D));
   rc = launch_query_side<FwdLauncher>(form, D, hb, p, T, Hq, Hkv, bounds_ws, st);
   if (rc || sp.parts <= 1) return rc;
-  const unsigned blocks = (unsigned)(((long long)T * Hq * (D / 8) + 255) / 256);
+  const unsigned blocks = (unsigned)((T + 31) / 32) * (unsigned)Hq;
   if (D == 128) hipLaunchKernelGGL(attn_merge_fwd_kernel<128>, dim3(blocks), dim3(256), 0, st, p, 128 / hb);
   else hipLaunchKernelGGL(attn_merge_fwd_kernel<64>, dim3(blocks), dim3(256), 0, st, p, 128 / hb);
   HIP_TRY(hipGetLastError());

@@ -33,8 +33,9 @@ int launch_attn_dkv3(int D, const AttnParams& p, hipStream_t st) {
 int attn_keyside_keys(int D) { return D == 128 ? 64 : 32; }
 
 int launch_attn_merge_bwd(int D, const AttnParams& p, int rb, hipStream_t st) {
-  const long long nq = p.parts_q > 1 ? (long long)p.T * p.Hq * (D / 8) : 0, nk = p.parts_k > 1 ? (long long)p.T * p.Hkv * (D / 8) : 0;
-  const dim3 grid((unsigned)((nq + 2 * nk + 255) / 256));
+  const int nq = p.parts_q > 1 ? (p.T + 31) / 32 * p.Hq : 0;
+  const long long nk = p.parts_k > 1 ? (long long)p.T * p.Hkv * (D / 8) : 0;
+  const dim3 grid((unsigned)(nq + (2 * nk + 255) / 256));
   if (D == 128) hipLaunchKernelGGL((attn_merge_bwd_kernel<128, 64>), grid, dim3(256), 0, st, p, rb, nq, nk);
   else hipLaunchKernelGGL((attn_merge_bwd_kernel<64, 32>), grid, dim3(256), 0, st, p, rb, nq, nk);
   HIP_TRY(hipGetLastError());
