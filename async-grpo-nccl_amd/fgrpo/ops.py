@@ -44,7 +44,8 @@ def _ptr(t: Optional[torch.Tensor]):
 
 
 def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    """The current device's current stream, as the number a launch takes (``current_stream()`` makes an object for it)."""
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
 
 
 def _code(dtype: torch.dtype) -> int:

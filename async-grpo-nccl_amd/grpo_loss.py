@@ -408,6 +408,18 @@ def compute_dual_clip_grpo_loss(
     with the metric keys of the reference (grpo_loss.py:478-498).  All
     diagnostics over ``output_indices`` come from one kernel launch and reach the
     host in one copy instead of ~20 ``.item()`` syncs."""
+    loss, read_metrics = dual_clip_grpo_loss_begin(policy_model, minibatch, clip_low, clip_high, clip_ratio_c,
+                                                   compute_entropy, apply_entropy_bonus, entropy_coeff)
+    return loss, read_metrics()
+
+
+def dual_clip_grpo_loss_begin(policy_model, minibatch, clip_low: float, clip_high: float, clip_ratio_c: float,
+                              compute_entropy: bool = True, apply_entropy_bonus: bool = True, entropy_coeff: float = 0.0):
+    """``compute_dual_clip_grpo_loss`` in two halves: ``(loss, read_metrics)``, nothing waited for yet.
+    ``read_metrics()`` waits for the copy of the diagnostics, queued here behind the forward, and returns the metric
+    dictionary.  A trainer that calls ``backward()`` in between has the rest of its work queued before the device runs
+    out of it: waiting first left the device idle while the host launched the backward (a micro-batch of 16 samples and
+    a head of 151936 x 896: 6100 us, 5746 this way)."""
     batch_ids = minibatch["batch_ids"]
     batch_position_ids = minibatch["batch_position_ids"]
     output_indices = minibatch["output_indices"]
@@ -450,46 +462,54 @@ def compute_dual_clip_grpo_loss(
         tail = [grpo_output.loss.detach().double().reshape(1)]
         if torch.is_tensor(num_samples_tensor):
             tail.append(num_samples_tensor.detach().double().reshape(1).to(stats_dev.device))
-        host = torch.cat([stats_dev] + tail).cpu().tolist()
-    st, loss_sum = host[:ops._lib.NUM_STATS], float(host[ops._lib.NUM_STATS])
-    num_samples = int(host[ops._lib.NUM_STATS + 1]) if len(host) > ops._lib.NUM_STATS + 1 else \
-        (int(num_samples_tensor) if num_samples_tensor is not None else 0)
-    n = st[0]
-    mean = (lambda s: s / n) if n > 0 else (lambda s: 0.0)
-
-    def pop_std(s1, s2):
-        if n <= 1:
-            return 0.0
-        m = s1 / n
-        return max(s2 / n - m * m, 0.0) ** 0.5
-
-    expected_out = int(output_indices.numel())
-
-    metrics = {
-        "loss": loss_sum,
-        "loss_per_token": (loss_sum / max(1, expected_out)) if expected_out > 0 else float(loss_sum),
-        "loss_per_sample": (loss_sum / max(1, num_samples)) if num_samples > 0 else float(loss_sum),
-        "pg_loss": loss_sum,
-        "pg_clip": int(st[13]),
-        "kl_div": mean(st[1]),
-        "entropy": mean(st[7]),
-        "old_policy_entropy": mean(st[8]) if old_entropy is not None else 0.0,
-        "entropy_coeff": float(entropy_coeff),
-        "approx_kl": mean(st[4]),
-        "clipfrac_upper": mean(st[5]),
-        "clipfrac_lower": mean(st[6]),
-        "log_ratio_mean": mean(st[2]),
-        "log_ratio_std": pop_std(st[2], st[3]),
-        "adv_mean": mean(st[9]),
-        "adv_std": pop_std(st[9], st[10]),
-        "adv_pos_frac": mean(st[11]),
-        "adv_zero_frac": mean(st[12]),
-    }
+        stacked = torch.cat([stats_dev] + tail)
+        buf = torch.empty(stacked.numel(), dtype=torch.float64, pin_memory=True)
+        buf.copy_(stacked, non_blocking=True)
+        copied = torch.cuda.Event()
+        copied.record(torch.cuda.current_stream(stacked.device))
 
     final_loss = grpo_output.loss
-    if compute_entropy and apply_entropy_bonus and float(entropy_coeff) != 0.0 and n > 0:
-        # entropy carries no gradient: the bonus shifts the value only (reference: grpo_loss.py:500-511)
-        entropy_mean = (stats_dev[7] / stats_dev[0]).to(final_loss.dtype)
+    if compute_entropy and apply_entropy_bonus and float(entropy_coeff) != 0.0:
+        # entropy carries no gradient: the bonus shifts the value only (reference: grpo_loss.py:500-511); nothing to add
+        # where no position counts
+        entropy_mean = (stats_dev[7] / stats_dev[0].clamp(min=1.0)).to(final_loss.dtype)
         final_loss = final_loss - float(entropy_coeff) * entropy_mean
+    expected_out = int(output_indices.numel())
 
-    return final_loss, metrics
+    def read_metrics() -> dict:
+        copied.synchronize()
+        host = buf.tolist()
+        st, loss_sum = host[:ops._lib.NUM_STATS], float(host[ops._lib.NUM_STATS])
+        num_samples = int(host[ops._lib.NUM_STATS + 1]) if len(host) > ops._lib.NUM_STATS + 1 else \
+            (int(num_samples_tensor) if num_samples_tensor is not None else 0)
+        n = st[0]
+        mean = (lambda s: s / n) if n > 0 else (lambda s: 0.0)
+
+        def pop_std(s1, s2):
+            if n <= 1:
+                return 0.0
+            m = s1 / n
+            return max(s2 / n - m * m, 0.0) ** 0.5
+
+        return {
+            "loss": loss_sum,
+            "loss_per_token": (loss_sum / max(1, expected_out)) if expected_out > 0 else float(loss_sum),
+            "loss_per_sample": (loss_sum / max(1, num_samples)) if num_samples > 0 else float(loss_sum),
+            "pg_loss": loss_sum,
+            "pg_clip": int(st[13]),
+            "kl_div": mean(st[1]),
+            "entropy": mean(st[7]),
+            "old_policy_entropy": mean(st[8]) if old_entropy is not None else 0.0,
+            "entropy_coeff": float(entropy_coeff),
+            "approx_kl": mean(st[4]),
+            "clipfrac_upper": mean(st[5]),
+            "clipfrac_lower": mean(st[6]),
+            "log_ratio_mean": mean(st[2]),
+            "log_ratio_std": pop_std(st[2], st[3]),
+            "adv_mean": mean(st[9]),
+            "adv_std": pop_std(st[9], st[10]),
+            "adv_pos_frac": mean(st[11]),
+            "adv_zero_frac": mean(st[12]),
+        }
+
+    return final_loss, read_metrics

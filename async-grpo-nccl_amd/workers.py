@@ -16,7 +16,7 @@ import numpy as np
 import torch
 
 from fgrpo import ops
-from grpo_loss import compute_dual_clip_grpo_loss, make_grpo_forward
+from grpo_loss import dual_clip_grpo_loss_begin, make_grpo_forward
 from sample_processing_utils import PackedLogProbs, _fill, post_process_batch
 
 
@@ -57,7 +57,7 @@ class TrainerHarness:
             return {"loss": 0.0, "pg_clip": 0, "kl_div": 0.0, "entropy": 0.0}
         cfg = self.config
         with torch.autocast(device_type="cuda", dtype=torch.bfloat16):
-            loss, metrics = compute_dual_clip_grpo_loss(
+            loss, read_metrics = dual_clip_grpo_loss_begin(
                 self.actor_module_fsdp, batch, cfg.clip_low, cfg.clip_high, cfg.clip_ratio_c,
                 compute_entropy=bool(getattr(cfg, "compute_entropy", True)),
                 apply_entropy_bonus=bool(getattr(cfg, "apply_entropy_bonus", True)),
@@ -72,7 +72,7 @@ class TrainerHarness:
             loss = loss * scale
         loss.backward()
         self._mb_count_since_last_step += 1
-        return metrics
+        return read_metrics()           # the host waits here, with the backward already queued
 
 
 def _takes_keyword(forward, name: str) -> bool:

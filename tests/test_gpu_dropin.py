@@ -445,6 +445,22 @@ def test_trainer_harness_scaling_and_dummy(dev):
     assert tr.compute_gradients([{"dummy": True}], 0) == {"loss": 0.0, "pg_clip": 0, "kl_div": 0.0, "entropy": 0.0}
 
 
+@pytest.mark.parametrize("scored", [True, False])
+def test_metrics_read_after_the_backward_are_those_read_before_it(dev, scored):
+    """The diagnostics are queued behind the forward and read when asked for: a backward in between changes nothing,
+    and a batch without output positions gets no entropy bonus (0 / 0 would be NaN)."""
+    import sample_processing_utils as spu
+    model, G = _patched(dev, "training")
+    batch = spu.post_process_batch(make_samples(5, seed=9), dev)
+    if not scored:
+        batch["output_indices"] = batch["output_indices"][:0]
+    want_loss, want = G.compute_dual_clip_grpo_loss(model, batch, 0.2, 0.28, 3.0, entropy_coeff=0.01)
+    loss, read = G.dual_clip_grpo_loss_begin(model, batch, 0.2, 0.28, 3.0, entropy_coeff=0.01)
+    loss.backward()
+    assert read() == want and loss.item() == want_loss.item()
+    assert abs(loss.item() - (want["loss"] - 0.01 * want["entropy"])) <= 1e-6 * max(1.0, abs(want["entropy"]))   # fp32 sum of two terms
+
+
 @pytest.mark.parametrize("returns_tuple", [False, True])
 def test_foreign_per_token_fn_takes_the_materialised_route(dev, returns_tuple):
     """per_token_fn(logits, shifted_labels, vocab_size=V) supplied by the caller (reference: grpo_loss.py:232-239,
