@@ -69,14 +69,17 @@ struct AttnParams {
   bf16_t* dv;
   // launches whose tiles are dealt to several work-groups (SPLIT kernels, see attn_parts); q: query side, k: key side
   int parts_q, per_q, blocks_q;      // most parts of a tile, steps a part is meant to walk, work-groups of one part
-  int parts_k, per_k, blocks_k;      // the same; steps: items of a wavefront
+  int parts_k, per_k, blocks_k;      // most parts of a tile, items of a wavefront a part walks at least, work-groups of an undivided launch
+  int extra_k, deal_k;               // work-groups beyond those, per XCD; work-groups of an XCD its items are meant for (attn_key_deal)
   float* part_q;         // [parts_q][ceil(T / 32)][Hq][32 x HD as attn_store_partial leaves them] O of the part, relative to its own maximum, or its dQ / scale
   float2* part_ml;       // [parts_q][Hq][T] forward: maximum and sum of the part
-  float* part_k;         // [parts_k][2][T][Hkv][HD] dK / scale and dV of the part
+  float* part_k;         // [work-group][2][keys of a tile][HD] dK / scale and dV of the part
+  int2* key_info;        // [key tile][Hkv] parts of the tile, work-group of the first
 };
 
 constexpr int kAttnMaxParts = 8;      // parts of a tile at most
 constexpr int kAttnMergeWide = 4;     // parts whose sums are fetched together
+constexpr int kAttnDealSlots = 256;   // key tiles an XCD can deal out
 // A tile that walks `steps` steps, all its work-group's own chain, may be dealt to several work-groups: each walks its
 // share and leaves fp32 sums, which a last launch adds up in a fixed order (no atomics: bit-reproducible).  How many,
 // every kernel of the call derives from the segment bounds.

@@ -141,8 +141,94 @@ inline long long attn_key_blocks(long long ntile, int pieces, int Hkv) {      //
   return 8 * (rounds * pieces + ((units - 8 * rounds) * pieces + 7) / 8);
 }
 
+// What a work-group walks: queries [q_begin, q_end) for the keys of `tile`
+struct KeyWork {
+  int tile, head, share, np;       // part `share` of the tile's np; tile < 0: no work
+  int q_begin, q_end, one_segment; // one segment holds every key of the tile
+};
+template <int kKeys>
+__device__ __forceinline__ void attn_key_bounds(const AttnParams& p, int k0, int& q_begin, int& q_end, int& one_segment) {
+  const int klast = min(k0 + kKeys, p.T) - 1, s0 = p.seg_start[k0];
+  q_begin = max(p.causal ? k0 : s0, 0);                        // inside [0, T]
+  q_end = min(p.seg_end[klast], p.T);
+  one_segment = s0 == p.seg_start[klast];
+}
+// inclusive sum over the lanes up to this one: rows of 16, then rows 0 -> 1, 2 -> 3 and 1 -> 2, 3
+__device__ __forceinline__ int wave_sum_upto(int x) {
+  x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false);      // row_shr 1, 2, 4, 8
+  x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, false);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, false);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, false);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);      // row_bcast 15
+  x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);      // row_bcast 31
+  return x;
+}
+
+// SPLIT launches: which part of which tile work-group `bid` takes.  How many parts a tile has follows from the items of all
+// tiles of its XCD, which every work-group reads (a lane a tile, order as in attn_key_pick) and adds up by itself: a part
+// is to walk `per` items, the XCD's items over the work-groups meant for them, or more until the parts fit the
+// work-groups there are.  The parts are numbered through, long tiles first, and work-group `bid` is part bid / 8 of XCD bid % 8;
+// the few that no part is left for end at once.
+// Dealt out by a mean segment's length instead, with work-groups for as many parts of every tile, a batch of several segments
+// had its longest tile to wait for or more work-groups than the device holds, most of them empty (each takes a CU's
+// LDS to find out).  dQ + dK/dV and the merge, us, before -> after: 2000 tokens in 7 segments, 28 / 4 heads of 128 74.6 -> 54.4;
+// 3000 in 4, 12 / 2 heads 122 -> 96; 9000 in 14, 12 / 2 heads 189 -> 140; 2000 in one, 12 / 2 heads 92 -> 78; 6000 in 12, 14 / 2
+// heads of 64 70.6 -> 61.3; 300 in one, 12 / 2 heads of 128 28.4 -> 28.9 (the reading and adding up).
+template <int kKeys>
+__device__ __forceinline__ KeyWork attn_key_deal(const AttnParams& p, int bid) {
+  constexpr int kPer128 = 128 / kKeys, NB = kAttnDealSlots / 64;
+  const int lane = threadIdx.x & 63, xcd = bid & 7, at = bid >> 3, slots = p.blocks_k >> 3, G = p.Hq / p.Hkv;
+  const int ntile = (p.T + kKeys - 1) / kKeys, n128 = (p.T + 127) / 128;
+  int tile[NB], head[NB], q_begin[NB], q_end[NB], one_segment[NB], chain[NB], sum = 0;
+#pragma unroll
+  for (int i = 0; i < NB; ++i) {
+    tile[i] = -1, head[i] = q_begin[i] = q_end[i] = one_segment[i] = chain[i] = 0;
+    const int slot = 64 * i + lane;
+    if (slot < slots) {
+      const KeyPick pick = attn_key_pick(8 * slot + xcd, n128, kPer128, p.Hkv);
+      const int t = pick.rank < 0 ? ntile : min(max(p.order_k[pick.rank], 0), n128 - 1) * kPer128 + pick.piece;
+      if (t < ntile) {
+        attn_key_bounds<kKeys>(p, t * kKeys, q_begin[i], q_end[i], one_segment[i]);
+        tile[i] = t, head[i] = pick.head, chain[i] = (attn_key_items(q_begin[i], q_end[i], G) + 3) / 4;
+      }
+    }
+    sum += chain[i];
+  }
+  auto total = [](int x) { return __builtin_amdgcn_readlane(wave_sum_upto(x), 63); };
+  sum = total(sum);
+  const int budget = slots + p.extra_k;
+  auto parts_at = [&](int i, int per) { return tile[i] < 0 ? 0 : attn_parts(chain[i], p.parts_k, per); };
+  int per = max(p.per_k, (sum + p.deal_k - 1) / p.deal_k);
+  const int sure = (sum + p.extra_k - 1) / p.extra_k;          // with it the parts fit: each tile rounds up by less than one
+  while (per < sure) {
+    int n = 0;
+#pragma unroll
+    for (int i = 0; i < NB; ++i) n += parts_at(i, per);
+    n = total(n);
+    if (n <= budget) break;
+    per = min(max(per + 1, (int)((long long)per * n / budget)), sure);
+  }
+  KeyWork out{-1, 0, 0, 1, 0, 0, 0};
+  int base = 0;
+#pragma unroll
+  for (int i = 0; i < NB; ++i) {
+    if (64 * i >= slots) break;
+    const int np = parts_at(i, per), upto = wave_sum_upto(np), share = at - (base + upto - np);
+    const unsigned long long hit = __ballot(share >= 0 && share < np);
+    if (hit != 0) {
+      const int l = __ffsll(hit) - 1;
+      out.tile = __builtin_amdgcn_readlane(tile[i], l), out.head = __builtin_amdgcn_readlane(head[i], l);
+      out.share = __builtin_amdgcn_readlane(share, l), out.np = __builtin_amdgcn_readlane(np, l);
+      out.q_begin = __builtin_amdgcn_readlane(q_begin[i], l), out.q_end = __builtin_amdgcn_readlane(q_end[i], l);
+      out.one_segment = __builtin_amdgcn_readlane(one_segment[i], l);
+    }
+    base += __builtin_amdgcn_readlane(upto, 63);
+  }
+  return out;
+}
+
 // KB key blocks of 32 (2: one wavefront per SIMD; 1, head dimension 64: two).  SPLIT: a tile's items are dealt to the
-// wavefronts of several work-groups (attn_parts), item n to wavefront n % (4 np) of them.
+// wavefronts of several work-groups (attn_key_deal), item n to wavefront n % (4 np) of them.
 template <int HD, int KB, bool SPLIT>
 __global__ __launch_bounds__(256, KB == 2 ? 1 : 2) void varlen_attn_dkv3_kernel(AttnParams p) {
   constexpr int kKeys = 32 * KB;
@@ -154,24 +240,28 @@ __global__ __launch_bounds__(256, KB == 2 ? 1 : 2) void varlen_attn_dkv3_kernel(
   const int lane = threadIdx.x & 63, h = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int G = p.Hq / p.Hkv;
-  const int share = SPLIT ? (int)blockIdx.x / p.blocks_k : 0, bid = (int)blockIdx.x - share * (SPLIT ? p.blocks_k : 0);
-  constexpr int kPer128 = 128 / kKeys;
-  const int ntile = (p.T + kKeys - 1) / kKeys, n128 = (p.T + 127) / 128;
-  const KeyPick pick = attn_key_pick(bid, n128, kPer128, p.Hkv);
-  if (pick.rank < 0) return;
-  const int hkv = pick.head;
-  const int tile = min(max(p.order_k[pick.rank], 0), n128 - 1) * kPer128 + pick.piece;      // clamped: the list may come from the caller
-  if (tile >= ntile) return;
-  const int k0 = tile * kKeys, klast = min(k0 + kKeys, p.T) - 1;
-  const int q_begin = max(__builtin_amdgcn_readfirstlane(p.causal ? k0 : p.seg_start[k0]), 0);      // inside [0, T]
-  const int q_end = min(__builtin_amdgcn_readfirstlane(p.seg_end[klast]), p.T);
-  // one segment holds every key of the tile: queries from `q_full` on that are complete blocks see all of it
-  const bool one_segment = __builtin_amdgcn_readfirstlane(p.seg_start[k0]) == __builtin_amdgcn_readfirstlane(p.seg_start[klast]);
+  KeyWork w{-1, 0, 0, 1, 0, 0, 0};
+  if constexpr (SPLIT) {
+    w = attn_key_deal<kKeys>(p, blockIdx.x);
+    if (w.tile < 0) return;
+    if (w.share == 0 && threadIdx.x == 0) p.key_info[w.tile * p.Hkv + w.head] = make_int2(w.np, blockIdx.x);
+  } else {
+    constexpr int kPer128 = 128 / kKeys;
+    const int ntile = (p.T + kKeys - 1) / kKeys, n128 = (p.T + 127) / 128;
+    const KeyPick pick = attn_key_pick(blockIdx.x, n128, kPer128, p.Hkv);
+    if (pick.rank < 0) return;
+    w.head = pick.head;
+    w.tile = min(max(p.order_k[pick.rank], 0), n128 - 1) * kPer128 + pick.piece;      // clamped: the list may come from the caller
+    if (w.tile >= ntile) return;
+    attn_key_bounds<kKeys>(p, w.tile * kKeys, w.q_begin, w.q_end, w.one_segment);
+  }
+  const int hkv = w.head, share = w.share, np = w.np, k0 = w.tile * kKeys, klast = min(k0 + kKeys, p.T) - 1;
+  const int q_begin = __builtin_amdgcn_readfirstlane(w.q_begin), q_end = __builtin_amdgcn_readfirstlane(w.q_end);
+  // where one segment holds every key of the tile, queries from `q_full` on that are complete blocks see all of it
+  const bool one_segment = __builtin_amdgcn_readfirstlane(w.one_segment);
   const int q_full = !one_segment ? 0x7fffffff : p.causal ? k0 + kKeys - 1 : q_begin;
   const int nqb = q_end > q_begin ? (q_end - q_begin + kDkv3Rows - 1) / kDkv3Rows : 0;
   const int NI = nqb * G;
-  const int np = SPLIT ? attn_parts((NI + 3) / 4, p.parts_k, p.per_k) : 1;
-  if (SPLIT && share >= np) return;
   const int first = wave + 4 * share, stride = 4 * np;          // this wavefront's items
   const int stride_g = SPLIT ? stride % G : 4, stride_b = SPLIT ? stride / G : 0;      // ... in heads and query blocks
 
@@ -590,7 +680,7 @@ __global__ __launch_bounds__(256, KB == 2 ? 1 : 2) void varlen_attn_dkv3_kernel(
       const int kk = k0 + row;
       const bool partial = SPLIT && np > 1;
       if (SPLIT && partial && kk < p.T) {
-        float4* dst = (float4*)(p.part_k + ((((long long)share * 2 + which) * p.T + kk) * p.Hkv + hkv) * HD + col * 8);
+        float4* dst = (float4*)(p.part_k + (((long long)blockIdx.x * 2 + which) * kKeys + row) * HD + col * 8);
         dst[0] = make_float4(x[0], x[1], x[2], x[3]);
         dst[1] = make_float4(x[4], x[5], x[6], x[7]);
       }
@@ -622,22 +712,22 @@ static __global__ __launch_bounds__(256) void attn_merge_bwd_kernel(AttnParams p
   if (which) idx -= nk;
   const int col = (int)(idx % (HD / 8)) * 8;
   const long long row = idx / (HD / 8);                        // key * Hkv + head
-  const int kk = (int)(row / p.Hkv);
-  const int k0 = kk / kKeys * kKeys, klast = min(k0 + kKeys, p.T) - 1;
-  const int items = attn_key_items(max(p.causal ? k0 : p.seg_start[k0], 0), min(p.seg_end[klast], p.T), p.Hq / p.Hkv);
-  const int np = attn_parts((items + 3) / 4, p.parts_k, p.per_k);
+  const int kk = (int)(row / p.Hkv), head = (int)(row % p.Hkv);
+  const int2 info = p.key_info[kk / kKeys * p.Hkv + head];
+  const int np = min(info.x, kAttnMaxParts);                   // parts, the work-group of the first (the others' 8 apart)
   if (np <= 1) return;
   float x[8];
 #pragma unroll
   for (int e = 0; e < 8; ++e) x[e] = 0.f;
-  const float* src = p.part_k + ((long long)which * p.T * p.Hkv + row) * HD + col;
-  const long long slice = 2LL * p.T * p.Hkv * HD;
+  constexpr int slice = 2 * kKeys * HD;
+  const int most = p.blocks_k + 8 * p.extra_k - 1 - 8 * (np - 1), first = min(max(info.y, 0), most);      // clamped: an order list of the caller's may leave a tile out
+  const float* src = p.part_k + (long long)first * slice + (which * kKeys + kk % kKeys) * HD + col;
 #pragma unroll
   for (int j0 = 0; j0 < kAttnMaxParts; j0 += kAttnMergeWide) {
     if (j0 >= np) break;
     float v[kAttnMergeWide][8];
 #pragma unroll
-    for (int u = 0; u < kAttnMergeWide; ++u) attn_load8(src + (j0 + u < np ? j0 + u : 0) * slice, v[u]);
+    for (int u = 0; u < kAttnMergeWide; ++u) attn_load8(src + (j0 + u < np ? j0 + u : 0) * (8LL * slice), v[u]);
 #pragma unroll
     for (int u = 0; u < kAttnMergeWide; ++u)
 #pragma unroll

@@ -1,4 +1,5 @@
 // Packed variable-length attention: C entry points, argument checks and launches (kernels in attn_kernels.h).
+#include <math.h>
 #include <string.h>
 
 #include "host_common.h"
@@ -11,6 +12,7 @@ namespace fgrpo {
 constexpr size_t kAttnSplitMaxBytes = 256u << 20;
 int launch_attn_dkv3(int D, const AttnParams& p, hipStream_t st);      // launch_attn_keyside.hip
 int attn_keyside_keys(int D);
+int attn_keyside_blocks(int D, int T, int Hkv);
 int launch_attn_merge_bwd(int D, const AttnParams& p, int rb, hipStream_t st);
 }
 
@@ -69,9 +71,10 @@ struct DqLauncher {
 // at most: the number of parts allowed for); one long segment among many short ones is judged by that mean and may stay
 // whole.  Decided by shapes alone.  Whole | dealt out, merge launch included, 12 / 2 heads of 128: one segment of 777
 // tokens, forward 25.2 | 19.2 us (16.7 now, see attn_merge_query_tile), backward 86.7 | 44.2 (38.9); of 6000 tokens 182 | 161 and 584 | 465; 3 segments of 1024 tokens,
-// backward (dK/dV alone is dealt out) 106 | 85, forward 29.2 | 42, which the estimate refuses.
+// forward 29.2 | 42, which the estimate refuses.
 struct SplitPlan {
   int parts = 1, per = 1;
+  int extra = 0, deal = 1;               // key side, see AttnParams
 };
 SplitPlan plan_split(long long wgs, int per_cu, double chain, bool causal, double step, size_t bytes_a_part) {
   SplitPlan best;
@@ -106,12 +109,56 @@ SplitPlan plan_query_split(const Tuning& tn, int form, int T, int n_seq, int Hq,
   return plan_split(wgs, 2, (double)T / n_seq / kAttnBK, causal, D == 128 ? 1.6 : forward ? 1.15 : 1.3,
                     (size_t)T * Hq * (D * 4 + (forward ? 8 : 0)));
 }
+// dK/dV under the causal mask: the same estimate, in items of a wavefront (`step` us each, `open` of them to open and close
+// a work-group), for the way attn_key_deal numbers the parts.  The longest segment of four or more is taken to be 1.75 means long
+// (lengths spread evenly; the kernel goes by the true ones).  Either every part is in flight at once - the items go by the
+// work-groups the tiles leave over - or, with about as many tiles as the device holds or more, the long tiles are cut to
+// one and a half times a CU's load, 40 items at most.  A first part that waits for a CU costs more than its own items: launches
+// order work-groups by shader engine, so 260 parts on 256 CUs took 120 us where 250 took 100 (3000 tokens in 4
+// segments, 12 / 2 heads of 128).  Whole | dealt out, dQ and merge included: 6000 tokens in 13 segments, 16 / 4
+// heads 150 | 123 (the estimate refuses it: the longest is 3.7 means); 4000 in 6, 28 / 4 heads 124 | 115; 5000 in one, 28 / 4
+// heads 645 | 609; 12345 in 23, 14 / 2 heads of 64 87 | 94 and 4000 in 5, 32 / 8 heads of 64 83 | 96, both refused.
 SplitPlan plan_key_split(int form, int T, int n_seq, int Hq, int Hkv, int D, int causal) {
   if (form == 1 || form == 2) return SplitPlan();
   const int keys = attn_keyside_keys(D);
   const long long wgs = (long long)((T + keys - 1) / keys) * Hkv;
-  const double chain = (double)T / n_seq / 32 * (Hq / Hkv) / 4;                // items of one of the four wavefronts
-  return plan_split(wgs, D == 128 ? 1 : 2, chain, causal, D == 128 ? 1.3 : 0.65, (size_t)T * Hkv * D * 8);
+  const int blocks = attn_keyside_blocks(D, T, Hkv), per_cu = D == 128 ? 1 : 2, slots = num_cus() * per_cu;
+  if (blocks > 8 * kAttnDealSlots) return SplitPlan();
+  const double spread = n_seq >= 4 ? 1.75 : 1.0, mean = (double)T / n_seq, longest = mean * spread;
+  const double items = (Hq / Hkv) / 4.0 / 32, step = D == 128 ? 1.4 : 0.65, open = D == 128 ? 6.0 : 4.0;      // of a wavefront, a token
+  SplitPlan s;
+  if (!causal) {
+    s = plan_split(wgs, per_cu, mean * items, causal, D == 128 ? 1.3 : 0.65, (size_t)T * Hkv * D * 8);
+    if (s.parts <= 1) return s;
+    s.extra = blocks / 8 * (s.parts - 1), s.deal = blocks / 8 * s.parts;
+    return s;
+  }
+  const double rest = T - longest, seen = n_seq >= 4 ? (longest * longest + rest * rest / (n_seq - 1)) / T : mean;
+  const double chain = longest * items, sum = wgs * (seen * 0.5 + 16 + (n_seq > 1 ? attn_keyside_keys(D) : 0)) * items;      // blocks of queries begun; tiles that reach into the next segment
+  auto shared = [&](double n) {
+    const double over = per_cu > 1 ? n / num_cus() - 1.0 : 0.0;
+    return step * (1.0 + 0.5 * (over < 0.0 ? 0.0 : over > 1.0 ? 1.0 : over));
+  };
+  auto most = [](double a, double b) { return a > b ? a : b; };
+  const double whole = most((chain + open) * shared((double)wgs), (sum + wgs * open) / slots * shared(2.0 * slots));
+  // a part more costs its sums, written and read; a longer part the wait for it
+  const double sums = attn_keyside_keys(D) * D * 16.0 / 3.0e6, least = floor(most(sqrt(sum * sums / step), 1.5) + 0.5);
+  const double cap = most(least, chain / kAttnMaxParts), load = sum / slots;
+  const double once = wgs < slots ? most(most(sum / (slots - 0.5 * wgs), chain * (2.0 - (double)slots / wgs)), cap) : 1e30;      // items a part walks: all parts in flight at once
+  const double fill = most(1.5 * load < 40.0 ? 1.5 * load : 40.0, cap);                                                    // ... or more of them than the device holds
+  auto parts = [&](double per) { return per < chain ? sum / per + 0.5 * wgs : (double)wgs; };
+  const double t_once = (once + open) * shared(parts(once));
+  const double t_fill = (load + parts(fill) * open / slots + 0.5 * fill + (wgs < slots ? 2.0 * open : 0.0)) * shared(2.0 * slots);
+  const bool fits = t_once < t_fill;
+  const double dealt = (fits ? t_once : t_fill) + 4.0 + most(parts(fits ? once : fill) - 0.5 * wgs, 0.0) * sums * 0.5;
+  if (dealt >= (fits ? 0.97 : 1.0) * whole) return s;
+  s.parts = kAttnMaxParts, s.per = (int)least;
+  s.extra = fits ? (slots - blocks) / 8 : (int)(load / fill * slots / 8) + 1;
+  s.deal = fits ? (slots - blocks / 2) / 8 : s.extra;
+  const int ways = (int)(T * items / least) + 1, bound = blocks / 8 * ((ways < kAttnMaxParts ? ways : kAttnMaxParts) - 1);      // if every tile had all queries
+  if (s.extra > bound) s.extra = bound;
+  if (s.extra < 1) s = SplitPlan();
+  return s;
 }
 size_t align256(size_t n) { return (n + 255) / 256 * 256; }
 size_t query_sums_bytes(const SplitPlan& s, int T, int Hq, int D) { return align256((size_t)s.parts * ((T + 31) / 32 * 32) * Hq * D * 4); }
@@ -119,7 +166,12 @@ size_t query_split_bytes(const SplitPlan& s, int T, int Hq, int D, bool forward)
   if (s.parts <= 1) return 0;
   return query_sums_bytes(s, T, Hq, D) + (forward ? align256((size_t)s.parts * T * Hq * 8) : 0);
 }
-size_t key_split_bytes(const SplitPlan& s, int T, int Hkv, int D) { return s.parts <= 1 ? 0 : align256((size_t)s.parts * T * Hkv * D * 8); }
+size_t key_sums_bytes(const SplitPlan& s, int T, int Hkv, int D) { return align256((size_t)(attn_keyside_blocks(D, T, Hkv) + 8 * s.extra) * attn_keyside_keys(D) * D * 8); }
+size_t key_split_bytes(const SplitPlan& s, int T, int Hkv, int D) {
+  if (s.parts <= 1) return 0;
+  const int keys = attn_keyside_keys(D);
+  return key_sums_bytes(s, T, Hkv, D) + align256((size_t)((T + keys - 1) / keys) * Hkv * sizeof(int2));
+}
 }  // namespace
 
 extern "C" {
@@ -261,9 +313,10 @@ int fgrpo_varlen_attn_bwd_ws(const void* dout, const void* q, const void* k, con
   else if (ws_bytes < need) return fail(FGRPO_ERR_WORKSPACE, "varlen_attn_bwd: workspace %zu < %zu", ws_bytes, need);
   else if (!aligned16(ws)) return fail(FGRPO_ERR_ALIGN, "varlen_attn_bwd: workspace must be 16-byte aligned");
   if (key_form != 3) sq = sk = SplitPlan();
-  p.parts_q = sq.parts, p.per_q = sq.per, p.parts_k = sk.parts, p.per_k = sk.per;
+  p.parts_q = sq.parts, p.per_q = sq.per, p.parts_k = sk.parts, p.per_k = sk.per, p.extra_k = sk.extra, p.deal_k = sk.deal;
   p.part_q = (float*)ws;
   p.part_k = (float*)((char*)ws + need_q);
+  p.key_info = (int2*)((char*)ws + need_q + key_sums_bytes(sk, T, Hkv, D));
   rc = launch_query_side<DqLauncher>(form, D, hb, p, T, Hq, Hkv, bounds_ws, st);
   if (rc) return rc;
   if (key_form == 3) {

@@ -5,14 +5,17 @@
 
 namespace fgrpo {
 
+int attn_keyside_keys(int D) { return D == 128 ? 64 : 32; }
+int attn_keyside_blocks(int D, int T, int Hkv) { return (int)attn_key_blocks((T + 127) / 128, 128 / attn_keyside_keys(D), Hkv); }      // every 128-key tile, in pieces
+
 template <int HD, int KB>
 static int launch(const AttnParams& p, hipStream_t st) {
   AttnParams a = p;
-  a.blocks_k = (int)attn_key_blocks((p.T + 127) / 128, 4 / KB, p.Hkv);      // every 128-key tile, in pieces of 32 KB keys
+  a.blocks_k = attn_keyside_blocks(HD, p.T, p.Hkv);
   if (p.parts_k > 1) {
     const int rc = raise_lds<varlen_attn_dkv3_kernel<HD, KB, true>>(kDkv3Lds<HD, KB>);
     if (rc) return rc;
-    hipLaunchKernelGGL((varlen_attn_dkv3_kernel<HD, KB, true>), dim3((unsigned)a.blocks_k * p.parts_k), dim3(256), (kDkv3Lds<HD, KB>), st, a);
+    hipLaunchKernelGGL((varlen_attn_dkv3_kernel<HD, KB, true>), dim3((unsigned)(a.blocks_k + 8 * p.extra_k)), dim3(256), (kDkv3Lds<HD, KB>), st, a);
   } else {
     const int rc = raise_lds<varlen_attn_dkv3_kernel<HD, KB, false>>(kDkv3Lds<HD, KB>);
     if (rc) return rc;
@@ -30,9 +33,9 @@ int launch_attn_dkv3(int D, const AttnParams& p, hipStream_t st) {
   return D == 128 ? launch<128, 2>(p, st) : launch<64, 1>(p, st);
 }
 
-int attn_keyside_keys(int D) { return D == 128 ? 64 : 32; }
-
-int launch_attn_merge_bwd(int D, const AttnParams& p, int rb, hipStream_t st) {
+int launch_attn_merge_bwd(int D, const AttnParams& params, int rb, hipStream_t st) {
+  AttnParams p = params;
+  p.blocks_k = attn_keyside_blocks(D, p.T, p.Hkv);
   const int nq = p.parts_q > 1 ? (p.T + 31) / 32 * p.Hq : 0;
   const long long nk = p.parts_k > 1 ? (long long)p.T * p.Hkv * (D / 8) : 0;
   const dim3 grid((unsigned)(nq + (2 * nk + 255) / 256));

@@ -75,6 +75,36 @@ def test_divided_tiles_against_the_oracle(dev, T, cu, Hq, Hkv, D, causal, sides)
         assert err <= tol, name
 
 
+def lengths(T, lo, hi):
+    g = torch.Generator().manual_seed(T + hi)
+    out = []
+    while sum(out) < T:
+        out.append(min(int(torch.randint(lo, hi + 1, (1,), generator=g)), T - sum(out)))
+    return out
+
+
+@pytest.mark.parametrize("T,lens,Hq,Hkv,D", [
+    (2000, [2000], 14, 2, 64), (2000, [2000], 12, 2, 128), (2000, lengths(2000, 128, 512), 28, 4, 128),      # all parts in flight at once, none to spare
+    (3000, [1916, 200, 700, 184], 12, 2, 128), (3001, lengths(3001, 128, 512), 28, 4, 128),
+    (4000, lengths(4000, 128, 1024), 28, 4, 128), (5000, [5000], 28, 4, 128), (9000, lengths(9000, 128, 2048), 12, 2, 128),      # more parts than the device holds
+    (9000, lengths(9000, 128, 2048), 14, 2, 64), (70, [70], 12, 1, 128), (5, [2, 3], 64, 1, 128)])           # more than 64 tiles an XCD; two tiles; one, left whole
+def test_key_tiles_dealt_by_their_items_agree_with_whole_ones(dev, T, lens, Hq, Hkv, D):
+    """Bounds as in test_divided_tiles_agree_with_whole_ones: the output that the backward starts from may come from parts too."""
+    from fgrpo import _lib, ops
+    q, k, v, do = operands(T, Hq, Hkv, D, dev)
+    cu = torch.tensor([0] + torch.tensor(lens).cumsum(0).tolist(), dtype=torch.int32, device=dev)
+    out, lse = ops.varlen_attn_fwd(q, k, v, cu, None, True)
+    want = ops.varlen_attn_bwd(do, q, k, v, out, lse, cu, None, True)
+    assert (_lib.load().fgrpo_varlen_attn_workspace(T, len(lens), Hq, Hkv, D, 1, 1) > 0) == (T > 5)
+
+    def once():
+        a = [x.clone().requires_grad_(True) for x in (q, k, v)]
+        return torch.autograd.grad(ops.varlen_attention(*a, cu, None, True), a, do)
+    for name, x, y, z in zip(("dq", "dk", "dv"), once(), want, once()):
+        assert torch.equal(x, z), f"{name} is not reproducible"
+        assert (x.float() - y.float()).norm() <= 2 ** -7 * y.float().norm(), name
+
+
 def test_workspace_is_checked(dev):
     from fgrpo import _lib
     lib = _lib.load()
