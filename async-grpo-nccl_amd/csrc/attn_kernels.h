@@ -68,24 +68,88 @@ struct AttnParams {
   bf16_t* dk;            // [T][Hkv][HD] contiguous
   bf16_t* dv;
   // launches whose tiles are dealt to several work-groups (SPLIT kernels, see attn_parts); q: query side, k: key side
-  int parts_q, per_q, blocks_q;      // most parts of a tile, steps a part is meant to walk, work-groups of one part
-  int parts_k, per_k, blocks_k;      // most parts of a tile, items of a wavefront a part walks at least, work-groups of an undivided launch
-  int extra_k, deal_k;               // work-groups beyond those, per XCD; work-groups of an XCD its items are meant for (attn_key_deal)
-  float* part_q;         // [parts_q][ceil(T / 32)][Hq][32 x HD as attn_store_partial leaves them] O of the part, relative to its own maximum, or its dQ / scale
-  float2* part_ml;       // [parts_q][Hq][T] forward: maximum and sum of the part
+  int parts_q, per_q, blocks_q;      // most parts of a tile, steps a part walks at least, work-groups of an undivided launch
+  int extra_q, deal_q;               // work-groups beyond those, per XCD; work-groups of an XCD its steps are meant for
+  int parts_k, per_k, blocks_k;      // the same; steps: items of a wavefront
+  int extra_k, deal_k;
+  float* part_q;         // [work-group][wavefront][32 x HD as attn_store_partial leaves them] O of the part, relative to its own maximum, or its dQ / scale
+  float2* part_ml;       // [work-group][wavefront][32] forward: maximum and sum of the part
+  int2* query_info;      // [query tile][Hkv] parts of the tile, work-group of the first (its first heads)
   float* part_k;         // [work-group][2][keys of a tile][HD] dK / scale and dV of the part
   int2* key_info;        // [key tile][Hkv] parts of the tile, work-group of the first
 };
 
 constexpr int kAttnMaxParts = 8;      // parts of a tile at most
 constexpr int kAttnMergeWide = 4;     // parts whose sums are fetched together
-constexpr int kAttnDealSlots = 256;   // key tiles an XCD can deal out
-// A tile that walks `steps` steps, all its work-group's own chain, may be dealt to several work-groups: each walks its
-// share and leaves fp32 sums, which a last launch adds up in a fixed order (no atomics: bit-reproducible).  How many,
-// every kernel of the call derives from the segment bounds.
-__device__ __forceinline__ int attn_parts(int steps, int parts, int per) {
-  const int n = (steps + per - 1) / per;
-  return n < 1 ? 1 : n > parts ? parts : n;
+constexpr int kAttnDealSlots = 256;   // tiles an XCD can deal out
+// A tile that walks `steps` steps, all its work-group's own chain, may be dealt to several work-groups (parts): each walks
+// its share and leaves fp32 sums, which a last launch adds up in a fixed order (no atomics: bit-reproducible).
+// n / d for 0 <= n < 2^21, d > 0: (n + 1/2) / d is at least 1 / (2 d) from a whole number, the error of product and reciprocal less.  An
+// integer division is some forty instructions, in series before a work-group's first load.
+__device__ __forceinline__ int small_div(int n, int d) { return (int)(((float)n + 0.5f) * __builtin_amdgcn_rcpf((float)d)); }
+__device__ __forceinline__ int attn_parts(int steps, int parts, int per) { return min(max(small_div(steps + per - 1, per), 1), parts); }
+// inclusive sum over the lanes up to this one: rows of 16, then rows 0 -> 1, 2 -> 3 and 1 -> 2, 3
+__device__ __forceinline__ int wave_sum_upto(int x) {
+  x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false);      // row_shr 1, 2, 4, 8
+  x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, false);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, false);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, false);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);      // row_bcast 15
+  x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);      // row_bcast 31
+  return x;
+}
+// Which part of which tile the work-group of number `at` in its XCD takes.  Lane l has the steps of the XCD's tiles l, l + 64,
+// .. (negative: no tile); every work-group reads them and adds them up by itself.  A part is to walk `per` steps, the XCD's
+// steps over the `deal` work-groups meant for them (`least` at least), or more until the parts fit the work-groups there
+// are, `slots` tiles of `width` work-groups each and `extra`.  The parts are numbered through in the order of the tiles,
+// longest first; the few work-groups that no part is left for end at once.
+// Dealt out by a mean segment's length instead, with work-groups for as many parts of every tile, a batch of several segments
+// had its longest tile to wait for, or more work-groups than the device holds, most of them empty (each takes a CU's
+// LDS to find out).  Forward | dQ, dK/dV and merge, us, before -> after, heads of 128 unless said: 3000 tokens in 4 segments, 12 / 2 heads
+// 48.6 | 122 -> 35.6 | 82.4; 1500 in 2 26.4 | 65.5 -> 21.1 | 44.4; 9000 in 14 48.0 | 189 -> 48.6 | 139; one of 2000 34.6 | 91.6 -> 31.8 | 74.1,
+// of 777 16.7 | 38.6 -> 16.5 | 36.7, of 300 11.4 | 28.4 -> 11.3 | 25.7; 2000 in 7, 28 / 4 heads 16.6 | 74.2 -> 16.7 | 53.5; 6000 in 12,
+// 14 / 2 heads of 64 21.9 | 70.6 -> 21.8 | 61.3.  What it costs a work-group, some 0.5 us before its first load, is why sums
+// and quotients are in as few instructions as they are (with integer divisions the forward of 777 tokens took 17.4 us).
+struct AttnDeal {
+  int slot, share, np, sub;        // part `share` of the np of the XCD's tile `slot`, work-group `sub` of its width; slot < 0: no work
+};
+template <int N>
+__device__ __forceinline__ AttnDeal attn_deal(const int (&steps)[N], int at, int slots, int width, int extra, int parts, int least, int deal) {
+  const int lane = threadIdx.x & 63, budget = slots * width + extra;
+  auto total = [](int x) { return __builtin_amdgcn_readlane(wave_sum_upto(x), 63); };
+  auto parts_at = [&](int i, int per) { return steps[i] < 0 ? 0 : attn_parts(steps[i], parts, per); };
+  int sum = 0;
+#pragma unroll
+  for (int i = 0; i < N; ++i) sum += max(steps[i], 0);
+  sum = total(sum) * width;
+  int per = least;
+  if (sum > per * deal) per = (sum + deal - 1) / deal;
+  if (sum > per * extra) {
+    const int sure = (sum + extra - 1) / extra;                // with it the parts fit: each tile rounds up by less than one
+    do {
+      int n = 0;
+#pragma unroll
+      for (int i = 0; i < N; ++i) n += parts_at(i, per);
+      n = total(n) * width;
+      if (n <= budget) break;
+      per = min(max(per + 1, (int)((long long)per * n / budget)), sure);
+    } while (per < sure);
+  }
+  AttnDeal out{-1, 0, 1, 0};
+  int base = 0;
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    if (64 * i >= slots) break;
+    const int np = parts_at(i, per), n = np * width, upto = wave_sum_upto(n), place = at - (base + upto - n);
+    const unsigned long long hit = __ballot(place >= 0 && place < n);
+    if (hit != 0) {
+      const int l = __ffsll(hit) - 1;
+      out.slot = 64 * i + l, out.np = __builtin_amdgcn_readlane(np, l), out.sub = __builtin_amdgcn_readlane(place, l);
+      while (out.sub >= width) out.sub -= width, ++out.share;
+    }
+    base += __builtin_amdgcn_readlane(upto, 63);
+  }
+  return out;
 }
 // keys a query tile of RB tokens from q0 on walks: [k_begin, k_end)
 __device__ __forceinline__ void attn_query_tile_keys(const AttnParams& p, int q0, int RB, int& k_begin, int& k_end) {
@@ -94,6 +158,40 @@ __device__ __forceinline__ void attn_query_tile_keys(const AttnParams& p, int q0
   k_end = min(p.causal ? last + 1 : p.seg_end[last], p.T);
 }
 __device__ __forceinline__ int attn_steps(int k_begin, int k_end) { return k_end > k_begin ? (k_end - k_begin + kAttnBK - 1) / kAttnBK : 0; }
+// What a work-group of the query-side kernels takes: tile, K/V head, heads `sub` of the group, and of its keys [k_begin, k_end) its part
+struct QueryWork {
+  int tile, head, sub, part, np, k_begin, k_end;      // tile < 0: no work
+};
+// SPLIT launches; NB work-groups share a tile and K/V head (AttnDeal::sub)
+template <int RB>
+__device__ __forceinline__ QueryWork attn_query_deal(const AttnParams& p, int bid, int NB) {
+  constexpr int N = kAttnDealSlots / 64;
+  const int lane = threadIdx.x & 63, xcd = bid & 7, slots = small_div(p.blocks_q >> 3, NB), ntile = (p.T + RB - 1) / RB;
+  int tile[N], head[N], k_begin[N], k_end[N], steps[N];
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    steps[i] = -1, tile[i] = head[i] = k_begin[i] = k_end[i] = 0;
+    const int slot = 64 * i + lane, unit = 8 * slot + xcd;
+    if (slot < slots && unit < ntile * p.Hkv) {
+      const int rank = small_div(unit, p.Hkv);
+      head[i] = unit - rank * p.Hkv;
+      tile[i] = min(max(p.order_q[rank], 0), ntile - 1);       // clamped: the list may come from the caller
+      attn_query_tile_keys(p, tile[i] * RB, RB, k_begin[i], k_end[i]);
+      steps[i] = attn_steps(k_begin[i], k_end[i]);
+    }
+  }
+  const AttnDeal d = attn_deal(steps, bid >> 3, slots, NB, p.extra_q, p.parts_q, p.per_q, p.deal_q);
+  QueryWork w{-1, 0, d.sub, d.share, d.np, 0, 0};
+#pragma unroll
+  for (int i = 0; i < N; ++i)
+    if (d.slot >= 0 && d.slot / 64 == i) {
+      const int l = d.slot % 64, all = __builtin_amdgcn_readlane(steps[i], l), first = __builtin_amdgcn_readlane(k_begin[i], l);
+      w.tile = __builtin_amdgcn_readlane(tile[i], l), w.head = __builtin_amdgcn_readlane(head[i], l);
+      w.k_begin = first + kAttnBK * __builtin_amdgcn_readfirstlane(small_div(all * d.share, d.np));
+      w.k_end = min(__builtin_amdgcn_readlane(k_end[i], l), first + kAttnBK * __builtin_amdgcn_readfirstlane(small_div(all * (d.share + 1), d.np)));
+    }
+  return w;
+}
 
 typedef short i16x4_t __attribute__((ext_vector_type(4)));
 
@@ -232,9 +330,7 @@ __device__ __forceinline__ void attn_store_rowmajor(const f32x16_t (&acc)[DB], f
 // ... and the same accumulator as it lies in the registers, in fp32: a part's sums of 32 tokens of one head, 1 KiB an instruction.
 // Columns 32 db + 8 g + 4 h .. + 3 of token n of the 32 are the 16 bytes at 64 (4 db + g) + 32 h + n.
 template <int HD>
-__device__ __forceinline__ float* attn_partial(const AttnParams& p, int part, int t, int hq) {
-  return p.part_q + (((long long)part * ((p.T + 31) / 32) + t / 32) * p.Hq + hq) * (32 * HD);
-}
+__device__ __forceinline__ float* attn_partial(const AttnParams& p, int wg, int wave) { return p.part_q + ((long long)wg * 4 + wave) * (32 * HD); }
 template <int DB>
 __device__ __forceinline__ void attn_store_partial(const f32x16_t (&acc)[DB], float* tile, int lane) {
 #pragma unroll
@@ -1406,35 +1502,36 @@ __global__ __launch_bounds__(256, 2) void varlen_attn_fwd2_kernel(AttnParams p) 
   // work-group -> (tile, K/V head, query heads): as in varlen_attn_fwd_kernel
   constexpr int WPH = 4 / HB, RB = 32 * WPH;
   const int G = p.Hq / p.Hkv, NB = (G + HB - 1) / HB;
-  const int part = SPLIT ? (int)blockIdx.x / p.blocks_q : 0, bid = (int)blockIdx.x - part * (SPLIT ? p.blocks_q : 0);
-  const int xcd = bid & 7, slot = bid >> 3;
-  const int unit = (slot / NB) * 8 + xcd;
+  const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
   const int ntile = (p.T + RB - 1) / RB;
-  if (unit >= ntile * p.Hkv) return;
-  const int hkv = unit % p.Hkv;
-  const int head_g = (slot % NB) * HB + wave / WPH;
+  QueryWork w{0, 0, slot % NB, 0, 1, 0, 0};
+  if constexpr (SPLIT) {
+    w = attn_query_deal<RB>(p, blockIdx.x, NB);
+    if (w.tile < 0) return;
+    if (w.part == 0 && w.sub == 0 && threadIdx.x == 0) p.query_info[w.tile * p.Hkv + w.head] = make_int2(w.np, blockIdx.x);
+  } else {
+    const int unit = (slot / NB) * 8 + xcd;
+    if (unit >= ntile * p.Hkv) return;
+    w.head = unit % p.Hkv, w.tile = min(max(p.order_q[unit / p.Hkv], 0), ntile - 1);
+  }
+  const int hkv = w.head, np = w.np;
+  const int head_g = w.sub * HB + wave / WPH;
   const bool head_ok = head_g < G;
   const int hq = hkv * G + (head_ok ? head_g : G - 1);
-  const int q0 = min(max(p.order_q[unit / p.Hkv], 0), ntile - 1) * RB;
-  const int last = min(q0 + RB, p.T) - 1;
+  const int q0 = w.tile * RB;
   // this wavefront's queries wfirst .. wlast, what they see, and the walk of the work-group: indices are clamped instead
   // of branched around, so that all of it is one round trip behind the tile number
   const int wfirst = q0 + 32 * (wave % WPH), wl = min(wfirst + 31, p.T - 1), wf = min(wfirst, wl);
   const int wrows = head_ok ? max(wl - wfirst + 1, 0) : 0;      // 32, fewer at the end of the axis, or none (a tile may end before its last wavefront's queries)
   const int tq = wfirst + (lane & 31);
   const bool valid = (lane & 31) < wrows, wave_full = wrows == 32;
-  const int s_first = p.seg_start[q0], s_wf = p.seg_start[wf], s_wl = p.seg_start[wl], s_tq = p.seg_start[min(tq, p.T - 1)];
-  int e_last = last + 1, e_wl = wl + 1, e_wf = wf + 1, e_tq = tq + 1;      // one past the last key seen
-  if (!p.causal) e_last = p.seg_end[last], e_wl = p.seg_end[wl], e_wf = p.seg_end[wf], e_tq = p.seg_end[min(tq, p.T - 1)];
-  int k_begin = max(__builtin_amdgcn_readfirstlane(s_first), 0);           // wavefront-uniform loop bounds, inside [0, T]
-  int k_end = min(__builtin_amdgcn_readfirstlane(e_last), p.T);
-  int np = 1;
-  if constexpr (SPLIT) {                   // this part's share of the steps
-    const int steps = attn_steps(k_begin, k_end);
-    np = attn_parts(steps, p.parts_q, p.per_q);
-    if (part >= np) return;
-    k_end = min(k_end, k_begin + kAttnBK * (steps * (part + 1) / np));
-    k_begin += kAttnBK * (steps * part / np);
+  const int s_wf = p.seg_start[wf], s_wl = p.seg_start[wl], s_tq = p.seg_start[min(tq, p.T - 1)];
+  int e_wl = wl + 1, e_wf = wf + 1, e_tq = tq + 1;      // one past the last key seen
+  if (!p.causal) e_wl = p.seg_end[wl], e_wf = p.seg_end[wf], e_tq = p.seg_end[min(tq, p.T - 1)];
+  int k_begin = w.k_begin, k_end = w.k_end;                                // wavefront-uniform loop bounds, inside [0, T]
+  if constexpr (!SPLIT) {
+    attn_query_tile_keys(p, q0, RB, k_begin, k_end);
+    k_begin = __builtin_amdgcn_readfirstlane(k_begin), k_end = __builtin_amdgcn_readfirstlane(k_end);
   }
   const bool wave_on = wrows > 0;
   const int w_lo = wave_on ? s_wf : 1, w_hi = wave_on ? e_wl - 1 : 0;
@@ -1609,9 +1706,9 @@ __global__ __launch_bounds__(256, 2) void varlen_attn_fwd2_kernel(AttnParams p) 
   const float l = l_lo + l_hi;
   if constexpr (SPLIT) {
     if (np > 1) {
-      if (wrows > 0) attn_store_partial(acc_o, attn_partial<HD>(p, part, wfirst, hq), lane);
+      if (wrows > 0) attn_store_partial(acc_o, attn_partial<HD>(p, blockIdx.x, wave), lane);
       if (valid) {
-        if (h == 0) p.part_ml[((long long)part * p.Hq + hq) * p.T + tq] = make_float2(m_run, l);
+        if (h == 0) p.part_ml[((long long)blockIdx.x * 4 + wave) * 32 + (lane & 31)] = make_float2(m_run, l);
       }
       return;
     }
@@ -1649,35 +1746,36 @@ __global__ __launch_bounds__(256, 2) void varlen_attn_dq2_kernel(AttnParams p) {
   // work-group -> (tile, K/V head, query heads): as in varlen_attn_dq_kernel
   constexpr int WPH = 4 / HB, RB = 32 * WPH;
   const int G = p.Hq / p.Hkv, NB = (G + HB - 1) / HB;
-  const int part = SPLIT ? (int)blockIdx.x / p.blocks_q : 0, bid = (int)blockIdx.x - part * (SPLIT ? p.blocks_q : 0);
-  const int xcd = bid & 7, slot = bid >> 3;
-  const int unit = (slot / NB) * 8 + xcd;
+  const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
   const int ntile = (p.T + RB - 1) / RB;
-  if (unit >= ntile * p.Hkv) return;
-  const int hkv = unit % p.Hkv;
-  const int head_g = (slot % NB) * HB + wave / WPH;
+  QueryWork w{0, 0, slot % NB, 0, 1, 0, 0};
+  if constexpr (SPLIT) {
+    w = attn_query_deal<RB>(p, blockIdx.x, NB);
+    if (w.tile < 0) return;
+    if (w.part == 0 && w.sub == 0 && threadIdx.x == 0) p.query_info[w.tile * p.Hkv + w.head] = make_int2(w.np, blockIdx.x);
+  } else {
+    const int unit = (slot / NB) * 8 + xcd;
+    if (unit >= ntile * p.Hkv) return;
+    w.head = unit % p.Hkv, w.tile = min(max(p.order_q[unit / p.Hkv], 0), ntile - 1);
+  }
+  const int hkv = w.head, np = w.np, part = w.part;
+  const int head_g = w.sub * HB + wave / WPH;
   const bool head_ok = head_g < G;
   const int hq = hkv * G + (head_ok ? head_g : G - 1);
-  const int q0 = min(max(p.order_q[unit / p.Hkv], 0), ntile - 1) * RB;
-  const int last = min(q0 + RB, p.T) - 1;
+  const int q0 = w.tile * RB;
   // this wavefront's queries wfirst .. wlast, what they see, and the walk of the work-group: indices are clamped instead
   // of branched around, so that all of it is one round trip behind the tile number
   const int wfirst = q0 + 32 * (wave % WPH), wl = min(wfirst + 31, p.T - 1), wf = min(wfirst, wl);
   const int wrows = head_ok ? max(wl - wfirst + 1, 0) : 0;      // 32, fewer at the end of the axis, or none (a tile may end before its last wavefront's queries)
   const int tq = wfirst + (lane & 31);
   const bool valid = (lane & 31) < wrows, wave_full = wrows == 32;
-  const int s_first = p.seg_start[q0], s_wf = p.seg_start[wf], s_wl = p.seg_start[wl], s_tq = p.seg_start[min(tq, p.T - 1)];
-  int e_last = last + 1, e_wl = wl + 1, e_wf = wf + 1, e_tq = tq + 1;      // one past the last key seen
-  if (!p.causal) e_last = p.seg_end[last], e_wl = p.seg_end[wl], e_wf = p.seg_end[wf], e_tq = p.seg_end[min(tq, p.T - 1)];
-  int k_begin = max(__builtin_amdgcn_readfirstlane(s_first), 0);           // wavefront-uniform loop bounds, inside [0, T]
-  int k_end = min(__builtin_amdgcn_readfirstlane(e_last), p.T);
-  int np = 1;
-  if constexpr (SPLIT) {                   // this part's share of the steps
-    const int steps = attn_steps(k_begin, k_end);
-    np = attn_parts(steps, p.parts_q, p.per_q);
-    if (part >= np) return;
-    k_end = min(k_end, k_begin + kAttnBK * (steps * (part + 1) / np));
-    k_begin += kAttnBK * (steps * part / np);
+  const int s_wf = p.seg_start[wf], s_wl = p.seg_start[wl], s_tq = p.seg_start[min(tq, p.T - 1)];
+  int e_wl = wl + 1, e_wf = wf + 1, e_tq = tq + 1;      // one past the last key seen
+  if (!p.causal) e_wl = p.seg_end[wl], e_wf = p.seg_end[wf], e_tq = p.seg_end[min(tq, p.T - 1)];
+  int k_begin = w.k_begin, k_end = w.k_end;                                // wavefront-uniform loop bounds, inside [0, T]
+  if constexpr (!SPLIT) {
+    attn_query_tile_keys(p, q0, RB, k_begin, k_end);
+    k_begin = __builtin_amdgcn_readfirstlane(k_begin), k_end = __builtin_amdgcn_readfirstlane(k_end);
   }
   const bool wave_on = wrows > 0;
   const int w_lo = wave_on ? s_wf : 1, w_hi = wave_on ? e_wl - 1 : 0;
@@ -1920,7 +2018,7 @@ __global__ __launch_bounds__(256, 2) void varlen_attn_dq2_kernel(AttnParams p) {
   }
   if constexpr (SPLIT) {
     if (np > 1) {
-      if (wrows > 0) attn_store_partial(acc, attn_partial<HD>(p, part, wfirst, hq), lane);
+      if (wrows > 0) attn_store_partial(acc, attn_partial<HD>(p, blockIdx.x, wave), lane);
       return;
     }
   }
@@ -1943,19 +2041,21 @@ __global__ __launch_bounds__(256, 2) void varlen_attn_dq2_kernel(AttnParams p) {
 // Bound by latency: a thread's time is its chain of round trips, so the loads of kAttnMergeWide parts go out together (the
 // first part again for those a tile does not have).  Partial sums used to lie by rows: a store of a part touched 32 rows, 32 bytes
 // of each, and took the address unit as long as eight.  Forward, merge included, | backward, us, before -> after: one segment of 777
-// tokens with 12 / 2 heads of 128 18.1 | 39.9 -> 16.7 | 38.9, of 2000 37.4 | 93.6 -> 34.1 | 91.5, of 3000 60.8 | 156.7 -> 56.8 | 153.5;
-// 900 with 14 / 2 heads of 64 16.5 | 30.4 -> 15.1 | 29.8.  (Read by threads along a row, with these sums 1 KiB apart, the merge
-// alone took 6 us more.)  Parts half as long or less, which cheaper merges might pay for, are slower still (777 tokens 18.7).
+// tokens with 12 / 2 heads of 128 18.1 | 39.9 -> 16.7 | 38.9, of 2000 37.4 | 93.6 -> 34.1 | 91.5;
+// 900 with 14 / 2 heads of 64 16.5 | 30.4 -> 15.1 | 29.8 (all of it with the parts of that time: see attn_deal).  (Read by threads along a row, with these sums 1 KiB apart, the merge
+// alone took 6 us more.)  Parts half as long, which cheaper merges might pay for, are slower still (777 tokens 18.7).
 template <int HD, bool FWD>
 __device__ __forceinline__ void attn_merge_query_tile(const AttnParams& p, int RB, int idx) {
   constexpr int NC = HD / 64;                              // pieces of eight columns a thread
   __shared__ __attribute__((aligned(16))) char smem[32 * HD * 2];
   const int t0 = idx / p.Hq * 32, hq = idx % p.Hq, n = threadIdx.x % 32, i0 = threadIdx.x / 32;
-  int k_begin, k_end;
-  attn_query_tile_keys(p, t0 / RB * RB, RB, k_begin, k_end);
-  const int np = attn_parts(attn_steps(k_begin, k_end), p.parts_q, p.per_q);
+  const int G = p.Hq / p.Hkv, HB = 128 / RB, NB = (G + HB - 1) / HB, head = hq % G;
+  const int2 info = p.query_info[t0 / RB * p.Hkv + hq / G];
+  const int np = min(info.x, kAttnMaxParts);
   if (np <= 1) return;
-  const int t = min(t0 + n, p.T - 1);
+  // the parts' work-groups: 8 NB apart, those of the next HB heads 8 on.  Clamped: an order list of the caller's may leave a tile out
+  const int most = p.blocks_q + 8 * p.extra_q - 1 - 8 * ((np - 1) * NB + head / HB), first = min(max(info.y, 0), most) + 8 * (head / HB);
+  const int wave = head % HB * (RB / 32) + t0 % RB / 32, t = min(t0 + n, p.T - 1);
   float x[NC][8];
 #pragma unroll
   for (int c = 0; c < NC; ++c)
@@ -1965,10 +2065,10 @@ __device__ __forceinline__ void attn_merge_query_tile(const AttnParams& p, int R
   float2 ml[kAttnMaxParts];
   if constexpr (FWD) {
 #pragma unroll
-    for (int j = 0; j < kAttnMaxParts; ++j) ml[j] = p.part_ml[((long long)(j < np ? j : 0) * p.Hq + hq) * p.T + t];
+    for (int j = 0; j < kAttnMaxParts; ++j) ml[j] = p.part_ml[((long long)(first + (j < np ? j : 0) * 8 * NB) * 4 + wave) * 32 + t - t0];
   }
-  const float* src = attn_partial<HD>(p, 0, t0, hq) + (64 * i0 + n) * 4;
-  const long long slice = (long long)((p.T + 31) / 32) * p.Hq * (32 * HD);
+  const float* src = attn_partial<HD>(p, first, wave) + (64 * i0 + n) * 4;
+  const long long slice = 8LL * NB * 4 * (32 * HD);
 #pragma unroll
   for (int j0 = 0; j0 < kAttnMaxParts; j0 += kAttnMergeWide) {
     if (j0 >= np) break;

@@ -143,7 +143,7 @@ inline long long attn_key_blocks(long long ntile, int pieces, int Hkv) {      //
 
 // What a work-group walks: queries [q_begin, q_end) for the keys of `tile`
 struct KeyWork {
-  int tile, head, share, np;       // part `share` of the tile's np; tile < 0: no work
+  int tile, head, share, np;       // part `share` of the tile's np (see attn_deal); tile < 0: no work
   int q_begin, q_end, one_segment; // one segment holds every key of the tile
 };
 template <int kKeys>
@@ -153,77 +153,36 @@ __device__ __forceinline__ void attn_key_bounds(const AttnParams& p, int k0, int
   q_end = min(p.seg_end[klast], p.T);
   one_segment = s0 == p.seg_start[klast];
 }
-// inclusive sum over the lanes up to this one: rows of 16, then rows 0 -> 1, 2 -> 3 and 1 -> 2, 3
-__device__ __forceinline__ int wave_sum_upto(int x) {
-  x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false);      // row_shr 1, 2, 4, 8
-  x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, false);
-  x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, false);
-  x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, false);
-  x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);      // row_bcast 15
-  x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);      // row_bcast 31
-  return x;
-}
-
-// SPLIT launches: which part of which tile work-group `bid` takes.  How many parts a tile has follows from the items of all
-// tiles of its XCD, which every work-group reads (a lane a tile, order as in attn_key_pick) and adds up by itself: a part
-// is to walk `per` items, the XCD's items over the work-groups meant for them, or more until the parts fit the
-// work-groups there are.  The parts are numbered through, long tiles first, and work-group `bid` is part bid / 8 of XCD bid % 8;
-// the few that no part is left for end at once.
-// Dealt out by a mean segment's length instead, with work-groups for as many parts of every tile, a batch of several segments
-// had its longest tile to wait for or more work-groups than the device holds, most of them empty (each takes a CU's
-// LDS to find out).  dQ + dK/dV and the merge, us, before -> after: 2000 tokens in 7 segments, 28 / 4 heads of 128 74.6 -> 54.4;
-// 3000 in 4, 12 / 2 heads 122 -> 96; 9000 in 14, 12 / 2 heads 189 -> 140; 2000 in one, 12 / 2 heads 92 -> 78; 6000 in 12, 14 / 2
-// heads of 64 70.6 -> 61.3; 300 in one, 12 / 2 heads of 128 28.4 -> 28.9 (the reading and adding up).
+// SPLIT launches: tiles in the order of attn_key_pick
 template <int kKeys>
 __device__ __forceinline__ KeyWork attn_key_deal(const AttnParams& p, int bid) {
-  constexpr int kPer128 = 128 / kKeys, NB = kAttnDealSlots / 64;
-  const int lane = threadIdx.x & 63, xcd = bid & 7, at = bid >> 3, slots = p.blocks_k >> 3, G = p.Hq / p.Hkv;
+  constexpr int kPer128 = 128 / kKeys, N = kAttnDealSlots / 64;
+  const int lane = threadIdx.x & 63, xcd = bid & 7, slots = p.blocks_k >> 3;
   const int ntile = (p.T + kKeys - 1) / kKeys, n128 = (p.T + 127) / 128;
-  int tile[NB], head[NB], q_begin[NB], q_end[NB], one_segment[NB], chain[NB], sum = 0;
+  int tile[N], head[N], q_begin[N], q_end[N], one_segment[N], items[N];
 #pragma unroll
-  for (int i = 0; i < NB; ++i) {
-    tile[i] = -1, head[i] = q_begin[i] = q_end[i] = one_segment[i] = chain[i] = 0;
+  for (int i = 0; i < N; ++i) {
+    tile[i] = items[i] = -1, head[i] = q_begin[i] = q_end[i] = one_segment[i] = 0;
     const int slot = 64 * i + lane;
     if (slot < slots) {
       const KeyPick pick = attn_key_pick(8 * slot + xcd, n128, kPer128, p.Hkv);
       const int t = pick.rank < 0 ? ntile : min(max(p.order_k[pick.rank], 0), n128 - 1) * kPer128 + pick.piece;
       if (t < ntile) {
         attn_key_bounds<kKeys>(p, t * kKeys, q_begin[i], q_end[i], one_segment[i]);
-        tile[i] = t, head[i] = pick.head, chain[i] = (attn_key_items(q_begin[i], q_end[i], G) + 3) / 4;
+        tile[i] = t, head[i] = pick.head, items[i] = (attn_key_items(q_begin[i], q_end[i], p.Hq / p.Hkv) + 3) / 4;
       }
     }
-    sum += chain[i];
   }
-  auto total = [](int x) { return __builtin_amdgcn_readlane(wave_sum_upto(x), 63); };
-  sum = total(sum);
-  const int budget = slots + p.extra_k;
-  auto parts_at = [&](int i, int per) { return tile[i] < 0 ? 0 : attn_parts(chain[i], p.parts_k, per); };
-  int per = max(p.per_k, (sum + p.deal_k - 1) / p.deal_k);
-  const int sure = (sum + p.extra_k - 1) / p.extra_k;          // with it the parts fit: each tile rounds up by less than one
-  while (per < sure) {
-    int n = 0;
+  const AttnDeal d = attn_deal(items, bid >> 3, slots, 1, p.extra_k, p.parts_k, p.per_k, p.deal_k);
+  KeyWork out{-1, 0, d.share, d.np, 0, 0, 0};
 #pragma unroll
-    for (int i = 0; i < NB; ++i) n += parts_at(i, per);
-    n = total(n);
-    if (n <= budget) break;
-    per = min(max(per + 1, (int)((long long)per * n / budget)), sure);
-  }
-  KeyWork out{-1, 0, 0, 1, 0, 0, 0};
-  int base = 0;
-#pragma unroll
-  for (int i = 0; i < NB; ++i) {
-    if (64 * i >= slots) break;
-    const int np = parts_at(i, per), upto = wave_sum_upto(np), share = at - (base + upto - np);
-    const unsigned long long hit = __ballot(share >= 0 && share < np);
-    if (hit != 0) {
-      const int l = __ffsll(hit) - 1;
+  for (int i = 0; i < N; ++i)
+    if (d.slot >= 0 && d.slot / 64 == i) {
+      const int l = d.slot % 64;
       out.tile = __builtin_amdgcn_readlane(tile[i], l), out.head = __builtin_amdgcn_readlane(head[i], l);
-      out.share = __builtin_amdgcn_readlane(share, l), out.np = __builtin_amdgcn_readlane(np, l);
       out.q_begin = __builtin_amdgcn_readlane(q_begin[i], l), out.q_end = __builtin_amdgcn_readlane(q_end[i], l);
       out.one_segment = __builtin_amdgcn_readlane(one_segment[i], l);
     }
-    base += __builtin_amdgcn_readlane(upto, 63);
-  }
   return out;
 }
 

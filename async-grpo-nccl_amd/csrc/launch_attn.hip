@@ -28,13 +28,17 @@ int attn_heads_per_group(const Tuning& tn, int G, int T, int n_seq) {
   return G >= 3 ? 4 : 1;
 }
 
+int attn_query_blocks(int hb, int T, int Hq, int Hkv) {                      // work-groups of an undivided launch: (tile, K/V head) units by eight, times the heads of a group
+  const int rb = 128 / hb, G = Hq / Hkv;
+  const long long units = (long long)((T + rb - 1) / rb) * Hkv;
+  return (int)((units + 7) / 8 * 8 * ((G + hb - 1) / hb));
+}
+
 template <template <int, int> class Launcher>
 int launch_query_side(int form, int D, int hb, AttnParams& p, int T, int Hq, int Hkv, int32_t* bounds_ws, hipStream_t st) {
-  const int rb = 128 / hb, G = Hq / Hkv;
   p.order_q = bounds_ws + attn_order_offset(T, hb == 1 ? 1 : hb == 2 ? 2 : 3);
-  const long long units = (long long)((T + rb - 1) / rb) * Hkv;            // (tile, K/V head)
-  p.blocks_q = (int)(((units + 7) / 8 * 8) * ((G + hb - 1) / hb));
-  const dim3 grid((unsigned)p.blocks_q * (p.parts_q > 1 ? p.parts_q : 1));
+  p.blocks_q = attn_query_blocks(hb, T, Hq, Hkv);
+  const dim3 grid((unsigned)(p.blocks_q + (p.parts_q > 1 ? 8 * p.extra_q : 0)));
   if (D == 128) {
     if (hb == 1) Launcher<128, 1>::run(form, grid, st, p);
     else if (hb == 2) Launcher<128, 2>::run(form, grid, st, p);
@@ -63,36 +67,36 @@ struct DqLauncher {
     else hipLaunchKernelGGL((varlen_attn_dq2_kernel<HD, HB>), grid, dim3(256), 0, st, p);
   }
 };
-// How the tiles of a launch are dealt to several work-groups (attn_parts).  A launch of few tiles ends when its longest
-// chain of steps does, however idle the device is; sharing a chain costs fp32 sums through memory and one more launch.
-// Both sides are estimated, in us, from what was measured: `step` for a step of a work-group alone on its CU, half as
-// much again where two share one; 4 us for the additional launch, 3 TB/s for the sums, written and read.  The tiles of a
-// causal launch walk 0 .. chain steps, evenly; segments of one call are taken to be as long as their mean (twice that
-// at most: the number of parts allowed for); one long segment among many short ones is judged by that mean and may stay
-// whole.  Decided by shapes alone.  Whole | dealt out, merge launch included, 12 / 2 heads of 128: one segment of 777
-// tokens, forward 25.2 | 19.2 us (16.7 now, see attn_merge_query_tile), backward 86.7 | 44.2 (38.9); of 6000 tokens 182 | 161 and 584 | 465; 3 segments of 1024 tokens,
-// forward 29.2 | 42, which the estimate refuses.
+// Whether the tiles of a launch are dealt to several work-groups, and to how many at most (the kernels then go by the true
+// lengths, see attn_deal).  A launch of few tiles ends when its longest chain of steps does, however idle the device is;
+// sharing a chain costs fp32 sums through memory and mostly one more launch.  Both sides are estimated, in us, from what was
+// measured: `step` for a step of a work-group alone on its CU, half as much again where two share one, `open` steps to
+// open and close a work-group.  Decided by shapes alone: the longest segment of four or more is taken to be 1.75 means
+// long (lengths spread evenly).  Whole | dealt out, merge launch included, 12 / 2 heads of 128: one segment of 777
+// tokens, forward 22.5 | 16.5 us, backward 77.8 | 36.7; of 2000 50.0 | 31.8 and 147 | 74.
 struct SplitPlan {
-  int parts = 1, per = 1;
-  int extra = 0, deal = 1;               // key side, see AttnParams
+  int parts = 1, per = 1;                // most parts of a tile, steps a part walks at least
+  int extra = 0, deal = 1;               // see AttnParams
+  int grid = 0;                          // work-groups of the launch
 };
-SplitPlan plan_split(long long wgs, int per_cu, double chain, bool causal, double step, size_t bytes_a_part) {
+double shared_step(double step, int per_cu, double n) {      // step time with n work-groups in flight
+  const double over = per_cu > 1 ? n / num_cus() - 1.0 : 0.0;
+  return step * (1.0 + 0.5 * (over < 0.0 ? 0.0 : over > 1.0 ? 1.0 : over));
+}
+// Without the mask: the tiles of a segment have equal chains.  Parts of a steps' count of their own; 4 us for the merge, 3 TB/s for the sums, written and read.
+SplitPlan plan_even(long long wgs, int blocks, int per_cu, double chain, double step, size_t bytes_a_part) {
   SplitPlan best;
-  const double cus = num_cus(), slots = cus * per_cu, fill = causal ? 0.5 : 1.0;
-  auto shared = [&](double n) {            // step time with n work-groups in flight
-    const double over = per_cu > 1 ? n / cus - 1.0 : 0.0;
-    return step * (1.0 + 0.5 * (over < 0.0 ? 0.0 : over > 1.0 ? 1.0 : over));
-  };
-  const double load = (double)wgs * chain * fill / slots * shared(2.0 * slots);
+  const double slots = (double)num_cus() * per_cu;
+  auto shared = [&](double n) { return shared_step(step, per_cu, n); };
+  const double load = (double)wgs * chain / slots * shared(2.0 * slots);
   const double whole = chain * shared((double)wgs) > load ? chain * shared((double)wgs) : load;
   double least = 0.85 * whole;
   for (int n = 2; n <= kAttnMaxParts; ++n) {
     const int per = (int)(chain / n) + 1;
     if ((size_t)n * bytes_a_part > kAttnSplitMaxBytes || per < 2) break;
-    const double x = chain / per;          // parts of the longest tile
-    const double mean = causal ? x / 2 + 0.5 : x, sums = causal ? mean - 1.0 / x : mean;
-    const double walk = per * shared(wgs * mean);
-    const double cost = (walk > load ? walk : load) + 4.0 + sums * (double)bytes_a_part * 2.0 / 3.0e6;
+    const double x = chain / per;          // parts of a tile
+    const double walk = per * shared(wgs * x);
+    const double cost = (walk > load ? walk : load) + 4.0 + x * (double)bytes_a_part * 2.0 / 3.0e6;
     if (cost >= least) continue;
     least = cost;
     const int parts = (int)(2.0 * x) + 1, fit = (int)(kAttnSplitMaxBytes / bytes_a_part);
@@ -100,77 +104,98 @@ SplitPlan plan_split(long long wgs, int per_cu, double chain, bool causal, doubl
     if (best.parts > fit) best.parts = fit;
     best.per = per;
   }
+  best.extra = blocks / 8 * (best.parts - 1), best.deal = blocks / 8 * best.parts;
   return best;
 }
-SplitPlan plan_query_split(const Tuning& tn, int form, int T, int n_seq, int Hq, int Hkv, int D, int causal, bool forward) {
-  if (form == 1 || (!forward && form == 3)) return SplitPlan();
-  const int hb = attn_heads_per_group(tn, Hq / Hkv, T, n_seq), rb = 128 / hb, G = Hq / Hkv;
-  const long long wgs = (long long)((T + rb - 1) / rb) * Hkv * ((G + hb - 1) / hb);
-  return plan_split(wgs, 2, (double)T / n_seq / kAttnBK, causal, D == 128 ? 1.6 : forward ? 1.15 : 1.3,
-                    (size_t)T * Hq * (D * 4 + (forward ? 8 : 0)));
-}
-// dK/dV under the causal mask: the same estimate, in items of a wavefront (`step` us each, `open` of them to open and close
-// a work-group), for the way attn_key_deal numbers the parts.  The longest segment of four or more is taken to be 1.75 means long
-// (lengths spread evenly; the kernel goes by the true ones).  Either every part is in flight at once - the items go by the
-// work-groups the tiles leave over - or, with about as many tiles as the device holds or more, the long tiles are cut to
-// one and a half times a CU's load, 40 items at most.  A first part that waits for a CU costs more than its own items: launches
-// order work-groups by shader engine, so 260 parts on 256 CUs took 120 us where 250 took 100 (3000 tokens in 4
-// segments, 12 / 2 heads of 128).  Whole | dealt out, dQ and merge included: 6000 tokens in 13 segments, 16 / 4
-// heads 150 | 123 (the estimate refuses it: the longest is 3.7 means); 4000 in 6, 28 / 4 heads 124 | 115; 5000 in one, 28 / 4
+// Under the causal mask the tiles of a segment walk 0 .. chain steps, evenly; `sum` steps of all tiles, `longest` steps a tile could have at most.
+// Either every part is in flight at once - the steps go by the work-groups the tiles leave over, of one a CU or of all - or, with about
+// as many tiles as the device holds or more, the long tiles are cut to one and a half times a work-group's share, 40 steps
+// at most.  A first part that waits for a CU costs more than its own steps: launches order work-groups by shader engine, so 260 parts
+// on 256 CUs took 120 us where 250 took 100 (dK/dV of 3000 tokens in 4 segments, 12 / 2 heads of 128).  Sums are taken at 6 TB/s, most
+// of them leaving while others still walk; a part is no shorter than its own are worth at 3 (`worth` times, `at_most`: measured at
+// 2 .. 12 steps).  dK/dV whole | dealt out, dQ and
+// merge included: 6000 tokens in 13 segments, 16 / 4 heads 150 | 123; 4000 in 6, 28 / 4 heads 124 | 115; 5000 in one, 28 / 4
 // heads 645 | 609; 12345 in 23, 14 / 2 heads of 64 87 | 94 and 4000 in 5, 32 / 8 heads of 64 83 | 96, both refused.
-SplitPlan plan_key_split(int form, int T, int n_seq, int Hq, int Hkv, int D, int causal) {
-  if (form == 1 || form == 2) return SplitPlan();
-  const int keys = attn_keyside_keys(D);
-  const long long wgs = (long long)((T + keys - 1) / keys) * Hkv;
-  const int blocks = attn_keyside_blocks(D, T, Hkv), per_cu = D == 128 ? 1 : 2, slots = num_cus() * per_cu;
-  if (blocks > 8 * kAttnDealSlots) return SplitPlan();
-  const double spread = n_seq >= 4 ? 1.75 : 1.0, mean = (double)T / n_seq, longest = mean * spread;
-  const double items = (Hq / Hkv) / 4.0 / 32, step = D == 128 ? 1.4 : 0.65, open = D == 128 ? 6.0 : 4.0;      // of a wavefront, a token
+SplitPlan plan_uneven(long long wgs, int blocks, int per_cu, double chain, double sum, double longest, double step, double open, double bytes_a_part, double worth, double at_most, double merge) {
   SplitPlan s;
-  if (!causal) {
-    s = plan_split(wgs, per_cu, mean * items, causal, D == 128 ? 1.3 : 0.65, (size_t)T * Hkv * D * 8);
-    if (s.parts <= 1) return s;
-    s.extra = blocks / 8 * (s.parts - 1), s.deal = blocks / 8 * s.parts;
-    return s;
-  }
-  const double rest = T - longest, seen = n_seq >= 4 ? (longest * longest + rest * rest / (n_seq - 1)) / T : mean;
-  const double chain = longest * items, sum = wgs * (seen * 0.5 + 16 + (n_seq > 1 ? attn_keyside_keys(D) : 0)) * items;      // blocks of queries begun; tiles that reach into the next segment
-  auto shared = [&](double n) {
-    const double over = per_cu > 1 ? n / num_cus() - 1.0 : 0.0;
-    return step * (1.0 + 0.5 * (over < 0.0 ? 0.0 : over > 1.0 ? 1.0 : over));
-  };
+  const double cus = num_cus(), slots = cus * per_cu, load = sum / slots;
+  auto shared = [&](double n) { return shared_step(step, per_cu, n); };
   auto most = [](double a, double b) { return a > b ? a : b; };
   const double whole = most((chain + open) * shared((double)wgs), (sum + wgs * open) / slots * shared(2.0 * slots));
-  // a part more costs its sums, written and read; a longer part the wait for it
-  const double sums = attn_keyside_keys(D) * D * 16.0 / 3.0e6, least = floor(most(sqrt(sum * sums / step), 1.5) + 0.5);
-  const double cap = most(least, chain / kAttnMaxParts), load = sum / slots;
-  const double once = wgs < slots ? most(most(sum / (slots - 0.5 * wgs), chain * (2.0 - (double)slots / wgs)), cap) : 1e30;      // items a part walks: all parts in flight at once
-  const double fill = most(1.5 * load < 40.0 ? 1.5 * load : 40.0, cap);                                                    // ... or more of them than the device holds
+  const double sums = bytes_a_part * 2.0 / 3.0e6, even = worth * sqrt(sum * sums / step), least = floor(most(even < at_most ? even : at_most, 1.5) + 0.5);
+  const double cap = most(least, chain / kAttnMaxParts);
   auto parts = [&](double per) { return per < chain ? sum / per + 0.5 * wgs : (double)wgs; };
-  const double t_once = (once + open) * shared(parts(once));
-  const double t_fill = (load + parts(fill) * open / slots + 0.5 * fill + (wgs < slots ? 2.0 * open : 0.0)) * shared(2.0 * slots);
-  const bool fits = t_once < t_fill;
-  const double dealt = (fits ? t_once : t_fill) + 4.0 + most(parts(fits ? once : fill) - 0.5 * wgs, 0.0) * sums * 0.5;
-  if (dealt >= (fits ? 0.97 : 1.0) * whole) return s;
-  s.parts = kAttnMaxParts, s.per = (int)least;
-  s.extra = fits ? (slots - blocks) / 8 : (int)(load / fill * slots / 8) + 1;
-  s.deal = fits ? (slots - blocks / 2) / 8 : s.extra;
-  const int ways = (int)(T * items / least) + 1, bound = blocks / 8 * ((ways < kAttnMaxParts ? ways : kAttnMaxParts) - 1);      // if every tile had all queries
+  double per = most(1.5 * load < 40.0 ? 1.5 * load : 40.0, cap), room = 0.0;
+  double walk = (load + parts(per) * open / slots + 0.5 * per + (wgs < slots ? 2.0 * open : 0.0)) * shared(2.0 * slots);
+  for (double r = cus; r <= slots; r += cus) {
+    if (wgs >= r) continue;
+    const double x = most(most(sum / (r - 0.5 * wgs), chain * (2.0 - r / wgs)), cap), t = (x + open) * shared(parts(x));
+    if (t < walk) walk = t, per = x, room = r;
+  }
+  if (walk + merge + most(parts(per) - 0.5 * wgs, 0.0) * sums * 0.5 >= whole) return s;
+  s.per = (int)least;
+  s.extra = room > 0.0 ? ((int)room - blocks) / 8 : (int)(load / per * slots / 8) + 1;
+  s.deal = room > 0.0 ? ((int)room - blocks / 2) / 8 : s.extra;
+  const int ways = (int)(longest / least) + 1, bound = blocks / 8 * ((ways < kAttnMaxParts ? ways : kAttnMaxParts) - 1);
   if (s.extra > bound) s.extra = bound;
-  if (s.extra < 1) s = SplitPlan();
+  if (s.extra >= 1 && (blocks + 8 * s.extra) * bytes_a_part <= kAttnSplitMaxBytes) s.parts = kAttnMaxParts;
+  return s;
+}
+// queries or keys that a token's segment has, and the longest segment
+struct SegmentGuess {
+  double longest, seen;
+};
+SegmentGuess guess_segments(int T, int n_seq) {
+  const double mean = (double)T / n_seq;
+  if (n_seq < 4) return SegmentGuess{mean, mean};
+  const double longest = 1.75 * mean, rest = T - longest;
+  return SegmentGuess{longest, (longest * longest + rest * rest / (n_seq - 1)) / T};
+}
+SplitPlan plan_query_split(const Tuning& tn, int form, int T, int n_seq, int Hq, int Hkv, int D, int causal, bool forward, bool merged) {
+  if (form == 1 || (!forward && form == 3)) return SplitPlan();
+  const int hb = attn_heads_per_group(tn, Hq / Hkv, T, n_seq), rb = 128 / hb, nb = (Hq / Hkv + hb - 1) / hb;
+  const int blocks = attn_query_blocks(hb, T, Hq, Hkv);
+  const long long wgs = (long long)((T + rb - 1) / rb) * Hkv * nb;
+  if (blocks / nb > 8 * kAttnDealSlots) return SplitPlan();
+  const double step = D == 128 ? 1.6 : forward ? 1.15 : 1.3;
+  SplitPlan s;
+  if (!causal) {
+    s = plan_even(wgs, blocks, 2, (double)T / n_seq / kAttnBK, step, (size_t)T * Hq * (D * 4 + (forward ? 8 : 0)));
+  } else {
+    const SegmentGuess g = guess_segments(T, n_seq);
+    const double sum = wgs * (g.seen * 0.5 + 32 + (n_seq > 1 ? rb : 0)) / kAttnBK;      // steps begun; tiles that reach into the next segment
+    s = plan_uneven(wgs, blocks, 2, g.longest / kAttnBK, sum, (double)T / kAttnBK, step, 1.5, 128.0 * D * 4, 1.35, 8.0, merged ? 0.5 : 4.0);
+  }
+  s.grid = blocks + 8 * s.extra;
+  return s;
+}
+SplitPlan plan_key_split(int form, int T, int n_seq, int Hq, int Hkv, int D, int causal) {
+  if (form == 1 || form == 2) return SplitPlan();
+  const int keys = attn_keyside_keys(D), blocks = attn_keyside_blocks(D, T, Hkv), per_cu = D == 128 ? 1 : 2;
+  const long long wgs = (long long)((T + keys - 1) / keys) * Hkv;
+  if (blocks > 8 * kAttnDealSlots) return SplitPlan();
+  const double items = (Hq / Hkv) / 4.0 / 32;           // of one of the four wavefronts, a token
+  SplitPlan s;
+  if (!causal) {
+    s = plan_even(wgs, blocks, per_cu, (double)T / n_seq * items, D == 128 ? 1.3 : 0.65, (size_t)T * Hkv * D * 8);
+  } else {
+    const SegmentGuess g = guess_segments(T, n_seq);
+    const double sum = wgs * (g.seen * 0.5 + 16 + (n_seq > 1 ? keys : 0)) * items;
+    s = plan_uneven(wgs, blocks, per_cu, g.longest * items, sum, T * items, D == 128 ? 1.4 : 0.65, D == 128 ? 6.0 : 4.0, keys * D * 8.0, 1.0, 1e30, 4.0);
+  }
+  s.grid = blocks + 8 * s.extra;
   return s;
 }
 size_t align256(size_t n) { return (n + 255) / 256 * 256; }
-size_t query_sums_bytes(const SplitPlan& s, int T, int Hq, int D) { return align256((size_t)s.parts * ((T + 31) / 32 * 32) * Hq * D * 4); }
-size_t query_split_bytes(const SplitPlan& s, int T, int Hq, int D, bool forward) {
-  if (s.parts <= 1) return 0;
-  return query_sums_bytes(s, T, Hq, D) + (forward ? align256((size_t)s.parts * T * Hq * 8) : 0);
+size_t query_sums_bytes(const SplitPlan& s, int D) { return align256((size_t)s.grid * 128 * D * 4); }
+size_t query_info_bytes(int T, int Hkv) { return align256((size_t)((T + 31) / 32) * Hkv * sizeof(int2)); }
+size_t query_split_bytes(const SplitPlan& s, int T, int Hkv, int D, bool forward) {
+  return s.parts <= 1 ? 0 : query_sums_bytes(s, D) + query_info_bytes(T, Hkv) + (forward ? align256((size_t)s.grid * 128 * sizeof(float2)) : 0);
 }
-size_t key_sums_bytes(const SplitPlan& s, int T, int Hkv, int D) { return align256((size_t)(attn_keyside_blocks(D, T, Hkv) + 8 * s.extra) * attn_keyside_keys(D) * D * 8); }
+size_t key_sums_bytes(const SplitPlan& s, int D) { return align256((size_t)s.grid * attn_keyside_keys(D) * D * 8); }
 size_t key_split_bytes(const SplitPlan& s, int T, int Hkv, int D) {
-  if (s.parts <= 1) return 0;
   const int keys = attn_keyside_keys(D);
-  return key_sums_bytes(s, T, Hkv, D) + align256((size_t)((T + keys - 1) / keys) * Hkv * sizeof(int2));
+  return s.parts <= 1 ? 0 : key_sums_bytes(s, D) + align256((size_t)((T + keys - 1) / keys) * Hkv * sizeof(int2));
 }
 }  // namespace
 
@@ -224,8 +249,9 @@ int fgrpo_varlen_attn_bounds(const int32_t* cu, int n_seq, int T, int causal, in
 size_t fgrpo_varlen_attn_workspace(int T, int n_seq, int Hq, int Hkv, int D, int causal, int backward) {
   if (T <= 0 || n_seq <= 0 || Hq <= 0 || Hkv <= 0 || Hq % Hkv != 0 || (D != 128 && D != 64)) return 0;
   const Tuning tn = g_tune;
-  const size_t q = query_split_bytes(plan_query_split(tn, tn.attn_qside, T, n_seq, Hq, Hkv, D, causal, !backward), T, Hq, D, !backward);
-  return backward ? q + key_split_bytes(plan_key_split(tn.attn_dkv, T, n_seq, Hq, Hkv, D, causal), T, Hkv, D) : q;
+  const SplitPlan sk = backward ? plan_key_split(tn.attn_dkv, T, n_seq, Hq, Hkv, D, causal) : SplitPlan();
+  const SplitPlan sq = plan_query_split(tn, tn.attn_qside, T, n_seq, Hq, Hkv, D, causal, !backward, sk.parts > 1);
+  return query_split_bytes(sq, T, Hkv, D, !backward) + key_split_bytes(sk, T, Hkv, D);
 }
 
 int fgrpo_varlen_attn_fwd(const void* q, const void* k, const void* v, long long q_st, long long q_sh, long long k_st,
@@ -255,14 +281,15 @@ int fgrpo_varlen_attn_fwd_ws(const void* q, const void* k, const void* v, long l
   }
   const Tuning tn = g_tune;   // one reading of the tuning state per call: the kernel launched is the one the split was planned for
   const int form = attn_query_form(tn.attn_qside, q_st, k_st, v_st, Hq, D), hb = attn_heads_per_group(tn, Hq / Hkv, T, n_seq);
-  SplitPlan sp = plan_query_split(tn, form, T, n_seq, Hq, Hkv, D, causal, true);
-  const size_t need = query_split_bytes(sp, T, Hq, D, true);
+  SplitPlan sp = plan_query_split(tn, form, T, n_seq, Hq, Hkv, D, causal, true, false);
+  const size_t need = query_split_bytes(sp, T, Hkv, D, true);
   if (!ws || need == 0) sp = SplitPlan();
   else if (ws_bytes < need) return fail(FGRPO_ERR_WORKSPACE, "varlen_attn_fwd: workspace %zu < %zu", ws_bytes, need);
   else if (!aligned16(ws)) return fail(FGRPO_ERR_ALIGN, "varlen_attn_fwd: workspace must be 16-byte aligned");
-  p.parts_q = sp.parts, p.per_q = sp.per;
+  p.parts_q = sp.parts, p.per_q = sp.per, p.extra_q = sp.extra, p.deal_q = sp.deal;
   p.part_q = (float*)ws;
-  p.part_ml = (float2*)((char*)ws + query_sums_bytes(sp, T, Hq, D));
+  p.query_info = (int2*)((char*)ws + query_sums_bytes(sp, D));
+  p.part_ml = (float2*)((char*)ws + query_sums_bytes(sp, D) + query_info_bytes(T, Hkv));
   rc = launch_query_side<FwdLauncher>(form, D, hb, p, T, Hq, Hkv, bounds_ws, st);
   if (rc || sp.parts <= 1) return rc;
   const unsigned blocks = (unsigned)((T + 31) / 32) * (unsigned)Hq;
@@ -307,16 +334,18 @@ int fgrpo_varlen_attn_bwd_ws(const void* dout, const void* q, const void* k, con
   const Tuning tn = g_tune;   // one reading of the tuning state per call: the kernel launched is the one the split was planned for
   const int form = attn_query_form(tn.attn_qside, q_st, k_st, v_st, Hq, D), hb = attn_heads_per_group(tn, Hq / Hkv, T, n_seq);
   const int key_form = attn_key_form(tn.attn_dkv, q_st, k_st, v_st, T, Hq, Hkv, D, attn_keyside_keys(D));
-  SplitPlan sq = plan_query_split(tn, form, T, n_seq, Hq, Hkv, D, causal, false), sk = plan_key_split(key_form, T, n_seq, Hq, Hkv, D, causal);
-  const size_t need_q = query_split_bytes(sq, T, Hq, D, false), need = need_q + key_split_bytes(sk, T, Hkv, D);
+  SplitPlan sk = plan_key_split(key_form, T, n_seq, Hq, Hkv, D, causal), sq = plan_query_split(tn, form, T, n_seq, Hq, Hkv, D, causal, false, sk.parts > 1);
+  const size_t need_q = query_split_bytes(sq, T, Hkv, D, false), need = need_q + key_split_bytes(sk, T, Hkv, D);
   if (!ws || need == 0) sq = sk = SplitPlan();
   else if (ws_bytes < need) return fail(FGRPO_ERR_WORKSPACE, "varlen_attn_bwd: workspace %zu < %zu", ws_bytes, need);
   else if (!aligned16(ws)) return fail(FGRPO_ERR_ALIGN, "varlen_attn_bwd: workspace must be 16-byte aligned");
   if (key_form != 3) sq = sk = SplitPlan();
-  p.parts_q = sq.parts, p.per_q = sq.per, p.parts_k = sk.parts, p.per_k = sk.per, p.extra_k = sk.extra, p.deal_k = sk.deal;
+  p.parts_q = sq.parts, p.per_q = sq.per, p.extra_q = sq.extra, p.deal_q = sq.deal;
+  p.parts_k = sk.parts, p.per_k = sk.per, p.extra_k = sk.extra, p.deal_k = sk.deal;
   p.part_q = (float*)ws;
+  p.query_info = (int2*)((char*)ws + query_sums_bytes(sq, D));
   p.part_k = (float*)((char*)ws + need_q);
-  p.key_info = (int2*)((char*)ws + need_q + key_sums_bytes(sk, T, Hkv, D));
+  p.key_info = (int2*)((char*)ws + need_q + key_sums_bytes(sk, D));
   rc = launch_query_side<DqLauncher>(form, D, hb, p, T, Hq, Hkv, bounds_ws, st);
   if (rc) return rc;
   if (key_form == 3) {

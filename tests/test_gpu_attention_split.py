@@ -87,9 +87,9 @@ def lengths(T, lo, hi):
     (2000, [2000], 14, 2, 64), (2000, [2000], 12, 2, 128), (2000, lengths(2000, 128, 512), 28, 4, 128),      # all parts in flight at once, none to spare
     (3000, [1916, 200, 700, 184], 12, 2, 128), (3001, lengths(3001, 128, 512), 28, 4, 128),
     (4000, lengths(4000, 128, 1024), 28, 4, 128), (5000, [5000], 28, 4, 128), (9000, lengths(9000, 128, 2048), 12, 2, 128),      # more parts than the device holds
-    (9000, lengths(9000, 128, 2048), 14, 2, 64), (70, [70], 12, 1, 128), (5, [2, 3], 64, 1, 128)])           # more than 64 tiles an XCD; two tiles; one, left whole
-def test_key_tiles_dealt_by_their_items_agree_with_whole_ones(dev, T, lens, Hq, Hkv, D):
-    """Bounds as in test_divided_tiles_agree_with_whole_ones: the output that the backward starts from may come from parts too."""
+    (9000, lengths(9000, 128, 2048), 14, 2, 64), (9000, [4300, 4700], 8, 2, 128), (1501, [1024, 477], 12, 2, 128), (70, [70], 12, 1, 128), (5, [2, 3], 64, 1, 128)])           # more than 64 tiles an XCD; two tiles; one, left whole
+def test_tiles_dealt_by_their_steps_agree_with_whole_ones(dev, T, lens, Hq, Hkv, D):
+    """Bounds as in test_divided_tiles_agree_with_whole_ones."""
     from fgrpo import _lib, ops
     q, k, v, do = operands(T, Hq, Hkv, D, dev)
     cu = torch.tensor([0] + torch.tensor(lens).cumsum(0).tolist(), dtype=torch.int32, device=dev)
@@ -99,8 +99,9 @@ def test_key_tiles_dealt_by_their_items_agree_with_whole_ones(dev, T, lens, Hq, 
 
     def once():
         a = [x.clone().requires_grad_(True) for x in (q, k, v)]
-        return torch.autograd.grad(ops.varlen_attention(*a, cu, None, True), a, do)
-    for name, x, y, z in zip(("dq", "dk", "dv"), once(), want, once()):
+        o = ops.varlen_attention(*a, cu, None, True)
+        return (o.detach(),) + torch.autograd.grad(o, a, do)
+    for name, x, y, z in zip(("out", "dq", "dk", "dv"), once(), (out, *want), once()):
         assert torch.equal(x, z), f"{name} is not reproducible"
         assert (x.float() - y.float()).norm() <= 2 ** -7 * y.float().norm(), name
 
