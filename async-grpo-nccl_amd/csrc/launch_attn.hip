@@ -71,8 +71,10 @@ struct DqLauncher {
 // lengths, see attn_deal).  A launch of few tiles ends when its longest chain of steps does, however idle the device is;
 // sharing a chain costs fp32 sums through memory and mostly one more launch.  Both sides are estimated, in us, from what was
 // measured: `step` for a step of a work-group alone on its CU, half as much again where two share one, `open` steps to
-// open and close a work-group.  Decided by shapes alone: the longest segment of four or more is taken to be 1.75 means
-// long (lengths spread evenly).  Whole | dealt out, merge launch included, 12 / 2 heads of 128: one segment of 777
+// open and close a work-group.  Decided by shapes and the length that the caller gives for the longest segment; where it
+// gives none, that of four or more is taken to be 1.75 means long (lengths spread evenly).  A wrong length costs time, nothing else.
+// Guessed | told, forward and backward, us: 6000 tokens in 13 segments, one of 1694, 16 / 4 heads 47.1, 148 | 39.7, 115; 1500 in 2,
+// one of 997, 14 / 2 heads of 64 20.1, 33.1 | 16.2, 32.8; 2000 in 3, one of 970, 12 / 2 heads 27.1, 57.5 | 23.3, 53.5.  Whole | dealt out, merge launch included, 12 / 2 heads of 128: one segment of 777
 // tokens, forward 22.5 | 16.5 us, backward 77.8 | 36.7; of 2000 50.0 | 31.8 and 147 | 74.
 struct SplitPlan {
   int parts = 1, per = 1;                // most parts of a tile, steps a part walks at least
@@ -126,7 +128,8 @@ SplitPlan plan_uneven(long long wgs, int blocks, int per_cu, double chain, doubl
   const double cap = most(least, chain / kAttnMaxParts);
   auto parts = [&](double per) { return per < chain ? sum / per + 0.5 * wgs : (double)wgs; };
   double per = most(1.5 * load < 40.0 ? 1.5 * load : 40.0, cap), room = 0.0;
-  double walk = (load + parts(per) * open / slots + 0.5 * per + (wgs < slots ? 2.0 * open : 0.0)) * shared(2.0 * slots);
+  const double spare = 1.0 - wgs / slots;
+  double walk = (load + parts(per) * open / slots + 0.5 * per + (spare < 0.0 ? 0.0 : spare < 0.25 ? 8.0 * spare : 2.0) * open) * shared(2.0 * slots);
   for (double r = cus; r <= slots; r += cus) {
     if (wgs >= r) continue;
     const double x = most(most(sum / (r - 0.5 * wgs), chain * (2.0 - r / wgs)), cap), t = (x + open) * shared(parts(x));
@@ -145,13 +148,15 @@ SplitPlan plan_uneven(long long wgs, int blocks, int per_cu, double chain, doubl
 struct SegmentGuess {
   double longest, seen;
 };
-SegmentGuess guess_segments(int T, int n_seq) {
+SegmentGuess guess_segments(int T, int n_seq, int max_len) {
   const double mean = (double)T / n_seq;
-  if (n_seq < 4) return SegmentGuess{mean, mean};
-  const double longest = 1.75 * mean, rest = T - longest;
+  if (n_seq == 1 || (max_len <= 0 && n_seq < 4)) return SegmentGuess{mean, mean};
+  double longest = max_len > 0 ? max_len : 1.75 * mean;
+  longest = longest < mean ? mean : longest > T ? T : longest;
+  const double rest = T - longest;
   return SegmentGuess{longest, (longest * longest + rest * rest / (n_seq - 1)) / T};
 }
-SplitPlan plan_query_split(const Tuning& tn, int form, int T, int n_seq, int Hq, int Hkv, int D, int causal, bool forward, bool merged) {
+SplitPlan plan_query_split(const Tuning& tn, int form, int T, int n_seq, int max_len, int Hq, int Hkv, int D, int causal, bool forward, bool merged) {
   if (form == 1 || (!forward && form == 3)) return SplitPlan();
   const int hb = attn_heads_per_group(tn, Hq / Hkv, T, n_seq), rb = 128 / hb, nb = (Hq / Hkv + hb - 1) / hb;
   const int blocks = attn_query_blocks(hb, T, Hq, Hkv);
@@ -162,14 +167,14 @@ SplitPlan plan_query_split(const Tuning& tn, int form, int T, int n_seq, int Hq,
   if (!causal) {
     s = plan_even(wgs, blocks, 2, (double)T / n_seq / kAttnBK, step, (size_t)T * Hq * (D * 4 + (forward ? 8 : 0)));
   } else {
-    const SegmentGuess g = guess_segments(T, n_seq);
+    const SegmentGuess g = guess_segments(T, n_seq, max_len);
     const double sum = wgs * (g.seen * 0.5 + 32 + (n_seq > 1 ? rb : 0)) / kAttnBK;      // steps begun; tiles that reach into the next segment
-    s = plan_uneven(wgs, blocks, 2, g.longest / kAttnBK, sum, (double)T / kAttnBK, step, 1.5, 128.0 * D * 4, 1.35, 8.0, merged ? 0.5 : 4.0);
+    s = plan_uneven(wgs, blocks, 2, g.longest / kAttnBK, sum, (double)T / kAttnBK, step, 1.5, 128.0 * D * 4, 1.35, 7.0, merged ? 0.5 : 4.0);
   }
   s.grid = blocks + 8 * s.extra;
   return s;
 }
-SplitPlan plan_key_split(int form, int T, int n_seq, int Hq, int Hkv, int D, int causal) {
+SplitPlan plan_key_split(int form, int T, int n_seq, int max_len, int Hq, int Hkv, int D, int causal) {
   if (form == 1 || form == 2) return SplitPlan();
   const int keys = attn_keyside_keys(D), blocks = attn_keyside_blocks(D, T, Hkv), per_cu = D == 128 ? 1 : 2;
   const long long wgs = (long long)((T + keys - 1) / keys) * Hkv;
@@ -179,7 +184,7 @@ SplitPlan plan_key_split(int form, int T, int n_seq, int Hq, int Hkv, int D, int
   if (!causal) {
     s = plan_even(wgs, blocks, per_cu, (double)T / n_seq * items, D == 128 ? 1.3 : 0.65, (size_t)T * Hkv * D * 8);
   } else {
-    const SegmentGuess g = guess_segments(T, n_seq);
+    const SegmentGuess g = guess_segments(T, n_seq, max_len);
     const double sum = wgs * (g.seen * 0.5 + 16 + (n_seq > 1 ? keys : 0)) * items;
     s = plan_uneven(wgs, blocks, per_cu, g.longest * items, sum, T * items, D == 128 ? 1.4 : 0.65, D == 128 ? 6.0 : 4.0, keys * D * 8.0, 1.0, 1e30, 4.0);
   }
@@ -247,10 +252,14 @@ int fgrpo_varlen_attn_bounds(const int32_t* cu, int n_seq, int T, int causal, in
 }
 
 size_t fgrpo_varlen_attn_workspace(int T, int n_seq, int Hq, int Hkv, int D, int causal, int backward) {
+  return fgrpo_varlen_attn_workspace_len(T, n_seq, 0, Hq, Hkv, D, causal, backward);
+}
+
+size_t fgrpo_varlen_attn_workspace_len(int T, int n_seq, int max_len, int Hq, int Hkv, int D, int causal, int backward) {
   if (T <= 0 || n_seq <= 0 || Hq <= 0 || Hkv <= 0 || Hq % Hkv != 0 || (D != 128 && D != 64)) return 0;
   const Tuning tn = g_tune;
-  const SplitPlan sk = backward ? plan_key_split(tn.attn_dkv, T, n_seq, Hq, Hkv, D, causal) : SplitPlan();
-  const SplitPlan sq = plan_query_split(tn, tn.attn_qside, T, n_seq, Hq, Hkv, D, causal, !backward, sk.parts > 1);
+  const SplitPlan sk = backward ? plan_key_split(tn.attn_dkv, T, n_seq, max_len, Hq, Hkv, D, causal) : SplitPlan();
+  const SplitPlan sq = plan_query_split(tn, tn.attn_qside, T, n_seq, max_len, Hq, Hkv, D, causal, !backward, sk.parts > 1);
   return query_split_bytes(sq, T, Hkv, D, !backward) + key_split_bytes(sk, T, Hkv, D);
 }
 
@@ -264,6 +273,14 @@ int fgrpo_varlen_attn_fwd(const void* q, const void* k, const void* v, long long
 
 int fgrpo_varlen_attn_fwd_ws(const void* q, const void* k, const void* v, long long q_st, long long q_sh, long long k_st,
                           long long k_sh, long long v_st, long long v_sh, const int32_t* cu, int n_seq, int T, int Hq,
+                          int Hkv, int D, float scale, int causal, void* out, float* lse, int32_t* bounds_ws,
+                          int bounds_valid, void* ws, size_t ws_bytes, void* stream) {
+  return fgrpo_varlen_attn_fwd_len(q, k, v, q_st, q_sh, k_st, k_sh, v_st, v_sh, cu, n_seq, 0, T, Hq, Hkv, D, scale, causal, out,
+                                   lse, bounds_ws, bounds_valid, ws, ws_bytes, stream);
+}
+
+int fgrpo_varlen_attn_fwd_len(const void* q, const void* k, const void* v, long long q_st, long long q_sh, long long k_st,
+                          long long k_sh, long long v_st, long long v_sh, const int32_t* cu, int n_seq, int max_len, int T, int Hq,
                           int Hkv, int D, float scale, int causal, void* out, float* lse, int32_t* bounds_ws,
                           int bounds_valid, void* ws, size_t ws_bytes, void* stream) {
   hipStream_t st = (hipStream_t)stream;
@@ -281,7 +298,7 @@ int fgrpo_varlen_attn_fwd_ws(const void* q, const void* k, const void* v, long l
   }
   const Tuning tn = g_tune;   // one reading of the tuning state per call: the kernel launched is the one the split was planned for
   const int form = attn_query_form(tn.attn_qside, q_st, k_st, v_st, Hq, D), hb = attn_heads_per_group(tn, Hq / Hkv, T, n_seq);
-  SplitPlan sp = plan_query_split(tn, form, T, n_seq, Hq, Hkv, D, causal, true, false);
+  SplitPlan sp = plan_query_split(tn, form, T, n_seq, max_len, Hq, Hkv, D, causal, true, false);
   const size_t need = query_split_bytes(sp, T, Hkv, D, true);
   if (!ws || need == 0) sp = SplitPlan();
   else if (ws_bytes < need) return fail(FGRPO_ERR_WORKSPACE, "varlen_attn_fwd: workspace %zu < %zu", ws_bytes, need);
@@ -312,6 +329,15 @@ int fgrpo_varlen_attn_bwd_ws(const void* dout, const void* q, const void* k, con
                           const int32_t* cu, int n_seq, int T, int Hq, int Hkv, int D, float scale, int causal, void* dq,
                           void* dk, void* dv, float* delta_ws, int32_t* bounds_ws, int bounds_valid, void* ws,
                              size_t ws_bytes, void* stream) {
+  return fgrpo_varlen_attn_bwd_len(dout, q, k, v, out, lse, q_st, q_sh, k_st, k_sh, v_st, v_sh, cu, n_seq, 0, T, Hq, Hkv, D, scale, causal, dq, dk,
+                                   dv, delta_ws, bounds_ws, bounds_valid, ws, ws_bytes, stream);
+}
+
+int fgrpo_varlen_attn_bwd_len(const void* dout, const void* q, const void* k, const void* v, const void* out, const float* lse,
+                          long long q_st, long long q_sh, long long k_st, long long k_sh, long long v_st, long long v_sh,
+                          const int32_t* cu, int n_seq, int max_len, int T, int Hq, int Hkv, int D, float scale, int causal, void* dq,
+                          void* dk, void* dv, float* delta_ws, int32_t* bounds_ws, int bounds_valid, void* ws,
+                             size_t ws_bytes, void* stream) {
   hipStream_t st = (hipStream_t)stream;
   int rc = check_attn("varlen_attn_bwd", q, k, v, q_st, q_sh, k_st, k_sh, v_st, v_sh, cu, n_seq, T, Hq, Hkv, D, scale, bounds_ws);
   if (rc) return rc;
@@ -334,7 +360,7 @@ int fgrpo_varlen_attn_bwd_ws(const void* dout, const void* q, const void* k, con
   const Tuning tn = g_tune;   // one reading of the tuning state per call: the kernel launched is the one the split was planned for
   const int form = attn_query_form(tn.attn_qside, q_st, k_st, v_st, Hq, D), hb = attn_heads_per_group(tn, Hq / Hkv, T, n_seq);
   const int key_form = attn_key_form(tn.attn_dkv, q_st, k_st, v_st, T, Hq, Hkv, D, attn_keyside_keys(D));
-  SplitPlan sk = plan_key_split(key_form, T, n_seq, Hq, Hkv, D, causal), sq = plan_query_split(tn, form, T, n_seq, Hq, Hkv, D, causal, false, sk.parts > 1);
+  SplitPlan sk = plan_key_split(key_form, T, n_seq, max_len, Hq, Hkv, D, causal), sq = plan_query_split(tn, form, T, n_seq, max_len, Hq, Hkv, D, causal, false, sk.parts > 1);
   const size_t need_q = query_split_bytes(sq, T, Hkv, D, false), need = need_q + key_split_bytes(sk, T, Hkv, D);
   if (!ws || need == 0) sq = sk = SplitPlan();
   else if (ws_bytes < need) return fail(FGRPO_ERR_WORKSPACE, "varlen_attn_bwd: workspace %zu < %zu", ws_bytes, need);

@@ -43,9 +43,9 @@ struct Api {
   FGRPO_ENTRY(fgrpo_grpo_step_chunked);
   FGRPO_ENTRY(fgrpo_scale_gradients);
   FGRPO_ENTRY(fgrpo_shift_labels);
-  FGRPO_ENTRY(fgrpo_varlen_attn_workspace);
-  FGRPO_ENTRY(fgrpo_varlen_attn_fwd_ws);
-  FGRPO_ENTRY(fgrpo_varlen_attn_bwd_ws);
+  FGRPO_ENTRY(fgrpo_varlen_attn_workspace_len);
+  FGRPO_ENTRY(fgrpo_varlen_attn_fwd_len);
+  FGRPO_ENTRY(fgrpo_varlen_attn_bwd_len);
 } api;
 
 void init(const std::unordered_map<std::string, uint64_t>& at) {
@@ -73,9 +73,9 @@ void init(const std::unordered_map<std::string, uint64_t>& at) {
   FGRPO_SET(fgrpo_grpo_step_chunked);
   FGRPO_SET(fgrpo_scale_gradients);
   FGRPO_SET(fgrpo_shift_labels);
-  FGRPO_SET(fgrpo_varlen_attn_workspace);
-  FGRPO_SET(fgrpo_varlen_attn_fwd_ws);
-  FGRPO_SET(fgrpo_varlen_attn_bwd_ws);
+  FGRPO_SET(fgrpo_varlen_attn_workspace_len);
+  FGRPO_SET(fgrpo_varlen_attn_fwd_len);
+  FGRPO_SET(fgrpo_varlen_attn_bwd_len);
 }
 
 void check(int rc, const char* what) { TORCH_CHECK(rc == 0, "fgrpo ", what, " failed (", rc, "): ", api.fgrpo_last_error()); }
@@ -372,8 +372,8 @@ Tensor attn_operand(const Tensor& t, const char* name) {
 int64_t bounds_numel(int64_t T) { return 2 * T + 2 * ((T + 127) / 128) + (T + 63) / 64 + (T + 31) / 32; }
 
 // scratch of a call on a batch with few tiles; none elsewhere
-Tensor attn_workspace(const Tensor& q, const Tensor& cu, int Hkv, bool causal, bool backward) {
-  const size_t n = api.fgrpo_varlen_attn_workspace((int)q.size(0), (int)cu.numel() - 1, (int)q.size(1), Hkv, (int)q.size(2), causal, backward);
+Tensor attn_workspace(const Tensor& q, const Tensor& cu, int max_len, int Hkv, bool causal, bool backward) {
+  const size_t n = api.fgrpo_varlen_attn_workspace_len((int)q.size(0), (int)cu.numel() - 1, max_len, (int)q.size(1), Hkv, (int)q.size(2), causal, backward);
   return n > 0 ? workspace(n, q) : Tensor();
 }
 
@@ -381,6 +381,7 @@ struct AttnArgs {
   Tensor cu, bounds;
   bool bounds_valid, causal;
   double scale;
+  int max_len;                 // the longest segment, 0: not known
 };
 
 struct VarlenAttention : torch::autograd::Function<VarlenAttention> {
@@ -391,10 +392,10 @@ struct VarlenAttention : torch::autograd::Function<VarlenAttention> {
     Tensor out = at::empty({T, Hq, D}, o), lse = at::empty({Hq, T}, o.dtype(at::kFloat));
     if (!a.bounds_valid) a.bounds = at::empty({bounds_numel(T)}, o.dtype(at::kInt));
     OnDevice d(q);
-    const Tensor ws = attn_workspace(q, a.cu, Hkv, a.causal, false);
+    const Tensor ws = attn_workspace(q, a.cu, a.max_len, Hkv, a.causal, false);
     if (T > 0)
-      check(api.fgrpo_varlen_attn_fwd_ws(ptr(q), ptr(k), ptr(v), q.stride(0), q.stride(1), k.stride(0), k.stride(1), v.stride(0),
-                                      v.stride(1), a.cu.data_ptr<int32_t>(), (int)a.cu.numel() - 1, T, Hq, Hkv, D,
+      check(api.fgrpo_varlen_attn_fwd_len(ptr(q), ptr(k), ptr(v), q.stride(0), q.stride(1), k.stride(0), k.stride(1), v.stride(0),
+                                      v.stride(1), a.cu.data_ptr<int32_t>(), (int)a.cu.numel() - 1, a.max_len, T, Hq, Hkv, D,
                                       (float)a.scale, a.causal, out.data_ptr(), fptr(lse), a.bounds.data_ptr<int32_t>(),
                                       a.bounds_valid, ws.defined() ? ws.data_ptr() : nullptr, ws.defined() ? (size_t)ws.numel() : 0, d.stream()),
             "varlen_attn_fwd");
@@ -402,6 +403,7 @@ struct VarlenAttention : torch::autograd::Function<VarlenAttention> {
       ctx->save_for_backward({q_, k_, v_, out, lse, a.cu, a.bounds});
       ctx->saved_data["scale"] = a.scale;
       ctx->saved_data["causal"] = a.causal;
+      ctx->saved_data["max_len"] = (int64_t)a.max_len;
     }
     return out;
   }
@@ -416,12 +418,13 @@ struct VarlenAttention : torch::autograd::Function<VarlenAttention> {
     const auto o = q.options().requires_grad(false);
     Tensor dq = at::empty({T, Hq, D}, o), dk = at::empty({T, Hkv, D}, o), dv = at::empty({T, Hkv, D}, o);
     Tensor delta = at::empty({Hq, T}, o.dtype(at::kFloat));
+    const int max_len = (int)ctx->saved_data["max_len"].toInt();
     OnDevice d(q);
-    const Tensor ws = attn_workspace(q, cu, Hkv, ctx->saved_data["causal"].toBool(), true);
+    const Tensor ws = attn_workspace(q, cu, max_len, Hkv, ctx->saved_data["causal"].toBool(), true);
     if (T > 0)
-      check(api.fgrpo_varlen_attn_bwd_ws(ptr(dout), ptr(q), ptr(k), ptr(v), ptr(out), fptr(lse), q.stride(0), q.stride(1),
+      check(api.fgrpo_varlen_attn_bwd_len(ptr(dout), ptr(q), ptr(k), ptr(v), ptr(out), fptr(lse), q.stride(0), q.stride(1),
                                       k.stride(0), k.stride(1), v.stride(0), v.stride(1), cu.data_ptr<int32_t>(),
-                                      (int)cu.numel() - 1, T, Hq, Hkv, D, (float)ctx->saved_data["scale"].toDouble(),
+                                      (int)cu.numel() - 1, max_len, T, Hq, Hkv, D, (float)ctx->saved_data["scale"].toDouble(),
                                       ctx->saved_data["causal"].toBool(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(),
                                       fptr(delta), bounds.data_ptr<int32_t>(), 1, ws.defined() ? ws.data_ptr() : nullptr,
                                       ws.defined() ? (size_t)ws.numel() : 0, d.stream()),
@@ -431,7 +434,7 @@ struct VarlenAttention : torch::autograd::Function<VarlenAttention> {
 };
 
 Tensor varlen_attention(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& cu, const std::optional<double>& scale,
-                        bool causal, const std::optional<Tensor>& bounds) {
+                        bool causal, const std::optional<Tensor>& bounds, int64_t max_len) {
   require_one_gpu(q, k, v, cu);
   TORCH_CHECK(q.dim() == 3 && k.dim() == 3 && k.sizes() == v.sizes() && k.size(0) == q.size(0) && k.size(2) == q.size(2),
               "fgrpo: q ", q.sizes(), ", k ", k.sizes(), ", v ", v.sizes(), " do not fit together");
@@ -441,6 +444,7 @@ Tensor varlen_attention(const Tensor& q, const Tensor& k, const Tensor& v, const
   a.cu = cu.to(at::kInt).contiguous();
   a.causal = causal;
   a.scale = scale.has_value() ? *scale : 1.0 / std::sqrt((double)q.size(2));
+  a.max_len = (int)std::min<int64_t>(std::max<int64_t>(max_len, 0), T);
   a.bounds_valid = bounds.has_value();
   if (a.bounds_valid) {
     a.bounds = *bounds;

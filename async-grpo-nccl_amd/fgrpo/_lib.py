@@ -74,6 +74,11 @@ SIGNATURES = {
                                       _vp, _vp, _vp, _i, _vp, _sz, _vp]),
     "fgrpo_varlen_attn_bwd_ws": (_i, [_vp, _vp, _vp, _vp, _vp, _vp, _ll, _ll, _ll, _ll, _ll, _ll, _vp, _i, _i, _i, _i, _i,
                                       _f, _i, _vp, _vp, _vp, _vp, _vp, _i, _vp, _sz, _vp]),
+    "fgrpo_varlen_attn_workspace_len": (_sz, [_i, _i, _i, _i, _i, _i, _i, _i]),
+    "fgrpo_varlen_attn_fwd_len": (_i, [_vp, _vp, _vp, _ll, _ll, _ll, _ll, _ll, _ll, _vp, _i, _i, _i, _i, _i, _i, _f, _i,
+                                       _vp, _vp, _vp, _i, _vp, _sz, _vp]),
+    "fgrpo_varlen_attn_bwd_len": (_i, [_vp, _vp, _vp, _vp, _vp, _vp, _ll, _ll, _ll, _ll, _ll, _ll, _vp, _i, _i, _i, _i, _i, _i,
+                                       _f, _i, _vp, _vp, _vp, _vp, _vp, _i, _vp, _sz, _vp]),
 }
 
 _lib = None

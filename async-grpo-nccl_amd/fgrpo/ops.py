@@ -1120,12 +1120,13 @@ class _VarlenAttention(torch.autograd.Function):
         return dq, dk, dv, None, None, None, None
 
 
-def varlen_attention(q, k, v, cu_seqlens, softmax_scale=None, causal=True, bounds=None) -> torch.Tensor:
+def varlen_attention(q, k, v, cu_seqlens, softmax_scale=None, causal=True, bounds=None, max_len: int = 0) -> torch.Tensor:
     """Differentiable packed self-attention on the HIP kernels (bf16 in, bf16 out).  ``bounds``: segment scratch of an
-    earlier call with the same ``cu_seqlens`` and ``causal`` (see ``attention_bounds``)."""
+    earlier call with the same ``cu_seqlens`` and ``causal`` (see ``attention_bounds``).  ``max_len``: length of the longest
+    segment, 0 where it is not known; a short batch is divided better with it, and a wrong one costs time, nothing else."""
     if torch.jit.is_tracing():
         return _VarlenAttention.apply(q, k, v, cu_seqlens, softmax_scale, bool(causal), bounds)
-    return _lib.native().varlen_attention(q, k, v, cu_seqlens, softmax_scale, bool(causal), bounds)
+    return _lib.native().varlen_attention(q, k, v, cu_seqlens, softmax_scale, bool(causal), bounds, max_len)
 
 
 def attention_bounds(cu_seqlens: torch.Tensor, T: int, causal: bool = True) -> torch.Tensor:

@@ -67,13 +67,19 @@ def prepare_from_position_ids(position_ids: torch.Tensor) -> Tuple[torch.Tensor,
     return cu, max_seqlen
 
 
+def _plain_length(n) -> int:
+    """A length to divide a batch by; 0 (not known) for anything but a plain int of a sensible size, a tensor above all:
+    its value would have to be waited for."""
+    return n if type(n) is int and 0 < n < 2 ** 31 else 0
+
+
 def flash_attn_varlen_func(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q=None, max_seqlen_k=None, dropout_p=0.0,
                            softmax_scale=None, causal=False, window_size=(-1, -1), softcap=0.0, alibi_slopes=None,
                            deterministic=False, return_attn_probs=False, block_table=None):
     """``q`` [total, Hq, D], ``k`` / ``v`` [total, Hkv, D] bf16 -> out [total, Hq, D] bf16 (differentiable).
     Self-attention over packed segments: ``cu_seqlens_q`` and ``cu_seqlens_k`` must describe the same segments,
-    as they do at the reference's call site (``gpu_process_worker.py:265-276``).  ``max_seqlen_*`` are accepted
-    and not needed."""
+    as they do at the reference's call site (``gpu_process_worker.py:265-276``).  ``max_seqlen_q``, where it is a
+    plain int, tells how long the longest segment is: nothing but how a short batch is divided goes by it."""
     if dropout_p not in (0, 0.0):
         raise RuntimeError("fgrpo varlen attention: dropout is not supported (the reference passes 0.0)")
     if tuple(window_size) != (-1, -1) or softcap not in (0, 0.0) or alibi_slopes is not None or block_table is not None:
@@ -84,7 +90,7 @@ def flash_attn_varlen_func(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q=Non
         if cu_seqlens_q.shape != cu_seqlens_k.shape or not torch.equal(cu_seqlens_q, cu_seqlens_k):
             raise RuntimeError("fgrpo varlen attention: queries and keys must share their segments (self-attention)")
     bounds = _bounds_for(cu_seqlens_q, q.shape[0], bool(causal)) if q.is_cuda else None
-    return ops.varlen_attention(q, k, v, cu_seqlens_q, softmax_scale, bool(causal), bounds)
+    return ops.varlen_attention(q, k, v, cu_seqlens_q, softmax_scale, bool(causal), bounds, _plain_length(max_seqlen_q))
 
 
 def varlen_attention_forward(module, query: torch.Tensor, key: torch.Tensor, value: torch.Tensor,
@@ -109,8 +115,9 @@ def varlen_attention_forward(module, query: torch.Tensor, key: torch.Tensor, val
     if is_causal is None:
         is_causal = bool(getattr(module, "is_causal", True))
     if position_ids is not None:
-        cu, _ = prepare_from_position_ids(position_ids)
+        cu, longest = prepare_from_position_ids(position_ids)
     else:
+        longest = L
         cu = torch.arange(0, (B + 1) * L, L, dtype=torch.int32, device=query.device)
     # [B, H, L, D] -> packed [B*L, H, D]; for B == 1 this is a view the kernels read in place
     q = query.transpose(1, 2).reshape(B * L, Hq, D)
@@ -121,7 +128,7 @@ def varlen_attention_forward(module, query: torch.Tensor, key: torch.Tensor, val
         q, k, v = q.to(torch.bfloat16), k.to(torch.bfloat16), v.to(torch.bfloat16)
     causal = bool(is_causal)
     bounds = _bounds_for(cu, B * L, causal) if position_ids is not None and q.is_cuda else None
-    out = ops.varlen_attention(q, k, v, cu, scaling, causal, bounds)
+    out = ops.varlen_attention(q, k, v, cu, scaling, causal, bounds, longest)
     return out.view(B, L, Hq, D).to(dt), None
 
 

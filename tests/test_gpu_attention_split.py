@@ -106,6 +106,25 @@ def test_tiles_dealt_by_their_steps_agree_with_whole_ones(dev, T, lens, Hq, Hkv,
         assert (x.float() - y.float()).norm() <= 2 ** -7 * y.float().norm(), name
 
 
+@pytest.mark.parametrize("longest", [1694, 1, 10 ** 9, 0, -5, None, 1694.0, torch.tensor(1694)])
+def test_the_longest_segment_a_caller_names_decides_no_result(dev, longest):
+    """True, wrong, out of range or of another type: bounds as in test_divided_tiles_agree_with_whole_ones."""
+    from fgrpo import _lib, ops
+    from varlen_attention import flash_attn_varlen_func
+    lens, Hq, Hkv, D = [1694, 400] + [300] * 13, 16, 4, 128
+    T = sum(lens)
+    need = lambda n: _lib.load().fgrpo_varlen_attn_workspace_len(T, len(lens), n, Hq, Hkv, D, 1, 0)
+    assert need(1694) > 0 and need(0) == 0 == need(1) and need(10 ** 9) == need(T)
+    q, k, v, do = operands(T, Hq, Hkv, D, dev)
+    cu = torch.tensor([0] + torch.tensor(lens).cumsum(0).tolist(), dtype=torch.int32, device=dev)
+    out, lse = ops.varlen_attn_fwd(q, k, v, cu, None, True)
+    want = (out, *ops.varlen_attn_bwd(do, q, k, v, out, lse, cu, None, True))
+    a = [x.clone().requires_grad_(True) for x in (q, k, v)]
+    o = flash_attn_varlen_func(*a, cu, cu, longest, longest, causal=True)
+    for name, x, y in zip(("out", "dq", "dk", "dv"), (o.detach(), *torch.autograd.grad(o, a, do)), want):
+        assert (x.float() - y.float()).norm() <= 2 ** -7 * y.float().norm(), name
+
+
 def test_workspace_is_checked(dev):
     from fgrpo import _lib
     lib = _lib.load()
