@@ -123,7 +123,9 @@ SplitPlan plan_uneven(long long wgs, int blocks, int per_cu, double chain, doubl
   const double cus = num_cus(), slots = cus * per_cu, load = sum / slots;
   auto shared = [&](double n) { return shared_step(step, per_cu, n); };
   auto most = [](double a, double b) { return a > b ? a : b; };
-  const double whole = most((chain + open) * shared((double)wgs), (sum + wgs * open) / slots * shared(2.0 * slots));
+  // more tiles than CUs, one a CU: 1.15 to 1.25 of what the longest tile or the load comes to, for the order by shader engine
+  // (dK/dV of 6000 tokens in 12 segments, 28 / 4 heads 99 us, of 9000 in 14 173; both dealt out, with dQ, 154 -> 139 and 270 -> 267)
+  const double whole = most((chain + open) * shared((double)wgs), (sum + wgs * open) / slots * shared(2.0 * slots)) * (per_cu == 1 && wgs > slots ? 1.15 : 1.0);
   const double sums = bytes_a_part * 2.0 / 3.0e6, even = worth * sqrt(sum * sums / step), least = floor(most(even < at_most ? even : at_most, 1.5) + 0.5);
   const double cap = most(least, chain / kAttnMaxParts);
   auto parts = [&](double per) { return per < chain ? sum / per + 0.5 * wgs : (double)wgs; };
