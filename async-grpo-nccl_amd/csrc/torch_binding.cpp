@@ -523,5 +523,6 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   // without the interpreter lock: a call may wait, for memory or for room in a full launch queue, and other threads run
   m.def("shift_labels", &shift_labels, py::call_guard<py::gil_scoped_release>());
   m.def("fused_step", &fused_step, py::call_guard<py::gil_scoped_release>());
-  m.def("varlen_attention", &varlen_attention, py::call_guard<py::gil_scoped_release>());
+  m.def("varlen_attention", &varlen_attention, py::arg("q"), py::arg("k"), py::arg("v"), py::arg("cu"), py::arg("scale"), py::arg("causal"),
+        py::arg("bounds"), py::arg("max_len") = 0, py::call_guard<py::gil_scoped_release>());
 }
