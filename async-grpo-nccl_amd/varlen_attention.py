@@ -128,7 +128,7 @@ def varlen_attention_forward(module, query: torch.Tensor, key: torch.Tensor, val
         q, k, v = q.to(torch.bfloat16), k.to(torch.bfloat16), v.to(torch.bfloat16)
     causal = bool(is_causal)
     bounds = _bounds_for(cu, B * L, causal) if position_ids is not None and q.is_cuda else None
-    out = ops.varlen_attention(q, k, v, cu, scaling, causal, bounds, longest)
+    out = ops.varlen_attention(q, k, v, cu, scaling, causal, bounds, _plain_length(longest))
     return out.view(B, L, Hq, D).to(dt), None
 
 
