@@ -37,6 +37,7 @@
 // Launch order: work-groups start in the order of a device-built list, tiles with the most steps first (a third of
 // a launch was tail before), and in the query-side kernels the query heads of one K/V group share an XCD.
 #pragma once
+#include "attn_plan.h"
 #include "lmhead_kernels.h"
 
 namespace fgrpo {
@@ -79,7 +80,6 @@ struct AttnParams {
   int2* key_info;        // [key tile][Hkv] parts of the tile, work-group of the first
 };
 
-constexpr int kAttnMaxParts = 8;      // parts of a tile at most
 constexpr int kAttnMergeWide = 4;     // parts whose sums are fetched together
 constexpr int kAttnDealSlots = 256;   // tiles an XCD can deal out
 // A tile that walks `steps` steps, all its work-group's own chain, may be dealt to several work-groups (parts): each walks
@@ -2051,10 +2051,9 @@ __device__ __forceinline__ void attn_merge_query_tile(const AttnParams& p, int R
   const int t0 = idx / p.Hq * 32, hq = idx % p.Hq, n = threadIdx.x % 32, i0 = threadIdx.x / 32;
   const int G = p.Hq / p.Hkv, HB = 128 / RB, NB = (G + HB - 1) / HB, head = hq % G;
   const int2 info = p.query_info[t0 / RB * p.Hkv + hq / G];
-  const int np = min(info.x, kAttnMaxParts);
-  if (np <= 1) return;
-  // the parts' work-groups: 8 NB apart, those of the next HB heads 8 on.  Clamped: an order list of the caller's may leave a tile out
-  const int most = p.blocks_q + 8 * p.extra_q - 1 - 8 * ((np - 1) * NB + head / HB), first = min(max(info.y, 0), most) + 8 * (head / HB);
+  const int np = info.x, skip = 8 * (head / HB);           // the parts' work-groups: 8 NB apart, those of the next HB heads 8 on
+  if (!attn_parts_inside(np, info.y, skip, 8 * NB, p.blocks_q + 8 * p.extra_q)) return;
+  const int first = info.y + skip;
   const int wave = head % HB * (RB / 32) + t0 % RB / 32, t = min(t0 + n, p.T - 1);
   float x[NC][8];
 #pragma unroll

@@ -673,13 +673,12 @@ static __global__ __launch_bounds__(256) void attn_merge_bwd_kernel(AttnParams p
   const long long row = idx / (HD / 8);                        // key * Hkv + head
   const int kk = (int)(row / p.Hkv), head = (int)(row % p.Hkv);
   const int2 info = p.key_info[kk / kKeys * p.Hkv + head];
-  const int np = min(info.x, kAttnMaxParts);                   // parts, the work-group of the first (the others' 8 apart)
-  if (np <= 1) return;
+  const int np = info.x, first = info.y;                       // parts, the work-group of the first (the others' 8 apart)
+  if (!attn_parts_inside(np, first, 0, 8, p.blocks_k + 8 * p.extra_k)) return;
   float x[8];
 #pragma unroll
   for (int e = 0; e < 8; ++e) x[e] = 0.f;
   constexpr int slice = 2 * kKeys * HD;
-  const int most = p.blocks_k + 8 * p.extra_k - 1 - 8 * (np - 1), first = min(max(info.y, 0), most);      // clamped: an order list of the caller's may leave a tile out
   const float* src = p.part_k + (long long)first * slice + (which * kKeys + kk % kKeys) * HD + col;
 #pragma unroll
   for (int j0 = 0; j0 < kAttnMaxParts; j0 += kAttnMergeWide) {
