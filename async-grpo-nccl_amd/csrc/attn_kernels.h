@@ -44,8 +44,6 @@ namespace fgrpo {
 
 // Every kernel is a template on the head dimension HD (128 or 64): LDS rows of 2*HD bytes in HD/8 16-byte chunks,
 // HD/16 MFMA k-steps per score, HD/32 output blocks of 32 columns.
-constexpr int kAttnBQ = 128;         // tokens per work-group (32 per wavefront)
-constexpr int kAttnBK = 64;          // tokens of the other side per step
 
 struct AttnParams {
   const bf16_t* q;       // [T][Hq][HD] with element strides q_st (token), q_sh (head)
@@ -68,7 +66,7 @@ struct AttnParams {
   bf16_t* dq;            // [T][Hq][HD] contiguous
   bf16_t* dk;            // [T][Hkv][HD] contiguous
   bf16_t* dv;
-  // launches whose tiles are dealt to several work-groups (SPLIT kernels, see attn_parts); q: query side, k: key side
+  // launches whose tiles are dealt to several work-groups (SPLIT kernels, see attn_deal); q: query side, k: key side
   int parts_q, per_q, blocks_q;      // most parts of a tile, steps a part walks at least, work-groups of an undivided launch
   int extra_q, deal_q;               // work-groups beyond those, per XCD; work-groups of an XCD its steps are meant for
   int parts_k, per_k, blocks_k;      // the same; steps: items of a wavefront
@@ -81,13 +79,9 @@ struct AttnParams {
 };
 
 constexpr int kAttnMergeWide = 4;     // parts whose sums are fetched together
-constexpr int kAttnDealSlots = 256;   // tiles an XCD can deal out
-// A tile that walks `steps` steps, all its work-group's own chain, may be dealt to several work-groups (parts): each walks
-// its share and leaves fp32 sums, which a last launch adds up in a fixed order (no atomics: bit-reproducible).
 // n / d for 0 <= n < 2^21, d > 0: (n + 1/2) / d is at least 1 / (2 d) from a whole number, the error of product and reciprocal less.  An
 // integer division is some forty instructions, in series before a work-group's first load.
 __device__ __forceinline__ int small_div(int n, int d) { return (int)(((float)n + 0.5f) * __builtin_amdgcn_rcpf((float)d)); }
-__device__ __forceinline__ int attn_parts(int steps, int parts, int per) { return min(max(small_div(steps + per - 1, per), 1), parts); }
 // inclusive sum over the lanes up to this one: rows of 16, then rows 0 -> 1, 2 -> 3 and 1 -> 2, 3
 __device__ __forceinline__ int wave_sum_upto(int x) {
   x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false);      // row_shr 1, 2, 4, 8
@@ -98,6 +92,8 @@ __device__ __forceinline__ int wave_sum_upto(int x) {
   x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);      // row_bcast 31
   return x;
 }
+// A tile that walks `steps` steps, all its work-group's own chain, may be dealt to several work-groups (parts): each walks
+// its share and leaves fp32 sums, which a last launch adds up in a fixed order (no atomics: bit-reproducible).
 // Which part of which tile the work-group of number `at` in its XCD takes.  Lane l has the steps of the XCD's tiles l, l + 64,
 // .. (negative: no tile); every work-group reads them and adds them up by itself.  A part is to walk `per` steps, the XCD's
 // steps over the `deal` work-groups meant for them (`least` at least), or more until the parts fit the work-groups there
@@ -117,24 +113,17 @@ template <int N>
 __device__ __forceinline__ AttnDeal attn_deal(const int (&steps)[N], int at, int slots, int width, int extra, int parts, int least, int deal) {
   const int lane = threadIdx.x & 63, budget = slots * width + extra;
   auto total = [](int x) { return __builtin_amdgcn_readlane(wave_sum_upto(x), 63); };
-  auto parts_at = [&](int i, int per) { return steps[i] < 0 ? 0 : attn_parts(steps[i], parts, per); };
+  auto parts_at = [&](int i, int per) { return steps[i] < 0 ? 0 : attn_parts(steps[i], parts, per, small_div); };
   int sum = 0;
 #pragma unroll
   for (int i = 0; i < N; ++i) sum += max(steps[i], 0);
   sum = total(sum) * width;
-  int per = least;
-  if (sum > per * deal) per = (sum + deal - 1) / deal;
-  if (sum > per * extra) {
-    const int sure = (sum + extra - 1) / extra;                // with it the parts fit: each tile rounds up by less than one
-    do {
-      int n = 0;
+  const int per = attn_part_steps(sum, budget, extra, least, deal, [&](int x) {
+    int n = 0;
 #pragma unroll
-      for (int i = 0; i < N; ++i) n += parts_at(i, per);
-      n = total(n) * width;
-      if (n <= budget) break;
-      per = min(max(per + 1, (int)((long long)per * n / budget)), sure);
-    } while (per < sure);
-  }
+    for (int i = 0; i < N; ++i) n += parts_at(i, x);
+    return total(n) * width;
+  });
   AttnDeal out{-1, 0, 1, 0};
   int base = 0;
 #pragma unroll

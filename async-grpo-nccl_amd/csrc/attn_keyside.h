@@ -45,7 +45,6 @@
 
 namespace fgrpo {
 
-constexpr int kDkv3Rows = 32;                                          // queries of an item
 template <int HD>
 constexpr int kDkv3Buf = 2 * kDkv3Rows * HD * 2 + 512;                 // Q | dO | lse | -delta of 32 queries
 template <int HD>
@@ -112,33 +111,6 @@ __device__ __forceinline__ void dkv3_acc_to_lds(uint32_t addr) {       // LDS in
 // Items of a key tile: 32-query blocks from q_begin on x query heads of the group
 __device__ __forceinline__ int attn_key_items(int q_begin, int q_end, int G) {
   return q_end > q_begin ? (q_end - q_begin + kDkv3Rows - 1) / kDkv3Rows * G : 0;
-}
-
-// Which 128-key tile, K/V head and piece (of kPer128 a tile is dealt in) work-group `bid` takes.  Work-groups go to the 8
-// XCDs round-robin (work-group b runs on XCD b % 8, each with its own L2).  All pieces of a tile and head run on one XCD, one
-// behind the other: they read the same Q and dO rows; and where the K/V heads divide eight, an XCD stays with one head.
-// The units (tile, head) that no longer go round the eight are dealt to all of them piece by piece.
-// With the pieces of a tile on several XCDs each row came through several L2s; dQ + dK/dV, before -> after: 32768 tokens
-// in segments of 128..512, 14 / 2 heads of 64 181 -> 148 us; 36000 in 128..2048, 16 / 4 heads of 128 654 -> 639; 9000 in
-// 128..1024, 28 / 4 heads 216.5 -> 213.7; 4 x 8192, 28 / 4 heads 5.70 -> 5.50 ms; 32 / 8 heads of 64 unchanged (the
-// same order as before).  Runs of neighbouring tiles on one XCD (256 .. 4096 tokens) were no better, and worse where they
-// disturbed the order by work; so were XCDs taken in alternating direction, which mixes the heads.
-struct KeyPick {
-  int rank, head, piece;       // rank: place in the launch order; negative: no work
-};
-__host__ __device__ inline KeyPick attn_key_pick(int bid, int ntile, int pieces, int Hkv) {
-  const int xcd = bid & 7, slot = bid >> 3, units = ntile * Hkv, rounds = units / 8;
-  int u = slot / pieces * 8 + xcd, piece = slot % pieces;
-  if (slot >= rounds * pieces) {
-    const int i = (slot - rounds * pieces) * 8 + xcd;
-    u = rounds * 8 + i / pieces, piece = i % pieces;
-    if (u >= units) return KeyPick{-1, 0, 0};
-  }
-  return KeyPick{u / Hkv, u % Hkv, piece};
-}
-inline long long attn_key_blocks(long long ntile, int pieces, int Hkv) {      // work-groups of a launch (or of one share): whole rows of eight
-  const long long units = ntile * Hkv, rounds = units / 8;
-  return 8 * (rounds * pieces + ((units - 8 * rounds) * pieces + 7) / 8);
 }
 
 // What a work-group walks: queries [q_begin, q_end) for the keys of `tile`

@@ -5,9 +5,6 @@
 
 namespace fgrpo {
 
-int attn_keyside_keys(int D) { return D == 128 ? 64 : 32; }
-int attn_keyside_blocks(int D, int T, int Hkv) { return (int)attn_key_blocks((T + 127) / 128, 128 / attn_keyside_keys(D), Hkv); }      // every 128-key tile, in pieces
-
 template <int HD, int KB>
 static int launch(const AttnParams& p, hipStream_t st) {
   AttnParams a = p;
