@@ -94,6 +94,9 @@ int launch(int cus, int heads, int which, const int* cu, int n, int max_len, int
   return 0;
 }
 
+int divided(int which, int T, int n, int max_len, int Hq, int Hkv, int D) {
+  return (which == 2 ? plan_key_split(256, 0, T, n, max_len, Hq, Hkv, D, 1) : plan_query_split(256, 0, 0, T, n, max_len, Hq, Hkv, D, 1, which == 0, 0)).parts > 1;
+}
 int heads(int wanted, int G, int T, int n) { return attn_heads_per_group(wanted, G, T, n); }
 
 // n / d by reciprocal, with the reciprocal one unit in the last place off either way
@@ -178,3 +181,13 @@ def test_every_tile_gets_its_parts_and_no_launch_more_than_it_has(plan, which, c
         assert rc <= 0, (rc, which, T, n, length, G * Hkv, Hkv, D, causal, heads)
         divided += rc == 0
     assert divided > 200
+
+
+@pytest.mark.parametrize("T,n,longest,Hq,Hkv,D,divided", [
+    (7359, 1, 7359, 28, 4, 128, False), (15330, 1, 15330, 12, 2, 128, False), (32768, 1, 32768, 4, 1, 128, False),
+    (28241, 14, 7263, 14, 2, 64, False), (32768, 30, 5808, 14, 2, 64, False), (12345, 22, 1821, 28, 4, 128, False),
+    (777, 1, 777, 12, 2, 128, True), (5000, 1, 5000, 28, 4, 128, True), (6000, 13, 1694, 16, 4, 128, True),
+    (9000, 14, 2048, 12, 2, 128, True), (2000, 1, 2000, 14, 2, 64, True)])
+def test_tiles_of_many_rounds_stay_whole_on_the_key_side(plan, T, n, longest, Hq, Hkv, D, divided):
+    """Whole, these were 3 to 9 % faster than dealt out, or slower where the launch is divided."""
+    assert bool(plan.divided(2, T, n, longest, Hq, Hkv, D)) == divided
