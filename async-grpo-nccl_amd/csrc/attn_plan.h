@@ -11,7 +11,7 @@ constexpr int kAttnBK = 64;           // tokens of the other side per step
 constexpr int kDkv3Rows = 32;         // queries of an item of the dK/dV kernel
 constexpr int kAttnMaxParts = 8;      // parts of a tile at most
 constexpr int kAttnDealSlots = 256;   // tiles an XCD can deal out
-constexpr size_t kAttnSplitMaxBytes = 256u << 20;
+constexpr size_t kAttnSplitMaxBytes = 256u << 20;      // partial sums of a launch at most: a backward has two, and tables beside them
 
 // Query heads per work-group of the query-side kernels (tile = 128 / heads tokens).  Short segments gain from short
 // tiles (less masked work on the diagonal and at segment boundaries) as long as the heads of a group fill the

@@ -97,6 +97,10 @@ int launch(int cus, int heads, int which, const int* cu, int n, int max_len, int
 int divided(int which, int T, int n, int max_len, int Hq, int Hkv, int D) {
   return (which == 2 ? plan_key_split(256, 0, T, n, max_len, Hq, Hkv, D, 1) : plan_query_split(256, 0, 0, T, n, max_len, Hq, Hkv, D, 1, which == 0, 0)).parts > 1;
 }
+unsigned long long sums(int which, int T, int n, int max_len, int Hq, int Hkv, int D, int causal) {
+  const SplitPlan s = which == 2 ? plan_key_split(256, 0, T, n, max_len, Hq, Hkv, D, causal) : plan_query_split(256, 0, 0, T, n, max_len, Hq, Hkv, D, causal, which == 0, 1);
+  return s.parts <= 1 ? 0 : which == 2 ? key_sums_bytes(s, D) : query_sums_bytes(s, D);
+}
 int heads(int wanted, int G, int T, int n) { return attn_heads_per_group(wanted, G, T, n); }
 
 // n / d by reciprocal, with the reciprocal one unit in the last place off either way
@@ -117,7 +121,9 @@ def plan(tmp_path_factory):
     with open(src, "w") as f:
         f.write(SOURCE)
     subprocess.run([os.environ.get("CXX", "g++"), "-std=c++17", "-O1", "-fPIC", "-shared", f"-I{CSRC}", src, "-o", lib], check=True)
-    return C.CDLL(lib)
+    lib = C.CDLL(lib)
+    lib.sums.restype = C.c_ulonglong
+    return lib
 
 
 def test_merges_follow_no_entry_out_of_the_launch(plan):
@@ -191,3 +197,18 @@ def test_every_tile_gets_its_parts_and_no_launch_more_than_it_has(plan, which, c
 def test_tiles_of_many_rounds_stay_whole_on_the_key_side(plan, T, n, longest, Hq, Hkv, D, divided):
     """Whole, these were 3 to 9 % faster than dealt out, or slower where the launch is divided."""
     assert bool(plan.divided(2, T, n, longest, Hq, Hkv, D)) == divided
+
+
+@pytest.mark.parametrize("causal", [0, 1])
+def test_partial_sums_of_a_launch_stay_within_256_mib(plan, causal):
+    """As they are allocated, by whole work-groups: the heads of a group that do not fill one (5 as 8) count.  A backward has two such
+    launches, and small tables beside the sums."""
+    rng = random.Random(7 + causal)
+    most = 0
+    for _ in range(60000):
+        T, Hkv, G = int(2 ** rng.uniform(8, 17)), rng.choice((1, 2, 3, 4, 8)), rng.choice((1, 2, 3, 5, 6, 7, 9, 13))
+        n, D, which = rng.choice((1, 1, 2, 3, 4, 8)), rng.choice((64, 128)), rng.randrange(3)
+        b = plan.sums(which, T, n, rng.choice((0, T, -(-T // n))), G * Hkv, Hkv, D, causal)
+        assert b <= 256 << 20, (which, T, n, G * Hkv, Hkv, D)
+        most = max(most, b)
+    assert most > (200 if causal else 80) << 20
