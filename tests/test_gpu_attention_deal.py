@@ -41,3 +41,50 @@ def test_an_order_list_that_leaves_tiles_out_reads_nothing_from_outside_the_work
     torch.cuda.synchronize()
     for x in (dq, dk, dv):
         assert (x[128:] == 77.0).all() and (x[:32] != 77.0).any()
+
+
+def launches(T, n_seq, longest, Hq, Hkv, D, causal):
+    """Which launches of a call deal their tiles out, as the call plans them: those that ask for scratch, dQ for what is left of the
+    backward's when a kernel that cannot is put in its place."""
+    from fgrpo import _lib
+    need = lambda backward: _lib.load().fgrpo_varlen_attn_workspace_len(T, n_seq, longest, Hq, Hkv, D, causal, backward)
+    found, both = "f" if need(0) else "", need(1)
+    try:
+        _lib.set_tuning(attn_qside=3)
+        keys = need(1)
+    finally:
+        _lib.set_tuning(attn_qside=0)
+    return found + ("q" if both > keys else "") + ("k" if keys else "")
+
+
+# segment lengths, query heads, K/V heads, head dimension, mask, which launches (f: forward, q: dQ, k: dK/dV) are dealt out; 1, 2 and 4
+# heads a work-group and one to five work-groups a group, all parts in flight or more than the device holds
+DEALT = [
+    ([1216, 84], 16, 4, 128, True, "fqk"), ([1500, 300, 40, 560, 200], 12, 2, 128, True, "fqk"), ([1500, 300, 40, 560, 200], 15, 3, 64, True, "fqk"),
+    ([1694] + [400] * 10 + [100, 206], 16, 4, 128, True, "fqk"), ([1500, 300, 40, 560, 200], 28, 4, 128, True, "qk"), ([9000], 5, 1, 128, True, "fqk"),
+    ([300, 4000, 1700, 1000, 1900, 100], 6, 3, 128, True, "fq"), ([8200, 3000, 100, 1700, 3000], 8, 8, 64, True, "fq"),
+    ([1, 1700, 1299, 400, 500, 100], 12, 6, 128, True, "fq"), ([12000, 8000], 3, 1, 128, True, "fqk"),
+    ([700], 5, 1, 128, False, "fqk"), ([1216, 84], 3, 1, 128, False, "fqk"), ([9000], 3, 1, 128, False, "fqk"), ([700], 4, 4, 128, False, "fq"),
+    ([1500, 300, 700, 1500], 2, 1, 128, False, "fq"), ([10, 2900, 40, 3000, 2050], 1, 1, 64, False, "fq"), ([300, 4000, 1700, 1000, 1900, 100], 5, 1, 128, False, "k"),
+    ([1500, 300, 40, 560, 200], 12, 2, 128, False, "k")]
+
+
+@pytest.mark.parametrize("lens,Hq,Hkv,D,causal,sides", DEALT)
+def test_the_launches_meant_are_dealt_out_and_agree_with_whole_ones(dev, lens, Hq, Hkv, D, causal, sides):
+    """With the longest segment named.  Two roundings to bf16 (probabilities, result) of 2^-9 at most on either side: 2^-7 of the
+    norm between them."""
+    from fgrpo import ops
+    T = sum(lens)
+    assert launches(T, len(lens), max(lens), Hq, Hkv, D, causal) == sides
+    q, k, v, do = operands(T, Hq, Hkv, D, dev)
+    cu = torch.tensor([0] + torch.tensor(lens).cumsum(0).tolist(), dtype=torch.int32, device=dev)
+    out, lse = ops.varlen_attn_fwd(q, k, v, cu, None, causal)
+    want = (out, *ops.varlen_attn_bwd(do, q, k, v, out, lse, cu, None, causal))
+
+    def once():
+        a = [x.clone().requires_grad_(True) for x in (q, k, v)]
+        o = ops.varlen_attention(*a, cu, None, causal, None, max(lens))
+        return (o.detach(),) + torch.autograd.grad(o, a, do)
+    for name, x, y, z in zip(("out", "dq", "dk", "dv"), once(), want, once()):
+        assert torch.equal(x, z), f"{name} is not reproducible"
+        assert (x.float() - y.float()).norm() <= 2 ** -7 * y.float().norm(), name
