@@ -16,8 +16,20 @@ import numpy as np
 import torch
 
 from fgrpo import ops
-from grpo_loss import dual_clip_grpo_loss_begin, make_grpo_forward
+from grpo_loss import compute_dual_clip_grpo_loss, dual_clip_grpo_loss_begin, make_grpo_forward
 from sample_processing_utils import PackedLogProbs, _fill, post_process_batch
+
+
+_PACKAGE_LOSS = compute_dual_clip_grpo_loss
+
+
+def _begin_loss(*args, **kwargs):
+    """``dual_clip_grpo_loss_begin``, unless a program has put a loss of its own in this module's place of
+    ``compute_dual_clip_grpo_loss``: that one is called, metrics and all."""
+    if compute_dual_clip_grpo_loss is _PACKAGE_LOSS:
+        return dual_clip_grpo_loss_begin(*args, **kwargs)
+    loss, metrics = compute_dual_clip_grpo_loss(*args, **kwargs)
+    return loss, lambda: metrics
 
 
 def prepare_actor_module(model, config=None, mode: str = "training", use_varlen_attention: bool = True):
@@ -57,7 +69,7 @@ class TrainerHarness:
             return {"loss": 0.0, "pg_clip": 0, "kl_div": 0.0, "entropy": 0.0}
         cfg = self.config
         with torch.autocast(device_type="cuda", dtype=torch.bfloat16):
-            loss, read_metrics = dual_clip_grpo_loss_begin(
+            loss, read_metrics = _begin_loss(
                 self.actor_module_fsdp, batch, cfg.clip_low, cfg.clip_high, cfg.clip_ratio_c,
                 compute_entropy=bool(getattr(cfg, "compute_entropy", True)),
                 apply_entropy_bonus=bool(getattr(cfg, "apply_entropy_bonus", True)),

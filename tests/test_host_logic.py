@@ -1,6 +1,8 @@
 """Host-side logic that needs no GPU: numpy forms of the batch-shaping helpers
 against the oracle, synthetic workload generators, and the refusal of CPU
 tensors by the product path."""
+import warnings
+
 import numpy as np
 import pytest
 import torch
@@ -405,3 +407,35 @@ def test_shares_of_a_narrow_last_token_tile(H, T, narrow):
     shares = -(-594 // int(9 / narrow))
     want = up(16 * 66 * T) + up(16 * shares * (T % 256)) + up(4 * T) + up(4 * V)
     assert _lib.load().fgrpo_logprob_fwd_workspace(T, H, V, _lib.BF16) == want
+
+
+@pytest.mark.parametrize("replaced", [False, True])
+def test_the_trainer_calls_the_loss_its_module_names(monkeypatch, replaced):
+    """``workers.compute_dual_clip_grpo_loss`` is the loss of ``grpo_loss``, and what a program puts in its place is what the
+    trainer calls; otherwise the metrics are read behind the backward."""
+    import grpo_loss
+    import workers
+    assert workers.compute_dual_clip_grpo_loss is grpo_loss.compute_dual_clip_grpo_loss
+    seen, x = [], torch.ones(3, requires_grad=True)
+    batch = {"_num_output_tokens_non_masked_host": 3.0}
+    monkeypatch.setattr(workers, "post_process_batch", lambda samples, device: batch)
+
+    def loss_of(model, minibatch, clip_low, clip_high, clip_ratio_c, **kw):
+        assert minibatch is batch and (clip_low, clip_high, clip_ratio_c) == (0.2, 0.28, 3.0)
+        assert kw == dict(compute_entropy=True, apply_entropy_bonus=True, entropy_coeff=0.0)
+        seen.append("loss")
+        return (x * x).sum()
+
+    def read():
+        seen.append("metrics behind" if x.grad is not None else "metrics before")
+        return {"loss": 3.0}
+    if replaced:
+        monkeypatch.setattr(workers, "compute_dual_clip_grpo_loss", lambda *a, **kw: (loss_of(*a, **kw), read()))
+    else:
+        monkeypatch.setattr(workers, "dual_clip_grpo_loss_begin", lambda *a, **kw: (loss_of(*a, **kw), read))
+    harness = workers.TrainerHarness(torch.nn.Linear(1, 1), device="cpu")
+    with warnings.catch_warnings():
+        warnings.simplefilter("ignore")                       # autocast for a device that is not there
+        assert harness.compute_gradients([{}]) == {"loss": 3.0}
+    assert seen == ["loss", "metrics before" if replaced else "metrics behind"]
+    assert torch.equal(x.grad, 2 * x.detach())
