@@ -98,7 +98,8 @@ constexpr bool attn_parts_inside(int np, int first, int skip, int stride, int gr
 // sharing a chain costs fp32 sums through memory and mostly one more launch.  Both sides are estimated, in us, from what was
 // measured: `step` for a step of a work-group alone on its CU, half as much again where two share one, `open` steps to
 // open and close a work-group.  Decided by shapes and the length that the caller gives for the longest segment; where it
-// gives none, that of four or more is taken to be 1.75 means long (lengths spread evenly).  A wrong length costs time, nothing else.
+// gives none, that of four or more is taken to be 1.75 means long (lengths spread evenly).  A wrong length costs time, and
+// another division means another order of the fp32 sums: the results are as good, not the same bits.
 // Guessed | told, forward and backward, us: 6000 tokens in 13 segments, one of 1694, 16 / 4 heads 47.1, 148 | 39.7, 115; 1500 in 2,
 // one of 997, 14 / 2 heads of 64 20.1, 33.1 | 16.2, 32.8; 2000 in 3, one of 970, 12 / 2 heads 27.1, 57.5 | 23.3, 53.5.  Whole | dealt out, merge launch included, 12 / 2 heads of 128: one segment of 777
 // tokens, forward 22.5 | 16.5 us, backward 77.8 | 36.7; of 2000 50.0 | 31.8 and 147 | 74.

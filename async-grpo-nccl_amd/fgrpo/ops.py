@@ -1123,7 +1123,8 @@ class _VarlenAttention(torch.autograd.Function):
 def varlen_attention(q, k, v, cu_seqlens, softmax_scale=None, causal=True, bounds=None, max_len: int = 0) -> torch.Tensor:
     """Differentiable packed self-attention on the HIP kernels (bf16 in, bf16 out).  ``bounds``: segment scratch of an
     earlier call with the same ``cu_seqlens`` and ``causal`` (see ``attention_bounds``).  ``max_len``: length of the longest
-    segment, 0 where it is not known; a short batch is divided better with it, and a wrong one costs time, nothing else."""
+    segment, 0 where it is not known; a short batch is divided better with it.  Results do not depend on it but for the order
+    of fp32 sums (other lengths: other bits, apart by up to 1e-3 of the norm); a wrong one costs time."""
     if torch.jit.is_tracing():
         return _VarlenAttention.apply(q, k, v, cu_seqlens, softmax_scale, bool(causal), bounds)
     return _lib.native().varlen_attention(q, k, v, cu_seqlens, softmax_scale, bool(causal), bounds, max_len)

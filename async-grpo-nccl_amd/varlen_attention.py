@@ -79,7 +79,9 @@ def flash_attn_varlen_func(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q=Non
     """``q`` [total, Hq, D], ``k`` / ``v`` [total, Hkv, D] bf16 -> out [total, Hq, D] bf16 (differentiable).
     Self-attention over packed segments: ``cu_seqlens_q`` and ``cu_seqlens_k`` must describe the same segments,
     as they do at the reference's call site (``gpu_process_worker.py:265-276``).  ``max_seqlen_q``, where it is a
-    plain int, tells how long the longest segment is: nothing but how a short batch is divided goes by it."""
+    plain int, tells how long the longest segment is.  How a short batch is divided goes by it, and with that the order of
+    its fp32 sums: a wrong length gives results as good as the right one's, but not the same bits (apart by up to 1e-3 of
+    the norm in bf16), and takes longer."""
     if dropout_p not in (0, 0.0):
         raise RuntimeError("fgrpo varlen attention: dropout is not supported (the reference passes 0.0)")
     if tuple(window_size) != (-1, -1) or softcap not in (0, 0.0) or alibi_slopes is not None or block_table is not None:

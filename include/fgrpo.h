@@ -354,8 +354,9 @@ int fgrpo_varlen_attn_fwd_ws(const void* q, const void* k, const void* v, long l
                              const int32_t* cu_seqlens, int n_seq, int T, int Hq, int Hkv, int D, float softmax_scale,
                              int causal, void* out, float* lse, int32_t* bounds_ws, int bounds_valid, void* ws,
                              size_t ws_bytes, void* stream);
-/* The same again, told the length of the longest segment (0: not known).  How tiles are dealt out goes by it; a wrong one costs
- * time, nothing else.  A workspace is asked for and used with the same length. */
+/* The same again, told the length of the longest segment (0: not known).  How tiles are dealt out goes by it, and with
+ * that the order of the fp32 sums: under another length results are as good but not the same bits, and a wrong one costs time.  A
+ * workspace is asked for and used with the same length. */
 size_t fgrpo_varlen_attn_workspace_len(int T, int n_seq, int max_len, int Hq, int Hkv, int D, int causal, int backward);
 int fgrpo_varlen_attn_fwd_len(const void* q, const void* k, const void* v, long long q_stride_t, long long q_stride_h,
                              long long k_stride_t, long long k_stride_h, long long v_stride_t, long long v_stride_h,
