@@ -145,10 +145,12 @@ inline SplitPlan plan_even(int cus, long long wgs, int blocks, int per_cu, doubl
 // 2 .. 12 steps).  dK/dV whole | dealt out, dQ and
 // merge included: 6000 tokens in 13 segments, 16 / 4 heads 150 | 123; 4000 in 6, 28 / 4 heads 124 | 115; 5000 in one, 28 / 4
 // heads 645 | 609; 12345 in 23, 14 / 2 heads of 64 87 | 94 and 4000 in 5, 32 / 8 heads of 64 83 | 96, both refused.
-// The more rounds the tiles make on the device, the better they even out by themselves, which the whole launch's estimate does not see: it
-// is trusted `rounds` less for each round after the first (key side; the query side's estimate holds).  dQ + dK/dV whole | dealt
-// out: one segment of 7359, 28 / 4 heads 1183 | 1272, of 15330, 12 / 2 heads 2107 | 2288; 28241 in 14, 14 / 2 heads of 64 721 | 790.  Of 4820
-// random divided calls 133 backward passes took over 3 % longer than with tiles dealt out by a mean segment, 45 do with this.
+// A launch of more than one round of tiles ends with its longest tile or with its load, and dealing out takes off only what that tile
+// walks beyond the load; the more rounds, the less of it the tiles in their order leave.  So the longest has to be 1 + `rounds` times the
+// rounds as long as the load (key side; on the query side the estimate holds).  dQ + dK/dV whole | dealt out: one segment of 7359 tokens,
+// 28 / 4 heads 1183 | 1272, of 15330, 12 / 2 heads 2107 | 2288; 28241 in 14, 14 / 2 heads of 64 721 | 790, all three 1.1 to 1.3 times.  Over 2177
+// launches of one to three rounds dealing out was worth it from 1.5 times the load on at 1.75 rounds, 1.75 at 3 (head dimension 64: 1.75 and 2.3);
+// by this line they take 0.6 % longer than with the better of both each, all whole 2.6 %, all dealt out 2.4.
 inline SplitPlan plan_uneven(int cus, long long wgs, int blocks, int per_cu, double chain, double sum, double longest, double step, double open, double bytes_a_part, double worth, double at_most, double merge, double rounds) {
   SplitPlan s;
   const double slots = (double)cus * per_cu, load = sum / slots;
@@ -168,8 +170,8 @@ inline SplitPlan plan_uneven(int cus, long long wgs, int blocks, int per_cu, dou
     const double x = most(most(sum / (r - 0.5 * wgs), chain * (2.0 - r / wgs)), cap), t = (x + open) * shared(parts(x));
     if (t < walk) walk = t, per = x, room = r;
   }
-  const double limit = room > 0.0 ? whole : whole * (1.0 - rounds * most(wgs / slots - 1.0, 0.0));
-  if (walk + merge + most(parts(per) - 0.5 * wgs, 0.0) * sums * 0.5 >= limit) return s;
+  if (walk + merge + most(parts(per) - 0.5 * wgs, 0.0) * sums * 0.5 >= whole) return s;
+  if (room == 0.0 && wgs > slots && chain < load * (1.0 + rounds * wgs / slots)) return s;
   s.per = (int)least;
   s.extra = room > 0.0 ? ((int)room - blocks) / 8 : (int)(load / per * slots / 8) + 1;
   s.deal = room > 0.0 ? ((int)room - blocks / 2) / 8 : s.extra;
@@ -220,7 +222,7 @@ inline SplitPlan plan_key_split(int cus, int form, int T, int n_seq, int max_len
   } else {
     const SegmentGuess g = guess_segments(T, n_seq, max_len);
     const double sum = wgs * (g.seen * 0.5 + 16 + (n_seq > 1 ? keys : 0)) * items;
-    s = plan_uneven(cus, wgs, blocks, per_cu, g.longest * items, sum, T * items, D == 128 ? 1.4 : 0.65, D == 128 ? 6.0 : 4.0, keys * D * 8.0, 1.0, 1e30, 4.0, 0.25);
+    s = plan_uneven(cus, wgs, blocks, per_cu, g.longest * items, sum, T * items, D == 128 ? 1.4 : 0.65, D == 128 ? 6.0 : 4.0, keys * D * 8.0, 1.0, 1e30, 4.0, D == 128 ? 0.25 : 0.45);
   }
   s.grid = blocks + 8 * s.extra;
   return s;

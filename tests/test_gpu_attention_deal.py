@@ -62,8 +62,8 @@ def launches(T, n_seq, longest, Hq, Hkv, D, causal):
 DEALT = [
     ([1216, 84], 16, 4, 128, True, "fqk"), ([1500, 300, 40, 560, 200], 12, 2, 128, True, "fqk"), ([1500, 300, 40, 560, 200], 15, 3, 64, True, "fqk"),
     ([1694] + [400] * 10 + [100, 206], 16, 4, 128, True, "fqk"), ([1500, 300, 40, 560, 200], 28, 4, 128, True, "qk"), ([9000], 5, 1, 128, True, "fqk"),
-    ([300, 4000, 1700, 1000, 1900, 100], 6, 3, 128, True, "fq"), ([8200, 3000, 100, 1700, 3000], 8, 8, 64, True, "fq"),
-    ([1, 1700, 1299, 400, 500, 100], 12, 6, 128, True, "fq"), ([12000, 8000], 3, 1, 128, True, "fqk"),
+    ([300, 4000, 1700, 1000, 1900, 100], 6, 3, 128, True, "fqk"), ([8200, 3000, 100, 1700, 3000], 8, 8, 64, True, "fq"),
+    ([1, 1700, 1299, 400, 500, 100], 12, 6, 128, True, "fqk"), ([12000, 8000], 3, 1, 128, True, "fqk"),
     ([700], 5, 1, 128, False, "fqk"), ([1216, 84], 3, 1, 128, False, "fqk"), ([9000], 3, 1, 128, False, "fqk"), ([700], 4, 4, 128, False, "fq"),
     ([1500, 300, 700, 1500], 2, 1, 128, False, "fq"), ([10, 2900, 40, 3000, 2050], 1, 1, 64, False, "fq"), ([300, 4000, 1700, 1000, 1900, 100], 5, 1, 128, False, "k"),
     ([1500, 300, 40, 560, 200], 12, 2, 128, False, "k")]
