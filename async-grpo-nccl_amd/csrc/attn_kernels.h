@@ -93,18 +93,19 @@ __device__ __forceinline__ int wave_sum_upto(int x) {
   return x;
 }
 // A tile that walks `steps` steps, all its work-group's own chain, may be dealt to several work-groups (parts): each walks
-// its share and leaves fp32 sums, which a last launch adds up in a fixed order (no atomics: bit-reproducible).
-// Which part of which tile the work-group of number `at` in its XCD takes.  Lane l has the steps of the XCD's tiles l, l + 64,
+// its share and leaves fp32 sums, which a last launch adds up in a fixed order (no atomics: bit-reproducible).  Here:
+// which part of which tile the work-group of number `at` in its XCD takes.  Lane l has the steps of the XCD's tiles l, l + 64,
 // .. (negative: no tile); every work-group reads them and adds them up by itself.  A part is to walk `per` steps, the XCD's
 // steps over the `deal` work-groups meant for them (`least` at least), or more until the parts fit the work-groups there
 // are, `slots` tiles of `width` work-groups each and `extra`.  The parts are numbered through in the order of the tiles,
 // longest first; the few work-groups that no part is left for end at once.
 // Dealt out by a mean segment's length instead, with work-groups for as many parts of every tile, a batch of several segments
 // had its longest tile to wait for, or more work-groups than the device holds, most of them empty (each takes a CU's
-// LDS to find out).  Forward | dQ, dK/dV and merge, us, before -> after, heads of 128 unless said: 3000 tokens in 4 segments, 12 / 2 heads
-// 48.6 | 122 -> 35.6 | 82.4; 1500 in 2 26.4 | 65.5 -> 21.1 | 44.4; 9000 in 14 48.0 | 189 -> 48.6 | 139; one of 2000 34.6 | 91.6 -> 31.8 | 74.1,
-// of 777 16.7 | 38.6 -> 16.5 | 36.7, of 300 11.4 | 28.4 -> 11.3 | 25.7; 2000 in 7, 28 / 4 heads 16.6 | 74.2 -> 16.7 | 53.5; 6000 in 12,
-// 14 / 2 heads of 64 21.9 | 70.6 -> 21.8 | 61.3.  What it costs a work-group, some 0.5 us before its first load, is why sums
+// LDS to find out).  Forward | dQ, dK/dV and merge, us, before -> after, heads of 128 unless said (the
+// vector work and partial sums of that time in it: of one segment of 777 that was most, of 3000 tokens a third): 3000 tokens in 4 segments, 12 / 2 heads 57.5 | 133 -> 36.3 | 85.9; 1500 in 2
+// 30.8 | 71.6 -> 21.8 | 45.4; 9000 in 14 54.5 | 197 -> 48.5 | 137; one of 2000 39.0 | 96.3 -> 32.5 | 75.0, of 777 19.4 | 41.8 -> 17.1 | 37.9,
+// of 300 12.3 | 30.1 -> 11.1 | 26.1; 2000 in 7, 28 / 4 heads 18.8 | 77.0 -> 17.0 | 53.9; 6000 in 12, 14 / 2 heads of 64 23.7 | 73.9 ->
+// 20.5 | 57.7.  What it costs a work-group, some 0.5 us before its first load, is why sums
 // and quotients are in as few instructions as they are (with integer divisions the forward of 777 tokens took 17.4 us).
 struct AttnDeal {
   int slot, share, np, sub;        // part `share` of the np of the XCD's tile `slot`, work-group `sub` of its width; slot < 0: no work

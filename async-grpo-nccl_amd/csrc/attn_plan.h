@@ -100,9 +100,12 @@ constexpr bool attn_parts_inside(int np, int first, int skip, int stride, int gr
 // open and close a work-group.  Decided by shapes and the length that the caller gives for the longest segment; where it
 // gives none, that of four or more is taken to be 1.75 means long (lengths spread evenly).  A wrong length costs time, and
 // another division means another order of the fp32 sums: the results are as good, not the same bits.
-// Guessed | told, forward and backward, us: 6000 tokens in 13 segments, one of 1694, 16 / 4 heads 47.1, 148 | 39.7, 115; 1500 in 2,
-// one of 997, 14 / 2 heads of 64 20.1, 33.1 | 16.2, 32.8; 2000 in 3, one of 970, 12 / 2 heads 27.1, 57.5 | 23.3, 53.5.  Whole | dealt out, merge launch included, 12 / 2 heads of 128: one segment of 777
-// tokens, forward 22.5 | 16.5 us, backward 77.8 | 36.7; of 2000 50.0 | 31.8 and 147 | 74.
+// Guessed | told, forward and backward, us: 6000 tokens in 13 segments, one of 1694, 16 / 4 heads 47.2, 149 | 40.7, 114; 1500 in 2,
+// one of 997, 14 / 2 heads of 64 20.3, 33.7 | 16.5, 33.2.  Where the guess is wrong because segments are equal it costs up to a fifth: forward of
+// 3052 tokens in five, 16 / 4 heads, 22.9 whole and 27.7 dealt out; a guess that spares these (the mean's estimate asked too) loses
+// more on uneven ones, up to 1.75 times.
+// Whole | dealt out, merge launch included, 12 / 2 heads of 128: one segment of 777 tokens, forward 22.6 | 17.1 us, backward 81.4 | 37.9; of 2000
+// 50.5 | 32.5 and 181 | 75.
 struct SplitPlan {
   int parts = 1, per = 1;                // most parts of a tile, steps a part walks at least
   int extra = 0, deal = 1;               // see AttnParams
@@ -143,11 +146,11 @@ inline SplitPlan plan_even(int cus, long long wgs, int blocks, int per_cu, doubl
 // on 256 CUs took 120 us where 250 took 100 (dK/dV of 3000 tokens in 4 segments, 12 / 2 heads of 128).  Sums are taken at 6 TB/s, most
 // of them leaving while others still walk; a part is no shorter than its own are worth at 3 (`worth` times, `at_most`: measured at
 // 2 .. 12 steps).  dK/dV whole | dealt out, dQ and
-// merge included: 6000 tokens in 13 segments, 16 / 4 heads 150 | 123; 4000 in 6, 28 / 4 heads 124 | 115; 5000 in one, 28 / 4
-// heads 645 | 609; 12345 in 23, 14 / 2 heads of 64 87 | 94 and 4000 in 5, 32 / 8 heads of 64 83 | 96, both refused.
+// merge included: 6000 tokens in 13 segments, 16 / 4 heads 149 | 114; 4000 in 6, 28 / 4 heads 139 | 119; 5000 in one, 28 / 4
+// heads 663 | 620; 12345 in 23, 14 / 2 heads of 64 87 | 94 and 4000 in 5, 32 / 8 heads of 64 83 | 96, both refused.
 // A launch of more than one round of tiles ends with its longest tile or with its load, and dealing out takes off only what that tile
-// walks beyond the load; the more rounds, the less of it the tiles in their order leave.  So the longest has to be 1 + `rounds` times the
-// rounds as long as the load (key side; on the query side the estimate holds).  dQ + dK/dV whole | dealt out: one segment of 7359 tokens,
+// walks beyond the load; the more rounds, the less of it the tiles in their order leave.  So the longest has to be
+// 1 + `rounds` * (rounds of tiles) times the load (key side; on the query side the estimate holds).  dQ + dK/dV whole | dealt out: one segment of 7359 tokens,
 // 28 / 4 heads 1183 | 1272, of 15330, 12 / 2 heads 2107 | 2288; 28241 in 14, 14 / 2 heads of 64 721 | 790, all three 1.1 to 1.3 times.  Over 2177
 // launches of one to three rounds dealing out was worth it from 1.5 times the load on at 1.75 rounds, 1.75 at 3 (head dimension 64: 1.75 and 2.3);
 // by this line they take 0.6 % longer than with the better of both each, all whole 2.6 %, all dealt out 2.4.
@@ -157,7 +160,7 @@ inline SplitPlan plan_uneven(int cus, long long wgs, int blocks, int per_cu, dou
   auto shared = [&](double n) { return shared_step(cus, step, per_cu, n); };
   auto most = [](double a, double b) { return a > b ? a : b; };
   // more tiles than CUs, one a CU: 1.15 to 1.25 of what the longest tile or the load comes to, for the order by shader engine
-  // (dK/dV of 6000 tokens in 12 segments, 28 / 4 heads 99 us, of 9000 in 14 173; both dealt out, with dQ, 154 -> 139 and 270 -> 267)
+  // (dK/dV of 6000 tokens in 12 segments, 28 / 4 heads 99 us, of 9000 in 14 173; both dealt out, with dQ, 152 -> 140 and 276 -> 270)
   const double whole = most((chain + open) * shared((double)wgs), (sum + wgs * open) / slots * shared(2.0 * slots)) * (per_cu == 1 && wgs > slots ? 1.15 : 1.0);
   const double sums = bytes_a_part * 2.0 / 3.0e6, even = worth * sqrt(sum * sums / step), least = floor(most(even < at_most ? even : at_most, 1.5) + 0.5);
   const double cap = most(least, chain / kAttnMaxParts);
