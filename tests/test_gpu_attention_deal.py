@@ -88,3 +88,35 @@ def test_the_launches_meant_are_dealt_out_and_agree_with_whole_ones(dev, lens, H
     for name, x, y, z in zip(("out", "dq", "dk", "dv"), once(), want, once()):
         assert torch.equal(x, z), f"{name} is not reproducible"
         assert (x.float() - y.float()).norm() <= 2 ** -7 * y.float().norm(), name
+
+
+def test_dealt_out_launches_are_capturable(dev):
+    """All three launches dealt out, their tables and sums written anew by every replay: same bits as an eager call on the inputs at hand."""
+    from fgrpo import ops
+    lens, Hq, Hkv, D = [1500, 300, 40, 560, 200], 12, 2, 128
+    T = sum(lens)
+    assert launches(T, len(lens), max(lens), Hq, Hkv, D, True) == "fqk"
+    cu = torch.tensor([0] + torch.tensor(lens).cumsum(0).tolist(), dtype=torch.int32, device=dev)
+    q, k, v, do = operands(T, Hq, Hkv, D, dev)
+    q, k, v = (x.requires_grad_(True) for x in (q, k, v))
+
+    def once():
+        o = ops.varlen_attention(q, k, v, cu, None, True, None, max(lens))
+        return (o.detach(),) + torch.autograd.grad(o, (q, k, v), do)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        once()
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        held = once()
+    for seed in range(3):
+        with torch.no_grad():
+            for x in (q, k, v, do):
+                x.copy_(torch.randn(x.shape, generator=torch.Generator().manual_seed(seed)))
+        want = once()
+        graph.replay()
+        torch.cuda.synchronize()
+        for name, x, y in zip(("out", "dq", "dk", "dv"), held, want):
+            assert torch.equal(x, y), (seed, name)
